@@ -6,7 +6,8 @@
 //
 //   gemm_fma    any element types and any sizes; float32 multiply-add in ascending k
 //               for every output, so an output does not depend on its place in the batch.
-//               It is the true 32-bit path and the fallback for K not a multiple of 8.
+//               It is the fallback for K not a multiple of 8 and for operands of two types; float32 by
+//               float32 goes to gemm_f32.hip, whose sums are the same bit for bit, where that takes it.
 //   gemm_mfma   16-bit operands on the matrix cores (32x32x16), tiles staged through
 //               LDS, optional split over K into a float32 workspace.
 //   gemv_mfma   up to 16 rows of X (row-major W), gemv_tiled up to 64 rows (tiled W): W is

@@ -1,0 +1,277 @@
+// Matrix products of float32 operands  C[M, N] = X[M, K] . W[N, K]^T  on the matrix cores, for the 32-bit path.
+//
+// v_mfma_f32_16x16x4_f32 adds its products one after the other in ascending k, each as a fused multiply-add rounded to
+// nearest, subnormal numbers kept: an accumulator that takes k in ascending order is bit for bit the chain of fmaf that
+// gemm_fma runs (compared on an MI355X over operands of every magnitude).  Both kernels here sum as gemm_fma does, chains
+// over 256 consecutive k that are added up in ascending order, so a result depends neither on the kernel nor on the batch,
+// and a call that these do not take (K no multiple of 16, an address that is not 16-byte aligned) gives the same numbers
+// through gemm_fma.
+//
+//   gemv_f32   few rows of X: W from memory straight into operand A, the waves of a workgroup take chains in turn
+//   gemm_f32   more rows: tiles of W and X through LDS
+//
+// The operands lie row-major, so a lane fetches four consecutive k of its row with one 16-byte load; what instruction j
+// wants instead is k = 4 j + lane / 16.  gemv_f32 turns one into the other in registers, by four swaps of half waves and
+// of quarters (v_permlane32_swap, v_permlane16_swap) for four instructions; gemm_f32 on the way into LDS.
+#include "gemm_common.h"
+
+#define CHAIN 256                       // consecutive k of one chain of multiply-adds (as in gemm_fma)
+
+__device__ __forceinline__ f32x4 mfma16_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+__device__ __forceinline__ void swap32(float& x, float& y) {      // x's upper half wave <-> y's lower half wave
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(p[0]);
+    y = __uint_as_float(p[1]);
+}
+__device__ __forceinline__ void swap16(float& x, float& y) {      // the same within either half
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    x = __uint_as_float(p[0]);
+    y = __uint_as_float(p[1]);
+}
+// Lane l holds k = 4 (l / 16) .. + 3 of a row; afterwards element j holds k = 4 j + l / 16.
+__device__ __forceinline__ void to_operand16(f32x4& v) {
+    float a = v[0], b = v[1], c = v[2], d = v[3];
+    swap32(a, c);
+    swap32(b, d);
+    swap16(a, b);
+    swap16(c, d);
+    v = f32x4{a, b, c, d};
+}
+
+// ===========================================================================
+// gemv_f32: 16 NT rows of W, 16 MT rows of X, KW waves.  Wave w takes the chains w, w + KW, ... and leaves each
+// finished one in LDS, where a wave per 16 x 16 tile adds them up in ascending order: K is shared by the waves and the sum
+// is still taken in one order.  Bound by the stream of W: 128,256 x 2,048 at 3 rows 180 us, 5.8 TB/s (gemm_fma: 942 us);
+// 16,384 x 2,048 27 us, 5.0 TB/s (222); short products end a few us after their stream (2,048 x 2,048 9.7 us, 201 before;
+// 2,048 x 8,192 28, 862 before).  U steps of 16 k whose loads go out together: 4, so that eight waves fit a SIMD (with 16
+// the first of these takes 187 us, the second 37).
+// ===========================================================================
+template <int NT, int MT, int KW, int U>
+__global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, Epilogue e) {
+    __shared__ f32x4 part[KW][NT * MT][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+    const float *wp[NT], *xp[MT];                    // rows beyond the last are the last again, and not stored
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wp[t] = W + (int64_t)min(n0 + 16 * t + r, e.N - 1) * K + 4 * g;
+#pragma unroll
+    for (int j = 0; j < MT; ++j) xp[j] = X + (int64_t)min(m0 + 16 * j + r, e.M - 1) * K + 4 * g;
+    const int chains = (K + CHAIN - 1) / CHAIN;
+    constexpr int OWN = (NT * MT + KW - 1) / KW;     // tiles whose sums this wave adds up
+    f32x4 total[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) total[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c0 = 0; c0 < chains; c0 += KW) {
+        const int c = c0 + wave;
+        if (c < chains) {
+            f32x4 acc[NT][MT];
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            const int k0 = c * CHAIN, steps = min(CHAIN, K - k0) >> 4;
+            for (int s0 = 0; s0 < steps; s0 += U) {
+                f32x4 a[U][NT], b[U][MT];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int k = k0 + 16 * min(s0 + u, steps - 1);      // (a step that is not there: the last again, unused)
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) a[u][t] = *(const f32x4*)(wp[t] + k);
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) b[u][j] = *(const f32x4*)(xp[j] + k);
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    if (s0 + u < steps) {
+#pragma unroll
+                        for (int t = 0; t < NT; ++t) to_operand16(a[u][t]);
+#pragma unroll
+                        for (int j = 0; j < MT; ++j) to_operand16(b[u][j]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                                for (int j = 0; j < MT; ++j) acc[t][j] = mfma16_f32(a[u][t][i], b[u][j][i], acc[t][j]);
+                    }
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int j = 0; j < MT; ++j) part[wave][t * MT + j][lane] = acc[t][j];
+        }
+        __syncthreads();
+        const int have = min(KW, chains - c0);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            const int q = wave + o * KW;
+            if (q < NT * MT)
+                for (int w = 0; w < have; ++w) total[o] += part[w][q][lane];
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+        const int q = wave + o * KW;
+        if (q < NT * MT) {
+            const float v[4] = {total[o][0], total[o][1], total[o][2], total[o][3]};
+            epilogue4(e, m0 + 16 * (q % MT) + r, n0 + 16 * (q / MT) + 4 * g, v);
+        }
+    }
+}
+
+// ===========================================================================
+// gemm_f32: 64 rows of W x 64 rows of X, 4 waves of 32 x 32 (four sums of 16 x 16, which do not wait for each other), 32 of K a
+// stage, three stages in LDS.  While a stage is multiplied out of registers, the operands of the next are read from LDS,
+// the one after that is written to LDS and the third is on its way from memory, so that a workgroup alone on its CU
+// keeps the matrix cores busy.  In LDS the sixteen k of a step lie as the instructions want them (k = 4 j + g at 4 g + j), dealt
+// out as they are written: swapped in registers as gemv_f32 does it, they cost a third of the matrix
+// instructions' own time.  Rows are 36 floats apart, which keeps the 16-byte reads of a quarter wave on different banks.
+// Bound by the matrix instructions (32 cycles each) and the writes to LDS: 28,672 x 4,096 at 2,048 rows 3.99 ms, 121
+// TFLOP/s; at 400 rows 2,048 x 2,048 41 us (gemm_fma: 233), 16,384 x 2,048 259 us (1,076).
+// ===========================================================================
+__global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, int tiles_m, int tiles, Epilogue e) {
+    constexpr int BK = 32, LD = BK + 4, ST = 2 * 64 * LD;              // a stage in LDS: rows of W, then rows of X
+    __shared__ f32x4 lds4[3 * ST / 4];
+    float* lds = (float*)lds4;
+    // workgroups go round the eight XCDs: each XCD takes a run of tiles, the rows of X fastest, so that a tile of W is
+    // fetched into one L2
+    const int id = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (id >= tiles) return;
+    const int n0 = id / tiles_m * 64, m0 = id % tiles_m * 64;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+    const int wn = (wave & 1) * 32, wm = (wave >> 1) * 32;
+    f32x4 acc[2][2], total[2][2];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = total[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // this thread fetches four of the first and of the second sixteen k of a row of W and of X: a wave then writes to sixteen
+    // rows of LDS at a time, each on banks of its own
+    const int row = tid >> 2, kc = (tid & 3) * 4;
+    const float *wp = W + (int64_t)min(n0 + row, e.N - 1) * K, *xp = X + (int64_t)min(m0 + row, e.M - 1) * K;
+    f32x4 st[4];
+    auto fetch = [&](int k0) {                       // (what lies beyond K is the row's end again, and not multiplied)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = min(k0 + 16 * u + kc, K - 4);
+            st[u] = *(const f32x4*)(wp + k);
+            st[2 + u] = *(const f32x4*)(xp + k);
+        }
+    };
+    const int put_at = row * LD + (tid & 3);
+    auto put = [&](int at) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) lds[4 * at + put_at + 64 * (c >> 1) * LD + 16 * (c & 1) + 4 * q] = st[c][q];
+    };
+    const int w_at = (wn + r) * (LD / 4) + g, x_at = (64 + wm + r) * (LD / 4) + g;
+    f32x4 op[2][2][4];                               // [stage's parity][sixteen of K][two blocks of W, two of X]
+    auto operands = [&](f32x4 (&o)[2][4], int at) {                  // (`at`: in pieces of 16 bytes)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                o[u][i] = lds4[at + w_at + 4 * i * LD + 4 * u];
+                o[u][2 + i] = lds4[at + x_at + 4 * i * LD + 4 * u];
+            }
+    };
+    auto multiply = [&](f32x4 (&o)[4]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = mfma16_f32(o[i >> 1][q], o[2 + (i & 1)][q], acc[i >> 1][i & 1]);
+    };
+    fetch(0);
+    put(0);
+    fetch(BK);
+    put(ST / 4);
+    fetch(2 * BK);
+    __syncthreads();
+    operands(op[0], 0);
+    int next = ST / 4, after = 2 * ST / 4, spent = 0;        // the stages in LDS: the next one, the one that is written now, the last one
+    for (int k0 = 0; k0 < K; k0 += 2 * BK) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int k = k0 + b * BK;
+            if (k >= K) break;
+            if (k && k % CHAIN == 0) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    total[i >> 1][i & 1] += acc[i >> 1][i & 1];
+                    acc[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+            }
+            operands(op[b ^ 1], next);
+            multiply(op[b][0]);
+            put(after);
+            fetch(k + 3 * BK);
+            // the order of the instructions: an operand's read, a write or a load under every matrix instruction
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                __builtin_amdgcn_sched_group_barrier(0x200, 2, 0);
+                __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            }
+            if (k + 16 < K) multiply(op[b][1]);
+            __syncthreads();
+            const int t = next;
+            next = after;
+            after = spent;
+            spent = t;
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const f32x4 t = total[i >> 1][i & 1] + acc[i >> 1][i & 1];
+        const float v[4] = {t[0], t[1], t[2], t[3]};
+        epilogue4(e, m0 + wm + 16 * (i & 1) + r, n0 + wn + 16 * (i >> 1) + 4 * g, v);
+    }
+}
+
+// ===========================================================================
+// C interface
+// ===========================================================================
+// kind: 0 = by the sizes, 1 = gemv_f32 (at most 128 rows), 2 = gemm_f32.
+extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, int mode, int M, int N, int K, int kind,
+                           const RopeStore* rs, hipStream_t stream) {
+    int rc = check_common(X, W, C, M, N, K, mode, out_dt);
+    if (rc) return rc;
+    if (K % 16 != 0 || (((uintptr_t)X | (uintptr_t)W) & 15) || kind < 0 || kind > 2 || (kind == 1 && M > 128)) return LI_UNSUPPORTED;
+    if (M == 0) return LI_OK;
+    Epilogue e;
+    rc = make_epilogue(e, C, mode, out_dt, M, N, rs);
+    if (rc) return rc;
+    const int chains = (K + CHAIN - 1) / CHAIN, blocks = (N + 15) / 16;
+    // gemv_f32 has its workgroups by the rows of W alone, gemm_f32 fills the chip only where both sides have enough
+    // rows.  us at 64 rows of X: 2,048 x 2,048 25 against 41, 2,048 x 8,192 89 against 160, but 16,384 x 2,048 71 against 49; at
+    // 32 rows 16,384 x 2,048 46 against 49
+    if (kind == 0) kind = M <= 32 || (M <= 64 && blocks < 1024) || (M <= 128 && blocks <= 256) ? 1 : 2;
+    if (kind == 1) {
+        const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4), nt = M > 8 && blocks >= 1024 ? 2 : 1;
+        // sixteen waves where half the CUs have no workgroup (2,048 x 8,192 at 3 rows: 28 against 32 us), else eight; two
+        // blocks of W a wave where there are workgroups enough (28,672 x 4,096 at 32 rows: 164 against 169 us)
+        const int kw = chains <= 4 ? 4 : (mt == 1 && chains >= 16 && blocks <= 256 ? 16 : 8);
+#define GO(NT, MT, KW, U)                                                                                                       \
+    if (nt == NT && mt == MT && kw == KW) {                                                                                     \
+        gemv_f32_kernel<NT, MT, KW, U><<<dim3((blocks + NT - 1) / NT, (M + 16 * MT - 1) / (16 * MT)), 64 * KW, 0, stream>>>(X, W, K, e);                             \
+        LI_CHECK_LAUNCH();                                                                                                      \
+        return LI_OK;                                                                                                           \
+    }
+        GO(1, 1, 4, 4) GO(1, 1, 8, 4) GO(1, 1, 16, 4) GO(1, 2, 4, 8) GO(1, 2, 8, 8) GO(1, 4, 4, 4) GO(1, 4, 8, 4)
+        GO(2, 1, 4, 4) GO(2, 1, 8, 4) GO(2, 2, 4, 4) GO(2, 2, 8, 4) GO(2, 4, 4, 4) GO(2, 4, 8, 4)
+#undef GO
+        return LI_UNSUPPORTED;
+    }
+    const int tiles_m = (M + 63) / 64;
+    const int64_t tiles = (int64_t)tiles_m * ((N + 63) / 64);
+    if (tiles > (1 << 30)) return LI_UNSUPPORTED;
+    gemm_f32_kernel<<<(int)((tiles + 7) / 8 * 8), 256, 0, stream>>>(X, W, K, tiles_m, (int)tiles, e);
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}

@@ -28,7 +28,8 @@ ATTN_SOURCE = "attention.hip"
 MIXER_SOURCES = ("mixers.hip",)
 # the headers a library's sources include (its stamp covers them)
 HEADERS = {"libli_core.so": ("common.h", "gemm_common.h", "no_alloc.h"), "libli_hybrid.so": ("common.h", "conv.h"),
-           "libli_recurrent.so": ("common.h", "conv.h"), "libli_experts.so": ("common.h", "gemm_common.h")}
+           "libli_recurrent.so": ("common.h", "conv.h"), "libli_experts.so": ("common.h", "gemm_common.h"),
+           "libli_f32.so": ("common.h", "gemm_common.h")}
 DEFAULT_HEADERS = ("common.h",)
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
@@ -186,6 +187,15 @@ def attention_library(head_dim: int, force=False):
     return _load(f"libli_attn_hd{head_dim}.so", (ATTN_SOURCE,), (f"-DHEAD_DIM={head_dim}",), force)
 
 
+F32_SOURCES = ("gemm_f32.hip",)
+
+
+def f32_library(force=False):
+    """The 32-bit path's matrix products (csrc/gemm_f32.hip): a library of its own, so that a model of 16-bit weights is
+    not kept waiting for kernels that it does not run."""
+    return _load("libli_f32.so", F32_SOURCES, (), force)
+
+
 def mixers_library(force=False):
     """The kernels of the other mixers and arrangements (csrc/mixers.hip): a library of its own, so that a
     model is not kept waiting for kernels that it does not run."""
@@ -259,9 +269,10 @@ def sigmoid_attention_library(key_dim: int, value_dim: int, force=False):
 
 def build_all(head_dims=(16, 32, 48, 64, 128), force=True, sigmoid_head_dims=((48, 32), (128, 128)),
               diff_head_dims=((32, 64), (64, 128))) -> None:
-    """Compile the core library, the mixers' library, the attention library for each head size given and the
+    """Compile the core library, the 32-bit products' and the mixers' libraries, the attention library for each head size given and the
     sigmoid attention library for each pair of head sizes given."""
     core_library(force=force)
+    f32_library(force=force)
     mixers_library(force=force)
     hybrid_library(force=force)
     recurrent_library(force=force)

@@ -311,7 +311,10 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
     lib = core()
     same16 = x.dtype == w.dtype and x.dtype in (torch.float16, torch.bfloat16)
     fast_ok = same16 and k % 8 == 0 and x.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0
-    kind = force or ("fma" if not fast_ok else ("gemv_mfma" if m <= 16 else ("big" if m > 32 else "mfma")))
+    # float32 by float32 on the matrix cores, bit for bit what gemm_fma gives (which takes what these do not: any K, any
+    # address)
+    f32_ok = x.dtype == w.dtype == torch.float32 and k % 16 == 0 and x.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0
+    kind = force or ("f32" if f32_ok else "fma" if not fast_ok else ("gemv_mfma" if m <= 16 else ("big" if m > 32 else "mfma")))
     if tiled:
         _need(fast_ok and kind != "fma", "a tiled weight needs 16-bit activations of its dtype")
         # up to 16 rows (32 for a small matrix) every wave fetches the rows of X itself; beyond that
@@ -405,7 +408,11 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
         if na is not None:
             out._li_normed = (normed, nxt, eps, out._version)
         return out
-    if kind == "fma":
+    if kind.startswith("f32"):                                 # "f32[:<kernel>]" (a test's choice)
+        _need(f32_ok, "gemm_f32: float32 operands, K a multiple of 16")
+        _check(build.f32_library().li_gemm_f32(_ptr(x), _ptr(wd), _ptr(out), out_dt, mode, m, n, k,
+                                               int(kind[4:] or 0), rs, _stream()), "gemm_f32")
+    elif kind == "fma":
         _check(lib.li_gemm_fma(_ptr(x), DT[x.dtype], _ptr(w), DT[w.dtype], _ptr(out), out_dt, mode,
                                m, n, k, rs, _stream()), "gemm_fma")
     elif kind == "gemv_mfma":

@@ -107,6 +107,35 @@ def test_linear_all_kernels_and_epilogues(ops, M, N, K, dt):
                 assert torch.allclose(out16.double(), ref, rtol=_tol(dt), atol=_tol(dt))
 
 
+# the edges of the tiles of 16 and 64 rows, of the chains of 256 k, of the steps of 16 and 32, and of the rules by rows and sizes
+F32_CASES = [(1, 1, 16), (3, 33, 48), (8, 16400, 256), (9, 16400, 272), (16, 130, 4352), (17, 257, 528), (33, 64, 1040), (40, 16400, 288),
+             (64, 100, 4096), (65, 64, 32), (100, 200, 2064), (128, 4112, 512), (129, 130, 304), (300, 514, 8208)]
+
+
+@pytest.mark.parametrize("M,N,K", F32_CASES)
+def test_float32_products_on_the_matrix_cores_are_bit_equal(ops, M, N, K):
+    """gemm_f32's kernels against gemm_fma, whose order of sums they keep: bit for bit, with rows of every magnitude."""
+    g = torch.Generator().manual_seed(M + N + K)
+    scale = torch.exp2(torch.randint(-40, 40, (N, 1), generator=g).float())
+    x, w = torch.randn(M, K, generator=g).to(DEV), (torch.randn(N, K, generator=g) * scale).to(DEV)
+    res = torch.randn(M, N, generator=g).to(DEV)
+    for kind in [None, "f32:2"] + (["f32:1"] if M <= 128 else []):
+        for mode in (0, 1, 2):
+            if mode == 2 and N % 2:
+                continue
+            outs = []
+            for k in ("fma", kind):
+                out = res.clone() if mode == 1 else None
+                outs.append(ops.linear(x, w, mode, out=out, force=k))
+            assert torch.equal(*outs), (kind, mode)
+    # an address that is not 16-byte aligned goes to gemm_fma
+    if N * K > 4:
+        flat = torch.empty(N * K + 1, device=DEV)
+        off = flat[1:].view(N, K)
+        off.copy_(w)
+        assert torch.equal(ops.linear(x, off), ops.linear(x, w))
+
+
 TILED_CASES = [(1, 64, 64), (3, 172, 96), (16, 40, 4096), (9, 16400, 256), (17, 100, 64), (64, 256, 512),
                (33, 4100, 2048), (48, 72, 8192), (50, 6144, 4096), (65, 48, 32), (97, 200, 14336), (30, 520, 96), (128, 16, 160),
                (70, 200, 1024), (96, 1000, 416), (128, 136, 2048), (129, 384, 320), (256, 520, 2048), (384, 512, 192), (300, 1000, 96)]
