@@ -480,6 +480,26 @@ def test_attention_whole_prompts_and_decode(ops, H, K, hd, lens, dt):
             assert err < tol, (splits, err)
 
 
+# many tokens, so that heads of a KV head share a workgroup (as many as 256 / hd holds and H / K has divisors for); lengths at
+# the edges of the sixteens and of the 256 keys that are taken at a time; with and without a window that cuts into both
+@pytest.mark.parametrize("H,K,hd,n", [(4, 1, 64, 273), (12, 2, 16, 256), (6, 2, 48, 259), (32, 8, 128, 40)])
+def test_float32_attention_with_heads_in_one_workgroup(ops, H, K, hd, n):
+    from llm_infer_amd.engine.step import StepContext
+    g = torch.Generator().manual_seed(hd + n)
+    k, v, q = (torch.randn(n, m, hd, generator=g) for m in (K, K, H))
+    cache, view = _fill_cache(ops, torch.float32, K, hd, [(0, k, v)])
+    ctx = StepContext(DEV, [0], [[0] * n], [0], [[]])
+    qd = q.to(DEV)
+    for window in (None, 37):
+        out = ops.attention_f32(qd, view.as_tuple(), ctx.pos, ctx.tok_slot, H, K, hd, hd ** -0.5, window)
+        assert (out.double().cpu() - _attn_ref(q, k, v, window)).abs().max().item() < 2e-5      # (as for whole prompts above)
+        # a token by itself, its heads in workgroups of their own: the same sums in the same order
+        for t in (0, 15, 16, n - 1):
+            one = ops.attention_f32(qd[t:t + 1].contiguous(), view.as_tuple(), ctx.pos[t:t + 1], ctx.tok_slot[t:t + 1], H, K, hd,
+                                    hd ** -0.5, window)
+            assert torch.equal(one[0], out[t]), (window, t)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 def test_attention_window_and_far_key(ops, dt):
     """One far key among hundreds stands out by its score; the window cuts it off exactly at its edge."""
