@@ -16,7 +16,7 @@ import torch
 
 from ..kernels import ops
 from ..tensor import Tensor
-from .step import StepShared, decode_splits, split_bucket
+from .step import StepShared, decode_splits, page_splits, split_bucket
 
 
 @contextlib.contextmanager
@@ -66,6 +66,9 @@ class _GraphContext(StepShared):
 
     def decode_splits(self, n_kv_heads, n_heads):
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket)
+
+    def page_splits(self, n_kv_heads, n_heads):
+        return page_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket)
 
 
 MAX_RECORDED_STEPS = 48        # recorded steps an engine keeps; the least recently used goes first

@@ -71,6 +71,10 @@ class StepContext(StepShared):
         """How many ways the decode attention of a mixer with these heads cuts each sequence's context."""
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
 
+    def page_splits(self, n_kv_heads: int, n_heads: int) -> int:
+        """The same for the kernel whose waves merge inside a workgroup, where a page a split is worth it."""
+        return page_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
+
 
 def split_bucket(max_ctx: int) -> int:
     """The most splits that a context of this length is worth (a power of two up to 64): at least two
@@ -90,3 +94,12 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
     want = max(1, 1024 // max(1, waves))
     s = max(1, min(want, bucket))
     return 1 << (s.bit_length() - 1)
+
+
+def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
+    """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one
+    page a split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64."""
+    # measured on MI355X (heads of 128, 8 KV heads; us with half as many splits and with these): batch 1 at 180 tokens 8.8
+    # and 6.8, at 400 9.5 and 7.5, at 900 11.0 and 9.6, at 1,500 12.6 and 11.4, at 2,048 10.8 and 10.0; batch 8 at 300 9.7
+    # and 8.6, at 900 13.7 and 12.9; batch 16 at 900 20.7 and 20.2; batch 4 at 2,048 the same
+    return decode_splits(n_seqs, n_kv_heads, n_heads, min(2 * bucket, 64))

@@ -183,12 +183,12 @@ class GatedAttention(Part):
         return shares
 
     def _splits(self, ctx) -> int:
-        """Splits of the keys for the softmax decoder's decode kernel: what the step asks for, but at least two pages a
-        split of what the mask leaves (a power of two)."""
-        splits = ctx.decode_splits(self.n_kv_heads, self.n_heads)
+        """Splits of the keys for the softmax decoder's decode kernel: what the step asks for, but at least a page a split of
+        what the mask leaves (a power of two)."""
+        splits = ctx.page_splits(self.n_kv_heads, self.n_heads)
         for span in (self.block, self.window):
             if span:
-                splits = min(splits, max(1, (span + self.keep_first) // 128))
+                splits = min(splits, max(1, (span + self.keep_first) // 64))
         return 1 << (splits.bit_length() - 1)
 
     def attend(self, h, ctx, views, owns_cache, proj=None, col0=0):
