@@ -298,9 +298,51 @@ struct XGroups {
     int64_t stride;
 };
 
+// The experts of a routed layer side by side: `w` [M, cols] the weight of every token for every expert (0: not chosen), `ff`
+// hidden columns an expert, what lies behind n experts belonging to column n (a shared expert, or nothing).  An expert that no
+// token chose is not read.  `over` EXPERTS_IN_K (the down product): its part of K, whose hidden values are zeros;
+// EXPERTS_IN_N: its rows of W, whose sums are zeros then; EXPERTS_GATED the same with gate and up rows interleaved, and
+// every hidden value, rounded to its type, times the token's weight (what scale_blocks does behind the product).  The
+// experts' matrices are most of what a decode step reads: with eight experts of which two are chosen one token needs a
+// quarter of them, four tokens two thirds (4,096 wide, experts of 3,584, a step of four tokens 0.91 -> 0.79 ms).
+enum { EXPERTS_NONE = 0, EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
+struct ExpertBlocks {
+    const float* w;
+    int cols, n, ff, over;
+};
+
+// The experts (bits) that a token of 0 .. M - 1 chose; the same for every wave that asks.
+__device__ __forceinline__ unsigned long long chosen_experts(const ExpertBlocks& x, int M) {
+    const int lane = threadIdx.x & 63;
+    bool any = false;
+    if (lane < x.cols)
+        for (int m = 0; m < M; ++m) any |= x.w[m * x.cols + lane] != 0.f;
+    return __builtin_amdgcn_ballot_w64(any);
+}
+
+// EXPERTS_GATED: row m, rows n .. n + 3 of W (two hidden columns).
+template <class T>
+__device__ __forceinline__ void store_weighted(const Epilogue& e, const ExpertBlocks& x, int m, int n, const float* v) {
+    if (m >= e.M || n >= e.N) return;
+    const int col = n >> 1;
+    T h[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int ex = min((col + j) / x.ff, x.n);
+        const float w = x.w[m * x.cols + ex];
+        const float y = e.mode == EPI_CLAMPGLU
+            ? clamped_glu(v[2 * j], v[2 * j + 1], col + j >= e.gp.tail_col ? e.gp.tail_limit : e.gp.limit, e.gp.alpha, e.gp.shift)
+            : gate_activation(v[2 * j], e.mode == EPI_GEGLU) * v[2 * j + 1];
+        h[j] = from_f32<T>(w == 0.f ? 0.f : to_f32(from_f32<T>(y)) * w);
+    }
+    typedef typename Vec<T>::v2 v2;
+    *(v2*)((T*)e.C + (int64_t)m * (e.N >> 1) + col) = v2{h[0], h[1]};
+}
+
 template <class T, int NT, int MT, int KW>
 __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
-                                                             int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg) {
+                                                             int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg,
+                                                             ExpertBlocks ex) {
     if (xg.rows) X += min((int)blockIdx.x * NT * 16 / xg.rows, xg.n - 1) * xg.stride;
     // NT tiles of 16 rows of W and MT tiles of 16 rows of X per wave; W comes from HBM once, the
     // rows of X from the caches (they are few)
@@ -314,7 +356,22 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     const int n_tiles = (e.N + 15) >> 4;
     const int steps = K >> 5;
     const int per = (steps + KW - 1) / KW;
-    const int s_begin = wave * per, s_end = min(steps, s_begin + per);
+    int s_begin = wave * per, s_end = min(steps, s_begin + per), s_next = U;
+    unsigned long long chosen = ~0ull;
+    if (ex.over != EXPERTS_NONE) {
+        chosen = chosen_experts(ex, e.M);
+        if (ex.over == EXPERTS_IN_K) {               // the waves take turns, so that what is left out is left out for all of them
+            s_begin = wave * U;
+            s_end = steps;
+            s_next = KW * U;
+        } else {
+            const int rows = ex.over == EXPERTS_GATED ? 2 * ex.ff : ex.ff;
+            const int first = min(tile0 * 16 / rows, ex.n), last = min((tile0 * 16 + NT * 16 - 1) / rows, ex.n);
+            bool any = false;
+            for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
+            if (!any) s_end = s_begin;
+        }
+    }
     const T* wt[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) wt[t] = Wt + ((int64_t)min(tile0 + t, n_tiles - 1) * steps * 64 + lane) * 8;
@@ -346,7 +403,13 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
             for (int c = 0; c < 8; ++c) ss_mine += (i + c < hi) ? v[c] : 0.f;
         }
     }
-    for (int s0 = s_begin; s0 < s_end; s0 += U) {
+    for (int s0 = s_begin; s0 < s_end; s0 += s_next) {
+        if (ex.over == EXPERTS_IN_K) {
+            const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U, steps) * 32 - 1) / ex.ff, ex.n);
+            bool any = false;
+            for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
+            if (!any) continue;
+        }
         v8 a[U][NT], b[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -438,7 +501,8 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             float v[4] = {acc[t][j][0], acc[t][j][1], acc[t][j][2], acc[t][j][3]};
-            epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+            if (ex.over == EXPERTS_GATED) store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+            else epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
         }
 }
 
@@ -776,7 +840,7 @@ extern "C" int li_gemv_tiled_blocks(int M, int N, int K, int nt, int kw) {
 }
 
 static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode, int M, int N, int K, int nt, int kw,
-                      const RopeStore* rs, const RowsOut* ro, const RowScale* rsc, XGroups xg, hipStream_t stream) {
+                      const RopeStore* rs, const RowsOut* ro, const RowScale* rsc, XGroups xg, ExpertBlocks ex, hipStream_t stream) {
     int rc = check_common(X, Wt, C, M, N, K, mode, out_dt);
     if (rc) return rc;
     if (dt != DT_F16 && dt != DT_BF16) return LI_BAD_ARG;
@@ -798,7 +862,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     const RowScale no_scale{};
 #define LAUNCH(T, NT, MT, KW) \
     gemv_tiled_kernel<T, NT, MT, KW><<<blocks, 64 * KW, 0, stream>>>((const T*)X, (const T*)Wt, K, e, \
-                                                                     ro ? *ro : no_out, rsc ? *rsc : no_scale, xg)
+                                                                     ro ? *ro : no_out, rsc ? *rsc : no_scale, xg, ex)
 #define PICK_KW(T, NT, MT)                                \
     do {                                                  \
         if (kw == 4) LAUNCH(T, NT, MT, 4);                \
@@ -831,7 +895,22 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
 extern "C" int li_gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,
                              int M, int N, int K, int nt, int kw, const RopeStore* rs, const RowsOut* ro,
                              const RowScale* rsc, hipStream_t stream) {
-    return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, nt, kw, rs, ro, rsc, XGroups{0, 1, 0}, stream);
+    return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, nt, kw, rs, ro, rsc, XGroups{0, 1, 0}, ExpertBlocks{}, stream);
+}
+
+// The experts of a routed layer side by side (see ExpertBlocks), for at most 16 rows.
+extern "C" int li_gemv_tiled_experts(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode, int M, int N, int K,
+                                     const RopeStore* rs, const RowsOut* ro, const float* weights, int cols, int n, int ff, int over,
+                                     hipStream_t stream) {
+    if (M > 16 || !weights || n < 1 || ff < 1 || cols < n || cols > 64 || over < EXPERTS_IN_K || over > EXPERTS_GATED) return LI_BAD_ARG;
+    const int64_t all = over == EXPERTS_IN_K ? K : over == EXPERTS_GATED ? N / 2 : N;
+    if ((int64_t)n * ff > all || (cols == n && (int64_t)n * ff != all)) return LI_BAD_ARG;       // (what lies behind needs its column)
+    const bool gated = mode == EPI_SWIGLU || mode == EPI_GEGLU || mode == EPI_CLAMPGLU;
+    if (over == EXPERTS_GATED && (!gated || (N & 3) || ((uintptr_t)C & 3) || out_dt != dt)) return LI_BAD_ARG;
+    if (over == EXPERTS_IN_N && gated) return LI_BAD_ARG;
+    if (mode == EPI_CLAMPGLU && (!rs || ((const GluParams*)rs)->bias)) return LI_BAD_ARG;
+    return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, 0, 0, rs, ro, nullptr, XGroups{0, 1, 0},
+                      ExpertBlocks{weights, cols, n, ff, over}, stream);
 }
 
 // X [groups, M, K]: the rows of W from g * group_rows on (a multiple of 32; the last group: all that are left) against X[g].
@@ -839,7 +918,7 @@ extern "C" int li_gemv_tiled_groups(const void* X, const void* Wt, int dt, void*
                                     int group_rows, hipStream_t stream) {
     if (groups < 1 || group_rows <= 0 || group_rows % 32 || (int64_t)(groups - 1) * group_rows >= N) return LI_BAD_ARG;
     return gemv_tiled(X, Wt, dt, C, out_dt, EPI_STORE, M, N, K, 0, 0, nullptr, nullptr, nullptr,
-                      XGroups{group_rows, groups, (int64_t)M * K}, stream);
+                      XGroups{group_rows, groups, (int64_t)M * K}, ExpertBlocks{}, stream);
 }
 
 extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,

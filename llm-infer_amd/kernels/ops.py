@@ -267,11 +267,26 @@ def _workspace(n_floats: int, device) -> torch.Tensor:
     return ws
 
 
+EXPERTS_IN_K, EXPERTS_IN_N, EXPERTS_GATED = 1, 2, 3
+
+
+def experts_fit(x, w, n_experts: int, top: int, ff: int, gated: bool) -> bool:
+    """True if the products of experts side by side should leave out those that no token chose (``linear``'s ``experts``): few
+    rows against a tiled weight, of which a quarter of the experts is likely to go unread.  Measured with eight experts and
+    two chosen: 4 tokens 22.1 against 24.3 ms (Risonex, width 4,096, 17 steps behind a prompt), 8 tokens, which leave
+    one expert in ten, 14.9 against 14.7 (Dupolorn, width 2,048)."""
+    rows = x.shape[0]
+    return (is_tiled(w) and x.dtype == w.dtype and rows <= 8 and (1.0 - top / n_experts) ** rows >= 0.25 and n_experts + 1 <= 64
+            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and (not gated or ff % 2 == 0))
+
+
 def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None = None,
-           out_dtype=None, force: str | None = None, _rope=None, params=None) -> torch.Tensor:
+           out_dtype=None, force: str | None = None, _rope=None, params=None, experts=None) -> torch.Tensor:
     """C = X W^T with the epilogue ``mode``: store, add into ``out`` (float32), or act(gate) * up over
     interleaved gate/up rows of W (C has N/2 columns; EPI_SWIGLU: silu, EPI_GEGLU: gelu).  EPI_BIAS stores the sums plus
     a bias, EPI_CLAMPGLU the clamped gated activation of biased sums; both take ``params`` (``glu_params``).
+    ``experts`` (where ``experts_fit`` says so): (weights float32 [m, experts (+ 1)], number, hidden columns of one, EXPERTS_...),
+    the experts that no token chose are not read; EXPERTS_GATED also multiplies every hidden value by its weight.
     ``force`` picks a kernel for tests."""
     tiled = is_tiled(w)
     wd = w
@@ -346,7 +361,15 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
                               row_scales.data_ptr() if row_scales is not None else None)
             if lazy is not None:
                 rsc = _finish_norm(lazy, x)
-            if tall:
+            if experts is not None:
+                weights, number, ff, over = experts
+                _dev(weights)
+                _need(lazy is None and weights.dtype == torch.float32 and weights.dim() == 2 and weights.shape[0] == m,
+                      "experts: float32 weights, a row for every token")
+                _check(lib.li_gemv_tiled_experts(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, rs,
+                                                 ctypes.byref(ro) if ro is not None else None, _ptr(weights), weights.shape[1],
+                                                 number, ff, over, _stream()), "gemv_tiled_experts")
+            elif tall:
                 _check(lib.li_gemm_rows(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, x.stride(0), 1, 4,
                                         rs, ctypes.byref(ro) if ro is not None else None, _stream()), "gemm_rows")
             else:

@@ -188,7 +188,8 @@ class RoutedExperts(Part):
     zero where it was not chosen; one product against the down matrices side by side then sums the experts.
     Every token so runs through every expert's matrices: the same numbers as running only the chosen ones, every
     matrix streamed once, no shapes that depend on the data (a step can be recorded), at n_experts / top times the
-    arithmetic.  Many tokens in a 16-bit model (``GROUPED_FROM`` rows an expert on average): the tokens are listed
+    arithmetic.  For few tokens (``ops.experts_fit``) the products leave out the experts that none of them chose, by the
+    routing weights on the device.  Many tokens in a 16-bit model (``GROUPED_FROM`` rows an expert on average): the tokens are listed
     by expert on the device, the host reads the eight or so counts, and every expert runs its own two products on
     its own tokens' rows, added into the residual rows expert by expert (a fixed order)."""
 
@@ -329,9 +330,9 @@ class RoutedExperts(Part):
             return Tensor.wrap(flat, "tiled", (n, k), stacked.owner, stacked)
         return ops.prepare_weight(own.contiguous())
 
-    def _hidden(self, rows, w_up, weights, idx, col, blocks, ff, tail):
+    def _hidden(self, rows, w_up, weights, idx, col, blocks, ff, tail, experts=None):
         """The hidden rows of experts without a gate: the activation of the up product's sums, with the routing weight."""
-        z = ops.linear(rows, w_up, out_dtype=torch.float32)
+        z = ops.linear(rows, w_up, out_dtype=torch.float32, experts=experts)
         return ops.expert_act(z, weights, blocks, ff, tail, self.activation, self.on_input, self.dtype, idx, col)
 
     def _grouped_plain(self, h, residual, weights):
@@ -384,18 +385,24 @@ class RoutedExperts(Part):
         return (self.per_expert is not None and self.n_experts > 0 and h.shape[0] * self.top >= self.GROUPED_FROM * self.n_experts
                 and not torch.cuda.is_current_stream_capturing())
 
-    def _dense_hidden(self, h, weights):
-        """The hidden rows of all experts side by side, every expert's block with the token's weight for it."""
+    def _dense(self, h, weights, mode, out=None):
+        """All experts side by side: the hidden rows, every expert's block with the token's weight for it, and the down product of
+        them with the epilogue ``mode`` into ``out``.  For few tokens the experts that none of them chose are not read (their
+        hidden values are zeros either way)."""
+        n, f, tail = self.n_experts, self.expert_ff, self.shared_ff
+        few = n > 0 and ops.experts_fit(h, self.w_gate_up, n, self.top, f, self.gated) and ops.is_tiled(self.w_down)
+        over = (weights, n, f, ops.EXPERTS_GATED if self.gated else ops.EXPERTS_IN_N) if few else None
         if not self.gated:
-            return self._hidden(h, self.w_gate_up, weights, None, None, self.n_experts, self.expert_ff, self.shared_ff)
-        if self.clamped:
-            # the shared expert's outputs, behind the others', take its own limit
-            t = ops.linear(h, self.w_gate_up, ops.EPI_CLAMPGLU, out_dtype=self.dtype,
-                           params=ops.glu_params(None, self.limit, self.shared_limit, self.alpha, self.up_shift,
-                                                 self.n_experts * self.expert_ff))
+            t = self._hidden(h, self.w_gate_up, weights, None, None, n, f, tail, over)
         else:
-            t = ops.linear(h, self.w_gate_up, ops.EPI_SWIGLU, out_dtype=self.dtype)
-        return ops.scale_blocks(t, weights, self.n_experts, self.expert_ff, self.shared_ff)
+            params = None
+            if self.clamped:                     # the shared expert's outputs, behind the others', take its own limit
+                params = ops.glu_params(None, self.limit, self.shared_limit, self.alpha, self.up_shift, n * f)
+            t = ops.linear(h, self.w_gate_up, ops.EPI_CLAMPGLU if self.clamped else ops.EPI_SWIGLU, out_dtype=self.dtype, params=params,
+                           experts=over)
+            if not few:
+                t = ops.scale_blocks(t, weights, n, f, tail)
+        return ops.linear(t, self.w_down, mode, out=out, experts=(weights, n, f, ops.EXPERTS_IN_K) if few else None)
 
     def forward_rows(self, h, ctx=None, view=None, owns_cache=True):
         """The result as rows that are still a sum (``ops.PairSum``); by pairs only (``makes_rows``)."""
@@ -409,7 +416,7 @@ class RoutedExperts(Part):
         weights = self._weights(h, residual, ctx)
         if self._is_grouped(h):
             return self._grouped(h, residual, weights)
-        ops.linear(self._dense_hidden(h, weights), self.w_down, ops.EPI_ADD, out=residual)
+        self._dense(h, weights, ops.EPI_ADD, residual)
 
     def forward_into(self, h, out, ctx=None, view=None, owns_cache=True):
         """The result written over the float32 rows ``out``."""
@@ -417,5 +424,5 @@ class RoutedExperts(Part):
             out.zero_()                          # the outputs that pass a token on, or the experts one by one, add into it
             self.forward(h, out, ctx)
         else:
-            ops.linear(self._dense_hidden(h, self._weights(h, out, ctx)), self.w_down, out=out)
+            self._dense(h, self._weights(h, out, ctx), ops.EPI_STORE, out)
         return None

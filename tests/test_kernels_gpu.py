@@ -136,6 +136,47 @@ def test_float32_products_on_the_matrix_cores_are_bit_equal(ops, M, N, K):
         assert torch.equal(ops.linear(x, off), ops.linear(x, w))
 
 
+# rows, experts, hidden columns of one and of a shared expert: widths that no tile or batch of steps divides, one expert, many
+EXPERT_CASES = [(1, 8, 40, 24), (8, 8, 3584, 3584), (3, 3, 272, 0), (2, 40, 48, 16), (5, 1, 96, 32)]
+
+
+@pytest.mark.parametrize("M,n,ff,tail", EXPERT_CASES)
+@pytest.mark.parametrize("dt", F16S)
+def test_products_of_chosen_experts(ops, M, n, ff, tail, dt):
+    """Experts side by side with those that no token chose left out, against the same products of all of them: the same sums
+    in the hidden rows; the down product takes its own in another order."""
+    d, g = 256, torch.Generator().manual_seed(M + n + ff)
+    x = torch.randn(M, d, generator=g).to(dt).to(DEV)
+    weights = torch.rand(M, n + int(tail > 0), generator=g) + 0.1
+    weights[:, torch.randperm(n, generator=g)[:n // 2 + 1]] = 0.0        # (one expert: chosen by nobody)
+    weights = weights.to(DEV)
+    cols = n * ff + tail
+    gu = ops.tile_weight((torch.randn(2 * cols, d, generator=g) / 16).to(dt).to(DEV))
+    up = ops.tile_weight((torch.randn(cols, d, generator=g) / 16).to(dt).to(DEV))
+    assert ops.experts_fit(x[:1], gu, 8, 2, ff, True) and not ops.experts_fit(x, gu, n, n, ff, True)
+    glu = ops.glu_params(None, 0.9, 0.7, 1.702, 1.0, n * ff)
+    for mode, params in ((2, None), (ops.EPI_CLAMPGLU, glu)):
+        all_ = ops.scale_blocks(ops.linear(x, gu, mode, out_dtype=dt, params=params), weights, n, ff, tail)
+        few = ops.linear(x, gu, mode, out_dtype=dt, params=params, experts=(weights, n, ff, ops.EXPERTS_GATED))
+        # one product times one weight, rounded to float32 on the way or at once to the type: at most a step of the type apart
+        step = 2.0 ** -10 if dt == torch.float16 else 2.0 ** -7
+        assert bool(((all_.float() - few.float()).abs() <= step * all_.float().abs()).all()), mode
+        assert (all_ != few).float().mean().item() < 1e-3, mode
+    z = [ops.linear(x, up, out_dtype=torch.float32, experts=e) for e in (None, (weights, n, ff, ops.EXPERTS_IN_N))]
+    hidden = [ops.expert_act(v, weights, n, ff, tail, "relu2", True, dt) for v in z]
+    assert torch.equal(*hidden)
+    if cols % 32 == 0:
+        wd = (torch.randn(d, cols, generator=g) / 16).to(dt).to(DEV)
+        down = ops.tile_weight(wd)
+        for mode in (0, 1):
+            res = torch.randn(M, d, generator=g).to(DEV)
+            ref = few.double() @ wd.double().t() + (res.double() if mode else 0.0)
+            out = ops.linear(few, down, mode, out=res, experts=(weights, n, ff, ops.EXPERTS_IN_K))
+            # sums of `cols` products in float32: half a rounding step for each addition at most
+            bound = 2.0 ** -24 * cols * (few.double().abs() @ wd.double().abs().t()).max().item() + 1e-6
+            assert (out.double() - ref).abs().max().item() < bound, mode
+
+
 TILED_CASES = [(1, 64, 64), (3, 172, 96), (16, 40, 4096), (9, 16400, 256), (17, 100, 64), (64, 256, 512),
                (33, 4100, 2048), (48, 72, 8192), (50, 6144, 4096), (65, 48, 32), (97, 200, 14336), (30, 520, 96), (128, 16, 160),
                (70, 200, 1024), (96, 1000, 416), (128, 136, 2048), (129, 384, 320), (256, 520, 2048), (384, 512, 192), (300, 1000, 96)]
