@@ -64,6 +64,62 @@ __global__ __launch_bounds__(64 * SORT_WAVES) void sort_pairs_kernel(const int* 
     if (threadIdx.x == 0) { p.counts[e] = total; p.offsets[e] = offset; }
 }
 
+// The same from dense routing weights [T, cols] (0: not chosen; the first n_experts columns): a token's pairs are its weights that
+// are not 0, at most `top`, experts ascending; weights [T, top] beside slot_of, and weight_of [P] beside row_of.  Workgroup e
+// counts the pairs of the experts before its own, a run of tokens a thread, then deals out its own.
+#define DENSE_THREADS 1024
+
+__global__ __launch_bounds__(DENSE_THREADS) void pairs_of_weights_kernel(const float* __restrict__ dense, int cols, int n_tokens,
+                                                                         int top, Pairs p, float* __restrict__ weights,
+                                                                         float* __restrict__ weight_of) {
+    __shared__ int mine_of[DENSE_THREADS];
+    __shared__ int before_sum;
+    const int e = blockIdx.x, tid = threadIdx.x;
+    const int per = (n_tokens + DENSE_THREADS - 1) / DENSE_THREADS, lo = min(n_tokens, tid * per), hi = min(n_tokens, lo + per);
+    int mine = 0, before = 0;
+    for (int t = lo; t < hi; ++t) {
+        const float* w = dense + (int64_t)t * cols;
+        for (int i = 0; i < e; ++i) before += w[i] != 0.f;
+        mine += w[e] != 0.f;
+    }
+    if (tid == 0) before_sum = 0;
+    mine_of[tid] = mine;
+    __syncthreads();
+    atomicAdd(&before_sum, before);                        // (whole numbers: the order does not matter)
+    for (int o = 1; o < DENSE_THREADS; o <<= 1) {          // running sums
+        const int u = tid >= o ? mine_of[tid - o] : 0;
+        __syncthreads();
+        mine_of[tid] += u;
+        __syncthreads();
+    }
+    int at = before_sum + mine_of[tid] - mine;
+    for (int t = lo; t < hi; ++t) {
+        const float* w = dense + (int64_t)t * cols;
+        int rank = 0;
+        for (int i = 0; i < e; ++i) rank += w[i] != 0.f;
+        if (w[e] != 0.f && rank < top) {
+            p.row_of[at] = t;
+            p.slot_of[(int64_t)t * top + rank] = at;
+            weights[(int64_t)t * top + rank] = weight_of[at] = w[e];
+            ++at;
+        }
+        if (e == (int)gridDim.x - 1)                       // what a token does not use of its `top`
+            for (int j = rank + (w[e] != 0.f); j < top; ++j) { p.slot_of[(int64_t)t * top + j] = -1; weights[(int64_t)t * top + j] = 0.f; }
+    }
+    if (tid == 0) { p.counts[e] = mine_of[DENSE_THREADS - 1]; p.offsets[e] = before_sum; }
+}
+
+extern "C" int li_pairs_of_weights(const float* dense, int cols, int n_tokens, int top, int n_experts, int* counts, int* offsets,
+                                   int* row_of, int* slot_of, float* weights, float* weight_of, hipStream_t stream) {
+    if (n_tokens <= 0) return LI_OK;
+    if (!dense || cols < n_experts || top < 1 || n_experts < 1 || !counts || !offsets || !row_of || !slot_of || !weights || !weight_of)
+        return LI_BAD_ARG;
+    pairs_of_weights_kernel<<<n_experts, DENSE_THREADS, 0, stream>>>(dense, cols, n_tokens, top, Pairs{counts, offsets, row_of, slot_of},
+                                                                     weights, weight_of);
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
 extern "C" int li_sort_pairs(const int* chosen, int n, int top, int n_experts, int* counts, int* offsets, int* row_of,
                              int* slot_of, hipStream_t stream) {
     if (n <= 0) return LI_OK;

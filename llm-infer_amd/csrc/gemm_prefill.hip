@@ -231,18 +231,20 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(const T* __restrict__ X, 
 // fetch and multiply no rows that are not there).  A: how many steps ahead of their use the loads of W are
 // issued (2; 4 for products of few rows, where one workgroup a CU has to keep enough of W in flight by itself:
 // 8 NI KiB a wave instead of 4 NI; 3 for 65 to 128 rows, where two workgroups may share a CU).
+// MODE_PAIRS: the products of several experts as one launch (PairTiles): a tile of X is up to BM consecutive pairs of one
+// expert, read through row_of, and the workgroup's W is that expert's.  How many tiles there are is counted here, from the
+// experts' counts; the grid holds as many as there can be.  Every epilogue of MODE -1, K whole (MODE_PAIRS_GLU: the clamped
+// gated activation).
+enum { MODE_PAIRS = -2, MODE_PAIRS_GLU = -3 };
+__host__ __device__ constexpr bool by_pairs(int mode) { return mode == MODE_PAIRS || mode == MODE_PAIRS_GLU; }
+
 // The epilogue of one quad: the clamped gated activation and the bias have instantiations of their own, so that the
 // kernel of all the others holds none of their code (and stays within its registers).
 template <int MODE>
 __device__ __forceinline__ void wreg_epilogue(const Epilogue& e, int m, int n, const float* v) {
-    if constexpr (MODE == EPI_CLAMPGLU || MODE == EPI_BIAS) epilogue_extra4(e, m, n, v);
+    if constexpr (MODE == EPI_CLAMPGLU || MODE == EPI_BIAS || MODE == MODE_PAIRS_GLU) epilogue_extra4(e, m, n, v);
     else epilogue4_base(e, m, n, v);
 }
-
-// MODE_PAIRS: the products of several experts as one launch (PairTiles): a tile of X is up to BM consecutive pairs of one
-// expert, read through row_of, and the workgroup's W is that expert's.  How many tiles there are is counted here, from the
-// experts' counts; the grid holds as many as there can be.  Every epilogue of MODE -1, K whole.
-enum { MODE_PAIRS = -2 };
 
 template <class T, int NI, int MODE, int MJ = 8, int A = 2>
 __global__ __launch_bounds__(256) void gemm_wreg_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
@@ -261,7 +263,7 @@ __global__ __launch_bounds__(256) void gemm_wreg_kernel(const T* __restrict__ X,
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave;
     int bx, by, bz, m0;
-    if constexpr (MODE == MODE_PAIRS) {
+    if constexpr (by_pairs(MODE)) {
         int all = 0;
         for (int e0 = 0; e0 < pt.n_experts; e0 += 64) {
             int tiles = e0 + lane < pt.n_experts ? (pt.counts[e0 + lane] + BM - 1) / BM : 0;
@@ -326,7 +328,7 @@ __global__ __launch_bounds__(256) void gemm_wreg_kernel(const T* __restrict__ X,
     for (int i = 0; i < PER_WAVE; ++i) {
         const int q = wave * PER_WAVE + i, p = lane >> 3;
         int row = min(m0 + 8 * q + p, e.M - 1);
-        if constexpr (MODE == MODE_PAIRS) { if (pt.row_of) row = pt.row_of[row]; }
+        if constexpr (by_pairs(MODE)) { if (pt.row_of) row = pt.row_of[row]; }
         xoff[i] = ((uint32_t)row * (uint32_t)K + 8 * ((lane & 7) ^ p)) * 2;
     }
     // Loads past the last step of K are not branched around: they fetch the last step again (into a buffer
@@ -748,21 +750,22 @@ extern "C" int li_gemm_wreg(const void* X, const void* Wt, int dt, void* C, int 
 }
 
 // The products of several experts as one launch: C[p] = epilogue(W_e X[row_of[p]]) for all n_pairs pairs (PairTiles; mode
-// EPI_STORE or EPI_SWIGLU; N, K of one expert's matrix; x_rows: rows of X).  tile as for li_gemm_wreg; few_rows 1: the tile
+// EPI_STORE, EPI_SWIGLU or EPI_CLAMPGLU with its parameters gp; N, K of one expert's matrix; x_rows: rows of X).  tile as for li_gemm_wreg; few_rows 1: the tile
 // has 64 pairs (tile 2 only).
 extern "C" int li_gemm_wreg_pairs(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode, int x_rows, int n_pairs,
                                   int N, int K, int tile, int few_rows, const int* counts, const int* offsets, const int* row_of,
-                                  int n_experts, int64_t w_stride, hipStream_t stream) {
+                                  int n_experts, int64_t w_stride, const GluParams* gp, hipStream_t stream) {
     int rc = check_common(X, Wt, C, n_pairs, N, K, mode, out_dt);
     if (rc) return rc;
-    if ((dt != DT_F16 && dt != DT_BF16) || (mode != EPI_STORE && mode != EPI_SWIGLU) || !counts || !offsets || n_experts < 1)
+    if ((dt != DT_F16 && dt != DT_BF16) || (mode != EPI_STORE && mode != EPI_SWIGLU && mode != EPI_CLAMPGLU) || !counts || !offsets ||
+        n_experts < 1 || (mode == EPI_CLAMPGLU && (!gp || gp->bias)))
         return LI_BAD_ARG;
     if (tile < 0 || tile > 2 || few_rows < 0 || few_rows > 1 || (few_rows && tile != 2) || (!row_of && x_rows < n_pairs)) return LI_BAD_ARG;
     if (K % 32 != 0 || ((uintptr_t)X & 15) || ((uintptr_t)Wt & 15) || w_stride % 8) return LI_UNSUPPORTED;
     if ((int64_t)x_rows * K * 2 >= ((int64_t)1 << 32)) return LI_UNSUPPORTED;
     if (n_pairs == 0) return LI_OK;
     Epilogue e;
-    rc = make_epilogue(e, C, mode, out_dt, n_pairs, N, nullptr);
+    rc = make_epilogue(e, C, mode, out_dt, n_pairs, N, (const RopeStore*)gp);
     if (rc) return rc;
     const int bn = 256 - 64 * tile, bm = few_rows ? 64 : 128, ahead = few_rows ? 4 : 2, wg_blocks = bn / 16;
     const PairTiles pt{counts, offsets, row_of, n_experts, w_stride};
@@ -771,9 +774,9 @@ extern "C" int li_gemm_wreg_pairs(const void* X, const void* Wt, int dt, void* C
     const size_t stages = (size_t)(ahead + 1) * 2 * (bm / 16) * 1024, strips = (size_t)4 * 2 * 16 * (bn / 4 + 4) * 4;
     const size_t lds = (stages > strips ? stages : strips) + (size_t)2 * bm * 4 + (256 + 16) * 4;
     const int k_whole = (K + 31) / 32 * 32;
-#define GO(T, NI, MJ, A)                                                                                  \
+#define GO_MODE(T, NI, MODE, MJ, A)                                                                       \
     do {                                                                                                  \
-        auto kfn = gemm_wreg_kernel<T, NI, MODE_PAIRS, MJ, A>;                                            \
+        auto kfn = gemm_wreg_kernel<T, NI, MODE, MJ, A>;                                                  \
         if (lds > 64 * 1024) {                                                                            \
             static bool allowed = false;           /* more than 64 KiB of LDS is asked for once */       \
             if (!allowed && hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) \
@@ -781,6 +784,11 @@ extern "C" int li_gemm_wreg_pairs(const void* X, const void* Wt, int dt, void* C
             allowed = true;                                                                               \
         }                                                                                                 \
         kfn<<<grid, block, lds, stream>>>((const T*)X, (const T*)Wt, K, k_whole, nullptr, e, wg_blocks, RowScale{}, pt); \
+    } while (0)
+#define GO(T, NI, MJ, A)                                           \
+    do {                                                           \
+        if (mode == EPI_CLAMPGLU) GO_MODE(T, NI, MODE_PAIRS_GLU, MJ, A); \
+        else GO_MODE(T, NI, MODE_PAIRS, MJ, A);                    \
     } while (0)
 #define LAUNCH(T)                                       \
     do {                                                \
@@ -792,6 +800,7 @@ extern "C" int li_gemm_wreg_pairs(const void* X, const void* Wt, int dt, void* C
     if (dt == DT_F16) LAUNCH(f16); else LAUNCH(bf16);
 #undef LAUNCH
 #undef GO
+#undef GO_MODE
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

@@ -2200,6 +2200,19 @@ def route_pairs(h, w_router, bias, n_experts: int, top: int, scale: float = 1.0)
     return p
 
 
+def pairs_of_weights(weights, n_experts: int, top: int) -> SortedPairs:
+    """The pairs of a dense table of routing weights (float32 [T, >= n_experts]; 0: not chosen; at most ``top`` a row are not 0).
+    ``weight_of`` float32 [T * top]: the weight of every pair."""
+    _dev(weights)
+    _need(weights.dtype == torch.float32 and weights.dim() == 2 and weights.shape[1] >= n_experts >= 1 and top >= 1, "pairs_of_weights: float32 [T, experts]")
+    t = weights.shape[0]
+    p = SortedPairs(t, top, n_experts, weights.device)
+    p.weight_of = torch.empty((t * top, 1), dtype=torch.float32, device=weights.device)
+    _check(experts().li_pairs_of_weights(_ptr(weights), weights.shape[1], t, top, n_experts, _ptr(p.counts), _ptr(p.offsets), _ptr(p.row_of),
+                                         _ptr(p.slot_of), _ptr(p.weights), _ptr(p.weight_of), _stream()), "pairs_of_weights")
+    return p
+
+
 @functools.lru_cache(maxsize=1024)
 def _pairs_plan(pairs: int, n_experts: int, n: int, k: int) -> tuple:
     """(tile, few_rows) of gemm_wreg's pairs mode: tiles of 64 pairs where an expert has about half of that, else the tile
@@ -2213,10 +2226,12 @@ def _pairs_plan(pairs: int, n_experts: int, n: int, k: int) -> tuple:
     return min(((_wreg_cost(t, 1, pairs + 64 * n_experts, n, k), t) for t in (0, 1, 2)))[1], 0
 
 
-def linear_pairs(x, w, p: SortedPairs, mode: int = EPI_STORE, gather: bool = True, out_dtype=None, force: str | None = None) -> torch.Tensor:
+def linear_pairs(x, w, p: SortedPairs, mode: int = EPI_STORE, gather: bool = True, out_dtype=None, force: str | None = None,
+                 params=None) -> torch.Tensor:
     """Every pair's product with its expert's matrix: ``w`` is the experts' matrices [N, K] stacked in one tiled matrix
     [E N, K] (N a multiple of 16); row p of the result belongs to pair p and comes of row ``row_of[p]`` of ``x`` (``gather``
-    False: row p).  EPI_STORE, or EPI_SWIGLU over interleaved gate/up rows.  ``force`` "gemv" or "wreg:<tile>:<few rows>"
+    False: row p).  EPI_STORE, EPI_SWIGLU over interleaved gate/up rows, or EPI_CLAMPGLU with ``params`` (``glu_params`` without a
+    bias; for more than ten pairs an expert).  ``force`` "gemv" or "wreg:<tile>:<few rows>"
     picks a kernel for tests."""
     _dev(x, w)
     rows, k = matrix_shape(w)
@@ -2225,12 +2240,13 @@ def linear_pairs(x, w, p: SortedPairs, mode: int = EPI_STORE, gather: bool = Tru
     _need(is_tiled(w) and rows == n * e and n % 16 == 0 and x.dtype == w.dtype and x.dim() == 2 and x.shape[1] == k and x.is_contiguous(),
           "linear_pairs: the experts' matrices stacked and tiled, rows of their type")
     _need(x.shape[0] == (p.t if gather else pairs), "linear_pairs: a row for every token (or for every pair)")
-    _need(mode in (EPI_STORE, EPI_SWIGLU), "linear_pairs: store or silu(gate) * up")
-    out = torch.empty((pairs, n // 2 if mode == EPI_SWIGLU else n), dtype=out_dtype or x.dtype, device=x.device)
+    _need(mode in (EPI_STORE, EPI_SWIGLU) or (mode == EPI_CLAMPGLU and isinstance(params, _GluParams) and params._bias is None),
+          "linear_pairs: store, silu(gate) * up, or the clamped activation without a bias")
+    out = torch.empty((pairs, n // 2 if mode in GATED else n), dtype=out_dtype or x.dtype, device=x.device)
     row_of = _ptr(p.row_of) if gather else None
     # few pairs an expert: its matrix is streamed once straight into the operands (measured as above: 8 pairs an expert 156.5
     # and 82.7 us against 169.6 and 84.7, 16 pairs 206 and 114 against 172 and 87)
-    kind = force or ("gemv" if pairs <= 10 * e else "wreg")
+    kind = force or ("gemv" if pairs <= 10 * e and mode != EPI_CLAMPGLU else "wreg")
     if kind == "gemv":
         _check(experts().li_experts_gemv(_ptr(x), _ptr(w), DT[x.dtype], _ptr(out), DT[out.dtype], mode, pairs, n, k, c_int64(n * k), e,
                                          _ptr(p.counts), _ptr(p.offsets), row_of, _stream()), "experts_gemv")
@@ -2239,7 +2255,8 @@ def linear_pairs(x, w, p: SortedPairs, mode: int = EPI_STORE, gather: bool = Tru
     if ":" in kind:
         tile, few = (int(v) for v in kind.split(":")[1:3])
     _check(core().li_gemm_wreg_pairs(_ptr(x), _ptr(w), DT[x.dtype], _ptr(out), DT[out.dtype], mode, x.shape[0], pairs, n, k, tile, few,
-                                     _ptr(p.counts), _ptr(p.offsets), row_of, e, c_int64(n * k), _stream()), "gemm_wreg_pairs")
+                                     _ptr(p.counts), _ptr(p.offsets), row_of, e, c_int64(n * k),
+                                     ctypes.byref(params) if mode == EPI_CLAMPGLU else None, _stream()), "gemm_wreg_pairs")
     return out
 
 

@@ -189,13 +189,16 @@ class RoutedExperts(Part):
     Every token so runs through every expert's matrices: the same numbers as running only the chosen ones, every
     matrix streamed once, no shapes that depend on the data (a step can be recorded), at n_experts / top times the
     arithmetic.  For few tokens (``ops.experts_fit``) the products leave out the experts that none of them chose, by the
-    routing weights on the device.  Many tokens in a 16-bit model (``GROUPED_FROM`` rows an expert on average): the tokens are listed
-    by expert on the device, the host reads the eight or so counts, and every expert runs its own two products on
-    its own tokens' rows, added into the residual rows expert by expert (a fixed order)."""
+    routing weights on the device.  Many tokens in a 16-bit model (``GROUPED_FROM / 2`` rows an expert on average): the pairs of
+    token and chosen expert are sorted by expert on the device and every expert multiplies its own pairs' rows, all experts in one
+    launch a product; a token's results are added into its residual row expert by expert (a fixed order).  Matrices that do
+    not tile, or steps too long for the pairs' buffers (``_pairs_hold``), from ``GROUPED_FROM`` rows on: the host reads the
+    counts, and every expert runs products of its own."""
 
-    # measured (eight experts of 3,584, two chosen, width 4,096): a prompt of 512 tokens 2.94 ms with every token
-    # through every expert and 3.46 sorted by expert (40 launches a layer and a wait for the counts against 3 launches),
-    # 1,024 tokens 4.90 and 4.86, 2,048 tokens 8.58 and 7.50
+    # measured (eight experts, two chosen, ms a prompt with every token through every expert, and by pairs): Risonex 4,096 wide
+    # 256 tokens 2.20 and 2.22, 512 3.00 and 2.84, 1,500 7.19 and 5.52; Favizen 256 1.61 and 1.56, 1,500 5.07 and 3.90; Dupolorn
+    # 2,048 wide 512 1.88 and 1.90, 1,500 3.37 and 3.07.  With the counts read by the host (40 launches a layer) it pays from twice as
+    # many rows on (Risonex 1,024 tokens 4.90 and 4.86)
     GROUPED_FROM = 256
     makes_rows = False          # by pairs: forward_rows hands over the rows as a sum (set when the weights are bound)
     writes_rows = True          # forward_into overwrites the rows it is handed
@@ -277,12 +280,20 @@ class RoutedExperts(Part):
         self.w_down = ops.prepare_weight(torch.cat(down, 1).contiguous())
         # for prompts: every expert's matrices by themselves (gate and up as row ranges of the stacked matrix where
         # its tiles allow, the down matrices as copies of their own)
-        self.per_expert = None
+        self.per_expert = self.pair_weights = None
         if self.dtype != torch.float32:
             parts, at = [], 0
-            for (p, f), g_u, d_ in zip(self._experts(), gu, down):
+            # the down matrices one behind the other, for products by pairs (tiled, a matrix at multiples of 16 rows)
+            n_rows = (2 if self.gated else 1) * self.expert_ff
+            stacked = None
+            if (self.n_experts and ops.is_tiled(self.w_gate_up) and n_rows % 16 == 0 and d % 16 == 0 and self.expert_ff % 32 == 0
+                    and all(t.dtype == self.dtype for t in down[:self.n_experts])):
+                stacked = ops.prepare_weight(torch.cat([t.as_subclass(torch.Tensor) for t in down[:self.n_experts]], 0).contiguous())
+                self.pair_weights = (self.w_gate_up.rows_from(0, self.n_experts * n_rows), stacked)
+            for i, ((p, f), g_u, d_) in enumerate(zip(self._experts(), gu, down)):
                 rows = 2 * f if self.gated else f
-                parts.append((self._rows(self.w_gate_up, at, rows, g_u), ops.prepare_weight(d_.contiguous())))
+                w_d = stacked.rows_from(i * d, d) if stacked is not None and i < self.n_experts else ops.prepare_weight(d_.contiguous())
+                parts.append((self._rows(self.w_gate_up, at, rows, g_u), w_d))
                 at += rows
             self.per_expert = parts
         rows = ([] if self.table_routing else [tensors[n["router"]].float()]) + \
@@ -343,9 +354,17 @@ class RoutedExperts(Part):
                 t = self._hidden(ops.gather_rows(h, idx[e], n), w_up, weights, idx[e], e, 1, self.expert_ff, 0)
                 ops.scatter_add_rows(residual, ops.linear(t, w_d, out_dtype=torch.float32), idx[e], weights, None)
         if self.shared_ff:
-            w_up, w_d = self.per_expert[self.n_experts]
+            self._shared(h, residual, weights)
+
+    def _shared(self, h, residual, weights):
+        """The shared expert by itself, added into the residual rows."""
+        w_up, w_d = self.per_expert[self.n_experts]
+        if not self.gated:
             t = self._hidden(h, w_up, weights, None, self.n_experts, 1, self.shared_ff, 0)
             ops.linear(t, w_d, ops.EPI_ADD, out=residual)
+            return
+        t = self._gated_hidden(h, w_up, self.shared_ff, self.shared_limit)
+        ops.scatter_add_rows(residual, ops.linear(t, w_d, out_dtype=torch.float32), None, weights, self.n_experts)
 
     def _gated_hidden(self, rows, w_gu, ff, limit):
         """One gated expert's hidden rows (no routing weight)."""
@@ -354,7 +373,34 @@ class RoutedExperts(Part):
         return ops.linear(rows, w_gu, ops.EPI_CLAMPGLU, out_dtype=self.dtype,
                           params=ops.glu_params(None, limit, None, self.alpha, self.up_shift))
 
+    def _by_pairs(self, h, residual, weights):
+        """Every expert's products on its own tokens' rows, all experts in one launch each and nothing read back: the pairs of
+        the dense weights, sorted by expert on the device."""
+        w_up, w_down = self.pair_weights
+        p = ops.pairs_of_weights(weights, self.n_experts, self.top)
+        if not self.gated:
+            z = ops.linear_pairs(h, w_up, p, out_dtype=torch.float32)
+            t = ops.expert_act(z, p.weight_of, 1, self.expert_ff, 0, self.activation, self.on_input, self.dtype, None, 0)
+        elif self.clamped:
+            t = ops.linear_pairs(h, w_up, p, ops.EPI_CLAMPGLU, params=ops.glu_params(None, self.limit, None, self.alpha, self.up_shift))
+        else:
+            t = ops.linear_pairs(h, w_up, p, ops.EPI_SWIGLU)
+        rows = ops.linear_pairs(t, w_down, p, gather=False, out_dtype=torch.float32)
+        # (experts without a gate have their weight in the hidden row)
+        ops.PairSum(rows, p.slot_of, p.weights if self.gated else torch.ones_like(p.weights)).add_to(residual)
+
+    def _pairs_hold(self, h) -> bool:
+        """True where the pairs' products take the step: rows below 4 GiB, and 4 GiB of float32 results at most."""
+        pairs, e = h.shape[0] * self.top, h.element_size()
+        return (self.pair_weights is not None and h.is_contiguous() and h.data_ptr() % 16 == 0 and h.numel() * e < (1 << 32)
+                and pairs * self.expert_ff * e < (1 << 32) and pairs * max(self.hidden_size, 0 if self.gated else self.expert_ff) <= (1 << 30))
+
     def _grouped(self, h, residual, weights):
+        if self._pairs_hold(h):
+            self._by_pairs(h, residual, weights)
+            if self.shared_ff:
+                self._shared(h, residual, weights)
+            return
         if not self.gated:
             return self._grouped_plain(h, residual, weights)
         idx, counts = ops.moe_buckets(weights, self.n_experts)
@@ -364,9 +410,7 @@ class RoutedExperts(Part):
                 t = self._gated_hidden(ops.gather_rows(h, idx[e], n), w_gu, self.expert_ff, self.limit)
                 ops.scatter_add_rows(residual, ops.linear(t, w_d, out_dtype=torch.float32), idx[e], weights, e)
         if self.shared_ff:
-            w_gu, w_d = self.per_expert[self.n_experts]
-            t = self._gated_hidden(h, w_gu, self.shared_ff, self.shared_limit)
-            ops.scatter_add_rows(residual, ops.linear(t, w_d, out_dtype=torch.float32), None, weights, self.n_experts)
+            self._shared(h, residual, weights)
 
     def _weights(self, h, residual, ctx):
         """The dense row of routing weights of every token (the shared expert's in the last column)."""
@@ -382,7 +426,8 @@ class RoutedExperts(Part):
 
     def _is_grouped(self, h) -> bool:
         """True where every expert runs its own two products on its own tokens' rows."""
-        return (self.per_expert is not None and self.n_experts > 0 and h.shape[0] * self.top >= self.GROUPED_FROM * self.n_experts
+        limit = self.GROUPED_FROM // 2 if self._pairs_hold(h) else self.GROUPED_FROM
+        return (self.per_expert is not None and self.n_experts > 0 and h.shape[0] * self.top >= limit * self.n_experts
                 and not torch.cuda.is_current_stream_capturing())
 
     def _dense(self, h, weights, mode, out=None):

@@ -177,6 +177,26 @@ def test_products_of_chosen_experts(ops, M, n, ff, tail, dt):
             assert (out.double() - ref).abs().max().item() < bound, mode
 
 
+@pytest.mark.parametrize("T,E,top", [(1, 1, 1), (3, 8, 2), (1023, 5, 3), (1024, 8, 2), (1025, 3, 3), (2500, 70, 4)])
+def test_pairs_of_dense_routing_weights(ops, T, E, top):
+    g = torch.Generator().manual_seed(T + E)
+    w = torch.zeros(T, E + 1)
+    for t in range(T):
+        n = int(torch.randint(0, min(top, E) + 1, (1,), generator=g))          # a token may have fewer than `top`, or none
+        w[t, torch.randperm(E, generator=g)[:n]] = torch.rand(n, generator=g) + 0.1
+    p = ops.pairs_of_weights(w.to(DEV), E, top)
+    rows = [t for e in range(E) for t in range(T) if w[t, e] != 0]
+    counts = [(w[:, e] != 0).sum().item() for e in range(E)]
+    assert p.counts.tolist() == counts and p.offsets.tolist() == [sum(counts[:e]) for e in range(E)]
+    assert p.row_of[:len(rows)].tolist() == rows
+    place, slots, own = {}, torch.full((T, top), -1), torch.zeros(T, top)
+    for i, (e, t) in enumerate((e, t) for e in range(E) for t in range(T) if w[t, e] != 0):
+        j = place.get(t, 0)
+        slots[t, j], own[t, j], place[t] = i, w[t, e], j + 1
+    assert torch.equal(p.slot_of.cpu().long(), slots) and torch.equal(p.weights.cpu(), own)
+    assert p.weight_of[:len(rows), 0].tolist() == [w[t, e].item() for e in range(E) for t in range(T) if w[t, e] != 0]
+
+
 TILED_CASES = [(1, 64, 64), (3, 172, 96), (16, 40, 4096), (9, 16400, 256), (17, 100, 64), (64, 256, 512),
                (33, 4100, 2048), (48, 72, 8192), (50, 6144, 4096), (65, 48, 32), (97, 200, 14336), (30, 520, 96), (128, 16, 160),
                (70, 200, 1024), (96, 1000, 416), (128, 136, 2048), (129, 384, 320), (256, 520, 2048), (384, 512, 192), (300, 1000, 96)]
