@@ -4,7 +4,7 @@
 //
 // One wave per (tile of up to 32 consecutive tokens of a sequence, query head); a decode step's tiles hold one
 // token, and four waves then take every fourth 32 keys each and merge their running maxima, sums and outputs
-// through LDS in wave order.  A token at position p sees the keys lo .. p, lo = p - p % block (block 0: 0; window w: at least p - w + 1).
+// through LDS in wave order (all waves a part of the columns).  A token at position p sees the keys lo .. p, lo = p - p % block (block 0: 0; window w: at least p - w + 1).
 // Keys are walked 32 at a time.  Per map m:  S^T = K_m Q_m^T  (rows keys, columns queries; operand A straight from
 // the page, which holds keys in operand order), online softmax down the rows (a query's 32 scores lie in the 16
 // accumulator elements of two lanes), then O_m^T += V^T P_m^T with the accumulators' own order of the keys, in which the
@@ -241,76 +241,105 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
             }
         if constexpr (!TWO) fetch_v(kt_next);
     }
-    if (split && nw > 1) {
-        // a tile of one token whose keys the waves have shared: wave 0 adds up their states in wave order
-        constexpr int W = 2 + VALUE_DIM;
-        if (HC || col == 0) {
+    if constexpr (!PROMPT) {
+        // a tile of one token whose keys the waves have shared: the states of the columns that exist go to LDS as [wave][map][column]
+        // (outputs, behind them maxima and sums), then a wave takes a column, four values a lane, and adds them up in wave order (by
+        // the first wave alone, a lane half a column: latents of 256 / 192, 16 heads, batch 8 at 300 keys 23.5 us a token's keys
+        // in one workgroup, so 14.4; in two 15.9 and 13.4; two maps of 64 / 128, 32 heads, batch 4 at 500 keys in eight 20.1 and 14.3)
+        constexpr int LDW = VALUE_DIM + 4;
+        const int cols = HC ? min(32, per_kv - (group % hc_tiles) * 32) : 1;
+        float* stats = lds + nw * MAPS * cols * LDW;
+        if (HC ? head_ok : col == 0) {
 #pragma unroll
             for (int a = 0; a < MAPS; ++a) {
-                float* mine = lds + ((wave * MAPS + a) * (HC ? 32 : 1) + (HC ? col : 0)) * W;
-                if (half == 0) { mine[0] = m[a]; mine[1] = l[a]; }
+                const int at = (wave * MAPS + a) * cols + (HC ? col : 0);
 #pragma unroll
                 for (int b = 0; b < DVB; ++b)
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) mine[2 + b * 32 + 8 * (r >> 2) + 4 * half + (r & 3)] = o[a][b][r];
+                    for (int q4 = 0; q4 < 4; ++q4)
+                        *(f32x4*)(lds + at * LDW + b * 32 + 8 * q4 + 4 * half) =
+                            f32x4{o[a][b][4 * q4], o[a][b][4 * q4 + 1], o[a][b][4 * q4 + 2], o[a][b][4 * q4 + 3]};
+                if (half == 0) *(f32x2*)(stats + 2 * at) = f32x2{m[a], l[a]};
             }
         }
         __syncthreads();
+        // the sums of map a, column c, values d .. d + 3 over the waves
+        auto merged = [&](int a, int c, int d, float& M, float& L, f32x4& sum) {
+            f32x2 ml[4];
+            M = -INFINITY;
+            L = 0.f;
+            sum = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                ml[v] = *(const f32x2*)(stats + 2 * ((v * MAPS + a) * cols + c));
+                M = fmaxf(M, ml[v][0]);
+            }
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const float f = ml[v][0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[v][0] - M);
+                L += ml[v][1] * f;
+                const f32x4 t = *(const f32x4*)(lds + ((v * MAPS + a) * cols + c) * LDW + d);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum[e] += t[e] * f;
+            }
+        };
+        const int h0 = HC ? (group / hc_tiles) * per_kv + (group % hc_tiles) * 32 : h;           // column 0's head
         if (HC && gridDim.z > 1) {
             // the keys were shared among workgroups too: this one's sums go to `shares_out` [token, head, share, map,
-            // 2 + VALUE_DIM] (every wave a part of the values) and diff_attn_merge_kernel finishes
-            if (has_query) {
+            // 2 + VALUE_DIM] and diff_attn_merge_kernel finishes
+#pragma unroll 2
+            for (int i = threadIdx.x; i < cols * (VALUE_DIM / 4); i += 256) {
+                const int c = i / (VALUE_DIM / 4), d = i % (VALUE_DIM / 4) * 4;
 #pragma unroll
                 for (int a = 0; a < MAPS; ++a) {
-                    float* mine = shares_out + ((((int64_t)t0 * H + hq) * gridDim.z + blockIdx.z) * MAPS + a) * W;
-                    float M = -INFINITY, L = 0.f, f[4];
-                    for (int v = 0; v < nw; ++v) M = fmaxf(M, lds[((v * MAPS + a) * 32 + col) * W]);
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const float* theirs = lds + ((v * MAPS + a) * 32 + col) * W;
-                        f[v] = v >= nw || theirs[0] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(theirs[0] - M);
-                        if (v < nw) L += theirs[1] * f[v];
-                    }
-                    if (wave == 0 && half == 0) { mine[0] = M; mine[1] = L; }
-                    for (int i = 2 * wave + half; i < VALUE_DIM / 4; i += 2 * nw) {
-                        float sum[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                        for (int v = 0; v < 4; ++v)
-#pragma unroll
-                            for (int q = 0; q < 4; ++q)
-                                if (v < nw) sum[q] += lds[((v * MAPS + a) * 32 + col) * W + 2 + 4 * i + q] * f[v];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q) mine[2 + 4 * i + q] = sum[q];
-                    }
+                    float M, L;
+                    f32x4 sum;
+                    merged(a, c, d, M, L, sum);
+                    float* mine = shares_out + ((((int64_t)t0 * H + h0 + c) * gridDim.z + blockIdx.z) * MAPS + a) * (2 + VALUE_DIM);
+                    if (d == 0) *(f32x2*)mine = f32x2{M, L};
+                    *(f32x2*)(mine + 2 + d) = f32x2{sum[0], sum[1]};
+                    *(f32x2*)(mine + 4 + d) = f32x2{sum[2], sum[3]};
                 }
             }
             return;
         }
-        if (wave != 0) return;
-        if (HC || col == 0) {
-            const int cs = HC ? 32 : 1, c0 = HC ? col : 0;
+        const int d = min(4 * lane, VALUE_DIM - 4);
+        const bool own = 4 * lane < VALUE_DIM;
+#pragma unroll 2
+        for (int c = wave; c < cols; c += nw) {
+            const int hc_head = h0 + c;
+            f32x4 val = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int a = 0; a < MAPS; ++a) {
-                float M = -INFINITY;
-                for (int w = 0; w < nw; ++w) M = fmaxf(M, lds[((w * MAPS + a) * cs + c0) * W]);
-                float L = 0.f;
+                float M, L;
+                f32x4 sum;
+                merged(a, c, d, M, L, sum);
+                if (sink) {
+                    // the sink joins every map's sum as one more weight, exp(sink - maximum), with nothing to add to the output
+                    const float s2 = sink[hc_head] * 1.4426950408889634f, M2 = fmaxf(M, s2), f = __builtin_amdgcn_exp2f(M - M2);
+                    L = L * f + __builtin_amdgcn_exp2f(s2 - M2);
 #pragma unroll
-                for (int b = 0; b < DVB; ++b)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) o[a][b][r] = 0.f;
-                for (int w = 0; w < nw; ++w) {
-                    const float* theirs = lds + ((w * MAPS + a) * cs + c0) * W;
-                    if (theirs[0] == -INFINITY) continue;
-                    const float f = __builtin_amdgcn_exp2f(theirs[0] - M);
-                    L += theirs[1] * f;
-#pragma unroll
-                    for (int b = 0; b < DVB; ++b)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) o[a][b][r] += theirs[2 + b * 32 + 8 * (r >> 2) + 4 * half + (r & 3)] * f;
+                    for (int e = 0; e < 4; ++e) sum[e] *= f;
                 }
-                m[a] = M; l[a] = L;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) val[e] = a == 0 ? sum[e] / L : val[e] - lambda * (sum[e] / L);
             }
+            float ss = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                if (!own || d + e >= dv) val[e] = 0.f;
+                ss += val[e] * val[e];
+            }
+            float rr = out_scale;
+            if (out_eps >= 0.f) rr = out_scale / sqrtf(wave_sum(ss) / (float)dv + out_eps);
+            const float* grow = gate ? gate + (int64_t)t0 * gate_stride + gate_col : nullptr;
+            if (gate && !gate_elem) rr *= 1.f / (1.f + expf(-grow[hc_head]));
+            T* orow = out + ((int64_t)t0 * H + hc_head) * dv;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (own && d + e < dv) orow[d + e] = from_f32<T>(val[e] * rr * (gate_elem ? 1.f / (1.f + expf(-grow[hc_head * dv + d + e])) : 1.f));
         }
+        return;
     }
     if (sink) {
         // the sink joins every map's sum as one more weight, exp(sink - maximum), with nothing to add to the output
@@ -435,7 +464,7 @@ extern "C" int li_diffattn(const void* q, void* out, int dt, const void* k_pages
     const int shares = hc && key_shares > 1 && part ? key_shares : 1;
     dim3 grid(n_tiles, hc ? G * ((per_kv + 31) / 32) : H / heads, shares);
     const int threads = split ? 256 : 64 * heads;
-    const size_t lds = split ? (size_t)4 * maps * (hc ? 32 : 1) * (2 + VALUE_DIM) * sizeof(float) : 0;
+    const size_t lds = split ? (size_t)4 * maps * (hc ? (per_kv < 32 ? per_kv : 32) : 1) * (VALUE_DIM + 4 + 2) * sizeof(float) : 0;
 #define GO1(T, M, P, C)                                                                                                              \
     do {                                                                                                                             \
         auto kfn = diff_attn_mfma_kernel<T, M, P, C>;                                                                                \

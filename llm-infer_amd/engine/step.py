@@ -97,9 +97,10 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
 
 
 def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
-    """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one
-    page a split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64."""
+    """Splits for the decode kernels of softmax, differential and latent attention: as ``decode_splits``, but down to one page a
+    split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64."""
     # measured on MI355X (heads of 128, 8 KV heads; us with half as many splits and with these): batch 1 at 180 tokens 8.8
     # and 6.8, at 400 9.5 and 7.5, at 900 11.0 and 9.6, at 1,500 12.6 and 11.4, at 2,048 10.8 and 10.0; batch 8 at 300 9.7
-    # and 8.6, at 900 13.7 and 12.9; batch 16 at 900 20.7 and 20.2; batch 4 at 2,048 the same
+    # and 8.6, at 900 13.7 and 12.9; batch 16 at 900 20.7 and 20.2; batch 4 at 2,048 the same.  Latents of 256 / 192 (16 heads, batch 8)
+    # at 300 13.4 and 11.3, at 1,000 14.9 and 12.5; two maps of 64 with values of 128 (32 / 8 heads, batch 4) at 500 17.6 and 14.3
     return decode_splits(n_seqs, n_kv_heads, n_heads, min(2 * bucket, 64))
