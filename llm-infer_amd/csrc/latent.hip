@@ -532,6 +532,12 @@ extern "C" int li_head_linear(const void* in, int in_dt, int64_t in_st, int in_s
 // before every segment where its contribution was; PASS 3 runs every segment again from there and writes y.
 // y float32 [T, H * dv].
 // ---------------------------------------------------------------------------
+// A number as it would be read back from memory: no multiply-add joins how it was computed with what comes after.
+__device__ __forceinline__ float rounded(float x) {
+    asm("" : "+v"(x));
+    return x;
+}
+
 __global__ void mlstm_gates_kernel(const float* __restrict__ proj, int stride, int i_col, int f_col,
                                    const float* __restrict__ i_bias, const float* __restrict__ f_bias, float cap,
                                    float* __restrict__ coef, int n_tokens, int H) {
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(64) void mlstm_scan_kernel(
         decay *= a;
         float nq = 0.f;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) { nl[v] = a * nl[v] + b * kt[v]; nq += nl[v] * qt[v]; }
+        for (int v = 0; v < NV; ++v) { nl[v] = fmaf(a, nl[v], b * kt[v]); nq = fmaf(nl[v], qt[v], nq); }
         if (PASS != 1) nq = wave_sum(nq);
         // the registers that hold this wave's rows of k_t and q_t (the second half of them where the rows are shared)
         constexpr int NH = (NMAX + 63) / 64;
@@ -657,8 +663,8 @@ __global__ __launch_bounds__(64) void mlstm_scan_kernel(
             const float kk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(kh[i >> 6]), i & 63));
             float qq = 0.f;
             if (PASS != 1) qq = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(qh[i >> 6]), i & 63));
-            s[i] = a * s[i] + kk * bx;
-            if (PASS != 1) acc += s[i] * qq;
+            s[i] = fmaf(kk, bx, a * s[i]);                   // (said, as in mlstm_step_kernel: the two agree bit for bit)
+            if (PASS != 1) acc = fmaf(s[i], qq, acc);
         }
         if (PASS != 1 && live) {
             float* to = y + (int64_t)(q0 + t) * H * dv + h * dv + col;
@@ -679,14 +685,112 @@ __global__ __launch_bounds__(64) void mlstm_scan_kernel(
     }
 }
 
-// n of every (sequence, head) from the scratch memory into the state (m, behind it, is mlstm_max_kernel's).
+// One token of every sequence (a decode step): gates, m and the recurrence in one launch, the operations and their order
+// mlstm_scan_kernel's, so that a token gives the same bits whichever of the two it comes through.  Bound by S, read and
+// written once.  The scan's registers for all of a column make straight-line code of some 30 KB, which a workgroup runs
+// once for a single token: fetching instructions was what took the time.  Here S passes through in batches of 16 rows,
+// four of them on their way at a time, in a loop; q and k are read from LDS, four rows a read.  A workgroup has 64
+// columns of dv, a wave for each 128 rows of S, and adds the waves' halves of y itself (no cleared rows, no atomics).
+// Measured, all of a decode step's launches: 8 sequences of 4 heads of 256 x 512 35.6 -> 17.0 us, 64 of them 81 -> 62 (537 MB
+// of state: 8.6 TB/s with what the caches hold), 1 of them 24 -> 14; 32 of 4 heads of 64 x 128 14 -> 9.4.
+template <int RSPLIT>
+__global__ __launch_bounds__(64 * RSPLIT) void mlstm_step_kernel(
+    const float* __restrict__ proj, int stride, int q_col, int k_col, int v_col, int i_col, int f_col,
+    const float* __restrict__ i_bias, const float* __restrict__ f_bias, float cap, float qscale, float* __restrict__ S_state,
+    const float* __restrict__ nm_state, float* __restrict__ nm_new, const int* __restrict__ seq_slot, float* __restrict__ y,
+    int H, int d, int dv) {
+    constexpr int U = 16, AHEAD = 4, ROWS = 128, NV = 2 * RSPLIT;
+    __shared__ f32x4 qs[RSPLIT * ROWS / 4], ks[RSPLIT * ROWS / 4];
+    __shared__ float other[RSPLIT > 1 ? 64 : 1];
+    const int seq = blockIdx.x, h = blockIdx.y, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int col = blockIdx.z * 64 + lane, r0 = wave * ROWS, rows = min(ROWS, d - r0);
+    const bool live = col < dv;
+    const int64_t slot = (int64_t)seq_slot[seq] * H + h;
+    float* S = S_state + (slot * d + r0) * dv + min(col, dv - 1);
+    float s[AHEAD][U];
+    auto load = [&](float (&into)[U], int r) {               // rows that the head does not have: its last, not used
+        if (r >= rows) return;
+#pragma unroll
+        for (int u = 0; u < U; ++u) into[u] = S[(int64_t)min(r + u, rows - 1) * dv];
+    };
+#pragma unroll
+    for (int g = 0; g < AHEAD; ++g) load(s[g], g * U);
+    const float* __restrict__ row = proj + (int64_t)seq * stride;
+    const float* __restrict__ nm = nm_state + slot * (d + 1);
+    const float gi = row[i_col + h] + (i_bias ? i_bias[h] : 0.f), gf = row[f_col + h] + (f_bias ? f_bias[h] : 0.f);
+    const float x = live ? row[v_col + h * dv + col] : 0.f, m = nm[d];
+    float nl[NV], qv[NV], kv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        const int i = v * 64 + lane;
+        qv[v] = i < d ? row[q_col + h * d + i] * qscale : 0.f;
+        kv[v] = i < d ? row[k_col + h * d + i] : 0.f;
+        nl[v] = i < d ? nm[i] : 0.f;
+    }
+    const float ig = rounded(cap * tanhf(gi / cap)), fg = rounded(lt_logsigmoid(cap * tanhf(gf / cap)));
+    const float mn = fmaxf(fg + m, ig);
+    const float a = rounded(expf(fg + m - mn)), b = rounded(expf(ig - mn)), em = rounded(expf(-mn)), bx = b * x;
+    float nq = 0.f;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        nl[v] = fmaf(a, nl[v], b * kv[v]);
+        nq = fmaf(nl[v], qv[v], nq);
+        if (v >> 1 == wave) {                                // a wave lays down its own rows
+            ((float*)qs)[v * 64 + lane] = qv[v];
+            ((float*)ks)[v * 64 + lane] = kv[v];
+        }
+    }
+    nq = wave_sum(nq);
+    if (blockIdx.z == 0 && wave == 0) {
+        float* to = nm_new + ((int64_t)seq * H + h) * (d + 1);
+#pragma unroll
+        for (int v = 0; v < NV; ++v) if (v * 64 + lane < d) to[v * 64 + lane] = nl[v];
+        if (lane == 0) to[d] = mn;
+    }
+    __syncthreads();
+    float acc = 0.f;
+    for (int r = 0; r < rows; r += AHEAD * U) {
+#pragma unroll
+        for (int g = 0; g < AHEAD; ++g) {
+            const int rg = r + g * U;
+            if (rg >= rows) break;
+            const int left = rows - rg;
+#pragma unroll
+            for (int u = 0; u < U; u += 4) {
+                const f32x4 k4 = ks[(r0 + rg + u) >> 2], q4 = qs[(r0 + rg + u) >> 2];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if (u + j < left) {
+                        s[g][u + j] = fmaf(k4[j], bx, a * s[g][u + j]);
+                        acc = fmaf(s[g][u + j], q4[j], acc);
+                    }
+                }
+            }
+            if (live) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) if (u < left) S[(int64_t)(rg + u) * dv] = s[g][u];
+            }
+            load(s[g], rg + AHEAD * U);
+        }
+    }
+    acc /= fmaxf(fabsf(nq), em) + 1e-6f;
+    if (RSPLIT > 1) {
+        if (wave) other[lane] = acc;
+        __syncthreads();
+        if (wave) return;
+        acc += other[lane];
+    }
+    if (live) y[(int64_t)seq * H * dv + h * dv + col] = acc;
+}
+
+// n of every (sequence, head), and with `len` d + 1 also m behind it, from the scratch memory into the state.
 __global__ void mlstm_commit_kernel(const float* __restrict__ nm_new, float* __restrict__ nm_state,
-                                    const int* __restrict__ seq_slot, const int* __restrict__ seq_qlen, int H, int d) {
+                                    const int* __restrict__ seq_slot, const int* __restrict__ seq_qlen, int H, int d, int len) {
     const int seq = blockIdx.x, h = blockIdx.y;
     if (seq_qlen && seq_qlen[seq] <= 0) return;
     const float* from = nm_new + ((int64_t)seq * H + h) * (d + 1);
     float* to = nm_state + ((int64_t)seq_slot[seq] * H + h) * (d + 1);
-    for (int i = threadIdx.x; i < d; i += blockDim.x) to[i] = from[i];
+    for (int i = threadIdx.x; i < len; i += blockDim.x) to[i] = from[i];
 }
 
 // One thread per element of a head's state (`per_head` of them, `state_stride` floats from head to head in the
@@ -718,7 +822,8 @@ __global__ void seg_combine_kernel(float* __restrict__ state, int64_t state_stri
         else MLSTM_GO(128, 4, 2, PASS, GRID);                                                                          \
     } while (0)
 
-// y must be cleared where d > 128 (two waves add their halves into it).  coef: scratch float32 [T, H, 3]; nm_new: scratch float32 [sequences, H, d + 1].  n_segs > 0 (with the segment lists and
+// Without seq_qlen every sequence has one token (mlstm_step_kernel; coef is not used).  Else y must be cleared where
+// d > 128 (two waves add their halves into it).  coef: scratch float32 [T, H, 3]; nm_new: scratch float32 [sequences, H, d + 1].  n_segs > 0 (with the segment lists and
 // scratch seg_S [segments, H, d, dv], seg_nrm [segments, H, d], seg_decay [segments, H]): the tokens run in segments.
 extern "C" int li_mlstm_scan(const float* proj, int stride, int q_col, int k_col, int v_col, int i_col, int f_col,
                              const float* i_bias, const float* f_bias, float cap, float qscale, float* S_state,
@@ -728,8 +833,19 @@ extern "C" int li_mlstm_scan(const float* proj, int stride, int q_col, int k_col
                              const int* seq_nseg, int n_segs, float* seg_S, float* seg_nrm, float* seg_decay,
                              hipStream_t stream) {
     if (n_seqs <= 0 || n_tokens <= 0) return LI_OK;
-    if (H <= 0 || d <= 0 || dv <= 0 || !(cap > 0.f) || !coef) return LI_BAD_ARG;
+    if (H <= 0 || d <= 0 || dv <= 0 || !(cap > 0.f) || (seq_qlen && !coef)) return LI_BAD_ARG;
     if (d > 256) return LI_UNSUPPORTED;
+    if (!seq_qlen && n_segs <= 0) {                          // a decode step
+        if (!nm_new || seq_qstart || n_tokens != n_seqs) return LI_BAD_ARG;
+        dim3 grid(n_seqs, H, (dv + 63) / 64);
+#define STEP(RS) mlstm_step_kernel<RS><<<grid, 64 * RS, 0, stream>>>(proj, stride, q_col, k_col, v_col, i_col, f_col, i_bias, f_bias, cap, \
+                                                                   qscale, S_state, nm_state, nm_new, seq_slot, y, H, d, dv)
+        if (d > 128) STEP(2); else STEP(1);
+#undef STEP
+        mlstm_commit_kernel<<<dim3(n_seqs, H), 64, 0, stream>>>(nm_new, nm_state, seq_slot, seq_qlen, H, d, d + 1);
+        LI_CHECK_LAUNCH();
+        return LI_OK;
+    }
     mlstm_gates_kernel<<<(n_tokens * H + 255) / 256, 256, 0, stream>>>(proj, stride, i_col, f_col, i_bias, f_bias, cap, coef,
                                                                        n_tokens, H);
     mlstm_max_kernel<<<n_seqs * H, 64, 0, stream>>>(coef, nm_state, seq_slot, seq_qstart, seq_qlen, H, d);
@@ -738,7 +854,7 @@ extern "C" int li_mlstm_scan(const float* proj, int stride, int q_col, int k_col
         if (!nm_new) return LI_BAD_ARG;
         dim3 grid(n_seqs, H, (dv + 63) / 64 * (d > 128 ? 2 : 1));
         MLSTM_LAUNCH(0, grid);
-        mlstm_commit_kernel<<<dim3(n_seqs, H), 64, 0, stream>>>(nm_new, nm_state, seq_slot, seq_qlen, H, d);
+        mlstm_commit_kernel<<<dim3(n_seqs, H), 64, 0, stream>>>(nm_new, nm_state, seq_slot, seq_qlen, H, d, d);
     } else {
         if (!seq_qstart || !seq_qlen || !seg_seq || !seg_t0 || !seg_n || !seq_seg0 || !seq_nseg || !seg_S || !seg_nrm || !seg_decay)
             return LI_BAD_ARG;

@@ -586,3 +586,31 @@ def test_command_line_reports_and_generates(lib, models):
     info = subprocess.run([sys.executable, os.path.join(root, "bin", "model_info"), folder], capture_output=True, text=True,
                           timeout=300)
     assert info.returncode == 0 and "Architecture: Dupolorn" in info.stdout and "The tensors fit the model." in info.stdout
+
+
+@pytest.mark.parametrize("H, d, dv", [(1, 1, 1), (3, 16, 64), (2, 17, 65), (2, 64, 40), (2, 81, 130), (1, 128, 64), (2, 129, 100), (1, 200, 33), (2, 256, 192)])
+def test_matrix_memory_of_one_token_is_the_walk(lib, H, d, dv):
+    """A decode step has a kernel of its own: y, S, n and m are the same bits as from the walk over a prompt of one
+    token, at edges of its batches of 16 rows, of 64 columns and of the 128 rows of a wave; other slots are not touched."""
+    from types import SimpleNamespace
+    from llm_infer_amd.kernels import ops
+    T, slots = 3, 5
+    g = torch.Generator().manual_seed(d + dv)
+    i_col = 2 * H * d + H * dv
+    proj = torch.randn(T, i_col + 2 * H, generator=g).to(DEV)
+    i_bias, f_bias = torch.randn(H, generator=g).to(DEV), torch.randn(H, generator=g).to(DEV)
+    slot = torch.tensor([3, 0, 4], dtype=torch.int32, device=DEV)
+    S0, n0 = torch.randn(slots, H, d, dv, generator=g).to(DEV), torch.randn(slots, H, d + 1, generator=g).to(DEV)
+    got = []
+    for walk in (False, True):
+        ctx = SimpleNamespace(seq_slot=slot, n_seqs=T, seq_qstart=None, seq_qlen=None)
+        if walk:
+            ctx.seq_qstart = torch.arange(T, dtype=torch.int32, device=DEV)
+            ctx.seq_qlen = torch.ones(T, dtype=torch.int32, device=DEV)
+        S, n = S0.clone(), n0.clone()
+        y = ops.mlstm_scan(proj, 0, H * d, 2 * H * d, i_col, i_col + H, i_bias, f_bias, 15.0, d ** -0.5, S, n, ctx, H, d, dv)
+        got.append((y, S, n))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    for s in (1, 2):
+        assert torch.equal(got[0][1][s], S0[s]) and torch.equal(got[0][2][s], n0[s])
