@@ -305,7 +305,7 @@ struct XGroups {
 // every hidden value, rounded to its type, times the token's weight (what scale_blocks does behind the product).  The
 // experts' matrices are most of what a decode step reads: with eight experts of which two are chosen one token needs a
 // quarter of them, four tokens two thirds (4,096 wide, experts of 3,584, a step of four tokens 0.91 -> 0.79 ms).
-enum { EXPERTS_NONE = 0, EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
+enum { EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
 struct ExpertBlocks {
     const float* w;
     int cols, n, ff, over;
@@ -339,10 +339,15 @@ __device__ __forceinline__ void store_weighted(const Epilogue& e, const ExpertBl
     *(v2*)((T*)e.C + (int64_t)m * (e.N >> 1) + col) = v2{h[0], h[1]};
 }
 
-template <class T, int NT, int MT, int KW>
+// EB: ExpertBlocks, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
+// cost a whole matrix's product some 0.3 us, 1% of a decode step.)
+struct NoExperts {};
+
+template <class T, int NT, int MT, int KW, class EB>
 __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
                                                              int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg,
-                                                             ExpertBlocks ex) {
+                                                             EB ex) {
+    constexpr bool EXPERTS = sizeof(EB) == sizeof(ExpertBlocks);
     if (xg.rows) X += min((int)blockIdx.x * NT * 16 / xg.rows, xg.n - 1) * xg.stride;
     // NT tiles of 16 rows of W and MT tiles of 16 rows of X per wave; W comes from HBM once, the
     // rows of X from the caches (they are few)
@@ -358,7 +363,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     const int per = (steps + KW - 1) / KW;
     int s_begin = wave * per, s_end = min(steps, s_begin + per), s_next = U;
     unsigned long long chosen = ~0ull;
-    if (ex.over != EXPERTS_NONE) {
+    if constexpr (EXPERTS) {
         chosen = chosen_experts(ex, e.M);
         if (ex.over == EXPERTS_IN_K) {               // the waves take turns, so that what is left out is left out for all of them
             s_begin = wave * U;
@@ -404,7 +409,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
         }
     }
     for (int s0 = s_begin; s0 < s_end; s0 += s_next) {
-        if (ex.over == EXPERTS_IN_K) {
+        if constexpr (EXPERTS) if (ex.over == EXPERTS_IN_K) {
             const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U, steps) * 32 - 1) / ex.ff, ex.n);
             bool any = false;
             for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
@@ -501,8 +506,11 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             float v[4] = {acc[t][j][0], acc[t][j][1], acc[t][j][2], acc[t][j][3]};
-            if (ex.over == EXPERTS_GATED) store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
-            else epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+            if constexpr (EXPERTS) if (ex.over == EXPERTS_GATED) {
+                store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+                continue;
+            }
+            epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
         }
 }
 
@@ -839,8 +847,9 @@ extern "C" int li_gemv_tiled_blocks(int M, int N, int K, int nt, int kw) {
     return blocks;
 }
 
+template <class EB>
 static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode, int M, int N, int K, int nt, int kw,
-                      const RopeStore* rs, const RowsOut* ro, const RowScale* rsc, XGroups xg, ExpertBlocks ex, hipStream_t stream) {
+                      const RopeStore* rs, const RowsOut* ro, const RowScale* rsc, XGroups xg, EB ex, hipStream_t stream) {
     int rc = check_common(X, Wt, C, M, N, K, mode, out_dt);
     if (rc) return rc;
     if (dt != DT_F16 && dt != DT_BF16) return LI_BAD_ARG;
@@ -861,7 +870,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     const RowsOut no_out{};
     const RowScale no_scale{};
 #define LAUNCH(T, NT, MT, KW) \
-    gemv_tiled_kernel<T, NT, MT, KW><<<blocks, 64 * KW, 0, stream>>>((const T*)X, (const T*)Wt, K, e, \
+    gemv_tiled_kernel<T, NT, MT, KW, EB><<<blocks, 64 * KW, 0, stream>>>((const T*)X, (const T*)Wt, K, e, \
                                                                      ro ? *ro : no_out, rsc ? *rsc : no_scale, xg, ex)
 #define PICK_KW(T, NT, MT)                                \
     do {                                                  \
@@ -873,9 +882,12 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     do {                                                  \
         if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
         else if (mt == 1 && nt == 2) PICK_KW(T, 2, 1);    \
-        else if (mt == 2 && nt == 1) PICK_KW(T, 1, 2);    \
-        else if (mt == 2 && nt == 2) PICK_KW(T, 2, 2);    \
-        else if (mt <= 4 && nt == 2) PICK_KW(T, 2, 4);    \
+        else if constexpr (sizeof(EB) != sizeof(ExpertBlocks)) { \
+            if (mt == 2 && nt == 1) PICK_KW(T, 1, 2);     \
+            else if (mt == 2 && nt == 2) PICK_KW(T, 2, 2); \
+            else if (mt <= 4 && nt == 2) PICK_KW(T, 2, 4); \
+            else return LI_BAD_ARG;                       \
+        }                                                 \
         else return LI_BAD_ARG;                           \
     } while (0)
     if (dt == DT_F16) PICK(f16); else PICK(bf16);
@@ -895,7 +907,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
 extern "C" int li_gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,
                              int M, int N, int K, int nt, int kw, const RopeStore* rs, const RowsOut* ro,
                              const RowScale* rsc, hipStream_t stream) {
-    return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, nt, kw, rs, ro, rsc, XGroups{0, 1, 0}, ExpertBlocks{}, stream);
+    return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, nt, kw, rs, ro, rsc, XGroups{0, 1, 0}, NoExperts{}, stream);
 }
 
 // The experts of a routed layer side by side (see ExpertBlocks), for at most 16 rows.
@@ -918,7 +930,7 @@ extern "C" int li_gemv_tiled_groups(const void* X, const void* Wt, int dt, void*
                                     int group_rows, hipStream_t stream) {
     if (groups < 1 || group_rows <= 0 || group_rows % 32 || (int64_t)(groups - 1) * group_rows >= N) return LI_BAD_ARG;
     return gemv_tiled(X, Wt, dt, C, out_dt, EPI_STORE, M, N, K, 0, 0, nullptr, nullptr, nullptr,
-                      XGroups{group_rows, groups, (int64_t)M * K}, ExpertBlocks{}, stream);
+                      XGroups{group_rows, groups, (int64_t)M * K}, NoExperts{}, stream);
 }
 
 extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,
