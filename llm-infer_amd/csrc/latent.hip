@@ -691,8 +691,8 @@ __global__ __launch_bounds__(64) void mlstm_scan_kernel(
 // once for a single token: fetching instructions was what took the time.  Here S passes through in batches of 16 rows,
 // four of them on their way at a time, in a loop; q and k are read from LDS, four rows a read.  A workgroup has 64
 // columns of dv, a wave for each 128 rows of S, and adds the waves' halves of y itself (no cleared rows, no atomics).
-// Measured, all of a decode step's launches: 8 sequences of 4 heads of 256 x 512 35.6 -> 17.0 us, 64 of them 81 -> 62 (537 MB
-// of state: 8.6 TB/s with what the caches hold), 1 of them 24 -> 14; 32 of 4 heads of 64 x 128 14 -> 9.4.
+// Measured, all of a decode step's launches: 8 sequences of 4 heads of 256 x 512 35.6 -> 17.3 us, 64 of them 81 -> 62 (268 MB of
+// state read and written, 4.3 TB/s, a copy's rate being 4.9), 1 of them 24 -> 14; 32 of 4 heads of 64 x 128 14 -> 9.2.
 template <int RSPLIT>
 __global__ __launch_bounds__(64 * RSPLIT) void mlstm_step_kernel(
     const float* __restrict__ proj, int stride, int q_col, int k_col, int v_col, int i_col, int f_col,
