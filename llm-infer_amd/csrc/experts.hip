@@ -64,9 +64,10 @@ __global__ __launch_bounds__(64 * SORT_WAVES) void sort_pairs_kernel(const int* 
     if (threadIdx.x == 0) { p.counts[e] = total; p.offsets[e] = offset; }
 }
 
-// The same from dense routing weights [T, cols] (0: not chosen; the first n_experts columns): a token's pairs are its weights that
-// are not 0, at most `top`, experts ascending; weights [T, top] beside slot_of, and weight_of [P] beside row_of.  Workgroup e
-// counts the pairs of the experts before its own, a run of tokens a thread, then deals out its own.
+// The same from dense routing weights [T, cols] (0: not chosen; the first n_experts columns): a token's pairs are the first `top`
+// of its weights that are not 0, experts ascending; weights [T, top] beside slot_of, and weight_of [P] beside row_of.  Workgroup e
+// counts the pairs of the experts before its own, a run of tokens a thread, then deals out its own: what is counted is what is
+// dealt out, so there are never more than T * top pairs whatever the table holds.
 #define DENSE_THREADS 1024
 
 __global__ __launch_bounds__(DENSE_THREADS) void pairs_of_weights_kernel(const float* __restrict__ dense, int cols, int n_tokens,
@@ -79,8 +80,10 @@ __global__ __launch_bounds__(DENSE_THREADS) void pairs_of_weights_kernel(const f
     int mine = 0, before = 0;
     for (int t = lo; t < hi; ++t) {
         const float* w = dense + (int64_t)t * cols;
-        for (int i = 0; i < e; ++i) before += w[i] != 0.f;
-        mine += w[e] != 0.f;
+        int rank = 0;
+        for (int i = 0; i < e; ++i) rank += w[i] != 0.f;
+        before += min(rank, top);
+        mine += w[e] != 0.f && rank < top;
     }
     if (tid == 0) before_sum = 0;
     mine_of[tid] = mine;

@@ -2201,7 +2201,8 @@ def route_pairs(h, w_router, bias, n_experts: int, top: int, scale: float = 1.0)
 
 
 def pairs_of_weights(weights, n_experts: int, top: int) -> SortedPairs:
-    """The pairs of a dense table of routing weights (float32 [T, >= n_experts]; 0: not chosen; at most ``top`` a row are not 0).
+    """The pairs of a dense table of routing weights (float32 [T, >= n_experts]; 0: not chosen; of a row with more than ``top`` that
+    are not 0 the first ``top``).
     ``weight_of`` float32 [T * top]: the weight of every pair."""
     _dev(weights)
     _need(weights.dtype == torch.float32 and weights.dim() == 2 and weights.shape[1] >= n_experts >= 1 and top >= 1, "pairs_of_weights: float32 [T, experts]")

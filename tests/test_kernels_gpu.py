@@ -197,6 +197,27 @@ def test_pairs_of_dense_routing_weights(ops, T, E, top):
     assert p.weight_of[:len(rows), 0].tolist() == [w[t, e].item() for e in range(E) for t in range(T) if w[t, e] != 0]
 
 
+@pytest.mark.parametrize("T,E,top", [(40, 9, 2), (1024, 8, 2), (1500, 70, 4)])
+def test_pairs_of_rows_with_more_weights_than_are_chosen(ops, T, E, top):
+    """A row with more than `top` weights has the pairs of the first `top`: what is counted is what is dealt out, so no place
+    beyond T * top is named (nothing checks on the host how many weights of a row are not 0)."""
+    g = torch.Generator().manual_seed(T)
+    w = torch.rand(T, E + 1, generator=g) + 0.1
+    w[torch.rand(T, E + 1, generator=g) < 0.5] = 0.0
+    w[::7, -2] = 0.25                                                          # an expert that many rows name last
+    assert int((w[:, :E] != 0).sum(1).max()) > top
+    p = ops.pairs_of_weights(w.to(DEV), E, top)
+    kept = [(w[t, :E] != 0).nonzero().flatten()[:top].tolist() for t in range(T)]
+    pairs = [(e, t) for e in range(E) for t in range(T) if e in kept[t]]
+    counts = [sum(e in k for k in kept) for e in range(E)]
+    assert p.counts.tolist() == counts and p.offsets.tolist() == [sum(counts[:e]) for e in range(E)]
+    assert p.row_of[:len(pairs)].tolist() == [t for _, t in pairs]
+    assert p.weight_of[:len(pairs), 0].tolist() == [w[t, e].item() for e, t in pairs]
+    slot = {pair: i for i, pair in enumerate(pairs)}
+    assert p.slot_of.tolist() == [[slot[e, t] for e in kept[t]] + [-1] * (top - len(kept[t])) for t in range(T)]
+    assert p.weights.tolist() == [[w[t, e].item() for e in kept[t]] + [0.0] * (top - len(kept[t])) for t in range(T)]
+
+
 TILED_CASES = [(1, 64, 64), (3, 172, 96), (16, 40, 4096), (9, 16400, 256), (17, 100, 64), (64, 256, 512),
                (33, 4100, 2048), (48, 72, 8192), (50, 6144, 4096), (65, 48, 32), (97, 200, 14336), (30, 520, 96), (128, 16, 160),
                (70, 200, 1024), (96, 1000, 416), (128, 136, 2048), (129, 384, 320), (256, 520, 2048), (384, 512, 192), (300, 1000, 96)]
