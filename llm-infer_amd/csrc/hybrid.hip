@@ -698,7 +698,8 @@ extern "C" int li_small_logits(const void* h, int dt, const float* w, float* out
 // ---------------------------------------------------------------------------
 // The router of a mixture of experts, one wave per token.  `logits` float32 [T, n_cols]: n_route router outputs,
 // then (has_gate 1) one column whose sigmoid weighs an expert that every token uses (has_gate 2: its weight is 1).  s = softmax over the n_route
-// outputs; the `top` outputs with the largest s + correction are chosen (the first of equals); their weights are
+// outputs; the `top` outputs with the largest s + correction are chosen (the first of equals; one whose correction is -inf only
+// where fewer than `top` others are left, one whose score is no number never); their weights are
 // s / (sum of the chosen s + 1e-20) * route_scale.  The first n_real outputs are experts with matrices: their
 // weights (0 where not chosen) go to `weights` [T, n_real (+ 1)], the gate's sigmoid into the last column.  The
 // outputs behind them pass the token's input on: residual[t] += (sum of their weights) * h[t].
@@ -713,7 +714,8 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
                                                        float route_scale, int sigmoid_scores, int renorm) {
     extern __shared__ float lds[];
     float* s = lds;                      // [n_route] softmax scores
-    float* c = s + n_route;              // [n_route] choice scores, -inf once chosen
+    float* c = s + n_route;              // [n_route] choice scores
+    constexpr int none = 0x7fffffff;
     const int t = blockIdx.x, lane = threadIdx.x;
     const float* z = logits + (int64_t)t * n_cols;
     float mx = -INFINITY;
@@ -734,23 +736,23 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
     for (int i = lane; i < wcols; i += 64) weights[(int64_t)t * wcols + i] = 0.f;
     __syncthreads();
     float chosen_sum = 0.f;
+    uint64_t taken = 0;                  // bit j: this lane's output lane + 64 j is chosen
     for (int k = 0; k < top; ++k) {
-        float best = -INFINITY; int bi = 0x7fffffff;
-        for (int i = lane; i < n_route; i += 64) if (c[i] > best) { best = c[i]; bi = i; }
+        float best = -INFINITY; int bi = none;
+        for (int i = lane, j = 0; i < n_route; i += 64, ++j)
+            if (!(taken >> j & 1) && (c[i] > best || (bi == none && c[i] == c[i]))) { best = c[i]; bi = i; }
         for (int o = 32; o > 0; o >>= 1) {
             const float ob = __shfl_xor(best, o, WAVE); const int oi = __shfl_xor(bi, o, WAVE);
-            if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
+            if (oi != none && (bi == none || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
         }
+        if (bi == none) break;           // (what is left is no number; the same for every lane)
         chosen_sum += s[bi];
-        __syncthreads();
-        if (lane == 0) c[bi] = -INFINITY;
-        __syncthreads();
+        if ((bi & 63) == lane) taken |= 1ull << (bi >> 6);
     }
     const float f = renorm ? route_scale / (chosen_sum + 1e-20f) : route_scale;
     float pass = 0.f;                    // the weight of the outputs that pass the input on
-    // every lane knows the chosen set through c == -inf
-    for (int i = lane; i < n_route; i += 64) {
-        if (c[i] == -INFINITY) {
+    for (int i = lane, j = 0; i < n_route; i += 64, ++j) {
+        if (taken >> j & 1) {
             const float w = s[i] * f;
             if (i < n_real) weights[(int64_t)t * wcols + i] = w; else pass += w;
         }

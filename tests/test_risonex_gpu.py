@@ -310,6 +310,61 @@ def test_router_choice_weights_and_identity(lib, dtype, n_real, n_identity, top)
         assert not torch.equal(chosen.sort(-1).values, without.sort(-1).values)
 
 
+def test_router_leaves_out_masked_outputs(lib):
+    """An output whose correction is -inf is not chosen while others are left, and has no weight then; where fewer than `top`
+    are left the first of the masked ones follow.  A score that is no number is never chosen."""
+    from llm_infer_amd.kernels import ops
+    inf = float("inf")
+    g = torch.Generator().manual_seed(5)
+    for n, top, masked in ((8, 2, [3]), (8, 2, [0, 7]), (130, 4, list(range(0, 130, 2))), (5, 3, [0, 1, 4]), (4096, 3, [0, 4095]), (3, 1, [0, 1, 2])):
+        T = 9
+        logits = torch.stack([torch.randperm(n, generator=g).float() * (3.0 / n) for _ in range(T)])
+        correction = torch.zeros(n)
+        correction[masked] = -inf
+        res = torch.zeros(T, 32, device=DEV)
+        w = ops.moe_route(logits.to(DEV), correction.to(DEV), torch.zeros(T, 32, device=DEV), res, n, n, top, 0, 1.0).cpu().double()
+        s = torch.softmax(logits.double(), -1)
+        order = [sorted(range(n), key=lambda i: (i in masked, 0.0 if i in masked else -s[t, i].item(), i))[:top] for t in range(T)]
+        ref = torch.zeros(T, n, dtype=torch.float64)
+        for t, chosen in enumerate(order):
+            ref[t, chosen] = s[t, chosen] / (s[t, chosen].sum() + 1e-20)
+        assert torch.equal(w != 0, ref != 0) and (w - ref).abs().max() < 1e-5, (n, top)
+    correction = torch.tensor([0.0, float("nan"), 0.5, 0.0])
+    w = ops.moe_route(torch.zeros(2, 4, device=DEV), correction.to(DEV), torch.zeros(2, 32, device=DEV), torch.zeros(2, 32, device=DEV), 4, 4, 4, 0, 1.0).cpu()
+    assert (w[:, [0, 2, 3]] - 1 / 3).abs().max() < 1e-5 and (w[:, 1] == 0).all()
+
+
+@pytest.mark.parametrize("ff", [48, 64])
+def test_experts_of_a_long_prompt_with_a_masked_one(lib, ff):
+    """A file that takes an expert out by a correction of -inf: every token through every expert, and sorted by expert (products
+    by pairs with 64 columns an expert, one expert after another with 48), give what the plain implementation gives."""
+    width, mlp = 96, M.moe(4, 2, ff, scale=1.3)
+    cfg = one_layer(M.mamba(2, 8, 8), mlp, width=width)
+    g = torch.Generator().manual_seed(18)
+    W = M.mlp_weights(mlp, width, g, torch.bfloat16)
+    W["router"] = torch.zeros(4, width, dtype=torch.bfloat16)
+    W["router"][torch.arange(4), torch.arange(4)] = 2.0
+    W["correction"] = torch.tensor([0.0, 0.0, float("-inf"), 0.0], dtype=torch.bfloat16)
+    part = build_part("feed_forward", cfg._feed_forward("", mlp), W, "bfloat16")
+    assert (part.pair_weights is not None) == (ff == 64)
+    T = 300
+    h = 0.3 * torch.randn(T, width, generator=g)
+    live = torch.tensor([0, 1, 3])
+    order = torch.stack([torch.randperm(3, generator=g) for _ in range(T)])
+    h[torch.arange(T), live[order[:, 0]]] += 3.0
+    h[torch.arange(T), live[order[:, 1]]] += 1.5
+    h[:, 2] += 4.0                                       # the masked expert would be every token's first
+    h = h.bfloat16()
+    chosen, _ = P.route(h.double(), M.widen(W), mlp["router"])
+    assert torch.equal(chosen.sort(-1).values, live[order[:, :2]].sort(-1).values)
+    ref = P.moe_ff(h.double(), M.widen(W), mlp)
+    for limit in (1, 10 ** 9):
+        part.GROUPED_FROM = limit
+        res = torch.zeros(T, width, device=DEV)
+        part.forward(h.to(DEV), res)
+        assert error(res.cpu(), ref) < TOL["bfloat16"], limit
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("mlp", [M.moe(5, 3, 40, identity=1, scale=2.0, shared=24), M.moe(3, 1, 56), M.moe(66, 4, 8, identity=4, shared=16),
                                  M.dense(72)])
