@@ -2209,7 +2209,7 @@ def pairs_of_weights(weights, n_experts: int, top: int) -> SortedPairs:
     t = weights.shape[0]
     p = SortedPairs(t, top, n_experts, weights.device)
     p.weight_of = torch.empty((t * top, 1), dtype=torch.float32, device=weights.device)
-    _check(experts().li_pairs_of_weights(_ptr(weights), weights.shape[1], t, top, n_experts, _ptr(p.counts), _ptr(p.offsets), _ptr(p.row_of),
+    _check(experts().li_pairs_of_weights(_ptr(weights), weights.shape[1], t, top, n_experts, _ptr(p.chosen), _ptr(p.counts), _ptr(p.offsets), _ptr(p.row_of),
                                          _ptr(p.slot_of), _ptr(p.weights), _ptr(p.weight_of), _stream()), "pairs_of_weights")
     return p
 

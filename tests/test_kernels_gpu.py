@@ -197,7 +197,7 @@ def test_pairs_of_dense_routing_weights(ops, T, E, top):
     assert p.weight_of[:len(rows), 0].tolist() == [w[t, e].item() for e in range(E) for t in range(T) if w[t, e] != 0]
 
 
-@pytest.mark.parametrize("T,E,top", [(40, 9, 2), (1024, 8, 2), (1500, 70, 4)])
+@pytest.mark.parametrize("T,E,top", [(40, 9, 2), (1024, 8, 2), (1500, 70, 4), (77, 20, 3), (33, 32, 1), (300, 64, 5), (130, 65, 2), (7, 5, 1)])
 def test_pairs_of_rows_with_more_weights_than_are_chosen(ops, T, E, top):
     """A row with more than `top` weights has the pairs of the first `top`: what is counted is what is dealt out, so no place
     beyond T * top is named (nothing checks on the host how many weights of a row are not 0)."""
