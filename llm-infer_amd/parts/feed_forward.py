@@ -192,14 +192,19 @@ class RoutedExperts(Part):
     routing weights on the device.  Many tokens in a 16-bit model (``GROUPED_FROM / 2`` rows an expert on average): the pairs of
     token and chosen expert are sorted by expert on the device and every expert multiplies its own pairs' rows, all experts in one
     launch a product; a token's results are added into its residual row expert by expert (a fixed order).  Matrices that do
-    not tile, or steps too long for the pairs' buffers (``_pairs_hold``), from ``GROUPED_FROM`` rows on: the host reads the
-    counts, and every expert runs products of its own."""
+    not tile, from ``GROUPED_FROM`` rows on: the host reads the counts, and every expert runs products of its own."""
 
-    # measured (eight experts, two chosen, ms a prompt with every token through every expert, and by pairs): Risonex 4,096 wide
-    # 256 tokens 2.20 and 2.22, 512 3.00 and 2.84, 1,500 7.19 and 5.52; Favizen 256 1.61 and 1.56, 1,500 5.07 and 3.90; Dupolorn
-    # 2,048 wide 512 1.88 and 1.90, 1,500 3.37 and 3.07.  With the counts read by the host (40 launches a layer) it pays from twice as
-    # many rows on (Risonex 1,024 tokens 4.90 and 4.86)
+    # measured, GPU us of the products with every token through every expert and by pairs, at 128 and 256 rows an expert: 8
+    # experts, 2 chosen, gated 3,584 of width 4,096 373 and 225, 625 and 331; gated 512 of 1,024 46 and 44, 63 and 47; without a
+    # gate 1,024 of 2,048 67 and 62, 101 and 71; 32 experts of 768, 4 chosen 347 and 140; 64 of 512, 6 chosen 580 and 183; 4 of 4,096,
+    # 1 chosen 128 and 88.  With the counts read by the host (40 launches a layer) it pays from twice as many rows on (Risonex
+    # 1,024 tokens 4.90 and 4.86 ms a prompt)
     GROUPED_FROM = 256
+    # The pairs' rows of one portion of a prompt hold at most this many float32 numbers (512 MiB; without a gate the up product's sums as
+    # many again): a prompt's working memory ends there instead of growing with its pairs, which are `top` times its tokens.
+    # Measured, ms and peak MiB in one portion, at 2^27 and at 2^25: 65,536 tokens, 8 experts of 3,584, width 4,096 10.5 and 2,947, 10.6
+    # and 737, 11.9 and 184; 32,768 tokens, 128 experts of 768, 8 chosen, width 2,048 3.7 and 2,438, 4.1 and 609, 6.7 and 152
+    PAIR_NUMBERS = 1 << 27
     makes_rows = False          # by pairs: forward_rows hands over the rows as a sum (set when the weights are bound)
     writes_rows = True          # forward_into overwrites the rows it is handed
 
@@ -375,25 +380,30 @@ class RoutedExperts(Part):
 
     def _by_pairs(self, h, residual, weights):
         """Every expert's products on its own tokens' rows, all experts in one launch each and nothing read back: the pairs of
-        the dense weights, sorted by expert on the device."""
+        the dense weights, sorted by expert on the device.  A long prompt in portions of its tokens (``PAIR_NUMBERS``)."""
         w_up, w_down = self.pair_weights
-        p = ops.pairs_of_weights(weights, self.n_experts, self.top)
-        if not self.gated:
-            z = ops.linear_pairs(h, w_up, p, out_dtype=torch.float32)
-            t = ops.expert_act(z, p.weight_of, 1, self.expert_ff, 0, self.activation, self.on_input, self.dtype, None, 0)
-        elif self.clamped:
-            t = ops.linear_pairs(h, w_up, p, ops.EPI_CLAMPGLU, params=ops.glu_params(None, self.limit, None, self.alpha, self.up_shift))
-        else:
-            t = ops.linear_pairs(h, w_up, p, ops.EPI_SWIGLU)
-        rows = ops.linear_pairs(t, w_down, p, gather=False, out_dtype=torch.float32)
-        # (experts without a gate have their weight in the hidden row)
-        ops.PairSum(rows, p.slot_of, p.weights if self.gated else torch.ones_like(p.weights)).add_to(residual)
+        most = max(1, self.PAIR_NUMBERS // (self.top * max(self.hidden_size, self.expert_ff)))
+        n = -(-h.shape[0] // most)
+        step = -(-h.shape[0] // n)
+        for t0 in range(0, h.shape[0], step):
+            rows_in = h[t0:t0 + step]
+            p = ops.pairs_of_weights(weights[t0:t0 + step], self.n_experts, self.top)
+            if not self.gated:
+                z = ops.linear_pairs(rows_in, w_up, p, out_dtype=torch.float32)
+                t = ops.expert_act(z, p.weight_of, 1, self.expert_ff, 0, self.activation, self.on_input, self.dtype, None, 0)
+                del z
+            elif self.clamped:
+                t = ops.linear_pairs(rows_in, w_up, p, ops.EPI_CLAMPGLU, params=ops.glu_params(None, self.limit, None, self.alpha, self.up_shift))
+            else:
+                t = ops.linear_pairs(rows_in, w_up, p, ops.EPI_SWIGLU)
+            rows = ops.linear_pairs(t, w_down, p, gather=False, out_dtype=torch.float32)
+            # (experts without a gate have their weight in the hidden row)
+            ops.PairSum(rows, p.slot_of, p.weights if self.gated else torch.ones_like(p.weights)).add_to(residual[t0:t0 + step])
+            del p, t, rows                      # (the next portion's take their place)
 
     def _pairs_hold(self, h) -> bool:
-        """True where the pairs' products take the step: rows below 4 GiB, and 4 GiB of float32 results at most."""
-        pairs, e = h.shape[0] * self.top, h.element_size()
-        return (self.pair_weights is not None and h.is_contiguous() and h.data_ptr() % 16 == 0 and h.numel() * e < (1 << 32)
-                and pairs * self.expert_ff * e < (1 << 32) and pairs * max(self.hidden_size, 0 if self.gated else self.expert_ff) <= (1 << 30))
+        """True where the pairs' products take the step's rows."""
+        return self.pair_weights is not None and h.is_contiguous() and h.data_ptr() % 16 == 0
 
     def _grouped(self, h, residual, weights):
         if self._pairs_hold(h):
