@@ -16,7 +16,7 @@ import torch
 
 from ..kernels import ops
 from ..tensor import Tensor
-from .step import StepShared, decode_splits, page_splits, split_bucket
+from .step import StepShared, decode_splits, page_shares, page_splits, split_bucket
 
 
 @contextlib.contextmanager
@@ -69,6 +69,9 @@ class _GraphContext(StepShared):
 
     def page_splits(self, n_kv_heads, n_heads):
         return page_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket)
+
+    def page_shares(self, n_kv_heads, n_heads):
+        return page_shares(self.n_seqs, n_kv_heads, n_heads, self._bucket)
 
 
 MAX_RECORDED_STEPS = 48        # recorded steps an engine keeps; the least recently used goes first

@@ -75,6 +75,10 @@ class StepContext(StepShared):
         """The same for the kernel whose waves merge inside a workgroup, where a page a split is worth it."""
         return page_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
 
+    def page_shares(self, n_kv_heads: int, n_heads: int) -> int:
+        """The same for the kernels in which a split is a workgroup of four waves."""
+        return page_shares(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
+
 
 def split_bucket(max_ctx: int) -> int:
     """The most splits that a context of this length is worth (a power of two up to 64): at least two
@@ -97,10 +101,19 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
 
 
 def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
-    """Splits for the decode kernels of softmax, differential and latent attention: as ``decode_splits``, but down to one page a
+    """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one page a
     split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64."""
-    # measured on MI355X (heads of 128, 8 KV heads; us with half as many splits and with these): batch 1 at 180 tokens 8.8
-    # and 6.8, at 400 9.5 and 7.5, at 900 11.0 and 9.6, at 1,500 12.6 and 11.4, at 2,048 10.8 and 10.0; batch 8 at 300 9.7
-    # and 8.6, at 900 13.7 and 12.9; batch 16 at 900 20.7 and 20.2; batch 4 at 2,048 the same.  Latents of 256 / 192 (16 heads, batch 8)
-    # at 300 13.4 and 11.3, at 1,000 14.9 and 12.5; two maps of 64 with values of 128 (32 / 8 heads, batch 4) at 500 17.6 and 14.3
+    # measured on MI355X (heads of 128, 8 KV heads; us with half as many splits and with these): batch 1 at 40 tokens 6.2 and 6.1,
+    # at 100 7.5 and 6.3, at 180 8.8 and 6.8, at 400 9.5 and 7.5, at 900 11.0 and 9.6, at 1,500 12.6 and 11.4, at 2,048 10.8
+    # and 10.0; batch 8 at 300 9.7 and 8.6, at 900 13.7 and 12.9; batch 16 at 900 20.7 and 20.2; batch 4 at 2,048 the same
     return decode_splits(n_seqs, n_kv_heads, n_heads, min(2 * bucket, 64))
+
+
+def page_shares(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
+    """Shares of a token's keys for the decode kernels of differential and latent attention, whose share is a workgroup of four
+    waves that merge inside it: as ``page_splits``, but one for the shortest contexts, whose waves have a page at most each."""
+    # measured on MI355X, us: latents of 256 / 192 (16 heads, batch 8) at 64 keys 9.6 in one share (10.7 in two, with the kernel that
+    # merges them), at 128 10.2 (11.4), at 192 12.2 (11.3); with half as many shares and with these 13.4 and 11.3 at 300, 14.9 and 12.5 at
+    # 1,000.  Two maps of 64 with values of 128 (32 / 8 heads, batch 4) at 64 9.9 (12.9), at 128 10.6 (13.6), at 192 13.9 (12.7);
+    # 17.6 and 14.3 at 500
+    return 1 if bucket == 1 else page_splits(n_seqs, n_kv_heads, n_heads, bucket)

@@ -98,7 +98,7 @@ class DifferentialAttention(Part):
         """Workgroups that share a token's keys in a decode step of a 16-bit model (a block bounds what a token sees)."""
         if self.dtype == torch.float32 or not ctx.is_decode:
             return 1
-        shares = ctx.page_splits(self.n_kv_heads, self.n_heads)
+        shares = ctx.page_shares(self.n_kv_heads, self.n_heads)
         if self.block:
             shares = min(shares, max(1, self.block // 128))
         return shares

@@ -246,6 +246,19 @@ def test_decode_splits_fill_the_chip_and_are_powers_of_two():
             assert s & (s - 1) == 0 and 1 <= s <= max(1, pages // 2)
 
 
+def test_splits_down_to_one_page():
+    """The softmax decoder's splits go down to a page each; where a split is a whole workgroup the shortest contexts are not cut."""
+    from llm_infer_amd.engine.step import page_shares, page_splits
+    for ctx in range(1, 9000, 37):
+        pages, bucket = (ctx + 63) // 64, split_bucket(ctx)
+        for n, k, h in ((1, 8, 32), (3, 1, 4), (8, 2, 2), (64, 8, 32), (8, 1, 16)):
+            s = page_splits(n, k, h, bucket)
+            assert s & (s - 1) == 0 and 1 <= s <= min(64, max(2, pages))
+            assert decode_splits(n, k, h, bucket) <= s <= 2 * decode_splits(n, k, h, bucket)
+            assert page_shares(n, k, h, bucket) == (1 if ctx <= 192 else s)
+    assert page_splits(1, 8, 32, 64) == 64 and page_shares(1, 8, 32, 64) == 64
+
+
 def test_the_prefill_product_plan():
     """What the planner of the prefill product hands the kernel: a tile it has, K split only where a split
     keeps at least 1,024 of K, few rows of X split (the chip has 256 CUs to fill), many rows not."""
