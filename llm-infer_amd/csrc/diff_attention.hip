@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
     }
     if (sink) {
         // the sink joins every map's sum as one more weight, exp(sink - maximum), with nothing to add to the output
-        const float s2 = sink[hq] * 1.4426950408889634f;
+        const float s2 = sink[h] * 1.4426950408889634f;
 #pragma unroll
         for (int a = 0; a < MAPS; ++a) {
             const float M = fmaxf(m[a], s2), f = __builtin_amdgcn_exp2f(m[a] - M);
@@ -369,17 +369,17 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
         }
     ss += __shfl_xor(ss, 32, WAVE);
     float rr = out_eps >= 0.f ? out_scale / sqrtf(ss / (float)dv + out_eps) : out_scale;
-    const float* grow = gate ? gate + (int64_t)(t0 + (HC || !has_query ? 0 : col)) * gate_stride + gate_col : nullptr;
+    const float* grow = gate ? gate + (int64_t)(t0 + (has_query ? col : 0)) * gate_stride + gate_col : nullptr;
     if (gate && !gate_elem && has_query)             // one number a (token, head)
-        rr *= 1.f / (1.f + expf(-grow[hq]));
+        rr *= 1.f / (1.f + expf(-grow[h]));
     if (has_query) {
-        T* orow = out + ((int64_t)(t0 + (HC ? 0 : col)) * H + hq) * dv;
+        T* orow = out + ((int64_t)(t0 + col) * H + h) * dv;
 #pragma unroll
         for (int b = 0; b < DVB; ++b)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int dim = b * 32 + 8 * (r >> 2) + 4 * half + (r & 3);
-                if (dim < dv) orow[dim] = from_f32<T>(o[0][b][r] * rr * (gate_elem ? 1.f / (1.f + expf(-grow[hq * dv + dim])) : 1.f));
+                if (dim < dv) orow[dim] = from_f32<T>(o[0][b][r] * rr * (gate_elem ? 1.f / (1.f + expf(-grow[h * dv + dim])) : 1.f));
             }
     }
     }      // the item's tiles
@@ -457,14 +457,17 @@ extern "C" int li_diffattn(const void* q, void* out, int dt, const void* k_pages
     const int split = tile_t0 ? 0 : 1, per_kv = H / G;
     const int heads = split ? 1 : (per_kv % 4 == 0 ? 4 : (per_kv % 2 == 0 ? 2 : 1));
     // a decode step with four or more query heads on a key/value head: the heads are a tile's columns
-    // (where the 32 columns' states of four waves fit into the 160 KiB of LDS: two maps of wide values do not)
-    const bool hc = split && per_kv >= 4 && (size_t)4 * maps * 32 * (2 + VALUE_DIM) * sizeof(float) <= 150 * 1024;
+    // (where the states of the columns that there are, of four waves, fit into the 160 KiB of LDS: two maps of 160 values do for
+    // up to 28 heads, of 256 for up to 18).  `states`: bytes of `columns` of them.  Maps of 16 with values of 160, 32 / 4 heads, batch 4:
+    // at 100 keys 11.8 us (a workgroup a head 10.6), at 300 in four shares 14.4 (18.5), at 1,000 in eight 15.6 (39.2)
+    auto states = [&](int columns) { return (size_t)4 * maps * columns * (VALUE_DIM + 4 + 2) * sizeof(float); };
+    const bool hc = split && per_kv >= 4 && states(per_kv < 32 ? per_kv : 32) <= 150 * 1024;
     // (then `key_shares` workgroups share a token's keys and leave their states in `part`, float32 [tokens, H, shares,
     // maps, 2 + VALUE_DIM], for a second kernel)
     const int shares = hc && key_shares > 1 && part ? key_shares : 1;
     dim3 grid(n_tiles, hc ? G * ((per_kv + 31) / 32) : H / heads, shares);
     const int threads = split ? 256 : 64 * heads;
-    const size_t lds = split ? (size_t)4 * maps * (hc ? (per_kv < 32 ? per_kv : 32) : 1) * (VALUE_DIM + 4 + 2) * sizeof(float) : 0;
+    const size_t lds = split ? states(hc ? (per_kv < 32 ? per_kv : 32) : 1) : 0;
 #define GO1(T, M, P, C)                                                                                                              \
     do {                                                                                                                             \
         auto kfn = diff_attn_mfma_kernel<T, M, P, C>;                                                                                \

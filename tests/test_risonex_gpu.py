@@ -190,6 +190,25 @@ def test_differential_attention_part(lib, dtype, H, G, d, dv, block, schedule):
     assert all(g_.pool.n_free == g_.n_pages - 1 for g_ in cache.groups)         # every page came back
 
 
+# two maps of values of 160: the states of so many heads of one token fit into LDS together (28 of 160 values), one more do not
+@pytest.mark.parametrize("H, G, dv", [(8, 2, 150), (28, 1, 160), (29, 1, 160)])
+def test_differential_attention_of_wide_values_and_many_heads(lib, H, G, dv):
+    width, eps, dtype = 96, 1e-5, "bfloat16"
+    mixer = M.attention(H, G, 16, dv, 4096, diff=0.3)
+    cfg = one_layer(mixer, width=width, eps=eps)
+    g = torch.Generator().manual_seed(H)
+    W = M.mixer_weights("attention", mixer[1], width, g, torch.bfloat16, sharp=2.0)
+    part = build_part("mixer", cfg._mixer("", cfg.layers[0]), W, dtype)
+    n = {"a": 203, "b": 30}                     # decoded with one share of the keys and, from 193 to 203, with several
+    h_of = {r: torch.randn(k, width, generator=g).to(DT[dtype]).float() for r, k in n.items()}
+    got, _ = run_mixer(part, h_of, [{"a": 190, "b": 27}] + [{"a": 1, "b": 1}] * 3 + [{"a": 1}] * 10, dtype)
+    for r in n:
+        ref = P.diff_attention(h_of[r].double(), M.widen(W), mixer[1], eps)
+        tol = max(TOL[dtype], 3 * error(P.diff_attention(h_of[r].double(), M.widen(W), mixer[1], eps, store=torch.bfloat16), ref))
+        assert error(got[r], ref) < tol, r
+        assert error(got[r][-3:], ref[-3:]) < 2 * tol, r         # the decoded ones by themselves
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_attention_sees_its_block_and_nothing_before_it(lib, dtype):
     """Keys made to stand out: the first map of a query looks for the first key of its own block (just inside),
