@@ -270,13 +270,16 @@ def _workspace(n_floats: int, device) -> torch.Tensor:
 EXPERTS_IN_K, EXPERTS_IN_N, EXPERTS_GATED = 1, 2, 3
 
 
-def experts_fit(x, w, n_experts: int, top: int, ff: int, gated: bool) -> bool:
+def experts_fit(x, w, n_experts: int, top: int, ff: int, gated: bool, n_outputs: int | None = None) -> bool:
     """True if the products of experts side by side should leave out those that no token chose (``linear``'s ``experts``): few
-    rows against a tiled weight, of which a quarter of the experts is likely to go unread.  Measured with eight experts and
-    two chosen: 4 tokens 22.1 against 24.3 ms (Risonex, width 4,096, 17 steps behind a prompt), 8 tokens, which leave
-    one expert in ten, 14.9 against 14.7 (Dupolorn, width 2,048)."""
-    rows = x.shape[0]
-    return (is_tiled(w) and x.dtype == w.dtype and rows <= 8 and (1.0 - top / n_experts) ** rows >= 0.25 and n_experts + 1 <= 64
+    rows against a tiled weight, of which a quarter of the experts is likely to go unread when every token chooses ``top`` of
+    ``n_outputs`` outputs (default: the experts; a router may have more, that pass a token on)."""
+    # measured, us of the three or four products with all experts read and with those left out, at 1, 4 and 8 rows: 8 gated of
+    # 3,584, 2 chosen, width 4,096 127 and 35, 122 and 81, 126 and 126; 8 without a gate of 1,024, width 2,048 19.5 and 12.5, 20.3 and
+    # 18.7, 21.3 and 24.1; 4 gated of 2,048, 1 chosen 24 and 12, 24 and 17; 32 of 768, 4 chosen 63 and 18, 60 and 32, 67 and 42; 60
+    # of 512, 6 chosen 81 and 20, 79 and 28, 86 and 40
+    rows, unread = x.shape[0], max(0.0, 1.0 - top / (n_outputs or n_experts))
+    return (is_tiled(w) and x.dtype == w.dtype and rows <= 8 and unread ** rows >= 0.25 and n_experts + 1 <= 64
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and (not gated or ff % 2 == 0))
 
 

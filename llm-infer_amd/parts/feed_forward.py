@@ -445,7 +445,7 @@ class RoutedExperts(Part):
         them with the epilogue ``mode`` into ``out``.  For few tokens the experts that none of them chose are not read (their
         hidden values are zeros either way)."""
         n, f, tail = self.n_experts, self.expert_ff, self.shared_ff
-        few = n > 0 and ops.experts_fit(h, self.w_gate_up, n, self.top, f, self.gated) and ops.is_tiled(self.w_down)
+        few = n > 0 and ops.experts_fit(h, self.w_gate_up, n, self.top, f, self.gated, n + self.n_identity) and ops.is_tiled(self.w_down)
         over = (weights, n, f, ops.EXPERTS_GATED if self.gated else ops.EXPERTS_IN_N) if few else None
         if not self.gated:
             t = self._hidden(h, self.w_gate_up, weights, None, None, n, f, tail, over)

@@ -177,6 +177,17 @@ def test_products_of_chosen_experts(ops, M, n, ff, tail, dt):
             assert (out.double() - ref).abs().max().item() < bound, mode
 
 
+def test_when_unchosen_experts_are_left_out(ops):
+    """By the share of experts that is likely to go unread: of all the router's outputs, those that pass a token on among them."""
+    w = ops.tile_weight(torch.zeros(64, 32, dtype=torch.bfloat16, device=DEV))
+    x = torch.zeros(9, 32, dtype=torch.bfloat16, device=DEV)
+    fit = lambda rows, n, top, outputs=None: ops.experts_fit(x[:rows], w, n, top, 16, True, outputs)
+    assert fit(4, 8, 2) and not fit(5, 8, 2) and fit(8, 60, 6) and not fit(9, 60, 6) and not fit(1, 64, 2)
+    assert not fit(2, 4, 4) and not fit(1, 1, 1)
+    assert fit(2, 2, 2, 4) and not fit(3, 2, 2, 4) and not fit(2, 2, 4, 4)      # two experts and two outputs that pass a token on
+    assert not fit(2, 2, 5, 6) and not fit(4, 1, 3, 4)                          # (more are chosen than there are experts)
+
+
 @pytest.mark.parametrize("T,E,top", [(1, 1, 1), (3, 8, 2), (1023, 5, 3), (1024, 8, 2), (1025, 3, 3), (2500, 70, 4)])
 def test_pairs_of_dense_routing_weights(ops, T, E, top):
     g = torch.Generator().manual_seed(T + E)
