@@ -392,6 +392,7 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
                 kind = f"rows:{nt}"
         if force is None and kind != "fma" and not kind.startswith("rows") and m * k * 2 < (1 << 32):
             kind = "wreg"
+    _need(experts is None, "experts: at most 16 rows of X (8 with an activation) against a tiled weight")
     if kind.startswith("rows"):                                # "rows[:<tiles of W a workgroup>]" (a test's choice)
         _need(tiled and fast_ok and m <= 128, "gemm_rows: a tiled weight, at most 128 rows of X")
         parts = kind.split(":")

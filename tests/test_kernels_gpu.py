@@ -177,6 +177,15 @@ def test_products_of_chosen_experts(ops, M, n, ff, tail, dt):
             assert (out.double() - ref).abs().max().item() < bound, mode
 
 
+def test_experts_are_refused_where_no_kernel_takes_them(ops):
+    """Not run as if every expert were chosen (which would leave the weights out)."""
+    w = torch.zeros(64, 32, dtype=torch.bfloat16, device=DEV)
+    x = torch.zeros(40, 32, dtype=torch.bfloat16, device=DEV)
+    for rows, wt, mode, over in ((40, ops.tile_weight(w), 0, ops.EXPERTS_IN_N), (40, ops.tile_weight(w), 2, ops.EXPERTS_GATED), (2, w, 0, ops.EXPERTS_IN_N)):
+        with pytest.raises(ops.KernelError):
+            ops.linear(x[:rows], wt, mode, experts=(torch.ones(rows, 2, device=DEV), 2, 16 if over == ops.EXPERTS_GATED else 32, over))
+
+
 def test_when_unchosen_experts_are_left_out(ops):
     """By the share of experts that is likely to go unread: of all the router's outputs, those that pass a token on among them."""
     w = ops.tile_weight(torch.zeros(64, 32, dtype=torch.bfloat16, device=DEV))
