@@ -16,6 +16,7 @@
 #include "gemm_common.h"
 
 #define CHAIN 256                       // consecutive k of one chain of multiply-adds (as in gemm_fma)
+#define F32_TILES ((1 << 24) - 8)       // tiles of gemm_f32's grid, in one dimension: a launch has fewer than 2^32 threads in each
 
 __device__ __forceinline__ f32x4 mfma16_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -270,7 +271,7 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
     }
     const int tiles_m = (M + 63) / 64;
     const int64_t tiles = (int64_t)tiles_m * ((N + 63) / 64);
-    if (tiles > (1 << 30)) return LI_UNSUPPORTED;
+    if (tiles > F32_TILES) return LI_UNSUPPORTED;
     gemm_f32_kernel<<<(int)((tiles + 7) / 8 * 8), 256, 0, stream>>>(X, W, K, tiles_m, (int)tiles, e);
     LI_CHECK_LAUNCH();
     return LI_OK;

@@ -267,6 +267,12 @@ def _workspace(n_floats: int, device) -> torch.Tensor:
     return ws
 
 
+def f32_fits(m: int, n: int, k: int) -> bool:
+    """True for the sizes of a float32 product that gemm_f32's kernels take: steps of 16 k, and tiles of 64 x 64 that one dimension
+    of a grid holds (all others run gemm_fma, whose grid has two)."""
+    return k % 16 == 0 and ((m + 63) // 64) * ((n + 63) // 64) <= (1 << 24) - 8
+
+
 EXPERTS_IN_K, EXPERTS_IN_N, EXPERTS_GATED = 1, 2, 3
 
 
@@ -331,7 +337,7 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
     fast_ok = same16 and k % 8 == 0 and x.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0
     # float32 by float32 on the matrix cores, bit for bit what gemm_fma gives (which takes what these do not: any K, any
     # address)
-    f32_ok = x.dtype == w.dtype == torch.float32 and k % 16 == 0 and x.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0
+    f32_ok = x.dtype == w.dtype == torch.float32 and f32_fits(m, n, k) and x.data_ptr() % 16 == 0 and wd.data_ptr() % 16 == 0
     kind = force or ("f32" if f32_ok else "fma" if not fast_ok else ("gemv_mfma" if m <= 16 else ("big" if m > 32 else "mfma")))
     if tiled:
         _need(fast_ok and kind != "fma", "a tiled weight needs 16-bit activations of its dtype")

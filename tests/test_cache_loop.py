@@ -259,6 +259,22 @@ def test_splits_down_to_one_page():
     assert page_splits(1, 8, 32, 64) == 64 and page_shares(1, 8, 32, 64) == 64
 
 
+def test_sizes_of_float32_products():
+    """The rule by which a product goes to the matrix cores is the one by which the library refuses it (before anything runs)."""
+    from ctypes import c_void_p
+
+    from llm_infer_amd.kernels import build, ops
+    lib, at = build.f32_library(), c_void_p(4096)
+    none = c_void_p(0)
+    big = 1 << 18                                                   # 2^12 tiles a side: 2^24
+    for m, n, k in ((big, big, 16), (big, big - 64, 16), (1 << 20, 1 << 20, 32), (big, 64, 40)):
+        takes = ops.f32_fits(m, n, k)
+        assert takes == (m == big and n == big - 64)
+        if not takes:
+            assert lib.li_gemm_f32(at, at, at, 0, 0, m, n, k, 2, none, none) == 2
+    assert ops.f32_fits(1, 1, 16) and ops.f32_fits(1 << 20, 128256, 4096) is False and ops.f32_fits(1 << 18, 128256, 4096)
+
+
 def test_the_prefill_product_plan():
     """What the planner of the prefill product hands the kernel: a tile it has, K split only where a split
     keeps at least 1,024 of K, few rows of X split (the chip has 256 CUs to fill), many rows not."""
