@@ -307,6 +307,7 @@ struct XGroups {
 // quarter of them, four tokens two thirds (4,096 wide, experts of 3,584, a step of four tokens 0.91 -> 0.79 ms).
 enum { EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
 struct ExpertBlocks {
+    static constexpr bool chosen_only = true;
     const float* w;
     int cols, n, ff, over;
 };
@@ -341,13 +342,15 @@ __device__ __forceinline__ void store_weighted(const Epilogue& e, const ExpertBl
 
 // EB: ExpertBlocks, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
 // cost a whole matrix's product some 0.3 us, 1% of a decode step.)
-struct NoExperts {};
+struct NoExperts {
+    static constexpr bool chosen_only = false;
+};
 
 template <class T, int NT, int MT, int KW, class EB>
 __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
                                                              int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg,
                                                              EB ex) {
-    constexpr bool EXPERTS = sizeof(EB) == sizeof(ExpertBlocks);
+    constexpr bool EXPERTS = EB::chosen_only;
     if (xg.rows) X += min((int)blockIdx.x * NT * 16 / xg.rows, xg.n - 1) * xg.stride;
     // NT tiles of 16 rows of W and MT tiles of 16 rows of X per wave; W comes from HBM once, the
     // rows of X from the caches (they are few)
@@ -882,7 +885,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     do {                                                  \
         if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
         else if (mt == 1 && nt == 2) PICK_KW(T, 2, 1);    \
-        else if constexpr (sizeof(EB) != sizeof(ExpertBlocks)) { \
+        else if constexpr (!EB::chosen_only) { \
             if (mt == 2 && nt == 1) PICK_KW(T, 1, 2);     \
             else if (mt == 2 && nt == 2) PICK_KW(T, 2, 2); \
             else if (mt <= 4 && nt == 2) PICK_KW(T, 2, 4); \
