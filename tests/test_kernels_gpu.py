@@ -136,6 +136,23 @@ def test_float32_products_on_the_matrix_cores_are_bit_equal(ops, M, N, K):
         assert torch.equal(ops.linear(x, off), ops.linear(x, w))
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 33, 48), (17, 257, 528), (100, 200, 2064), (129, 130, 304)])
+def test_float32_products_of_subnormal_numbers_are_bit_equal(ops, M, N, K):
+    """Operands, products and sums below 2^-126: no kernel takes them for zeros."""
+    g = torch.Generator().manual_seed(M + K)
+    tiny = 2.0 ** -126
+    for sx, sw in ((2.0 ** -70, 2.0 ** -70), (tiny / 64, 1.0), (1.0, tiny / 1024), (2.0 ** -60, 2.0 ** -66)):
+        x, w = (torch.randn(M, K, generator=g) * sx).to(DEV), (torch.randn(N, K, generator=g) * sw).to(DEV)
+        ref = ops.linear(x, w, force="fma")
+        assert bool((ref != 0).any()) and ref.abs().min().item() < tiny
+        for kind in [None, "f32:2"] + (["f32:1"] if M <= 128 else []):
+            assert torch.equal(ops.linear(x, w, force=kind), ref), (sx, sw, kind)
+        # what flushing products below 2^-126 would give is something else
+        assert not torch.equal(torch.where(ref.abs() < tiny, torch.zeros_like(ref), ref), ref)
+    one = (torch.randn(M, K, generator=g) * tiny / 8).to(DEV)
+    assert bool((one.abs() < tiny).any()) and bool((ops.linear(one, torch.ones(N, K, device=DEV)) != 0).any())
+
+
 # rows, experts, hidden columns of one and of a shared expert: widths that no tile or batch of steps divides, one expert, many
 EXPERT_CASES = [(1, 8, 40, 24), (8, 8, 3584, 3584), (3, 3, 272, 0), (2, 40, 48, 16), (5, 1, 96, 32)]
 
