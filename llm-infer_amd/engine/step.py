@@ -111,9 +111,15 @@ def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
 
 def page_shares(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:
     """Shares of a token's keys for the decode kernels of differential and latent attention, whose share is a workgroup of four
-    waves that merge inside it: as ``page_splits``, but one for the shortest contexts, whose waves have a page at most each."""
-    # measured on MI355X, us: latents of 256 / 192 (16 heads, batch 8) at 64 keys 9.6 in one share (10.7 in two, with the kernel that
-    # merges them), at 128 10.2 (11.4), at 192 12.2 (11.3); with half as many shares and with these 13.4 and 11.3 at 300, 14.9 and 12.5 at
-    # 1,000.  Two maps of 64 with values of 128 (32 / 8 heads, batch 4) at 64 9.9 (12.9), at 128 10.6 (13.6), at 192 13.9 (12.7);
-    # 17.6 and 14.3 at 500
-    return 1 if bucket == 1 else page_splits(n_seqs, n_kv_heads, n_heads, bucket)
+    waves that merge inside it (a power of two): down to one page each as ``page_splits``, one for the shortest contexts,
+    and no more workgroups than CUs."""
+    # measured on MI355X, us.  One share: latents of 256 / 192 (16 heads, batch 8) at 64 keys 9.6 (10.7 in two, with the kernel that
+    # merges them), at 128 10.2 (11.4), at 192 12.2 (11.3); two maps of 64 with values of 128 (32 / 8 heads, batch 4) at 64 9.9
+    # (12.9), at 128 10.6 (13.6), at 192 13.9 (12.7).  Longer contexts, shares that make 256 workgroups (and twice as many): latents
+    # of 32 heads, batch 32 at 2,000 24.7 (34.3), batch 64 at 1,000 24.8 (33.9), batch 16 at 4,000 23.9 (33.7); two maps, batch 4
+    # at 2,000 19.6 (23.9), batch 8 at 600 18.7 (22.1), batch 16 at 600 22.9 (26.4), batch 32 at 300 19.6 (27.2).  Fewer than
+    # that, a page a share (and two): latents batch 1 at 300 13.2 (14.7), at 600 13.3 (15.0), at 4,000 14.6 (15.6), but
+    # at 2,000, two pages after all, 14.5 (13.6)
+    groups = n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 31) // 32)
+    s = 1 if bucket == 1 else max(1, min(2 * bucket, 64, 256 // max(1, groups)))
+    return 1 << (s.bit_length() - 1)

@@ -255,8 +255,11 @@ def test_splits_down_to_one_page():
             s = page_splits(n, k, h, bucket)
             assert s & (s - 1) == 0 and 1 <= s <= min(64, max(2, pages))
             assert decode_splits(n, k, h, bucket) <= s <= 2 * decode_splits(n, k, h, bucket)
-            assert page_shares(n, k, h, bucket) == (1 if ctx <= 192 else s)
-    assert page_splits(1, 8, 32, 64) == 64 and page_shares(1, 8, 32, 64) == 64
+            shares = page_shares(n, k, h, bucket)
+            assert shares & (shares - 1) == 0 and 1 <= shares <= s and (ctx > 192 or shares == 1)
+            assert shares == 1 or shares * n * k * ((h // k + 31) // 32) <= 256
+    assert page_splits(1, 8, 32, 64) == 64 and page_shares(1, 8, 32, 64) == 32 and page_shares(1, 1, 32, 64) == 64
+    assert page_shares(32, 1, 32, 16) == 8 and page_shares(64, 8, 32, 16) == 1 and page_shares(8, 8, 32, 4) == 4
 
 
 def test_sizes_of_float32_products():
