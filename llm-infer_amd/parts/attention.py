@@ -90,7 +90,7 @@ class Attention(Part):
             a = ops.attention_f32(q, kv, ctx.pos, ctx.tok_slot, H, K, hd, self.scale, self.window)
         elif ctx.is_decode:
             a = ops.attention_decode(q, kv, ctx.seq_slot, ctx.seq_ctx, ctx.n_seqs, H, K, hd, self.scale,
-                                     self.window, ctx.page_splits(K, H))
+                                     self.window, ctx.page_splits(K, H, hd))
         else:
             a = ops.attention_prefill(q, kv, ops.prefill_meta(ctx), H, K, hd, self.scale, self.window)
         ops.linear(a.view(a.shape[0], H * hd), self.wo, ops.EPI_ADD, out=residual)

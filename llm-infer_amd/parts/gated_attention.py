@@ -185,7 +185,7 @@ class GatedAttention(Part):
     def _splits(self, ctx) -> int:
         """Splits of the keys for the softmax decoder's decode kernel: what the step asks for, but at least a page a split of
         what the mask leaves (a power of two)."""
-        splits = ctx.page_splits(self.n_kv_heads, self.n_heads)
+        splits = ctx.page_splits(self.n_kv_heads, self.n_heads, self.head_dim)
         for span in (self.block, self.window):
             if span:
                 splits = min(splits, max(1, (span + self.keep_first) // 64))

@@ -252,13 +252,16 @@ def test_splits_down_to_one_page():
     for ctx in range(1, 9000, 37):
         pages, bucket = (ctx + 63) // 64, split_bucket(ctx)
         for n, k, h in ((1, 8, 32), (3, 1, 4), (8, 2, 2), (64, 8, 32), (8, 1, 16)):
-            s = page_splits(n, k, h, bucket)
-            assert s & (s - 1) == 0 and 1 <= s <= min(64, max(2, pages))
-            assert decode_splits(n, k, h, bucket) <= s <= 2 * decode_splits(n, k, h, bucket)
+            few = decode_splits(n, k, h, bucket)
+            for hd in (64, 128, 160, 256):
+                s = page_splits(n, k, h, bucket, hd)
+                assert s & (s - 1) == 0 and 1 <= s <= min(64, max(2, pages)) and s in (few, 2 * few)
+                assert hd > 160 or s <= 4 or s == few or s * n * k * ((h // k + 31) // 32) <= 512
             shares = page_shares(n, k, h, bucket)
-            assert shares & (shares - 1) == 0 and 1 <= shares <= s and (ctx > 192 or shares == 1)
+            assert shares & (shares - 1) == 0 and 1 <= shares <= 2 * few and (ctx > 192 or shares == 1)
             assert shares == 1 or shares * n * k * ((h // k + 31) // 32) <= 256
-    assert page_splits(1, 8, 32, 64) == 64 and page_shares(1, 8, 32, 64) == 32 and page_shares(1, 1, 32, 64) == 64
+    assert page_splits(1, 8, 32, 64, 128) == 64 and page_splits(1, 8, 32, 4, 128) == 4 and page_splits(1, 8, 32, 4, 256) == 8
+    assert page_splits(2, 8, 32, 32, 128) == 32 and page_splits(2, 8, 32, 16, 128) == 32 and page_shares(1, 8, 32, 64) == 32 and page_shares(1, 1, 32, 64) == 64
     assert page_shares(32, 1, 32, 16) == 8 and page_shares(64, 8, 32, 16) == 1 and page_shares(8, 8, 32, 4) == 4
 
 
