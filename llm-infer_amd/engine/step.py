@@ -102,17 +102,18 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
 
 def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int, head_dim: int) -> int:
     """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one page a
-    split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64.  Heads of up to 160 keep four splits,
-    which merge inside a workgroup, and are not split further for more waves than half the chip's SIMDs."""
+    split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64.  Heads of up to 160 are not split
+    beyond four, which merge inside a workgroup, for more waves than half the chip's SIMDs, and those below 128 not into eight."""
     # measured on MI355X, us with half as many splits and with these.  Heads of 128, 8 KV heads, batch 1 at 40 tokens 6.2 and 6.1,
-    # at 100 7.5 and 6.3, at 250 7.6 and 6.7, at 1,000 9.9 and 9.0, at 2,000 11.3 and 10.4, at 4,000 14.1 and 11.7; batch 32 at 250 10.7 and
-    # 10.5.  Kept at four (eight): 128, batch 1 at 500 8.2 (8.7), at 900 10.3 (9.2), batch 8 at 500 10.2 (10.8), batch 16 at 500 11.3
-    # (13.1), at 900 15.5 (17.9); 64, batch 8 at 500 8.6 (10.2).  1,024 waves: 128, batch 4 at 4,000 18.1 (18.6), batch 8 at 1,900 17.0
-    # (17.8), batch 2 at 8,000 18.6 (19.6); 160, 4 KV heads, 64 splits at 8,000 19.0 (20.0).  Heads of 256, 2 KV heads, whose pages are longer: batch 1 at 500 30 and 18, batch 32 at
-    # 1,000 67 and 49
+    # at 100 7.5 and 6.3, at 250 7.6 and 6.7, at 500 8.2 and 8.6, at 777 10.3 and 9.2 (with a soft cap and gates 12.5 and 10.3), at 1,000
+    # 9.9 and 9.0, at 2,000 11.3 and 10.4, at 4,000 14.1 and 11.7; batch 32 at 250 10.7 and 10.5.  Not taken (what more would take): 128,
+    # batch 16 at 500 11.3 (13.1), at 900 15.5 (17.9), batch 4 at 4,000 18.1 (18.6), batch 8 at 1,900 17.0 (17.8), batch 2 at 8,000 18.6
+    # (19.6); 64, batch 1 at 500 7.6 (8.6), at 900 8.5 (8.7), batch 8 at 500 8.6 (10.2), at 900 11.0 (10.6); 96, batch 1 at 700 8.1
+    # (9.0), batch 8 at 900 12.1 (11.8); 160, 4 KV heads, 64 splits at 8,000 19.0 (20.0).  Heads of 256, 2 KV heads, whose pages are
+    # longer: batch 1 at 500 30 and 18, batch 32 at 1,000 67 and 49
     few, many = (decode_splits(n_seqs, n_kv_heads, n_heads, min(b, 64)) for b in (bucket, 2 * bucket))
     waves = many * n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 31) // 32)
-    return few if head_dim <= 160 and many > 4 and (few == 4 or waves > 512 or (many == 64 and head_dim > 128)) else many
+    return few if head_dim <= 160 and many > 4 and (waves > 512 or (few == 4 and head_dim < 128) or (many == 64 and head_dim > 128)) else many
 
 
 def page_shares(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> int:

@@ -260,8 +260,8 @@ def test_splits_down_to_one_page():
             shares = page_shares(n, k, h, bucket)
             assert shares & (shares - 1) == 0 and 1 <= shares <= 2 * few and (ctx > 192 or shares == 1)
             assert shares == 1 or shares * n * k * ((h // k + 31) // 32) <= 256
-    assert page_splits(1, 8, 32, 64, 128) == 64 and page_splits(1, 8, 32, 4, 128) == 4 and page_splits(1, 8, 32, 4, 256) == 8
-    assert page_splits(2, 8, 32, 32, 128) == 32 and page_splits(2, 8, 32, 16, 128) == 32 and page_shares(1, 8, 32, 64) == 32 and page_shares(1, 1, 32, 64) == 64
+    assert page_splits(1, 8, 32, 64, 128) == 64 and page_splits(1, 8, 32, 4, 64) == 4 and page_splits(1, 8, 32, 4, 128) == 8 and page_splits(16, 8, 32, 4, 256) == 8
+    assert page_splits(2, 8, 32, 32, 128) == 32 and page_splits(16, 8, 32, 4, 128) == 4 and page_splits(2, 8, 32, 16, 128) == 32 and page_shares(1, 8, 32, 64) == 32 and page_shares(1, 1, 32, 64) == 64
     assert page_shares(32, 1, 32, 16) == 8 and page_shares(64, 8, 32, 16) == 1 and page_shares(8, 8, 32, 4) == 4
 
 
