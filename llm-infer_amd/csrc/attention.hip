@@ -920,8 +920,10 @@ extern "C" int li_attn_f32(const float* q, float* out, const void* k, const void
     if (check_heads(H, K)) return LI_BAD_ARG;
     if (n_tokens <= 0) return LI_OK;
     CachePtrs c{k, v, page_stride, page_table, max_pages};
-    // heads of a KV head that share a workgroup (and the loads of its keys), where there are workgroups enough without it: one
-    // head a workgroup is shorter for few tokens (3 of 32 heads of 64 at 200 keys 9.7 against 12.5 us)
+    // heads of a KV head that share a workgroup (and the loads of its keys), where there are workgroups enough without it.  us
+    // with one head a workgroup and with them shared: 32 / 8 heads of 64 at 200 keys 4 tokens 9.3 and 12.2, 32 10.7 and 12.3, 48
+    // 14.7 and 15.0, 64 16.0 and 14.3, 200 36 and 26; at 1,000 keys 32 51 and 58, 48 57 and 59, 64 68 and 59; at 60 keys 100 13.8 and
+    // 14.9, 200 21.9 and 20.3.  32 / 8 heads of 128 at 200 keys 24 18.2 and 18.9, 32 19.3 and 18.8, 48 24.4 and 20.1
     int hg = (int64_t)n_tokens * H <= 1024 ? 1 : 256 / HD;
     while ((H / K) % hg) --hg;
     dim3 grid(n_tokens, H / hg), block(256);

@@ -2,7 +2,7 @@
 //
 // v_mfma_f32_16x16x4_f32 adds its products one after the other in ascending k, each as a fused multiply-add rounded to
 // nearest, subnormal numbers kept: an accumulator that takes k in ascending order is bit for bit the chain of fmaf that
-// gemm_fma runs (compared on an MI355X over operands of every magnitude).  Both kernels here sum as gemm_fma does, chains
+// gemm_fma runs (compared on an MI355X, operands, products and sums below 2^-126 among them).  Both kernels here sum as gemm_fma does, chains
 // over 256 consecutive k that are added up in ascending order, so a result depends neither on the kernel nor on the batch,
 // and a call that these do not take (K no multiple of 16, an address that is not 16-byte aligned) gives the same numbers
 // through gemm_fma.
@@ -130,8 +130,10 @@ __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restri
 // keeps the matrix cores busy.  In LDS the sixteen k of a step lie as the instructions want them (k = 4 j + g at 4 g + j), dealt
 // out as they are written: swapped in registers as gemv_f32 does it, they cost a third of the matrix
 // instructions' own time.  Rows are 36 floats apart, which keeps the 16-byte reads of a quarter wave on different banks.
-// Bound by the matrix instructions (32 cycles each) and the writes to LDS: 28,672 x 4,096 at 2,048 rows 3.99 ms, 121
-// TFLOP/s; at 400 rows 2,048 x 2,048 41 us (gemm_fma: 233), 16,384 x 2,048 259 us (1,076).
+// Bound by the matrix instructions (32 cycles each): 28,672 x 4,096 at 2,048 rows 3.99 ms, 121 TFLOP/s, the matrix cores busy three
+// quarters of the time, LDS a quarter (a third of that bank conflicts of the writes), waves waiting for LDS 4% of theirs.  Few
+// tiles: a tile's own instructions one after another, at 400 rows 2,048 x 2,048 27 of 41 us (gemm_fma: 233); 16,384 x 2,048
+// 259 us (1,076).
 // ===========================================================================
 __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, int tiles_m, int tiles, Epilogue e) {
     constexpr int BK = 32, LD = BK + 4, ST = 2 * 64 * LD;              // a stage in LDS: rows of W, then rows of X

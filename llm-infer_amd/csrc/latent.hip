@@ -686,7 +686,8 @@ __global__ __launch_bounds__(64) void mlstm_scan_kernel(
 }
 
 // One token of every sequence (a decode step): gates, m and the recurrence in one launch, the operations and their order
-// mlstm_scan_kernel's, so that a token gives the same bits whichever of the two it comes through.  Bound by S, read and
+// mlstm_scan_kernel's, so that a token gives the same bits whichever of the two it comes through.  (The new n and m go to scratch
+// memory, since all of a head's workgroups read the old ones; mlstm_commit_kernel behind it puts them into the state.)  Bound by S, read and
 // written once.  The scan's registers for all of a column make straight-line code of some 30 KB, which a workgroup runs
 // once for a single token: fetching instructions was what took the time.  Here S passes through in batches of 16 rows,
 // four of them on their way at a time, in a loop; q and k are read from LDS, four rows a read.  A workgroup has 64
