@@ -67,7 +67,7 @@ class _GraphContext(StepShared):
     def decode_splits(self, n_kv_heads, n_heads):
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket)
 
-    def page_splits(self, n_kv_heads, n_heads, head_dim):
+    def page_splits(self, n_kv_heads, n_heads, head_dim=128):
         return page_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket, head_dim)
 
     def page_shares(self, n_kv_heads, n_heads):

@@ -71,8 +71,9 @@ class StepContext(StepShared):
         """How many ways the decode attention of a mixer with these heads cuts each sequence's context."""
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
 
-    def page_splits(self, n_kv_heads: int, n_heads: int, head_dim: int) -> int:
-        """The same for the kernel whose waves merge inside a workgroup, where a page a split can be worth it."""
+    def page_splits(self, n_kv_heads: int, n_heads: int, head_dim: int = 128) -> int:
+        """The same for the kernel whose waves merge inside a workgroup, where a page a split can be worth it (``head_dim``: the
+        line between the two depends on it; a mixer that does not say gets that of 128)."""
         return page_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx), head_dim)
 
     def page_shares(self, n_kv_heads: int, n_heads: int) -> int:

@@ -265,6 +265,16 @@ def test_splits_down_to_one_page():
     assert page_shares(32, 1, 32, 16) == 8 and page_shares(64, 8, 32, 16) == 1 and page_shares(8, 8, 32, 4) == 4
 
 
+def test_splits_asked_of_a_step_without_a_head_size():
+    """A mixer may leave the head size out, in a step and in a recorded one."""
+    from llm_infer_amd.engine.decode import _GraphContext
+    from llm_infer_amd.engine.step import StepContext
+    n, ctx = 2, 800
+    bufs = {name: torch.zeros(n, dtype=torch.int32) for name in ("tokens", "pos", "ctx", "slots", "rows")}
+    for step in (StepContext("cpu", list(range(n)), [[1]] * n, [ctx] * n, [[0]] * n), _GraphContext(bufs, n, split_bucket(ctx + 1))):
+        assert step.page_splits(8, 32) == step.page_splits(8, 32, 128) == 8 and step.page_splits(8, 32, 64) == 4
+
+
 def test_sizes_of_float32_products():
     """The rule by which a product goes to the matrix cores is the one by which the library refuses it (before anything runs)."""
     from ctypes import c_void_p
