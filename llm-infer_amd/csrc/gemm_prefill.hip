@@ -1,5 +1,6 @@
 // The products of more than 16 rows of X: gemm_wreg against a tiled weight, gemm_big against a
 // row-major one.  Epilogues, layouts and the split-K reduction are in gemm_common.h.
+#include <type_traits>
 #include "gemm_common.h"
 
 __device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) {
@@ -243,11 +244,81 @@ __host__ __device__ constexpr bool by_pairs(int mode) { return mode == MODE_PAIR
 template <int MODE>
 __device__ __forceinline__ void wreg_epilogue(const Epilogue& e, int m, int n, const float* v) {
     if constexpr (MODE == EPI_CLAMPGLU || MODE == EPI_BIAS || MODE == MODE_PAIRS_GLU) epilogue_extra4(e, m, n, v);
-    else epilogue4_base(e, m, n, v);
+    else if constexpr (MODE == EPI_STORE || MODE == EPI_SWIGLU || MODE == EPI_GEGLU) {
+        Epilogue one = e;
+        one.mode = MODE;
+        epilogue4_base(one, m, n, v);
+    } else epilogue4_base(e, m, n, v);
+}
+
+// The epilogue of results that lie in rows of their own (no residual, no cache; the mode known when it is compiled): every column of the wave's is there, the rows of C are 16-byte aligned and of type OT.  A lane has
+// 4 consecutive columns of one row for every block of 16.  What is stored is computed in the registers where they lie, laid
+// down in LDS by rows, and read back so that a lane stores 16 bytes.  All of it is unrolled: an activation's exponential and
+// quotient take some 150 cycles from their first instruction to the last, and quad after quad, as the loop over every epilogue
+// goes through them, with 4 bytes a lane a store, they were 5 to 20% of a product (us before and after, bfloat16, gate and up:
+// 12,700 x 28,672 x 4,096 2,396 and 2,201, 33,186 x 16,384 x 2,048 1,831 and 1,639, 777 x 16,384 x 2,048 64 and 50; plain
+// store 12,700 x 4,096 x 4,096 341 and 318).
+template <class OT, int NI, int MJ, int MODE>
+__device__ __forceinline__ void rows_out(const Epilogue& e, const f32x4 (&acc)[NI][MJ], unsigned char* stage, int lane, int m0, int nb) {
+    constexpr bool GATED_MODE = MODE == EPI_SWIGLU || MODE == EPI_GEGLU || MODE == EPI_CLAMPGLU;
+    constexpr int STRIPS = 2;                                  // of 16 rows a turn
+    constexpr int ROW = (GATED_MODE ? 8 : 16) * NI * (int)sizeof(OT), PITCH = ROW + 16, CHUNKS = ROW / 16, ALL = STRIPS * 16 * CHUNKS;
+    const int r = lane & 15, g = lane >> 4;
+    const int width = GATED_MODE ? e.N >> 1 : e.N, c0 = GATED_MODE ? nb >> 1 : nb;
+    unsigned char* C = (unsigned char*)e.C;
+#pragma unroll
+    for (int j0 = 0; j0 < MJ; j0 += STRIPS) {
+#pragma unroll
+        for (int j = 0; j < STRIPS; ++j)
+#pragma unroll
+            for (int i = 0; i < NI; ++i) {
+                f32x4 v = acc[i][j0 + j];
+                unsigned char* at = stage + (j * 16 + r) * PITCH;
+                if constexpr (MODE == EPI_BIAS || MODE == EPI_CLAMPGLU) {
+                    const int n = nb + 16 * i + 4 * g;
+                    if (e.gp.bias) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) v[q] += e.gp.bias[n + q];
+                    }
+                }
+                if constexpr (GATED_MODE) {
+                    struct alignas(2 * sizeof(OT)) Two { OT v[2]; } two;
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) {
+                        float h;
+                        if constexpr (MODE == EPI_CLAMPGLU)
+                            h = clamped_glu(v[2 * q], v[2 * q + 1], c0 + 8 * i + 2 * g + q >= e.gp.tail_col ? e.gp.tail_limit : e.gp.limit,
+                                            e.gp.alpha, e.gp.shift);
+                        else h = gate_activation(v[2 * q], MODE == EPI_GEGLU) * v[2 * q + 1];
+                        two.v[q] = from_f32<OT>(h);
+                    }
+                    *(Two*)(at + (8 * i + 2 * g) * sizeof(OT)) = two;
+                } else {
+                    if constexpr (MODE == EPI_BIAS) {
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            if (e.gp.act == 1) { const float t = fmaxf(v[q], 0.f); v[q] = t * t; }
+                            else if (e.gp.act == 2) v[q] = tanhf(v[q]);
+                        }
+                    }
+                    struct alignas(4 * sizeof(OT)) Four { OT v[4]; };
+                    *(Four*)(at + (16 * i + 4 * g) * sizeof(OT)) = Four{{from_f32<OT>(v[0]), from_f32<OT>(v[1]), from_f32<OT>(v[2]), from_f32<OT>(v[3])}};
+                }
+            }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < (ALL + 63) / 64; ++q) {
+            const int c = q * 64 + lane, row = c / CHUNKS, part = c - row * CHUNKS, m = m0 + 16 * j0 + row;
+            if ((ALL % 64 == 0 || c < ALL) && m < e.M)
+                *(f32x4*)(C + ((int64_t)m * width + c0) * sizeof(OT) + part * 16) = *(const f32x4*)(stage + row * PITCH + part * 16);
+        }
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_sched_barrier(0);                     // nothing of the next turn before it (registers)
+    }
 }
 
 template <class T, int NI, int MODE, int MJ = 8, int A = 2>
-__global__ __launch_bounds__(256) void gemm_wreg_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
+__global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
                                                         int K, int k_per_split, float* __restrict__ ws, Epilogue e,
                                                         int wg_blocks, RowScale rsc, PairTiles pt) {
     typedef typename Vec<T>::v8 v8;
@@ -512,6 +583,26 @@ __global__ __launch_bounds__(256) void gemm_wreg_kernel(const T* __restrict__ X,
     float* stage = (float*)smem_raw + wave * (2 * STRIP);
     const int r = lane & 15, g = lane >> 4;
     const int nb = n0 + wn * (16 * NI);                 // this wave's first column
+    // the epilogue by whole rows, for those that know their mode: results of X's type or float32
+    constexpr bool PAIRS = by_pairs(MODE);
+    if constexpr (MODE == EPI_STORE || MODE == EPI_SWIGLU || MODE == EPI_GEGLU || MODE == EPI_BIAS || MODE == EPI_CLAMPGLU || PAIRS) {
+        static_assert(2 * STRIP * 4 >= 2 * 16 * (64 * NI + 16), "rows_out's rows fit two strips");
+        constexpr int SAME = std::is_same<T, f16>::value ? DT_F16 : DT_BF16;
+        const bool gated = e.mode == EPI_SWIGLU || e.mode == EPI_GEGLU || e.mode == EPI_CLAMPGLU;
+        const int row_bytes = (gated ? e.N >> 1 : e.N) * (e.out_dt == DT_F32 ? 4 : 2);
+        if (nb + 16 * NI <= n_end && !((uintptr_t)e.C & 15) && row_bytes % 16 == 0 && gridDim.z == 1 &&
+            (e.out_dt == SAME || (e.out_dt == DT_F32 && !(PAIRS && gated)))) {
+            unsigned char* rows = (unsigned char*)stage;
+            if constexpr (MODE == MODE_PAIRS_GLU) rows_out<T, NI, MJ, EPI_CLAMPGLU>(e, acc, rows, lane, m0, nb);
+            else if constexpr (MODE == MODE_PAIRS) {
+                if (e.mode == EPI_SWIGLU) rows_out<T, NI, MJ, EPI_SWIGLU>(e, acc, rows, lane, m0, nb);
+                else if (e.out_dt == DT_F32) rows_out<float, NI, MJ, EPI_STORE>(e, acc, rows, lane, m0, nb);
+                else rows_out<T, NI, MJ, EPI_STORE>(e, acc, rows, lane, m0, nb);
+            } else if (e.out_dt == DT_F32) rows_out<float, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
+            else rows_out<T, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
+            return;
+        }
+    }
     auto to_stage = [&](int j, int place) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) *(f32x4*)(stage + place * STRIP + r * SLD + 16 * i + 4 * g) = acc[i][j];
@@ -703,7 +794,8 @@ extern "C" int li_gemm_wreg(const void* X, const void* Wt, int dt, void* C, int 
     // the kernels of one epilogue: the residual sum into float32 with whole quads of columns; the
     // rotation with a table of angles
     const int one = splits > 1 ? -1 : (mode == EPI_ADD && N % 4 == 0) ? EPI_ADD : (mode == EPI_ROPE && e.rs.cos_sin) ? EPI_ROPE
-                    : (mode == EPI_CLAMPGLU || mode == EPI_BIAS) ? mode : -1;
+                    : (mode == EPI_CLAMPGLU || mode == EPI_BIAS) ? mode
+                    : ((mode == EPI_SWIGLU || mode == EPI_GEGLU || mode == EPI_STORE) && !few_rows && !rsc) ? mode : -1;
 #define GO(T, NI, MODE, MJ, A)                                                                            \
     do {                                                                                                  \
         auto kfn = gemm_wreg_kernel<T, NI, MODE, MJ, A>;                                                  \
@@ -724,17 +816,25 @@ extern "C" int li_gemm_wreg(const void* X, const void* Wt, int dt, void* C, int 
         else if (one == EPI_BIAS) GO(T, NI, EPI_BIAS, MJ, A); \
         else GO(T, NI, -1, MJ, A);                        \
     } while (0)
+#define BY_EVERY_MODE(T, NI, MJ, A)                       \
+    do {                                                  \
+        if (one == EPI_SWIGLU) GO(T, NI, EPI_SWIGLU, MJ, A); \
+        else if (one == EPI_GEGLU) GO(T, NI, EPI_GEGLU, MJ, A); \
+        else if (one == EPI_STORE) GO(T, NI, EPI_STORE, MJ, A); \
+        else BY_MODE(T, NI, MJ, A);                       \
+    } while (0)
 #define LAUNCH(T)                                       \
     do {                                                \
-        if (tile == 0) BY_MODE(T, 4, 8, 2);             \
-        else if (tile == 1) BY_MODE(T, 3, 8, 2);        \
+        if (tile == 0) BY_EVERY_MODE(T, 4, 8, 2);       \
+        else if (tile == 1) BY_EVERY_MODE(T, 3, 8, 2);  \
         else if (few_rows == 1) BY_MODE(T, 2, 4, 4);    \
         else if (few_rows == 2) BY_MODE(T, 2, 8, 4);    \
         else if (few_rows == 3) BY_MODE(T, 2, 8, 3);    \
-        else BY_MODE(T, 2, 8, 2);                       \
+        else BY_EVERY_MODE(T, 2, 8, 2);                 \
     } while (0)
     if (dt == DT_F16) LAUNCH(f16); else LAUNCH(bf16);
 #undef LAUNCH
+#undef BY_EVERY_MODE
 #undef BY_MODE
 #undef GO
     LI_CHECK_LAUNCH();

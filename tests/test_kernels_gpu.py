@@ -308,6 +308,42 @@ def test_linear_tiled_weights(ops, M, N, K, dt):
 
 
 @pytest.mark.parametrize("dt", F16S)
+@pytest.mark.parametrize("M,N,K", [(129, 72, 32), (130, 256, 64), (257, 200, 160), (300, 1000, 96), (511, 528, 96), (384, 1024, 256)])
+def test_tiled_products_write_whole_rows(ops, M, N, K, dt):
+    """The epilogues that store whole rows of a tile, 16 bytes a lane, beside the ones that go through it quad by quad (taken
+    where a wave's columns are not all there or the rows are not aligned to 16 bytes): the same numbers bit for bit, for every
+    tile, kind of result and type, and nothing written beside them."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(dt).to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV)
+    bias = torch.randn(N, generator=g).to(DEV)
+    wt = ops.tile_weight(w)
+    s = x.double() @ w.double().t()
+    b = s + bias.double()
+    glu = lambda v: torch.clamp(v[:, 0::2], max=1.0) * torch.sigmoid(1.702 * torch.clamp(v[:, 0::2], max=1.0)) * (v[:, 1::2].clamp(-1.0, 1.0) + 1)  # noqa: E731
+    refs = {(0, None): s, (2, None): torch.nn.functional.silu(s[:, 0::2]) * s[:, 1::2],
+            (4, None): torch.nn.functional.gelu(s[:, 0::2], approximate="tanh") * s[:, 1::2],
+            (5, "plain"): b, (5, "relu2"): torch.relu(b) ** 2, (5, "tanh"): torch.tanh(b), (6, None): glu(b)}
+    for (mode, act), ref in refs.items():
+        params = ops.glu_params(bias=bias, act=None if act == "plain" else act) if mode >= 5 else None
+        for out_dt in (dt, torch.float32):
+            for kind in ("wreg:0", "wreg:1", "wreg:2"):
+                rows = ref.shape[1]
+                got = []
+                for offset in (0, 8 // (2 if out_dt == dt else 4)):              # rows that begin 16 and 8 bytes aligned
+                    flat = torch.full((M * rows + 64,), 7.0, dtype=out_dt, device=DEV)
+                    out = flat[offset:offset + M * rows].view(M, rows)
+                    ops.linear(x, wt, mode, out=out, force=kind, params=params)
+                    assert (flat[:offset] == 7.0).all() and (flat[offset + M * rows:] == 7.0).all()
+                    got.append(out)
+                assert torch.equal(*got), (mode, act, out_dt, kind)
+                # 2e-4 for K sums in float32 as above, and half a unit in the last place of what is stored
+                ulp = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[out_dt]
+                err = (got[0].double() - ref).abs() - ulp * ref.abs()
+                assert err.max().item() < 2e-4 * (1 + ref.abs().max().item()), (mode, act, out_dt, kind)
+
+
+@pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M,d,K2,N2", [(1, 4096, 4096, 6144), (8, 4096, 14336, 28672), (16, 96, 160, 200), (5, 2048, 64, 128256),
                                        (12, 4096, 14336, 28672), (16, 4096, 4096, 22016), (14, 4096, 4096, 6144)])
 def test_norm_split_over_two_products(ops, M, d, K2, N2, dt):
