@@ -215,8 +215,8 @@ __global__ __launch_bounds__(256) void gemm_big_kernel(const T* __restrict__ X, 
 // X goes through LDS (global_load_lds).  Four waves, each with 16 NI rows of W and all 128 rows of X of the
 // tile (64 NI x 128); two workgroups (three of the narrowest tile) share a CU.  A step is 64 of K: between
 // two barriers a wave issues 16 NI matrix instructions, and the LDS reads of the next fragments of X and
-// the loads of W two steps ahead are issued between them, so that outside the matrix instructions a step
-// has only its wait, its barrier and four loads of X.  What was measured on the way (M = 8,192, random
+// the loads of X and W two steps ahead are issued between them, so that outside the matrix instructions a step
+// has only its wait and its barrier.  What was measured on the way (M = 8,192, random
 // float16): one barrier per 32 of K with all LDS reads before the matrix instructions 1.08 to 1.12 PFLOP/s;
 // reads under the matrix instructions and 64 of K a barrier 1.11 to 1.18; X fetched as whole 128-byte
 // lines instead of two half lines a row 1.23 to 1.32 (the CU's cache takes a request per line touched).
@@ -381,12 +381,15 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     const int n_halves = (ke - kb) >> 5, n_steps = (n_halves + 1) >> 1;
     const int w_blocks = (e.N + 15) >> 4, steps = K >> 5;
 
-    // this wave's rows of W: NI blocks of 16, each a run of 1 KiB units along K
+    // this wave's rows of W: NI blocks of 16, each a run of 1 KiB units along K of which lane l loads 16 bytes at 16 l; the
+    // addresses are the same for the whole wave and stay in scalar registers
     const T* wsrc[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) {
         const int blk = min(n0 / 16 + min(wn * NI + i, wg_blocks - 1), w_blocks - 1);
-        wsrc[i] = Wt + (((int64_t)blk * steps + (kb >> 5)) * 64 + lane) * 8;
+        const uint64_t at = (uint64_t)(Wt + ((int64_t)blk * steps + (kb >> 5)) * 512);
+        wsrc[i] = (const T*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32) |
+                             (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)at));
     }
     // This wave's share of a stage of X.  A 1 KiB unit holds 8 rows x 64 of K, so that the 8 lanes of a row
     // fetch one whole 128-byte line (16 rows x 32 of K, the operand's own order, would fetch two half
@@ -408,25 +411,20 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     // chunk again (the row may end there); nothing reads what they bring.
     const int last = n_halves - 1;
     const uint32_t odd_back = ((n_halves & 1) && ((lane & 7) ^ (lane >> 3)) >= 4) ? 64 : 0;
-    auto fill = [&](int s, int buf_off) {
+    auto fill_one = [&](int i, int s, int buf_off) {              // load i of the stage of step s
         const int st = min(s, n_steps - 1);
         const int64_t at = (int64_t)st * 128;
         const uint32_t back = st == n_steps - 1 ? odd_back : 0;
-#pragma unroll
-        for (int i = 0; i < PER_WAVE; ++i) {
-            const int q = wave * PER_WAVE + i;
-            __builtin_amdgcn_global_load_lds(
-                (const __attribute__((address_space(1))) void*)(xbase + at + (xoff[i] - back)),
-                (__attribute__((address_space(3))) void*)(smem_raw + buf_off + q * 1024), 16, 0, 0);
-        }
+        const int q = wave * PER_WAVE + i;
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(xbase + at + (xoff[i] - back)),
+            (__attribute__((address_space(3))) void*)(smem_raw + buf_off + q * 1024), 16, 0, 0);
     };
     // The loads of W are written as instructions so that the compiler does not place waits for them (at
     // the loop's head it would wait for every load in flight); the waits are placed by hand below.
-    auto fetch_w = [&](int half, v8 (&a)[NI]) {
-        const int64_t at = (int64_t)min(half, last) * 512;
-#pragma unroll
-        for (int i = 0; i < NI; ++i)
-            asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(a[i]) : "v"(wsrc[i] + at) : "memory");
+    auto fetch_one = [&](int i, int half, v8 (&a)[NI]) {          // block i of the fragments of a half step
+        const T* from = wsrc[i] + (int64_t)min(half, last) * 512;
+        asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
     };
 
     f32x4 acc[NI][MJ];
@@ -437,9 +435,11 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
 
     // Half a step: the matrix instructions on one slot of W's fragments and on the fragments of X that are
     // in b[]; as soon as the instructions that use b[j] are issued, b[j] is read again for the half after
-    // this one, so the LDS reads run under the matrix instructions, and so do the loads of W, which go
-    // into a slot as soon as its half is issued.  Between two barriers a wave issues 16 NI matrix
-    // instructions, and outside them only the wait, the barrier and its four loads of X.
+    // this one, so the LDS reads run under the matrix instructions, and so do the loads of a step, dealt out over the
+    // groups one by one: W's into a slot in the half after the one that used it up.  Between two barriers a wave issues 16 NI
+    // matrix instructions, and outside them only the wait and the barrier.  (With a half's loads of W behind it and the four
+    // of X at the step's head, a burst of loads that the other waves issue too, us, bfloat16: 12,700 x 28,672 x 4,096 2,284 and
+    // dealt out 2,238; 33,186 x 16,384 x 2,048 1,712 and 1,675; 12,700 x 4,096 x 4,096 371 and 357.)
     // The LDS reads are written as instructions too, with the waits by hand: the read of b[j] is followed
     // by seven others before b[j] is used, and LDS reads complete in order, so "at most 7 in flight" is the
     // wait before every group of matrix instructions.  (Left to the compiler, each half begins with a wait
@@ -452,38 +452,44 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     const uint32_t lds_lane = lds_base + ((lane >> 4) ^ (lane & 7)) * 16;
     const uint32_t lds_lane2 = lds_base + ((4 + (lane >> 4)) ^ (lane & 7)) * 16;
 #define WREG_READ(J, FROM) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b[J]) : "v"(FROM), "n"((J) * 2048));
-#define WREG_GROUP(J, A, NEXT)                                                             \
+#define WREG_GROUP(J, A, NEXT, LOADS)                                                      \
     {                                                                                      \
         __builtin_amdgcn_s_waitcnt(0xC07F | ((MJ - 1) << 8));   /* lgkmcnt(MJ - 1), nothing else */ \
         __builtin_amdgcn_sched_barrier(0);                                                 \
         _Pragma("unroll") for (int i = 0; i < NI; ++i) acc[i][J] = mfma16(A[i], b[J], acc[i][J]); \
         __builtin_amdgcn_sched_barrier(0);                                                 \
         WREG_READ(J, NEXT)                                                                 \
+        LOADS(std::integral_constant<int, J>{});                                           \
         __builtin_amdgcn_sched_barrier(0);                                                 \
     }
 #define WREG_EIGHT(F, ...) F(0, __VA_ARGS__) F(1, __VA_ARGS__) F(2, __VA_ARGS__) F(3, __VA_ARGS__) \
     if constexpr (MJ == 8) { F(4, __VA_ARGS__) F(5, __VA_ARGS__) F(6, __VA_ARGS__) F(7, __VA_ARGS__) }
-#define WREG_HALF(A, NEXT)                                                                 \
+#define WREG_HALF(A, NEXT, LOADS)                                                          \
     {                                                                                      \
         const uint32_t next_ = (NEXT);                                                     \
-        WREG_EIGHT(WREG_GROUP, A, next_)                                                   \
+        WREG_EIGHT(WREG_GROUP, A, next_, LOADS)                                            \
     }
 
     // (The host gives every split of K at least one step.  Without this line the compiler builds a path
     // for no steps on which the ring's registers are written while the first loads are in flight.)
     if (n_steps <= 0) return;
-    // In flight, in order: at the head of step s the loads of X of step s + A are issued, in its middle
-    // those of W's first half of step s + A, at its end those of the second half.  Step s needs X of step
-    // s + 1 (its second half reads ahead into it) and its own W: everything up to the loads of X of step s + 1,
-    // i.e. all but the 2 NI loads that followed them in their step and the A - 2 whole steps issued since.
+    // In flight, in order: in the first half of step s the loads of X of step s + A and of W's second half of step
+    // s + A - 1 (whose slot the step before has used up), in its second half those of W's first half of step s + A.  Step s
+    // needs X of step s + 1 (its second half reads ahead into it) and its own W: everything up to the first half of step
+    // s + 1 - A, i.e. all but the NI loads of that step's second half and the A - 2 whole steps issued since.
     v8 ring[SLOTS][NI];
-    constexpr int PER_STEP = PER_WAVE + 2 * NI, AHEAD = 2 * NI + (A - 2) * PER_STEP;
-    static_assert((A - 1) * PER_STEP <= 63 && AHEAD <= 63, "the waits' counts");
+    constexpr int PER_STEP = PER_WAVE + 2 * NI, AHEAD = NI + (A - 2) * PER_STEP, FIRST = (A - 1) * PER_STEP - NI;
+    static_assert(FIRST <= 63 && AHEAD <= 63, "the waits' counts");
 #pragma unroll
     for (int a = 0; a < A; ++a) {
-        fill(a, a * STAGE);
-        fetch_w(2 * a, ring[2 * a]);
-        fetch_w(2 * a + 1, ring[2 * a + 1]);
+#pragma unroll
+        for (int i = 0; i < PER_WAVE; ++i) fill_one(i, a, a * STAGE);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) fetch_one(i, 2 * a, ring[2 * a]);
+        if (a < A - 1) {
+#pragma unroll
+            for (int i = 0; i < NI; ++i) fetch_one(i, 2 * a + 1, ring[2 * a + 1]);
+        }
     }
     // RowScale (MODE -1, at most 16 rows of X, K whole; the host sees to it): the partial sums of squares of row
     // tid % 16 are dealt to the 16 groups of 16 threads; they are fetched behind the first loads, and everything is
@@ -510,7 +516,7 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
         }
     }
     // X of step 0 has landed (and W of step 0 with it)
-    if (!scaled) __builtin_amdgcn_s_waitcnt(0x0F70 | (((A - 1) * PER_STEP) & 15) | ((((A - 1) * PER_STEP) >> 4) << 14));
+    if (!scaled) __builtin_amdgcn_s_waitcnt(0x0F70 | (FIRST & 15) | ((FIRST >> 4) << 14));
     __builtin_amdgcn_s_barrier();
     WREG_EIGHT(WREG_READ, lds_lane)
     int cur = 0;                                                   // byte offset of the buffer of step s
@@ -525,13 +531,23 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
                 // publishes the one and frees the other
                 __builtin_amdgcn_s_waitcnt(0x0070 | (MJ << 8) | (AHEAD & 15) | ((AHEAD >> 4) << 14));
                 __builtin_amdgcn_s_barrier();
-                fill(s + u + A, free_buf);
                 __builtin_amdgcn_sched_barrier(0);
-                WREG_HALF(ring[2 * u], lds_lane2 + cur)
-                fetch_w(2 * (s + u + A), ring[2 * u]);
-                __builtin_amdgcn_sched_barrier(0);
-                if (2 * (s + u) + 1 < n_halves) WREG_HALF(ring[2 * u + 1], lds_lane + nxt)
-                fetch_w(2 * (s + u + A) + 1, ring[2 * u + 1]);
+                auto first_loads = [&](auto group) {
+                    constexpr int ALL = PER_WAVE + NI;
+#pragma unroll
+                    for (int t = 0; t < ALL; ++t)
+                        if (t * MJ / ALL == decltype(group)::value) {
+                            if (t < PER_WAVE) fill_one(t, s + u + A, free_buf);
+                            else fetch_one(t - PER_WAVE, 2 * (s + u + A) - 1, ring[(2 * u + SLOTS - 1) % SLOTS]);
+                        }
+                };
+                auto second_loads = [&](auto group) {
+#pragma unroll
+                    for (int t = 0; t < NI; ++t)
+                        if (t * MJ / NI == decltype(group)::value) fetch_one(t, 2 * (s + u + A), ring[2 * u]);
+                };
+                WREG_HALF(ring[2 * u], lds_lane2 + cur, first_loads)
+                if (2 * (s + u) + 1 < n_halves) WREG_HALF(ring[2 * u + 1], lds_lane + nxt, second_loads)
                 __builtin_amdgcn_sched_barrier(0);
                 cur = nxt;
             }
