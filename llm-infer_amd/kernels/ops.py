@@ -508,9 +508,13 @@ def _finish_norm(lazy: "LazyNorm", x: torch.Tensor) -> _RowScale:
 _WREG_TILES = {0: (256, 128), 1: (192, 128), 2: (128, 128)}
 # Microseconds that one round of workgroups takes, measured on MI355X, as (a, c): a K / 4096 + c.  Entry i
 # is a round with i + 1 workgroups on every CU: two share a CU (three of the narrowest tile), and those of a
-# last round that is less full run at the shorter time.
-_WREG_ROUND_US = {0: ((53.0, 9.0), (103.0, 5.0)), 1: ((35.0, 13.0), (73.0, 12.0)),
-                  2: ((31.4, 3.4), (57.1, 3.8), (89.0, 0.0))}
+# last round that is less full run at the shorter time.  (Between the residual sum's times and the gated activation's; a
+# full round of the widest tile, us at K = 2,048, 4,096 and 14,336: 69 and 55, 110 and 98, 366 and 345.)
+_WREG_ROUND_US = {0: ((53.0, 9.0), (98.0, 7.0)), 1: ((42.0, 4.0), (77.0, 6.0)),
+                  2: ((31.4, 3.4), (56.0, 3.8), (95.0, 0.0))}
+# The same for at most one workgroup a CU behind full rounds: with a short K they run beside the last of those, with a long one
+# they begin late (us at K = 2,048, 4,096 and 14,336 behind four rounds: 17, 45, 197; 17, 27, 270; 14, 22, 200).
+_WREG_TAIL_US = {0: (60.0, -14.0), 1: (85.0, -30.0), 2: (62.0, -20.0)}
 
 
 def _wreg_blocks(tile: int, splits: int, m: int, n: int) -> int:
@@ -538,8 +542,9 @@ def _wreg_cost(tile: int, splits: int, m: int, n: int, k: int) -> float:
     full, rest = divmod(groups, 256 * len(times))
     k_split = -(-(-(-k // splits)) // 32) * 32
     us = 0.0
-    for count, (a, c) in ((full, times[-1]), (1 if rest else 0, times[-(-rest // 256) - 1])):
-        us += count * (a * wg_blocks * 16 / bn * k_split / 4096 + c)
+    last = _WREG_TAIL_US[tile] if full and rest <= 256 else times[-(-rest // 256) - 1]
+    for count, (a, c) in ((full, times[-1]), (1 if rest else 0, last)):
+        us += count * max(10.0, a * wg_blocks * 16 / bn * k_split / 4096 + c)
     # W streams at 5.5 TB/s when every CU has a workgroup, at less with fewer workgroups
     main = max(us, n * k * 2 / (5.5e6 * min(1.0, groups / 256)))
     if tile == 2 and m <= 64:
