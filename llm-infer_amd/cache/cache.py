@@ -27,6 +27,7 @@ from dataclasses import dataclass
 import numpy as np
 import torch
 
+from ..kernels import ops
 from ..tensor import Tensor
 from .slots import CacheError, PagePool, SlotAllocator
 from .specs import KVSpec, StateSpec
@@ -71,6 +72,7 @@ class KVGroup:
         self.max_pages = (max_positions + PAGE - 1) // PAGE
         self.pool = PagePool(n_pages, first=1)
         self.table_host = np.zeros((n_slots, self.max_pages), dtype=np.int32)
+        self.table_sent = np.zeros_like(self.table_host)            # what the device's table holds
         self.pages_of = [dict() for _ in range(n_slots)]            # slot -> {page index in sequence: page}
         self.device, self.dtype = device, dtype
         self._views = {}
@@ -154,16 +156,18 @@ class KVGroup:
         have.clear()
         self.table_host[slot, :] = NULL_PAGE
 
-    def flush(self, dirty: set, fresh: list) -> None:
+    def flush(self, dirty: set, fresh: list, also=()) -> None:
+        """Brings the device's rows of the slots ``dirty`` up to date and clears the pages ``fresh``.  ``also``: another table's
+        words that change in the same launch (``ops.cache_edit``)."""
         if self.storage is None:
             return
-        if fresh:
-            idx = torch.tensor(sorted(fresh), dtype=torch.int64, device=self.device)
-            self.storage.index_fill_(0, idx, 0)
-        if dirty:
-            rows = sorted(dirty)
-            idx = torch.tensor(rows, dtype=torch.int64, device=self.device)
-            self.page_table.index_copy_(0, idx, torch.from_numpy(self.table_host[rows]).to(self.device))
+        rows = np.array(sorted(dirty), dtype=np.int64)
+        row, page = np.nonzero(self.table_host[rows] != self.table_sent[rows])
+        row = rows[row]
+        values = self.table_host[row, page]
+        if len(row) or fresh or also:
+            ops.cache_edit([(self.page_table, row * self.max_pages + page, values), *also], self.storage, fresh)
+        self.table_sent[row, page] = values
 
 
 class StateGroup:
@@ -177,11 +181,6 @@ class StateGroup:
 
     def view(self, entry: int) -> StateView:
         return StateView(self.storage[self.entries.index(entry)], self.spec)
-
-    def reset(self, slots) -> None:
-        if self.storage is not None and slots:
-            idx = torch.tensor(sorted(slots), dtype=torch.int64, device=self.device)
-            self.storage.index_fill_(1, idx, 0)
 
 
 class Cache:
@@ -236,11 +235,8 @@ class Cache:
     def alloc_slot(self) -> int:
         s = self.slots.alloc()
         self.lens[s] = 0
-        for g in self.groups:
-            if isinstance(g, StateGroup):
-                g.reset([s])
         if self.lens_dev is not None:
-            self.lens_dev[s] = 0
+            ops.clear_rows([g.storage for g in self.groups if isinstance(g, StateGroup)] + [self.lens_dev.view(1, -1)], s)
         return s
 
     def free_slot(self, slot: int) -> None:
@@ -252,7 +248,7 @@ class Cache:
 
     def grow(self, slots, new_lens, sync_lens: bool = True, filled: bool = False) -> None:
         """Make room for each slot to reach its new length, then record the lengths.  All page
-        tables and fresh pages are updated with one small copy and one fill per group.
+        tables, lengths and fresh pages are updated with one launch per group.
         ``filled``: the caller writes every position between the old and the new length before
         anything reads the cache (a step does), so pages that lie wholly in between are not cleared."""
         for slot, n in zip(slots, new_lens):
@@ -260,36 +256,43 @@ class Cache:
                 raise CacheError(f"a sequence of {n} tokens exceeds the model's {self.max_positions} positions")
             if slot not in self.slots._held:
                 raise CacheError(f"slot {slot} is not held")
-        for g in self.groups:
-            if not isinstance(g, KVGroup):
-                continue
-            dirty, fresh = set(), []
-            try:
-                for slot, n in zip(slots, new_lens):
-                    g.reserve(slot, self.lens[slot], n, dirty, fresh, filled)
-            finally:
-                g.flush(dirty, fresh)
+        changes, grown = [], False
+        try:
+            for g in self.groups:
+                if isinstance(g, KVGroup):
+                    changes.append((g, set(), []))
+                    for slot, n in zip(slots, new_lens):
+                        g.reserve(slot, self.lens[slot], n, *changes[-1][1:], filled)
+            grown = True
+        finally:
+            self._flush(changes, slots if grown and sync_lens else (), new_lens)
         for slot, n in zip(slots, new_lens):
             self.lens[slot] = n
-        if sync_lens and self.lens_dev is not None and slots:
-            idx = torch.tensor(list(slots), dtype=torch.int64, device=self.device)
-            self.lens_dev.index_copy_(0, idx, torch.tensor(list(new_lens), dtype=torch.int32, device=self.device))
+
+    def _flush(self, changes, slots, lens) -> None:
+        """What changed in each group (group, slots, pages to clear) and the lengths of ``slots`` onto the device."""
+        if self.lens_dev is None:
+            return
+        words = [(self.lens_dev, np.array(slots, dtype=np.int64), np.array(lens))] if len(slots) else []
+        for g, dirty, fresh in changes:
+            g.flush(dirty, fresh, words)
+            words = []                    # (they went with the first group)
+        if words:
+            ops.cache_edit(words)
 
     def truncate(self, slots, lens) -> None:
         """Takes sequences back to earlier lengths (a step that failed after ``grow``): the lengths are
         restored and the pages beyond them given back, so that a later step finds them cleared or fills
         them itself.  State groups are not restored: what a mixer has already written into its state stays."""
+        changes = []
         for g in self.groups:
             if isinstance(g, KVGroup):
-                dirty = set()
+                changes.append((g, set(), ()))
                 for slot, n in zip(slots, lens):
-                    g.release_from(slot, n, dirty)
-                g.flush(dirty, [])
+                    g.release_from(slot, n, changes[-1][1])
+        self._flush(changes, slots, lens)
         for slot, n in zip(slots, lens):
             self.lens[slot] = n
-        if self.lens_dev is not None and slots:
-            idx = torch.tensor(list(slots), dtype=torch.int64, device=self.device)
-            self.lens_dev.index_copy_(0, idx, torch.tensor(list(lens), dtype=torch.int32, device=self.device))
 
     def trim_windows(self, slots) -> None:
         for g in self.groups:

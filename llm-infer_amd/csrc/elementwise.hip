@@ -269,6 +269,104 @@ extern "C" int li_decode_prepare(const int* seq_slot, int* lens, int* pos, int* 
     return LI_OK;
 }
 
+// ---------------------------------------------------------------------------
+// Bookkeeping of the cache between steps: single words of its tables (page tables, lengths, sampling state) and pages
+// to be cleared, both listed in the kernel's own arguments, so that nothing is uploaded and the host does not wait.
+// Bound by the launch.  A page-table update by index and row tensors was three uploads from pageable memory and two kernels, each
+// upload waiting for all work before it: with 48 live sequences every other decode step paid 0.1 ms for that.
+// ---------------------------------------------------------------------------
+enum { EDIT_WORDS = 896 };                       // 3.5 KiB of arguments; a launch takes 4
+
+struct CacheEdits {
+    int n0, n1, n_pages;
+    int data[EDIT_WORDS];                        // (word, value) pairs of dst0, those of dst1, pages
+};
+
+enum { CLEAR_BLOCK = 256 * 16 * 8 };             // bytes that a workgroup clears: eight stores a thread
+
+__global__ __launch_bounds__(256) void cache_edit_kernel(int* __restrict__ dst0, int* __restrict__ dst1,
+                                                         uint4* __restrict__ pages, int64_t page_bytes, int per_page,
+                                                         const CacheEdits e) {
+    if (blockIdx.x == 0) {
+        for (int i = threadIdx.x; i < e.n0; i += 256) dst0[e.data[2 * i]] = e.data[2 * i + 1];
+        const int* d = e.data + 2 * e.n0;
+        for (int i = threadIdx.x; i < e.n1; i += 256) dst1[d[2 * i]] = d[2 * i + 1];
+        return;
+    }
+    const int b = blockIdx.x - 1;
+    uint4* p = pages + (int64_t)e.data[2 * (e.n0 + e.n1) + b / per_page] * (page_bytes / 16);
+    const int64_t from = (int64_t)(b % per_page) * (CLEAR_BLOCK / 16);
+    const int64_t to = min(from + CLEAR_BLOCK / 16, page_bytes / 16);
+    for (int64_t i = from + threadIdx.x; i < to; i += 256) p[i] = make_uint4(0, 0, 0, 0);
+}
+
+// words: n0 pairs for dst0, n1 pairs for dst1, n_pages pages of page_bytes bytes each behind `pages`.
+extern "C" int li_cache_edit(int* dst0, int n0, int* dst1, int n1, void* pages, int64_t page_bytes, int n_pages,
+                             const int* words, hipStream_t stream) {
+    if (n0 < 0 || n1 < 0 || n_pages < 0 || 2 * ((int64_t)n0 + n1) + n_pages > EDIT_WORDS) return LI_BAD_ARG;
+    if (n0 + n1 + n_pages == 0) return LI_OK;
+    if ((n0 && !dst0) || (n1 && !dst1) || (n_pages && (!pages || page_bytes <= 0 || page_bytes % 16 || (uintptr_t)pages % 16))) return LI_BAD_ARG;
+    CacheEdits e;
+    e.n0 = n0, e.n1 = n1, e.n_pages = n_pages;
+    for (int i = 0; i < 2 * (n0 + n1) + n_pages; i++) e.data[i] = words[i];
+    const int64_t per_page = n_pages ? (page_bytes + CLEAR_BLOCK - 1) / CLEAR_BLOCK : 1;
+    if (1 + n_pages * per_page > 0x7fffffff) return LI_UNSUPPORTED;
+    cache_edit_kernel<<<(unsigned)(1 + n_pages * per_page), 256, 0, stream>>>(dst0, dst1, (uint4*)pages, page_bytes, (int)per_page, e);
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
+// What a sequence keeps outside the pages starts at zero: one row of every table (group) of fixed-size state, for each of
+// the group's entries.  One launch for all groups; an index fill for each was an upload and a kernel a group, 0.2 ms of host
+// time a sequence in a model of four groups.
+enum { CLEAR_GROUPS = 32 };
+
+struct ClearGroup {
+    char* row;                                   // the slot's row of the group's first entry
+    int64_t entry_stride, row_bytes;
+    int64_t entries;
+};
+
+struct ClearGroups {
+    ClearGroup g[CLEAR_GROUPS];
+};
+
+template <class U> __device__ __forceinline__ void clear_units(char* p, int64_t bytes, U zero) {
+    U* u = (U*)p;
+    for (int64_t i = threadIdx.x; i < bytes / (int64_t)sizeof(U); i += 256) u[i] = zero;
+}
+
+__global__ __launch_bounds__(256) void clear_rows_kernel(const ClearGroups groups) {
+    int g = 0, entry = blockIdx.y;
+    while (entry >= groups.g[g].entries) entry -= (int)groups.g[g++].entries;
+    const ClearGroup c = groups.g[g];
+    const int64_t from = (int64_t)blockIdx.x * CLEAR_BLOCK;
+    if (from >= c.row_bytes) return;
+    char* p = c.row + entry * c.entry_stride + from;
+    const int64_t n = min((int64_t)CLEAR_BLOCK, c.row_bytes - from);
+    const uint64_t odd = (uint64_t)(uintptr_t)p | (uint64_t)n;
+    if (odd % 16 == 0) clear_units<uint4>(p, n, make_uint4(0, 0, 0, 0));
+    else if (odd % 4 == 0) clear_units<uint32_t>(p, n, 0u);
+    else clear_units<uint8_t>(p, n, 0);
+}
+
+extern "C" int li_clear_rows(const ClearGroup* groups, int n, hipStream_t stream) {
+    if (n < 0 || n > CLEAR_GROUPS) return LI_BAD_ARG;
+    ClearGroups all = {};
+    int64_t entries = 0, most = 0;
+    for (int i = 0; i < n; i++) {
+        if (!groups[i].row || groups[i].entries < 0 || groups[i].row_bytes < 0) return LI_BAD_ARG;
+        all.g[i] = groups[i];
+        entries += groups[i].entries;
+        most = groups[i].row_bytes > most ? groups[i].row_bytes : most;
+    }
+    if (entries == 0 || most == 0) return LI_OK;
+    if (entries > 65535 || most > (int64_t)CLEAR_BLOCK * 0x7fffffff) return LI_UNSUPPORTED;
+    clear_rows_kernel<<<dim3((unsigned)((most + CLEAR_BLOCK - 1) / CLEAR_BLOCK), (unsigned)entries), 256, 0, stream>>>(all);
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
 // out[i] = act(gate[i]) * up[i] for separate gate and up rows:  gu [T, 2F] float32 with
 // gate_j at column 2j and up_j at column 2j+1  ->  h [T, F].  (src/model/block.cpp:203-214)
 // act: gate_activation of common.h (silu, or the reference's gelu).

@@ -8,6 +8,7 @@ import ctypes
 import functools
 from ctypes import c_float, c_int, c_int64, c_uint64, c_void_p
 
+import numpy as np
 import torch
 
 from . import build
@@ -693,6 +694,57 @@ def decode_prepare(seq_slot, lens, pos, ctx, n, scratch_slot: int = -1, inv_freq
                                     _ptr(inv_freq), _ptr(table), inv_freq.numel() if inv_freq is not None else 0,
                                     _stream()), "decode_prepare")
     return table
+
+
+EDIT_WORDS = 896         # what li_cache_edit takes in one launch
+
+
+def cache_edit(edits=(), storage=None, pages=()) -> None:
+    """``edits``: up to two (tensor, words, values), numpy int32 arrays: 32-bit word ``words[i]`` of the tensor becomes ``values[i]``.
+    ``pages``: rows of ``storage`` [pages, elements] that become zero.  All of it travels in the kernel's arguments."""
+    _need(len(edits) <= 2, "cache_edit: at most two tables")
+    jobs = []
+    for t, words, values in edits:
+        _dev(t)
+        limit = t.numel() * t.element_size() // 4
+        _need(t.element_size() % 4 == 0, "cache_edit: 32-bit words")
+        _need(len(words) == len(values) and (len(words) == 0 or (words.min() >= 0 and words.max() < limit)), "cache_edit: words outside the table")
+        jobs.append((t, np.stack([words, values], axis=1).astype(np.int32)))
+    while len(jobs) < 2:
+        jobs.append((None, np.zeros((0, 2), dtype=np.int32)))
+    pages = np.asarray(pages, dtype=np.int32)
+    page_bytes = 0
+    if len(pages):
+        _dev(storage)
+        _need(storage.dim() == 2 and pages.min() >= 0 and pages.max() < storage.shape[0], "cache_edit: pages outside the pool")
+        page_bytes = storage.shape[1] * storage.element_size()
+    (t0, d0), (t1, d1) = jobs
+    while len(d0) or len(d1) or len(pages):
+        a = d0[:EDIT_WORDS // 2]
+        b = d1[:EDIT_WORDS // 2 - len(a)]
+        c = pages[:EDIT_WORDS - 2 * (len(a) + len(b))]
+        data = np.concatenate([a.ravel(), b.ravel(), c])
+        _check(core().li_cache_edit(_ptr(t0), len(a), _ptr(t1), len(b), _ptr(storage), c_int64(page_bytes), len(c),
+                                    c_void_p(data.ctypes.data), _stream()), "cache_edit")
+        d0, d1, pages = d0[len(a):], d1[len(b):], pages[len(c):]
+
+
+class _ClearGroup(ctypes.Structure):
+    _fields_ = [("row", c_void_p), ("entry_stride", c_int64), ("row_bytes", c_int64), ("entries", c_int64)]
+
+
+def clear_rows(tables, row: int) -> None:
+    """Row ``row`` of every table [entries, rows, ...] becomes zero, for all of its entries."""
+    for first in range(0, len(tables), 32):
+        part = tables[first:first + 32]
+        groups = (_ClearGroup * len(part))()
+        for g, t in zip(groups, part):
+            _dev(t)
+            _need(t.dim() >= 2 and 0 <= row < t.shape[1], "clear_rows: no such row")
+            stride = t.stride(0) * t.element_size()
+            row_bytes = stride // t.shape[1]
+            g.row, g.entry_stride, g.row_bytes, g.entries = t.data_ptr() + row * row_bytes, stride, row_bytes, t.shape[0]
+        _check(core().li_clear_rows(groups, len(part), _stream()), "clear_rows")
 
 
 # ---------------------------------------------------------------------------

@@ -9,6 +9,7 @@ index) only, not on the batch it runs in, and seed 0 is an ordinary fixed seed.
 """
 from __future__ import annotations
 
+import numpy as np
 import torch
 
 from ..kernels import ops
@@ -28,10 +29,9 @@ class Sampler:
 
     def start(self, cache, slots, request_indices) -> None:
         """Set each sequence's generator to the start of its own stream."""
-        rows = torch.tensor([[request_key(self.seed, r), 0] for r in request_indices], dtype=torch.int64,
-                            device=cache.device)
-        idx = torch.tensor(list(slots), dtype=torch.int64, device=cache.device)
-        cache.seq_state.index_copy_(0, idx, rows)
+        keys = np.array([[request_key(self.seed, r), 0] for r in request_indices], dtype=np.int64).view(np.int32)
+        words = 4 * np.array(list(slots), dtype=np.int64)[:, None] + np.arange(4)
+        ops.cache_edit([(cache.seq_state, words.ravel(), keys.ravel())])
 
     def sample(self, logits: torch.Tensor, seq_slot: torch.Tensor, cache, out=None, temperature_dev=None) -> torch.Tensor:
         """logits float32 [B, V], seq_slot int32 [B] -> token ids int32 [B] on the device.

@@ -558,6 +558,48 @@ def test_linear_refuses_what_it_cannot_do(ops):
 
 
 # ---------------------------------------------------------------------------
+# the cache's bookkeeping
+# ---------------------------------------------------------------------------
+@pytest.mark.parametrize("n0,n1,n_pages", [(0, 0, 0), (1, 0, 0), (0, 3, 1), (448, 0, 0), (448, 1, 0), (300, 200, 7), (0, 0, 900), (1000, 449, 897)])
+def test_cache_edit(ops, n0, n1, n_pages):
+    """Words and pages around what one launch's arguments hold (896 numbers); pages of one workgroup and of several."""
+    import numpy as np
+    rng = np.random.default_rng(n0 * 7 + n1 + n_pages)
+    a = torch.arange(4096, dtype=torch.int32, device=DEV).view(64, 64)
+    b = torch.arange(1000, dtype=torch.int64, device=DEV)
+    for elems in (64, 32768 // 2 + 64):
+        pool = torch.randint(1, 99, (1000 if elems == 64 else 40, elems), device=DEV).half()
+        want_a, want_b, want_pool = a.clone(), b.clone(), pool.clone()
+        wa, wb = rng.permutation(4096)[:n0], rng.permutation(2000)[:n1]
+        va, vb = rng.integers(-9, 9, len(wa)), rng.integers(0, 9, len(wb))
+        pages = rng.permutation(len(pool))[:n_pages]
+        want_a.view(-1)[torch.from_numpy(wa).to(DEV)] = torch.from_numpy(va).int().to(DEV)
+        want_b.view(torch.int32)[torch.from_numpy(wb).to(DEV)] = torch.from_numpy(vb).int().to(DEV)
+        want_pool[torch.from_numpy(pages).to(DEV)] = 0
+        got_a, got_b = a.clone(), b.clone()
+        ops.cache_edit([(got_a, wa, va), (got_b, wb, vb)], pool, pages)
+        assert torch.equal(got_a, want_a) and torch.equal(got_b, want_b) and torch.equal(pool, want_pool)
+    with pytest.raises(ops.KernelError, match="outside"):
+        ops.cache_edit([(got_a, np.array([4096]), np.array([0]))])
+    with pytest.raises(ops.KernelError, match="outside"):
+        ops.cache_edit((), pool, [len(pool)])
+
+
+def test_clear_rows(ops):
+    """Rows of 16-byte, 4-byte and odd lengths, longer than a workgroup's share, and more tables than one launch takes."""
+    shapes = [((3, 5, 7), torch.float32), ((2, 5, 3), torch.float16), ((1, 5), torch.int32), ((4, 5, 64, 300), torch.float32),
+              ((1, 5, 2), torch.int64)] * 7
+    tables = [torch.randint(1, 99, s, device=DEV).to(dt) for s, dt in shapes]
+    want = [t.clone() for t in tables]
+    for t in want:
+        t[:, 3] = 0
+    ops.clear_rows(tables, 3)
+    assert all(torch.equal(t, w) for t, w in zip(tables, want))
+    with pytest.raises(ops.KernelError, match="no such row"):
+        ops.clear_rows(tables, 5)
+
+
+# ---------------------------------------------------------------------------
 # attention over the paged cache
 # ---------------------------------------------------------------------------
 def _fill_cache(ops, dtype, K, hd, seqs, n_slots=8, window=None):
