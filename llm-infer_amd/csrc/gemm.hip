@@ -346,32 +346,33 @@ struct NoExperts {
     static constexpr bool chosen_only = false;
 };
 
-template <class T, int NT, int MT, int KW, class EB>
+template <class T, int NT, int MT, int KW, class EB, bool HALF = false>
 __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
                                                              int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg,
                                                              EB ex) {
     constexpr bool EXPERTS = EB::chosen_only;
-    if (xg.rows) X += min((int)blockIdx.x * NT * 16 / xg.rows, xg.n - 1) * xg.stride;
+    const int tile0 = HALF ? blockIdx.x >> 1 : blockIdx.x * NT;
+    if (xg.rows) X += min(tile0 * 16 / xg.rows, xg.n - 1) * xg.stride;
     // NT tiles of 16 rows of W and MT tiles of 16 rows of X per wave; W comes from HBM once, the
     // rows of X from the caches (they are few)
     typedef typename Vec<T>::v8 v8;
-    constexpr int U = (NT + MT) <= 2 ? 8 : ((NT + MT) <= 4 ? 4 : 2);   // 32-element steps of K in flight
+    constexpr int U = (NT + MT) <= 2 ? 8 : ((NT + MT) <= 4 ? 4 : 2);   // loads in flight, each of
+    constexpr int SL = HALF ? 2 : 1;                                   // so many 32-element steps of K
     __shared__ float part[KW][NT * MT][64][4];
     __shared__ float ss_wave[KW][16];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, g = lane >> 4;
-    const int tile0 = blockIdx.x * NT;
     const int n_tiles = (e.N + 15) >> 4;
     const int steps = K >> 5;
-    const int per = (steps + KW - 1) / KW;
-    int s_begin = wave * per, s_end = min(steps, s_begin + per), s_next = U;
+    const int per = ((steps + KW - 1) / KW + SL - 1) / SL * SL;
+    int s_begin = wave * per, s_end = min(steps, s_begin + per), s_next = U * SL;
     unsigned long long chosen = ~0ull;
     if constexpr (EXPERTS) {
         chosen = chosen_experts(ex, e.M);
         if (ex.over == EXPERTS_IN_K) {               // the waves take turns, so that what is left out is left out for all of them
-            s_begin = wave * U;
+            s_begin = wave * U * SL;
             s_end = steps;
-            s_next = KW * U;
+            s_next = KW * U * SL;
         } else {
             const int rows = ex.over == EXPERTS_GATED ? 2 * ex.ff : ex.ff;
             const int first = min(tile0 * 16 / rows, ex.n), last = min((tile0 * 16 + NT * 16 - 1) / rows, ex.n);
@@ -381,14 +382,19 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
         }
     }
     const T* wt[NT];
+    // HALF: rows 8 h .. 8 h + 7 of a tile (h: the workgroup's half).  Lanes of r < 8 hold those at step s, the others the same
+    // rows at step s + 1, and likewise the columns of X: of the 16 x 16 sums the two diagonal quarters are wanted, and added
+    const int half = HALF ? blockIdx.x & 1 : 0, later = HALF ? r >> 3 : 0;
+    const int w_lane = HALF ? later * 64 + 16 * g + 8 * half + (r & 7) : lane;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wt[t] = Wt + ((int64_t)min(tile0 + t, n_tiles - 1) * steps * 64 + lane) * 8;
+    for (int t = 0; t < NT; ++t) wt[t] = Wt + ((int64_t)min(tile0 + t, n_tiles - 1) * steps * 64 + w_lane) * 8;
     bool have_x[MT];
     const T* xrow[MT];
 #pragma unroll
     for (int j = 0; j < MT; ++j) {
-        have_x[j] = 16 * j + r < e.M;
-        xrow[j] = X + (int64_t)(have_x[j] ? 16 * j + r : 0) * K + 8 * g;
+        const int row = HALF ? r & 7 : 16 * j + r;
+        have_x[j] = row < e.M;
+        xrow[j] = X + (int64_t)(have_x[j] ? row : 0) * K + 32 * later + 8 * g;
     }
     f32x4 acc[NT][MT];
 #pragma unroll
@@ -413,7 +419,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     }
     for (int s0 = s_begin; s0 < s_end; s0 += s_next) {
         if constexpr (EXPERTS) if (ex.over == EXPERTS_IN_K) {
-            const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U, steps) * 32 - 1) / ex.ff, ex.n);
+            const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U * SL, steps) * 32 - 1) / ex.ff, ex.n);
             bool any = false;
             for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
             if (!any) continue;
@@ -421,12 +427,13 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
         v8 a[U][NT], b[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const bool in = s0 + u < s_end;
+            const int s = s0 + u * SL;
+            const bool in = s + later < s_end;
             const v8 z = {};
 #pragma unroll
-            for (int t = 0; t < NT; ++t) a[u][t] = in ? *(const v8*)(wt[t] + (int64_t)(s0 + u) * 512) : z;
+            for (int t = 0; t < NT; ++t) a[u][t] = in ? *(const v8*)(wt[t] + (int64_t)s * 512) : z;
 #pragma unroll
-            for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + (s0 + u) * 32) : z;
+            for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
         }
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -460,6 +467,12 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                     acc[t][j][q] = v;
                 }
     }
+    if constexpr (HALF) {
+        // rows 4 g + q (g < 2) of column r (r < 8): the sums of even steps here, those of odd steps 40 lanes on
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc[0][0][q] += __shfl_down(acc[0][0][q], 40, WAVE);
+    }
+    const bool mine = !HALF || (r < 8 && g < 2);                      // this lane's sums are results
     if (MT == 1 && rsc.ss) {
         // this lane's row: the waves' sums in wave order, then 1 / (scale * rms)
         float ss = ss_wave[0][r];
@@ -482,8 +495,8 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
             const float scale = ro.row_scale ? ro.row_scale[m & 15] : ro.scale;
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int n = (tile0 + t) * 16 + 4 * g;
-                if (m < e.M && n < e.N) {
+                const int n = (tile0 + t) * 16 + 8 * half + 4 * g;
+                if (mine && m < e.M && n < e.N) {
                     float* c = (float*)e.C + (int64_t)m * e.N + n;
                     f32x4 o = *(f32x4*)c;
                     const f32x4 wv = *(const f32x4*)(ro.w + n);
@@ -510,10 +523,10 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
         for (int j = 0; j < MT; ++j) {
             float v[4] = {acc[t][j][0], acc[t][j][1], acc[t][j][2], acc[t][j][3]};
             if constexpr (EXPERTS) if (ex.over == EXPERTS_GATED) {
-                store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+                if (mine) store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 8 * half + 4 * g, v);
                 continue;
             }
-            epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 4 * g, v);
+            if (mine) epilogue4(e, 16 * j + r, (tile0 + t) * 16 + 8 * half + 4 * g, v);
         }
 }
 
@@ -833,9 +846,25 @@ extern "C" int li_tile_weight(const void* W, void* out, int dt, int N, int K, hi
 
 // ro (may be null; mode EPI_ADD, at most 16 rows): RowsOut, with li_gemv_tiled_blocks(...) partial sums a
 // row.  rsc (may be null; at most 16 rows): RowScale.
-static void gemv_tiled_shape(int M, int N, int K, int& nt, int& kw, int& blocks) {
+// nt -1: half a tile a workgroup (at most 8 rows).  plain: no experts and neither half of a norm.
+static void gemv_tiled_shape(int M, int N, int K, int& nt, int& kw, int& blocks, bool plain = false) {
     const int n_tiles = (N + 15) / 16;
     const int mt = (M + 15) / 16;
+    // Half a tile a workgroup.  Up to 128 tiles it gives twice as many CUs a workgroup (us with whole tiles and halves:
+    // 2,048 x 2,048 at 1 and 8 rows 4.1 and 3.9, 4.5 and 4.3; 2,048 x 8,192 10.3 and 8.4, 12.1 and 9.8; 2,048 x 18,432 20.5 and
+    // 15.2, 23.0 and 17.7); from 129 to 255 a second round of half workgroups costs more than it gives (2,176 x 8,192 9.8 and 11.0).
+    // Beyond, one row gains from finer shares (4,096 x 4,096 8.8 and 8.2, 12,544 x 4,096 21.1 and 19.3, 28,672 x 4,096 41.1 and
+    // 39.2, 128,256 x 4,096 166 and 163), two and three where W is neither tall nor long (4,096 x 8,192 14.8 and 13.6, 6,144 x
+    // 4,096 11.5 and 10.8, 12,544 x 4,096 20.9 and 19.5; but 4,096 x 14,336 21.7 and 22.6, 28,672 x 4,096 39.9 and 40.3): a
+    // workgroup fetches all rows of X, so halves fetch them twice as often.  Not where a norm rides along: every workgroup fetches
+    // the partial sums of squares of all that made them (a chat of one sequence on the 8B shape 82.6 ms, with halves 83.1).
+    if (nt == 0 && M <= 8 && (n_tiles <= 128 || (plain && n_tiles >= 256 && (M == 1 || (M <= 3 && n_tiles <= 800 && K <= 8192)))))
+        nt = -1;
+    if (nt < 0) {
+        blocks = 2 * n_tiles;
+        if (kw <= 0) kw = n_tiles <= 128 || (K >= 8192 && n_tiles <= 512) ? 8 : 4;
+        return;
+    }
     if (nt <= 0) nt = (mt >= 2 || (M > 12 && N >= 6144)) ? 2 : 1;            // measured on MI355X (16 rows, 6,144 x 4,096: 14.5 against 16.3 us)
     if (mt >= 3) nt = 2;
     blocks = (n_tiles + nt - 1) / nt;
@@ -868,12 +897,12 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     if (rc) return rc;
     const int mt = (M + 15) / 16;
     int blocks = 0;
-    gemv_tiled_shape(M, N, K, nt, kw, blocks);
-    if (kw < 2) return LI_BAD_ARG;
+    gemv_tiled_shape(M, N, K, nt, kw, blocks, !EB::chosen_only && !ro && !rsc);
+    if (kw < 2 || (nt < 0 && M > 8)) return LI_BAD_ARG;
     const RowsOut no_out{};
     const RowScale no_scale{};
-#define LAUNCH(T, NT, MT, KW) \
-    gemv_tiled_kernel<T, NT, MT, KW, EB><<<blocks, 64 * KW, 0, stream>>>((const T*)X, (const T*)Wt, K, e, \
+#define LAUNCH(T, NT, MT, KW, ...) \
+    gemv_tiled_kernel<T, NT, MT, KW, EB __VA_OPT__(,) __VA_ARGS__><<<blocks, 64 * KW, 0, stream>>>((const T*)X, (const T*)Wt, K, e, \
                                                                      ro ? *ro : no_out, rsc ? *rsc : no_scale, xg, ex)
 #define PICK_KW(T, NT, MT)                                \
     do {                                                  \
@@ -883,7 +912,10 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     } while (0)
 #define PICK(T)                                           \
     do {                                                  \
-        if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
+        if (nt < 0 && kw == 8) LAUNCH(T, 1, 1, 8, true);  \
+        else if (nt < 0 && kw == 4 && !EB::chosen_only) LAUNCH(T, 1, 1, 4, true); \
+        else if (nt < 0) return LI_BAD_ARG;               \
+        else if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
         else if (mt == 1 && nt == 2) PICK_KW(T, 2, 1);    \
         else if constexpr (!EB::chosen_only) { \
             if (mt == 2 && nt == 1) PICK_KW(T, 1, 2);     \

@@ -960,7 +960,7 @@ def untile(w: Tensor) -> torch.Tensor:
 
 
 def gemv_tiled(x, w: Tensor, mode=EPI_STORE, out_dtype=None, nt=0, kw=0):
-    """gemv_tiled with a chosen shape of workgroup (for tuning and tests)."""
+    """gemv_tiled with a chosen shape of workgroup (for tuning and tests; ``nt`` -1: half a tile of W's rows a workgroup)."""
     m, k = x.shape
     n = w.logical[0]
     n_out = n // 2 if mode in GATED else n

@@ -308,6 +308,28 @@ def test_linear_tiled_weights(ops, M, N, K, dt):
 
 
 @pytest.mark.parametrize("dt", F16S)
+@pytest.mark.parametrize("M", [1, 2, 7, 8])
+@pytest.mark.parametrize("N,K", [(8, 32), (16, 64), (24, 96), (100, 544), (2048, 1056), (2050, 160), (4096, 8192)])
+def test_half_tiles(ops, M, N, K, dt):
+    """gemv_tiled with half a tile of W's rows a workgroup: odd numbers of steps, a last tile of less than half its rows, every
+    epilogue; the same sums of W's rows as with whole tiles but for the order of K (K sums in float32: 2e-4 as above)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(dt).to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV)
+    res = torch.randn(M, N, generator=g).to(DEV)
+    wt = ops.tile_weight(w)
+    for kw in (4, 8):
+        for mode in (0, 2, 4):
+            ref = _linear_ref(x, w, mode)
+            out = ops.gemv_tiled(x, wt, mode, torch.float32, -1, kw)
+            assert (out.double() - ref).abs().max().item() < 2e-4 * (1 + ref.abs().max().item()), (kw, mode)
+    out = ops.linear(x, wt, 1, out=res.clone())              # (whichever the rule takes)
+    assert (out.double() - _linear_ref(x, w, 1, res)).abs().max().item() < 2e-4 * 6
+    with pytest.raises(ops.KernelError):
+        ops.gemv_tiled(torch.zeros(9, K, dtype=dt, device=DEV), wt, nt=-1)
+
+
+@pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M,N,K", [(129, 72, 32), (130, 256, 64), (257, 200, 160), (300, 1000, 96), (511, 528, 96), (384, 1024, 256)])
 def test_tiled_products_write_whole_rows(ops, M, N, K, dt):
     """The epilogues that store whole rows of a tile, 16 bytes a lane, beside the ones that go through it quad by quad (taken
