@@ -45,38 +45,48 @@ __device__ __forceinline__ void to_operand16(f32x4& v) {
 // finished one in LDS, where a wave per 16 x 16 tile adds them up in ascending order: K is shared by the waves and the sum
 // is still taken in one order.  Bound by the stream of W: 128,256 x 2,048 at 3 rows 180 us, 5.8 TB/s (gemm_fma: 942 us);
 // 16,384 x 2,048 27 us, 5.0 TB/s (222); short products end a few us after their stream (2,048 x 2,048 9.7 us, 201 before;
-// 2,048 x 8,192 28, 862 before).  U steps of 16 k whose loads go out together: 4, so that eight waves fit a SIMD (with 16
+// 2,048 x 8,192 29, 862 before), and with a workgroup on half the CUs the matrix instructions take as long as the stream.
+// HALF (at most 8 rows of X): 8 rows of W a workgroup.  The lanes of r < 8 hold a chain of them, the others the next chain of the
+// same rows, and likewise the columns of X: of the 16 x 16 sums the two diagonal quarters are the two chains, each in its
+// order.  Twice the workgroups and no instruction more: 2,048 x 2,048 9.8 -> 7.6 us at 3 rows, 2,048 x 8,192 29.0 -> 19.6 (8 rows
+// 32.5 -> 24.0); 4,096 x 4,096 17.5 and 18.3, where every CU has its workgroup without it.  U steps of 16 k whose loads go out together: 4, so that eight waves fit a SIMD (with 16
 // the first of these takes 187 us, the second 37).
 // ===========================================================================
-template <int NT, int MT, int KW, int U>
+template <int NT, int MT, int KW, int U, bool HALF = false>
 __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, Epilogue e) {
     __shared__ f32x4 part[KW][NT * MT][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * 16 * NT, m0 = blockIdx.y * 16 * MT;
+    constexpr int ROWS = HALF ? 8 : 16, CL = HALF ? 2 : 1;               // rows of W, and of X, of a tile; chains of one accumulator
+    const int n0 = blockIdx.x * ROWS * NT, m0 = blockIdx.y * ROWS * MT;
+    const int row = HALF ? r & 7 : r, later = HALF ? r >> 3 : 0;         // (HALF: lanes of r >= 8 hold the same rows in the next chain)
     const float *wp[NT], *xp[MT];                    // rows beyond the last are the last again, and not stored
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wp[t] = W + (int64_t)min(n0 + 16 * t + r, e.N - 1) * K + 4 * g;
+    for (int t = 0; t < NT; ++t) wp[t] = W + (int64_t)min(n0 + 16 * t + row, e.N - 1) * K + 4 * g;
 #pragma unroll
-    for (int j = 0; j < MT; ++j) xp[j] = X + (int64_t)min(m0 + 16 * j + r, e.M - 1) * K + 4 * g;
+    for (int j = 0; j < MT; ++j) xp[j] = X + (int64_t)min(m0 + 16 * j + row, e.M - 1) * K + 4 * g;
     const int chains = (K + CHAIN - 1) / CHAIN;
     constexpr int OWN = (NT * MT + KW - 1) / KW;     // tiles whose sums this wave adds up
     f32x4 total[OWN];
 #pragma unroll
     for (int o = 0; o < OWN; ++o) total[o] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int c0 = 0; c0 < chains; c0 += KW) {
-        const int c = c0 + wave;
+    for (int c0 = 0; c0 < chains; c0 += KW * CL) {
+        const int c = c0 + wave * CL;
         if (c < chains) {
             f32x4 acc[NT][MT];
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int j = 0; j < MT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // (HALF: the first chain of a pair is whole, the second may be short or missing; what it has no steps for it takes
+            // from the row's end, and that is not added)
             const int k0 = c * CHAIN, steps = min(CHAIN, K - k0) >> 4;
+            const int mine = HALF && later ? max(0, min(CHAIN, K - k0 - CHAIN)) >> 4 : steps;
+            const int from = HALF && later ? min(k0 + CHAIN, K - 16) : k0;
             for (int s0 = 0; s0 < steps; s0 += U) {
                 f32x4 a[U][NT], b[U][MT];
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int k = k0 + 16 * min(s0 + u, steps - 1);      // (a step that is not there: the last again, unused)
+                    const int k = from + 16 * max(0, min(s0 + u, mine - 1));      // (a step that is not there: the last again, unused)
 #pragma unroll
                     for (int t = 0; t < NT; ++t) a[u][t] = *(const f32x4*)(wp[t] + k);
 #pragma unroll
@@ -85,6 +95,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restri
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     if (s0 + u < steps) {
+                        if (HALF && s0 + u >= mine) a[u][0] = b[u][0] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                         for (int t = 0; t < NT; ++t) to_operand16(a[u][t]);
 #pragma unroll
@@ -104,12 +115,16 @@ __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restri
                 for (int j = 0; j < MT; ++j) part[wave][t * MT + j][lane] = acc[t][j];
         }
         __syncthreads();
-        const int have = min(KW, chains - c0);
+        const int have = min(KW, (chains - c0 + CL - 1) / CL);
 #pragma unroll
         for (int o = 0; o < OWN; ++o) {
             const int q = wave + o * KW;
             if (q < NT * MT)
-                for (int w = 0; w < have; ++w) total[o] += part[w][q][lane];
+                for (int w = 0; w < have; ++w) {
+                    total[o] += part[w][q][lane];
+                    // rows 4 g + q (g < 2) of column r (r < 8): the second chain's sums lie 40 lanes on
+                    if (HALF && c0 + 2 * w + 1 < chains) total[o] += part[w][q][(lane + 40) & 63];
+                }
         }
         __syncthreads();
     }
@@ -118,7 +133,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restri
         const int q = wave + o * KW;
         if (q < NT * MT) {
             const float v[4] = {total[o][0], total[o][1], total[o][2], total[o][3]};
-            epilogue4(e, m0 + 16 * (q % MT) + r, n0 + 16 * (q / MT) + 4 * g, v);
+            if (!HALF || (r < 8 && g < 2)) epilogue4(e, m0 + 16 * (q % MT) + r, n0 + 16 * (q / MT) + 4 * g, v);
         }
     }
 }
@@ -257,9 +272,19 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
     if (kind == 0) kind = M <= 32 || (M <= 64 && blocks < 1024) || (M <= 128 && blocks <= 256) ? 1 : 2;
     if (kind == 1) {
         const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4), nt = M > 8 && blocks >= 1024 ? 2 : 1;
-        // sixteen waves where half the CUs have no workgroup (2,048 x 8,192 at 3 rows: 28 against 32 us), else eight; two
+        // sixteen waves where half the CUs have no workgroup (2,048 x 8,192 at 3 rows, whole blocks: 28 against 32 us), else eight; two
         // blocks of W a wave where there are workgroups enough (28,672 x 4,096 at 32 rows: 164 against 169 us)
         const int kw = chains <= 4 ? 4 : (mt == 1 && chains >= 16 && blocks <= 256 ? 16 : 8);
+        // up to 128 blocks and 8 rows: half blocks, so that every CU has a workgroup, a wave for each pair of chains
+        if (M <= 8 && blocks <= 128) {
+            const int pairs = (chains + 1) / 2;
+            const unsigned grid = (N + 7) / 8;
+            if (pairs <= 4) gemv_f32_kernel<1, 1, 4, 8, true><<<grid, 256, 0, stream>>>(X, W, K, e);
+            else if (pairs <= 8) gemv_f32_kernel<1, 1, 8, 8, true><<<grid, 512, 0, stream>>>(X, W, K, e);
+            else gemv_f32_kernel<1, 1, 16, 8, true><<<grid, 1024, 0, stream>>>(X, W, K, e);
+            LI_CHECK_LAUNCH();
+            return LI_OK;
+        }
 #define GO(NT, MT, KW, U)                                                                                                       \
     if (nt == NT && mt == MT && kw == KW) {                                                                                     \
         gemv_f32_kernel<NT, MT, KW, U><<<dim3((blocks + NT - 1) / NT, (M + 16 * MT - 1) / (16 * MT)), 64 * KW, 0, stream>>>(X, W, K, e);                             \

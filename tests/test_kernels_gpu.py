@@ -110,6 +110,8 @@ def test_linear_all_kernels_and_epilogues(ops, M, N, K, dt):
 # the edges of the tiles of 16 and 64 rows, of the chains of 256 k, of the steps of 16 and 32, and of the rules by rows and sizes
 F32_CASES = [(1, 1, 16), (3, 33, 48), (8, 16400, 256), (9, 16400, 272), (16, 130, 4352), (17, 257, 528), (33, 64, 1040), (40, 16400, 288),
              (64, 100, 4096), (65, 64, 32), (100, 200, 2064), (128, 4112, 512), (129, 130, 304), (300, 514, 8208)]
+# half blocks: chains that are single, short, missing beside the last; one to sixteen pairs and more than one round of them
+F32_CASES += [(1, 8, 256), (2, 7, 272), (8, 2048, 768), (7, 2050, 2320), (5, 100, 4112), (8, 40, 8448), (4, 64, 16400)]
 
 
 @pytest.mark.parametrize("M,N,K", F32_CASES)
