@@ -148,7 +148,7 @@ __global__ void rope_store_kernel(const float* __restrict__ qkv, int row_stride,
     int64_t page = 0;
     if (K > 0) page = page_table[(int64_t)tok_slot[t] * max_pages + p / PAGE];
     const int tp = p % PAGE;
-    for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
+    for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < n_pairs; i += blockDim.x * gridDim.y) {
         const int head = i / half, j = i - head * half;
         int d0, d1;
         bool rotate = false;
@@ -192,7 +192,10 @@ extern "C" int li_rope_store(const float* qkv, int row_stride, const float* inv_
         row_stride < (H + 2 * K) * hd)
         return LI_BAD_ARG;
     if (K > 0 && (hd % 16 != 0)) return LI_UNSUPPORTED;
-    dim3 grid(n_tokens), block(256);
+    // few tokens: a token's pairs over several workgroups, since a thread's pairs come one after the other (a sine and cosine each;
+    // 3 tokens of 32 + 16 heads of 64: 6.8 -> 4.5 us)
+    const int64_t n_pairs = (int64_t)(H + 2 * K) * (hd / 2);
+    dim3 grid(n_tokens, n_tokens < 256 ? (unsigned)((n_pairs + 255) / 256 < 64 ? (n_pairs + 255) / 256 : 64) : 1u), block(256);
 #define LAUNCH(T)                                                                                        \
     rope_store_kernel<T><<<grid, block, 0, stream>>>(qkv, row_stride, inv_freq, rotary_dim, half_pairing, \
                                                      pos, tok_slot, page_table, max_pages, page_stride, (T*)q_out, \
