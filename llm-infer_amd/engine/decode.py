@@ -42,7 +42,7 @@ class PlainDecodeRunner:
         self.engine, self.sampler = engine, sampler
 
     def run(self, slots, tokens, may_follow: bool = False):
-        logits = self.engine.step(slots, [[t] for t in tokens])
+        logits = self.engine._step(slots, [[t] for t in tokens], None, record=False)
         slot_dev = torch.tensor(slots, dtype=torch.int32, device=self.engine.device)
         return self.sampler.sample(logits, slot_dev, self.engine.cache).tolist()
 

@@ -57,7 +57,7 @@ class Engine:
         self._graphs = {}
         self._graph_bufs = None
         self.decode_counts = {"eager": 0, "recorded": 0, "replayed": 0}      # what the recorded-step runner did
-        # short prompts are recorded too (engine/prefill.py); False runs every prefill step eagerly
+        # short prompts, and steps of one token, are recorded too (engine/prefill.py); False runs every step that is called for by itself eagerly
         self.record_prefill = True
         self._prefill = None
 
@@ -124,10 +124,13 @@ class Engine:
         """slots[i]: a held slot; tokens[i]: that sequence's next tokens (at least one);
         want[i]: places among these tokens whose logits are returned (default: the last).
         Returns float32 [sum(len(want[i])), vocab] in the order of the sequences and of want."""
+        return self._step(slots, tokens, want, self.record_prefill)
+
+    def _step(self, slots, tokens, want, record: bool) -> torch.Tensor:
         ctx = self.prepare(slots, tokens, want, upload=False)
         try:
             logits = None
-            if self.record_prefill:
+            if record:
                 if self._prefill is None:
                     from .prefill import PrefillRecorder
                     self._prefill = PrefillRecorder()

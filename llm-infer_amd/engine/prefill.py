@@ -14,6 +14,10 @@ graph, as for decoding.  The reference replays a recorded graph per token in the
 
 Only parts that say so are recorded (``prefill_recordable``): a part that plans on the host from the step's
 lengths (``ctx.host_qlens``) would have its plan frozen into the graph.
+
+A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on every model that
+the runner records (a decode step plans nothing on the host); its key holds the bucket of context lengths too.  An
+eager one takes the host 0.7 to 0.95 ms on models of four layers, the device 0.35 to 0.6.
 """
 from __future__ import annotations
 
@@ -21,8 +25,8 @@ import numpy as np
 import torch
 
 from ..kernels import ops
-from .decode import batch_bucket, recording
-from .step import StepShared
+from .decode import _GraphContext, batch_bucket, recording
+from .step import StepShared, split_bucket
 
 MAX_TOKENS = 512          # a longer step keeps the device busy longer than the host needs to enqueue it
 MAX_SEQS = 16
@@ -52,8 +56,10 @@ class PrefillRecorder:
     def takes(self, eng, ctx) -> bool:
         """A step of whole prompts (or chunks of them) that is small enough, on a model whose parts can all
         be recorded."""
-        if ctx.is_decode or ctx.n_want == 0 or ctx.n_tokens > MAX_TOKENS or ctx.n_seqs > MAX_SEQS:
+        if ctx.n_want == 0 or ctx.n_tokens > MAX_TOKENS or ctx.n_seqs > MAX_SEQS:
             return False
+        if ctx.is_decode:
+            return eng.model.recordable()
         if getattr(self, "_model_ok", None) is None:
             model = eng.model
             mixers = [m for ms in model.layer_mixers for m in ms]
@@ -96,6 +102,26 @@ class PrefillRecorder:
         put("tile_q0", tile_q0, 1 << 30)                  # a tile that begins beyond its sequence does nothing
         return packed
 
+    @staticmethod
+    def _fill_decode(ctx, rows, wants, scratch):
+        """The same for a step of one token a sequence: tokens, positions, contexts and slots of ``rows`` rows, wanted rows.
+        Rows beyond the sequences are idle ones on the scratch slot, with a context of one token."""
+        packed = np.zeros(4 * rows + wants, dtype=np.int32)
+        n, at = ctx.n_seqs, packed[:4 * rows].reshape(4, rows)
+        at[0, :n], at[1, :n] = ctx.host_tokens, ctx.host_lens_before
+        at[2] = at[1] + 1
+        at[3, :n], at[3, n:] = ctx.host_slots, scratch
+        packed[4 * rows:4 * rows + ctx.n_want] = ctx.host_want_rows
+        return packed
+
+    @staticmethod
+    def _decode_context(buf, rows, wants, bucket):
+        names = ("tokens", "pos", "ctx", "slots")
+        fields = {name: buf[i * rows:(i + 1) * rows] for i, name in enumerate(names)}
+        ctx = _GraphContext(dict(fields, rows=buf[4 * rows:]), rows, bucket)
+        ctx.n_want, ctx.want_rows = wants, buf[4 * rows:4 * rows + wants]
+        return ctx
+
     # -- the step --------------------------------------------------------------------
     def run(self, eng, ctx):
         """The logits of the step [n_want, vocab], or None if this step is to be run eagerly (the first time
@@ -103,25 +129,33 @@ class PrefillRecorder:
         rows = batch_bucket(ctx.n_tokens, MAX_TOKENS)
         seqs = batch_bucket(ctx.n_seqs, MAX_SEQS)
         wants = batch_bucket(ctx.n_want, rows)
-        key = (rows, seqs, wants)
+        bucket = split_bucket(ctx.max_ctx) if ctx.is_decode else None
+        key = (rows, seqs, wants, bucket)
         entry = self.graphs.pop(key, None)
         if entry is None:
             self.graphs[key] = "seen"
             self.counts["eager"] += 1
             self._trim()
             return None
-        layout, total = self._layout(rows, seqs, wants)
+        if ctx.is_decode:
+            packed = self._fill_decode(ctx, rows, wants, eng.cache.scratch_slot)
+        else:
+            layout, total = self._layout(rows, seqs, wants)
+            packed = self._fill(ctx, layout, total, eng.cache.scratch_slot)
         if key not in self._buffers:
-            self._buffers[key] = torch.zeros((total,), dtype=torch.int32, device=eng.device)
+            self._buffers[key] = torch.zeros((len(packed),), dtype=torch.int32, device=eng.device)
         buf = self._buffers[key]
-        buf.copy_(torch.from_numpy(self._fill(ctx, layout, total, eng.cache.scratch_slot)))
+        buf.copy_(torch.from_numpy(packed))
         if entry == "seen":
-            fields = {name: buf[at:at + n] for name, (at, n) in layout.items()}
-            tiles = {"tile_seq": fields.pop("tile_seq"), "tile_q0": fields.pop("tile_q0"), "n_tiles": layout["tile_seq"][1]}
             graph = torch.cuda.CUDAGraph()
             with recording(graph):
-                rec = _RecordedContext(fields, rows, seqs, wants, eng.device)
-                rec.shared(ops.PREFILL_TILES_KEY, lambda: tiles)
+                if ctx.is_decode:
+                    rec = self._decode_context(buf, rows, wants, bucket)
+                else:
+                    fields = {name: buf[at:at + n] for name, (at, n) in layout.items()}
+                    tiles = {"tile_seq": fields.pop("tile_seq"), "tile_q0": fields.pop("tile_q0"), "n_tiles": layout["tile_seq"][1]}
+                    rec = _RecordedContext(fields, rows, seqs, wants, eng.device)
+                    rec.shared(ops.PREFILL_TILES_KEY, lambda: tiles)
                 logits = eng.model.forward(rec, eng.cache)
             entry = (graph, logits)
             self.counts["recorded"] += 1

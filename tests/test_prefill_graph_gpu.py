@@ -96,3 +96,32 @@ def test_generation_through_recorded_prompts_and_steps(tmp_path):
         for p, w in zip(prompts, want):
             assert eng.generate([p], max_new_tokens=6, temperature=0.0) == [w]
     assert eng._prefill.counts["replayed"] >= 4
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_recorded_single_token_steps_give_the_eager_logits(dtype, tmp_path):
+    """Steps of one token for each sequence, called for by themselves: eager, recorded and replayed, with idle rows, across a
+    bucket of context lengths, with sequences that change between replays; the eager engine runs the same rows."""
+    import llm_infer_amd
+    folder, _ = _model(tmp_path, dict(TINY_A, max_position_embeddings=1024), "bfloat16")
+    eager = llm_infer_amd.load(folder, dtype=dtype, max_tokens=8192)
+    eager.record_prefill = False
+    rec = llm_infer_amd.load(folder, dtype=dtype, max_tokens=8192)
+    g = torch.Generator().manual_seed(6)
+    lens = (3, 64, 65, 250, 7)
+    prompts = [torch.randint(0, TINY_A["vocab_size"], (n,), generator=g).tolist() for n in lens]
+    slots = {e: [e.alloc_slot() for _ in lens] for e in (eager, rec)}
+    for e in (eager, rec):
+        e.step(slots[e], prompts)
+    for which in ([0], [0, 1, 2, 3, 4], [3, 1, 4], [2, 0]):
+        for step in range(7):
+            toks = torch.randint(0, TINY_A["vocab_size"], (len(which),), generator=g).tolist()
+            want = None if step % 3 else [[0] if i % 2 == 0 else [] for i in range(len(which))]
+            a, b = (e.step([slots[e][i] for i in which], [[t] for t in toks], want) for e in (eager, rec))
+            assert a.shape == b.shape
+            if dtype == "float32":
+                assert torch.equal(a, b), (which, step)
+            else:
+                # other rows in the step, so other kernels: equal up to the rounding of 16-bit steps
+                assert (a - b).abs().max().item() < 0.05 * a.std().item(), (which, step)
+    assert rec._prefill.counts["replayed"] >= 10
