@@ -10,6 +10,7 @@ from ..config.spec import ModelSpec
 from ..kernels import ops
 from ..parts.base import Part, cache_specs_of, collect_params
 from ..parts.block import SubLayer
+from ..parts.norm import RMSNorm
 from ..registry import lookup
 
 
@@ -155,6 +156,14 @@ class DecoderModel(Part):
                 for e in self.schedule for m in self.layer_mixers[e.layer]
                 for j, spec in enumerate(cache_specs_of(m))] + self._embedding_specs()
 
+    def _norms_of_entry(self, i) -> list:
+        """The RMS norms (weight, eps, type) that read the residual stream as the layer of schedule entry ``i`` begins, where
+        the layer says so (``input_norms``) and nothing rewrites the stream ahead of it: at most two, the others run by themselves."""
+        if i >= len(self.schedule) or self._before[i] is not None:
+            return []
+        asks = getattr(self.layers[self.schedule[i].layer], "input_norms", None)
+        return [(n.weight, n.eps, dt) for n, dt in (asks() if asks else ()) if isinstance(n, RMSNorm) and n.weight is not None][:2]
+
     # -- the forward pass of one step ---------------------------------------
     def forward(self, ctx, cache) -> torch.Tensor:
         """Runs the step's tokens through the schedule; returns float32 logits [n_want, vocab]."""
@@ -167,9 +176,12 @@ class DecoderModel(Part):
             # the stream's values side by side: the embedding's output, then the result of every run that an
             # ``after`` part follows (the run works in place on the row that the part before it has written)
             history = torch.empty((self._n_after + 2,) + tuple(x0.shape), dtype=torch.float32, device=x0.device)
-            history[0].copy_(x0)
-            history[1].copy_(x0)
-            x, n_hist = history[1], 1
+            x, n_hist, norms = history[1], 1, self._norms_of_entry(0)
+            if norms and ops.average_norms_fit(x0, None, x, norms):
+                ops.average_norms(x0.unsqueeze(0), 1, None, x, norms, also=history[0])
+            else:
+                history[0].copy_(x0)
+                x.copy_(x0)
         entered = False              # the layer before has taken what this entry's ``before`` part adds along
         for i, e in enumerate(self.schedule):
             if entered:
@@ -198,7 +210,9 @@ class DecoderModel(Part):
                 layer.forward(x, ctx, views, e.cache_from is None)
             if self._after[i] is not None:
                 n_hist += 1                      # x is history[n_hist - 1], now a finished value of the stream
-                x = self.stream_parts[self._after[i]].forward_after(history, n_hist, history[n_hist], ctx)
+                part = self.stream_parts[self._after[i]]
+                norms = self._norms_of_entry(i + 1) if getattr(part, "takes_norms", False) else ()
+                x = part.forward_after(history, n_hist, history[n_hist], ctx, **({"norms": norms} if norms else {}))
         if ctx.n_want == 0:
             return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=x.device)
         h = self.final_norm.forward(x, ctx.want_rows)

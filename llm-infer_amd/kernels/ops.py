@@ -170,13 +170,10 @@ def prepared_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype):
     """The norm of all rows of ``x`` if the product that last added into ``x`` has taken it already (with K
     split, the kernel that adds the partial sums has the finished rows in its hands): same weight tensor,
     same eps and type, and nothing has written to ``x`` since; else None."""
-    rec = getattr(x, "_li_normed", None)
-    if rec is None:
-        return None
-    normed, weight, rec_eps, version = rec
-    if weight is not w or rec_eps != eps or version != x._version or normed.dtype != out_dtype or normed.shape != x.shape:
-        return None
-    return normed
+    for normed, weight, rec_eps, version in getattr(x, "_li_normed", None) or ():
+        if weight is w and rec_eps == eps and version == x._version and normed.dtype == out_dtype and normed.shape == x.shape:
+            return normed
+    return None
 
 
 # (the weight tensor says which norm it is: a layer norm that a pass has taken along is found in the same way)
@@ -440,7 +437,7 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
                                 ctypes.byref(rsc) if rsc is not None else None, _stream()),
                "gemm_wreg")
         if na is not None:
-            out._li_normed = (normed, nxt, eps, out._version)
+            out._li_normed = [(normed, nxt, eps, out._version)]
         return out
     if kind.startswith("f32"):                                 # "f32[:<kernel>]" (a test's choice)
         _need(f32_ok, "gemm_f32: float32 operands, K a multiple of 16")
@@ -1068,7 +1065,7 @@ def layernorm_add(x, y, weight, bias, eps: float, next_norm=None) -> torch.Tenso
         normed = torch.empty(x.shape, dtype=n_dt, device=x.device)
     _layernorm_add(x, y, weight, bias, eps, nw, nb, n_eps, normed)
     if normed is not None:
-        x._li_normed = (normed, nw, float(n_eps), x._version)
+        x._li_normed = [(normed, nw, float(n_eps), x._version)]
     return x
 
 
@@ -1785,6 +1782,39 @@ def depth_average(history: torch.Tensor, n: int, weights: torch.Tensor, out: tor
     return out
 
 
+class _RowNorm(ctypes.Structure):
+    _fields_ = [("w", c_void_p), ("out", c_void_p), ("eps", c_float), ("dt", c_int)]
+
+
+def average_norms(history: torch.Tensor, n: int, weights, out: torch.Tensor, norms, also=None) -> torch.Tensor:
+    """``depth_average`` (``weights`` None: the rows of ``history`` [1, T, width] as they are) that also takes the RMS norms which
+    read the finished rows next, ``norms``: up to two (weight, eps, dtype).  ``prepared_rmsnorm`` finds them as long as nothing
+    writes into ``out``.  ``also``: a second tensor that receives the rows."""
+    _dev(history, weights, out, also, *(w for w, _, _ in norms))
+    rows, d = out.shape
+    _need(history.dtype == torch.float32 and history.dim() == 3 and 1 <= n <= history.shape[0], "average_norms: float32 [runs, T, width]")
+    _need(weights is not None or n == 1, "average_norms: weights for more than one term")
+    _need(weights is None or (weights.dtype == torch.float32 and weights.numel() >= n), "average_norms: a float32 weight for every term")
+    for t in (out,) + ((also,) if also is not None else ()):
+        _need(t.dtype == torch.float32 and tuple(t.shape) == tuple(history.shape[1:]), "average_norms out: float32 [T, width]")
+        _drop_row_stats(t)
+    _need(1 <= len(norms) <= 2 and all(w.dtype == torch.float32 and w.shape == (d,) for w, _, _ in norms), "average_norms: one or two float32 weights [width]")
+    made = [torch.empty(out.shape, dtype=dt, device=out.device) for _, _, dt in norms]
+    recs = [_RowNorm(w.data_ptr(), m.data_ptr(), eps, DT[m.dtype]) for (w, eps, _), m in zip(norms, made)] + [_RowNorm()]
+    _check(hybrid().li_average_norms(_ptr(history), c_int64(history.stride(0)), _ptr(weights), n, _ptr(out), _ptr(also), rows, d,
+                                     ctypes.byref(recs[0]), ctypes.byref(recs[1]), _stream()), "average_norms")
+    out._li_normed = [(m, w, float(eps), out._version) for m, (w, eps, _) in zip(made, norms)]
+    return out
+
+
+def average_norms_fit(history, weights, out, norms) -> bool:
+    """Whether ``average_norms`` takes these: rows of a multiple of 4 and at most 8,192, addresses of 16 bytes."""
+    d = out.shape[-1]
+    tensors = [history, out] + [w for w, _, _ in norms]
+    return (1 <= len(norms) <= 2 and d % 4 == 0 and d <= 8192 and all(t.data_ptr() % 16 == 0 for t in tensors)
+            and all(w.dtype == torch.float32 and w.shape == (d,) for w, _, _ in norms))
+
+
 def softcap(x: torch.Tensor, cap: float) -> torch.Tensor:
     """x <- cap * tanh(x / cap) in place (float32)."""
     _dev(x)
@@ -2172,7 +2202,7 @@ def rmsnorm_add(x, y, weight, eps: float, bias=None, next_norm=None, also=None) 
                                        _ptr(add_rows), _ptr(add_vec), _ptr(nw), c_float(n_eps), _ptr(normed), DT[n_dt], _stream()),
                "rmsnorm_add")
     if normed is not None:
-        x._li_normed = (normed, nw, float(n_eps), x._version)
+        x._li_normed = [(normed, nw, float(n_eps), x._version)]
     return x
 
 

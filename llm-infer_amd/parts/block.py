@@ -102,6 +102,10 @@ class ParallelBlock(Block):
             if s.norm is None or s.post_norm is not None:
                 raise ValueError("a parallel block has one norm before each part and none after it")
 
+    def input_norms(self):
+        """What reads the residual stream first: (norm, type of its result) of every branch."""
+        return [(s.norm, torch.float32 if getattr(s.part, "reads_float32", False) else s.norm.dtype) for s in self.sublayers]
+
     def forward(self, x, ctx, cache_views, owns_cache=True):
         views = iter(cache_views)
         ops.expect_norm(x, None)                 # the rows are complete only after the last part: no norm rides along

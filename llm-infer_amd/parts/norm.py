@@ -40,7 +40,8 @@ class RMSNorm(Part):
         it on to ``ops.linear`` untouched (``takes_lazy_norm``); then, where the product before has prepared
         this norm (a decode step), an ``ops.LazyNorm`` is returned and the product that reads it finishes it."""
         if out_dtype is not None and out_dtype != self.dtype:
-            return ops.rmsnorm(x, self.weight, self.eps, out_dtype, rows)
+            ready = ops.prepared_rmsnorm(x, self.weight, self.eps, out_dtype) if rows is None else None
+            return ready if ready is not None else ops.rmsnorm(x, self.weight, self.eps, out_dtype, rows)
         if lazy and rows is None:
             deferred = ops.lazy_rmsnorm(x, self.weight, self.eps, self.dtype)
             if deferred is not None:

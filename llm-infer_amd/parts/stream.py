@@ -81,8 +81,13 @@ class DepthAverage(Part):
     def bind(self, tensors):
         self.weight = tensors[self.name]
 
-    def forward_after(self, history, n, out, ctx):
-        """``history`` float32 [runs, T, width] of which the first ``n`` hold X_0 .. X_{n-1}; writes ``out``."""
+    takes_norms = True          # forward_after accepts ``norms``
+
+    def forward_after(self, history, n, out, ctx, norms=()):
+        """``history`` float32 [runs, T, width] of which the first ``n`` hold X_0 .. X_{n-1}; writes ``out``.  ``norms``: up to two
+        RMS norms (weight, eps, type) that read it next, taken in the same pass where its kernel takes them."""
         if n != self.n_terms:
             raise ValueError(f"depth average over {self.n_terms} terms after {n} values of the stream")
+        if norms and ops.average_norms_fit(history, self.weight, out, norms):
+            return ops.average_norms(history, n, self.weight, out, norms)
         return ops.depth_average(history, n, self.weight, out)

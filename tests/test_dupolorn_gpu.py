@@ -184,6 +184,33 @@ def test_scalar_norm_softcap_and_depth_average(lib):
         assert (dev[:5].cpu() - hist[:5]).abs().max() == 0
 
 
+@pytest.mark.parametrize("rows,width", [(1, 4), (9, 64), (3, 260), (8, 2048), (2, 4100), (3, 8192)])
+def test_average_with_the_norms_that_follow(lib, rows, width):
+    """Average and norms in one pass are, bit for bit, the separate kernels', for one norm and two of every type; a write into the
+    rows makes them void."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + width)
+    hist = torch.randn(5, rows, width, generator=g).to(DEV)
+    w = torch.randn(4, generator=g).to(DEV)
+    nw = [(torch.randn(width, generator=g)).to(DEV) for _ in range(2)]
+    for n, weights in ((4, w), (1, w), (1, None)):
+        for types in ((torch.float32, torch.float16), (torch.bfloat16, torch.float32), (torch.float16,)):
+            norms = [(a, 1e-5 * (i + 1), dt) for i, (a, dt) in enumerate(zip(nw, types))]
+            ref = hist[0].clone() if weights is None else ops.depth_average(hist, n, weights, torch.empty_like(hist[0]))
+            out, also = torch.empty_like(ref), torch.empty_like(ref)
+            src = hist[:1] if weights is None else hist
+            assert ops.average_norms_fit(src, weights, out, norms)
+            ops.average_norms(src, n, weights, out, norms, also)
+            assert torch.equal(out, ref) and torch.equal(also, ref)
+            for a, eps, dt in norms:
+                assert torch.equal(ops.prepared_rmsnorm(out, a, eps, dt), ops.rmsnorm(ref, a, eps, dt)), (n, types, dt)
+                assert ops.prepared_rmsnorm(out, a, eps * 3, dt) is None
+            out.add_(1.0)
+            assert all(ops.prepared_rmsnorm(out, a, eps, dt) is None for a, eps, dt in norms)
+    odd = torch.empty(rows, 75, device=DEV)
+    assert not ops.average_norms_fit(odd, None, odd, [(torch.ones(75, device=DEV), 1e-5, torch.float32)])
+
+
 @pytest.mark.parametrize("taps", [1, 2, 3, 6])
 def test_convolution_ahead_of_a_mixer(lib, taps):
     """The convolution alone: whole, in portions shorter than its reach, and one token at a time."""
