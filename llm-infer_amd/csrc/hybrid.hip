@@ -696,11 +696,67 @@ __global__ __launch_bounds__(256) void small_logits_kernel(const T* __restrict__
     }
 }
 
+// The same sums, bit for bit, for rows of up to 4,096 elements in whole quads: a wave takes TOK tokens, a lane four neighbouring
+// partial sums of the 256, so that the operands come 16 and 8 bytes at a time, h once for JB outputs, and only lanes exchange sums.
+// Bound by its loads' latency for few tokens, by the weights' way from L2 for many: 2,253 tokens x 9 outputs of 4,096 75 -> 21 us,
+// 8,000 x 16 459 -> 63, 300 x 9 12.0 -> 8.7, 4 tokens 4.15 -> 4.0.
+template <class T, int TOK, int JB>
+__global__ void small_logits_wave_kernel(const T* __restrict__ h, const float* __restrict__ w, float* __restrict__ out,
+                                         const float* __restrict__ bias, int n_rows, int width, int n) {
+#pragma clang fp contract(off)
+    struct alignas(4 * sizeof(T)) Quad { T v[4]; };
+    const int lane = threadIdx.x & 63;
+    const int t0 = (blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * TOK, j0 = blockIdx.y * JB;
+    if (t0 >= n_rows) return;
+    float acc[TOK][JB][4] = {};
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int i = u * 256 + 4 * lane;
+        if (i >= width) break;
+        Quad x[TOK];
+        f32x4 wv[JB];
+#pragma unroll
+        for (int k = 0; k < TOK; ++k) x[k] = *(const Quad*)(h + (int64_t)min(t0 + k, n_rows - 1) * width + i);
+#pragma unroll
+        for (int j = 0; j < JB; ++j) wv[j] = *(const f32x4*)(w + (int64_t)min(j0 + j, n - 1) * width + i);
+#pragma unroll
+        for (int k = 0; k < TOK; ++k)
+#pragma unroll
+            for (int j = 0; j < JB; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const float product = wv[j][q] * to_f32(x[k].v[q]);
+                    acc[k][j][q] += product;
+                }
+    }
+#pragma unroll
+    for (int k = 0; k < TOK; ++k)
+#pragma unroll
+        for (int j = 0; j < JB; ++j) {
+            // a wave of the other kernel holds the partial sums of 16 of these lanes: its exchanges in its order
+#pragma unroll
+            for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) acc[k][j][q] += __shfl_xor(acc[k][j][q], o, WAVE);
+            const float even = acc[k][j][0] + acc[k][j][2], odd = acc[k][j][1] + acc[k][j][3], part = even + odd;
+            float sum = 0.f;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) sum += __shfl(part, 16 * v, WAVE);
+            if (lane == 0 && t0 + k < n_rows && j0 + j < n) out[(int64_t)(t0 + k) * n + j0 + j] = bias ? sum + bias[j0 + j] : sum;
+        }
+}
+
 extern "C" int li_small_logits(const void* h, int dt, const float* w, float* out, const float* bias, int n_rows, int width, int n,
                                hipStream_t stream) {
     if (n_rows <= 0 || n <= 0) return LI_OK;
     if (width <= 0 || n > 65535) return LI_BAD_ARG;
-    if (n_rows >= 256) {                                   // many tokens: four a workgroup share every weight fetched
+    if (width % 4 == 0 && width <= 4096 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)h & (dt == DT_F32 ? 15 : 7)) == 0) {
+        if (n_rows >= 256) {                               // many tokens: two a wave, four outputs at a time
+            DISPATCH_T(dt, (small_logits_wave_kernel<T, 2, 4><<<dim3((n_rows + 7) / 8, (n + 3) / 4), 256, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+        } else {
+            DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1><<<dim3(n_rows, n), 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+        }
+    } else if (n_rows >= 256) {                            // many tokens: four a workgroup share every weight fetched
         dim3 grid((n_rows + 3) / 4, n);
         DISPATCH_T(dt, (small_logits_kernel<T, 4><<<grid, 256, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
     } else {

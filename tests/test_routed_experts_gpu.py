@@ -143,3 +143,24 @@ def test_clamped_activation_by_pairs_in_every_kernel(dtype, E, K, F, counts):
         for force in (None, "wreg:0:0", "wreg:1:0", "wreg:2:0", "wreg:2:1"):
             got = ops.linear_pairs(x.to(DEV), wt, p, ops.EPI_CLAMPGLU, gather, force=force, params=params).cpu()
             assert got.dtype == dtype and bool(((got.double() - ref).abs() <= bound).all()), (gather, force)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 255, 256, 263])
+@pytest.mark.parametrize("width,n", [(4, 1), (260, 4), (2048, 9), (4092, 17), (4096, 3), (4100, 2)])
+def test_router_logits_are_the_same_bits_whatever_the_kernel(rows, width, n):
+    """Rows in whole quads run on a wave each; the same rows one element off their alignment on a workgroup an output: the order of
+    every sum is one and the same (a choice of experts near a tie does not depend on the kernel)."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + width)
+    w, bias = torch.randn(n, width, generator=g).cuda(), torch.randn(n, generator=g).cuda()
+    for dt in (torch.float32, torch.float16, torch.bfloat16):
+        h = torch.randn(rows, width, generator=g).to(dt).cuda()
+        flat = torch.empty(rows * width + 1, dtype=dt, device="cuda")
+        off = flat[1:].view(rows, width)
+        off.copy_(h)
+        for b in (None, bias):
+            got = ops.small_logits(h, w, b)
+            assert torch.equal(got, ops.small_logits(off, w, b))
+            ref = h.double() @ w.double().t() + (0 if b is None else b.double())
+            # float32 sums of `width` products (a pairwise tree of 256 sums of 16): 24 roundings of the terms' magnitudes at most
+            assert ((got.double() - ref).abs() <= 24 * 2.0 ** -24 * (h.double().abs() @ w.double().abs().t() + 1)).all()
