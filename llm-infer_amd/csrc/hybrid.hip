@@ -648,12 +648,52 @@ __global__ void gated_group_norm_kernel(const float* __restrict__ y, const float
         out[(int64_t)t * n + grp * part + i] = from_f32<T>(yr[i] * siluf_(zr[i]) * r * w[grp * part + i]);
 }
 
+// The same, value for value, where a thread has at most V elements: they are fetched together and once, and stay in registers (an
+// exponential and a division each).  8,192 in one group: 4 rows 7.1 -> 5.7 us, 2,253 rows
+// 56 -> 37.
+template <class T, int V>
+__global__ void gated_group_norm_once_kernel(const float* __restrict__ y, const float* __restrict__ zrows, int z_stride,
+                                             int z_col, const float* __restrict__ w, T* __restrict__ out, int n, int groups,
+                                             float eps) {
+    __shared__ float scratch[16];
+    const int t = blockIdx.x, grp = blockIdx.y, part = n / groups;
+    const float* yr = y + (int64_t)t * n + grp * part;
+    const float* zr = zrows + (int64_t)t * z_stride + z_col + grp * part;
+    float v[V], z[V];
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int i = min((int)(threadIdx.x + k * blockDim.x), part - 1);
+        v[k] = yr[i];
+        z[k] = zr[i];
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        v[k] = v[k] * siluf_(z[k]);
+        if ((int)(threadIdx.x + k * blockDim.x) < part) ss += v[k] * v[k];
+    }
+    const float r = 1.f / sqrtf(block_sum(ss, scratch) / (float)part + eps);
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+        const int i = threadIdx.x + k * blockDim.x;
+        if (i < part) out[(int64_t)t * n + grp * part + i] = from_f32<T>(v[k] * r * w[grp * part + i]);
+    }
+}
+
 extern "C" int li_gated_group_norm(const float* y, const float* zrows, int z_stride, int z_col, const float* w, void* out,
                                    int dt, int n_rows, int n, int groups, float eps, hipStream_t stream) {
     if (n_rows <= 0) return LI_OK;
     if (n <= 0 || groups <= 0 || n % groups) return LI_BAD_ARG;
     dim3 grid(n_rows, groups);
     const int threads = n / groups >= 4096 ? 1024 : (n / groups >= 1024 ? 512 : 256);
+    const int pieces = (n / groups + threads - 1) / threads;
+    if (pieces <= 8) {
+#define GO(V) gated_group_norm_once_kernel<T, V><<<grid, threads, 0, stream>>>(y, zrows, z_stride, z_col, w, (T*)out, n, groups, eps)
+        DISPATCH_T(dt, { if (pieces <= 2) GO(2); else if (pieces <= 4) GO(4); else GO(8); });
+#undef GO
+        LI_CHECK_LAUNCH();
+        return LI_OK;
+    }
     DISPATCH_T(dt, (gated_group_norm_kernel<T><<<grid, threads, 0, stream>>>(y, zrows, z_stride, z_col, w, (T*)out, n, groups, eps)));
     LI_CHECK_LAUNCH();
     return LI_OK;

@@ -1,4 +1,5 @@
-"""The state-space recurrence of a prompt by chunks, as products of matrices, against the recurrence in 64 bits."""
+"""The state-space recurrence of a prompt by chunks, as products of matrices, against the recurrence in 64 bits, and the gated norm
+behind it."""
 import types
 
 import pytest
@@ -76,3 +77,18 @@ def test_sizes_that_chunks_do_not_take_are_refused():
         with pytest.raises(ops.KernelError):
             ops.ssm_scan(torch.zeros(3, dv + 2 * N, device=DEV), torch.zeros(3, 1, device=DEV), 0, torch.zeros(1, device=DEV),
                          torch.zeros(1, device=DEV), None, torch.zeros(1, 1, N, dv, device=DEV), ctx, 1, 1, N, dv, seg, True)
+
+
+# elements of a group around what a thread keeps (2, 4 and 8 of them for 256, 512 and 1,024 threads), and beyond that
+@pytest.mark.parametrize("part", [1, 255, 512, 513, 1023, 1024, 1025, 2048, 2049, 4095, 4096, 4097, 8192, 8193])
+@pytest.mark.parametrize("groups", [1, 3])
+def test_gated_norm_of_every_width(part, groups):
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(part + groups)
+    n = part * groups
+    y, rows, w = torch.randn(3, n, generator=g), torch.randn(3, n + 5, generator=g), torch.randn(n, generator=g)
+    got = ops.gated_group_norm(y.to(DEV), rows.to(DEV), 5, w.to(DEV), groups, 1e-4, torch.float32).cpu().double()
+    v = (y.double() * torch.nn.functional.silu(rows[:, 5:].double())).view(3, groups, part)
+    want = (v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-4)).view(3, n) * w.double()
+    # an exponential, a division, a root and four products of 32 bits, and the sum of squares' own rounding: under 16 roundings
+    assert ((got - want).abs() <= 16 * 2.0 ** -24 * want.abs() + 1e-7).all()
