@@ -48,7 +48,7 @@ class PrefillRecorder:
     object, and a reference back would keep both alive until the garbage collector finds the cycle)."""
 
     def __init__(self):
-        self.graphs = {}                   # key -> "seen" | (graph, logits)
+        self.graphs = {}                   # key -> "once" | "seen" | (graph, logits)
         self.counts = {"eager": 0, "recorded": 0, "replayed": 0}
         self._buffers = {}                 # key -> (device buffer, layout)
 
@@ -125,15 +125,17 @@ class PrefillRecorder:
     # -- the step --------------------------------------------------------------------
     def run(self, eng, ctx):
         """The logits of the step [n_want, vocab], or None if this step is to be run eagerly (the first time
-        its key is seen)."""
+        its key is seen, or the second)."""
         rows = batch_bucket(ctx.n_tokens, MAX_TOKENS)
         seqs = batch_bucket(ctx.n_seqs, MAX_SEQS)
         wants = batch_bucket(ctx.n_want, rows)
         bucket = split_bucket(ctx.max_ctx) if ctx.is_decode else None
         key = (rows, seqs, wants, bucket)
         entry = self.graphs.pop(key, None)
-        if entry is None:
-            self.graphs[key] = "seen"
+        # a recording takes some milliseconds: a step of one token is recorded when it comes for the third time (one behind a prompt
+        # and one at a request's end are no loop)
+        if entry is None or (entry == "once" and ctx.is_decode):
+            self.graphs[key] = "once" if entry is None and ctx.is_decode else "seen"
             self.counts["eager"] += 1
             self._trim()
             return None
@@ -169,7 +171,7 @@ class PrefillRecorder:
     def _trim(self):
         while len(self.graphs) > MAX_RECORDED:
             old = next(iter(self.graphs))
-            if self.graphs[old] != "seen":
+            if self.graphs[old] not in ("seen", "once"):
                 torch.cuda.synchronize()             # it may still be running
             del self.graphs[old]
             self._buffers.pop(old, None)
