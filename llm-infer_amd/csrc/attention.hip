@@ -60,6 +60,8 @@ struct AttnExtras {
 template <class T>
 struct WaveAttn {
     typedef typename Vec<T>::v8 v8;
+    static constexpr int ROWS = 32, KF = 2 * KS, VF = DB * 4;
+    typedef f32x16 Scores[2];
     v8 q[KS];
     f32x16 o[DB];
     float m, l;
@@ -186,6 +188,147 @@ struct WaveAttn {
     }
 
     __device__ __forceinline__ float total() const { return l + __shfl_xor(l, 32, WAVE); }
+    // this lane's elements of its row's output
+    __device__ __forceinline__ void lay_down(float* to) const {
+        const int lane = threadIdx.x & 63;
+#pragma unroll
+        for (int blk = 0; blk < DB; ++blk)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int d = 32 * blk + 8 * g + 4 * (lane >> 5);
+                if (d < HD) *(f32x4*)(to + d) = f32x4{o[blk][4 * g], o[blk][4 * g + 1], o[blk][4 * g + 2], o[blk][4 * g + 3]};
+            }
+    }
+};
+
+__device__ __forceinline__ f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0); }
+
+// The same for a decode step whose KV head serves at most 16 query heads, with 16 x 16 x 32 instructions on the same pages: half the
+// rows of a tile, so half the registers for q, scores and output, half the matrix and vector work, and two waves a SIMD
+// without accumulation registers (whose moves were part of every step of the softmax).  Head sizes that are multiples of 32.
+// A row of a score tile stands for whichever key the loads give it: tile X of 32 keys has key 16 (i / 8) + 8 X + 4 (i / 4 % 2) +
+// i % 4 of them in row i, so that a lane group's probabilities of both tiles are, as they lie, the eight keys that a lane
+// group of a page's values holds.
+// 32 / 8 heads of 128, us with tiles of 32 rows and of 16: batch 1 at 500 tokens 7.6 and 6.2, batch 4 at 500 9.1 and 7.7, batch 32 at
+// 250 9.6 and 8.5, batch 48 at 16 to 528 24.3 and 18.8 (in four splits each), batch 8 at 8,160 55.6 and 54.8 (memory); of 64, batch 8
+// at 500 8.3 and 6.8; 16 / 2 heads of 256, batch 32 at 1,000 50 and 21.
+template <class T>
+struct WaveAttn16 {
+    typedef typename Vec<T>::v8 v8;
+    static constexpr int ROWS = 16, KF = 2 * KS, VF = DB * 4, QF = HD >= 32 ? HD / 32 : 1, OF = HD / 16;
+    typedef f32x4 Scores[4];                          // [32 keys][tile]
+    v8 q[QF];
+    f32x4 o[OF];
+    float m, l;
+
+    __device__ __forceinline__ void init(const T* qrow) {
+        const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+        for (int s = 0; s < QF; ++s) {
+            v8 z = {};
+            q[s] = qrow ? *(const v8*)(qrow + 32 * s + 8 * g) : z;
+        }
+#pragma unroll
+        for (int b = 0; b < OF; ++b) o[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        m = -INFINITY;
+        l = 0.f;
+    }
+    __device__ __forceinline__ void load_k(const T* kpage, v8 (&kf)[KF]) const {
+        const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+        const int key = 16 * (i >> 3) + 4 * (i >> 2 & 1) + (i & 3);
+        const T* p = kpage + ((g >> 1) * 64 + key + 32 * (g & 1)) * 8;
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int k = 0; k < QF; ++k) kf[(a * 2 + x) * QF + k] = *(const v8*)(p + ((a * KS + 2 * k) * 64 + 8 * x) * 8);
+    }
+    __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[VF]) const {
+        const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+        const T* p = vpage + ((g >> 1) * 64 + i + 32 * (g & 1)) * 8;
+#pragma unroll
+        for (int d = 0; d < OF; ++d)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) vf[d * 2 + a] = *(const v8*)(p + (((d >> 1) * 4 + 2 * a) * 64 + 16 * (d & 1)) * 8);
+    }
+    __device__ __forceinline__ int key_of(int tile, int r) const {
+        const int g = (threadIdx.x & 63) >> 4;
+        return 32 * (tile >> 1) + 16 * (g >> 1) + 8 * (tile & 1) + 4 * (g & 1) + r;
+    }
+    __device__ __forceinline__ void scores(const v8 (&kf)[KF], Scores& s, int t0, int lo, int hi, float scale2, bool masked,
+                                           float per, float cap, float cap_per, int keep) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            s[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < QF; ++k) s[b] = mfma16(kf[b * QF + k], q[k], s[b]);
+        }
+        if (cap != 0.f) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[b][r] = soft_cap(s[b][r], cap, cap_per);
+        }
+        if (per != 0.f) {
+#pragma unroll
+            for (int b = 0; b < 4; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) s[b][r] = fmaf(-per, (float)(hi - t0 - key_of(b, r)), s[b][r]);
+        }
+        float mx = -INFINITY;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (masked) {
+                    const int t = t0 + key_of(b, r);
+                    s[b][r] = ((t >= lo || t < keep) && t <= hi) ? s[b][r] : -INFINITY;
+                }
+                mx = fmaxf(mx, s[b][r]);
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
+        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE)) * scale2;
+        const float m_new = fmaxf(m, mx), m_safe = (m_new == -INFINITY) ? 0.f : m_new;
+        const float alpha = __builtin_amdgcn_exp2f(m - m_safe);
+        float psum = 0.f;
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                s[b][r] = __builtin_amdgcn_exp2f(fmaf(s[b][r], scale2, -m_safe));
+                psum += s[b][r];
+            }
+        l = l * alpha + psum;
+        m = m_new;
+        if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {
+#pragma unroll
+            for (int b = 0; b < OF; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[b][r] *= alpha;
+        }
+    }
+    __device__ __forceinline__ void mix(const v8 (&vf)[VF], const Scores& s) {
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            v8 pf;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pf[i] = from_f32<T>(s[2 * a + (i >> 2)][i & 3]);
+#pragma unroll
+            for (int d = 0; d < OF; ++d) o[d] = mfma16(vf[d * 2 + a], pf, o[d]);
+        }
+    }
+    __device__ __forceinline__ float total() const {
+        const float half = l + __shfl_xor(l, 16, WAVE);
+        return half + __shfl_xor(half, 32, WAVE);
+    }
+    // this lane's elements of its row's output
+    __device__ __forceinline__ void lay_down(float* to) const {
+        const int g = (threadIdx.x & 63) >> 4;
+#pragma unroll
+        for (int b = 0; b < OF; ++b) *(f32x4*)(to + 16 * b + 4 * g) = o[b];
+    }
 };
 
 // ---------------------------------------------------------------------------
@@ -567,24 +710,24 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void attn_prefill_kernel(
 // query heads: often 4 of the tile's 32): done by the first wave on the whole tile they took as long as two pages.  32 / 8 heads of
 // 128, batch 1: 30 tokens 6.3 -> 5.5 us, 200 tokens in 4 splits 8.9 -> 6.1, 777 in 4 with cap and a gate an element 22.0 -> 12.6;
 // batch 48 at 16 to 530 tokens 22.4 -> 20.7.
-template <class T, int W>
-__global__ __launch_bounds__(64 * W) void attn_decode_kernel(
+template <class T, int W, class A>
+__global__ __launch_bounds__(64 * W, A::ROWS == 16 && HD <= 128 ? 2 : 1) void attn_decode_kernel(
     const T* __restrict__ q, T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     CachePtrs c, const int* __restrict__ seq_slot, const int* __restrict__ seq_ctx, int H, int K, float scale,
     int window, AttnExtras ex) {
     constexpr int OLD = HD + 4;                               // floats from one row's output to the next in LDS
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int b = blockIdx.x, G = H / K, gchunks = (G + 31) / 32;
+    const int b = blockIdx.x, G = H / K, gchunks = (G + A::ROWS - 1) / A::ROWS;
     const int kvh = blockIdx.y / gchunks, gc = blockIdx.y % gchunks;
     const int S = gridDim.z * W, split = blockIdx.z * W + wave;
     const int grid_splits = gridDim.z, grid_split = blockIdx.z;
-    const int hg = gc * 32 + (lane & 31);
+    const int hg = gc * A::ROWS + (lane & (A::ROWS - 1));
     const bool live = hg < G;
     const int h = kvh * G + hg;
     const int ctx = seq_ctx[b];
     const int pos = ctx - 1;
-    WaveAttn<T> a;
+    A a;
     a.init(live ? q + ((int64_t)b * H + h) * HD : nullptr);
     int lo = window > 0 ? max(0, pos - window + 1) : 0;
     if (ex.block > 0) lo = max(lo, pos - pos % ex.block);
@@ -600,8 +743,8 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
     const float scale2 = scale * LOG2E;
     // keys of page p+1 are loaded while the values of page p are mixed, values of page p while
     // its scores are computed
-    typename WaveAttn<T>::v8 kf[2 * KS], vf[DB * 4];
-    f32x16 s[2];
+    typename A::v8 kf[A::KF], vf[A::VF];
+    typename A::Scores s;
     const T* kbase = (const T*)c.k + (int64_t)kvh * k_head_elems(HD);
     const T* vbase = (const T*)c.v + (int64_t)kvh * v_head_elems(HD);
     if (p0 < p1) a.load_k(kbase + (int64_t)table[page_of(p0)] * c.page_stride, kf);
@@ -615,38 +758,24 @@ __global__ __launch_bounds__(64 * W) void attn_decode_kernel(
     }
     // The waves lay the states of the rows that exist down as [wave][row][dim] (maxima and sums behind them), and all threads
     // add them in wave order, four dimensions at a time:  M = max m,  o = sum o_w 2^(m_w - M),  l = sum l_w 2^(m_w - M)
-    const int rows = min(32, G - gc * 32), row = lane & 31;
+    const int rows = min(A::ROWS, G - gc * A::ROWS), row = lane & (A::ROWS - 1);
     float* sm = (float*)smem_raw;
     float* ml = sm + W * rows * OLD;                          // [W][rows][m, l]
     const float sum = a.total();
     if (W == 1 && grid_splits > 1) {                          // one wave's state as it lies, for the merge kernel
         if (!live) return;
         const int64_t slot = ((int64_t)b * H + h) * grid_splits + grid_split;
-        float* po = part_o + slot * HD;
-#pragma unroll
-        for (int blk = 0; blk < DB; ++blk)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * blk + 8 * g + 4 * (lane >> 5);
-                if (d < HD) *(f32x4*)(po + d) = f32x4{a.o[blk][4 * g], a.o[blk][4 * g + 1], a.o[blk][4 * g + 2], a.o[blk][4 * g + 3]};
-            }
-        if (lane < 32) *(f32x2*)(part_ml + slot * 2) = f32x2{a.m, sum};
+        a.lay_down(part_o + slot * HD);
+        if (lane < A::ROWS) *(f32x2*)(part_ml + slot * 2) = f32x2{a.m, sum};
         return;
     }
     if (live) {
-        float* mine = sm + (wave * rows + row) * OLD;
-#pragma unroll
-        for (int blk = 0; blk < DB; ++blk)
-#pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int d = 32 * blk + 8 * g + 4 * (lane >> 5);
-                if (d < HD) *(f32x4*)(mine + d) = f32x4{a.o[blk][4 * g], a.o[blk][4 * g + 1], a.o[blk][4 * g + 2], a.o[blk][4 * g + 3]};
-            }
-        if (lane < 32) *(f32x2*)(ml + (wave * rows + row) * 2) = f32x2{a.m, sum};
+        a.lay_down(sm + (wave * rows + row) * OLD);
+        if (lane < A::ROWS) *(f32x2*)(ml + (wave * rows + row) * 2) = f32x2{a.m, sum};
     }
     __syncthreads();
     for (int i = threadIdx.x; i < rows * (HD / 4); i += 64 * W) {
-        const int rw = i / (HD / 4), d = i % (HD / 4) * 4, h = kvh * G + gc * 32 + rw;
+        const int rw = i / (HD / 4), d = i % (HD / 4) * 4, h = kvh * G + gc * A::ROWS + rw;
         f32x2 st[W];
         float M = -INFINITY, total = 0.f;
         f32x4 o = {0.f, 0.f, 0.f, 0.f};
@@ -876,9 +1005,12 @@ static int launch_decode(const void* q, void* out, float* part_o, float* part_ml
                          const int* seq_ctx, int n_seqs, int H, int K, float scale, int window, int parts,
                          AttnExtras ex, hipStream_t stream) {
     const int G = H / K;
-    dim3 grid(n_seqs, K * ((G + 31) / 32), parts), block(64 * W);
-    const size_t lds = (size_t)W * (G < 32 ? G : 32) * (HD + 4 + 2) * sizeof(float);
-    auto kfn = attn_decode_kernel<T, W>;
+    const bool few = HD % 32 == 0 && G <= 16;                // (more query heads of a KV head, or other head sizes: tiles of 32 rows)
+    const int rows = few ? 16 : 32;
+    dim3 grid(n_seqs, K * ((G + rows - 1) / rows), parts), block(64 * W);
+    const size_t lds = (size_t)W * (G < rows ? G : rows) * (HD + 4 + 2) * sizeof(float);
+    auto kfn = attn_decode_kernel<T, W, WaveAttn<T>>;
+    if constexpr (HD % 32 == 0) if (few) kfn = attn_decode_kernel<T, W, WaveAttn16<T>>;
     if (lds > 48 * 1024 &&
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return LI_HIP_ERROR;

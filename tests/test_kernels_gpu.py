@@ -701,6 +701,41 @@ def test_attention_whole_prompts_and_decode(ops, H, K, hd, lens, dt):
             assert err < tol, (splits, err)
 
 
+# query heads of a KV head around the 16 rows of the narrow tile (beyond them the tile of 32 rows, and chunks of it), for head sizes
+# of one 32 up to the largest; contexts of one key, at the edges of a score tile's eights and of a page
+@pytest.mark.parametrize("G,K,hd", [(1, 2, 32), (15, 1, 64), (16, 2, 128), (17, 1, 128), (4, 3, 96), (33, 1, 32), (7, 1, 256), (16, 1, 160)])
+@pytest.mark.parametrize("dt", F16S)
+def test_decode_attention_in_tiles_of_16_and_32_rows(ops, G, K, hd, dt):
+    g = torch.Generator().manual_seed(G * 100 + hd)
+    H, lens, scale = G * K, [1, 8, 25, 63, 64, 65, 130, 300], hd ** -0.5
+    seqs = [(i, torch.randn(n, K, hd, generator=g).to(dt), torch.randn(n, K, hd, generator=g).to(dt)) for i, n in enumerate(lens)]
+    q = (torch.randn(len(lens), H, hd, generator=g) * 1.5).to(dt)
+    sink, slopes = torch.randn(H, generator=g), torch.rand(H, generator=g) * 0.1
+    cache, view = _fill_cache(ops, dt, K, hd, seqs)
+    slot, ctx = (torch.tensor(v, dtype=torch.int32, device=DEV) for v in (list(range(len(lens))), lens))
+    # as test_attention_whole_prompts_and_decode: half a unit in the last place of probabilities and results of the order of 1, four times
+    tol = {torch.float16: 3e-3, torch.bfloat16: 2.5e-2}[dt]
+    for extra in ({}, {"window": 70, "keep_first": 5}, {"sink": sink, "slopes": slopes, "softcap": 20.0}):
+        refs = []
+        for i, (_, k, v) in enumerate(seqs):
+            n = lens[i]
+            s = torch.einsum("hd,nhd->hn", q[i].double(), k.double().repeat_interleave(G, 1)) * scale
+            j = torch.arange(n)
+            if "softcap" in extra:
+                s = 20.0 * torch.tanh(s / 20.0) - slopes.double()[:, None] * (n - 1 - j)
+            if "window" in extra:
+                s = s.masked_fill((j <= n - 1 - 70) & (j >= 5), -math.inf)
+            if "sink" in extra:
+                p = torch.softmax(torch.cat([s, sink.double()[:, None]], 1), 1)[:, :n]
+            else:
+                p = torch.softmax(s, 1)
+            refs.append(torch.einsum("hn,nhd->hd", p, v.double().repeat_interleave(G, 1)))
+        kw = {name: t.to(DEV) if torch.is_tensor(t) else t for name, t in extra.items() if name != "window"}
+        for splits in (1, 2, 4, 8):
+            out = ops.attention_decode(q.to(DEV), view.as_tuple(), slot, ctx, len(lens), H, K, hd, scale, extra.get("window"), splits, **kw)
+            assert (out.double().cpu() - torch.stack(refs)).abs().max().item() < tol, (splits, list(extra))
+
+
 # many tokens, so that heads of a KV head share a workgroup (as many as 256 / hd holds and H / K has divisors for); lengths at
 # the edges of the sixteens and of the 256 keys that are taken at a time; with and without a window that cuts into both
 @pytest.mark.parametrize("H,K,hd,n", [(4, 1, 64, 273), (12, 2, 16, 256), (6, 2, 48, 259), (32, 8, 128, 40)])
