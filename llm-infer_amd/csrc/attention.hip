@@ -747,13 +747,21 @@ __global__ __launch_bounds__(64 * W, A::ROWS == 16 && HD <= 128 ? 2 : 1) void at
     typename A::Scores s;
     const T* kbase = (const T*)c.k + (int64_t)kvh * k_head_elems(HD);
     const T* vbase = (const T*)c.v + (int64_t)kvh * v_head_elems(HD);
-    if (p0 < p1) a.load_k(kbase + (int64_t)table[page_of(p0)] * c.page_stride, kf);
-    for (int p = p0; p < p1; ++p) {
+    // (the page table's entries are on their way two pages ahead, so that an address does not wait for one: batch 1 at 2,000 tokens
+    // in 4 splits 18.3 -> 13.5 us, batch 8 at 8,160 in 16 54.8 -> 53.7)
+    int now = 0, next = 0, after = 0;
+    if (p0 < p1) {
+        now = table[page_of(p0)];
+        next = table[page_of(min(p0 + 1, p1 - 1))];
+        a.load_k(kbase + (int64_t)now * c.page_stride, kf);
+    }
+    for (int p = p0; p < p1; ++p, now = next, next = after) {
         const int page = page_of(p), t0 = page * PAGE;
-        a.load_v(vbase + (int64_t)table[page] * c.page_stride, vf);
+        a.load_v(vbase + (int64_t)now * c.page_stride, vf);
+        after = table[page_of(min(p + 2, p1 - 1))];
         a.scores(kf, s, t0, lo, live ? pos : -1, scale2, (t0 < lo && t0 + PAGE > ex.keep) || t0 + PAGE - 1 > pos, bias_per, cap,
                  cap_per, ex.keep);
-        if (p + 1 < p1) a.load_k(kbase + (int64_t)table[page_of(p + 1)] * c.page_stride, kf);
+        if (p + 1 < p1) a.load_k(kbase + (int64_t)next * c.page_stride, kf);
         a.mix(vf, s);
     }
     // The waves lay the states of the rows that exist down as [wave][row][dim] (maxima and sums behind them), and all threads
