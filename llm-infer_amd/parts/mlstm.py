@@ -73,7 +73,7 @@ class MatrixLSTM(Part):
         # sequence in order, which gives the same bits however a prompt is cut
         segments = None
         if self.dtype != torch.float32 and not ctx.is_decode and getattr(ctx, "host_qlens", None):
-            waves_a_token = H * ((dv + 63) // 64)
+            waves_a_token = H * ((dv + 63) // 64) * (2 if d > 128 else 1)        # (wide keys: two waves a column block)
             length = max(16, min(ops.SSM_SEGMENT, 1 << max(0, (ctx.n_tokens * waves_a_token // ops.SSM_WAVES).bit_length() - 1)))
             if max(ctx.host_qlens) > length:
                 segments = ops.ssm_segments(ctx, length)
