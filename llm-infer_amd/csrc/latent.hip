@@ -878,7 +878,8 @@ __global__ void mlstm_commit_kernel(const float* __restrict__ nm_new, float* __r
 }
 
 // One thread per element of a head's state (`per_head` of them, `state_stride` floats from head to head in the
-// state): walks the sequence's segments in order.
+// state): walks the sequence's segments in order, four of them on their way from memory at a time (a store to the segment before
+// kept the next load behind it: 103 segments of 4 heads of 256 x 512 137 -> 106 us, 4.1 TB/s).
 __global__ void seg_combine_kernel(float* __restrict__ state, int64_t state_stride, const int* __restrict__ seq_slot,
                                    const int* __restrict__ seq_seg0, const int* __restrict__ seq_nseg,
                                    float* __restrict__ seg_buf, const float* __restrict__ seg_decay, int H, int64_t per_head) {
@@ -887,11 +888,20 @@ __global__ void seg_combine_kernel(float* __restrict__ state, int64_t state_stri
     for (int64_t e = (int64_t)blockIdx.z * blockDim.x + threadIdx.x; e < per_head; e += (int64_t)gridDim.z * blockDim.x) {
         float* X = state + ((int64_t)seq_slot[seq] * H + h) * state_stride + e;
         float x = *X;
-        for (int c = c0; c < c0 + nc; ++c) {
-            float* L = seg_buf + ((int64_t)c * H + h) * per_head + e;
-            const float own = *L;
-            *L = x;
-            x = seg_decay[(int64_t)c * H + h] * x + own;
+        for (int c = c0; c < c0 + nc; c += 4) {
+            float own[4], decay[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int at = min(c + u, c0 + nc - 1);
+                own[u] = seg_buf[((int64_t)at * H + h) * per_head + e];
+                decay[u] = seg_decay[(int64_t)at * H + h];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (c + u >= c0 + nc) break;
+                seg_buf[((int64_t)(c + u) * H + h) * per_head + e] = x;
+                x = decay[u] * x + own[u];
+            }
         }
         *X = x;
     }
@@ -990,7 +1000,10 @@ __global__ __launch_bounds__(256) void gated_head_norm_vec_kernel(const float* _
     if (live) *(Out4*)(out + (int64_t)u * dv + i) = o;
 }
 
-template <class T>
+// V: a lane's elements are fetched together, with their weights and gates, and kept (heads of up to 64 V); 0: any width, every
+// element fetched twice.  The same values either way.  8 rows of 4 heads of 512 5.5 -> 3.4 us, 1,582
+// rows 11.0 -> 7.7.
+template <class T, int V>
 __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __restrict__ y, const float* __restrict__ w,
                                                               const float* __restrict__ gate, int64_t gate_stride,
                                                               T* __restrict__ out, int n_units, int H, int dv, float eps,
@@ -1000,6 +1013,26 @@ __global__ __launch_bounds__(256) void gated_head_norm_kernel(const float* __res
     const int t = unit / H, h = unit - t * H;
     const float* yr = y + (int64_t)unit * dv;
     float ss = 0.f;
+    if constexpr (V > 0) {
+        float v[V], wv[V], z[V];
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            const int i = min(lane + 64 * k, dv - 1);
+            v[k] = yr[i];
+            wv[k] = w ? w[w_shared ? i : h * dv + i] : 1.f;
+            z[k] = gate ? gate[(int64_t)t * gate_stride + h * dv + i] : 0.f;
+        }
+#pragma unroll
+        for (int k = 0; k < V; ++k) if (lane + 64 * k < dv) ss += v[k] * v[k];
+        const float r = 1.f / sqrtf(wave_sum(ss) / (float)dv + eps);
+#pragma unroll
+        for (int k = 0; k < V; ++k) {
+            float x = v[k] * r * wv[k];
+            if (gate) x *= gate_silu ? z[k] * lt_sigmoid(z[k]) : lt_sigmoid(z[k]);
+            if (lane + 64 * k < dv) out[(int64_t)unit * dv + lane + 64 * k] = from_f32<T>(x);
+        }
+        return;
+    }
     for (int i = lane; i < dv; i += 64) ss += yr[i] * yr[i];
     const float r = 1.f / sqrtf(wave_sum(ss) / (float)dv + eps);
     for (int i = lane; i < dv; i += 64) {
@@ -1026,8 +1059,9 @@ extern "C" int li_gated_head_norm(const float* y, const float* w, const float* g
         LI_CHECK_LAUNCH();
         return LI_OK;
     }
-    DISPATCH_T(dt, (gated_head_norm_kernel<T><<<(units + 3) / 4, 256, 0, stream>>>(y, w, gate, gate_stride, (T*)out, units, H, dv, eps,
-                                                                             w_shared, gate_silu)));
+#define GO(V) gated_head_norm_kernel<T, V><<<(units + 3) / 4, 256, 0, stream>>>(y, w, gate, gate_stride, (T*)out, units, H, dv, eps, w_shared, gate_silu)
+    DISPATCH_T(dt, { if (dv <= 128) GO(2); else if (dv <= 512) GO(8); else GO(0); });
+#undef GO
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

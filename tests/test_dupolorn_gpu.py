@@ -211,6 +211,27 @@ def test_average_with_the_norms_that_follow(lib, rows, width):
     assert not ops.average_norms_fit(odd, None, odd, [(torch.ones(75, device=DEV), 1e-5, torch.float32)])
 
 
+@pytest.mark.parametrize("dv", [1, 63, 65, 127, 129, 511, 512, 513])
+def test_head_norm_of_every_width(lib, dv):
+    """Widths around what a lane keeps (2 and 8 elements) and beyond it, with and without weight and gate."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dv)
+    H, rows = 3, 5
+    y, gate, w = torch.randn(rows, H * dv, generator=g), torch.randn(rows, H * dv + 7, generator=g), torch.randn(H * dv, generator=g)
+    for weight, silu in ((w, False), (w[:dv], True), (None, None)):
+        got = ops.gated_head_norm(y.to(DEV), None if weight is None else weight.to(DEV).contiguous(), None if silu is None else gate.to(DEV), 7, H, 1e-3,
+                                  torch.float32, bool(silu)).cpu().double()
+        v = y.double().view(rows, H, dv)
+        ref = (v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-3)).reshape(rows, H * dv)
+        if weight is not None:
+            ref = ref * (weight.double() if weight.numel() == H * dv else weight.double().repeat(H))
+        if silu is not None:
+            z = gate[:, 7:].double()
+            ref = ref * torch.sigmoid(z) * (z if silu else 1)
+        # a root, a division, an exponential and four products of 32 bits, and the sum of squares' own rounding: under 16 roundings
+        assert ((got - ref).abs() <= 16 * 2.0 ** -24 * ref.abs() + 1e-7).all()
+
+
 @pytest.mark.parametrize("taps", [1, 2, 3, 6])
 def test_convolution_ahead_of_a_mixer(lib, taps):
     """The convolution alone: whole, in portions shorter than its reach, and one token at a time."""
