@@ -15,8 +15,8 @@ graph, as for decoding.  The reference replays a recorded graph per token in the
 Only parts that say so are recorded (``prefill_recordable``): a part that plans on the host from the step's
 lengths (``ctx.host_qlens``) would have its plan frozen into the graph.
 
-A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on every model that
-the runner records (a decode step plans nothing on the host); its key holds the bucket of context lengths too.  An
+A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on every model of this library's own parts that
+the runner records (a decode step of theirs plans nothing on the host); its key holds the bucket of context lengths too.  An
 eager one takes the host 0.7 to 0.95 ms on models of four layers, the device 0.35 to 0.6.
 """
 from __future__ import annotations
@@ -43,6 +43,18 @@ class _RecordedContext(StepShared):
             setattr(self, name, t)
 
 
+def _only_own_parts(model) -> bool:
+    """True if every part of the model is this library's: a part from outside may read of a step what a recorded one does not
+    have (``host_slots``), and so far only a decode runner recorded it."""
+    stack = list(model.children())
+    while stack:
+        part = stack.pop()
+        if type(part).__module__.split(".")[0] != __name__.split(".")[0]:
+            return False
+        stack += list(part.children()) if hasattr(part, "children") else []
+    return True
+
+
 class PrefillRecorder:
     """The recorded prefill steps of one engine (which is handed in with every call: the engine holds this
     object, and a reference back would keep both alive until the garbage collector finds the cycle)."""
@@ -59,7 +71,9 @@ class PrefillRecorder:
         if ctx.n_want == 0 or ctx.n_tokens > MAX_TOKENS or ctx.n_seqs > MAX_SEQS:
             return False
         if ctx.is_decode:
-            return eng.model.recordable()
+            if getattr(self, "_own_parts", None) is None:
+                self._own_parts = eng.model.recordable() and _only_own_parts(eng.model)
+            return self._own_parts
         if getattr(self, "_model_ok", None) is None:
             model = eng.model
             mixers = [m for ms in model.layer_mixers for m in ms]
