@@ -114,7 +114,7 @@ def test_recorded_single_token_steps_give_the_eager_logits(dtype, tmp_path):
     for e in (eager, rec):
         e.step(slots[e], prompts)
     for which in ([0], [0, 1, 2, 3, 4], [3, 1, 4], [2, 0]):
-        for step in range(7):
+        for step in range(10):
             toks = torch.randint(0, TINY_A["vocab_size"], (len(which),), generator=g).tolist()
             want = None if step % 3 else [[0] if i % 2 == 0 else [] for i in range(len(which))]
             a, b = (e.step([slots[e][i] for i in which], [[t] for t in toks], want) for e in (eager, rec))
