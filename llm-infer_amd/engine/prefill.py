@@ -15,11 +15,13 @@ graph, as for decoding.  The reference replays a recorded graph per token in the
 Only parts that say so are recorded (``prefill_recordable``): a part that plans on the host from the step's
 lengths (``ctx.host_qlens``) would have its plan frozen into the graph.
 
-A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on every model of this library's own parts that
+A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on models of up to ``MAX_STEP_BYTES``, of this library's own parts, that
 the runner records (a decode step of theirs plans nothing on the host); its key holds the bucket of context lengths too.  An
 eager one takes the host 0.7 to 0.95 ms on models of four layers, the device 0.35 to 0.6.
 """
 from __future__ import annotations
+
+import math
 
 import numpy as np
 import torch
@@ -30,6 +32,9 @@ from .step import StepShared, split_bucket
 
 MAX_TOKENS = 512          # a longer step keeps the device busy longer than the host needs to enqueue it
 MAX_SEQS = 16
+# largest model (bytes of its matrices) whose steps of one token are recorded: beyond, the step is the device's (the 8B shape, batch
+# 1: 3.2 ms eagerly, the host's 3.0 of them meanwhile, 3.15 replayed), and a recording of many layers takes 10 ms
+MAX_STEP_BYTES = 6 << 30
 MAX_RECORDED = 32         # recorded prefill steps an engine keeps; the least recently used goes first
 
 
@@ -41,6 +46,10 @@ class _RecordedContext(StepShared):
         self.n_tokens, self.n_seqs, self.n_want, self.device = n_tokens, n_seqs, n_want, device
         for name, t in fields.items():
             setattr(self, name, t)
+
+
+def _matrix_bytes(model) -> int:
+    return sum(math.prod(p.shape) for p in model.params().values() if len(p.shape) == 2) * model.dtype.itemsize
 
 
 def _only_own_parts(model) -> bool:
@@ -71,9 +80,10 @@ class PrefillRecorder:
         if ctx.n_want == 0 or ctx.n_tokens > MAX_TOKENS or ctx.n_seqs > MAX_SEQS:
             return False
         if ctx.is_decode:
-            if getattr(self, "_own_parts", None) is None:
-                self._own_parts = eng.model.recordable() and _only_own_parts(eng.model)
-            return self._own_parts
+            if getattr(self, "_steps_ok", None) is None:
+                self._steps_ok = (_matrix_bytes(eng.model) <= MAX_STEP_BYTES and eng.model.recordable()
+                                  and _only_own_parts(eng.model))
+            return self._steps_ok
         if getattr(self, "_model_ok", None) is None:
             model = eng.model
             mixers = [m for ms in model.layer_mixers for m in ms]
