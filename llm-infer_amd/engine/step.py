@@ -105,7 +105,7 @@ def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int, head_di
     """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one page a
     split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64.  Heads of up to 160 are not split
     beyond four, which merge inside a workgroup, for more waves than half the chip's SIMDs, and those below 128 not into eight."""
-    # measured on MI355X, us with half as many splits and with these.  Heads of 128, 8 KV heads, batch 1 at 40 tokens 6.2 and 6.1,
+    # measured on MI355X with tiles of 32 rows, us with half as many splits and with these.  Heads of 128, 8 KV heads, batch 1 at 40 tokens 6.2 and 6.1,
     # at 100 7.5 and 6.3, at 250 7.6 and 6.7, at 500 8.2 and 8.6, at 777 10.3 and 9.2 (with a soft cap and gates 12.5 and 10.3), at 1,000
     # 9.9 and 9.0, at 2,000 11.3 and 10.4, at 4,000 14.1 and 11.7; batch 32 at 250 10.7 and 10.5.  Not taken (what more would take): 128,
     # batch 16 at 500 11.3 (13.1), at 900 15.5 (17.9), batch 4 at 4,000 18.1 (18.6), batch 8 at 1,900 17.0 (17.8), batch 2 at 8,000 18.6
