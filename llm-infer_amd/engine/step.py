@@ -112,13 +112,12 @@ def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int, head_di
     # (19.6); 64, batch 1 at 500 7.6 (8.6), at 900 8.5 (8.7), batch 8 at 500 8.6 (10.2), at 900 11.0 (10.6); 96, batch 1 at 700 8.1
     # (9.0), batch 8 at 900 12.1 (11.8); 160, 4 KV heads, 64 splits at 8,000 19.0 (20.0).  Heads of 256, 2 KV heads, whose pages are
     # longer: batch 1 at 500 30 and 18, batch 32 at 1,000 67 and 49
-    # Two splits where four would make more than 1,024 waves, and contexts of up to some 1,000 tokens: four after all, since two
-    # waves of the tile of 16 rows share a SIMD.  8 KV heads, us in two and four: heads of 128, batch 40 at 16 to 528 tokens 17.7 and
-    # 15.4, 48 21.0 and 19.0, 64 20.4 and 18.8, 48 at 16 to 1,000 31.5 and 27.2, 64 at 900 48.3 and 48.8 (at 4,000 176 and
-    # 179); heads of 64, 48 at 16 to 528 10.8 and 10.1, 64 at 16 to 1,000 22.7 and 19.7
+    # Two splits where four would make more than 1,024 waves: four after all, since two waves of the tile of 16 rows share a SIMD.  8 KV heads, us in two and four: heads of 128, batch 40 at 16 to 528 tokens 17.7 and
+    # 15.4, 48 21.0 and 19.0, 64 20.4 and 18.8, 48 at 16 to 1,000 31.5 and 27.2, 64 at 900 48.3 and 48.8, at 4,000 179.8
+    # and 177.1, at 8,000 362 and 346 (tiles of 32 rows, two splits: 174.5 and 354); heads of 64, 48 at 16 to 528 10.8 and 10.1, 64 at 16 to 1,000 22.7 and 19.7
     few, many = (decode_splits(n_seqs, n_kv_heads, n_heads, min(b, 64)) for b in (bucket, 2 * bucket))
     waves = many * n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 31) // 32)
-    if few == many == 2 and 2 <= bucket <= 8 and head_dim <= 128 and head_dim % 32 == 0 and n_heads <= 16 * n_kv_heads:
+    if few == many == 2 and head_dim <= 128 and head_dim % 32 == 0 and n_heads <= 16 * n_kv_heads:
         return 4
     return few if head_dim <= 160 and many > 4 and (waves > 512 or (few == 4 and head_dim < 128) or (many == 64 and head_dim > 128)) else many
 
