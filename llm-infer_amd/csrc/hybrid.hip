@@ -542,7 +542,7 @@ __global__ __launch_bounds__(64) void ssm_scan_kernel(
     if (PASS == 1 && lane == 0 && blockIdx.z == 0) plan.seg_decay[(int64_t)blockIdx.x * P + h] = expf(log_decay);
 }
 
-// One thread per element of a head's state: walks the sequence's segments in order, four of them on their way from memory at a time.
+// One thread per element of a head's state: walks the sequence's segments in order.
 __global__ void ssm_combine_kernel(float* __restrict__ state, const int* __restrict__ seq_slot,
                                    const int* __restrict__ seq_seg0, const int* __restrict__ seq_nseg,
                                    float* __restrict__ seg_state, const float* __restrict__ seg_decay, int P, int64_t per_head) {
@@ -551,31 +551,14 @@ __global__ void ssm_combine_kernel(float* __restrict__ state, const int* __restr
     for (int64_t e = (int64_t)blockIdx.z * blockDim.x + threadIdx.x; e < per_head; e += (int64_t)gridDim.z * blockDim.x) {
         float* S = state + ((int64_t)seq_slot[seq] * P + h) * per_head + e;
         float s = *S;
-        for (int c = c0; c < c0 + nc; c += 4) {
-            float own[4], decay[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int at = min(c + u, c0 + nc - 1);
-                own[u] = seg_state[((int64_t)at * P + h) * per_head + e];
-                decay[u] = seg_decay[(int64_t)at * P + h];
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                if (c + u >= c0 + nc) break;
-                seg_state[((int64_t)(c + u) * P + h) * per_head + e] = s;
-                s = decay[u] * s + own[u];
-            }
+        for (int c = c0; c < c0 + nc; ++c) {
+            float* L = seg_state + ((int64_t)c * P + h) * per_head + e;
+            const float own = *L;
+            *L = s;
+            s = seg_decay[(int64_t)c * P + h] * s + own;
         }
         *S = s;
     }
-}
-
-extern "C" int li_ssm_combine(float* state, const int* seq_slot, const int* seq_seg0, const int* seq_nseg, float* seg_state,
-                              const float* seg_decay, int n_seqs, int P, int64_t per_head, hipStream_t stream) {
-    const dim3 grid(n_seqs, P, (unsigned)((per_head + 255) / 256));
-    ssm_combine_kernel<<<grid, 256, 0, stream>>>(state, seq_slot, seq_seg0, seq_nseg, seg_state, seg_decay, P, per_head);
-    LI_CHECK_LAUNCH();
-    return LI_OK;
 }
 
 #define SSM_GO(NM, GRID, PLAN) ssm_scan_kernel<NM, SSM_PASS><<<GRID, 64, 0, stream>>>(xbc, xbc_stride, proj, proj_stride, dt_col, \
@@ -619,8 +602,9 @@ extern "C" int li_ssm_scan_segments(const float* xbc, int xbc_stride, const floa
 #define SSM_PASS 1
     SSM_LAUNCH(grid, plan);
 #undef SSM_PASS
-    const int rc = li_ssm_combine(state, seq_slot, seq_seg0, seq_nseg, seg_state, seg_decay, n_seqs, P, (int64_t)N * dv, stream);
-    if (rc) return rc;
+    const int64_t per_head = (int64_t)N * dv;
+    dim3 cgrid(n_seqs, P, (unsigned)((per_head + 255) / 256));
+    ssm_combine_kernel<<<cgrid, 256, 0, stream>>>(state, seq_slot, seq_seg0, seq_nseg, seg_state, seg_decay, P, per_head);
     plan.pass = 3;
 #define SSM_PASS 3
     SSM_LAUNCH(grid, plan);

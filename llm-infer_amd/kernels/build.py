@@ -202,12 +202,12 @@ def mixers_library(force=False):
     return _load("libli_mixers.so", MIXER_SOURCES, (), force)
 
 
-HYBRID_SOURCES = ("hybrid.hip", "ssm_chunks.hip", "latent.hip", "gated.hip")
+HYBRID_SOURCES = ("hybrid.hip", "latent.hip", "gated.hip")
 
 
 def hybrid_library(force=False):
     """The kernels of hybrid decoders (csrc/hybrid.hip: differential attention over blocks of positions, the
-    state-space recurrence and its convolution, the experts' router; csrc/ssm_chunks.hip: that recurrence for prompts; csrc/latent.hip: latent attention's
+    state-space recurrence and its convolution, the experts' router; csrc/latent.hip: latent attention's
     preparation and products per head, the matrix-memory recurrence, the bigram embedding, the depth-weighted
     average of the residual stream; csrc/gated.hip: the norm of a sub-layer's output with the residual sum, the rotation
     of half-paired dimensions with the cache write, the clamped gated activation, experts by table): a library of its own,

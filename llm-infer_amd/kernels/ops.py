@@ -1578,7 +1578,6 @@ def conv_silu(rows, col0, channels, weight, bias, history, ctx, out_dtype=torch.
     return out
 
 
-SSM_CHUNK = 64             # tokens of a chunk of ``ssm_scan``'s matrix form
 SSM_SEGMENT = 128          # most tokens of a segment when a prompt's recurrence runs in segments side by side
 SSM_WAVES = 3072           # segments are made short enough for about this many waves (three a SIMD)
 
@@ -1600,33 +1599,16 @@ def ssm_segments(ctx, length: int | None = None) -> dict:
         k, b = len(seg_seq), len(seq_seg0)
         flat = torch.tensor(seg_seq + seg_t0 + seg_n + seq_seg0 + seq_nseg, dtype=torch.int32).to(ctx.device)
         return {"seg_seq": flat[:k], "seg_t0": flat[k:2 * k], "seg_n": flat[2 * k:3 * k], "seq_seg0": flat[3 * k:3 * k + b],
-                "seq_nseg": flat[3 * k + b:], "n": k, "length": length}
+                "seq_nseg": flat[3 * k + b:], "n": k}
     return ctx.shared(("ssm_segments", length), make)
 
 
-def ssm_chunks_fit(n_state: int, dv: int) -> bool:
-    """Whether ``ssm_scan`` takes this state as products of matrices."""
-    return n_state % 16 == 0 and n_state <= 256 and dv % 16 == 0
-
-
-def ssm_chunks_pay(qlens, heads: int, n_state: int, dv: int) -> bool:
-    """Whether a step's recurrence is faster as products of matrices by chunks of 64 tokens than token by token."""
-    # measured on MI355X, us token by token and in chunks, 128 heads of 128 x 64: one sequence of 20 tokens 56 and 40, 100 230 and
-    # 55, 2,000 4,640 and 288; 16 sequences of 20 97 and 177, of 64 265 and 221; 8 of 33 91 and 109.  A token of the
-    # longest sequence takes 2.3 us, more from a thousand waves on; a chunk its states' way to memory and back
-    waves = len(qlens) * heads * -(-dv // 64)
-    chunks = sum(-(-n // SSM_CHUNK) for n in qlens)
-    return max(qlens) * 2.3 * max(1.0, waves / 1100) > 38 + chunks * heads * n_state * dv * 8.5 / (1 << 20)
-
-
-def ssm_scan(xbc, proj, dt_col, dt_bias, a_log, d_skip, state, ctx, heads, groups, n_state, dv, segments=None,
-             chunks: bool = False) -> torch.Tensor:
+def ssm_scan(xbc, proj, dt_col, dt_bias, a_log, d_skip, state, ctx, heads, groups, n_state, dv, segments=None) -> torch.Tensor:
     """The selective state-space recurrence in float32.  ``xbc`` float32 [T, heads * dv + 2 groups n_state] (x | B |
     C), the raw step sizes in ``proj`` columns dt_col .. dt_col + heads; ``state`` float32 [slots, heads, n_state,
     dv], read and left up to date; returns y float32 [T, heads * dv].  ``segments`` (``ssm_segments``): the tokens
     run in segments side by side, each twice (first for what it adds to the state, then, from the state before it,
-    for y); None: every sequence token by token in order.  ``chunks`` (where ``ssm_chunks_fit``): the segments are of at most
-    SSM_CHUNK tokens and run as products of float32 matrices."""
+    for y); None: every sequence token by token in order."""
     _dev(xbc, proj, dt_bias, a_log, d_skip, state)
     _f32_rows(xbc, "ssm x/B/C")
     _f32_rows(proj, "ssm projections")
@@ -1648,15 +1630,6 @@ def ssm_scan(xbc, proj, dt_col, dt_bias, a_log, d_skip, state, ctx, heads, group
             _i32(segments[name], n, "ssm " + name)
         seg_state = torch.empty((k, heads, n_state, dv), dtype=torch.float32, device=xbc.device)
         seg_decay = torch.empty((k, heads), dtype=torch.float32, device=xbc.device)
-        if chunks:
-            _need(ssm_chunks_fit(n_state, dv) and segments["length"] <= SSM_CHUNK, "ssm in chunks: state and values of multiples of 16, chunks of 64 tokens")
-            scores = torch.empty((k, groups, SSM_CHUNK, SSM_CHUNK), dtype=torch.float32, device=xbc.device)
-            _check(hybrid().li_ssm_chunks(
-                _ptr(xbc), xbc.shape[1], _ptr(proj), proj.shape[1], dt_col, _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state),
-                _ptr(ctx.seq_slot), _ptr(qstart), _ptr(y), ctx.n_seqs, heads, groups, n_state, dv, _ptr(segments["seg_seq"]),
-                _ptr(segments["seg_t0"]), _ptr(segments["seg_n"]), _ptr(segments["seq_seg0"]), _ptr(segments["seq_nseg"]), k,
-                _ptr(scores), _ptr(seg_state), _ptr(seg_decay), _stream()), "ssm_chunks")
-            return y
         _check(hybrid().li_ssm_scan_segments(
             _ptr(xbc), xbc.shape[1], _ptr(proj), proj.shape[1], dt_col, _ptr(dt_bias), _ptr(a_log), _ptr(d_skip), _ptr(state),
             _ptr(ctx.seq_slot), _ptr(qstart), _ptr(qlen), _ptr(y), ctx.n_seqs, heads, groups, n_state, dv,
