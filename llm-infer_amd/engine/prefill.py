@@ -15,9 +15,12 @@ graph, as for decoding.  The reference replays a recorded graph per token in the
 Only parts that say so are recorded (``prefill_recordable``): a part that plans on the host from the step's
 lengths (``ctx.host_qlens``) would have its plan frozen into the graph.
 
-A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded likewise on models of up to ``MAX_STEP_BYTES``, of this library's own parts, that
-the runner records (a decode step of theirs plans nothing on the host); its key holds the bucket of context lengths too.  An
-eager one takes the host 0.7 to 0.95 ms on models of four layers, the device 0.35 to 0.6.
+A step of one token for each sequence, called for by itself instead of through a decode runner, is recorded
+likewise on models of up to ``MAX_STEP_BYTES``, of this library's own parts, that the runner records (a decode
+step of theirs plans nothing on the host).  It is not padded: a recording is for so many sequences and wanted
+rows and the bucket of context lengths, and runs the kernels that the eager step runs, so that a call gives the
+same bits the first time and the tenth.  An eager one takes the host 0.7 to 0.95 ms on models of four layers, the
+device 0.35 to 0.6.
 """
 from __future__ import annotations
 
@@ -127,33 +130,34 @@ class PrefillRecorder:
         return packed
 
     @staticmethod
-    def _fill_decode(ctx, rows, wants, scratch):
-        """The same for a step of one token a sequence: tokens, positions, contexts and slots of ``rows`` rows, wanted rows.
-        Rows beyond the sequences are idle ones on the scratch slot, with a context of one token."""
-        packed = np.zeros(4 * rows + wants, dtype=np.int32)
-        n, at = ctx.n_seqs, packed[:4 * rows].reshape(4, rows)
-        at[0, :n], at[1, :n] = ctx.host_tokens, ctx.host_lens_before
-        at[2] = at[1] + 1
-        at[3, :n], at[3, n:] = ctx.host_slots, scratch
-        packed[4 * rows:4 * rows + ctx.n_want] = ctx.host_want_rows
+    def _fill_decode(ctx):
+        """The same for a step of one token a sequence: tokens, positions, contexts, slots and wanted rows, each array on a
+        multiple of four elements (16 bytes)."""
+        n = (ctx.n_seqs + 3) // 4 * 4
+        packed = np.zeros(4 * n + ctx.n_want, dtype=np.int32)
+        before = np.array(ctx.host_lens_before)
+        for i, values in enumerate((ctx.host_tokens, before, before + 1, ctx.host_slots, ctx.host_want_rows)):
+            packed[i * n:i * n + len(values)] = values
         return packed
 
     @staticmethod
     def _decode_context(buf, rows, wants, bucket):
-        names = ("tokens", "pos", "ctx", "slots")
-        fields = {name: buf[i * rows:(i + 1) * rows] for i, name in enumerate(names)}
-        ctx = _GraphContext(dict(fields, rows=buf[4 * rows:]), rows, bucket)
-        ctx.n_want, ctx.want_rows = wants, buf[4 * rows:4 * rows + wants]
+        n = (rows + 3) // 4 * 4
+        fields = {name: buf[i * n:] for i, name in enumerate(("tokens", "pos", "ctx", "slots", "rows"))}
+        ctx = _GraphContext(fields, rows, bucket)
+        ctx.n_want, ctx.want_rows = wants, fields["rows"][:wants]
         return ctx
 
     # -- the step --------------------------------------------------------------------
     def run(self, eng, ctx):
         """The logits of the step [n_want, vocab], or None if this step is to be run eagerly (the first time
         its key is seen, or the second)."""
-        rows = batch_bucket(ctx.n_tokens, MAX_TOKENS)
-        seqs = batch_bucket(ctx.n_seqs, MAX_SEQS)
-        wants = batch_bucket(ctx.n_want, rows)
-        bucket = split_bucket(ctx.max_ctx) if ctx.is_decode else None
+        rows, seqs, wants, bucket = ctx.n_tokens, ctx.n_seqs, ctx.n_want, None
+        if ctx.is_decode:
+            bucket = split_bucket(ctx.max_ctx)
+        else:
+            rows, seqs = batch_bucket(rows, MAX_TOKENS), batch_bucket(seqs, MAX_SEQS)
+            wants = batch_bucket(wants, rows)
         key = (rows, seqs, wants, bucket)
         entry = self.graphs.pop(key, None)
         # a recording takes some milliseconds: a step of one token is recorded when it comes for the third time (one behind a prompt
@@ -164,7 +168,7 @@ class PrefillRecorder:
             self._trim()
             return None
         if ctx.is_decode:
-            packed = self._fill_decode(ctx, rows, wants, eng.cache.scratch_slot)
+            packed = self._fill_decode(ctx)
         else:
             layout, total = self._layout(rows, seqs, wants)
             packed = self._fill(ctx, layout, total, eng.cache.scratch_slot)

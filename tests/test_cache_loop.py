@@ -363,6 +363,21 @@ def test_the_index_arrays_of_a_recorded_prefill_step():
     assert all(at % 4 == 0 for at, _ in layout.values()) and total % 4 == 0
 
 
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 16])
+def test_the_index_arrays_of_a_recorded_single_token_step(n):
+    """As many rows as the step has, no padded ones, each array on 16 bytes."""
+    from llm_infer_amd.engine.prefill import PrefillRecorder
+    from llm_infer_amd.engine.step import StepContext
+    lens = [3 + 7 * i for i in range(n)]
+    ctx = StepContext(None, [9 + i for i in range(n)], [[20 + i] for i in range(n)], lens, [[0] if i % 3 == 0 else [] for i in range(n)], upload=False)
+    packed = torch.from_numpy(PrefillRecorder._fill_decode(ctx))
+    rec = PrefillRecorder._decode_context(packed, n, ctx.n_want, 1)
+    assert (rec.n_seqs, rec.n_tokens, rec.n_want) == (n, n, ctx.n_want)
+    got = [t.tolist() for t in (rec.token_ids, rec.pos, rec.seq_ctx, rec.seq_slot, rec.want_rows)]
+    assert got == [[20 + i for i in range(n)], lens, [v + 1 for v in lens], [9 + i for i in range(n)], list(range(0, n, 3))]
+    assert all((t.data_ptr() - packed.data_ptr()) % 16 == 0 for t in (rec.token_ids, rec.pos, rec.seq_ctx, rec.seq_slot, rec.want_rows))
+
+
 def test_cache_rounding_option_is_for_a_float32_cache():
     with pytest.raises(CacheError, match="kv_round"):
         Cache([KVSpec(1, 16)], 256, 128, torch.bfloat16, None, 2, kv_round=torch.float16)

@@ -98,9 +98,32 @@ def test_generation_through_recorded_prompts_and_steps(tmp_path):
     assert eng._prefill.counts["replayed"] >= 4
 
 
+@pytest.mark.parametrize("dtype", ["float16", "bfloat16"])
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 6, 7, 9, 11, 13, 16])
+def test_a_single_token_step_gives_the_same_bits_recorded_or_not(dtype, n, tmp_path):
+    """The same call on the same state, eagerly (the first two), recorded and replayed, for numbers of sequences around those at which
+    products take another kernel (a vocabulary of 257 tiles of 16: half tiles up to three rows); all rows wanted, and some."""
+    import llm_infer_amd
+    cfg = dict(TINY_A, max_position_embeddings=1024, hidden_size=256, intermediate_size=688, vocab_size=4104)
+    folder, _ = _model(tmp_path, cfg, dtype)
+    eng = llm_infer_amd.load(folder, dtype=dtype, max_tokens=8192)
+    g = torch.Generator().manual_seed(n)
+    lens = [1 + 17 * i for i in range(n)]
+    slots = [eng.alloc_slot() for _ in lens]
+    eng.step(slots, [torch.randint(0, cfg["vocab_size"], (k,), generator=g).tolist() for k in lens])
+    toks = [[t] for t in torch.randint(0, cfg["vocab_size"], (n,), generator=g).tolist()]
+    for want in (None, [[0] if i % 2 == 0 else [] for i in range(n)]):
+        got = []
+        for _ in range(5):
+            got.append(eng.step(slots, toks, want))
+            eng.cache.truncate(slots, lens)
+        assert all(torch.equal(got[0], other) for other in got[1:])
+    assert eng._prefill.counts["replayed"] >= 2
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 def test_recorded_single_token_steps_give_the_eager_logits(dtype, tmp_path):
-    """Steps of one token for each sequence, called for by themselves: eager, recorded and replayed, with idle rows, across a
+    """Steps of one token for each sequence, called for by themselves: eager, recorded and replayed, across a
     bucket of context lengths, with sequences that change between replays; the eager engine runs the same rows."""
     import llm_infer_amd
     folder, _ = _model(tmp_path, dict(TINY_A, max_position_embeddings=1024), "bfloat16")
@@ -119,9 +142,5 @@ def test_recorded_single_token_steps_give_the_eager_logits(dtype, tmp_path):
             want = None if step % 3 else [[0] if i % 2 == 0 else [] for i in range(len(which))]
             a, b = (e.step([slots[e][i] for i in which], [[t] for t in toks], want) for e in (eager, rec))
             assert a.shape == b.shape
-            if dtype == "float32":
-                assert torch.equal(a, b), (which, step)
-            else:
-                # other rows in the step, so other kernels: equal up to the rounding of 16-bit steps
-                assert (a - b).abs().max().item() < 0.05 * a.std().item(), (which, step)
+            assert torch.equal(a, b), (which, step)                # to the bit: the same rows, so the same kernels
     assert rec._prefill.counts["replayed"] >= 10
