@@ -38,7 +38,9 @@ MAX_SEQS = 16
 # largest model (bytes of its matrices) whose steps of one token are recorded: beyond, the step is the device's (the 8B shape, batch
 # 1: 3.2 ms eagerly, the host's 3.0 of them meanwhile, 3.15 replayed), and a recording of many layers takes 10 ms
 MAX_STEP_BYTES = 6 << 30
-MAX_RECORDED = 32         # recorded prefill steps an engine keeps; the least recently used goes first
+# what an engine keeps of each kind, prompts and steps of one token; the least recently used goes first.  Kept apart: a loop of steps
+# over many batch sizes and context lengths would push every prompt's recording out, each time with a wait for the device
+MAX_RECORDED = 32
 
 
 class _RecordedContext(StepShared):
@@ -72,9 +74,10 @@ class PrefillRecorder:
     object, and a reference back would keep both alive until the garbage collector finds the cycle)."""
 
     def __init__(self):
-        self.graphs = {}                   # key -> "once" | "seen" | (graph, logits)
+        self.graphs = {}                   # prompts: key -> "seen" | (graph, logits, index arrays on the device)
+        self.step_graphs = {}              # steps of one token: key -> (graph, logits, index arrays)
+        self._step_seen = {}               # those called for once or twice: key -> "once" | "seen"
         self.counts = {"eager": 0, "recorded": 0, "replayed": 0}
-        self._buffers = {}                 # key -> (device buffer, layout)
 
     # -- which steps ---------------------------------------------------------------
     def takes(self, eng, ctx) -> bool:
@@ -159,11 +162,15 @@ class PrefillRecorder:
             rows, seqs = batch_bucket(rows, MAX_TOKENS), batch_bucket(seqs, MAX_SEQS)
             wants = batch_bucket(wants, rows)
         key = (rows, seqs, wants, bucket)
-        entry = self.graphs.pop(key, None)
+        graphs = self.step_graphs if ctx.is_decode else self.graphs
+        entry = graphs.pop(key, None) or self._step_seen.pop(key, None)
         # a recording takes some milliseconds: a step of one token is recorded when it comes for the third time (one behind a prompt
         # and one at a request's end are no loop)
-        if entry is None or (entry == "once" and ctx.is_decode):
-            self.graphs[key] = "once" if entry is None and ctx.is_decode else "seen"
+        if entry is None or entry == "once":
+            if ctx.is_decode:
+                self._step_seen[key] = "seen" if entry else "once"
+            else:
+                graphs[key] = "seen"
             self.counts["eager"] += 1
             self._trim()
             return None
@@ -172,11 +179,8 @@ class PrefillRecorder:
         else:
             layout, total = self._layout(rows, seqs, wants)
             packed = self._fill(ctx, layout, total, eng.cache.scratch_slot)
-        if key not in self._buffers:
-            self._buffers[key] = torch.zeros((len(packed),), dtype=torch.int32, device=eng.device)
-        buf = self._buffers[key]
-        buf.copy_(torch.from_numpy(packed))
         if entry == "seen":
+            buf = torch.from_numpy(packed).to(eng.device)
             graph = torch.cuda.CUDAGraph()
             with recording(graph):
                 if ctx.is_decode:
@@ -187,19 +191,22 @@ class PrefillRecorder:
                     rec = _RecordedContext(fields, rows, seqs, wants, eng.device)
                     rec.shared(ops.PREFILL_TILES_KEY, lambda: tiles)
                 logits = eng.model.forward(rec, eng.cache)
-            entry = (graph, logits)
+            entry = (graph, logits, buf)
             self.counts["recorded"] += 1
         else:
+            entry[2].copy_(torch.from_numpy(packed))
             self.counts["replayed"] += 1
         entry[0].replay()
-        self.graphs[key] = entry
+        graphs[key] = entry
         self._trim()
         return entry[1][:ctx.n_want].clone()
 
     def _trim(self):
-        while len(self.graphs) > MAX_RECORDED:
-            old = next(iter(self.graphs))
-            if self.graphs[old] not in ("seen", "once"):
-                torch.cuda.synchronize()             # it may still be running
-            del self.graphs[old]
-            self._buffers.pop(old, None)
+        for graphs in (self.graphs, self.step_graphs):
+            while len(graphs) > MAX_RECORDED:
+                old = next(iter(graphs))
+                if graphs[old] != "seen":
+                    torch.cuda.synchronize()             # it may still be running
+                del graphs[old]
+        while len(self._step_seen) > 16 * MAX_RECORDED:
+            del self._step_seen[next(iter(self._step_seen))]

@@ -378,6 +378,45 @@ def test_the_index_arrays_of_a_recorded_single_token_step(n):
     assert all((t.data_ptr() - packed.data_ptr()) % 16 == 0 for t in (rec.token_ids, rec.pos, rec.seq_ctx, rec.seq_slot, rec.want_rows))
 
 
+def test_recorded_prompts_and_single_token_steps_do_not_push_each_other_out(monkeypatch):
+    """Recordings (stand-ins here: a graph that does nothing) of both kinds are bounded, each by itself: the least recently used goes
+    first, and what has come once or twice only is forgotten before it costs a recording."""
+    import contextlib
+    import types
+    from llm_infer_amd.engine import prefill
+    from llm_infer_amd.engine.step import StepContext
+    waits = []
+    monkeypatch.setattr(prefill, "recording", lambda graph: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: types.SimpleNamespace(replay=lambda: None))
+    monkeypatch.setattr(torch.cuda, "synchronize", lambda: waits.append(1))
+    eng = types.SimpleNamespace(device="cpu", cache=types.SimpleNamespace(scratch_slot=0), model=types.SimpleNamespace(
+        forward=lambda ctx, cache: torch.zeros(ctx.n_want, 3)))
+    rec = prefill.PrefillRecorder()
+
+    def step(n, before, tokens=1):
+        return rec.run(eng, StepContext("cpu", list(range(1, n + 1)), [[5] * tokens] * n, [before] * n, [[0]] * n, upload=False))
+    assert step(1, 0, 40) is None and step(1, 0, 40).shape == (1, 3)                    # a prompt: recorded the second time
+    assert rec.counts == {"eager": 1, "recorded": 1, "replayed": 0}
+    kinds = [(n, before) for n in range(1, 17) for before in (100, 300, 600, 1200)]
+    for n, before in kinds[:prefill.MAX_RECORDED]:
+        assert [step(n, before) is None for _ in range(4)] == [True, True, False, False]
+    assert not waits and len(rec.step_graphs) == prefill.MAX_RECORDED
+    step(1, 0, 40)
+    assert rec.counts["replayed"] == prefill.MAX_RECORDED + 1                           # the prompt's recording is still there
+    for _ in range(2):                                                                  # others, too rare to be recorded
+        for n, before in kinds[prefill.MAX_RECORDED:]:
+            assert step(n, before) is None
+    assert not waits and step(*kinds[0]) is not None and rec.counts["recorded"] == prefill.MAX_RECORDED + 1
+    step(*kinds[-1])                                                                    # one more recording: the oldest goes
+    assert len(waits) == 1 and len(rec.step_graphs) == prefill.MAX_RECORDED and len(rec.graphs) == 1
+    assert step(*kinds[1]) is None and step(*kinds[0]) is not None
+    for n in range(1, 17):
+        for before in range(1, 9000, 64):
+            for want in range(1, n + 1):
+                rec.run(eng, StepContext("cpu", list(range(1, n + 1)), [[5]] * n, [before] * n, [[0]] * want + [[]] * (n - want), upload=False))
+    assert max(len(rec.step_graphs), len(rec.graphs)) <= prefill.MAX_RECORDED and len(rec._step_seen) <= 16 * prefill.MAX_RECORDED
+
+
 def test_cache_rounding_option_is_for_a_float32_cache():
     with pytest.raises(CacheError, match="kv_round"):
         Cache([KVSpec(1, 16)], 256, 128, torch.bfloat16, None, 2, kv_round=torch.float16)
