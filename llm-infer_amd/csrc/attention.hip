@@ -710,7 +710,11 @@ __global__ __launch_bounds__(256, HD <= 128 ? 2 : 1) void attn_prefill_kernel(
 // query heads: often 4 of the tile's 32): done by the first wave on the whole tile they took as long as two pages.  32 / 8 heads of
 // 128, batch 1: 30 tokens 6.3 -> 5.5 us, 200 tokens in 4 splits 8.9 -> 6.1, 777 in 4 with cap and a gate an element 22.0 -> 12.6;
 // batch 48 at 16 to 530 tokens 22.4 -> 20.7.
-template <class T, int W, class A>
+// AHEAD: the page table's entries are on their way two pages ahead, so that an address does not wait for one (batch 1 at 2,000 tokens
+// in 4 splits 18.3 -> 13.5 us, batch 8 at 8,160 in 16 54.8 -> 53.7, 64 at 1,000 to 8,192 in 4 245.9 -> 238.9).  Not where the waves of
+// a full chip all walk long chains to the same end: there memory is the bound, and loads that go out sooner only get in each
+// other's way (figures: launch_decode).
+template <class T, int W, class A, bool AHEAD>
 __global__ __launch_bounds__(64 * W, A::ROWS == 16 && HD <= 128 ? 2 : 1) void attn_decode_kernel(
     const T* __restrict__ q, T* __restrict__ out, float* __restrict__ part_o, float* __restrict__ part_ml,
     CachePtrs c, const int* __restrict__ seq_slot, const int* __restrict__ seq_ctx, int H, int K, float scale,
@@ -747,22 +751,32 @@ __global__ __launch_bounds__(64 * W, A::ROWS == 16 && HD <= 128 ? 2 : 1) void at
     typename A::Scores s;
     const T* kbase = (const T*)c.k + (int64_t)kvh * k_head_elems(HD);
     const T* vbase = (const T*)c.v + (int64_t)kvh * v_head_elems(HD);
-    // (the page table's entries are on their way two pages ahead, so that an address does not wait for one: batch 1 at 2,000 tokens
-    // in 4 splits 18.3 -> 13.5 us, batch 8 at 8,160 in 16 54.8 -> 53.7)
-    int now = 0, next = 0, after = 0;
-    if (p0 < p1) {
-        now = table[page_of(p0)];
-        next = table[page_of(min(p0 + 1, p1 - 1))];
-        a.load_k(kbase + (int64_t)now * c.page_stride, kf);
-    }
-    for (int p = p0; p < p1; ++p, now = next, next = after) {
-        const int page = page_of(p), t0 = page * PAGE;
-        a.load_v(vbase + (int64_t)now * c.page_stride, vf);
-        after = table[page_of(min(p + 2, p1 - 1))];
-        a.scores(kf, s, t0, lo, live ? pos : -1, scale2, (t0 < lo && t0 + PAGE > ex.keep) || t0 + PAGE - 1 > pos, bias_per, cap,
-                 cap_per, ex.keep);
-        if (p + 1 < p1) a.load_k(kbase + (int64_t)next * c.page_stride, kf);
-        a.mix(vf, s);
+    if constexpr (AHEAD) {
+        int now = 0, next = 0, after = 0;
+        if (p0 < p1) {
+            now = table[page_of(p0)];
+            next = table[page_of(min(p0 + 1, p1 - 1))];
+            a.load_k(kbase + (int64_t)now * c.page_stride, kf);
+        }
+        for (int p = p0; p < p1; ++p, now = next, next = after) {
+            const int page = page_of(p), t0 = page * PAGE;
+            a.load_v(vbase + (int64_t)now * c.page_stride, vf);
+            after = table[page_of(min(p + 2, p1 - 1))];
+            a.scores(kf, s, t0, lo, live ? pos : -1, scale2, (t0 < lo && t0 + PAGE > ex.keep) || t0 + PAGE - 1 > pos, bias_per, cap,
+                     cap_per, ex.keep);
+            if (p + 1 < p1) a.load_k(kbase + (int64_t)next * c.page_stride, kf);
+            a.mix(vf, s);
+        }
+    } else {
+        if (p0 < p1) a.load_k(kbase + (int64_t)table[page_of(p0)] * c.page_stride, kf);
+        for (int p = p0; p < p1; ++p) {
+            const int page = page_of(p), t0 = page * PAGE;
+            a.load_v(vbase + (int64_t)table[page] * c.page_stride, vf);
+            a.scores(kf, s, t0, lo, live ? pos : -1, scale2, (t0 < lo && t0 + PAGE > ex.keep) || t0 + PAGE - 1 > pos, bias_per, cap,
+                     cap_per, ex.keep);
+            if (p + 1 < p1) a.load_k(kbase + (int64_t)table[page_of(p + 1)] * c.page_stride, kf);
+            a.mix(vf, s);
+        }
     }
     // The waves lay the states of the rows that exist down as [wave][row][dim] (maxima and sums behind them), and all threads
     // add them in wave order, four dimensions at a time:  M = max m,  o = sum o_w 2^(m_w - M),  l = sum l_w 2^(m_w - M)
@@ -1030,14 +1044,21 @@ extern "C" int li_attn_decode_parts(int splits) { return splits < 1 ? 0 : splits
 template <class T, int W>
 static int launch_decode(const void* q, void* out, float* part_o, float* part_ml, CachePtrs c, const int* seq_slot,
                          const int* seq_ctx, int n_seqs, int H, int K, float scale, int window, int parts,
-                         AttnExtras ex, hipStream_t stream) {
+                         bool steady, AttnExtras ex, hipStream_t stream) {
     const int G = H / K;
-    const bool few = HD % 32 == 0 && G <= 16;                // (more query heads of a KV head, or other head sizes: tiles of 32 rows)
+    // Tiles of 16 rows, unless a KV head serves more query heads or the head size is another.  `steady` (the caller's rule:
+    // engine/step.py): a full chip whose waves walk 32 pages and more, all of them to about the same end.  These take tiles of 32
+    // rows and the page table's entries as they come: 32 / 8 heads of 128, us so and with tiles of 16 rows and entries ahead: batch 8 at
+    // 32,768 tokens in 16 splits 191.0 and 197.2, 16 at 16,384 in 8 191.4 and 198.6, 64 at 8,100 350.8 in 2 and 360.0 in 4, 128
+    // at 8,224 in one 705.7 and 715.0; heads of 64, 64 at 8,224 178.9 in 2 and 185.8 in 4.  Short of that (batch 8 at 8,224 58.6
+    // and 57.9, at 16,384 100.5 and 101.3) or with contexts of 1,000 to 8,192 (64: 266.4 and 238.9) the others are as fast or faster.
+    const bool by_32 = steady && HD <= 128, few = HD % 32 == 0 && G <= 16 && !by_32;
     const int rows = few ? 16 : 32;
     dim3 grid(n_seqs, K * ((G + rows - 1) / rows), parts), block(64 * W);
     const size_t lds = (size_t)W * (G < rows ? G : rows) * (HD + 4 + 2) * sizeof(float);
-    auto kfn = attn_decode_kernel<T, W, WaveAttn<T>>;
-    if constexpr (HD % 32 == 0) if (few) kfn = attn_decode_kernel<T, W, WaveAttn16<T>>;
+    auto kfn = attn_decode_kernel<T, W, WaveAttn<T>, true>;
+    if constexpr (HD % 32 == 0) if (few) kfn = attn_decode_kernel<T, W, WaveAttn16<T>, true>;
+    if constexpr (HD <= 128) if (by_32) kfn = attn_decode_kernel<T, W, WaveAttn<T>, false>;
     if (lds > 48 * 1024 &&
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return LI_HIP_ERROR;
@@ -1052,7 +1073,7 @@ static int launch_decode(const void* q, void* out, float* part_o, float* part_ml
 
 extern "C" int li_attn_decode(const void* q, void* out, int dt, const void* k, const void* v, int64_t page_stride,
                               const int* page_table, int max_pages, const int* seq_slot, const int* seq_ctx,
-                              int n_seqs, int H, int K, float scale, int window, int splits, float* part_o,
+                              int n_seqs, int H, int K, float scale, int window, int splits, int steady, float* part_o,
                               float* part_ml, int key_block, const float* sink, const float* slopes, const float* gate,
                               int gate_stride, int gate_col, int gate_elem, float softcap, int keep, hipStream_t stream) {
     if (check_heads(H, K) || splits < 1 || splits > 64) return LI_BAD_ARG;
@@ -1066,9 +1087,9 @@ extern "C" int li_attn_decode(const void* q, void* out, int dt, const void* k, c
     if (n_seqs <= 0) return LI_OK;
     CachePtrs c{k, v, page_stride, page_table, max_pages};
 #define GO(T)                                                                                                      \
-    (w == 4 ? launch_decode<T, 4>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, ex, stream) \
-     : w == 2 ? launch_decode<T, 2>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, ex, stream) \
-              : launch_decode<T, 1>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, ex, stream))
+    (w == 4 ? launch_decode<T, 4>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, steady != 0, ex, stream) \
+     : w == 2 ? launch_decode<T, 2>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, steady != 0, ex, stream) \
+              : launch_decode<T, 1>(q, out, part_o, part_ml, c, seq_slot, seq_ctx, n_seqs, H, K, scale, window, parts, steady != 0, ex, stream))
     return dt == DT_F16 ? GO(f16) : GO(bf16);
 #undef GO
 }

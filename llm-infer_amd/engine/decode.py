@@ -16,7 +16,7 @@ import torch
 
 from ..kernels import ops
 from ..tensor import Tensor
-from .step import StepShared, decode_splits, page_shares, page_splits, split_bucket
+from .step import StepShared, decode_splits, page_shares, page_splits, split_bucket, steady_pages, steady_splits
 
 
 @contextlib.contextmanager
@@ -52,23 +52,26 @@ class PlainDecodeRunner:
 
 class _GraphContext(StepShared):
     """The step description of a recorded decode step: fixed device buffers.  The lengths of the
-    sequences are known to it only as a bucket (``split_bucket``), which is what the split count of a
-    decode attention depends on."""
+    sequences are known to it only as a bucket (``split_bucket``) and, where they are all about as long, pages
+    (``steady_pages``), which is what the split count of a decode attention depends on."""
     is_decode = True
 
-    def __init__(self, bufs, n, bucket):
+    def __init__(self, bufs, n, bucket, pages=0):
         self.n_seqs = self.n_tokens = self.n_want = n
         self.token_ids, self.pos, self.seq_ctx = bufs["tokens"][:n], bufs["pos"][:n], bufs["ctx"][:n]
         self.tok_slot = self.seq_slot = bufs["slots"][:n]
         self.want_rows = bufs["rows"][:n]
         self.device = self.token_ids.device
-        self._bucket = bucket
+        self._bucket, self.steady_pages = bucket, pages
 
     def decode_splits(self, n_kv_heads, n_heads):
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket)
 
-    def page_splits(self, n_kv_heads, n_heads, head_dim=128):
-        return page_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket, head_dim)
+    def page_splits(self, n_kv_heads, n_heads, head_dim=128, reach=None):
+        return page_splits(self.n_seqs, n_kv_heads, n_heads, self._bucket, head_dim, self.steady_pages, reach)
+
+    def steady_splits(self, n_kv_heads, n_heads, head_dim, splits, reach=None):
+        return steady_splits(self.n_seqs, n_kv_heads, n_heads, head_dim, splits, self.steady_pages, reach)
 
     def page_shares(self, n_kv_heads, n_heads):
         return page_shares(self.n_seqs, n_kv_heads, n_heads, self._bucket)
@@ -91,7 +94,7 @@ def batch_bucket(n: int, limit: int) -> int:
 class GraphDecodeRunner:
     """Replays a recorded step while the set of live sequences stays the same; when it
     changes, the slots and tokens are uploaded anew and the graph of the new size is used.
-    A step is keyed by (rows, bucket of context lengths, sampling mode): the rows are the number of live
+    A step is keyed by (rows, bucket of context lengths, pages of contexts that are all about as long, sampling mode): the rows are the number of live
     sequences rounded up to a ``batch_bucket`` (idle rows run on the cache's scratch slot and their tokens
     are dropped); the temperature is read from the device, so it is no part of the key.  The first step of an
     engine is run eagerly (whatever is built or loaded at first use must not happen while a graph is being
@@ -123,9 +126,9 @@ class GraphDecodeRunner:
         wanted = [w for w in wanted if w is not None]
         self._table = wanted[0] if len(wanted) == 1 else None
 
-    def _body(self, n, bucket):
+    def _body(self, n, bucket, pages):
         eng, b = self.engine, self.bufs
-        ctx = _GraphContext(b, n, bucket)
+        ctx = _GraphContext(b, n, bucket, pages)
         table = ops.decode_prepare(b["slots"], eng.cache.lens_dev, b["pos"], b["ctx"], n, eng.cache.scratch_slot,
                                    self._table[1] if self._table else None)
         if table is not None:
@@ -150,23 +153,23 @@ class GraphDecodeRunner:
             b["slots"][:rows].copy_(torch.tensor(padded, dtype=torch.int32))
             b["tokens"][:rows].copy_(torch.tensor(list(tokens) + [0] * (rows - n), dtype=torch.int32))
             self.current = padded
-        bucket = split_bucket(max(new_lens))
+        bucket, pages = split_bucket(max(new_lens)), steady_pages(new_lens)
         hot = self.sampler.temperature > 0.0
         if hot and b.get("temperature_value") != self.sampler.temperature:
             b["temperature"].fill_(self.sampler.temperature)
             b["temperature_value"] = self.sampler.temperature
-        key = (rows, bucket, hot)
+        key = (rows, bucket, pages, hot)
         graphs, counts = eng._graphs, eng.decode_counts
         entry = graphs.pop(key, None)            # taken out and put back: the dict is in order of last use
         if entry is None and not graphs:
-            self._body(rows, bucket)             # the engine's first decode step
+            self._body(rows, bucket, pages)             # the engine's first decode step
             entry = "seen"
             counts["eager"] += 1
         else:
             if entry is None or entry == "seen":
                 g = torch.cuda.CUDAGraph()
                 with recording(g):
-                    self._body(rows, bucket)
+                    self._body(rows, bucket, pages)
                 entry = g
                 counts["recorded"] += 1
             else:

@@ -144,10 +144,10 @@ class PrefillRecorder:
         return packed
 
     @staticmethod
-    def _decode_context(buf, rows, wants, bucket):
+    def _decode_context(buf, rows, wants, bucket, pages=0):
         n = (rows + 3) // 4 * 4
         fields = {name: buf[i * n:] for i, name in enumerate(("tokens", "pos", "ctx", "slots", "rows"))}
-        ctx = _GraphContext(fields, rows, bucket)
+        ctx = _GraphContext(fields, rows, bucket, pages)
         ctx.n_want, ctx.want_rows = wants, fields["rows"][:wants]
         return ctx
 
@@ -157,7 +157,7 @@ class PrefillRecorder:
         its key is seen, or the second)."""
         rows, seqs, wants, bucket = ctx.n_tokens, ctx.n_seqs, ctx.n_want, None
         if ctx.is_decode:
-            bucket = split_bucket(ctx.max_ctx)
+            bucket = (split_bucket(ctx.max_ctx), ctx.steady_pages)
         else:
             rows, seqs = batch_bucket(rows, MAX_TOKENS), batch_bucket(seqs, MAX_SEQS)
             wants = batch_bucket(wants, rows)
@@ -184,7 +184,7 @@ class PrefillRecorder:
             graph = torch.cuda.CUDAGraph()
             with recording(graph):
                 if ctx.is_decode:
-                    rec = self._decode_context(buf, rows, wants, bucket)
+                    rec = self._decode_context(buf, rows, wants, *bucket)
                 else:
                     fields = {name: buf[at:at + n] for name, (at, n) in layout.items()}
                     tiles = {"tile_seq": fields.pop("tile_seq"), "tile_q0": fields.pop("tile_q0"), "n_tiles": layout["tile_seq"][1]}

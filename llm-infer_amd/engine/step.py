@@ -2,6 +2,8 @@
 their sequences, and where their sequences live in the cache."""
 from __future__ import annotations
 
+import math
+
 import numpy as np
 import torch
 
@@ -38,6 +40,7 @@ class StepContext(StepShared):
         self.n_tokens = sum(qlens)
         self.is_decode = all(q == 1 for q in qlens) and all(l >= 1 for l in lens_before)
         self.max_ctx = max((l + q for l, q in zip(lens_before, qlens)), default=0)
+        self.steady_pages = steady_pages([l + q for l, q in zip(lens_before, qlens)])
         self.host_slots, self.host_qlens, self.host_lens_before = list(slots), qlens, list(lens_before)
         qstart = np.concatenate([[0], np.cumsum(qlens)])[:-1] if qlens else np.zeros(0)
         flat = [t for seq in tokens for t in seq]
@@ -71,10 +74,15 @@ class StepContext(StepShared):
         """How many ways the decode attention of a mixer with these heads cuts each sequence's context."""
         return decode_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx))
 
-    def page_splits(self, n_kv_heads: int, n_heads: int, head_dim: int = 128) -> int:
+    def page_splits(self, n_kv_heads: int, n_heads: int, head_dim: int = 128, reach: int | None = None) -> int:
         """The same for the kernel whose waves merge inside a workgroup, where a page a split can be worth it (``head_dim``: the
-        line between the two depends on it; a mixer that does not say gets that of 128)."""
-        return page_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx), head_dim)
+        line between the two depends on it; a mixer that does not say gets that of 128; ``reach``: the most positions that a
+        token sees)."""
+        return page_splits(self.n_seqs, n_kv_heads, n_heads, split_bucket(self.max_ctx), head_dim, self.steady_pages, reach)
+
+    def steady_splits(self, n_kv_heads: int, n_heads: int, head_dim: int, splits: int, reach: int | None = None) -> bool:
+        """Whether so many splits are what ``ops.attention_decode`` calls steady; ``reach``: the most positions that a token sees."""
+        return steady_splits(self.n_seqs, n_kv_heads, n_heads, head_dim, splits, self.steady_pages, reach)
 
     def page_shares(self, n_kv_heads: int, n_heads: int) -> int:
         """The same for the kernels in which a split is a workgroup of four waves."""
@@ -101,24 +109,56 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
     return 1 << (s.bit_length() - 1)
 
 
-def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int, head_dim: int) -> int:
+def steady_pages(lens) -> int:
+    """Pages (the nearest power of two) of the contexts of a step whose sequences are all about as long, the shortest at least
+    seven eighths of the longest; 0 for other steps, and where that is less than 64.  It is what a recorded step knows beside the
+    bucket (``split_bucket``)."""
+    shortest = min(lens, default=0)
+    if shortest == 0 or 8 * shortest < 7 * max(lens):
+        return 0
+    pages = 1 << round(math.log2((shortest + PAGE - 1) // PAGE))
+    return pages if pages >= 64 else 0
+
+
+def steady_splits(n_seqs: int, n_kv_heads: int, n_heads: int, head_dim: int, splits: int, pages: int, reach: int | None = None) -> bool:
+    """Whether a decode step's splits fill the chip with waves that walk long chains of pages to the same end (``pages``:
+    ``steady_pages``; ``reach``: the most positions that a token sees), for which ``ops.attention_decode`` has another form of its kernel."""
+    # measured on MI355X at 8 and 32 KV heads, all contexts of one length, the other form and this one (figures of heads of 128 beside
+    # it, in attention.hip): with 768 waves neither is the faster one (batch 24 at 16,384 264.5 and 278.3, 12 281.6 and 271.1 at
+    # 32,768; heads of 64, batch 48 at 8,192 145.7 and 169.1); two splits, which the other form takes as four, from 32 pages each
+    # on (64 at 4,096 194.6 and 191.3, of 64 96.4 and 93.4), one from 64 on (128 at 2,048 197.3 and 198.8, at 4,096 365.3 and
+    # 361.2), more from as many bytes on as 32 pages of heads of 128 (of 64, 16 at 16,384 96.7 and 98.8, at 32,768 187.9 and
+    # 184.4).  Other heads: the other form (64 at 8,192, of 96 271 and 272, of 80 254 and 258; of 32 by a third, of 256 three times)
+    if head_dim not in (64, 112, 128) or splits != decode_splits(n_seqs, n_kv_heads, n_heads, 64):
+        return False
+    if reach:
+        pages = min(pages, reach // PAGE)
+    waves = splits * n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 31) // 32)
+    return waves >= 1024 and pages >= splits * {1: 64, 2: 32}.get(splits, 4096 // head_dim)
+
+
+def page_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int, head_dim: int, pages: int = 0, reach: int | None = None) -> int:
     """Splits for the softmax decoder's decode kernel (``ops.attention_decode``): as ``decode_splits``, but down to one page a
     split (a bucket stands for 2 to 4 times as many pages, the first for 1 to 3), at most 64.  Heads of up to 160 are not split
-    beyond four, which merge inside a workgroup, for more waves than half the chip's SIMDs, and those below 128 not into eight."""
-    # measured on MI355X with tiles of 32 rows, us with half as many splits and with these.  Heads of 128, 8 KV heads, batch 1 at 40 tokens 6.2 and 6.1,
-    # at 100 7.5 and 6.3, at 250 7.6 and 6.7, at 500 8.2 and 8.6, at 777 10.3 and 9.2 (with a soft cap and gates 12.5 and 10.3), at 1,000
-    # 9.9 and 9.0, at 2,000 11.3 and 10.4, at 4,000 14.1 and 11.7; batch 32 at 250 10.7 and 10.5.  Not taken (what more would take): 128,
-    # batch 16 at 500 11.3 (13.1), at 900 15.5 (17.9), batch 4 at 4,000 18.1 (18.6), batch 8 at 1,900 17.0 (17.8), batch 2 at 8,000 18.6
-    # (19.6); 64, batch 1 at 500 7.6 (8.6), at 900 8.5 (8.7), batch 8 at 500 8.6 (10.2), at 900 11.0 (10.6); 96, batch 1 at 700 8.1
-    # (9.0), batch 8 at 900 12.1 (11.8); 160, 4 KV heads, 64 splits at 8,000 19.0 (20.0).  Heads of 256, 2 KV heads, whose pages are
-    # longer: batch 1 at 500 30 and 18, batch 32 at 1,000 67 and 49
-    # Two splits where four would make more than 1,024 waves: four after all, since two waves of the tile of 16 rows share a SIMD.  8 KV heads, us in two and four: heads of 128, batch 40 at 16 to 528 tokens 17.7 and
-    # 15.4, 48 21.0 and 19.0, 64 20.4 and 18.8, 48 at 16 to 1,000 31.5 and 27.2, 64 at 900 48.3 and 48.8, at 4,000 179.8
-    # and 177.1, at 8,000 362 and 346 (tiles of 32 rows, two splits: 174.5 and 354); heads of 64, 48 at 16 to 528 10.8 and 10.1, 64 at 16 to 1,000 22.7 and 19.7
+    beyond four, which merge inside a workgroup, for more waves than half the chip's SIMDs, and those below 128 not into eight.
+    ``pages``, ``reach``: as for ``steady_splits``."""
+    # measured on MI355X with tiles of 32 rows, us with half as many splits and with these.  Heads of 128, 8 KV heads, batch 1 at 40
+    # tokens 6.2 and 6.1, at 100 7.5 and 6.3, at 250 7.6 and 6.7, at 500 8.2 and 8.6, at 777 10.3 and 9.2 (with a soft cap and gates 12.5
+    # and 10.3), at 1,000 9.9 and 9.0, at 2,000 11.3 and 10.4, at 4,000 14.1 and 11.7; batch 32 at 250 10.7 and 10.5.  Not taken
+    # (what more would take): 128, batch 16 at 500 11.3 (13.1), at 900 15.5 (17.9), batch 4 at 4,000 18.1 (18.6), batch 8 at 1,900
+    # 17.0 (17.8), batch 2 at 8,000 18.6 (19.6); 64, batch 1 at 500 7.6 (8.6), at 900 8.5 (8.7), batch 8 at 500 8.6 (10.2), at 900
+    # 11.0 (10.6); 96, batch 1 at 700 8.1 (9.0), batch 8 at 900 12.1 (11.8); 160, 4 KV heads, 64 splits at 8,000 19.0 (20.0).  Heads
+    # of 256, 2 KV heads, whose pages are longer: batch 1 at 500 30 and 18, batch 32 at 1,000 67 and 49
+    # Two splits where four would make more than 1,024 waves: four after all, since two waves of the tile of 16 rows share a SIMD,
+    # unless the two are steady.  8 KV heads, us in two and four: heads of 128, batch 40 at 16 to 528 tokens 18.2 and 18.2, 48 18.7 and
+    # 18.7, 64 20.8 and 20.9, 64 at 900 57.0 and 55.7, at 1,056 65.1 and 61.8, at 1,000 to 8,192 245.7 and 238.9; heads of 64,
+    # 48 at 16 to 528 11.1 and 10.9, 64 at 1,056 33.3 and 30.0.  More than 512 waves in one split keep the one (open: us in one,
+    # two and four of heads of 128, 65 at 16 to 528 23.0, 21.4 and 20.8, 96 26.3, 25.5 and 27.7, 128 38.8, 38.6 and 38.7; 96 at 1,000
+    # 72.7, 76.7 and 78.9, 128 at 2,048 183.1, 186.5 and 191.0; 32 KV heads, 17 at 2,000 107.5, 109.5 and 112.0)
     few, many = (decode_splits(n_seqs, n_kv_heads, n_heads, min(b, 64)) for b in (bucket, 2 * bucket))
     waves = many * n_seqs * n_kv_heads * ((n_heads // n_kv_heads + 31) // 32)
     if few == many == 2 and head_dim <= 128 and head_dim % 32 == 0 and n_heads <= 16 * n_kv_heads:
-        return 4
+        return 2 if steady_splits(n_seqs, n_kv_heads, n_heads, head_dim, 2, pages, reach) else 4
     return few if head_dim <= 160 and many > 4 and (waves > 512 or (few == 4 and head_dim < 128) or (many == 64 and head_dim > 128)) else many
 
 

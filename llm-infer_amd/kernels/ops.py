@@ -827,9 +827,10 @@ def attention_prefill(q, kv, meta, n_heads, n_kv_heads, head_dim, scale, window,
 
 def attention_decode(q, kv, seq_slot, seq_ctx, n_seqs, n_heads, n_kv_heads, head_dim, scale, window,
                      splits: int = 1, block=None, sink=None, slopes=None, gate=None, gate_col: int = 0, softcap: float | None = None, gate_elem: bool = False,
-                     keep_first: int = 0) -> torch.Tensor:
+                     keep_first: int = 0, steady: bool = False) -> torch.Tensor:
     """16-bit attention for one new token per sequence; q [B, H, hd].  ``block``, ``sink``, ``slopes``, ``gate``,
-    ``gate_elem``, ``softcap``, ``keep_first``: as for ``attention_prefill``."""
+    ``gate_elem``, ``softcap``, ``keep_first``: as for ``attention_prefill``.  ``steady``: the splits are many long chains of pages of about the
+    same length (``step.steady_splits``), for which another form of the kernel is the faster one."""
     k_pages, v_pages, page_stride, page_table = kv
     _dev(q, k_pages, v_pages, page_table, seq_slot, seq_ctx, sink, slopes, gate)
     for name, vec in (("sink", sink), ("slopes", slopes)):
@@ -853,7 +854,7 @@ def attention_decode(q, kv, seq_slot, seq_ctx, n_seqs, n_heads, n_kv_heads, head
     _check(lib.li_attn_decode(
         _ptr(q), _ptr(out), DT[q.dtype], _ptr(k_pages), _ptr(v_pages), c_int64(page_stride), _ptr(page_table),
         page_table.shape[1], _ptr(seq_slot), _ptr(seq_ctx), n_seqs, n_heads, n_kv_heads, c_float(scale),
-        int(window or 0), splits, _ptr(part_o), _ptr(part_ml), int(block or 0), _ptr(sink), _ptr(slopes), _ptr(gate),
+        int(window or 0), splits, int(steady), _ptr(part_o), _ptr(part_ml), int(block or 0), _ptr(sink), _ptr(slopes), _ptr(gate),
         gate.stride(0) if gate is not None else 0, int(gate_col), int(bool(gate_elem and gate is not None)),
         c_float(softcap or 0.0), int(keep_first), _stream()), "attn_decode")
     return out

@@ -89,8 +89,9 @@ class Attention(Part):
         if self.dtype == torch.float32:
             a = ops.attention_f32(q, kv, ctx.pos, ctx.tok_slot, H, K, hd, self.scale, self.window)
         elif ctx.is_decode:
+            splits = ctx.page_splits(K, H, hd, self.window)
             a = ops.attention_decode(q, kv, ctx.seq_slot, ctx.seq_ctx, ctx.n_seqs, H, K, hd, self.scale,
-                                     self.window, ctx.page_splits(K, H, hd))
+                                     self.window, splits, steady=ctx.steady_splits(K, H, hd, splits, self.window))
         else:
             a = ops.attention_prefill(q, kv, ops.prefill_meta(ctx), H, K, hd, self.scale, self.window)
         ops.linear(a.view(a.shape[0], H * hd), self.wo, ops.EPI_ADD, out=residual)

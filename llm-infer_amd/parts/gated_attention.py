@@ -182,10 +182,16 @@ class GatedAttention(Part):
                 shares = min(shares, max(1, (span + self.keep_first) // 128))
         return shares
 
+    @property
+    def reach(self) -> int | None:
+        """The most positions that a token sees, None without a mask."""
+        spans = [n for n in (self.block, self.window) if n]
+        return min(spans) + self.keep_first if spans else None
+
     def _splits(self, ctx) -> int:
         """Splits of the keys for the softmax decoder's decode kernel: what the step asks for, but at least a page a split of
         what the mask leaves (a power of two)."""
-        splits = ctx.page_splits(self.n_kv_heads, self.n_heads, self.head_dim)
+        splits = ctx.page_splits(self.n_kv_heads, self.n_heads, self.head_dim, self.reach)
         for span in (self.block, self.window):
             if span:
                 splits = min(splits, max(1, (span + self.keep_first) // 64))
@@ -218,9 +224,10 @@ class GatedAttention(Part):
             # a wave per (sequence, key/value head, split of the keys that the mask leaves))
             gate, gate_col = proj if self.gate else None, col0 + self.gate_col
             if ctx.is_decode:
+                splits = self._splits(ctx)
                 a = ops.attention_decode(q, kv, ctx.seq_slot, ctx.seq_ctx, ctx.n_seqs, H, G, d, self.scale, self.window,
-                                         self._splits(ctx), self.block, self.sinks, self.slopes, gate, gate_col, self.softcap, self.gate_elem,
-                                         self.keep_first)
+                                         splits, self.block, self.sinks, self.slopes, gate, gate_col, self.softcap, self.gate_elem,
+                                         self.keep_first, ctx.steady_splits(G, H, d, splits, self.reach))
             else:
                 a = ops.attention_prefill(q, kv, ops.prefill_meta(ctx), H, G, d, self.scale, self.window, self.block, self.sinks,
                                           self.slopes, gate, gate_col, self.softcap, self.gate_elem, self.keep_first)

@@ -265,6 +265,36 @@ def test_splits_down_to_one_page():
     assert page_shares(32, 1, 32, 16) == 8 and page_shares(64, 8, 32, 16) == 1 and page_shares(8, 8, 32, 4) == 4
 
 
+def test_long_contexts_of_one_length_keep_their_splits_and_their_form():
+    """Two splits become four, and tiles of 16 rows take over, but not where the waves of a full chip walk many pages to the same end."""
+    from llm_infer_amd.engine.decode import _GraphContext
+    from llm_infer_amd.engine.step import StepContext, page_splits, steady_pages, steady_splits
+    assert [steady_pages([n] * 3) for n in (0, 1, 2880, 2881, 4096, 5760, 5761 + 64, 8192, 16384, 32700, 100_000)] == [0, 0, 0, 64, 64, 64, 128, 128, 256, 512, 2048]
+    assert steady_pages([8192, 7168]) == 128 and steady_pages([8192, 7167]) == 0 and steady_pages([]) == 0
+    bufs = {name: torch.zeros(64, dtype=torch.int32) for name in ("tokens", "pos", "ctx", "slots", "rows")}
+
+    def of_both(n, lens, k, h, hd, reach=None):
+        eager = StepContext("cpu", list(range(n)), [[1]] * n, [v - 1 for v in lens], [[0]] * n, upload=False)
+        recorded = _GraphContext(bufs, n, split_bucket(max(lens)), steady_pages(lens))
+        out = []
+        for step in (eager, recorded):
+            splits = step.page_splits(k, h, hd, reach)
+            out.append((splits, step.steady_splits(k, h, hd, splits, reach)))
+        assert out[0] == out[1]
+        return out[0]
+    # batch, lengths, KV heads, heads, head size -> splits, steady
+    for n, lens, k, h, hd, want in ((64, 8190, 8, 32, 128, (2, True)), (64, 2000, 8, 32, 128, (4, False)), (48, 8190, 8, 32, 128, (4, False)),
+                                    (8, 8190, 8, 32, 128, (16, False)), (8, 32700, 8, 32, 128, (16, True)), (32, 4000, 8, 32, 128, (4, False)),
+                                    (16, 300, 32, 32, 128, (4, False)), (16, 4090, 32, 32, 128, (2, True)), (64, 8190, 8, 32, 32, (4, False)),
+                                    (16, 16380, 8, 32, 64, (8, False)), (16, 32700, 8, 32, 64, (8, True)), (64, 8190, 2, 16, 256, (8, False))):
+        assert of_both(n, [lens] * n, k, h, hd) == want, (n, lens, k, h, hd)
+    assert of_both(64, [1000] + [8190] * 63, 8, 32, 128) == (4, False)                  # lengths of their own
+    assert of_both(64, [8190] * 64, 8, 32, 128, 1024) == (4, False)                    # a window: few pages however long the context
+    # both sides of 512 waves in one split
+    assert [page_splits(n, 8, 32, 4, 128) for n in (32, 33, 64, 65, 128)] == [4, 4, 4, 1, 1] and [page_splits(n, 32, 32, 4, 128) for n in (8, 16, 17)] == [4, 4, 1]
+    assert page_splits(128, 8, 32, 32, 128, 64) == 1 and steady_splits(128, 8, 32, 128, 1, 64) and not steady_splits(128, 8, 32, 128, 1, 32)
+
+
 def test_splits_asked_of_a_step_without_a_head_size():
     """A mixer may leave the head size out, in a step and in a recorded one."""
     from llm_infer_amd.engine.decode import _GraphContext

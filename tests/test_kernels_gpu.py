@@ -702,8 +702,10 @@ def test_attention_whole_prompts_and_decode(ops, H, K, hd, lens, dt):
 
 
 # query heads of a KV head around the 16 rows of the narrow tile (beyond them the tile of 32 rows, and chunks of it), for head sizes
-# of one 32 up to the largest; contexts of one key, at the edges of a score tile's eights and of a page
-@pytest.mark.parametrize("G,K,hd", [(1, 2, 32), (15, 1, 64), (16, 2, 128), (17, 1, 128), (4, 3, 96), (33, 1, 32), (7, 1, 256), (16, 1, 160)])
+# of one 32 up to the largest, and sizes of 16 that are none of 32; contexts of one key, at the edges of a score tile's eights and of a
+# page; the form for steady splits too (heads of up to 128 have it, the others take no notice)
+@pytest.mark.parametrize("G,K,hd", [(1, 2, 32), (15, 1, 64), (16, 2, 128), (17, 1, 128), (4, 3, 96), (33, 1, 32), (7, 1, 256), (16, 1, 160),
+                                    (3, 2, 80), (18, 1, 112), (33, 2, 64)])
 @pytest.mark.parametrize("dt", F16S)
 def test_decode_attention_in_tiles_of_16_and_32_rows(ops, G, K, hd, dt):
     g = torch.Generator().manual_seed(G * 100 + hd)
@@ -731,9 +733,10 @@ def test_decode_attention_in_tiles_of_16_and_32_rows(ops, G, K, hd, dt):
                 p = torch.softmax(s, 1)
             refs.append(torch.einsum("hn,nhd->hd", p, v.double().repeat_interleave(G, 1)))
         kw = {name: t.to(DEV) if torch.is_tensor(t) else t for name, t in extra.items() if name != "window"}
-        for splits in (1, 2, 4, 8):
-            out = ops.attention_decode(q.to(DEV), view.as_tuple(), slot, ctx, len(lens), H, K, hd, scale, extra.get("window"), splits, **kw)
-            assert (out.double().cpu() - torch.stack(refs)).abs().max().item() < tol, (splits, list(extra))
+        for splits, steady in ((1, False), (2, False), (4, False), (8, False), (1, True), (2, True), (4, True), (8, True)):
+            out = ops.attention_decode(q.to(DEV), view.as_tuple(), slot, ctx, len(lens), H, K, hd, scale, extra.get("window"), splits,
+                                       steady=steady, **kw)
+            assert (out.double().cpu() - torch.stack(refs)).abs().max().item() < tol, (splits, steady, list(extra))
 
 
 # many tokens, so that heads of a KV head share a workgroup (as many as 256 / hd holds and H / K has divisors for); lengths at
