@@ -112,9 +112,10 @@ def decode_splits(n_seqs: int, n_kv_heads: int, n_heads: int, bucket: int) -> in
 def steady_pages(lens) -> int:
     """Pages (the nearest power of two) of the contexts of a step whose sequences are all about as long, the shortest at least
     seven eighths of the longest; 0 for other steps, and where that is less than 64.  It is what a recorded step knows beside the
-    bucket (``split_bucket``)."""
+    bucket (``split_bucket``), so it is 0 for fewer than 8 sequences too: their splits are short of a full chip, or of 32 pages up
+    to contexts of 64 thousand, and a long conversation is not recorded anew for it."""
     shortest = min(lens, default=0)
-    if shortest == 0 or 8 * shortest < 7 * max(lens):
+    if len(lens) < 8 or shortest == 0 or 8 * shortest < 7 * max(lens):
         return 0
     pages = 1 << round(math.log2((shortest + PAGE - 1) // PAGE))
     return pages if pages >= 64 else 0

@@ -269,8 +269,8 @@ def test_long_contexts_of_one_length_keep_their_splits_and_their_form():
     """Two splits become four, and tiles of 16 rows take over, but not where the waves of a full chip walk many pages to the same end."""
     from llm_infer_amd.engine.decode import _GraphContext
     from llm_infer_amd.engine.step import StepContext, page_splits, steady_pages, steady_splits
-    assert [steady_pages([n] * 3) for n in (0, 1, 2880, 2881, 4096, 5760, 5761 + 64, 8192, 16384, 32700, 100_000)] == [0, 0, 0, 64, 64, 64, 128, 128, 256, 512, 2048]
-    assert steady_pages([8192, 7168]) == 128 and steady_pages([8192, 7167]) == 0 and steady_pages([]) == 0
+    assert [steady_pages([n] * 8) for n in (0, 1, 2880, 2881, 4096, 5760, 5761 + 64, 8192, 16384, 32700, 100_000)] == [0, 0, 0, 64, 64, 64, 128, 128, 256, 512, 2048]
+    assert steady_pages([8192] * 7 + [7168]) == 128 and steady_pages([8192] * 7 + [7167]) == steady_pages([8192] * 7) == steady_pages([]) == 0
     bufs = {name: torch.zeros(64, dtype=torch.int32) for name in ("tokens", "pos", "ctx", "slots", "rows")}
 
     def of_both(n, lens, k, h, hd, reach=None):
