@@ -78,6 +78,7 @@ class PrefillRecorder:
         self.step_graphs = {}              # steps of one token: key -> (graph, logits, index arrays)
         self._step_seen = {}               # those called for once or twice: key -> "once" | "seen"
         self.counts = {"eager": 0, "recorded": 0, "replayed": 0}
+        self._stream = None                # where the last recording was replayed
 
     # -- which steps ---------------------------------------------------------------
     def takes(self, eng, ctx) -> bool:
@@ -179,6 +180,11 @@ class PrefillRecorder:
         else:
             layout, total = self._layout(rows, seqs, wants)
             packed = self._fill(ctx, layout, total, eng.cache.scratch_slot)
+        # a recording's index arrays and results are its own: a step on another stream waits for the one before it
+        stream = torch.cuda.current_stream(eng.device)
+        if self._stream is not None and stream != self._stream:
+            stream.wait_stream(self._stream)
+        self._stream = stream
         if entry == "seen":
             buf = torch.from_numpy(packed).to(eng.device)
             graph = torch.cuda.CUDAGraph()

@@ -417,6 +417,7 @@ def test_recorded_prompts_and_single_token_steps_do_not_push_each_other_out(monk
     from llm_infer_amd.engine.step import StepContext
     waits = []
     monkeypatch.setattr(prefill, "recording", lambda graph: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: "one")
     monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: types.SimpleNamespace(replay=lambda: None))
     monkeypatch.setattr(torch.cuda, "synchronize", lambda: waits.append(1))
     eng = types.SimpleNamespace(device="cpu", cache=types.SimpleNamespace(scratch_slot=0), model=types.SimpleNamespace(
@@ -445,6 +446,37 @@ def test_recorded_prompts_and_single_token_steps_do_not_push_each_other_out(monk
             for want in range(1, n + 1):
                 rec.run(eng, StepContext("cpu", list(range(1, n + 1)), [[5]] * n, [before] * n, [[0]] * want + [[]] * (n - want), upload=False))
     assert max(len(rec.step_graphs), len(rec.graphs)) <= prefill.MAX_RECORDED and len(rec._step_seen) <= 16 * prefill.MAX_RECORDED
+
+
+def test_a_recorded_step_on_another_stream_waits_for_the_one_before(monkeypatch):
+    """A recording's index arrays are filled anew for every step and its results lie where the last one's lay: what runs on another
+    stream comes after what still reads them."""
+    import contextlib
+    import types
+    from llm_infer_amd.engine import prefill
+    from llm_infer_amd.engine.step import StepContext
+    did = []
+
+    class Stream:
+        def __init__(self, name):
+            self.name = name
+
+        def wait_stream(self, other):
+            did.append((self.name, "waits for", other.name))
+    streams = {name: Stream(name) for name in "ab"}
+    on = ["a"]
+    monkeypatch.setattr(prefill, "recording", lambda graph: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: streams[on[0]])
+    monkeypatch.setattr(torch.cuda, "CUDAGraph", lambda: types.SimpleNamespace(replay=lambda: did.append((on[0], "replays"))))
+    eng = types.SimpleNamespace(device="cpu", cache=types.SimpleNamespace(scratch_slot=0), model=types.SimpleNamespace(
+        forward=lambda ctx, cache: torch.zeros(ctx.n_want, 3)))
+    rec = prefill.PrefillRecorder()
+    for tokens, before, eager in ((1, 7, 2), (40, 0, 1)):                          # a step of one token, a prompt
+        did.clear()
+        for name in "aaaabba":
+            on[0] = name
+            rec.run(eng, StepContext("cpu", [3], [[5] * tokens], [before], [[0]], upload=False))
+        assert did == [("a", "replays")] * (4 - eager) + [("b", "waits for", "a")] + [("b", "replays")] * 2 + [("a", "waits for", "b"), ("a", "replays")]
 
 
 def test_cache_rounding_option_is_for_a_float32_cache():
