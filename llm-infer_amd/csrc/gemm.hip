@@ -934,11 +934,9 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
 }
 
 
-// Up to 128 rows of X against a tiled weight, every epilogue its own (gemm_rows).  nt: 1 or 2 tiles of 16 rows
-// of W a workgroup, kw: 4 or 8 waves that share K (8: up to 64 rows of X) (0: chosen here); ldx: elements from
-// one row of X to the next.  ro (or null; mode EPI_ADD, at most 16 rows, one tile a workgroup): RowsOut, with one
-// partial sum a row for each of the N / 16 workgroups.
-
+// Few rows of X against a tiled weight.  nt: 1 or 2 tiles of 16 rows of W a workgroup, -1 half a tile (up to 8 rows of X);
+// kw: 4 or 8 waves that share K; 0: chosen here.  ro (or null; mode EPI_ADD, at most 16 rows): RowsOut, with one partial sum a row
+// for each workgroup (li_gemv_tiled_blocks says how many).
 extern "C" int li_gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,
                              int M, int N, int K, int nt, int kw, const RopeStore* rs, const RowsOut* ro,
                              const RowScale* rsc, hipStream_t stream) {
@@ -968,6 +966,10 @@ extern "C" int li_gemv_tiled_groups(const void* X, const void* Wt, int dt, void*
                       XGroups{group_rows, groups, (int64_t)M * K}, NoExperts{}, stream);
 }
 
+// Up to 128 rows of X against a tiled weight, every epilogue its own (gemm_rows).  nt: 1 or 2 tiles of 16 rows
+// of W a workgroup, kw: 4 or 8 waves that share K (8: up to 64 rows of X) (0: chosen here); ldx: elements from
+// one row of X to the next.  ro (or null; mode EPI_ADD, at most 16 rows, one tile a workgroup): RowsOut, with one
+// partial sum a row for each of the N / 16 workgroups.
 extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode,
                             int M, int N, int K, int ldx, int nt, int kw, const RopeStore* rs, const RowsOut* ro,
                             hipStream_t stream) {

@@ -46,11 +46,14 @@ __device__ __forceinline__ void to_operand16(f32x4& v) {
 // is still taken in one order.  Bound by the stream of W: 128,256 x 2,048 at 3 rows 180 us, 5.8 TB/s (gemm_fma: 942 us);
 // 16,384 x 2,048 27 us, 5.0 TB/s (222); short products end a few us after their stream (2,048 x 2,048 9.7 us, 201 before;
 // 2,048 x 8,192 29, 862 before), and with a workgroup on half the CUs the matrix instructions take as long as the stream.
-// HALF (at most 8 rows of X): 8 rows of W a workgroup.  The lanes of r < 8 hold a chain of them, the others the next chain of the
-// same rows, and likewise the columns of X: of the 16 x 16 sums the two diagonal quarters are the two chains, each in its
-// order.  Twice the workgroups and no instruction more: 2,048 x 2,048 9.8 -> 7.6 us at 3 rows, 2,048 x 8,192 29.0 -> 19.6 (8 rows
-// 32.5 -> 24.0); 4,096 x 4,096 17.5 and 18.3, where every CU has its workgroup without it.  U steps of 16 k whose loads go out together: 4, so that eight waves fit a SIMD (with 16
-// the first of these takes 187 us, the second 37).
+// U steps of 16 k whose loads go out together: 4, so that eight waves fit a SIMD (with 16 the first of these takes 187 us, the
+// second 37).
+// HALF (at most 8 rows of X): 8 rows of W a workgroup, and wave w takes pairs of neighbouring chains, 2 w and 2 w + 1, then those
+// 2 KW on.  The lanes of r < 8 hold the first chain of a pair, the others the second of the same rows, and likewise the columns
+// of X: of the 16 x 16 sums the two diagonal quarters are the two chains, each in its order.  Twice the workgroups and no
+// instruction more: 2,048 x 2,048 9.8 -> 7.6 us at 3 rows, 2,048 x 8,192 29.0 -> 19.6 (8 rows 32.5 -> 24.0); 4,096 x 4,096 17.5
+// and 18.3, where every CU has its workgroup without it.  U is 8 here, four or five waves a SIMD: a CU has one workgroup anyway
+// (3 rows, U of 4 and 8: 2,048 x 512 7.8 and 5.9 us, 2,048 x 2,048 9.4 and 7.4, 2,048 x 8,192 19.6 and 19.3).
 // ===========================================================================
 template <int NT, int MT, int KW, int U, bool HALF = false>
 __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, Epilogue e) {
