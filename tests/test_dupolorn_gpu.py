@@ -232,6 +232,25 @@ def test_head_norm_of_every_width(lib, dv):
         assert ((got - ref).abs() <= 16 * 2.0 ** -24 * ref.abs() + 1e-7).all()
 
 
+@pytest.mark.parametrize("dv, times", [(1, 5), (33, 2), (127, 2), (129, 1), (200, 1), (511, 1), (512, 1)])
+def test_head_norm_is_the_same_kept_in_registers_or_not(lib, dv, times):
+    """A head followed by zeros up to ``4 ** times`` its width, with eps divided by as much, has 2 ** times the norm's factor,
+    exactly (powers of two): beyond 512 by the kernel that fetches its elements twice, up to there by the one that keeps them."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(dv)
+    H, rows, wide = 3, 5, dv * 4 ** times
+    assert wide > 512
+    y, gate, w = torch.randn(rows, H, dv, generator=g), torch.randn(rows, H, dv, generator=g), torch.randn(H, dv, generator=g)
+    eps = 2.0 ** -10
+
+    def run(width):
+        def pad(t):
+            return torch.nn.functional.pad(t, (0, width - dv)).reshape(*t.shape[:-2], H * width).contiguous().to(DEV)
+        gates = torch.cat([torch.zeros(rows, 1, device=DEV), pad(gate)], 1).contiguous()       # (a column ahead: no aligned rows)
+        return ops.gated_head_norm(pad(y), pad(w), gates, 1, H, eps * dv / width, torch.float32, True).view(rows, H, width)[..., :dv]
+    assert torch.equal(run(dv) * 2.0 ** times, run(wide))
+
+
 @pytest.mark.parametrize("taps", [1, 2, 3, 6])
 def test_convolution_ahead_of_a_mixer(lib, taps):
     """The convolution alone: whole, in portions shorter than its reach, and one token at a time."""

@@ -148,3 +148,18 @@ def test_gated_norm_of_every_width(part, groups):
     want = (v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-4)).view(3, n) * w.double()
     # an exponential, a division, a root and four products of 32 bits, and the sum of squares' own rounding: under 16 roundings
     assert ((got - want).abs() <= 16 * 2.0 ** -24 * want.abs() + 1e-7).all()
+
+
+@pytest.mark.parametrize("part", [4096, 5000, 8191, 8192])
+def test_gated_norm_is_the_same_kept_in_registers_or_not(part):
+    """A row followed by three times as many zeros, with a quarter of eps, has twice the norm's factor, exactly: beyond 8,192 elements
+    by the kernel that fetches them twice, up to there, with as many threads, by the one that keeps them."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(part)
+    y, z, w = torch.randn(3, part, generator=g), torch.randn(3, part, generator=g), torch.randn(part, generator=g)
+
+    def run(times):
+        def pad(t):
+            return torch.nn.functional.pad(t, (0, (times - 1) * part)).contiguous().to(DEV)
+        return ops.gated_group_norm(pad(y), pad(z), 0, pad(w), 1, 2.0 ** -10 / times, torch.float32)[:, :part]
+    assert torch.equal(2 * run(1), run(4))
