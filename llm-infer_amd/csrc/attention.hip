@@ -86,12 +86,12 @@ struct WaveAttn {
     __device__ __forceinline__ void load_k(const T* kpage, v8 (&kf)[2 * KS]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) kf[i] = *(const v8*)(kpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < 2 * KS; ++i) kf[i] = load_once<v8>(kpage + (i * 64 + lane) * 8);
     }
     __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[DB * 4]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < DB * 4; ++i) vf[i] = *(const v8*)(vpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < DB * 4; ++i) vf[i] = load_once<v8>(vpage + (i * 64 + lane) * 8);
     }
 
     // Scores of the page's keys (starting at key t0) against this wave's rows, mask, running
@@ -243,7 +243,7 @@ struct WaveAttn16 {
 #pragma unroll
             for (int x = 0; x < 2; ++x)
 #pragma unroll
-                for (int k = 0; k < QF; ++k) kf[(a * 2 + x) * QF + k] = *(const v8*)(p + ((a * KS + 2 * k) * 64 + 8 * x) * 8);
+                for (int k = 0; k < QF; ++k) kf[(a * 2 + x) * QF + k] = load_once<v8>(p + ((a * KS + 2 * k) * 64 + 8 * x) * 8);
     }
     __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[VF]) const {
         const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
@@ -251,7 +251,7 @@ struct WaveAttn16 {
 #pragma unroll
         for (int d = 0; d < OF; ++d)
 #pragma unroll
-            for (int a = 0; a < 2; ++a) vf[d * 2 + a] = *(const v8*)(p + (((d >> 1) * 4 + 2 * a) * 64 + 16 * (d & 1)) * 8);
+            for (int a = 0; a < 2; ++a) vf[d * 2 + a] = load_once<v8>(p + (((d >> 1) * 4 + 2 * a) * 64 + 16 * (d & 1)) * 8);
     }
     __device__ __forceinline__ int key_of(int tile, int r) const {
         const int g = (threadIdx.x & 63) >> 4;

@@ -322,7 +322,7 @@ __global__ __launch_bounds__(64 * KW) void experts_gemv_kernel(const T* __restri
             for (int u = 0; u < U; ++u) {
                 const bool in = s0 + u < s_end;
                 const v8 z = {};
-                a[u] = in ? *(const v8*)(wt + (int64_t)(s0 + u) * 512) : z;
+                a[u] = in ? load_once<v8>(wt + (int64_t)(s0 + u) * 512) : z;
 #pragma unroll
                 for (int j = 0; j < MT; ++j) b[u][j] = in && have[j] ? *(const v8*)(xrow[j] + (s0 + u) * 32) : z;
             }

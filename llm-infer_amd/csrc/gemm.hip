@@ -431,7 +431,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
             const bool in = s + later < s_end;
             const v8 z = {};
 #pragma unroll
-            for (int t = 0; t < NT; ++t) a[u][t] = in ? *(const v8*)(wt[t] + (int64_t)s * 512) : z;
+            for (int t = 0; t < NT; ++t) a[u][t] = in ? load_once<v8>(wt[t] + (int64_t)s * 512) : z;
 #pragma unroll
             for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
         }
@@ -633,7 +633,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(const T* __restrict_
                     const int step = 2 * dd + h;
                     const unsigned char* from = (in && step < steps) ? wbase[t] + (int64_t)step * 1024
                                                                      : (const unsigned char*)zero_kib;
-                    asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[u][h][t]) : "v"(woff), "s"(from) : "memory");
+                    asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[u][h][t]) : "v"(woff), "s"(from) : "memory");
                 }
         };
         // where lane (r, g) finds row r, chunk 4 h + g of fragment 0 in a stage: unit r / 8, place

@@ -424,7 +424,9 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     // the loop's head it would wait for every load in flight); the waits are placed by hand below.
     auto fetch_one = [&](int i, int half, v8 (&a)[NI]) {          // block i of the fragments of a half step
         const T* from = wsrc[i] + (int64_t)min(half, last) * 512;
-        asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
+        // (a tile with W three or four steps ahead holds all rows of X: W is read once, as by load_once)
+        if constexpr (A >= 3) asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
+        else asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
     };
 
     f32x4 acc[NI][MJ];
