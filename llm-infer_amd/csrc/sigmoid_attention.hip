@@ -52,15 +52,16 @@ struct WaveSigmoid {
 #pragma unroll
             for (int r = 0; r < 16; ++r) o[b][r] = 0.f;
     }
-    __device__ __forceinline__ void load_k(const T* kpage, v8 (&kf)[2 * KS]) const {
+    // (ONCE: straight from the cache's page, which nothing else reads)
+    template <bool ONCE> __device__ __forceinline__ void load_k(const T* kpage, v8 (&kf)[2 * KS]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) kf[i] = *(const v8*)(kpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < 2 * KS; ++i) kf[i] = ONCE ? load_once<v8>(kpage + (i * 64 + lane) * 8) : *(const v8*)(kpage + (i * 64 + lane) * 8);
     }
-    __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[DB * 4]) const {
+    template <bool ONCE> __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[DB * 4]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < DB * 4; ++i) vf[i] = *(const v8*)(vpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < DB * 4; ++i) vf[i] = ONCE ? load_once<v8>(vpage + (i * 64 + lane) * 8) : *(const v8*)(vpage + (i * 64 + lane) * 8);
     }
 
     // The weights of the page's 64 keys (the first is key t0) for this wave's rows: this lane's row sees keys
@@ -184,8 +185,8 @@ __global__ __launch_bounds__(256) void sigmoid_prefill_kernel(
             const T* ks = smem + stage * (KE + VE);
             const T* vs = ks + KE;
             v8 kf[2 * KS], vf[DB * 4];
-            a.load_k(ks, kf);
-            a.load_v(vs, vf);
+            a.template load_k<false>(ks, kf);
+            a.template load_v<false>(vs, vf);
             const bool inside = all_valid && p * PAGE >= lo_max && p * PAGE + PAGE - 1 <= pos_min;
             a.weights(kf, s, p * PAGE, lo, hi, scale2, bias2, !inside);
             a.mix(vf, s);
@@ -234,11 +235,11 @@ __global__ __launch_bounds__(64) void sigmoid_decode_kernel(
     f32x16 s[2];
     const T* kbase = (const T*)c.k + (int64_t)g * k_head_elems(KD);
     const T* vbase = (const T*)c.v + (int64_t)g * v_head_elems(VD);
-    if (p0 < p1) a.load_k(kbase + (int64_t)table[p0] * c.page_stride, kf);
+    if (p0 < p1) a.template load_k<true>(kbase + (int64_t)table[p0] * c.page_stride, kf);
     for (int p = p0; p < p1; ++p) {
-        a.load_v(vbase + (int64_t)table[p] * c.page_stride, vf);
+        a.template load_v<true>(vbase + (int64_t)table[p] * c.page_stride, vf);
         a.weights(kf, s, p * PAGE, lo, live ? pos : -1, scale2, bias2, p * PAGE < lo || p * PAGE + PAGE - 1 > pos);
-        if (p + 1 < p1) a.load_k(kbase + (int64_t)table[p + 1] * c.page_stride, kf);
+        if (p + 1 < p1) a.template load_k<true>(kbase + (int64_t)table[p + 1] * c.page_stride, kf);
         a.mix(vf, s);
     }
     if (!live) return;
