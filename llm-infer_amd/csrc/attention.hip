@@ -149,7 +149,7 @@ struct WaveAttn {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[b][r]);
         }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE)) * scale2;
+        mx = max_halves(mx) * scale2;
         const float m_new = fmaxf(m, mx);
         const float m_safe = (m_new == -INFINITY) ? 0.f : m_new;
         // the hardware's 2^x as it is: results below the smallest normal number become 0, which
@@ -187,7 +187,7 @@ struct WaveAttn {
         }
     }
 
-    __device__ __forceinline__ float total() const { return l + __shfl_xor(l, 32, WAVE); }
+    __device__ __forceinline__ float total() const { return sum_halves(l); }
     // this lane's elements of its row's output
     __device__ __forceinline__ void lay_down(float* to) const {
         const int lane = threadIdx.x & 63;
@@ -288,8 +288,7 @@ struct WaveAttn16 {
                 }
                 mx = fmaxf(mx, s[b][r]);
             }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, WAVE));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE)) * scale2;
+        mx = max_halves(max_quarters(mx)) * scale2;
         const float m_new = fmaxf(m, mx), m_safe = (m_new == -INFINITY) ? 0.f : m_new;
         const float alpha = __builtin_amdgcn_exp2f(m - m_safe);
         float psum = 0.f;
@@ -320,8 +319,7 @@ struct WaveAttn16 {
         }
     }
     __device__ __forceinline__ float total() const {
-        const float half = l + __shfl_xor(l, 16, WAVE);
-        return half + __shfl_xor(half, 32, WAVE);
+        return sum_halves(sum_quarters(l));
     }
     // this lane's elements of its row's output
     __device__ __forceinline__ void lay_down(float* to) const {
@@ -472,7 +470,7 @@ struct PrefillWave {
     // The running maximum takes in a page's largest score mx; alpha is what the sums so far are
     // to be multiplied by before that page is added.
     __device__ __forceinline__ void take_max(float mx, float scale2) {
-        mx = fmaxf(mx, __shfl_xor(mx, 32, WAVE)) * scale2;
+        mx = max_halves(mx) * scale2;
         const float m_new = fmaxf(m, mx);
         m_safe = (m_new == -INFINITY) ? 0.f : m_new;
         alpha = __builtin_amdgcn_exp2f(m - m_safe);
@@ -515,7 +513,7 @@ struct PrefillWave {
         if (MAX) take_max(mx, scale2);
     }
 
-    __device__ __forceinline__ float total() const { return l + __shfl_xor(l, 32, WAVE); }
+    __device__ __forceinline__ float total() const { return sum_halves(l); }
 };
 
 template <class T>

@@ -54,26 +54,82 @@ template <class V> __device__ __forceinline__ V load_once(const void* p) {
     return __builtin_bit_cast(V, __builtin_nontemporal_load((const f32x4*)p));
 }
 
+// Values of other lanes by the vector unit alone: swaps of half waves and of rows of 16 lanes, moves within a row.  (__shfl is a
+// round trip through the LDS unit, some 50 ns each in a chain that nothing runs beside: a wave's sum is six of them.  The same lanes
+// are added in the same order, a + b for b + a, so the bits are the same; but a product that is summed is rounded first, where the
+// compiler made the first addition one multiply-add.  Requests: Dopivik, batch 1, 6.89 -> 6.77 ms, Manirax 14.2 -> 14.05, 8B chat 75.8
+// -> 75.5; batches of 4 and more the same.)  Every lane of the wave must be active.
+template <int CTRL> __device__ __forceinline__ float row_move(float v) {           // a move within every row of 16 lanes
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+#define ROW_ROR(n) (0x120 + (n))
+#define QUAD_SWAP2 0x4E                                // lanes 2, 3, 0, 1 of every four
+#define QUAD_SWAP1 0xB1                                // lanes 1, 0, 3, 2
+struct LanePair { float lo, hi; };
+__device__ __forceinline__ LanePair halves(float v) {  // the values of this lane's place in the lower and the upper half wave
+    auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return LanePair{__uint_as_float(p[0]), __uint_as_float(p[1])};
+}
+__device__ __forceinline__ LanePair quarters(float v) { // and in the first and second 16 lanes of its half
+    auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return LanePair{__uint_as_float(p[0]), __uint_as_float(p[1])};
+}
+__device__ __forceinline__ float sum_halves(float v) { const LanePair p = halves(v); return p.lo + p.hi; }        // v + that of lane ^ 32
+__device__ __forceinline__ float sum_quarters(float v) { const LanePair p = quarters(v); return p.lo + p.hi; }    // v + that of lane ^ 16
+__device__ __forceinline__ float max_halves(float v) { const LanePair p = halves(v); return fmaxf(p.lo, p.hi); }
+__device__ __forceinline__ float max_quarters(float v) { const LanePair p = quarters(v); return fmaxf(p.lo, p.hi); }
+
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, WAVE);
-    return v;
+    v = sum_quarters(sum_halves(v));
+    v += row_move<ROW_ROR(8)>(v);
+    v += row_move<ROW_ROR(4)>(v);                      // (a row repeats every 8 lanes by now: 4 back is 4 on)
+    v += row_move<QUAD_SWAP2>(v);
+    return v + row_move<QUAD_SWAP1>(v);
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, WAVE));
-    return v;
+    v = max_quarters(max_halves(v));
+    v = fmaxf(v, row_move<ROW_ROR(8)>(v));
+    v = fmaxf(v, row_move<ROW_ROR(4)>(v));
+    v = fmaxf(v, row_move<QUAD_SWAP2>(v));
+    return fmaxf(v, row_move<QUAD_SWAP1>(v));
 }
 
-// Sum over a block of up to 1024 threads; `scratch` holds 16 floats of LDS.
+// Sums over the 16 lanes of a row, every lane's the same.
+__device__ __forceinline__ float row_sum(float v) {
+    v += row_move<ROW_ROR(8)>(v);
+    v += row_move<ROW_ROR(4)>(v);
+    v += row_move<QUAD_SWAP2>(v);
+    return v + row_move<QUAD_SWAP1>(v);
+}
+// A wave's choice among pairs (value, index): `take(value, index)` compares another lane's pair with this lane's `v`, `i` and
+// takes it over if it is the better one.  Lane 0 compares its own with those of lanes 32, 16, 8, 4, 2 and 1 on, in this order.
+template <class F> __device__ __forceinline__ void wave_choice(float& v, int& i, F take) {
+    const auto moved = [&](auto move) { take(move(v), __float_as_int(move(__int_as_float(i)))); };
+    const LanePair hv = halves(v), hi = halves(__int_as_float(i));
+    v = hv.lo; i = __float_as_int(hi.lo);
+    take(hv.hi, __float_as_int(hi.hi));
+    const LanePair qv = quarters(v), qi = quarters(__int_as_float(i));
+    v = qv.lo; i = __float_as_int(qi.lo);
+    take(qv.hi, __float_as_int(qi.hi));
+    moved([](float x) { return row_move<ROW_ROR(8)>(x); });
+    moved([](float x) { return row_move<ROW_ROR(12)>(x); });
+    moved([](float x) { return row_move<QUAD_SWAP2>(x); });
+    moved([](float x) { return row_move<QUAD_SWAP1>(x); });
+}
+
+// Sum over a block of up to 1024 threads; `scratch` holds 16 floats of LDS.  (All sixteen are read at once, the waves' added in
+// their order: a loop over as many as there are waits for one after the other.)
 __device__ __forceinline__ float block_sum(float v, float* scratch) {
     v = wave_sum(v);
     const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) scratch[w] = v;
     __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < nw; ++i) t += scratch[i];
+    float s[16], t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) s[i] = scratch[i];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t = i < nw ? t + s[i] : t;
     return t;
 }
 __device__ __forceinline__ float block_max(float v, float* scratch) {

@@ -198,7 +198,7 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
                     tmax = fmaxf(tmax, acc[r]);
                 }
             }
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+            tmax = max_halves(tmax);
             const float mn = fmaxf(m[a], tmax);
             float f = 1.f, sum = 0.f;
             float pr[16];
@@ -210,7 +210,7 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
 #pragma unroll
                 for (int r = 0; r < 16; ++r) { pr[r] = __builtin_amdgcn_exp2f(acc[r] - mn); sum += pr[r]; }
             }
-            sum += __shfl_xor(sum, 32, WAVE);
+            sum = sum_halves(sum);
             l[a] = l[a] * f + sum;
             m[a] = mn;
             if (f != 1.f) {
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256) void diff_attn_mfma_kernel(
             o[0][b][r] = v;
             ss += v * v;
         }
-    ss += __shfl_xor(ss, 32, WAVE);
+    ss = sum_halves(ss);
     float rr = out_eps >= 0.f ? out_scale / sqrtf(ss / (float)dv + out_eps) : out_scale;
     const float* grow = gate ? gate + (int64_t)(t0 + (has_query ? col : 0)) * gate_stride + gate_col : nullptr;
     if (gate && !gate_elem && has_query)             // one number a (token, head)

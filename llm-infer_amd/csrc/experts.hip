@@ -201,13 +201,11 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const T* __re
                 const int i = c * 64 + lane;
                 if (i < n && !(taken >> c & 1) && (zs[c] > best || bi == 0x7fffffff)) { best = zs[c]; bi = i; }
             }
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) {
-                const float ob = __shfl_xor(best, o, WAVE); const int oi = __shfl_xor(bi, o, WAVE);
+            wave_choice(best, bi, [&](float ob, int oi) {
                 if (oi != 0x7fffffff && (bi == 0x7fffffff || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
-            }
+            });
             bi = __builtin_amdgcn_readfirstlane(bi);       // (one choice for the wave, also where logits are no numbers)
-            best = __shfl(best, 0, WAVE);
+            best = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(best)));
             if (k == 0) mx = best;
             sum += expf(best - mx);
             if ((bi & 63) == lane) taken |= 1u << (bi >> 6);

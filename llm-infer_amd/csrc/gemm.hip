@@ -443,8 +443,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                 for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[u][t], b[u][j], acc[t][j]);
     }
     if (MT == 1 && rsc.ss) {
-        ss_mine += __shfl_xor(ss_mine, 16, WAVE);
-        ss_mine += __shfl_xor(ss_mine, 32, WAVE);
+        ss_mine = sum_halves(sum_quarters(ss_mine));
         if (g == 0) ss_wave[wave][r] = ss_mine;
     }
     if (KW > 1) {
@@ -470,7 +469,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     if constexpr (HALF) {
         // rows 4 g + q (g < 2) of column r (r < 8): the sums of even steps here, those of odd steps 40 lanes on
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc[0][0][q] += __shfl_down(acc[0][0][q], 40, WAVE);
+        for (int q = 0; q < 4; ++q) acc[0][0][q] += row_move<ROW_ROR(8)>(halves(acc[0][0][q]).hi);
     }
     const bool mine = !HALF || (r < 8 && g < 2);                      // this lane's sums are results
     if (MT == 1 && rsc.ss) {
@@ -511,8 +510,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                     *(typename Vec<T>::v4*)((T*)ro.xw + (int64_t)m * e.N + n) = xw;
                 }
             }
-            sq[j] += __shfl_xor(sq[j], 16, WAVE);
-            sq[j] += __shfl_xor(sq[j], 32, WAVE);
+            sq[j] = sum_halves(sum_quarters(sq[j]));
             if (g == 0) ro.ss[(int64_t)blockIdx.x * 16 + m] = sq[j];      // (rows beyond M: zeros)
         }
         return;
@@ -720,8 +718,7 @@ __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(const T* __restrict_
                     }
                     *(typename Vec<T>::v4*)((T*)ro.xw + (int64_t)m * e.N + col) = xw;
                 }
-                sq += __shfl_xor(sq, 16, WAVE);
-                sq += __shfl_xor(sq, 32, WAVE);
+                sq = sum_halves(sum_quarters(sq));
                 if (g == 0) ro.ss[(int64_t)blockIdx.x * 16 + r] = sq;          // (rows beyond M: zeros)
             }
         } else if (e.mode == EPI_ROPE && e.rs.cos_sin) {

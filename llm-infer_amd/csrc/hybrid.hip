@@ -759,13 +759,11 @@ __global__ void small_logits_wave_kernel(const T* __restrict__ h, const float* _
         for (int j = 0; j < JB; ++j) {
             // a wave of the other kernel holds the partial sums of 16 of these lanes: its exchanges in its order
 #pragma unroll
-            for (int o = 8; o > 0; o >>= 1)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) acc[k][j][q] += __shfl_xor(acc[k][j][q], o, WAVE);
+            for (int q = 0; q < 4; ++q) acc[k][j][q] = row_sum(acc[k][j][q]);
             const float even = acc[k][j][0] + acc[k][j][2], odd = acc[k][j][1] + acc[k][j][3], part = even + odd;
             float sum = 0.f;
 #pragma unroll
-            for (int v = 0; v < 4; ++v) sum += __shfl(part, 16 * v, WAVE);
+            for (int v = 0; v < 4; ++v) sum += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(part), 16 * v));
             if (lane == 0 && t0 + k < n_rows && j0 + j < n) out[(int64_t)(t0 + k) * n + j0 + j] = bias ? sum + bias[j0 + j] : sum;
         }
 }
@@ -837,10 +835,9 @@ __global__ __launch_bounds__(64) void moe_route_kernel(const float* __restrict__
         float best = -INFINITY; int bi = none;
         for (int i = lane, j = 0; i < n_route; i += 64, ++j)
             if (!(taken >> j & 1) && (c[i] > best || (bi == none && c[i] == c[i]))) { best = c[i]; bi = i; }
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o, WAVE); const int oi = __shfl_xor(bi, o, WAVE);
+        wave_choice(best, bi, [&](float ob, int oi) {
             if (oi != none && (bi == none || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
-        }
+        });
         if (bi == none) break;           // (what is left is no number; the same for every lane)
         chosen_sum += s[bi];
         if ((bi & 63) == lane) taken |= 1ull << (bi >> 6);

@@ -508,8 +508,7 @@ __global__ __launch_bounds__(256) void wkv_chunk_kernel(const float* __restrict_
                 }
             }
         }
-        acc += __shfl_xor(acc, 16, WAVE);
-        acc += __shfl_xor(acc, 32, WAVE);
+        acc = sum_halves(sum_quarters(acc));
         if (cg == 0 && valid) sA[(base + t) * LDM + base + s] = acc;
     }
     if (wave == 3) {                               // tokens 16..31 against 0..15

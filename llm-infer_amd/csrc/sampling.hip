@@ -26,12 +26,9 @@ extern "C" float li_uniform01(uint64_t key, uint64_t counter) { return uniform01
 // first maximum of one chunk of a row, then one workgroup per row picks among the chunks.  Ties go
 // to the lowest index at every stage.
 __device__ __forceinline__ void first_max_reduce(float& best, int& best_i, float* sv, int* si) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        const float ov = __shfl_xor(best, o, WAVE);
-        const int oi = __shfl_xor(best_i, o, WAVE);
+    wave_choice(best, best_i, [&](float ov, int oi) {
         if (ov > best || (ov == best && oi < best_i)) { best = ov; best_i = oi; }
-    }
+    });
     const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     if ((threadIdx.x & 63) == 0) { sv[w] = best; si[w] = best_i; }
     __syncthreads();
