@@ -143,6 +143,35 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
     return t;
 }
 
+// Rows gathered from a table: threads of a workgroup take four elements each; a row of the few tokens of a decode step is
+// shared by as many workgroups as it takes (an element at a time by one workgroup, which waited for memory 16 times a row
+// of 4,096: 4,096 wide, bfloat16, with its launch, 1 row 3.9 -> 1.2 us, 8 rows 6.4 -> 1.7; with positions 9.7 -> 2.0 and 14.0 -> 2.4).
+#define GATHER_THREADS 256
+static inline dim3 gather_grid(int n_tokens, int d) {
+    return dim3(n_tokens, n_tokens < 256 ? (d + 4 * GATHER_THREADS - 1) / (4 * GATHER_THREADS) : 1);
+}
+// f(element, n) for this thread's elements of a row of d: four together, n of them in the row
+template <class F> __device__ __forceinline__ void gather_row(int d, F f) {
+    for (int i = 4 * (blockIdx.y * GATHER_THREADS + threadIdx.x); i < d; i += 4 * GATHER_THREADS * gridDim.y) f(i, min(4, d - i));
+}
+template <class T> struct alignas(4 * sizeof(T)) Quad { T v[4]; };
+// four elements of a row at p (whole: one load), the row's last n where there are no four
+template <class T> __device__ __forceinline__ f32x4 quad_of(const T* p, int n, bool whole) {
+    f32x4 r = {0.f, 0.f, 0.f, 0.f};
+    if (whole) {
+        const Quad<T> q = *(const Quad<T>*)p;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) r[k] = to_f32(q.v[k]);
+    } else {
+        for (int k = 0; k < n; ++k) r[k] = to_f32(p[k]);
+    }
+    return r;
+}
+__device__ __forceinline__ void put_quad(float* p, f32x4 v, int n, bool whole) {
+    if (whole) *(f32x4*)p = v;
+    else for (int k = 0; k < n; ++k) p[k] = v[k];
+}
+
 // A power of two near 1 / (8 rms) for a row whose root mean square is `rms`: what the rows of a residual
 // stream are multiplied by before they are rounded to float16 on their way from one product to the norm
 // inside the next (gemm.hip, RowsOut), so that they lie in the middle of that type's range whatever the

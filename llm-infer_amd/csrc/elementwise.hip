@@ -14,14 +14,15 @@ __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict_
     tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);   // ids are checked on the host; never read outside
     const T* row = table + (int64_t)tok * d;
     float* out = x + (int64_t)t * d;
-    for (int i = threadIdx.x; i < d; i += blockDim.x) out[i] = to_f32(row[i]);
+    const bool whole = (d & 3) == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0;
+    gather_row(d, [&](int i, int n) { put_quad(out + i, quad_of(row + i, n, whole), n, whole); });
 }
 
 extern "C" int li_embed(const void* table, int table_dt, const int* tokens, float* x,
                         int n_tokens, int d, int vocab, hipStream_t stream) {
     if (n_tokens <= 0) return LI_OK;
     if (d <= 0 || vocab <= 0) return LI_BAD_ARG;
-    dim3 grid(n_tokens), block(256);
+    dim3 grid = gather_grid(n_tokens, d), block(GATHER_THREADS);
     if (table_dt == DT_F32) embed_kernel<float><<<grid, block, 0, stream>>>((const float*)table, tokens, x, d, vocab);
     else if (table_dt == DT_F16) embed_kernel<f16><<<grid, block, 0, stream>>>((const f16*)table, tokens, x, d, vocab);
     else if (table_dt == DT_BF16) embed_kernel<bf16><<<grid, block, 0, stream>>>((const bf16*)table, tokens, x, d, vocab);

@@ -35,21 +35,26 @@ __global__ void embed_pos_kernel(const T* __restrict__ table, const int* __restr
     const int t = blockIdx.x;
     const T* row = table + (int64_t)tokens[t] * d;
     const float p = pos ? (float)pos[t] : 0.f;
-    for (int i = threadIdx.x; i < d; i += blockDim.x) {
-        float v = to_f32(row[i]) * scale;
-        if (freq) {
-            const float a = p * freq[i >> 1];
-            v += (i & 1) ? cosf(a) : sinf(a);
+    const bool whole = (d & 3) == 0 && (((uintptr_t)table | (uintptr_t)out) & 15) == 0;
+    gather_row(d, [&](int i, int n) {
+        f32x4 v = quad_of(row + i, n, whole);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] *= scale;
+            if (freq && k < n) {
+                const float a = p * freq[(i + k) >> 1];
+                v[k] += (k & 1) ? cosf(a) : sinf(a);
+            }
         }
-        out[(int64_t)t * d + i] = v;
-    }
+        put_quad(out + (int64_t)t * d + i, v, n, whole);
+    });
 }
 
 extern "C" int li_embed_pos(const void* table, int dt, const int* tokens, const int* pos, const float* freq, float* out,
                             int n, int d, float scale, hipStream_t stream) {
     if (n <= 0) return LI_OK;
     if (d <= 0) return LI_BAD_ARG;
-    DISPATCH_T(dt, (embed_pos_kernel<T><<<n, 256, 0, stream>>>((const T*)table, tokens, pos, freq, out, d, scale)));
+    DISPATCH_T(dt, (embed_pos_kernel<T><<<gather_grid(n, d), GATHER_THREADS, 0, stream>>>((const T*)table, tokens, pos, freq, out, d, scale)));
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

@@ -42,7 +42,14 @@ __global__ void embed_bigram_kernel(const T* __restrict__ table, const T* __rest
     }
     const T* e = table + (int64_t)tok * d;
     const T* b = bigram + row * d;
-    for (int i = threadIdx.x; i < d; i += blockDim.x) out[(int64_t)t * d + i] = to_f32(e[i]) * scale + to_f32(b[i]);
+    const bool whole = (d & 3) == 0 && (((uintptr_t)table | (uintptr_t)bigram | (uintptr_t)out) & 15) == 0;
+    gather_row(d, [&](int i, int n) {
+        f32x4 v = quad_of(e + i, n, whole);
+        const f32x4 bv = quad_of(b + i, n, whole);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = v[k] * scale + bv[k];
+        put_quad(out + (int64_t)t * d + i, v, n, whole);
+    });
 }
 
 __global__ void last_token_kernel(const int* __restrict__ tokens, const int* __restrict__ seq_slot,
@@ -60,7 +67,7 @@ extern "C" int li_embed_bigram(const void* table, const void* bigram, int dt, co
                                int64_t mul_cur, int buckets, hipStream_t stream) {
     if (n <= 0) return LI_OK;
     if (d <= 0 || buckets <= 0 || n_seqs <= 0) return LI_BAD_ARG;
-    DISPATCH_T(dt, (embed_bigram_kernel<T><<<n, 256, 0, stream>>>((const T*)table, (const T*)bigram, tokens, pos, tok_slot,
+    DISPATCH_T(dt, (embed_bigram_kernel<T><<<gather_grid(n, d), GATHER_THREADS, 0, stream>>>((const T*)table, (const T*)bigram, tokens, pos, tok_slot,
                                                                   prev_state, out, d, scale, mul_prev, mul_cur, buckets)));
     last_token_kernel<<<(n_seqs + 255) / 256, 256, 0, stream>>>(tokens, seq_slot, seq_qstart, seq_qlen, prev_state, n_seqs);
     LI_CHECK_LAUNCH();

@@ -37,6 +37,8 @@ __device__ __forceinline__ void first_max_reduce(float& best, int& best_i, float
             if (sv[i] > best || (sv[i] == best && si[i] < best_i)) { best = sv[i]; best_i = si[i]; }
 }
 
+#define ARGMAX_CHUNK 4096               // logits of a chunk at the most
+
 __global__ __launch_bounds__(256) void argmax_chunks_kernel(const float* __restrict__ logits, int V, int chunk,
                                                             float* __restrict__ part_v, int* __restrict__ part_i) {
     __shared__ float sv[4];
@@ -45,9 +47,13 @@ __global__ __launch_bounds__(256) void argmax_chunks_kernel(const float* __restr
     const int lo = blockIdx.y * chunk, hi = min(V, lo + chunk);
     float best = -INFINITY;
     int best_i = 0x7fffffff;
-    for (int i = lo + threadIdx.x; i < hi; i += blockDim.x) {
-        const float v = row[i];
-        if (v > best || best_i == 0x7fffffff) { best = v; best_i = i; }      // ascending i: strict > keeps the first
+    float v[ARGMAX_CHUNK / 256];                         // all on their way at once (one after the other: 8 rows of 128,256 with both launches 9.7 -> 4.8 us, 1 row of 32,000 7.4 -> 5.1)
+#pragma unroll
+    for (int k = 0; k < ARGMAX_CHUNK / 256; ++k) v[k] = row[min(lo + (int)threadIdx.x + 256 * k, hi - 1)];
+#pragma unroll
+    for (int k = 0; k < ARGMAX_CHUNK / 256; ++k) {
+        const int i = lo + threadIdx.x + 256 * k;
+        if (i < hi && (v[k] > best || best_i == 0x7fffffff)) { best = v[k]; best_i = i; }      // ascending i: strict > keeps the first
     }
     first_max_reduce(best, best_i, sv, si);
     if (threadIdx.x == 0) {
@@ -213,7 +219,7 @@ __global__ __launch_bounds__(64) void token_prob_kernel(const float* __restrict_
 }
 
 // part_v, part_i: workspace of n_rows * li_argmax_chunks(V) entries each
-extern "C" int li_argmax_chunks(int V) { return V <= 4096 ? 1 : (V + 4095) / 4096; }
+extern "C" int li_argmax_chunks(int V) { return V <= ARGMAX_CHUNK ? 1 : (V + ARGMAX_CHUNK - 1) / ARGMAX_CHUNK; }
 
 extern "C" int li_argmax(const float* logits, int n_rows, int V, float* part_v, int* part_i, int* out,
                          hipStream_t stream) {
