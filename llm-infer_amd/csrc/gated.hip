@@ -283,9 +283,73 @@ extern "C" int li_rot_store(const float* rows, int stride, int q_col, int k_col,
 #define RA_THREADS 256
 #define RA_KEEP 8          // 4 elements x RA_KEEP x RA_THREADS = 8,192 elements kept
 
-// EARLY (the few rows of a decode step): everything the row needs is asked for at once (y, the bias, x and the weight), so
-// that a row waits for memory once and not once a phase; many rows fill the chip anyway and do better with fewer registers.
-template <class TN, bool EARLY>
+// The few rows of a decode step: everything the row needs is asked for at once, with addresses that need no branch (what lies
+// beyond the row is its last quad again and counts nowhere), so that a row waits for memory once.  Bound by the latency of its
+// one workgroup.  With its launch, behind a product: 1 row of 2,048 4.15 -> 2.7 us, of 4,096
+// 5.0 -> 3.0, 8 rows of 4,096 5.4 -> 3.6 (loads that were branched around waited for each other).
+template <class TN, int NC>
+__global__ __launch_bounds__(RA_THREADS) void rmsnorm_add_few_kernel(float* __restrict__ x, const float* __restrict__ y,
+                                                                     const float* __restrict__ b, const float* __restrict__ w,
+                                                                     float eps, int width, const float* __restrict__ add_rows,
+                                                                     const float* __restrict__ add_vec, const float* __restrict__ next_w,
+                                                                     float next_eps, TN* __restrict__ next) {
+    struct alignas(4 * sizeof(TN)) Out4 { TN v[4]; };
+    __shared__ float scratch[16];
+    const int64_t row = (int64_t)blockIdx.x * width;
+    const int quads = width >> 2;
+    int at[NC];
+    bool in[NC];
+    f32x4 ys[NC], xs[NC], ws[NC], bs[NC], nw[NC], av[NC], ar[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        in[c] = (int)threadIdx.x + c * RA_THREADS < quads;
+        at[c] = 4 * min((int)threadIdx.x + c * RA_THREADS, quads - 1);
+        ys[c] = *(const f32x4*)(y + row + at[c]);
+        xs[c] = *(const f32x4*)(x + row + at[c]);
+        ws[c] = *(const f32x4*)(w + at[c]);
+    }
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        bs[c] = b ? *(const f32x4*)(b + at[c]) : zero;
+        nw[c] = next_w ? *(const f32x4*)(next_w + at[c]) : zero;
+        av[c] = add_vec ? *(const f32x4*)(add_vec + at[c]) : zero;
+        ar[c] = add_rows ? *(const f32x4*)(add_rows + row + at[c]) : zero;
+    }
+    float ss = 0.f, s2 = 0.f;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        f32x4& v = ys[c];
+        if (b) { v[0] += bs[c][0]; v[1] += bs[c][1]; v[2] += bs[c][2]; v[3] += bs[c][3]; }
+        if (in[c]) ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
+    }
+    const float r = 1.f / sqrtf(block_sum(ss, scratch) / (float)width + eps);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        f32x4& o = xs[c];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            o[q] += ys[c][q] * r * ws[c][q];
+            if (add_vec) o[q] += add_rows ? av[c][q] + ar[c][q] : av[c][q];
+        }
+        if (in[c]) {
+            *(f32x4*)(x + row + at[c]) = o;
+            s2 += o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
+        }
+    }
+    if (!next_w) return;
+    const float r2 = 1.f / sqrtf(block_sum(s2, scratch) / (float)width + next_eps);
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        if (!in[c]) continue;
+        Out4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v.v[q] = from_f32<TN>(xs[c][q] * r2 * nw[c][q]);
+        *(Out4*)(next + row + at[c]) = v;
+    }
+}
+
+template <class TN>
 __global__ __launch_bounds__(RA_THREADS) void rmsnorm_add_kernel(float* __restrict__ x, const float* __restrict__ y,
                                                                  const float* __restrict__ b, const float* __restrict__ w,
                                                                  float eps, int width, const float* __restrict__ add_rows,
@@ -298,25 +362,13 @@ __global__ __launch_bounds__(RA_THREADS) void rmsnorm_add_kernel(float* __restri
     TN* nr = next + row * width;
     float ss = 0.f, s2 = 0.f;
     if ((width & 3) == 0 && width <= 4 * RA_KEEP * RA_THREADS) {
-        f32x4 keep[RA_KEEP], xs[RA_KEEP], ws[RA_KEEP], nw[RA_KEEP], ad[RA_KEEP];
+        f32x4 keep[RA_KEEP], xs[RA_KEEP], ws[RA_KEEP];
         const int quads = width >> 2;
 #pragma unroll
         for (int c = 0; c < RA_KEEP; ++c) {
             const int i = threadIdx.x + c * RA_THREADS;
             if (i < quads) {
                 f32x4 v = *(const f32x4*)(yr + 4 * i);
-                if (EARLY) {
-                    xs[c] = *(const f32x4*)(xr + 4 * i);
-                    ws[c] = *(const f32x4*)(w + 4 * i);
-                    if (next_w) nw[c] = *(const f32x4*)(next_w + 4 * i);
-                    if (add_vec) {
-                        ad[c] = *(const f32x4*)(add_vec + 4 * i);
-                        if (add_rows) {
-                            const f32x4 e = *(const f32x4*)(add_rows + row * width + 4 * i);
-                            ad[c][0] += e[0]; ad[c][1] += e[1]; ad[c][2] += e[2]; ad[c][3] += e[3];
-                        }
-                    }
-                }
                 if (b) { const f32x4 bb = *(const f32x4*)(b + 4 * i); v[0] += bb[0]; v[1] += bb[1]; v[2] += bb[2]; v[3] += bb[3]; }
                 keep[c] = v;
                 ss += v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3];
@@ -327,29 +379,23 @@ __global__ __launch_bounds__(RA_THREADS) void rmsnorm_add_kernel(float* __restri
         for (int c = 0; c < RA_KEEP; ++c) {
             const int i = threadIdx.x + c * RA_THREADS;
             if (i < quads) {
-                if (!EARLY) {
-                    xs[c] = *(const f32x4*)(xr + 4 * i);
-                    ws[c] = *(const f32x4*)(w + 4 * i);
-                }
+                xs[c] = *(const f32x4*)(xr + 4 * i);
+                ws[c] = *(const f32x4*)(w + 4 * i);
                 f32x4 o = xs[c];
                 o[0] += keep[c][0] * r * ws[c][0]; o[1] += keep[c][1] * r * ws[c][1];
                 o[2] += keep[c][2] * r * ws[c][2]; o[3] += keep[c][3] * r * ws[c][3];
                 if (add_vec) {
-                    f32x4 e;
-                    if (EARLY) e = ad[c];
-                    else {
-                        e = *(const f32x4*)(add_vec + 4 * i);
-                        if (add_rows) {
-                            const f32x4 e2 = *(const f32x4*)(add_rows + row * width + 4 * i);
-                            e[0] += e2[0]; e[1] += e2[1]; e[2] += e2[2]; e[3] += e2[3];
-                        }
+                    f32x4 e = *(const f32x4*)(add_vec + 4 * i);
+                    if (add_rows) {
+                        const f32x4 e2 = *(const f32x4*)(add_rows + row * width + 4 * i);
+                        e[0] += e2[0]; e[1] += e2[1]; e[2] += e2[2]; e[3] += e2[3];
                     }
                     o[0] += e[0]; o[1] += e[1]; o[2] += e[2]; o[3] += e[3];
                 }
                 *(f32x4*)(xr + 4 * i) = o;
                 keep[c] = o;
                 s2 += o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
-                if (next_w) ws[c] = EARLY ? nw[c] : *(const f32x4*)(next_w + 4 * i);
+                if (next_w) ws[c] = *(const f32x4*)(next_w + 4 * i);
             }
         }
         if (!next_w) return;
@@ -386,12 +432,18 @@ extern "C" int li_rmsnorm_add(float* x, const float* y, const float* b, const fl
     if (n_rows <= 0) return LI_OK;
     if (width <= 0 || !x || !y || !w || (next_w && !next) || (add_rows && !add_vec)) return LI_BAD_ARG;
     if (!next_w) next_dt = DT_F32;
-    if (n_rows <= 64)
-        DISPATCH_T(next_dt, (rmsnorm_add_kernel<T, true><<<n_rows, RA_THREADS, 0, stream>>>(x, y, b, w, eps, width, add_rows, add_vec, next_w,
-                                                                                       next_eps, (T*)next)));
-    else
-        DISPATCH_T(next_dt, (rmsnorm_add_kernel<T, false><<<n_rows, RA_THREADS, 0, stream>>>(x, y, b, w, eps, width, add_rows, add_vec, next_w,
-                                                                                       next_eps, (T*)next)));
+    // (many rows fill the chip anyway and do better with fewer registers; the same values either way)
+    const int quads = width >> 2;
+    if (n_rows <= 64 && (width & 3) == 0 && quads <= RA_KEEP * RA_THREADS) {
+#define GO(NC) rmsnorm_add_few_kernel<T, NC><<<n_rows, RA_THREADS, 0, stream>>>(x, y, b, w, eps, width, add_rows, add_vec, next_w, next_eps, (T*)next)
+        DISPATCH_T(next_dt, {
+            if (quads <= RA_THREADS) GO(1); else if (quads <= 2 * RA_THREADS) GO(2);
+            else if (quads <= 4 * RA_THREADS) GO(4); else GO(RA_KEEP);
+        });
+#undef GO
+    } else
+        DISPATCH_T(next_dt, (rmsnorm_add_kernel<T><<<n_rows, RA_THREADS, 0, stream>>>(x, y, b, w, eps, width, add_rows, add_vec, next_w,
+                                                                                     next_eps, (T*)next)));
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

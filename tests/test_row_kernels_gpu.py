@@ -44,3 +44,95 @@ def test_argmax_first_of_the_largest(ops, v):
     x[3, -1] = 70.0
     x[4, 0] = 70.0
     assert ops.argmax(x).tolist() == [int((r == r.max()).nonzero()[0]) for r in x.cpu()]
+
+
+def _rms(v, eps):
+    return (v.pow(2).mean(1, keepdim=True) + eps).sqrt()
+
+
+def _ln(v, eps):
+    d = v - v.mean(1, keepdim=True)
+    return d / (d.pow(2).mean(1, keepdim=True) + eps).sqrt()
+
+
+def _close(got, want):
+    """Within what float32 sums and some ten roundings of a row leave: 2e-6 of its size, and half a unit of a 16-bit type."""
+    unit = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[got.dtype]
+    err = (got.double() - want).abs()
+    assert (err <= 2e-6 * want.abs().amax(1, keepdim=True) + (unit * 1.01) * want.abs()).all(), err.max()
+
+
+# rows that leave waves without elements, quads a thread of 1, 2, 4 and 8, the last that is kept and the first that is not
+WIDTHS = [4, 60, 256, 260, 1024, 1028, 2048, 2052, 4096, 4100, 8188, 8192, 8196]
+
+
+@pytest.mark.parametrize("width", WIDTHS + [37])
+def test_normed_sum_of_few_rows_and_many(ops, width):
+    x, y, z = (torch.randn(65, width, device=DEV) for _ in range(3))
+    w, b, nw, v = (torch.rand(width, device=DEV) + 0.5 for _ in range(4))
+    for bias in (None, b):
+        for also in (None, (None, v), (z, v)):
+            want = x.double() + (lambda t: t / _rms(t, 1e-5) * w.double())(y.double() + (bias.double() if bias is not None else 0))
+            if also:
+                want = want + v.double() + (z.double() if also[0] is not None else 0)
+            made = {}
+            for rows in (1, 64, 65):
+                out = x[:rows].clone()
+                extra = also and (also[0] if also[0] is None else z[:rows].contiguous(), v)
+                ops.rmsnorm_add(out, y[:rows].contiguous(), w, 1e-5, bias, (nw, 1e-6, torch.float16), extra)
+                made[rows] = (out, ops.prepared_rmsnorm(out, nw, 1e-6, torch.float16))
+                _close(out, want[:rows])
+                _close(made[rows][1], (want / _rms(want, 1e-6) * nw.double())[:rows])
+            for rows in (1, 64):                              # the two kernels give the same values
+                assert all(torch.equal(a, c[:rows]) for a, c in zip(made[rows], made[65]))
+
+
+@pytest.mark.parametrize("mean", [0.0, 3.0])
+@pytest.mark.parametrize("width", WIDTHS + [37])
+def test_layer_norms_of_sums(ops, width, mean):
+    x, y, y2 = (torch.randn(9, width, device=DEV) + mean for _ in range(3))
+    w, b, nw, nb = (torch.rand(width, device=DEV) + 0.5 for _ in range(4))
+    xd, yd, y2d = x.double(), y.double(), y2.double()
+    out = x.clone()
+    ops.layernorm_add(out, y, w, b, 1e-5, (nw, nb, 1e-5, torch.bfloat16))
+    want = xd + _ln(yd, 1e-5) * w.double() + b.double()
+    _close(out, want)
+    _close(ops.prepared_norm(out, nw, 1e-5, torch.bfloat16), _ln(want, 1e-5) * nw.double() + nb.double())
+    pair = ops.NormedPair(y, w, y2, b, 1e-5, 0.5)
+    out = x.clone()
+    ops.layernorm_add(out, pair, nw, nb, 1e-5)
+    both = 0.5 * (yd / _rms(yd, 1e-5) * w.double() + y2d / _rms(y2d, 1e-5) * b.double())
+    _close(out, xd + _ln(both, 1e-5) * nw.double() + nb.double())
+    for adds in ([(y, 0.5)], [(y, 0.5), (y2, 2.0)]):
+        out = x.clone()
+        copy = ops.add_layernorm(out, 2.0, adds, w, 1e-5, torch.bfloat16)
+        want = _ln(2 * xd + sum(s * t.double() for t, s in adds), 1e-5) * w.double()
+        _close(out, want)
+        assert torch.equal(copy, out.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("n", WIDTHS + [37, 14336, 16384, 16388])
+def test_gated_norm_and_polynorm_of_a_row(ops, n):
+    o, w = torch.randn(3, n, device=DEV), torch.rand(n, device=DEV) + 0.5
+    want = o.double() / _rms(o.double(), 1e-5) * w.double()
+    for stride, col in ((n, 0), (n + 8, 4), (n + 3, 3)):           # gates that are 16-byte aligned and not
+        gate = torch.randn(3, stride, device=DEV)
+        _close(ops.gated_rmsnorm(o, w, gate, col, 1e-5, torch.float16), want * torch.sigmoid(gate[:, col:col + n].double()))
+    coef = torch.tensor([0.5, -0.3, 0.2, 0.1], device=DEV)
+    d = o.double()
+    _close(ops.polynorm(o, coef, 1e-5, torch.bfloat16), sum(c * d ** k / _rms(d ** k, 1e-5) for k, c in ((1, 0.5), (2, -0.3), (3, 0.2))) + 0.1)
+
+
+@pytest.mark.parametrize("terms", [1, 3, 4, 5, 9])
+@pytest.mark.parametrize("width", WIDTHS[:-1])
+def test_average_over_depth_with_its_norms(ops, width, terms):
+    hist, weights = torch.randn(terms + 1, 3, width, device=DEV), torch.rand(terms, device=DEV)
+    weights[0] = 0.0                                               # (a term of weight 0 that is not finite shows all the same)
+    nw = torch.rand(width, device=DEV) + 0.5
+    norms = [(nw, 1e-5, torch.float16), (nw, 1e-6, torch.float32)]
+    out = torch.empty(3, width, device=DEV)
+    ops.average_norms(hist, terms, weights, out, norms)
+    plain = ops.depth_average(hist, terms, weights, torch.empty_like(out))
+    assert torch.equal(out, plain)
+    for w, eps, dt in norms:
+        assert torch.equal(ops.prepared_norm(out, w, eps, dt), ops.rmsnorm(plain, w, eps, dt))
