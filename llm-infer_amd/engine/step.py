@@ -5,7 +5,8 @@ from __future__ import annotations
 import math
 
 import numpy as np
-import torch
+
+from ..kernels import ops
 
 PAGE = 64
 
@@ -65,7 +66,7 @@ class StepContext(StepShared):
         packed = np.zeros(int(offs[-1]) + 4, dtype=np.int32)
         for (_, v), o, s in zip(fields, offs, sizes):
             packed[int(o):int(o) + s] = np.asarray(v, dtype=np.int32)
-        dev = torch.from_numpy(packed).to(device)
+        dev = ops.upload(packed, device)
         for (name, _), o, s in zip(fields, offs, sizes):
             setattr(self, name, dev[int(o):int(o) + s])
         self._packed = dev

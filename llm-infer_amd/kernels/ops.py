@@ -31,13 +31,14 @@ def _ptr(t):
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", torch.cuda.current_device)      # (the operands lie on the GPU: it has been initialised)
 
 
 def _stream():
     """The current HIP stream of the current device (looked up for every launch: a graph is
     recorded on a stream of its own)."""
     if _raw_stream is not None:
-        return c_void_p(_raw_stream(torch.cuda.current_device()))
+        return c_void_p(_raw_stream(_raw_device()))
     return c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
@@ -53,9 +54,20 @@ def _need(cond: bool, msg: str):
 
 def _dev(*tensors):
     for t in tensors:
-        if t is not None:
-            _need(t.is_cuda, "kernel operands must lie on the GPU")
-            _need(t.is_contiguous(), "kernel operands must be contiguous")
+        if t is not None and not (t.is_cuda and t.is_contiguous()):
+            raise KernelError("kernel operands must lie on the GPU" if not t.is_cuda else "kernel operands must be contiguous")
+
+
+def upload(values, device) -> torch.Tensor:
+    """int32 ``values`` (numbers, or rows of them) on ``device``, for the index arrays of a step.  They go through page-locked memory,
+    which torch keeps until the copy is done, so the copy stands in line with the step's kernels and the host goes on; out of
+    ordinary memory it waits for everything that is queued, and the device then for the host's next launches."""
+    values = np.asarray(values, dtype=np.int32)
+    if torch.device(device).type != "cuda":
+        return torch.from_numpy(values).to(device)
+    staged = torch.empty(values.shape, dtype=torch.int32, pin_memory=True)
+    staged.numpy()[...] = values
+    return staged.to(device, non_blocking=True)
 
 
 _core = None
@@ -308,7 +320,8 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
         else:
             x = x.tensor()
     _dev(x, wd, out)
-    _need(x.dim() == 2 and len(w_shape) == 2 and x.shape[1] == w_shape[1], f"linear: x {tuple(x.shape)} w {w_shape}")
+    if not (x.dim() == 2 and len(w_shape) == 2 and x.shape[1] == w_shape[1]):
+        raise KernelError(f"linear: x {tuple(x.shape)} w {w_shape}")
     m, k = x.shape
     n = w_shape[0]
     n_out = n // 2 if mode in GATED else n
@@ -323,8 +336,8 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
         _need(_rope is not None, "the rotation epilogue needs its arguments (use linear_rope_store)")
     elif out is None:
         out = torch.empty((m, n_out), dtype=out_dtype or x.dtype, device=x.device)
-    if mode != EPI_ROPE:
-        _need(out.shape == (m, n_out), f"linear: out {tuple(out.shape)}, expected {(m, n_out)}")
+    if mode != EPI_ROPE and out.shape != (m, n_out):
+        raise KernelError(f"linear: out {tuple(out.shape)}, expected {(m, n_out)}")
     out_dt = DT[out.dtype] if out is not None else 0
     if mode in GATED:
         _need(n % 2 == 0, "a gated epilogue needs an even number of rows of W")
@@ -788,7 +801,7 @@ def prefill_meta(ctx) -> dict:
     sequence's tokens)."""
     def tiles():
         tile_seq, tile_q0 = prefill_tiles(ctx.host_qlens)
-        both = torch.tensor([tile_seq, tile_q0], dtype=torch.int32).to(ctx.device)
+        both = upload([tile_seq, tile_q0], ctx.device)
         return {"tile_seq": both[0], "tile_q0": both[1], "n_tiles": len(tile_seq)}
     return dict(ctx.shared(PREFILL_TILES_KEY, tiles), seq_slot=ctx.seq_slot,
                 seq_qstart=ctx.seq_qstart, seq_qlen=ctx.seq_qlen, seq_ctx=ctx.seq_ctx)
@@ -1257,7 +1270,7 @@ def decay_chunks(ctx) -> dict:
     """The chunk lists of a step on the device, made and uploaded once per step by the first layer that asks."""
     def make():
         chunk_seq, chunk_t0, seq_chunk0 = decay_chunk_lists(ctx.host_qlens)
-        flat = torch.tensor(chunk_seq + chunk_t0 + seq_chunk0, dtype=torch.int32).to(ctx.device)
+        flat = upload(chunk_seq + chunk_t0 + seq_chunk0, ctx.device)
         n = len(chunk_seq)
         return {"chunk_seq": flat[:n], "chunk_t0": flat[n:2 * n], "seq_chunk0": flat[2 * n:], "n_chunks": n}
     return ctx.shared(("decay_attention_chunks", DECAY_CHUNK), make)
@@ -1472,7 +1485,7 @@ def diff_tiles(ctx, block=None, window=None, keep_first: int = 0):
 
     def make():
         t0, n = diff_tile_pairs(ctx.host_qlens, ctx.host_lens_before, int(block or 0), int(window or 0), int(keep_first))
-        both = torch.tensor([t0, n], dtype=torch.int32).to(ctx.device)
+        both = upload([t0, n], ctx.device)
         return both[0], both[1], len(t0) // 2
     return ctx.shared(("diff_attention_tiles", DIFF_TILE, int(block or 0), int(window or 0), int(keep_first)), make)
 
@@ -1598,7 +1611,7 @@ def ssm_segments(ctx, length: int | None = None) -> dict:
                 seg_n.append(min(length, n - t0))
             seq_nseg.append(len(seg_seq) - seq_seg0[-1])
         k, b = len(seg_seq), len(seq_seg0)
-        flat = torch.tensor(seg_seq + seg_t0 + seg_n + seq_seg0 + seq_nseg, dtype=torch.int32).to(ctx.device)
+        flat = upload(seg_seq + seg_t0 + seg_n + seq_seg0 + seq_nseg, ctx.device)
         return {"seg_seq": flat[:k], "seg_t0": flat[k:2 * k], "seg_n": flat[2 * k:3 * k], "seq_seg0": flat[3 * k:3 * k + b],
                 "seq_nseg": flat[3 * k + b:], "n": k}
     return ctx.shared(("ssm_segments", length), make)
