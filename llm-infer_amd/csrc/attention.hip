@@ -20,7 +20,6 @@
 // float32 kernel: one workgroup per (token, head), keys in ascending order, so a
 // result does not depend on how the step was cut or batched.
 #include "common.h"
-#include <type_traits>
 
 #ifndef HEAD_DIM
 #error "compile with -DHEAD_DIM=<head size>"
@@ -871,12 +870,8 @@ __global__ void attn_merge_kernel(const float* __restrict__ part_o, const float*
 // scores, then a dimension of a head's output: every sum runs in ascending order of dimensions or keys, so a result does not
 // depend on the batch or on hg.  Bound by those chains (one multiply-add a key) and, for many tokens, by the loads of keys and
 // values; both come four numbers at a time, values for four tokens of a dimension.  32 / 8 heads of 64, contexts of
-// up to 200: 400 tokens 38 us (188 with a load a number and a workgroup a head), 3 tokens 9.7 (30), 2 tokens at
-// 1,000 31 (140).
+// up to 200: 400 tokens 38 us (188 with a load a number and a workgroup a head).
 // ---------------------------------------------------------------------------
-// PAGES: a whole page's values on their way together instead of sixteen tokens', for the few tokens of a decode step (more
-// registers: 200 tokens at 200 keys 45 and 51 us): 3 tokens at 200 8.6 -> 7.4, 2 at 1,000 47 -> 33, of 128 3 at 200 16.8 -> 13.9.
-template <bool PAGES>
 __global__ __launch_bounds__(256) void attn_f32_kernel(
     const float* __restrict__ q, float* __restrict__ out, CachePtrs c, const int* __restrict__ pos_of,
     const int* __restrict__ tok_slot, int H, int K, int hg, float scale, int window) {
@@ -948,22 +943,6 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
             float psum = 0.f, acc = o * alpha;
             for (int b = t16; b < t0 + n; b += 16) {
                 const float* vp = vbase + (int64_t)table[b / PAGE] * c.page_stride;
-                if (PAGES && b % PAGE == 0 && b >= t0 && b + PAGE <= t0 + n) {
-                    f32x4 vv[PAGE / 4];
-#pragma unroll
-                    for (int u = 0; u < PAGE / 4; ++u) vv[u] = *(const f32x4*)(vp + v_offset(4 * u, d, HD));
-#pragma unroll
-                    for (int u = 0; u < PAGE / 4; ++u) {
-                        const f32x4 ww = sp4[j][(b - t16) / 4 + u];
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            psum += ww[i];
-                            acc = fmaf(ww[i], vv[u][i], acc);
-                        }
-                    }
-                    b += PAGE - 16;
-                    continue;
-                }
                 if (b >= t0 && b + 16 <= t0 + n) {
                     f32x4 vv[4], ww[4];
 #pragma unroll
@@ -988,6 +967,121 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(
         }
     }
     if (owns) out[(tok * H + h0 + j) * HD + d] = o / l;
+}
+
+// The same sums, bit for bit, for the few tokens of a decode step: a workgroup a head, whose time is the way of its loads, one
+// behind the other.  The page table's entries come in one load, the first page of values is on its way before the scores are
+// worked on, the next one while a page is added up, and a page that the context or the window cuts is fetched as a whole too (its
+// keys outside are passed over).  More registers, fewer waves: not for many tokens (the rule is beside the launch).  us in a
+// recorded chain, before (a page's values fetched when its weights were there, the last keys one by one) and now, 32 / 8 heads of
+// 64: 3 tokens at 200 10.5 -> 6.6, 1 at 60 9.5 -> 5.4, 2 at 1,000 32.6 -> 18.2, 2 at 4,000 115 -> 61, 32 at 200 12.2 -> 11.0; of 128: 3 at
+// 200 13.3 -> 8.1, 2 at 1,000 44.6 -> 23.9.  Bound now by the chain of a head's sums and three meetings every 256 keys.
+__global__ __launch_bounds__(256) void attn_f32_few_kernel(
+    const float* __restrict__ q, float* __restrict__ out, CachePtrs c, const int* __restrict__ pos_of,
+    const int* __restrict__ tok_slot, int H, int K, float scale, int window) {
+    __shared__ f32x4 sq[HD / 4];
+    __shared__ f32x4 sp4[256 / 4 + PAGE / 4];         // weights, from the first page's start on
+    __shared__ float smax[4];
+    constexpr int KB = HD < 64 ? HD / 4 : 16;         // loads of a key's dimensions on their way together
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int64_t tok = blockIdx.x;
+    const int h = blockIdx.y, kvh = h / (H / K);
+    const int pos = pos_of[tok];
+    const int lo = window > 0 ? max(0, pos - window + 1) : 0;
+    const int* table = c.page_table + (int64_t)tok_slot[tok] * c.max_pages;
+    const float* kbase = (const float*)c.k + (int64_t)kvh * k_head_elems(HD);
+    const float* vbase = (const float*)c.v + (int64_t)kvh * v_head_elems(HD);
+    if (tid < HD / 4) sq[tid] = ((const f32x4*)(q + (tok * H + h) * HD))[tid];
+    __syncthreads();
+    const bool adds = wave * 64 < HD;                 // a wave with dimensions of the output
+    const int d = min(tid, HD - 1);
+    float m = -INFINITY, l = 0.f, o = 0.f;
+    for (int t0 = lo; t0 <= pos; t0 += 256) {
+        const int t = t0 + tid, end = min(t0 + 256, pos + 1), b0 = t0 / PAGE * PAGE;
+        const int tk = min(t, pos);
+        // the entries of the (at most 5) pages from b0 on, one a lane; a wave's 64 keys lie in two of them at most
+        const int entry = table[min(b0 / PAGE + (tid & 7), pos / PAGE)];
+        const int pk = (t0 + 64 * wave) / PAGE - b0 / PAGE;
+        const int e0 = __builtin_amdgcn_readlane(entry, pk), e1 = __builtin_amdgcn_readlane(entry, pk + 1);
+        const float* kp = kbase + (int64_t)(t / PAGE - b0 / PAGE == pk ? e0 : e1) * c.page_stride;
+        f32x4 kk[KB], vv[PAGE / 4];
+        float dot = 0.f;
+        auto keys = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < KB; ++i)
+                if (i0 + i < HD / 4) kk[i] = ((const f32x4*)(kp + k_offset(tk % PAGE, 4 * (i0 + i) & ~7, HD)))[i & 1];
+        };
+        auto dots = [&](int i0) {
+#pragma unroll
+            for (int i = 0; i < KB; ++i)
+                if (i0 + i < HD / 4) {
+                    const f32x4 qq = sq[i0 + i];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) dot = fmaf(qq[e], kk[i][e], dot);
+                }
+        };
+        auto values = [&](int page) {
+            const float* vp = vbase + (int64_t)__builtin_amdgcn_readlane(entry, page) * c.page_stride;
+#pragma unroll
+            for (int u = 0; u < PAGE / 4; ++u) vv[u] = *(const f32x4*)(vp + v_offset(4 * u, d, HD));
+        };
+        keys(0);
+        if (adds) {
+            values(0);
+            dots(0);
+            asm volatile("; %0" : "+v"(dot));         // (keeps this form apart from the other, which has no values behind it)
+        } else {
+            dots(0);
+        }
+#pragma unroll
+        for (int i0 = KB; i0 < HD / 4; i0 += KB) { keys(i0); dots(i0); }
+        const float s = t <= pos ? dot * scale : -INFINITY;
+        __syncthreads();                              // (the weights and maxima of the keys before have been read)
+        const float w = wave_max(s);
+        if ((tid & 63) == 0) smax[wave] = w;
+        __syncthreads();
+        const float m_new = fmaxf(m, fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3])));
+        if (t <= pos) ((float*)sp4)[t - b0] = expf(s - m_new);
+        const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
+        m = m_new;
+        __syncthreads();
+        if (adds) {
+            float psum = 0.f, acc = o * alpha;        // in ascending order of the keys
+            for (int b = b0; b < end; b += PAGE) {
+                f32x4 now[PAGE / 4];
+#pragma unroll
+                for (int u = 0; u < PAGE / 4; ++u) now[u] = vv[u];
+                if (b + PAGE < end) values((b - b0) / PAGE + 1);
+                if (b >= t0 && b + PAGE <= end) {
+#pragma unroll
+                    for (int u = 0; u < PAGE / 4; ++u) {
+                        const f32x4 ww = sp4[(b - b0) / 4 + u];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            psum += ww[i];
+                            acc = fmaf(ww[i], now[u][i], acc);
+                        }
+                    }
+                } else {                              // a page that is cut: the sums with the keys outside are not taken
+#pragma unroll
+                    for (int u = 0; u < PAGE / 4; ++u) {
+                        if (b + 4 * u >= end || b + 4 * u + 4 <= t0) continue;
+                        const f32x4 ww = sp4[(b - b0) / 4 + u];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const bool in = b + 4 * u + i >= t0 && b + 4 * u + i < end;
+                            const float p = psum + ww[i], a = fmaf(ww[i], now[u][i], acc);
+                            psum = in ? p : psum;
+                            acc = in ? a : acc;
+                        }
+                    }
+                }
+            }
+            l = l * alpha + psum;
+            o = acc;
+        }
+    }
+    if (tid < HD) out[(tok * H + h) * HD + tid] = o / l;
 }
 
 // ---------------------------------------------------------------------------
@@ -1101,12 +1195,13 @@ extern "C" int li_attn_f32(const float* q, float* out, const void* k, const void
     // heads of a KV head that share a workgroup (and the loads of its keys), where there are workgroups enough without it.  us
     // with one head a workgroup and with them shared: 32 / 8 heads of 64 at 200 keys 4 tokens 9.3 and 12.2, 32 10.7 and 12.3, 48
     // 14.7 and 15.0, 64 16.0 and 14.3, 200 36 and 26; at 1,000 keys 32 51 and 58, 48 57 and 59, 64 68 and 59; at 60 keys 100 13.8 and
-    // 14.9, 200 21.9 and 20.3.  32 / 8 heads of 128 at 200 keys 24 18.2 and 18.9, 32 19.3 and 18.8, 48 24.4 and 20.1
+    // 14.9, 200 21.9 and 20.3.  32 / 8 heads of 128 at 200 keys 24 18.2 and 18.9, 32 19.3 and 18.8, 48 24.4 and 20.1.  Up to there the
+    // kernel for few tokens too: 32 tokens at 200 keys 11.0 and 14.9 with this one at a head a workgroup, at 1,000 57.8 and 77.6
     int hg = (int64_t)n_tokens * H <= 1024 ? 1 : 256 / HD;
     while ((H / K) % hg) --hg;
     dim3 grid(n_tokens, H / hg), block(256);
-    if ((int64_t)n_tokens * H <= 1024) attn_f32_kernel<true><<<grid, block, 0, stream>>>(q, out, c, pos, tok_slot, H, K, hg, scale, window);
-    else attn_f32_kernel<false><<<grid, block, 0, stream>>>(q, out, c, pos, tok_slot, H, K, hg, scale, window);
+    if ((int64_t)n_tokens * H <= 1024) attn_f32_few_kernel<<<grid, block, 0, stream>>>(q, out, c, pos, tok_slot, H, K, scale, window);
+    else attn_f32_kernel<<<grid, block, 0, stream>>>(q, out, c, pos, tok_slot, H, K, hg, scale, window);
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

@@ -759,6 +759,29 @@ def test_float32_attention_with_heads_in_one_workgroup(ops, H, K, hd, n):
             assert torch.equal(one[0], out[t]), (window, t)
 
 
+# a token by itself (the kernel for few tokens) against all of a prompt together, bit for bit: contexts that end at the edges of
+# pages and of the 256 keys taken at a time, windows that begin within a page, at its edge and beyond 256 keys; what lies behind a
+# token in its page is no number and must not reach it
+@pytest.mark.parametrize("H,K,hd", [(4, 1, 16), (6, 2, 64), (5, 1, 112), (3, 1, 256)])
+def test_float32_attention_of_few_tokens(ops, H, K, hd):
+    from llm_infer_amd.engine.step import StepContext
+    g = torch.Generator().manual_seed(hd)
+    n, held = 450, 400
+    k, v, q = (torch.randn(n, m, hd, generator=g) for m in (K, K, H))
+    v[held:] = float("nan")
+    cache, view = _fill_cache(ops, torch.float32, K, hd, [(0, k, v)])
+    ctx = StepContext(DEV, [0], [[0] * n], [0], [[]])
+    qd = q.to(DEV)
+    for window in (None, 37, 64, 100, 300):
+        every = ops.attention_f32(qd, view.as_tuple(), ctx.pos, ctx.tok_slot, H, K, hd, hd ** -0.5, window)[:held]
+        assert torch.isfinite(every).all()
+        for some in ([0, 62, 63], [64, 127, 128, 191], [254, 255, 256], [319, 320, held - 1]):
+            t = torch.tensor(some, device=DEV)
+            few = ops.attention_f32(qd[t].contiguous(), view.as_tuple(), t.to(torch.int32), ctx.tok_slot[t].contiguous(), H, K, hd,
+                                    hd ** -0.5, window)
+            assert torch.equal(few, every[t]), (window, some)
+
+
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
 def test_attention_window_and_far_key(ops, dt):
     """One far key among hundreds stands out by its score; the window cuts it off exactly at its edge."""
