@@ -122,77 +122,89 @@ extern "C" int li_sort_pairs(const int* chosen, int n, int top, int n_experts, i
 }
 
 // ---------------------------------------------------------------------------
-// The router, 16 tokens a workgroup of 16 waves: logits z = W h + b against the tiled 16-bit matrix W [n, K] on the matrix
-// cores, the waves sharing W's tiles of 16 rows and, where there are fewer tiles than waves, K.  W is the sum of `parts`
-// 16-bit matrices one behind the other (each of n rows rounded up to 16: the rounding of W and the roundings of what is
-// left, one matrix where the file's own numbers are 16-bit), so products are those of a float32 W, summed in float32.  Then a wave a token: the `top` largest logits (the first of
-// equals), their weights the softmax over them alone times `scale`.  chosen and weights [T, top], experts ascending.
-// With one workgroup (up to 16 tokens) it also sorts the pairs.
+// The router, 16 tokens at a time, in two launches: logits z = W h + b against the tiled 16-bit matrix W [n, K] on the matrix
+// cores, then the choice.  W is the sum of `parts` 16-bit matrices one behind the other (each of n rows rounded up to 16: the
+// rounding of W and the roundings of what is left, one matrix where the file's own numbers are 16-bit), so products are those of
+// a float32 W, summed in float32.  For a tile of 16 rows of W `kw` waves share K, sixteen waves for all tiles where there are no
+// more tiles than that.  Each is a workgroup of its own: one workgroup of them all is bound by what a CU takes in (W and X,
+// 0.2 to 0.5 MB for 16 x 4,096).  us in a recorded chain, one launch with a workgroup for 16 tokens and these two, 8 tokens:
+// 16 x 4,096 in one part 8.4 -> 5.8, in three 15.3 -> 6.5, 64 x 4,096 18.3 -> 8.6 and 42.8 -> 13.2, 8 x 2,048 6.7 -> 5.2 and 9.6 -> 5.8;
+// 600 tokens x 16 x 4,096 13.4 -> 10.7 and 22.5 -> 12.5, 4,096 tokens 19.1 -> 20.7 and 27.9 -> 29.0 (every CU had its workgroup).
 // ---------------------------------------------------------------------------
 #define ROUTER_WAVES 16
 #define ROUTER_MAX 512
 
-// NC: outputs in groups of 64 that a wave holds, ceil(n / 64) rounded up to 1 or 8.
-template <class T, int NC>
-__global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
-                                                                   const float* __restrict__ bias, int parts, int n_tokens, int K,
-                                                                   int n, int top, float scale, int* __restrict__ chosen,
-                                                                   float* __restrict__ weights, Pairs p) {
+static __host__ __device__ __forceinline__ int router_share(int tiles) { return tiles >= ROUTER_WAVES ? 1 : ROUTER_WAVES / tiles; }
+
+// sums [token / 16][tile * kw + share][lane][4]: a share's accumulators, element q of a lane the output 4 (lane / 16) + q of the
+// tile and the token lane % 16
+template <class T>
+__global__ __launch_bounds__(64) void router_sums_kernel(const T* __restrict__ X, const T* __restrict__ Wt, float* __restrict__ sums,
+                                                         int parts, int n_tokens, int K, int tiles, int kw) {
     typedef typename Vec<T>::v8 v8;
-    constexpr int U = 8;
-    extern __shared__ float lds[];
-    __shared__ float part[ROUTER_WAVES][64][4];
-    float* z = lds;                                        // [16][n]
-    int* picked = (int*)(lds + 16 * n);                    // [16][top]: the chosen experts, for the sort
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-    const int t0 = blockIdx.x * 16, steps = K >> 5, tiles = (n + 15) >> 4;
-    // kw waves share K for a tile; at_once tiles are worked on at a time
-    const int kw = tiles >= ROUTER_WAVES ? 1 : ROUTER_WAVES / tiles, at_once = ROUTER_WAVES / kw;
-    const int share = wave % kw, per = (steps + kw - 1) / kw, s_begin = share * per, s_end = min(steps, s_begin + per);
+    constexpr int U = 8, AHEAD = 3;                        // batches of loads on their way together
+    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4, t0 = blockIdx.x * 16;
+    const int steps = K >> 5, tile = blockIdx.y / kw, share = blockIdx.y % kw;
+    const int per = (steps + kw - 1) / kw, s_begin = share * per, s_end = min(steps, s_begin + per);
+    const int batches = s_end > s_begin ? (s_end - s_begin + U - 1) / U : 0, total = parts * batches;
     const bool have = t0 + r < n_tokens;
     const T* xrow = X + (int64_t)(have ? t0 + r : t0) * K + 8 * g;
-    for (int first = 0; first < tiles; first += at_once) {
-        const int tile = first + wave / kw;
-        const bool on = wave / kw < at_once && tile < tiles;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        if (on) {
-            for (int pt = 0; pt < parts; ++pt) {
-            const T* wt = Wt + ((int64_t)(pt * tiles + tile) * steps * 64 + lane) * 8;
-            for (int s0 = s_begin; s0 < s_end; s0 += U) {
-                v8 a[U], b[U];
+    v8 a[AHEAD][U], b[AHEAD][U];
+    auto load = [&](int i, v8 (&av)[U], v8 (&bv)[U]) {     // the parts one after the other, K ascending in each
+        const int pt = i / batches, s0 = s_begin + i % batches * U;
+        const T* wt = Wt + ((int64_t)(pt * tiles + tile) * steps * 64 + lane) * 8;
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    const v8 zero = {};
-                    const bool in = s0 + u < s_end;
-                    a[u] = in ? *(const v8*)(wt + (int64_t)(s0 + u) * 512) : zero;
-                    b[u] = in && have ? *(const v8*)(xrow + (s0 + u) * 32) : zero;
-                }
-#pragma unroll
-                for (int u = 0; u < U; ++u) acc = mfma16(a[u], b[u], acc);
-            }
-            }
+        for (int u = 0; u < U; ++u) {
+            const v8 zero = {};
+            const bool in = s0 + u < s_end;
+            av[u] = in ? *(const v8*)(wt + (int64_t)(s0 + u) * 512) : zero;
+            bv[u] = in && have ? *(const v8*)(xrow + (s0 + u) * 32) : zero;
         }
+    };
 #pragma unroll
-        for (int q = 0; q < 4; ++q) part[wave][lane][q] = acc[q];
-        __syncthreads();
-        if (on && share == 0) {
+    for (int k = 0; k < AHEAD; ++k) if (k < total) load(k, a[k], b[k]);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int i = 0; i < total; i += AHEAD) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                float v = part[wave][lane][q];
-                for (int k = 1; k < kw; ++k) v += part[wave + k][lane][q];
-                const int j = tile * 16 + 4 * g + q;
-                if (j < n) z[r * n + j] = v + (bias ? bias[j] : 0.f);
-            }
+        for (int k = 0; k < AHEAD; ++k) {
+            if (i + k >= total) break;
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc = mfma16(a[k][u], b[k][u], acc);
+            if (i + k + AHEAD < total) load(i + k + AHEAD, a[k], b[k]);
         }
-        __syncthreads();
     }
+    *(f32x4*)(sums + (((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * 64 + lane) * 4) = acc;
+}
+
+// The choice, a wave a token: its logits are the shares' sums in ascending order; the `top` largest (the first of equals), their
+// weights the softmax over them alone times `scale`.  chosen and weights [T, top], experts ascending.  With one workgroup (up
+// to 16 tokens) it also sorts the pairs.
+// NC: outputs in groups of 64 that a wave holds, ceil(n / 64) rounded up to 1 or 8.
+template <int NC>
+__global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const float* __restrict__ sums, const float* __restrict__ bias,
+                                                                   int n_tokens, int n, int kw, int top, float scale,
+                                                                   int* __restrict__ chosen, float* __restrict__ weights, Pairs p) {
+    constexpr int SHARES = NC == 1 ? ROUTER_WAVES : 3;     // kw at the most: n > 64 has five tiles or more
+    extern __shared__ int picked[];                        // [16][top]: the chosen experts, for the sort
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int t0 = blockIdx.x * 16, tiles = (n + 15) >> 4;
     const int t = t0 + wave;
     if (t < n_tokens) {                                    // (a wave's token, the same for all its lanes)
-        float* zt = z + wave * n;
         float mx = 0.f, sum = 0.f;
         float zs[NC];
 #pragma unroll
-        for (int c = 0; c < NC; ++c) zs[c] = c * 64 + lane < n ? zt[c * 64 + lane] : -INFINITY;
+        for (int c = 0; c < NC; ++c) {
+            const int j = min(c * 64 + lane, n - 1);
+            const float* at = sums + (((int64_t)blockIdx.x * tiles + (j >> 4)) * kw * 64 + ((j >> 2) & 3) * 16 + wave) * 4 + (j & 3);
+            const float own = bias ? bias[j] : 0.f;
+            float v[SHARES];
+#pragma unroll
+            for (int k = 0; k < SHARES; ++k) v[k] = at[(int64_t)min(k, kw - 1) * 256];
+            float z = v[0];
+#pragma unroll
+            for (int k = 1; k < SHARES; ++k) z = k < kw ? z + v[k] : z;
+            zs[c] = c * 64 + lane < n ? z + own : -INFINITY;
+        }
         uint32_t taken = 0;                                // bit c: this lane's output c * 64 + lane is chosen
         for (int k = 0; k < top; ++k) {
             float best = -INFINITY; int bi = 0x7fffffff;
@@ -251,22 +263,23 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const T* __re
     }
 }
 
-// counts (and the other three) not null with up to 16 tokens: the pairs are sorted too.
+// counts (and the other three) not null with up to 16 tokens: the pairs are sorted too.  sums: float32, 256 * max(16, ceil(n / 16))
+// for every 16 tokens.
 extern "C" int li_router(const void* X, const void* Wt, int dt, const float* bias, int parts, int n_tokens, int K, int n, int top, float scale,
-                         int* chosen, float* weights, int* counts, int* offsets, int* row_of, int* slot_of, hipStream_t stream) {
+                         int* chosen, float* weights, int* counts, int* offsets, int* row_of, int* slot_of, float* sums, hipStream_t stream) {
     if (n_tokens <= 0) return LI_OK;
-    if (!X || !Wt || !chosen || !weights || n < 1 || top < 1 || top > n || parts < 1 || parts > 3) return LI_BAD_ARG;
-    if (n > ROUTER_MAX || K < 32 || K % 32 || ((uintptr_t)X & 15) || ((uintptr_t)Wt & 15)) return LI_UNSUPPORTED;
+    if (!X || !Wt || !chosen || !weights || !sums || n < 1 || top < 1 || top > n || parts < 1 || parts > 3) return LI_BAD_ARG;
+    if (n > ROUTER_MAX || n + top > 640 || K < 32 || K % 32 || ((uintptr_t)X & 15) || ((uintptr_t)Wt & 15) || ((uintptr_t)sums & 15)) return LI_UNSUPPORTED;
     if (counts && (n_tokens > 16 || !offsets || !row_of || !slot_of)) return LI_BAD_ARG;
     const Pairs p{counts, offsets, row_of, slot_of};
-    const size_t lds = (size_t)16 * (n + top) * sizeof(float);
-    if (lds > 40 * 1024) return LI_UNSUPPORTED;
-    const int blocks = (n_tokens + 15) / 16;
-#define GO(T, NC) router_kernel<T, NC><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>((const T*)X, (const T*)Wt, bias, parts, n_tokens, K, n, top, scale, chosen, weights, p)
-    if (dt == DT_F16) { if (n <= 64) GO(f16, 1); else GO(f16, 8); }
-    else if (dt == DT_BF16) { if (n <= 64) GO(bf16, 1); else GO(bf16, 8); }
-#undef GO
+    const int blocks = (n_tokens + 15) / 16, tiles = (n + 15) / 16, kw = router_share(tiles);
+    dim3 grid(blocks, tiles * kw);
+    if (dt == DT_F16) router_sums_kernel<f16><<<grid, 64, 0, stream>>>((const f16*)X, (const f16*)Wt, sums, parts, n_tokens, K, tiles, kw);
+    else if (dt == DT_BF16) router_sums_kernel<bf16><<<grid, 64, 0, stream>>>((const bf16*)X, (const bf16*)Wt, sums, parts, n_tokens, K, tiles, kw);
     else return LI_BAD_ARG;
+    const size_t lds = (size_t)16 * top * sizeof(int);
+    if (n <= 64) router_kernel<1><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>(sums, bias, n_tokens, n, kw, top, scale, chosen, weights, p);
+    else router_kernel<8><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>(sums, bias, n_tokens, n, kw, top, scale, chosen, weights, p);
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

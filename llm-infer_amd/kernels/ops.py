@@ -2304,8 +2304,9 @@ def route_pairs(h, w_router, bias, n_experts: int, top: int, scale: float = 1.0)
     p = SortedPairs(t, top, n, h.device)
     lists = (_ptr(p.counts), _ptr(p.offsets), _ptr(p.row_of), _ptr(p.slot_of))
     small = t <= 16                                        # one workgroup has every token: it sorts the pairs too
+    sums = torch.empty(((t + 15) // 16 * max(16, (n + 15) // 16) * 256,), dtype=torch.float32, device=h.device)
     _check(experts().li_router(_ptr(h), _ptr(w_router), DT[h.dtype], _ptr(bias), parts, t, k, n, top, c_float(scale), _ptr(p.chosen),
-                               _ptr(p.weights), *(lists if small else (None,) * 4), _stream()), "router")
+                               _ptr(p.weights), *(lists if small else (None,) * 4), _ptr(sums), _stream()), "router")
     if not small:
         _check(experts().li_sort_pairs(_ptr(p.chosen), t * top, top, n, *lists, _stream()), "sort_pairs")
     return p

@@ -271,6 +271,25 @@ def test_router_and_the_sorted_pairs(lib, E, top, dtype):
             assert torch.allclose(p.weights.cpu().double(), 2.5 * torch.softmax(zz.gather(1, p.chosen.cpu().long()), -1), atol=5e-6)
 
 
+# K in one batch of loads a share, in several that run out in the middle of one, with a last share that is shorter or has none
+@pytest.mark.parametrize("E,K", [(16, 288), (16, 4128), (70, 1056), (300, 1312)])
+def test_router_sums_by_shares_of_k(lib, E, K):
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(E + K)
+    for stored in (torch.bfloat16, torch.float32):
+        W = (torch.randn(E, K, generator=g) * K ** -0.5).to(stored).float()
+        wr = ops.router_weight(W.to(DEV), torch.bfloat16)
+        for T in (3, 20):
+            h = torch.randn(T, K, generator=g).to(torch.bfloat16)
+            z = h.double() @ W.double().T
+            best = torch.topk(z, 5, -1).values
+            # logits of the order of 1: some 400 roundings of 2^-24 in a chain, three parts of W; 1e-4 is beyond their sum
+            keep = (best[:, 3] - best[:, 4]) > 1e-4
+            h, z = h[keep].contiguous(), z[keep]
+            chosen = torch.topk(z, 4, -1).indices.sort(-1).values
+            check_pairs(ops.route_pairs(h.to(DEV), wr, None, E, 4), chosen, torch.softmax(z.gather(1, chosen), -1))
+
+
 def test_the_first_of_equal_logits_is_chosen_and_numbers_that_are_none_do_no_harm(lib):
     from llm_infer_amd.kernels import ops
     h = torch.ones(20, 32, dtype=torch.bfloat16, device=DEV)
