@@ -728,8 +728,9 @@ __global__ __launch_bounds__(256) void small_logits_kernel(const T* __restrict__
 // The same sums, bit for bit, for rows of up to 4,096 elements in whole quads: a wave takes TOK tokens, a lane four neighbouring
 // partial sums of the 256, so that the operands come 16 and 8 bytes at a time, h once for JB outputs, and only lanes exchange sums.
 // Bound by its loads' latency for few tokens, by the weights' way from L2 for many: 2,253 tokens x 9 outputs of 4,096 75 -> 21 us,
-// 8,000 x 16 459 -> 63, 300 x 9 12.0 -> 8.7, 4 tokens 4.15 -> 4.0.
-template <class T, int TOK, int JB>
+// 8,000 x 16 459 -> 63, 300 x 9 12.0 -> 8.7.  B: quads of a lane on their way together, all of a row for few tokens (one by one and
+// then, us in a recorded chain, 4 tokens x 9 outputs of 4,096 3.5 -> 2.2, 8 x 16 of 2,048 2.2 -> 1.8, 255 x 16 of 4,096 7.2 -> 6.1); eight are enough for half as wide a row.
+template <class T, int TOK, int JB, int B>
 __global__ void small_logits_wave_kernel(const T* __restrict__ h, const float* __restrict__ w, float* __restrict__ out,
                                          const float* __restrict__ bias, int n_rows, int width, int n) {
 #pragma clang fp contract(off)
@@ -739,24 +740,29 @@ __global__ void small_logits_wave_kernel(const T* __restrict__ h, const float* _
     if (t0 >= n_rows) return;
     float acc[TOK][JB][4] = {};
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int i = u * 256 + 4 * lane;
-        if (i >= width) break;
-        Quad x[TOK];
-        f32x4 wv[JB];
+    for (int u = 0; u < (B > 1 ? B : 16); u += B) {
+        if (B == 1 && u * 256 + 4 * lane >= width) break;
+        Quad x[B][TOK];
+        f32x4 wv[B][JB];
 #pragma unroll
-        for (int k = 0; k < TOK; ++k) x[k] = *(const Quad*)(h + (int64_t)min(t0 + k, n_rows - 1) * width + i);
+        for (int b = 0; b < B; ++b) {
+            const int i = min((u + b) * 256 + 4 * lane, width - 4);
 #pragma unroll
-        for (int j = 0; j < JB; ++j) wv[j] = *(const f32x4*)(w + (int64_t)min(j0 + j, n - 1) * width + i);
+            for (int k = 0; k < TOK; ++k) x[b][k] = *(const Quad*)(h + (int64_t)min(t0 + k, n_rows - 1) * width + i);
 #pragma unroll
-        for (int k = 0; k < TOK; ++k)
+            for (int j = 0; j < JB; ++j) wv[b][j] = *(const f32x4*)(w + (int64_t)min(j0 + j, n - 1) * width + i);
+        }
 #pragma unroll
-            for (int j = 0; j < JB; ++j)
+        for (int b = 0; b < B; ++b)
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float product = wv[j][q] * to_f32(x[k].v[q]);
-                    acc[k][j][q] += product;
-                }
+            for (int k = 0; k < TOK; ++k)
+#pragma unroll
+                for (int j = 0; j < JB; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const float product = wv[b][j][q] * to_f32(x[b][k].v[q]), with = acc[k][j][q] + product;
+                        acc[k][j][q] = B == 1 || (u + b) * 256 + 4 * lane < width ? with : acc[k][j][q];
+                    }
     }
 #pragma unroll
     for (int k = 0; k < TOK; ++k)
@@ -779,9 +785,11 @@ extern "C" int li_small_logits(const void* h, int dt, const float* w, float* out
     if (width <= 0 || n > 65535) return LI_BAD_ARG;
     if (width % 4 == 0 && width <= 4096 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)h & (dt == DT_F32 ? 15 : 7)) == 0) {
         if (n_rows >= 256) {                               // many tokens: two a wave, four outputs at a time
-            DISPATCH_T(dt, (small_logits_wave_kernel<T, 2, 4><<<dim3((n_rows + 7) / 8, (n + 3) / 4), 256, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+            DISPATCH_T(dt, (small_logits_wave_kernel<T, 2, 4, 1><<<dim3((n_rows + 7) / 8, (n + 3) / 4), 256, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
         } else {
-            DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1><<<dim3(n_rows, n), 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+            dim3 grid(n_rows, n);
+            if (width <= 2048) DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1, 8><<<grid, 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+            else DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1, 16><<<grid, 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
         }
     } else if (n_rows >= 256) {                            // many tokens: four a workgroup share every weight fetched
         dim3 grid((n_rows + 3) / 4, n);

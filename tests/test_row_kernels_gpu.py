@@ -136,3 +136,15 @@ def test_average_over_depth_with_its_norms(ops, width, terms):
     assert torch.equal(out, plain)
     for w, eps, dt in norms:
         assert torch.equal(ops.prepared_norm(out, w, eps, dt), ops.rmsnorm(plain, w, eps, dt))
+
+
+# a row shorter than a wave's first loads, ragged against them, whole, of the wider form and beyond it; few tokens against many
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("t,width,n", [(1, 4, 1), (3, 260, 8), (5, 2048, 16), (2, 2052, 9), (255, 1028, 17), (4, 4096, 9), (2, 66, 4), (2, 4100, 4)])
+def test_router_logits_of_few_tokens(ops, dtype, t, width, n):
+    h, w, bias = torch.randn(t, width, device=DEV).to(dtype), torch.randn(n, width, device=DEV) * width ** -0.5, torch.randn(n, device=DEV)
+    z = ops.small_logits(h, w, bias)
+    want = h.double() @ w.double().T + bias.double()
+    # 16 sums of a lane, 4 of lanes, 2 of quads, 4 of waves: some 30 roundings at the most, 2^-19 of the products' absolute sum
+    assert ((z - want).abs() <= 2.0 ** -19 * (1 + h.double().abs() @ w.double().abs().T + bias.double().abs())).all()
+    assert torch.equal(ops.small_logits(h.repeat(256 // t + 1, 1), w, bias)[:t], z)
