@@ -768,8 +768,8 @@ extern "C" int li_sigmoid_attn(const void* q, void* out, int dt, const void* k_p
 // ---------------------------------------------------------------------------
 // Linear attention with a constant decay per head, token by token:
 //   S <- decay[h] * S + k_t v_t^T,   o_t = S^T q_t,        q, k, v = silu of the projections
-// One workgroup per (sequence, head).  The state S [d, dv] of the pair is float32; it is read from
-// `state[slot, h]` when the workgroup starts and written back when the sequence's tokens of this step are
+// One workgroup per (sequence, head), or several that share the head's columns (they do not meet).  The state S [d, dv] of the
+// pair is float32; it is read from `state[slot, h]` when the workgroup starts and written back when the sequence's tokens of this step are
 // done, so a prompt in one step, in portions, or token by token does the same arithmetic in the same order.
 // Thread (rg, j) keeps rows rg*ROWS .. rg*ROWS+ROWS-1 of column j in registers; the partial sums of o over the
 // row groups are added in ascending order through LDS.
@@ -777,29 +777,32 @@ extern "C" int li_sigmoid_attn(const void* q, void* out, int dt, const void* k_p
 //   seq_qstart / seq_qlen null: one token per sequence, row i of the step belongs to sequence i (decoding)
 // TR: q, k and v take this type's values after the silu (float: as they are), so that a 16-bit model's
 // decoding multiplies the numbers that its chunked kernel for prompts multiplies.
+// WHOLE: d is a multiple of ROWS, and no row of S is asked for under a condition, each of which waited for the row before.  A
+// decode step is bound by the way of its loads and stores: us in a recorded chain, rows under conditions and now, 16 heads of
+// 128 x 128, 1 sequence 8.5 -> 4.2, 4 8.3 -> 4.8, 16 12.0 -> 10.2; 8 of 64 x 64 3.6 -> 2.3; 4 of 80 x 96 (not whole) 5.5 -> 3.1.
 // ---------------------------------------------------------------------------
 template <class T> __device__ __forceinline__ float rounded_to(float v) { return to_f32(from_f32<T>(v)); }
 template <> __device__ __forceinline__ float rounded_to<float>(float v) { return v; }
 
-template <int ROWS, class TR>
+template <int ROWS, class TR, bool WHOLE>
 __global__ void decay_attn_kernel(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
                                   float* __restrict__ state, const float* __restrict__ decay,
                                   const int* __restrict__ seq_slot, const int* __restrict__ seq_qstart,
                                   const int* __restrict__ seq_qlen, float* __restrict__ out, int H, int d, int dv) {
     extern __shared__ float lds[];
-    const int RG = blockDim.x / dv;
+    const int cols = dv / gridDim.z, RG = blockDim.x / cols;
     float* sq = lds;                    // [d]
     float* sk = sq + d;                 // [d]
-    float* sv = sk + d;                 // [dv]
-    float* red = sv + dv;               // [RG, dv]
-    const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x;
-    const int j = tid % dv, rg = tid / dv, r0 = rg * ROWS;
+    float* sv = sk + d;                 // [cols]
+    float* red = sv + cols;             // [RG, cols]
+    const int seq = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * cols, tid = threadIdx.x;
+    const int jc = tid % cols, j = j0 + jc, rg = tid / cols, r0 = rg * ROWS;
     const int q0 = seq_qstart ? seq_qstart[seq] : seq, n = seq_qlen ? seq_qlen[seq] : 1;
     float* S = state + (((int64_t)seq_slot[seq] * H + h) * d) * dv;
     const float lam = decay[h];
     float s[ROWS];
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) s[r] = r0 + r < d ? S[(int64_t)(r0 + r) * dv + j] : 0.f;
+    for (int r = 0; r < ROWS; ++r) s[r] = S[(int64_t)(WHOLE ? r0 + r : min(r0 + r, d - 1)) * dv + j];
     for (int t = 0; t < n; ++t) {
         const float* row = proj + (int64_t)(q0 + t) * stride;
         __syncthreads();
@@ -807,27 +810,27 @@ __global__ void decay_attn_kernel(const float* __restrict__ proj, int stride, in
             sq[i] = rounded_to<TR>(siluf(row[q_off + h * d + i]));
             sk[i] = rounded_to<TR>(siluf(row[k_off + h * d + i]));
         }
-        for (int i = tid; i < dv; i += blockDim.x) sv[i] = rounded_to<TR>(siluf(row[v_off + h * dv + i]));
+        for (int i = tid; i < cols; i += blockDim.x) sv[i] = rounded_to<TR>(siluf(row[v_off + h * dv + j0 + i]));
         __syncthreads();
-        const float vj = sv[j];
+        const float vj = sv[jc];
         float part = 0.f;
 #pragma unroll
         for (int r = 0; r < ROWS; ++r) {
-            if (r0 + r < d) {
+            if (WHOLE || r0 + r < d) {
                 s[r] = lam * s[r] + sk[r0 + r] * vj;
                 part += s[r] * sq[r0 + r];
             }
         }
-        red[rg * dv + j] = part;
+        red[rg * cols + jc] = part;
         __syncthreads();
         if (rg == 0) {
             float o = 0.f;
-            for (int g = 0; g < RG; ++g) o += red[g * dv + j];
+            for (int g = 0; g < RG; ++g) o += red[g * cols + jc];
             out[(int64_t)(q0 + t) * H * dv + h * dv + j] = o;
         }
     }
 #pragma unroll
-    for (int r = 0; r < ROWS; ++r) if (r0 + r < d) S[(int64_t)(r0 + r) * dv + j] = s[r];
+    for (int r = 0; r < ROWS; ++r) if (WHOLE || r0 + r < d) S[(int64_t)(r0 + r) * dv + j] = s[r];
 }
 
 extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off, int v_off, float* state,
@@ -839,14 +842,21 @@ extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off
     while (rows < 64 && ((d + rows - 1) / rows) * dv > 512) rows *= 2;
     const int RG = (d + rows - 1) / rows;
     if (RG * dv > 1024) return LI_UNSUPPORTED;
-    dim3 grid(n_seqs, H), block(RG * dv);
-    const size_t lds = (size_t)(2 * d + dv + RG * dv) * sizeof(float);
-#define GO1(R, TR) decay_attn_kernel<R, TR><<<grid, block, lds, stream>>>(proj, stride, q_off, k_off, v_off, state, \
+    // few sequences: a head's columns over several workgroups, a line of 128 bytes of a row of S each at the least, until every CU
+    // has one (16 heads of 128 x 128, 1 sequence 6.4 -> 4.1 us, 8 7.6 -> 6.6)
+    int split = 1;
+    while ((int64_t)n_seqs * H * split < 256 && dv % (2 * split) == 0 && dv / (2 * split) >= 32) split *= 2;
+    const int cols = dv / split;
+    dim3 grid(n_seqs, H, split), block(RG * cols);
+    const size_t lds = (size_t)(2 * d + cols + RG * cols) * sizeof(float);
+#define GO2(R, TR, WHOLE) decay_attn_kernel<R, TR, WHOLE><<<grid, block, lds, stream>>>(proj, stride, q_off, k_off, v_off, state, \
         decay, seq_slot, seq_qstart, seq_qlen, out, H, d, dv)
+#define GO1(R, TR) do { if (d % R == 0) GO2(R, TR, true); else GO2(R, TR, false); } while (0)
 #define GO(R) do { if (round_dt == DT_F32) GO1(R, float); else if (round_dt == DT_F16) GO1(R, f16); else GO1(R, bf16); } while (0)
     if (rows == 4) GO(4); else if (rows == 8) GO(8); else if (rows == 16) GO(16); else if (rows == 32) GO(32); else GO(64);
 #undef GO
 #undef GO1
+#undef GO2
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

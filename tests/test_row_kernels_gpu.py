@@ -148,3 +148,29 @@ def test_router_logits_of_few_tokens(ops, dtype, t, width, n):
     # 16 sums of a lane, 4 of lanes, 2 of quads, 4 of waves: some 30 roundings at the most, 2^-19 of the products' absolute sum
     assert ((z - want).abs() <= 2.0 ** -19 * (1 + h.double().abs() @ w.double().abs().T + bias.double().abs())).all()
     assert torch.equal(ops.small_logits(h.repeat(256 // t + 1, 1), w, bias)[:t], z)
+
+
+# rows of a state that divide among a thread's and not, columns that split over workgroups and not; a sequence alone (its heads'
+# columns over several workgroups where they can) and among 256 (a workgroup a head), step by step, bit for bit, and against 64 bits
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,d,dv", [(4, 80, 96), (16, 128, 128), (3, 33, 64), (2, 256, 64), (5, 20, 48), (1, 7, 1), (2, 128, 256)])
+def test_decay_recurrence_of_one_sequence_and_many(ops, dtype, H, d, dv):
+    n, steps = 256, 3
+    decay = torch.linspace(0.5, 0.99, H, device=DEV)
+    many, alone = torch.randn(n, H, d, dv, device=DEV), None
+    alone = many[7:8].clone()
+    S = alone.double()[0].cpu()
+    rounded = dtype if dtype != torch.float32 else None
+    for _ in range(steps):
+        proj = torch.randn(n, H * (2 * d + dv), device=DEV)
+        o = ops.decay_attention(proj, 0, H * d, 2 * H * d, many, decay, torch.arange(n, device=DEV, dtype=torch.int32), None, None, n, H, d, dv,
+                                round_to=rounded)
+        one = ops.decay_attention(proj[7:8].contiguous(), 0, H * d, 2 * H * d, alone, decay, torch.zeros(1, device=DEV, dtype=torch.int32), None, None, 1,
+                                  H, d, dv, round_to=rounded)
+        assert torch.equal(one[0], o[7]) and torch.equal(alone[0], many[7])
+        if rounded is None:
+            q, k, v = (torch.nn.functional.silu(p.double()) for p in proj[7].cpu().split([H * d, H * d, H * dv]))
+            S = decay.double().cpu()[:, None, None] * S + k.view(H, d, 1) * v.view(H, 1, dv)
+            want = (S * q.view(H, d, 1)).sum(1)
+            # some 100 roundings of 2^-24 in a sum of up to 256 products of the order of 1
+            assert ((one[0].view(H, dv).double().cpu() - want).abs() <= 2.0 ** -17 * (S * q.view(H, d, 1)).abs().sum(1) + 1e-6).all()
