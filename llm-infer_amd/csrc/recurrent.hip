@@ -234,15 +234,24 @@ __global__ __launch_bounds__(64 * SCAN_WAVES * CB) void delta_scan_kernel(const 
     __shared__ __attribute__((aligned(16))) float sk[3][DP], sq[3][DP];
     __shared__ float part[2][CB][SCAN_WAVES][2][64], sq_sum[2][CB];
     const int seq = blockIdx.x, h = blockIdx.y, e = h / (H / G), tid = threadIdx.x, lane = tid & 63;
-    const int wave = (tid >> 6) % SCAN_WAVES, cb = (tid >> 6) / SCAN_WAVES;
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_id % SCAN_WAVES, cb = wave_id / SCAN_WAVES;
     const int col = (blockIdx.z * CB + cb) * 64 + lane, C = 2 * G * d + H * dv, r0 = wave * NR;
     const int q0 = st.seq_qstart ? st.seq_qstart[seq] : seq, n = st.seq_qlen ? st.seq_qlen[seq] : 1;
     if (n <= 0) return;
     const bool live = col < dv;
     float* S = state + (((int64_t)st.seq_slot[seq] * H + h) * d) * dv + col;
     float s[NR];
+    // a wave whose rows and columns are all there asks for them under no condition, each of which was a branch.  A decode step, us in
+    // a recorded chain, before and now: 1 sequence, 16 heads of 128 x 128 5.3 -> 3.7, 8 of 256 x 256 7.6 -> 4.8, 16 of 64 x 64 3.5 -> 3.0;
+    // 16 sequences 8.1, 13.7 -> 13.2, 4.1 -> 3.5
+    const bool whole = r0 + NR <= d && col - lane + 64 <= dv;
+    if (whole) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) s[r] = (live && r0 + r < d) ? S[(int64_t)(r0 + r) * dv] : 0.f;
+        for (int r = 0; r < NR; ++r) s[r] = S[(int64_t)(r0 + r) * dv];
+    } else {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) s[r] = (live && r0 + r < d) ? S[(int64_t)(r0 + r) * dv] : 0.f;
+    }
     auto stage = [&](int t) {
         const float* row = qkv + (int64_t)(q0 + t) * C;
         for (int i = tid; i < DP; i += 64 * SCAN_WAVES * CB) {
@@ -283,7 +292,10 @@ __global__ __launch_bounds__(64 * SCAN_WAVES * CB) void delta_scan_kernel(const 
 #pragma unroll
         for (int r = 0; r < NR; ++r) s[r] = g * s[r] + k[r] * u;
     }
-    if (live) {
+    if (whole) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) S[(int64_t)(r0 + r) * dv] = s[r];
+    } else if (live) {
 #pragma unroll
         for (int r = 0; r < NR; ++r) if (r0 + r < d) S[(int64_t)(r0 + r) * dv] = s[r];
     }
@@ -513,15 +525,23 @@ __global__ __launch_bounds__(64 * SCAN_WAVES * CB) void wkv_scan_kernel(const fl
     __shared__ __attribute__((aligned(16))) float sr[3][DP], sk[3][DP], sw[3][DP];
     __shared__ float part[2][CB][SCAN_WAVES][64], ruk[3][SCAN_WAVES * CB], sq_sum[2][CB];
     const int seq = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
-    const int wave = (tid >> 6) % SCAN_WAVES, cb = (tid >> 6) / SCAN_WAVES, r0 = wave * NR;
+    const int wave_id = __builtin_amdgcn_readfirstlane(tid >> 6), wave = wave_id % SCAN_WAVES, cb = wave_id / SCAN_WAVES, r0 = wave * NR;
     const int col = (blockIdx.z * CB + cb) * 64 + lane;
     const int q0 = st.seq_qstart ? st.seq_qstart[seq] : seq, n = st.seq_qlen ? st.seq_qlen[seq] : 1;
     if (n <= 0) return;
     const bool live = col < d;
     float* S = state + (((int64_t)st.seq_slot[seq] * H + h) * d) * d + col;
     float s[NR];
+    // (no condition on a row, as in delta_scan_kernel: 1 sequence, 32 heads of 64 3.6 -> 2.8 us, 16 of 128 5.3 -> 3.7, 8 of 256 7.3 -> 4.9;
+    // 16 sequences 5.0 -> 4.4, 8.0 -> 7.6, 18.4 -> 12.6)
+    const bool whole = r0 + NR <= d && col - lane + 64 <= d;
+    if (whole) {
 #pragma unroll
-    for (int r = 0; r < NR; ++r) s[r] = (live && r0 + r < d) ? S[(int64_t)(r0 + r) * d] : 0.f;
+        for (int r = 0; r < NR; ++r) s[r] = S[(int64_t)(r0 + r) * d];
+    } else {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) s[r] = (live && r0 + r < d) ? S[(int64_t)(r0 + r) * d] : 0.f;
+    }
     static_assert(DP <= 64 * SCAN_WAVES, "a thread a key channel");
     const float ub = tid < d ? bonus[h * d + tid] : 0.f;
     auto stage = [&](int t) {
@@ -570,7 +590,10 @@ __global__ __launch_bounds__(64 * SCAN_WAVES * CB) void wkv_scan_kernel(const fl
         }
         if (wave == 0 && live) store_head(ho, tok, H * d, h, d, col, o, ss);
     }
-    if (live) {
+    if (whole) {
+#pragma unroll
+        for (int r = 0; r < NR; ++r) S[(int64_t)(r0 + r) * d] = s[r];
+    } else if (live) {
 #pragma unroll
         for (int r = 0; r < NR; ++r) if (r0 + r < d) S[(int64_t)(r0 + r) * d] = s[r];
     }

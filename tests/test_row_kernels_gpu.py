@@ -174,3 +174,43 @@ def test_decay_recurrence_of_one_sequence_and_many(ops, dtype, H, d, dv):
             want = (S * q.view(H, d, 1)).sum(1)
             # some 100 roundings of 2^-24 in a sum of up to 256 products of the order of 1
             assert ((one[0].view(H, dv).double().cpu() - want).abs() <= 2.0 ** -17 * (S * q.view(H, d, 1)).abs().sum(1) + 1e-6).all()
+
+
+# one token a sequence with a state whose rows and columns are all there (fetched under no condition), and with rows or columns that a
+# wave has not; three steps in a row against 64 bits
+@pytest.mark.parametrize("rows,cols", [(64, 64), (128, 128), (64, 40), (100, 64), (7, 130), (16, 64), (256, 64)])
+def test_recurrences_with_whole_and_ragged_states(ops, rows, cols):
+    from types import SimpleNamespace
+    n, H = 3, 2
+    ctx = SimpleNamespace(seq_slot=torch.tensor([2, 0, 1], dtype=torch.int32, device=DEV), n_seqs=n, n_tokens=n)
+    slot = ctx.seq_slot.long()
+    r = lambda *s: torch.randn(*s, device=DEV)
+    # a sum of up to 256 products takes up to 8 + rows / 4 roundings of 2^-24 in a row; three steps, factors of the order of 1
+    near = lambda got, want, size: bool(((got.double() - want).abs() <= 2.0 ** -16 * (1 + size)).all())
+    delta, ssm, wkv = r(n, H, rows, cols), r(n, H, rows, cols), r(n, H, rows, rows)
+    D, M, W = (s.double()[slot].clone() for s in (delta, ssm, wkv))
+    for _ in range(3):
+        x, g, kq = r(n, 2 * H * rows + H * cols) * rows ** -0.5, torch.stack([-torch.rand(n, H, device=DEV), torch.rand(n, H, device=DEV)], -1), r(n, H)
+        q, k, v = (p.double() for p in x.split([H * rows, H * rows, H * cols], 1))
+        q, k, v = q.view(n, H, rows, 1), k.view(n, H, rows, 1), v.view(n, H, 1, cols)
+        kq = (q * k).sum((2, 3)).float().contiguous()
+        o = ops.delta_scan(x, g.contiguous(), kq, delta, ctx, H, H, rows, cols).view(n, H, cols)
+        D = D * g[..., 0].double().exp()[..., None, None]
+        D = D + k * (g[..., 1].double()[..., None, None] * (v - (D * k).sum(2, keepdim=True)))
+        assert near(o, (D * q).sum(2), (D * q).abs().sum(2)) and near(delta[slot], D, D.abs())
+
+        xbc, proj, bias, alog, skip = r(n, H * cols + 2 * rows), r(n, H), r(H), r(H) * 0.3, r(H)
+        y = ops.ssm_scan(xbc, proj, 0, bias, alog, skip, ssm, ctx, H, 1, rows, cols, None).view(n, H, cols)
+        xs, B, C = (p.double() for p in xbc.split([H * cols, rows, rows], 1))
+        dt = torch.nn.functional.softplus(proj.double() + bias.double())[..., None, None]
+        M = M * (-alog.double().exp()[:, None, None] * dt).exp() + dt * B.view(n, 1, rows, 1) * xs.view(n, H, 1, cols)
+        want = (M * C.view(n, 1, rows, 1)).sum(2) + skip.double()[:, None] * xs.view(n, H, cols)
+        assert near(y, want, (M * C.view(n, 1, rows, 1)).abs().sum(2)) and near(ssm[slot], M, M.abs())
+
+        a, kk, vv, raw, bonus = r(n, H * rows), r(n, H * rows), r(n, H * rows), r(n, H * rows), r(H, rows)
+        o = ops.wkv_scan(a, kk, vv, raw, bonus, wkv, ctx, H, rows).view(n, H, rows)
+        ad, kd, vd = a.double().view(n, H, rows, 1), kk.double().view(n, H, rows, 1), vv.double().view(n, H, 1, rows)
+        seen = W + bonus.double()[..., None] * kd * vd
+        assert near(o, (seen * ad).sum(2), (seen * ad).abs().sum(2))
+        W = W * (-raw.double().view(n, H, rows, 1).exp()).exp() + kd * vd
+        assert near(wkv[slot], W, W.abs())
