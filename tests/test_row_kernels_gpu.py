@@ -214,3 +214,26 @@ def test_recurrences_with_whole_and_ragged_states(ops, rows, cols):
         assert near(o, (seen * ad).sum(2), (seen * ad).abs().sum(2))
         W = W * (-raw.double().view(n, H, rows, 1).exp()).exp() + kd * vd
         assert near(wkv[slot], W, W.abs())
+
+
+# value sizes in whole fours (four dimensions a store) and not, one split and several, against the kernel that takes a key after
+# the other
+@pytest.mark.parametrize("dk,dv,vdim", [(16, 32, 32), (16, 30, 32), (64, 64, 64), (64, 49, 64), (64, 60, 64)])
+def test_sigmoid_attention_value_sizes(ops, dk, dv, vdim):
+    H, G, n, B = 6, 2, 150, 3
+    pages = 3
+    k = (torch.randn(B * pages, G, 64 * dk, device=DEV) * 0.5).bfloat16()
+    v = torch.randn(B * pages, G, 64 * ((vdim + 31) // 32 * 32), device=DEV).bfloat16()
+    table = torch.arange(B * pages, device=DEV, dtype=torch.int32).view(B, pages).contiguous()
+    slot = torch.arange(B, device=DEV, dtype=torch.int32)
+    wide = max(k.stride(0), v.stride(0))                           # pages of keys and of values have one stride
+    k, v = (torch.nn.functional.pad(p.view(B * pages, -1), (0, wide - p.stride(0))).contiguous() for p in (k, v))
+    kv = (k, v, k.stride(0), table)
+    q = torch.randn(B, H, dk, device=DEV).bfloat16()
+    ctx = torch.tensor([n, 64, 1], device=DEV, dtype=torch.int32)
+    want = ops.sigmoid_attention(q, kv, ctx - 1, slot, None, H, G, dk, dv, vdim, dk ** -0.5).float()
+    for splits in (1, 3):
+        got = ops.sigmoid_attention_decode(q, kv, slot, ctx, B, None, H, G, dk, dv, vdim, dk ** -0.5, None, splits).float()
+        # weights as two 16-bit numbers and in float32: 2^-16 of the up to 150 addends' absolute sum, some 120; then both round to 8
+        # bits, where sums that differ by a hair may become neighbours, up to 2^-7 of their size apart
+        assert got.shape == want.shape and ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -9).all(), splits
