@@ -559,13 +559,33 @@ __global__ __launch_bounds__(64) void head_linear_few_kernel(const TI* __restric
         }
     }
     if (!t_ok) return;
+    T* orow = out + (int64_t)col * out_st + (int64_t)h * out_sh;
+    const float* grow = gate ? gate + (int64_t)col * gate_st + (int64_t)h * n_out : nullptr;
+    // four outputs lie together: where the rows allow it, four stores (and gates) a lane instead of sixteen (a latent attention model's step of 8
+    // sequences, six such products: 0.5%)
+    if (n_out % 4 == 0 && (((uintptr_t)out | (out_st * sizeof(T)) | ((int64_t)out_sh * sizeof(T))) & (4 * sizeof(T) - 1)) == 0 &&
+        (!gate || (((uintptr_t)gate | (gate_st * 4)) & 15) == 0)) {
+#pragma unroll
+        for (int r = 0; r < 16; r += 4) {
+            const int j = j0 + 2 * r + 4 * half;
+            if (j >= n_out) continue;
+            f32x4 v = {acc[r], acc[r + 1], acc[r + 2], acc[r + 3]};
+            if (gate) {
+                const f32x4 z = *(const f32x4*)(grow + j);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] *= lt_sigmoid(z[e]);
+            }
+            *(typename Vec<T>::v4*)(orow + j) = typename Vec<T>::v4{from_f32<T>(v[0]), from_f32<T>(v[1]), from_f32<T>(v[2]), from_f32<T>(v[3])};
+        }
+        return;
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         const int j = j0 + 8 * (r >> 2) + 4 * half + (r & 3);
         if (j < n_out) {
             float v = acc[r];
-            if (gate) v *= lt_sigmoid(gate[(int64_t)col * gate_st + (int64_t)h * n_out + j]);
-            out[(int64_t)col * out_st + (int64_t)h * out_sh + j] = from_f32<T>(v);
+            if (gate) v *= lt_sigmoid(grow[j]);
+            orow[j] = from_f32<T>(v);
         }
     }
 }

@@ -237,3 +237,22 @@ def test_sigmoid_attention_value_sizes(ops, dk, dv, vdim):
         # weights as two 16-bit numbers and in float32: 2^-16 of the up to 150 addends' absolute sum, some 120; then both round to 8
         # bits, where sums that differ by a hair may become neighbours, up to 2^-7 of their size apart
         assert got.shape == want.shape and ((got - want).abs() <= 2.0 ** -7 * want.abs() + 2.0 ** -9).all(), splits
+
+
+# outputs of a head in whole fours and not, rows and heads that begin at fours and not, with and without a gate
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("n_in,n_out,col,pad", [(64, 64, 0, 0), (64, 64, 2, 0), (128, 36, 0, 4), (40, 100, 4, 3), (96, 33, 0, 0), (8, 6, 0, 2)])
+def test_products_per_head_of_few_tokens(ops, dtype, n_in, n_out, col, pad):
+    H, t = 3, 5
+    w, x = (torch.randn(H, n_out, n_in, device=DEV) * n_in ** -0.5).to(dtype), torch.randn(t, H * n_in, device=DEV).to(dtype)
+    want = torch.einsum("hji,thi->thj", w.double().cpu(), x.double().cpu().view(t, H, n_in))
+    for gate_col in (None, 0, 1):
+        out = torch.full((t, col + H * (n_out + pad) + 1), 7.0, device=DEV, dtype=dtype)
+        gate = torch.randn(t, H * n_out + 5, device=DEV)
+        kw = {} if gate_col is None else {"gate": gate, "gate_col": gate_col}
+        ops.head_linear(x, 0, n_in, w, out, col, n_out + pad, **kw)
+        ref = want if gate_col is None else want * torch.sigmoid(gate.double().cpu())[:, gate_col:gate_col + H * n_out].view(t, H, n_out)
+        got = out[:, col:col + H * (n_out + pad)].reshape(t, H, n_out + pad).double().cpu()
+        eps = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+        assert ((got[:, :, :n_out] - ref).abs() <= eps * ref.abs() + 2.0 ** -16).all()       # one rounding, and float32 sums
+        assert (got[:, :, n_out:] == 7.0).all() and (out[:, :col] == 7.0).all() and (out[:, -1] == 7.0).all()
