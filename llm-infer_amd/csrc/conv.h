@@ -20,8 +20,11 @@ struct ConvWindow {
     float u[TAPS];
     __device__ __forceinline__ void start(const float* at, int64_t stride, int inside, int p, const float* hist, int channels, int c) {
 #pragma unroll
-        for (int b = 0; b < TAPS; ++b)
-            u[b] = b <= inside ? at[-b * stride] : (p - b >= 0 ? hist[(int64_t)(TAPS - 1 - (b - inside)) * channels + c] : 0.f);
+        for (int b = 0; b < TAPS; ++b) {         // (an address by choice, not a load: a branch each would be waited for one by one)
+            const float* from = b <= inside ? at - b * stride : hist + (int64_t)(TAPS - 1 - (b - inside)) * channels + c;
+            const float v = *from;
+            u[b] = b <= inside || p - b >= 0 ? v : 0.f;
+        }
     }
     __device__ __forceinline__ void next(float v) {        // the next token of the same sequence
 #pragma unroll
