@@ -56,9 +56,9 @@ template <class V> __device__ __forceinline__ V load_once(const void* p) {
 
 // Values of other lanes by the vector unit alone: swaps of half waves and of rows of 16 lanes, moves within a row.  (__shfl is a
 // round trip through the LDS unit, some 50 ns each in a chain that nothing runs beside: a wave's sum is six of them.  The same lanes
-// are added in the same order, a + b for b + a, so the bits are the same; but a product that is summed is rounded first, where the
-// compiler made the first addition one multiply-add.  Requests: Dopivik, batch 1, 6.89 -> 6.77 ms, Manirax 14.2 -> 14.05, 8B chat 75.8
-// -> 75.5; batches of 4 and more the same.)  Every lane of the wave must be active.
+// are added in the same order, a + b for b + a, so the bits are the same; where a product is summed, wave_sum_product keeps the
+// multiply-add that the compiler makes of a product and a __shfl.  Requests: Dopivik, batch 1, 6.89 -> 6.77 ms, Manirax 14.2 -> 14.05, 8B
+// chat 75.8 -> 75.5; batches of 4 and more the same.)  Every lane of the wave must be active.
 template <int CTRL> __device__ __forceinline__ float row_move(float v) {           // a move within every row of 16 lanes
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
@@ -79,12 +79,19 @@ __device__ __forceinline__ float sum_quarters(float v) { const LanePair p = quar
 __device__ __forceinline__ float max_halves(float v) { const LanePair p = halves(v); return fmaxf(p.lo, p.hi); }
 __device__ __forceinline__ float max_quarters(float v) { const LanePair p = quarters(v); return fmaxf(p.lo, p.hi); }
 
-__device__ __forceinline__ float wave_sum(float v) {
-    v = sum_quarters(sum_halves(v));
+__device__ __forceinline__ float half_sum(float v) {   // over the lanes of this lane's half wave
+    v = sum_quarters(v);
     v += row_move<ROW_ROR(8)>(v);
     v += row_move<ROW_ROR(4)>(v);                      // (a row repeats every 8 lanes by now: 4 back is 4 on)
     v += row_move<QUAD_SWAP2>(v);
     return v + row_move<QUAD_SWAP1>(v);
+}
+__device__ __forceinline__ float wave_sum(float v) { return half_sum(sum_halves(v)); }
+// wave_sum of a * b with the first addition and the lane's own product one multiply-add: a rounding less.  (The other half's
+// product is rounded, so the two halves' results may differ in their last bit.)
+__device__ __forceinline__ float wave_sum_product(float a, float b) {
+    const LanePair p = halves(a * b);
+    return half_sum(fmaf(a, b, (threadIdx.x & 32) ? p.lo : p.hi));
 }
 __device__ __forceinline__ float wave_max(float v) {
     v = max_quarters(max_halves(v));
@@ -119,8 +126,7 @@ template <class F> __device__ __forceinline__ void wave_choice(float& v, int& i,
 
 // Sum over a block of up to 1024 threads; `scratch` holds 16 floats of LDS.  (All sixteen are read at once, the waves' added in
 // their order: a loop over as many as there are waits for one after the other.)
-__device__ __forceinline__ float block_sum(float v, float* scratch) {
-    v = wave_sum(v);
+__device__ __forceinline__ float sum_of_waves(float v, float* scratch) {       // v: a wave's number, in its lane 0
     const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     __syncthreads();
     if ((threadIdx.x & 63) == 0) scratch[w] = v;
@@ -132,6 +138,7 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
     for (int i = 0; i < 16; ++i) t = i < nw ? t + s[i] : t;
     return t;
 }
+__device__ __forceinline__ float block_sum(float v, float* scratch) { return sum_of_waves(wave_sum(v), scratch); }
 __device__ __forceinline__ float block_max(float v, float* scratch) {
     v = wave_max(v);
     const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;

@@ -411,7 +411,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void diff_attn_merge_kernel(const fl
         const float s2 = sink ? sink[h] * 1.4426950408889634f : -INFINITY;
         const float M = fmaxf(wave_max(ms), s2);
         const float fs = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - M);
-        const float L = wave_sum(ls * fs) + (sink ? __builtin_amdgcn_exp2f(s2 - M) : 0.f);
+        const float L = wave_sum_product(ls, fs) + (sink ? __builtin_amdgcn_exp2f(s2 - M) : 0.f);
         float O = 0.f;
         for (int s0 = 0; s0 < S; s0 += 16) {
             float t[16];
@@ -426,7 +426,7 @@ __global__ __launch_bounds__(MERGE_THREADS) void diff_attn_merge_kernel(const fl
     if (MAPS == 2) x -= lambda * val[MAPS - 1];
     if (i >= dv) x = 0.f;
     float rr = out_scale;
-    if (out_eps >= 0.f) rr = out_scale / sqrtf(block_sum(x * x, scratch) / (float)dv + out_eps);
+    if (out_eps >= 0.f) rr = out_scale / sqrtf(sum_of_waves(wave_sum_product(x, x), scratch) / (float)dv + out_eps);
     const float* grow = gate ? gate + (unit / H) * gate_stride + gate_col : nullptr;
     if (gate && !gate_elem) rr *= 1.f / (1.f + expf(-grow[h]));
     if (i < dv) out[unit * dv + i] = from_f32<T>(x * rr * (gate_elem ? 1.f / (1.f + expf(-grow[h * dv + i])) : 1.f));

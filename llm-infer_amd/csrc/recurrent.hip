@@ -155,7 +155,9 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(DeltaPrep p) {
                 sq += q[v] * q[v];
                 sk += k[v] * k[v];
             }
-            const float rq = qs / sqrtf(wave_sum(sq) + DELTA_UNIT_EPS), rk = 1.f / sqrtf(wave_sum(sk) + DELTA_UNIT_EPS);
+            if constexpr (NV == 1) { sq = wave_sum_product(q[0], q[0]); sk = wave_sum_product(k[0], k[0]); }
+            else { sq = wave_sum(sq); sk = wave_sum(sk); }
+            const float rq = qs / sqrtf(sq + DELTA_UNIT_EPS), rk = 1.f / sqrtf(sk + DELTA_UNIT_EPS);
             if (HALF) {
                 bf16* out = (bf16*)p.rows + (int64_t)t * channels;
 #pragma unroll
@@ -565,7 +567,7 @@ __global__ __launch_bounds__(64 * SCAN_WAVES * CB) void wkv_scan_kernel(const fl
             w = expf(-expf(raw[(int64_t)(q0 + t) * H * d + h * d + tid]));
         }
         if (tid < DP) { sr[t % 3][tid] = rr; sk[t % 3][tid] = kk; sw[t % 3][tid] = w; }
-        const float b = wave_sum(rr * ub * kk);
+        const float b = wave_sum_product(rr * ub, kk);
         if (lane == 0) ruk[t % 3][tid >> 6] = b;
     };
     stage(0);

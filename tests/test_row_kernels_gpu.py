@@ -216,6 +216,19 @@ def test_recurrences_with_whole_and_ragged_states(ops, rows, cols):
         assert near(wkv[slot], W, W.abs())
 
 
+# the first addition of a wave's sum takes its product unrounded: (1 + 2^-12)^2 in lane 0 and its rounding, with the other sign, half a wave
+# on leave 2^-24
+@pytest.mark.parametrize("d", [64, 128])
+def test_a_bonus_enters_its_sum_unrounded(ops, d):
+    from types import SimpleNamespace
+    ctx = SimpleNamespace(seq_slot=torch.zeros(1, dtype=torch.int32, device=DEV), n_seqs=1, n_tokens=1)
+    r, k, bonus, v = torch.zeros(1, d, device=DEV), torch.zeros(1, d, device=DEV), torch.ones(1, d, device=DEV), torch.ones(1, d, device=DEV)
+    r[0, 0] = k[0, 0] = 1 + 2.0 ** -12
+    r[0, 32], k[0, 32] = -(1 + 2.0 ** -11), 1.0
+    o = ops.wkv_scan(r, k, v, torch.zeros_like(r), bonus, torch.zeros(1, 1, d, d, device=DEV), ctx, 1, d)
+    assert torch.equal(o, torch.full_like(o, 2.0 ** -24))
+
+
 # value sizes in whole fours (four dimensions a store) and not, one split and several, against the kernel that takes a key after
 # the other
 @pytest.mark.parametrize("dk,dv,vdim", [(16, 32, 32), (16, 30, 32), (64, 64, 64), (64, 49, 64), (64, 60, 64)])
