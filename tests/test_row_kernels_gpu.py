@@ -1,4 +1,5 @@
 """The kernels of a decode step that have a row or a few to work on, at the edges of what a thread and a workgroup take."""
+import numpy as np
 import pytest
 import torch
 
@@ -109,6 +110,24 @@ def test_layer_norms_of_sums(ops, width, mean):
         want = _ln(2 * xd + sum(s * t.double() for t, s in adds), 1e-5) * w.double()
         _close(out, want)
         assert torch.equal(copy, out.to(torch.bfloat16))
+
+
+# whole numbers whose mean is 0 and whose squares add up to less than 2^24: every sum is exact in float32 in any order, if the mean is taken
+# before the deviations, and then only roots, divisions and products round, once each (numpy's are correctly rounded, as the kernels' are)
+@pytest.mark.parametrize("width", WIDTHS + [37])
+def test_a_layer_norms_deviations_are_from_the_rows_mean(ops, width):
+    v = np.random.default_rng(width).integers(-8, 9, (9, width)).astype(np.float32)
+    v[:, -1] -= v.sum(1)
+    v += np.sign(v[:, :1] + 0.5) * (np.arange(width) == 0) - np.sign(v[:, :1] + 0.5) * (np.arange(width) == width - 1)
+    dev, one = (v * v).sum(1, keepdims=True), torch.ones(width, device=DEV)
+    assert v.dtype == np.float32 and (v.sum(1) == 0).all() and dev.max() < 2 ** 24 and dev.min() > 0
+    rows = torch.from_numpy(v).to(DEV)
+    out = rows.clone()
+    ops.add_layernorm(out, 1.0, [(torch.zeros_like(out), 1.0)], one, 0.0)
+    assert np.array_equal(out.cpu().numpy(), v / np.sqrt(dev / np.float32(width)))
+    out = torch.zeros(9, width, device=DEV)
+    ops.layernorm_add(out, rows, one, torch.zeros(width, device=DEV), 0.0)
+    assert np.array_equal(out.cpu().numpy(), v * (np.float32(1) / np.sqrt(dev * (np.float32(1) / np.float32(width)))))
 
 
 @pytest.mark.parametrize("n", WIDTHS + [37, 14336, 16384, 16388])
