@@ -287,7 +287,10 @@ extern "C" int li_router(const void* X, const void* Wt, int dt, const float* bia
 // ---------------------------------------------------------------------------
 // An expert's product on its own pairs' rows, few of them: C[pair] = epilogue(W_e X[row_of[pair]]) for the pairs of
 // the blockIdx.y-th expert that has any (row_of null: X[pair]).  gemv_tiled's structure: a workgroup takes 16 rows of W_e
-// for the whole of K, its KW waves share K; 16 MT pairs at a time (W is read again, from the caches, for the next ones).
+// for the whole of K, its KW waves share K; 16 MT pairs at a time (W is read again, from the caches, for the next ones; only the
+// last time past them).  us, 16 experts, up 7,168 x 4,096, all reads of W past the caches, none, and so: 8 pairs each 157, 163, 157; a
+// quarter of the experts with 32 each 106, 94, 90; one with 64, 8 in the mean 181, 177, 168; 64 experts of 1,536 x 2,048, 10 each 98, 100,
+// 98, a quarter with 32 each 53, 46, 46.
 // ---------------------------------------------------------------------------
 template <class T, int MT, int KW>
 __global__ __launch_bounds__(64 * KW) void experts_gemv_kernel(const T* __restrict__ X, const T* __restrict__ Wt, int K,
@@ -327,21 +330,25 @@ __global__ __launch_bounds__(64 * KW) void experts_gemv_kernel(const T* __restri
             xrow[j] = X + (int64_t)(row_of ? row_of[pair] : pair) * K + 8 * g;
             acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
-        for (int s0 = s_begin; s0 < s_end; s0 += U) {
-            v8 a[U], b[U][MT];
+        auto product = [&](auto last) {
+            for (int s0 = s_begin; s0 < s_end; s0 += U) {
+                v8 a[U], b[U][MT];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const bool in = s0 + u < s_end;
-                const v8 z = {};
-                a[u] = in ? load_once<v8>(wt + (int64_t)(s0 + u) * 512) : z;
+                for (int u = 0; u < U; ++u) {
+                    const bool in = s0 + u < s_end;
+                    const v8 z = {};
+                    const T* from = wt + (int64_t)(s0 + u) * 512;
+                    a[u] = !in ? z : decltype(last)::value ? load_once<v8>(from) : *(const v8*)from;
 #pragma unroll
-                for (int j = 0; j < MT; ++j) b[u][j] = in && have[j] ? *(const v8*)(xrow[j] + (s0 + u) * 32) : z;
+                    for (int j = 0; j < MT; ++j) b[u][j] = in && have[j] ? *(const v8*)(xrow[j] + (s0 + u) * 32) : z;
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) acc[j] = mfma16(a[u], b[u][j], acc[j]);
             }
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int j = 0; j < MT; ++j) acc[j] = mfma16(a[u], b[u][j], acc[j]);
-        }
+        };
+        if (r0 + 16 * MT >= count) product(std::true_type{}); else product(std::false_type{});
         if (r0) __syncthreads();                           // wave 0 has read the sums of the pairs before
 #pragma unroll
         for (int j = 0; j < MT; ++j)
