@@ -334,6 +334,7 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wn = wave;
     int bx, by, bz, m0;
+    [[maybe_unused]] bool one_tile = false;             // all rows of X that meet this W are this tile's
     if constexpr (by_pairs(MODE)) {
         int all = 0;
         for (int e0 = 0; e0 < pt.n_experts; e0 += 64) {
@@ -366,6 +367,7 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
         const int first = __builtin_amdgcn_readfirstlane(pt.offsets[expert]);
         m0 = first + row0;
         e.M = first + rows;
+        one_tile = rows <= BM;
         Wt += expert * pt.w_stride;
     } else {
         tile_of_workgroup(8, bx, by, bz, gridDim.x);
@@ -420,15 +422,6 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
             (const __attribute__((address_space(1))) void*)(xbase + at + (xoff[i] - back)),
             (__attribute__((address_space(3))) void*)(smem_raw + buf_off + q * 1024), 16, 0, 0);
     };
-    // The loads of W are written as instructions so that the compiler does not place waits for them (at
-    // the loop's head it would wait for every load in flight); the waits are placed by hand below.
-    auto fetch_one = [&](int i, int half, v8 (&a)[NI]) {          // block i of the fragments of a half step
-        const T* from = wsrc[i] + (int64_t)min(half, last) * 512;
-        // (a tile with W three or four steps ahead holds all rows of X: W is read once, as by load_once)
-        if constexpr (A >= 3) asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
-        else asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[i]) : "v"(lane * 16), "s"(from) : "memory");
-    };
-
     f32x4 acc[NI][MJ];
 #pragma unroll
     for (int i = 0; i < NI; ++i)
@@ -446,7 +439,6 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     // by seven others before b[j] is used, and LDS reads complete in order, so "at most 7 in flight" is the
     // wait before every group of matrix instructions.  (Left to the compiler, each half begins with a wait
     // for all eight, the last of which has only just been issued.)
-    v8 b[MJ];
     // where lane (r = lane % 16, g = lane / 16) finds row r, chunk 4 h + g (half h) of fragment 0: unit
     // r / 8, place 8 (r % 8) + ((4 h + g) ^ r % 8); fragment j lies 2 KiB on
     const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)smem_raw +
@@ -479,7 +471,26 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     // s + A - 1 (whose slot the step before has used up), in its second half those of W's first half of step s + A.  Step s
     // needs X of step s + 1 (its second half reads ahead into it) and its own W: everything up to the first half of step
     // s + 1 - A, i.e. all but the NI loads of that step's second half and the A - 2 whole steps issued since.
-    v8 ring[SLOTS][NI];
+    // RowScale (MODE -1, at most 16 rows of X, K whole; the host sees to it): the partial sums of squares of row
+    // tid % 16 are dealt to the 16 groups of 16 threads; they are fetched behind the first loads, and everything is
+    // waited for once (the loop's counts are upper bounds and stay right with fewer loads in flight).  The groups'
+    // sums lie behind the stages of X, where the epilogue finds them.
+    constexpr int STRIPS_BYTES = 4 * 2 * 16 * (16 * NI + 4) * 4;
+    constexpr int INFO = XBUFS * STAGE > STRIPS_BYTES ? XBUFS * STAGE : STRIPS_BYTES;     // behind the stages and the strips
+    float* row_ss = (float*)(smem_raw + INFO + 2 * BM * 4);                               // [16 groups][16 rows], then [16] factors
+    bool scaled = false;
+    // ONCE: nothing else reads this workgroup's rows of W, which pass the caches as by load_once
+    auto products = [&](auto once) {
+    constexpr bool ONCE = decltype(once)::value;
+    // The loads of W are written as instructions so that the compiler does not place waits for them (at
+    // the loop's head it would wait for every load in flight); the waits are placed by hand below.
+    auto fetch_one = [&](int i, int half, v8 (&a)[NI]) {          // block i of the fragments of a half step
+        const T* from = wsrc[i] + (int64_t)min(half, last) * 512;
+        const int at = lane * 16;
+        if constexpr (ONCE) asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[i]) : "v"(at), "s"(from) : "memory");
+        else asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[i]) : "v"(at), "s"(from) : "memory");
+    };
+    v8 ring[SLOTS][NI], b[MJ];
     constexpr int PER_STEP = PER_WAVE + 2 * NI, AHEAD = NI + (A - 2) * PER_STEP, FIRST = (A - 1) * PER_STEP - NI;
     static_assert(FIRST <= 63 && AHEAD <= 63, "the waits' counts");
 #pragma unroll
@@ -493,14 +504,6 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
             for (int i = 0; i < NI; ++i) fetch_one(i, 2 * a + 1, ring[2 * a + 1]);
         }
     }
-    // RowScale (MODE -1, at most 16 rows of X, K whole; the host sees to it): the partial sums of squares of row
-    // tid % 16 are dealt to the 16 groups of 16 threads; they are fetched behind the first loads, and everything is
-    // waited for once (the loop's counts are upper bounds and stay right with fewer loads in flight).  The groups'
-    // sums lie behind the stages of X, where the epilogue finds them.
-    constexpr int STRIPS_BYTES = 4 * 2 * 16 * (16 * NI + 4) * 4;
-    constexpr int INFO = XBUFS * STAGE > STRIPS_BYTES ? XBUFS * STAGE : STRIPS_BYTES;     // behind the stages and the strips
-    float* row_ss = (float*)(smem_raw + INFO + 2 * BM * 4);                               // [16 groups][16 rows], then [16] factors
-    bool scaled = false;
     if constexpr (MODE == -1) {
         scaled = rsc.ss != nullptr;
         if (scaled) {
@@ -570,6 +573,16 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
 #pragma unroll
     for (int j = 0; j < MJ; ++j) asm volatile("" ::"v"(b[j]));
     __builtin_amdgcn_sched_barrier(0);
+    };
+    // A tile with W three or four steps ahead holds all rows of X, so W is read once; in pairs mode it does where an expert's pairs fit one
+    // tile, while the matrix of an expert of more is read by every tile of it.  us, ordinary loads, all past the caches, and so: 16
+    // experts, up 7,168 x 4,096, 32 pairs each 178, 164, 164, half of them with 80 each 114, 169, 114, one with 200 and 32 in the mean 187, 186,
+    // 172; 64 experts of 1,536 x 2,048, 32 each 74, 69, 69, half with 80 53, 68, 52
+    if constexpr (by_pairs(MODE) && A >= 3) {
+        if (one_tile) products(std::true_type{});
+        else products(std::false_type{});
+    } else
+        products(std::bool_constant<(A >= 3)>{});
 
     // Epilogue through LDS, a strip of 16 rows of X x 16 NI rows of W at a time: accumulator q of a 16x16
     // block is W row 4 (lane / 16) + q, X row lane % 16; read back, consecutive lanes hold consecutive
