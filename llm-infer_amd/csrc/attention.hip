@@ -56,7 +56,8 @@ struct AttnExtras {
     float softcap;
 };
 
-template <class T>
+// ONCE: a page is read by this workgroup alone (load_once)
+template <class T, bool ONCE = true>
 struct WaveAttn {
     typedef typename Vec<T>::v8 v8;
     static constexpr int ROWS = 32, KF = 2 * KS, VF = DB * 4;
@@ -85,12 +86,12 @@ struct WaveAttn {
     __device__ __forceinline__ void load_k(const T* kpage, v8 (&kf)[2 * KS]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < 2 * KS; ++i) kf[i] = load_once<v8>(kpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < 2 * KS; ++i) kf[i] = ONCE ? load_once<v8>(kpage + (i * 64 + lane) * 8) : *(const v8*)(kpage + (i * 64 + lane) * 8);
     }
     __device__ __forceinline__ void load_v(const T* vpage, v8 (&vf)[DB * 4]) const {
         const int lane = threadIdx.x & 63;
 #pragma unroll
-        for (int i = 0; i < DB * 4; ++i) vf[i] = load_once<v8>(vpage + (i * 64 + lane) * 8);
+        for (int i = 0; i < DB * 4; ++i) vf[i] = ONCE ? load_once<v8>(vpage + (i * 64 + lane) * 8) : *(const v8*)(vpage + (i * 64 + lane) * 8);
     }
 
     // Scores of the page's keys (starting at key t0) against this wave's rows, mask, running
@@ -1148,9 +1149,14 @@ static int launch_decode(const void* q, void* out, float* part_o, float* part_ml
     const int rows = few ? 16 : 32;
     dim3 grid(n_seqs, K * ((G + rows - 1) / rows), parts), block(64 * W);
     const size_t lds = (size_t)W * (G < rows ? G : rows) * (HD + 4 + 2) * sizeof(float);
+    // A KV head of more than 32 query heads has a workgroup for every 32, which all read its pages: those stay in the caches.  us past
+    // them and so, one KV head: 96 heads of 128, batch 128 at 2,000 59.6 and 41.8, 128, batch 256 at 4,096 241 and 179, 64, batch 32 at
+    // 2,000 22.7 and 20.0, batch 1 at 4,000 10.7 and 10.8, batch 4 at 500 9.0 and 9.5; 128 heads of 96, batch 64 at 4,000 38.9 and 36.9;
+    // 128 of 64, batch 256 at 4,096 149 and 113, 64 of 64, batch 128 at 2,000 19.5 and 20.5; 64 of 256, batch 1 at 4,000 49.6 and 37.9
     auto kfn = attn_decode_kernel<T, W, WaveAttn<T>, true>;
     if constexpr (HD % 32 == 0) if (few) kfn = attn_decode_kernel<T, W, WaveAttn16<T>, true>;
-    if constexpr (HD <= 128) if (by_32) kfn = attn_decode_kernel<T, W, WaveAttn<T>, false>;
+    if (G > 32) kfn = attn_decode_kernel<T, W, WaveAttn<T, false>, true>;
+    if constexpr (HD <= 128) if (by_32) kfn = G > 32 ? attn_decode_kernel<T, W, WaveAttn<T, false>, false> : attn_decode_kernel<T, W, WaveAttn<T>, false>;
     if (lds > 48 * 1024 &&
         hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
         return LI_HIP_ERROR;

@@ -251,8 +251,9 @@ def test_a_bonus_enters_its_sum_unrounded(ops, d):
 # value sizes in whole fours (four dimensions a store) and not, one split and several, against the kernel that takes a key after
 # the other
 @pytest.mark.parametrize("dk,dv,vdim", [(16, 32, 32), (16, 30, 32), (64, 64, 64), (64, 49, 64), (64, 60, 64)])
-def test_sigmoid_attention_value_sizes(ops, dk, dv, vdim):
-    H, G, n, B = 6, 2, 150, 3
+@pytest.mark.parametrize("H", [6, 66])                 # query heads of a KV head for one workgroup and for two
+def test_sigmoid_attention_value_sizes(ops, dk, dv, vdim, H):
+    G, n, B = 2, 150, 3
     pages = 3
     k = (torch.randn(B * pages, G, 64 * dk, device=DEV) * 0.5).bfloat16()
     v = torch.randn(B * pages, G, 64 * ((vdim + 31) // 32 * 32), device=DEV).bfloat16()
