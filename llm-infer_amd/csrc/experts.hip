@@ -129,7 +129,11 @@ extern "C" int li_sort_pairs(const int* chosen, int n, int top, int n_experts, i
 // more tiles than that.  Each is a workgroup of its own: one workgroup of them all is bound by what a CU takes in (W and X,
 // 0.2 to 0.5 MB for 16 x 4,096).  us in a recorded chain, one launch with a workgroup for 16 tokens and these two, 8 tokens:
 // 16 x 4,096 in one part 8.4 -> 5.8, in three 15.3 -> 6.5, 64 x 4,096 18.3 -> 8.6 and 42.8 -> 13.2, 8 x 2,048 6.7 -> 5.2 and 9.6 -> 5.8;
-// 600 tokens x 16 x 4,096 13.4 -> 10.7 and 22.5 -> 12.5, 4,096 tokens 19.1 -> 20.7 and 27.9 -> 29.0 (every CU had its workgroup).
+// 600 tokens x 16 x 4,096 13.4 -> 10.7 and 22.5 -> 12.5.  Where nearly every CU has a workgroup of 16 tokens anyway, one launch
+// does it all after all (router_one_kernel; the same values): us in one launch and in two, with the sort, in one part and in three, 4,096
+// tokens x 16 x 4,096 19.5, 21.0 and 28.3, 29.7, x 64 x 4,096 46.5, 48.9 and 81.1, 83.5, x 8 x 2,048 17.0, 18.6 and 21.7, 22.3, x 256 x 4,096 109, 111
+// and 248, 250; 3,584 18.5, 19.4 and 27.6, 28.0, 44.1, 45.7 and 79.3, 80.9, x 512 x 2,048 119, 111 and 257, 232; 3,328 18.7, 19.1 and 27.3, 26.9;
+// 4,112 28.7, 22.7 and 46.6, 31.5; 8,192 35.7, 33.9 and 52.6, 49.2, 88.6, 90.2 and 158, 160.
 // ---------------------------------------------------------------------------
 #define ROUTER_WAVES 16
 #define ROUTER_MAX 512
@@ -176,9 +180,107 @@ __global__ __launch_bounds__(64) void router_sums_kernel(const T* __restrict__ X
     *(f32x4*)(sums + (((int64_t)blockIdx.x * gridDim.y + blockIdx.y) * 64 + lane) * 4) = acc;
 }
 
-// The choice, a wave a token: its logits are the shares' sums in ascending order; the `top` largest (the first of equals), their
-// weights the softmax over them alone times `scale`.  chosen and weights [T, top], experts ascending.  With one workgroup (up
-// to 16 tokens) it also sorts the pairs.
+// The choice for a wave's token t, whose logits zs its lanes hold (output c * 64 + lane in zs[c], -infinity beyond n): the `top` largest (the
+// first of equals), their weights the softmax over them alone times `scale`.  chosen and weights [T, top], experts ascending; `picked`
+// (may be null) receives the chosen experts too, from token t0 on.
+template <int NC>
+__device__ __forceinline__ void choose(const float (&zs)[NC], int t, int t0, int n, int top, float scale, int* __restrict__ chosen,
+                                       float* __restrict__ weights, int* picked) {
+    const int lane = threadIdx.x & 63;
+    float mx = 0.f, sum = 0.f;
+    uint32_t taken = 0;                                // bit c: this lane's output c * 64 + lane is chosen
+    for (int k = 0; k < top; ++k) {
+        float best = -INFINITY; int bi = 0x7fffffff;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int i = c * 64 + lane;
+            if (i < n && !(taken >> c & 1) && (zs[c] > best || bi == 0x7fffffff)) { best = zs[c]; bi = i; }
+        }
+        wave_choice(best, bi, [&](float ob, int oi) {
+            if (oi != 0x7fffffff && (bi == 0x7fffffff || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
+        });
+        bi = __builtin_amdgcn_readfirstlane(bi);       // (one choice for the wave, also where logits are no numbers)
+        best = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(best)));
+        if (k == 0) mx = best;
+        sum += expf(best - mx);
+        if ((bi & 63) == lane) taken |= 1u << (bi >> 6);
+    }
+    int rank = 0;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) {
+        const bool mine = taken >> c & 1;
+        const uint64_t mask = __builtin_amdgcn_ballot_w64(mine);
+        if (mine) {
+            const int64_t at = (int64_t)t * top + rank + __builtin_popcountll(mask & ((1ull << lane) - 1));
+            chosen[at] = c * 64 + lane;
+            if (picked) picked[at - (int64_t)t0 * top] = c * 64 + lane;
+            weights[at] = expf(zs[c] - mx) / sum * scale;
+        }
+        rank += __builtin_popcountll(mask);
+    }
+}
+
+// Everything in one launch, 16 tokens a workgroup: the waves share W's tiles, and K where there are fewer tiles than waves, as above.
+template <class T, int NC>
+__global__ __launch_bounds__(64 * ROUTER_WAVES) void router_one_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
+                                                                       const float* __restrict__ bias, int parts, int n_tokens, int K,
+                                                                       int n, int top, float scale, int* __restrict__ chosen,
+                                                                       float* __restrict__ weights) {
+    typedef typename Vec<T>::v8 v8;
+    constexpr int U = 8;
+    extern __shared__ float z[];                           // [16][n]
+    __shared__ float part[ROUTER_WAVES][64][4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int t0 = blockIdx.x * 16, steps = K >> 5, tiles = (n + 15) >> 4;
+    const int kw = router_share(tiles), at_once = ROUTER_WAVES / kw;              // tiles that are worked on at a time
+    const int share = wave % kw, per = (steps + kw - 1) / kw, s_begin = share * per, s_end = min(steps, s_begin + per);
+    const bool have = t0 + r < n_tokens;
+    const T* xrow = X + (int64_t)(have ? t0 + r : t0) * K + 8 * g;
+    for (int first = 0; first < tiles; first += at_once) {
+        const int tile = first + wave / kw;
+        const bool on = wave / kw < at_once && tile < tiles;
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        if (on) {
+            for (int pt = 0; pt < parts; ++pt) {
+                const T* wt = Wt + ((int64_t)(pt * tiles + tile) * steps * 64 + lane) * 8;
+                for (int s0 = s_begin; s0 < s_end; s0 += U) {
+                    v8 a[U], b[U];
+#pragma unroll
+                    for (int u = 0; u < U; ++u) {
+                        const v8 zero = {};
+                        const bool in = s0 + u < s_end;
+                        a[u] = in ? *(const v8*)(wt + (int64_t)(s0 + u) * 512) : zero;
+                        b[u] = in && have ? *(const v8*)(xrow + (s0 + u) * 32) : zero;
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; ++u) acc = mfma16(a[u], b[u], acc);
+                }
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) part[wave][lane][q] = acc[q];
+        __syncthreads();
+        if (on && share == 0) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float v = part[wave][lane][q];
+                for (int k = 1; k < kw; ++k) v += part[wave + k][lane][q];
+                const int j = tile * 16 + 4 * g + q;
+                if (j < n) z[r * n + j] = v + (bias ? bias[j] : 0.f);
+            }
+        }
+        __syncthreads();
+    }
+    const int t = t0 + wave;
+    if (t >= n_tokens) return;                             // (a wave's token, the same for all its lanes)
+    float zs[NC];
+#pragma unroll
+    for (int c = 0; c < NC; ++c) zs[c] = c * 64 + lane < n ? z[wave * n + c * 64 + lane] : -INFINITY;
+    choose<NC>(zs, t, t0, n, top, scale, chosen, weights, nullptr);
+}
+
+// The second launch, a wave a token: its logits are the shares' sums in ascending order.  With one workgroup (up to 16 tokens) it
+// also sorts the pairs.
 // NC: outputs in groups of 64 that a wave holds, ceil(n / 64) rounded up to 1 or 8.
 template <int NC>
 __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const float* __restrict__ sums, const float* __restrict__ bias,
@@ -190,7 +292,6 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const float* 
     const int t0 = blockIdx.x * 16, tiles = (n + 15) >> 4;
     const int t = t0 + wave;
     if (t < n_tokens) {                                    // (a wave's token, the same for all its lanes)
-        float mx = 0.f, sum = 0.f;
         float zs[NC];
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -205,36 +306,7 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const float* 
             for (int k = 1; k < SHARES; ++k) z = k < kw ? z + v[k] : z;
             zs[c] = c * 64 + lane < n ? z + own : -INFINITY;
         }
-        uint32_t taken = 0;                                // bit c: this lane's output c * 64 + lane is chosen
-        for (int k = 0; k < top; ++k) {
-            float best = -INFINITY; int bi = 0x7fffffff;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const int i = c * 64 + lane;
-                if (i < n && !(taken >> c & 1) && (zs[c] > best || bi == 0x7fffffff)) { best = zs[c]; bi = i; }
-            }
-            wave_choice(best, bi, [&](float ob, int oi) {
-                if (oi != 0x7fffffff && (bi == 0x7fffffff || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
-            });
-            bi = __builtin_amdgcn_readfirstlane(bi);       // (one choice for the wave, also where logits are no numbers)
-            best = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(best)));
-            if (k == 0) mx = best;
-            sum += expf(best - mx);
-            if ((bi & 63) == lane) taken |= 1u << (bi >> 6);
-        }
-        int rank = 0;
-#pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const bool mine = taken >> c & 1;
-            const uint64_t mask = __builtin_amdgcn_ballot_w64(mine);
-            if (mine) {
-                const int64_t at = (int64_t)t * top + rank + __builtin_popcountll(mask & ((1ull << lane) - 1));
-                chosen[at] = c * 64 + lane;
-                picked[at - (int64_t)t0 * top] = c * 64 + lane;
-                weights[at] = expf(zs[c] - mx) / sum * scale;
-            }
-            rank += __builtin_popcountll(mask);
-        }
+        choose<NC>(zs, t, t0, n, top, scale, chosen, weights, picked);
     }
     if (gridDim.x == 1 && p.counts) {
         __syncthreads();
@@ -263,20 +335,36 @@ __global__ __launch_bounds__(64 * ROUTER_WAVES) void router_kernel(const float* 
     }
 }
 
-// counts (and the other three) not null with up to 16 tokens: the pairs are sorted too.  sums: float32, 256 * max(16, ceil(n / 16))
-// for every 16 tokens.
+// float32 numbers of workspace that li_router wants; 0: one launch, without any (workgroups of 16 tokens for 7/8 of the 256 CUs and more, but
+// not for more than all of them; figures above).
+extern "C" int64_t li_router_sums(int n_tokens, int n) {
+    const int blocks = (n_tokens + 15) / 16, tiles = (n + 15) / 16;
+    if (n < 1 || (blocks > 224 && blocks <= 256)) return 0;
+    return (int64_t)blocks * tiles * router_share(tiles) * 256;
+}
+
+// counts (and the other three) not null with up to 16 tokens: the pairs are sorted too.  sums: li_router_sums of them.
 extern "C" int li_router(const void* X, const void* Wt, int dt, const float* bias, int parts, int n_tokens, int K, int n, int top, float scale,
                          int* chosen, float* weights, int* counts, int* offsets, int* row_of, int* slot_of, float* sums, hipStream_t stream) {
     if (n_tokens <= 0) return LI_OK;
-    if (!X || !Wt || !chosen || !weights || !sums || n < 1 || top < 1 || top > n || parts < 1 || parts > 3) return LI_BAD_ARG;
+    if (!X || !Wt || !chosen || !weights || n < 1 || top < 1 || top > n || parts < 1 || parts > 3 || (dt != DT_F16 && dt != DT_BF16)) return LI_BAD_ARG;
+    // (n + top: what this entry takes; LDS would hold more, 64 bytes an output or a choice.  The caller has a path for the others)
     if (n > ROUTER_MAX || n + top > 640 || K < 32 || K % 32 || ((uintptr_t)X & 15) || ((uintptr_t)Wt & 15) || ((uintptr_t)sums & 15)) return LI_UNSUPPORTED;
-    if (counts && (n_tokens > 16 || !offsets || !row_of || !slot_of)) return LI_BAD_ARG;
+    if (counts && (n_tokens > 16 || !offsets || !row_of || !slot_of || !sums)) return LI_BAD_ARG;
     const Pairs p{counts, offsets, row_of, slot_of};
     const int blocks = (n_tokens + 15) / 16, tiles = (n + 15) / 16, kw = router_share(tiles);
+    if (!sums) {
+        const size_t lds = (size_t)16 * n * sizeof(float);
+#define GO(T, NC) router_one_kernel<T, NC><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>((const T*)X, (const T*)Wt, bias, parts, n_tokens, K, n, top, scale, chosen, weights)
+        if (dt == DT_F16) { if (n <= 64) GO(f16, 1); else GO(f16, 8); }
+        else { if (n <= 64) GO(bf16, 1); else GO(bf16, 8); }
+#undef GO
+        LI_CHECK_LAUNCH();
+        return LI_OK;
+    }
     dim3 grid(blocks, tiles * kw);
     if (dt == DT_F16) router_sums_kernel<f16><<<grid, 64, 0, stream>>>((const f16*)X, (const f16*)Wt, sums, parts, n_tokens, K, tiles, kw);
-    else if (dt == DT_BF16) router_sums_kernel<bf16><<<grid, 64, 0, stream>>>((const bf16*)X, (const bf16*)Wt, sums, parts, n_tokens, K, tiles, kw);
-    else return LI_BAD_ARG;
+    else router_sums_kernel<bf16><<<grid, 64, 0, stream>>>((const bf16*)X, (const bf16*)Wt, sums, parts, n_tokens, K, tiles, kw);
     const size_t lds = (size_t)16 * top * sizeof(int);
     if (n <= 64) router_kernel<1><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>(sums, bias, n_tokens, n, kw, top, scale, chosen, weights, p);
     else router_kernel<8><<<blocks, 64 * ROUTER_WAVES, lds, stream>>>(sums, bias, n_tokens, n, kw, top, scale, chosen, weights, p);

@@ -2252,6 +2252,7 @@ def experts():
     global _experts
     if _experts is None:
         _experts = build.experts_library()
+        _experts.li_router_sums.restype = c_int64
     return _experts
 
 
@@ -2304,7 +2305,8 @@ def route_pairs(h, w_router, bias, n_experts: int, top: int, scale: float = 1.0)
     p = SortedPairs(t, top, n, h.device)
     lists = (_ptr(p.counts), _ptr(p.offsets), _ptr(p.row_of), _ptr(p.slot_of))
     small = t <= 16                                        # one workgroup has every token: it sorts the pairs too
-    sums = torch.empty(((t + 15) // 16 * max(16, (n + 15) // 16) * 256,), dtype=torch.float32, device=h.device)
+    room = experts().li_router_sums(t, n)                  # 0: a number of tokens for which one launch is the faster way
+    sums = torch.empty((room,), dtype=torch.float32, device=h.device) if room else None
     _check(experts().li_router(_ptr(h), _ptr(w_router), DT[h.dtype], _ptr(bias), parts, t, k, n, top, c_float(scale), _ptr(p.chosen),
                                _ptr(p.weights), *(lists if small else (None,) * 4), _ptr(sums), _stream()), "router")
     if not small:

@@ -290,6 +290,21 @@ def test_router_sums_by_shares_of_k(lib, E, K):
             check_pairs(ops.route_pairs(h.to(DEV), wr, None, E, 4), chosen, torch.softmax(z.gather(1, chosen), -1))
 
 
+# one launch for all (3,585 to 4,096 tokens) and two: a token's choice and weights are the same, bit for bit, in any company
+@pytest.mark.parametrize("E,K,top", [(5, 64, 2), (16, 2080, 4), (40, 96, 3), (100, 64, 8), (512, 32, 128)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+def test_router_in_one_launch_and_in_two(lib, E, K, top, dtype):
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(E)
+    h, b = torch.randn(4097, K, generator=g).to(DT[dtype]).to(DEV), torch.randn(E, generator=g).to(DEV)
+    wr = ops.router_weight((torch.randn(E, K, generator=g) * K ** -0.5).to(DEV), DT[dtype])
+    two = ops.route_pairs(h, wr, b, E, top)
+    for T in (3584, 3585, 3590, 4096):
+        p = ops.route_pairs(h[:T], wr, b, E, top)
+        assert torch.equal(p.chosen, two.chosen[:T]) and torch.equal(p.weights, two.weights[:T]), T
+        assert torch.equal(p.counts.cpu().long(), torch.bincount(p.chosen.flatten().long().cpu(), minlength=E)), T
+
+
 def test_the_first_of_equal_logits_is_chosen_and_numbers_that_are_none_do_no_harm(lib):
     from llm_infer_amd.kernels import ops
     h = torch.ones(20, 32, dtype=torch.bfloat16, device=DEV)
