@@ -781,8 +781,8 @@ extern "C" int li_sigmoid_attn(const void* q, void* out, int dt, const void* k_p
 template <class T> __device__ __forceinline__ float rounded_to(float v) { return to_f32(from_f32<T>(v)); }
 template <> __device__ __forceinline__ float rounded_to<float>(float v) { return v; }
 
-template <int ROWS, class TR, bool WHOLE>
-__global__ void decay_attn_kernel(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
+template <int ROWS, class TR, bool WHOLE, int THREADS>
+__global__ __launch_bounds__(THREADS) void decay_attn_kernel(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
                                   float* __restrict__ state, const float* __restrict__ decay,
                                   const int* __restrict__ seq_slot, const int* __restrict__ seq_qstart,
                                   const int* __restrict__ seq_qlen, float* __restrict__ out, int H, int d, int dv) {
@@ -843,12 +843,24 @@ extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off
     // has one (16 heads of 128 x 128, 1 sequence 6.4 -> 4.1 us, 8 7.6 -> 6.6)
     int split = 1;
     while ((int64_t)n_seqs * H * split < 256 && dv % (2 * split) == 0 && dv / (2 * split) >= 32) split *= 2;
+    if (rows == 64 && RG * (dv / split) > 512 && dv % (2 * split) == 0) split *= 2;       // (so that 64 rows have the registers, below)
     const int cols = dv / split;
+    // 32 and 64 rows a thread with all their loads on their way want up to 227 registers: in workgroups of up to 512 threads they have
+    // them (1,024 threads have 128 each, and 18 to 95 of them were spilled).  One token a sequence, 16 heads, us with 1,024 and with 512: 128 x
+    // 128, 1 sequence 4.8 and 4.3, 16 9.6 and 7.7, 64 32.9 and 28.5; 128 x 256 11.6 and 5.0, 33.8 and 11.8, 99 and 49; 256 x 256 13.1 and 5.5, 53
+    // and 26, 236 and 103; 200 x 256 (rows not whole) 11.2 and 9.8, 27.8 and 27.9, 99 and 90.  Whole rows in 1,024 threads are the worse ones
+    // there (256 x 255, 1 sequence 32.5, not as whole ones 14.6).  Tokens one behind the other ask for waves instead, two workgroups a CU:
+    // 32 sequences of 50 tokens, 128 x 128 107 and 179, 128 x 256 205 and 231, 200 x 256 543 and 893, but where a CU has one
+    // workgroup at the most, 2 sequences of 200, 8 heads, 128 x 256 442 and 328, 256 x 256 476 and 358
+    const bool step = !seq_qlen, few = step || (rows == 64 && (int64_t)n_seqs * H * split <= 256);
     dim3 grid(n_seqs, H, split), block(RG * cols);
     const size_t lds = (size_t)(2 * d + cols + RG * cols) * sizeof(float);
-#define GO2(R, TR, WHOLE) decay_attn_kernel<R, TR, WHOLE><<<grid, block, lds, stream>>>(proj, stride, q_off, k_off, v_off, state, \
+#define GO2(R, TR, WHOLE, N) decay_attn_kernel<R, TR, WHOLE, N><<<grid, block, lds, stream>>>(proj, stride, q_off, k_off, v_off, state, \
         decay, seq_slot, seq_qstart, seq_qlen, out, H, d, dv)
-#define GO1(R, TR) do { if (d % R == 0) GO2(R, TR, true); else GO2(R, TR, false); } while (0)
+#define GO1(R, TR) do { \
+        if (R >= 32 && few && RG * cols <= 512) { if (d % R == 0) GO2(R, TR, true, R < 32 ? 1024 : 512); else GO2(R, TR, false, R < 32 ? 1024 : 512); } \
+        else if (d % R == 0 && (R < 64 || !step)) GO2(R, TR, true, 1024); \
+        else GO2(R, TR, false, 1024); } while (0)
 #define GO(R) do { if (round_dt == DT_F32) GO1(R, float); else if (round_dt == DT_F16) GO1(R, f16); else GO1(R, bf16); } while (0)
     if (rows == 4) GO(4); else if (rows == 8) GO(8); else if (rows == 16) GO(16); else if (rows == 32) GO(32); else GO(64);
 #undef GO

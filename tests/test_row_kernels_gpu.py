@@ -195,6 +195,29 @@ def test_decay_recurrence_of_one_sequence_and_many(ops, dtype, H, d, dv):
             assert ((one[0].view(H, dv).double().cpu() - want).abs() <= 2.0 ** -17 * (S * q.view(H, d, 1)).abs().sum(1) + 1e-6).all()
 
 
+# tokens one by one and all at once, for one workgroup a CU and for more, of 32 and 64 rows a thread, whole and not, columns that split and
+# that do not: the same arithmetic in the same order
+@pytest.mark.parametrize("d,dv", [(64, 64), (128, 128), (100, 128), (128, 256), (256, 256), (200, 256), (256, 255), (200, 255)])
+@pytest.mark.parametrize("n", [1, 70])
+def test_decayed_attention_steps_and_prompts(ops, d, dv, n):
+    H, T = 4, 5
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    proj, decay = torch.randn(n * T, H * (2 * d + dv), device=DEV), torch.rand(H, device=DEV) * 0.5 + 0.5
+    at_once = torch.randn(n, H, d, dv, device=DEV)
+    by_one, S = at_once.clone(), at_once[0].double().cpu()
+    args = (0, H * d, 2 * H * d)
+    o = ops.decay_attention(proj, *args, at_once, decay, i32(list(range(n))), i32([i * T for i in range(n)]), i32([T] * n), n, H, d, dv)
+    for t in range(T):
+        one = ops.decay_attention(proj[t::T].contiguous(), *args, by_one, decay, i32(list(range(n))), None, None, n, H, d, dv)
+        assert torch.equal(one, o[t::T])
+        q, k, v = (torch.nn.functional.silu(p.double()) for p in proj[t].cpu().split([H * d, H * d, H * dv]))
+        S = decay.double().cpu()[:, None, None] * S + k.view(H, d, 1) * v.view(H, 1, dv)
+        size = (S * q.view(H, d, 1)).abs().sum(1)
+        # some 100 roundings of 2^-24 in a sum of up to 256 products of the order of 1
+        assert ((one[0].view(H, dv).double().cpu() - (S * q.view(H, d, 1)).sum(1)).abs() <= 2.0 ** -17 * size + 1e-6).all()
+    assert torch.equal(at_once, by_one)
+
+
 # one token a sequence with a state whose rows and columns are all there (fetched under no condition), and with rows or columns that a
 # wave has not; three steps in a row against 64 bits
 @pytest.mark.parametrize("rows,cols", [(64, 64), (128, 128), (64, 40), (100, 64), (7, 130), (16, 64), (256, 64)])
