@@ -150,7 +150,7 @@ __device__ __forceinline__ float block_total(float v, float (&mine)[16], int wav
 // The same with 16-byte loads: N4 pieces of four elements a thread (d a multiple of 4, 16-byte aligned rows), of up to 512 threads
 // up to two pieces.  With its launch, alpha x + y1 + y2 and its norm behind a product: 1 row of 2,048 2.5 -> 2.3 us, of 4,096 3.1 -> 2.6 (a
 // piece after the other and four barriers; now everything at once and two).
-template <class TC, int N4>
+template <class TC, int N4, bool TOGETHER>
 __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restrict__ x, float alpha,
                                                                  const float* __restrict__ y1, float s1,
                                                                  const float* __restrict__ y2, float s2,
@@ -166,18 +166,13 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     f32x4 v[N4], av[N4], bv[N4], wv[N4];
     int at[N4];
-    // (everything at once, without a branch: what lies beyond the row is its last piece again and counts nowhere)
-#pragma unroll
-    for (int u = 0; u < N4; ++u) {
-        at[u] = min((int)(threadIdx.x + u * blockDim.x), n4 - 1);
+    float s = 0.f, ss = 0.f;
+    auto fetch = [&](int u) {
         v[u] = x4[at[u]];
         av[u] = a4[at[u]];
-        wv[u] = w4[at[u]];
         bv[u] = b4 ? b4[at[u]] : zero;
-    }
-    float s = 0.f, ss = 0.f;
-#pragma unroll
-    for (int u = 0; u < N4; ++u) {
+    };
+    auto add = [&](int u) {
         const bool in = (int)(threadIdx.x + u * blockDim.x) < n4;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -186,6 +181,21 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
             v[u][q] = alpha * v[u][q] + y;
             s = in ? s + v[u][q] : s;
         }
+    };
+    // TOGETHER: everything at once, without a branch: what lies beyond the row is its last piece again and counts nowhere.  In workgroups
+    // of more than 512 threads (rows of more than 8,192) the pieces come one by one and their weights last: eight at once do not fit the
+    // registers (1 row of 32,768 18.6 us, one by one 9.4), and four leave a CU one workgroup (300 rows of 16,384 19.6 and 17.9, 1 row 6.5 and 6.3)
+#pragma unroll
+    for (int u = 0; u < N4; ++u) at[u] = min((int)(threadIdx.x + u * blockDim.x), n4 - 1);
+    if constexpr (TOGETHER) {
+#pragma unroll
+        for (int u = 0; u < N4; ++u) { fetch(u); wv[u] = w4[at[u]]; }
+#pragma unroll
+        for (int u = 0; u < N4; ++u) add(u);
+    } else {
+#pragma unroll
+        for (int u = 0; u < N4; ++u)
+            if ((int)(threadIdx.x + u * blockDim.x) < n4) { fetch(u); add(u); }
     }
     const float mean = block_total<W>(s, st[0], waves) / (float)d;
 #pragma unroll
@@ -201,6 +211,7 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
         if ((int)(threadIdx.x + u * blockDim.x) < n4) {
             f32x4 r;
             Out4 c4;
+            if (!TOGETHER) wv[u] = w4[at[u]];
 #pragma unroll
             for (int q = 0; q < 4; ++q) { r[q] = v[u][q] / sd * wv[u][q]; c4.v[q] = from_f32<TC>(r[q]); }
             x4[at[u]] = r;
@@ -219,8 +230,9 @@ extern "C" int li_add_layernorm(float* x, float alpha, const float* y1, float s1
     if (aligned && d <= 32 * 1024) {
         const int n4 = d / 4, per = n4 <= 512 ? 1 : (n4 <= 1024 ? 2 : (n4 <= 4096 ? 4 : 8));
         dim3 vb(((n4 + per - 1) / per + 63) / 64 * 64);
-#define GO1(TC, N) add_layernorm_vec_kernel<TC, N><<<grid, vb, 0, stream>>>(x, alpha, y1, s1, y2, s2, w, eps, (TC*)copy, d)
-#define GO(TC) do { if (per == 1) GO1(TC, 1); else if (per == 2) GO1(TC, 2); else if (per == 4) GO1(TC, 4); else GO1(TC, 8); } while (0)
+#define GO1(TC, N, TOGETHER) add_layernorm_vec_kernel<TC, N, TOGETHER><<<grid, vb, 0, stream>>>(x, alpha, y1, s1, y2, s2, w, eps, (TC*)copy, d)
+#define GO(TC) do { if (per == 1) GO1(TC, 1, true); else if (per == 2) GO1(TC, 2, true); else if (vb.x <= 512) GO1(TC, 4, true); \
+                    else if (per == 4) GO1(TC, 4, false); else GO1(TC, 8, false); } while (0)
         if (!copy || copy_dt == DT_F32) GO(float);
         else if (copy_dt == DT_F16) GO(f16);
         else if (copy_dt == DT_BF16) GO(bf16);

@@ -112,6 +112,18 @@ def test_layer_norms_of_sums(ops, width, mean):
         assert torch.equal(copy, out.to(torch.bfloat16))
 
 
+# rows whose pieces come one by one: four and eight a thread, the last workgroup of 512 threads and the first of more, the last row that is
+# kept in registers and the first that is not
+@pytest.mark.parametrize("width", [8192, 8196, 16384, 16388, 32768, 32772])
+def test_layer_norms_of_sums_of_wide_rows(ops, width):
+    x, y, y2, w = torch.randn(3, width, device=DEV), torch.randn(3, width, device=DEV) + 2, torch.randn(3, width, device=DEV), torch.rand(width, device=DEV) + 0.5
+    for adds in ([(y, 0.5)], [(y, 0.5), (y2, 2.0)]):
+        out = x.clone()
+        copy = ops.add_layernorm(out, 2.0, adds, w, 1e-5, torch.float16)
+        _close(out, _ln(2 * x.double() + sum(s * t.double() for t, s in adds), 1e-5) * w.double())
+        assert torch.equal(copy, out.to(torch.float16))
+
+
 # whole numbers whose mean is 0 and whose squares add up to less than 2^24: every sum is exact in float32 in any order, if the mean is taken
 # before the deviations, and then only roots, divisions and products round, once each (numpy's are correctly rounded, as the kernels' are)
 @pytest.mark.parametrize("width", WIDTHS + [37])
