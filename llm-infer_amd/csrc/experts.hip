@@ -381,7 +381,7 @@ extern "C" int li_router(const void* X, const void* Wt, int dt, const float* bia
 // 98, a quarter with 32 each 53, 46, 46.
 // ---------------------------------------------------------------------------
 template <class T, int MT, int KW>
-__global__ __launch_bounds__(64 * KW) void experts_gemv_kernel(const T* __restrict__ X, const T* __restrict__ Wt, int K,
+__global__ __launch_bounds__(64 * KW, 4) void experts_gemv_kernel(const T* __restrict__ X, const T* __restrict__ Wt, int K,
                                                                int64_t w_stride, Epilogue e, int n_experts,
                                                                const int* __restrict__ counts, const int* __restrict__ offsets,
                                                                const int* __restrict__ row_of) {
