@@ -61,10 +61,13 @@ def _dev(*tensors):
 def upload(values, device) -> torch.Tensor:
     """int32 ``values`` (numbers, or rows of them) on ``device``, for the index arrays of a step.  They go through page-locked memory,
     which torch keeps until the copy is done, so the copy stands in line with the step's kernels and the host goes on; out of
-    ordinary memory it waits for everything that is queued, and the device then for the host's next launches."""
+    ordinary memory it waits for everything that is queued, and the device then for the host's next launches.  Not while a graph is
+    recorded: it would hold the copy, out of memory that is used for something else by the time of a replay."""
     values = np.asarray(values, dtype=np.int32)
     if torch.device(device).type != "cuda":
         return torch.from_numpy(values).to(device)
+    if torch.cuda.is_current_stream_capturing():
+        raise KernelError("index arrays are uploaded before a graph is recorded, not into it")
     staged = torch.empty(values.shape, dtype=torch.int32, pin_memory=True)
     staged.numpy()[...] = values
     return staged.to(device, non_blocking=True)

@@ -36,6 +36,38 @@ def test_gathered_rows(ops, dtype, n, d, shift):
     assert ((got - want).abs() <= bound).all()
 
 
+# index arrays one behind the other while the device is busy, of one row, two rows and none: every one keeps its own values
+def test_uploads_behind_queued_work(ops):
+    a = torch.randn(4096, 4096, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(20):
+        a = (a @ a).clamp_(-1, 1)
+    values = [[[i * 1000 + j for j in range(1 + i * 37 % 5000)]] * (1 + i % 2) for i in range(200)] + [[], [[], []]]
+    there = [ops.upload(v if len(v) != 1 else v[0], DEV) for v in values]
+    for v, t in zip(values, there):
+        assert t.dtype == torch.int32 and t.tolist() == (v if len(v) != 1 else v[0])
+
+
+# also where the page-locked memory is there already and nothing else would refuse
+def test_no_upload_into_a_graph(ops):
+    from llm_infer_amd.kernels.ops import KernelError
+    x = torch.zeros(4, device=DEV)
+    for _ in range(4):
+        ops.upload([7, 7, 7], DEV)
+        torch.cuda.synchronize()
+    free = [torch.empty(3, dtype=torch.int32, pin_memory=True) for _ in range(4)]
+    del free
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        x.add_(1.0)
+        with pytest.raises(KernelError):
+            ops.upload([1, 2, 3], DEV)
+    for n in (1, 2, 3):
+        graph.replay()
+        assert x.tolist() == [float(n)] * 4
+
+
 # one chunk, the edges between chunks and between a thread's elements, ties: the first of the largest
 @pytest.mark.parametrize("v", [1, 63, 255, 257, 4095, 4096, 4097, 8193, 32000])
 def test_argmax_first_of_the_largest(ops, v):
