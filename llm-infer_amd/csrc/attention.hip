@@ -1030,7 +1030,9 @@ __global__ __launch_bounds__(256) void attn_f32_few_kernel(
         if (adds) {
             values(0);
             dots(0);
-            asm volatile("; %0" : "+v"(dot));         // (keeps this form apart from the other, which has no values behind it)
+            // (keeps this form apart from the other, which has no values behind it: merged, both would wait for the values first.  It costs no
+            // instruction, and were the two merged all the same, results would stay as they are)
+            asm volatile("; %0" : "+v"(dot));
         } else {
             dots(0);
         }

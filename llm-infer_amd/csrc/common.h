@@ -79,13 +79,14 @@ __device__ __forceinline__ float sum_quarters(float v) { const LanePair p = quar
 __device__ __forceinline__ float max_halves(float v) { const LanePair p = halves(v); return fmaxf(p.lo, p.hi); }
 __device__ __forceinline__ float max_quarters(float v) { const LanePair p = quarters(v); return fmaxf(p.lo, p.hi); }
 
-__device__ __forceinline__ float half_sum(float v) {   // over the lanes of this lane's half wave
-    v = sum_quarters(v);
+// Sums over the 16 lanes of a row, over a half wave and over the wave, every lane's the same.
+__device__ __forceinline__ float row_sum(float v) {
     v += row_move<ROW_ROR(8)>(v);
     v += row_move<ROW_ROR(4)>(v);                      // (a row repeats every 8 lanes by now: 4 back is 4 on)
     v += row_move<QUAD_SWAP2>(v);
     return v + row_move<QUAD_SWAP1>(v);
 }
+__device__ __forceinline__ float half_sum(float v) { return row_sum(sum_quarters(v)); }
 __device__ __forceinline__ float wave_sum(float v) { return half_sum(sum_halves(v)); }
 // wave_sum of a * b with the first addition and the lane's own product one multiply-add: a rounding less.  (The other half's
 // product is rounded, so the two halves' results may differ in their last bit.)
@@ -101,15 +102,9 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(v, row_move<QUAD_SWAP1>(v));
 }
 
-// Sums over the 16 lanes of a row, every lane's the same.
-__device__ __forceinline__ float row_sum(float v) {
-    v += row_move<ROW_ROR(8)>(v);
-    v += row_move<ROW_ROR(4)>(v);
-    v += row_move<QUAD_SWAP2>(v);
-    return v + row_move<QUAD_SWAP1>(v);
-}
 // A wave's choice among pairs (value, index): `take(value, index)` compares another lane's pair with this lane's `v`, `i` and
-// takes it over if it is the better one.  Lane 0 compares its own with those of lanes 32, 16, 8, 4, 2 and 1 on, in this order.
+// takes it over if it is the better one.  Lane 0 compares its own with those of lanes 32, 16, 8, 4, 2 and 1 on, in this order; where `take`
+// orders all pairs (no value is no number), every lane ends with the same one.
 template <class F> __device__ __forceinline__ void wave_choice(float& v, int& i, F take) {
     const auto moved = [&](auto move) { take(move(v), __float_as_int(move(__int_as_float(i)))); };
     const LanePair hv = halves(v), hi = halves(__int_as_float(i));

@@ -190,7 +190,7 @@ def test_gated_norm_and_polynorm_of_a_row(ops, n):
 @pytest.mark.parametrize("width", WIDTHS[:-1])
 def test_average_over_depth_with_its_norms(ops, width, terms):
     hist, weights = torch.randn(terms + 1, 3, width, device=DEV), torch.rand(terms, device=DEV)
-    weights[0] = 0.0                                               # (a term of weight 0 that is not finite shows all the same)
+    hist[terms] = torch.nan                                        # behind the last term: nothing of it may be seen
     nw = torch.rand(width, device=DEV) + 0.5
     norms = [(nw, 1e-5, torch.float16), (nw, 1e-6, torch.float32)]
     out = torch.empty(3, width, device=DEV)
@@ -199,6 +199,15 @@ def test_average_over_depth_with_its_norms(ops, width, terms):
     assert torch.equal(out, plain)
     for w, eps, dt in norms:
         assert torch.equal(ops.prepared_norm(out, w, eps, dt), ops.rmsnorm(plain, w, eps, dt))
+    each = hist[:terms].double() * weights.double()[:, None, None]
+    # a rounding of 2^-24 for every product and sum
+    assert ((out - each.sum(0)).abs() <= 2 * terms * 2.0 ** -24 * each.abs().sum(0)).all()
+    weights[0] = 0.0                                               # a term of weight 0 that is not finite shows, there and nowhere else
+    hist[0, 1, width - 1], hist[0, 2, 0] = torch.inf, torch.nan
+    got = ops.average_norms(hist, terms, weights, torch.empty_like(out), norms)
+    bad = torch.zeros(3, width, dtype=torch.bool, device=DEV)
+    bad[1, width - 1] = bad[2, 0] = True
+    assert torch.equal(got.isnan(), bad) and torch.equal(ops.depth_average(hist, terms, weights, torch.empty_like(out)).isnan(), bad)
 
 
 # a row shorter than a wave's first loads, ragged against them, whole, of the wider form and beyond it; few tokens against many
