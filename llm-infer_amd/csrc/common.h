@@ -152,26 +152,17 @@ __device__ __forceinline__ float block_max(float v, float* scratch) {
 static inline dim3 gather_grid(int n_tokens, int d) {
     return dim3(n_tokens, n_tokens < 256 ? (d + 4 * GATHER_THREADS - 1) / (4 * GATHER_THREADS) : 1);
 }
-// f(element, n) for this thread's elements of a row of d: four together, n of them in the row
-template <class F> __device__ __forceinline__ void gather_row(int d, F f) {
-    for (int i = 4 * (blockIdx.y * GATHER_THREADS + threadIdx.x); i < d; i += 4 * GATHER_THREADS * gridDim.y) f(i, min(4, d - i));
+// For this thread's elements of a row of d: quad(i) for four from i on, or, where the rows do not allow a load for four, one(i),
+// neighbouring elements by neighbouring threads (514 wide, 4,000 rows 4.2 us, four to a thread 6.3)
+template <class Q, class E> __device__ __forceinline__ void gather_row(int d, bool quads, Q quad, E one) {
+    const int at = blockIdx.y * GATHER_THREADS + threadIdx.x, step = GATHER_THREADS * gridDim.y;
+    if (quads) for (int i = 4 * at; i < d; i += 4 * step) quad(i);
+    else for (int i = at; i < d; i += step) one(i);
 }
 template <class T> struct alignas(4 * sizeof(T)) Quad { T v[4]; };
-// four elements of a row at p (whole: one load), the row's last n where there are no four
-template <class T> __device__ __forceinline__ f32x4 quad_of(const T* p, int n, bool whole) {
-    f32x4 r = {0.f, 0.f, 0.f, 0.f};
-    if (whole) {
-        const Quad<T> q = *(const Quad<T>*)p;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) r[k] = to_f32(q.v[k]);
-    } else {
-        for (int k = 0; k < n; ++k) r[k] = to_f32(p[k]);
-    }
-    return r;
-}
-__device__ __forceinline__ void put_quad(float* p, f32x4 v, int n, bool whole) {
-    if (whole) *(f32x4*)p = v;
-    else for (int k = 0; k < n; ++k) p[k] = v[k];
+template <class T> __device__ __forceinline__ f32x4 quad_of(const T* p) {       // four elements, one load
+    const Quad<T> q = *(const Quad<T>*)p;
+    return f32x4{to_f32(q.v[0]), to_f32(q.v[1]), to_f32(q.v[2]), to_f32(q.v[3])};
 }
 
 // A power of two near 1 / (8 rms) for a row whose root mean square is `rms`: what the rows of a residual

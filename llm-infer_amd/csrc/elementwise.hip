@@ -15,7 +15,7 @@ __global__ void embed_kernel(const T* __restrict__ table, const int* __restrict_
     const T* row = table + (int64_t)tok * d;
     float* out = x + (int64_t)t * d;
     const bool whole = (d & 3) == 0 && (((uintptr_t)table | (uintptr_t)x) & 15) == 0;
-    gather_row(d, [&](int i, int n) { put_quad(out + i, quad_of(row + i, n, whole), n, whole); });
+    gather_row(d, whole, [&](int i) { *(f32x4*)(out + i) = quad_of(row + i); }, [&](int i) { out[i] = to_f32(row[i]); });
 }
 
 extern "C" int li_embed(const void* table, int table_dt, const int* tokens, float* x,

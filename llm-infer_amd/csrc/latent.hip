@@ -43,13 +43,14 @@ __global__ void embed_bigram_kernel(const T* __restrict__ table, const T* __rest
     const T* e = table + (int64_t)tok * d;
     const T* b = bigram + row * d;
     const bool whole = (d & 3) == 0 && (((uintptr_t)table | (uintptr_t)bigram | (uintptr_t)out) & 15) == 0;
-    gather_row(d, [&](int i, int n) {
-        f32x4 v = quad_of(e + i, n, whole);
-        const f32x4 bv = quad_of(b + i, n, whole);
+    float* o = out + (int64_t)t * d;
+    gather_row(d, whole, [&](int i) {
+        f32x4 v = quad_of(e + i);
+        const f32x4 bv = quad_of(b + i);
 #pragma unroll
         for (int k = 0; k < 4; ++k) v[k] = v[k] * scale + bv[k];
-        put_quad(out + (int64_t)t * d + i, v, n, whole);
-    });
+        *(f32x4*)(o + i) = v;
+    }, [&](int i) { o[i] = to_f32(e[i]) * scale + to_f32(b[i]); });
 }
 
 __global__ void last_token_kernel(const int* __restrict__ tokens, const int* __restrict__ seq_slot,
