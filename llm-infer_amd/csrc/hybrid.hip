@@ -750,7 +750,8 @@ __global__ __launch_bounds__(256) void small_logits_kernel(const T* __restrict__
 // partial sums of the 256, so that the operands come 16 and 8 bytes at a time, h once for JB outputs, and only lanes exchange sums.
 // Bound by its loads' latency for few tokens, by the weights' way from L2 for many: 2,253 tokens x 9 outputs of 4,096 75 -> 21 us,
 // 8,000 x 16 459 -> 63, 300 x 9 12.0 -> 8.7.  B: quads of a lane on their way together, all of a row for few tokens (one by one and
-// then, us in a recorded chain, 4 tokens x 9 outputs of 4,096 3.5 -> 2.2, 8 x 16 of 2,048 2.2 -> 1.8, 255 x 16 of 4,096 7.2 -> 6.1); eight are enough for half as wide a row.
+// then, us in a recorded chain, 4 tokens x 9 outputs of 4,096 3.5 -> 2.2, 8 x 16 of 2,048 2.2 -> 1.8, 255 x 16 of 4,096 7.2 -> 6.1), and no more than the row has (eight for 64
+// wide: 255 x 64 outputs 5.9 -> 9.9).
 template <class T, int TOK, int JB, int B>
 __global__ void small_logits_wave_kernel(const T* __restrict__ h, const float* __restrict__ w, float* __restrict__ out,
                                          const float* __restrict__ bias, int n_rows, int width, int n) {
@@ -809,8 +810,9 @@ extern "C" int li_small_logits(const void* h, int dt, const float* w, float* out
             DISPATCH_T(dt, (small_logits_wave_kernel<T, 2, 4, 1><<<dim3((n_rows + 7) / 8, (n + 3) / 4), 256, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
         } else {
             dim3 grid(n_rows, n);
-            if (width <= 2048) DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1, 8><<<grid, 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
-            else DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1, 16><<<grid, 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)));
+#define GO(B) DISPATCH_T(dt, (small_logits_wave_kernel<T, 1, 1, B><<<grid, 64, 0, stream>>>((const T*)h, w, out, bias, n_rows, width, n)))
+            if (width <= 256) GO(1); else if (width <= 512) GO(2); else if (width <= 1024) GO(4); else if (width <= 2048) GO(8); else GO(16);
+#undef GO
         }
     } else if (n_rows >= 256) {                            // many tokens: four a workgroup share every weight fetched
         dim3 grid((n_rows + 3) / 4, n);
