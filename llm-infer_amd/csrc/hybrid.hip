@@ -509,7 +509,8 @@ __global__ __launch_bounds__(64) void ssm_scan_kernel(
     // a state whose rows and columns are all there is asked for, and left, under no condition, each of which was a branch.  A decode
     // step, us in a recorded chain, before and now: 128 heads of 128 x 64, 1 sequence 11.8 -> 6.6, 4 14.1 -> 9.4, 16 24.1 -> 22.8; 64 heads
     // of 64 x 64 6.3 -> 3.9, 6.7 -> 4.1, 10.0 -> 8.6, of 256 x 64 25.6 -> 10.9, 29.0 -> 13.6, 30.2 -> 26.3
-    const bool whole = N == NMAX && col - lane + 64 <= dv;
+    // (a head whose last columns fill no wave: only where all waves run at once; 32 heads of 64 x 100, 16 sequences 8.5 -> 7.9, but 64 21.1 -> 24.8)
+    const bool whole = N == NMAX && col - lane + 64 <= dv && (dv % 64 == 0 || gridDim.x * gridDim.y * gridDim.z <= 1024);
     if (whole) {
 #pragma unroll
         for (int i = 0; i < NMAX; ++i) s[i] = PASS != 1 ? S[(int64_t)i * dv] : 0.f;
