@@ -43,7 +43,7 @@ __global__ void embed_pos_kernel(const T* __restrict__ table, const int* __restr
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             v[k] *= scale;
-            if (freq && k < n) {
+            if (freq) {
                 const float a = p * freq[(i + k) >> 1];
                 v[k] += (k & 1) ? cosf(a) : sinf(a);
             }
