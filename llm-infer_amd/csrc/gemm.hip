@@ -425,16 +425,24 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
             if (!any) continue;
         }
         v8 a[U][NT], b[U][MT];
+        auto fetch = [&](auto once) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int s = s0 + u * SL;
-            const bool in = s + later < s_end;
-            const v8 z = {};
+            for (int u = 0; u < U; ++u) {
+                const int s = s0 + u * SL;
+                const bool in = s + later < s_end;
+                const v8 z = {};
 #pragma unroll
-            for (int t = 0; t < NT; ++t) a[u][t] = in ? load_once<v8>(wt[t] + (int64_t)s * 512) : z;
+                for (int t = 0; t < NT; ++t) {
+                    const T* from = wt[t] + (int64_t)s * 512;
+                    a[u][t] = !in ? z : decltype(once)::value ? load_once<v8>(from) : *(const v8*)from;
+                }
 #pragma unroll
-            for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
-        }
+                for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
+            }
+        };
+        // (17 to 32 rows: a matrix of less than 32 MiB through the caches; figures at li_gemm_rows)
+        if (MT == 1 || (int64_t)e.N * K >= 1 << 24) fetch(std::true_type{});
+        else fetch(std::false_type{});
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -543,7 +551,8 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
 // ===========================================================================
 static __device__ __attribute__((aligned(1024))) unsigned char zero_kib[1024];      // never written
 
-template <class T, int NT, int MT, int KW, int D>
+// ONCE: W past the caches (load_once).
+template <class T, int NT, int MT, int KW, int D, bool ONCE>
 __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(const T* __restrict__ X, const T* __restrict__ Wt,
                                                             int K, int ldx, Epilogue e, RowsOut ro) {
     typedef typename Vec<T>::v8 v8;
@@ -631,7 +640,8 @@ __global__ __launch_bounds__(64 * KW) void gemm_rows_kernel(const T* __restrict_
                     const int step = 2 * dd + h;
                     const unsigned char* from = (in && step < steps) ? wbase[t] + (int64_t)step * 1024
                                                                      : (const unsigned char*)zero_kib;
-                    asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[u][h][t]) : "v"(woff), "s"(from) : "memory");
+                    if constexpr (ONCE) asm volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(a[u][h][t]) : "v"(woff), "s"(from) : "memory");
+                    else asm volatile("global_load_dwordx4 %0, %1, %2" : "=v"(a[u][h][t]) : "v"(woff), "s"(from) : "memory");
                 }
         };
         // where lane (r, g) finds row r, chunk 4 h + g of fragment 0 in a stage: unit r / 8, place
@@ -989,10 +999,15 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
         return LI_BAD_ARG;
     const RowsOut no_out{};
     const int blocks = (tiles + nt - 1) / nt;
+    // Matrices of less than 32 MiB stay in the caches beyond 16 rows: all of a small model's matrices together fit them, and in a large
+    // model these are bound by latency.  us past the caches and through them, of 100 MB of such matrices in turn and of 1.6 GB: 64 rows x
+    // 2,048 x 2,048 8.9 and 7.4, 8.3 and 8.5, x 512 x 4,096 12.2 and 9.1, 11.9 and 12.1, x 3,072 x 2,048 9.7 and 8.4, 8.7 and 8.8; 24 rows x 2,048 x
+    // 2,048 9.9 and 8.6, 9.2 and 9.5; larger ones, 48 rows x 4,096 x 4,096 17.1 and 15.4, 13.0 and 13.5, x 6,144 x 4,096 (600 MB) 17.6 and 18.4
+    const bool once = (int64_t)N * K * 2 >= 32 << 20;
     // stages of 64 of K a wave: what 128 KiB of LDS hold for the workgroup's waves
-#define GO(T, NT, MT, KW, D)                                                                              \
+#define LAUNCH(T, NT, MT, KW, D, ONCE)                                                                    \
     do {                                                                                                  \
-        auto kfn = gemm_rows_kernel<T, NT, MT, KW, D>;                                                    \
+        auto kfn = gemm_rows_kernel<T, NT, MT, KW, D, ONCE>;                                              \
         const size_t lds = (size_t)KW * D * 2 * MT * 1024;                                                \
         static bool allowed = false;               /* more than 64 KiB of LDS is asked for once */       \
         if (!allowed) {                                                                                   \
@@ -1001,6 +1016,11 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
             allowed = true;                                                                               \
         }                                                                                                 \
         kfn<<<blocks, 64 * KW, lds, stream>>>((const T*)X, (const T*)Wt, K, ldx, e, ro ? *ro : no_out);   \
+    } while (0)
+#define GO(T, NT, MT, KW, D)                                              \
+    do {                                                                  \
+        if (NT == 2 || MT == 1 || once) LAUNCH(T, NT, MT, KW, D, true);   \
+        else LAUNCH(T, NT, MT, KW, D, NT == 2 || MT == 1);                \
     } while (0)
 #define BY_MT(T, NT)                                            \
     do {                                                        \
@@ -1021,6 +1041,7 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
 #undef PICK
 #undef BY_MT
 #undef GO
+#undef LAUNCH
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

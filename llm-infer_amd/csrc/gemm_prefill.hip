@@ -581,6 +581,11 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     if constexpr (by_pairs(MODE) && A >= 3) {
         if (one_tile) products(std::true_type{});
         else products(std::false_type{});
+    } else if constexpr (MODE == -1 && A == 3) {
+        // (65 to 128 rows with K split: 128 rows x 4,096 x 14,336 40.3 us past the caches and 37.5 through them, x 2,048 x 8,192 23.7 and 21.9,
+        // 100 rows 36.6 and 35.3; whole K, x 28,672 x 4,096 56.9 and 61.2)
+        if (gridDim.z == 1) products(std::true_type{});
+        else products(std::false_type{});
     } else
         products(std::bool_constant<(A >= 3)>{});
 
