@@ -1142,7 +1142,7 @@ __global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const float* _
 
 // The same values with a thread's elements in registers, all fetched at once, for rows of up to N * blockDim.x.
 // Bound by the latency of a row's one workgroup.  With its launch, behind a product: 1 row of 2,048 3.0 -> 2.4 us, of 4,096 3.9 -> 3.0; 300
-// rows of 2,048 4.9 -> 3.6, 2,000 rows 11.4 -> 9.0.  (16 bytes a load instead: 2.2 and 2.8 us for one row, 9.4 for 2,000; but other elements
+// rows of 2,048 4.9 -> 3.6, 2,000 rows 11.4 -> 9.0, 256 rows of 8,192 13.3 -> 10.7.  (16 bytes a load instead: 2.2 and 2.8 us for one row, 9.4 for 2,000, 12.4 for 1,000 rows of 5,120 where this takes 18.1; but other elements
 // to a thread, so other bits.)
 template <class TO, int N>
 __global__ __launch_bounds__(1024) void gated_rmsnorm_reg_kernel(const float* __restrict__ o, const float* __restrict__ w,
@@ -1179,6 +1179,7 @@ extern "C" int li_gated_rmsnorm(const float* o, const float* w, const float* gat
 #define GO1(TO, N) gated_rmsnorm_reg_kernel<TO, N><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps)
 #define GO(TO) do { \
         if (n <= 4 * threads) GO1(TO, 4); else if (n <= 8 * threads) GO1(TO, 8); else if (n <= 16 * threads) GO1(TO, 16); \
+        else if (n <= 32 * threads) GO1(TO, 32); \
         else gated_rmsnorm_kernel<TO><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps); } while (0)
     if (out_dt == DT_F32) GO(float); else if (out_dt == DT_F16) GO(f16); else if (out_dt == DT_BF16) GO(bf16);
     else return LI_BAD_ARG;
