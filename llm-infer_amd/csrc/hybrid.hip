@@ -475,7 +475,7 @@ extern "C" int li_conv_history(const float* in, int stride, int col0, float* his
 // D_seg, leaving the state before every segment where its contribution was; pass 3 runs every segment again from
 // that state and writes y.  Twice the arithmetic, and as many waves as there are segments instead of sequences.
 struct ScanPlan {
-    int pass;                   // 0: a sequence's tokens in order; 1 and 3: see above
+    int pass;                   // 0: a sequence's tokens in order (one token a sequence: the kernel's pass 4); 1 and 3: see above
     const int* seg_seq;         // [segments] the sequence of a segment
     const int* seg_t0;          // [segments] its first token among the sequence's tokens of this step
     const int* seg_n;           // [segments] its tokens
@@ -489,14 +489,15 @@ __global__ __launch_bounds__(64) void ssm_scan_kernel(
     const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ D,
     float* __restrict__ state, const int* __restrict__ seq_slot, const int* __restrict__ seq_qstart,
     const int* __restrict__ seq_qlen, float* __restrict__ y, int P, int G, int N, int dv, ScanPlan plan) {
+    constexpr bool STEP = PASS == 4;
     const int h = blockIdx.y, lane = threadIdx.x, col = blockIdx.z * 64 + lane;
     const int g = h / (P / G), inner = P * dv;
     int q0, n;
     float* S;
-    if (PASS == 0) {
+    if (PASS == 0 || STEP) {
         const int seq = blockIdx.x;
         q0 = seq_qstart ? seq_qstart[seq] : seq;
-        n = seq_qlen ? seq_qlen[seq] : 1;
+        n = STEP ? 1 : seq_qlen[seq];
         S = state + (((int64_t)seq_slot[seq] * P + h) * N) * dv + col;
     } else {
         const int seg = blockIdx.x;
@@ -506,14 +507,16 @@ __global__ __launch_bounds__(64) void ssm_scan_kernel(
     }
     const bool live = col < dv;
     float s[NMAX];
-    // a state whose rows and columns are all there is asked for, and left, under no condition, each of which was a branch.  A decode
+    // A step's state whose rows and columns are all there is asked for, and left, under no condition, each of which was a branch (steps
+    // alone: beside the loop over a prompt's tokens the second form cost it registers, 4 prompts of 300 tokens, 128 heads of 128 x 64 713 -> 768 us, x
+    // 100 rows 672 -> 729).  A decode
     // step, us in a recorded chain, before and now: 128 heads of 128 x 64, 1 sequence 11.8 -> 6.6, 4 14.1 -> 9.4, 16 24.1 -> 22.8; 64 heads
     // of 64 x 64 6.3 -> 3.9, 6.7 -> 4.1, 10.0 -> 8.6, of 256 x 64 25.6 -> 10.9, 29.0 -> 13.6, 30.2 -> 26.3
     // (a head whose last columns fill no wave: only where all waves run at once; 32 heads of 64 x 100, 16 sequences 8.5 -> 7.9, but 64 21.1 -> 24.8)
-    const bool whole = N == NMAX && col - lane + 64 <= dv && (dv % 64 == 0 || gridDim.x * gridDim.y * gridDim.z <= 1024);
+    const bool whole = STEP && N == NMAX && col - lane + 64 <= dv && (dv % 64 == 0 || gridDim.x * gridDim.y * gridDim.z <= 1024);
     if (whole) {
 #pragma unroll
-        for (int i = 0; i < NMAX; ++i) s[i] = PASS != 1 ? S[(int64_t)i * dv] : 0.f;
+        for (int i = 0; i < NMAX; ++i) s[i] = S[(int64_t)i * dv];
     } else {
 #pragma unroll
         for (int i = 0; i < NMAX; ++i) s[i] = (live && i < N && PASS != 1) ? S[(int64_t)i * dv] : 0.f;
@@ -559,7 +562,7 @@ __global__ __launch_bounds__(64) void ssm_scan_kernel(
         }
         if (live && PASS != 1) y[(int64_t)(q0 + t) * inner + h * dv + col] = acc + dh * xt;
     }
-    if (PASS != 3 && whole) {
+    if (whole) {
 #pragma unroll
         for (int i = 0; i < NMAX; ++i) S[(int64_t)i * dv] = s[i];
     } else if (live && PASS != 3) {
@@ -606,9 +609,15 @@ extern "C" int li_ssm_scan(const float* xbc, int xbc_stride, const float* proj, 
     if (N > 256) return LI_UNSUPPORTED;
     dim3 grid(n_seqs, P, (dv + 63) / 64);
     ScanPlan plan{0, nullptr, nullptr, nullptr, nullptr, nullptr};
-#define SSM_PASS 0
-    SSM_LAUNCH(grid, plan);
+    if (!seq_qlen) {
+#define SSM_PASS 4
+        SSM_LAUNCH(grid, plan);
 #undef SSM_PASS
+    } else {
+#define SSM_PASS 0
+        SSM_LAUNCH(grid, plan);
+#undef SSM_PASS
+    }
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

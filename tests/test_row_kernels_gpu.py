@@ -271,6 +271,26 @@ def test_decayed_attention_steps_and_prompts(ops, d, dv, n):
     assert torch.equal(at_once, by_one)
 
 
+# tokens one by one and all at once, by the kernel that knows of one token and by the one that walks a prompt: the same bits
+@pytest.mark.parametrize("rows,cols", [(16, 64), (20, 30), (64, 64), (128, 64), (100, 100), (256, 70)])
+@pytest.mark.parametrize("n", [1, 40])
+def test_state_space_steps_and_prompts(ops, rows, cols, n):
+    from types import SimpleNamespace
+    H, T = 4, 5
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    step = SimpleNamespace(seq_slot=i32(list(range(n))), n_seqs=n, n_tokens=n)
+    prompt = SimpleNamespace(seq_slot=step.seq_slot, n_seqs=n, n_tokens=n * T, seq_qstart=i32([i * T for i in range(n)]), seq_qlen=i32([T] * n))
+    xbc, proj = torch.randn(n * T, H * cols + 2 * rows, device=DEV), torch.randn(n * T, H, device=DEV)
+    bias, alog, skip = torch.randn(H, device=DEV), torch.randn(H, device=DEV) * 0.3, torch.randn(H, device=DEV)
+    at_once = torch.randn(n, H, rows, cols, device=DEV)
+    by_one = at_once.clone()
+    y = ops.ssm_scan(xbc, proj, 0, bias, alog, skip, at_once, prompt, H, 1, rows, cols, None)
+    for t in range(T):
+        one = ops.ssm_scan(xbc[t::T].contiguous(), proj[t::T].contiguous(), 0, bias, alog, skip, by_one, step, H, 1, rows, cols, None)
+        assert torch.equal(one, y[t::T])
+    assert torch.equal(at_once, by_one)
+
+
 # one token a sequence with a state whose rows and columns are all there (fetched under no condition), and with rows or columns that a
 # wave has not; three steps in a row against 64 bits
 @pytest.mark.parametrize("rows,cols", [(64, 64), (128, 128), (64, 40), (100, 64), (7, 130), (16, 64), (256, 64)])
