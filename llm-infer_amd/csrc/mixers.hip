@@ -1125,29 +1125,50 @@ extern "C" int li_decay_attn_chunked(const float* proj, int stride, int q_off, i
 // out = o / sqrt(mean(o^2) + eps) * w * sigmoid(gate): the RMS norm over all heads of a token together, and
 // the gate.  o [T, n] float32; gate: float32 rows of `gate_stride` elements.
 // ---------------------------------------------------------------------------
-template <class TO>
-__global__ void gated_rmsnorm_kernel(const float* __restrict__ o, const float* __restrict__ w,
-                                     const float* __restrict__ gate, int gate_stride, TO* __restrict__ out, int n,
-                                     float eps) {
+// Rows longer than threads hold in registers, B of a thread's elements on their way together, twice (one by one and so: 1 row of
+// 20,480 12.3 -> 11.0 us, of 32,768 18.0 -> 15.4, 300 rows of 16,384 41 -> 22, 2,000 rows 86 -> 76).
+template <class TO, int B>
+__global__ __launch_bounds__(1024) void gated_rmsnorm_kernel(const float* __restrict__ o, const float* __restrict__ w,
+                                                             const float* __restrict__ gate, int gate_stride, TO* __restrict__ out, int n,
+                                                             float eps) {
     __shared__ float scratch[16];
     const int64_t t = blockIdx.x;
-    const float* orow = o + t * n;
-    const float* grow = gate + t * gate_stride;
+    const float *orow = o + t * n, *grow = gate + t * gate_stride;
+    const int step = blockDim.x;
     float ss = 0.f;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) { const float v = orow[i]; ss += v * v; }
+    for (int i0 = threadIdx.x; i0 < n; i0 += B * step) {
+        float v[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) v[u] = orow[min(i0 + u * step, n - 1)];
+#pragma unroll
+        for (int u = 0; u < B; ++u) { const float with = fmaf(v[u], v[u], ss); ss = i0 + u * step < n ? with : ss; }
+    }
     const float rms = sqrtf(block_sum(ss, scratch) / (float)n + eps);
-    for (int i = threadIdx.x; i < n; i += blockDim.x)
-        out[t * n + i] = from_f32<TO>(orow[i] / rms * w[i] * sigmoidf(grow[i]));
+    for (int i0 = threadIdx.x; i0 < n; i0 += B * step) {
+        float v[B], g[B], wv[B];
+#pragma unroll
+        for (int u = 0; u < B; ++u) {
+            const int i = min(i0 + u * step, n - 1);
+            v[u] = orow[i];
+            g[u] = grow[i];
+            wv[u] = w[i];
+        }
+#pragma unroll
+        for (int u = 0; u < B; ++u)
+            if (i0 + u * step < n) out[t * n + i0 + u * step] = from_f32<TO>(v[u] / rms * wv[u] * sigmoidf(g[u]));
+    }
 }
 
-// The same values with a thread's elements in registers, all fetched at once, for rows of up to N * blockDim.x.
-// Bound by the latency of a row's one workgroup.  With its launch, behind a product: 1 row of 2,048 3.0 -> 2.4 us, of 4,096 3.9 -> 3.0; 300
-// rows of 2,048 4.9 -> 3.6, 2,000 rows 11.4 -> 9.0, 256 rows of 8,192 13.3 -> 10.7.  (16 bytes a load instead: 2.2 and 2.8 us for one row, 9.4 for 2,000, 12.4 for 1,000 rows of 5,120 where this takes 18.1; but other elements
-// to a thread, so other bits.)
-template <class TO, int N>
-__global__ __launch_bounds__(1024) void gated_rmsnorm_reg_kernel(const float* __restrict__ o, const float* __restrict__ w,
-                                                                 const float* __restrict__ gate, int gate_stride, TO* __restrict__ out,
-                                                                 int n, float eps) {
+// The same values with a thread's elements in registers, all fetched at once, for rows of up to N * blockDim.x.  THREADS: the most of a
+// workgroup (24 and 32 elements want more than the 128 registers that a thread of 1,024 has: 16 of them were spilled).
+// Bound by the latency of a row's one workgroup, many rows by memory.  With its launch, one by one, so, and in batches as above: 1
+// row of 2,048 4.0, 4.0, 3.9 us, of 4,096 4.7, 4.1, 4.7, of 16,384 10.4, 8.3, 9.0; 256 rows of 4,096 8.4, 5.4, 6.2, of 8,192 14.0, 8.2, 9.5; 2,000 rows of
+// 4,096 22.2, 16.3, 18.9, of 5,120 27.4, 20.3, 24.6, of 8,192 40.2, 30.7, 36.9 (32 elements with the spills 45.7).  (16 bytes a load: behind a
+// product 2.2 and 2.8 us for one row of 2,048 and 4,096 where this takes 2.4 and 3.0; but other elements to a thread, so other bits.)
+template <class TO, int N, int THREADS>
+__global__ __launch_bounds__(THREADS) void gated_rmsnorm_reg_kernel(const float* __restrict__ o, const float* __restrict__ w,
+                                                                    const float* __restrict__ gate, int gate_stride, TO* __restrict__ out,
+                                                                    int n, float eps) {
     __shared__ float scratch[16];
     const int64_t t = blockIdx.x;
     const float *orow = o + t * n, *grow = gate + t * gate_stride;
@@ -1176,11 +1197,11 @@ extern "C" int li_gated_rmsnorm(const float* o, const float* w, const float* gat
     if (n <= 0 || gate_stride < n) return LI_BAD_ARG;
     const int wide = min(1024, (n / 4 + 63) / 64 * 64);
     const int threads = n_rows < 256 && wide > 64 ? wide : (n >= 1024 ? 256 : 64);
-#define GO1(TO, N) gated_rmsnorm_reg_kernel<TO, N><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps)
+#define GO1(TO, N, THREADS) gated_rmsnorm_reg_kernel<TO, N, THREADS><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps)
 #define GO(TO) do { \
-        if (n <= 4 * threads) GO1(TO, 4); else if (n <= 8 * threads) GO1(TO, 8); else if (n <= 16 * threads) GO1(TO, 16); \
-        else if (n <= 32 * threads) GO1(TO, 32); \
-        else gated_rmsnorm_kernel<TO><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps); } while (0)
+        if (n <= 4 * threads) GO1(TO, 4, 1024); else if (n <= 8 * threads) GO1(TO, 8, 1024); else if (n <= 16 * threads) GO1(TO, 16, 1024); \
+        else if (threads <= 256 && n <= 24 * threads) GO1(TO, 24, 256); else if (threads <= 256 && n <= 32 * threads) GO1(TO, 32, 256); \
+        else gated_rmsnorm_kernel<TO, 8><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps); } while (0)
     if (out_dt == DT_F32) GO(float); else if (out_dt == DT_F16) GO(f16); else if (out_dt == DT_BF16) GO(bf16);
     else return LI_BAD_ARG;
 #undef GO

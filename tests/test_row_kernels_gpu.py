@@ -186,6 +186,15 @@ def test_gated_norm_and_polynorm_of_a_row(ops, n):
     _close(ops.polynorm(o, coef, 1e-5, torch.bfloat16), sum(c * d ** k / _rms(d ** k, 1e-5) for k, c in ((1, 0.5), (2, -0.3), (3, 0.2))) + 0.1)
 
 
+# many rows, a workgroup of 256 threads: the last and first of 16, 24 and 32 elements a thread, and of batches of 8
+@pytest.mark.parametrize("n", [4096, 4097, 6144, 6145, 8192, 8193, 10240, 10241])
+def test_gated_norm_of_many_wide_rows(ops, n):
+    o, w, gate = torch.randn(256, n, device=DEV), torch.rand(n, device=DEV) + 0.5, torch.randn(256, n, device=DEV)
+    want = o.double() / _rms(o.double(), 1e-5) * w.double() * torch.sigmoid(gate.double())
+    for dt in (torch.float16, torch.float32):
+        _close(ops.gated_rmsnorm(o, w, gate, 0, 1e-5, dt), want)
+
+
 @pytest.mark.parametrize("terms", [1, 3, 4, 5, 9])
 @pytest.mark.parametrize("width", WIDTHS[:-1])
 def test_average_over_depth_with_its_norms(ops, width, terms):
