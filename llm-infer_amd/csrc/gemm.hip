@@ -440,7 +440,9 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                 for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
             }
         };
-        // (17 to 32 rows: a matrix of less than 32 MiB through the caches; figures at li_gemm_rows)
+        // (17 to 32 rows: a matrix of less than 32 MiB through the caches; figures at li_gemm_rows.  Up to 16 rows past them, us through the
+        // caches and past them, 2 GB of such matrices in turn: 1 row x 1,024 x 1,024 3.5 and 2.9, x 2,048 x 2,048 4.4 and 3.8, 16 rows 4.6 and 4.0, 6.2
+        // and 5.6, x 4,096 x 4,096 10.4 and 9.5; 180 MB, a model that the caches hold: 3.1 and 3.0, 4.0 and 3.9, 3.8 and 4.0, 5.1 and 5.7, 8.4 and 9.3)
         if (MT == 1 || (int64_t)e.N * K >= 1 << 24) fetch(std::true_type{});
         else fetch(std::false_type{});
 #pragma unroll

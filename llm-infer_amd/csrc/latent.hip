@@ -133,7 +133,8 @@ __global__ void average_norms_kernel(const float* __restrict__ hist, int64_t str
     const int n4 = d >> 2;
     // (four terms and the norms' weights on their way at once, with addresses that need no branch: a quad beyond the row is its
     // last one again and counts nowhere; a term after the other: 1 row of 2,048,
-    // five terms and two norms with their launch 5.7 -> 3.9 us, of 4,096 11.7 -> 5.1)
+    // five terms and two norms with their launch 5.7 -> 3.9 us, of 4,096 11.7 -> 5.1; 2,000 rows, three terms: of 1,024 8.4 -> 9.0, of 2,048 16.6 -> 15.6,
+    // of 4,096 29.4 -> 27.9)
     f32x4 xv[V], wv[2][V];
     int at[V];
 #pragma unroll
