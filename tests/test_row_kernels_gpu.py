@@ -186,6 +186,18 @@ def test_gated_norm_and_polynorm_of_a_row(ops, n):
     _close(ops.polynorm(o, coef, 1e-5, torch.bfloat16), sum(c * d ** k / _rms(d ** k, 1e-5) for k, c in ((1, 0.5), (2, -0.3), (3, 0.2))) + 0.1)
 
 
+# a row's sum over every number of waves that a workgroup may have (whole numbers: exact in any order, and a wave left out or taken twice shows)
+@pytest.mark.parametrize("waves", range(1, 17))
+def test_sums_over_any_number_of_waves(ops, waves):
+    n = 256 * waves
+    v = np.random.default_rng(waves).integers(-8, 9, (3, n)).astype(np.float32)
+    v[:, :64] = 16.0 + waves
+    squares = (v * v).sum(1, keepdims=True)
+    assert squares.max() < 2 ** 24
+    out = ops.gated_rmsnorm(torch.from_numpy(v).to(DEV), torch.ones(n, device=DEV), torch.full((3, n), 100.0, device=DEV), 0, 0.0, torch.float32)
+    assert np.array_equal(out.cpu().numpy(), v / np.sqrt(squares / np.float32(n)))     # (the sigmoid of 100 is 1)
+
+
 # many rows, a workgroup of 256 threads: the last and first of 16, 24 and 32 elements a thread, and of batches of 8
 @pytest.mark.parametrize("n", [4096, 4097, 6144, 6145, 8192, 8193, 10240, 10241])
 def test_gated_norm_of_many_wide_rows(ops, n):
