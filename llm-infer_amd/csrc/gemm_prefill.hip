@@ -435,6 +435,11 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     // matrix instructions, and outside them only the wait and the barrier.  (With a half's loads of W behind it and the four
     // of X at the step's head, a burst of loads that the other waves issue too, us, bfloat16: 12,700 x 28,672 x 4,096 2,284 and
     // dealt out 2,238; 33,186 x 16,384 x 2,048 1,712 and 1,675; 12,700 x 4,096 x 4,096 371 and 357.)
+    // Every other group takes W's fragments backwards, so that of the two operands of an instruction one is always the one before's:
+    // on random numbers the chip is held by its power, and an operand that does not change costs less of it (a loop of such
+    // instructions alone, 64 x 128 a wave, float16: both operands changing 1.81 PFLOP/s, the same order in every group 1.86, this one
+    // 1.90; bfloat16 1.95, 1.96, 2.00; of 32x32x16 instructions 1.63 and 1.77).  A prompt of 2,048 tokens on the 8B shape 27.45 -> 27.34
+    // ms, 32 ragged prompts on the 1B shape 66.2 -> 65.8.
     // The LDS reads are written as instructions too, with the waits by hand: the read of b[j] is followed
     // by seven others before b[j] is used, and LDS reads complete in order, so "at most 7 in flight" is the
     // wait before every group of matrix instructions.  (Left to the compiler, each half begins with a wait
@@ -450,7 +455,10 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
     {                                                                                      \
         __builtin_amdgcn_s_waitcnt(0xC07F | ((MJ - 1) << 8));   /* lgkmcnt(MJ - 1), nothing else */ \
         __builtin_amdgcn_sched_barrier(0);                                                 \
-        _Pragma("unroll") for (int i = 0; i < NI; ++i) acc[i][J] = mfma16(A[i], b[J], acc[i][J]); \
+        _Pragma("unroll") for (int t = 0; t < NI; ++t) {                                   \
+            const int i = (J) & 1 ? NI - 1 - t : t;                                        \
+            acc[i][J] = mfma16(A[i], b[J], acc[i][J]);                                     \
+        }                                                                                  \
         __builtin_amdgcn_sched_barrier(0);                                                 \
         WREG_READ(J, NEXT)                                                                 \
         LOADS(std::integral_constant<int, J>{});                                           \
