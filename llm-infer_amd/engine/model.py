@@ -156,13 +156,32 @@ class DecoderModel(Part):
                 for e in self.schedule for m in self.layer_mixers[e.layer]
                 for j, spec in enumerate(cache_specs_of(m))] + self._embedding_specs()
 
-    def _norms_of_entry(self, i) -> list:
+    def _views_of(self, i, cache) -> list:
+        """One cache view for each mixer of schedule entry ``i``, or the list of its views for one that asks several things of the cache."""
+        return [[cache.view(u) for u in self._seen[i, k]] if multi else cache.view(self._seen[i, k][0])
+                for k, multi in enumerate(self._multi[self.schedule[i].layer])]
+
+    def _norms_of_entry(self, i, ctx, cache) -> tuple:
         """The RMS norms (weight, eps, type) that read the residual stream as the layer of schedule entry ``i`` begins, where
-        the layer says so (``input_norms``) and nothing rewrites the stream ahead of it: at most two, the others run by themselves."""
+        the layer says so (``input_norms``) and nothing rewrites the stream ahead of it: at most two, the others run by themselves.  With them
+        the short convolution that reads one of them (``input_convs``) in a step of one token a sequence, as ``ops.average_norms`` takes
+        it, or None."""
         if i >= len(self.schedule) or self._before[i] is not None:
-            return []
-        asks = getattr(self.layers[self.schedule[i].layer], "input_norms", None)
-        return [(n.weight, n.eps, dt) for n, dt in (asks() if asks else ()) if isinstance(n, RMSNorm) and n.weight is not None][:2]
+            return [], None
+        entry = self.schedule[i]
+        layer = self.layers[entry.layer]
+        if not hasattr(layer, "input_norms"):
+            return [], None
+        convs = [None] * len(layer.sublayers)
+        if ctx.n_tokens == ctx.n_seqs and entry.cache_from is None and hasattr(layer, "input_convs"):
+            convs = layer.input_convs(self._views_of(i, cache))
+        norms, conv = [], None
+        for (n, dt), c in zip(layer.input_norms(), convs):
+            if isinstance(n, RMSNorm) and n.weight is not None and len(norms) < 2:
+                if c is not None and conv is None and ops.norm_conv_fits(*c[:2]):
+                    conv = (len(norms),) + tuple(c)
+                norms.append((n.weight, n.eps, dt))
+        return norms, conv
 
     # -- the forward pass of one step ---------------------------------------
     def forward(self, ctx, cache) -> torch.Tensor:
@@ -176,9 +195,9 @@ class DecoderModel(Part):
             # the stream's values side by side: the embedding's output, then the result of every run that an
             # ``after`` part follows (the run works in place on the row that the part before it has written)
             history = torch.empty((self._n_after + 2,) + tuple(x0.shape), dtype=torch.float32, device=x0.device)
-            x, n_hist, norms = history[1], 1, self._norms_of_entry(0)
+            x, n_hist, (norms, conv) = history[1], 1, self._norms_of_entry(0, ctx, cache)
             if norms and ops.average_norms_fit(x0, None, x, norms):
-                ops.average_norms(x0.unsqueeze(0), 1, None, x, norms, also=history[0])
+                ops.average_norms(x0.unsqueeze(0), 1, None, x, norms, also=history[0], conv=conv, ctx=ctx)
             else:
                 history[0].copy_(x0)
                 x.copy_(x0)
@@ -191,9 +210,7 @@ class DecoderModel(Part):
                 x = part.forward(x, x0, ctx, e.pass_no) if getattr(part, "takes_pass", False) else part.forward(x, x0, ctx)
             elif x is x0 and self.stream_parts and history is None:
                 x = ops.copy_rows(x0)            # the layers add in place, and a later part reads the embedding's output
-            # one view for a mixer, or the list of its views for one that asks several things of the cache
-            views = [[cache.view(u) for u in self._seen[i, k]] if multi else cache.view(self._seen[i, k][0])
-                     for k, multi in enumerate(self._multi[e.layer])]
+            views = self._views_of(i, cache)
             layer = self.layers[e.layer]
             if getattr(layer, "takes_next_norm", False):
                 # the norm that reads the residual stream after this layer: the next layer's first
@@ -211,8 +228,8 @@ class DecoderModel(Part):
             if self._after[i] is not None:
                 n_hist += 1                      # x is history[n_hist - 1], now a finished value of the stream
                 part = self.stream_parts[self._after[i]]
-                norms = self._norms_of_entry(i + 1) if getattr(part, "takes_norms", False) else ()
-                x = part.forward_after(history, n_hist, history[n_hist], ctx, **({"norms": norms} if norms else {}))
+                norms, conv = self._norms_of_entry(i + 1, ctx, cache) if getattr(part, "takes_norms", False) else ([], None)
+                x = part.forward_after(history, n_hist, history[n_hist], ctx, **({"norms": norms, "conv": conv} if norms else {}))
         if ctx.n_want == 0:
             return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=x.device)
         h = self.final_norm.forward(x, ctx.want_rows)

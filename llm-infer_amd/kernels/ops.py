@@ -178,6 +178,8 @@ def _drop_row_stats(x) -> None:
             x._li_rows = None
         if getattr(x, "_li_normed", None) is not None:
             x._li_normed = None
+        if getattr(x, "_li_convolved", None) is not None:      # (its history has moved on: it cannot be taken again)
+            raise KernelError("rows are written over before the convolution that was taken of their norm has been read")
         x = getattr(x, "_base", None)
 
 
@@ -193,6 +195,27 @@ def prepared_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype):
 
 # (the weight tensor says which norm it is: a layer norm that a pass has taken along is found in the same way)
 prepared_norm = prepared_rmsnorm
+
+
+class ConvolvedRows:
+    """What a part reads that begins with a short convolution over its normed rows, where the pass before has taken norm and
+    convolution along (``average_norms``): ``rows`` in the part's type.  The sequences' histories are up to date."""
+
+    def __init__(self, rows):
+        self.rows = rows
+
+
+def prepared_conv(x: torch.Tensor, w: torch.Tensor, eps: float, conv_w: torch.Tensor, history: torch.Tensor):
+    """The ``ConvolvedRows`` that ``average_norms`` has left of the norm (``w``, ``eps``) of ``x`` and the convolution ``conv_w`` with
+    this ``history``, once; None where it has taken none."""
+    rec = getattr(x, "_li_convolved", None)
+    if rec is None:
+        return None
+    u, weight, rec_eps, taps, state, version = rec
+    _need(weight is w and rec_eps == eps and taps is conv_w and state == history.data_ptr() and version == x._version,
+          "the convolution taken of these rows' norm is not the one that is asked for")
+    x._li_convolved = None
+    return ConvolvedRows(u)
 
 
 def lazy_rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype):
@@ -1803,10 +1826,17 @@ class _RowNorm(ctypes.Structure):
     _fields_ = [("w", c_void_p), ("out", c_void_p), ("eps", c_float), ("dt", c_int)]
 
 
-def average_norms(history: torch.Tensor, n: int, weights, out: torch.Tensor, norms, also=None) -> torch.Tensor:
+class _NormConv(ctypes.Structure):
+    _fields_ = [("w", c_void_p), ("hist", c_void_p), ("pos", c_void_p), ("tok_slot", c_void_p), ("out", c_void_p), ("dt", c_int),
+                ("taps", c_int), ("of", c_int)]
+
+
+def average_norms(history: torch.Tensor, n: int, weights, out: torch.Tensor, norms, also=None, conv=None, ctx=None) -> torch.Tensor:
     """``depth_average`` (``weights`` None: the rows of ``history`` [1, T, width] as they are) that also takes the RMS norms which
     read the finished rows next, ``norms``: up to two (weight, eps, dtype).  ``prepared_rmsnorm`` finds them as long as nothing
-    writes into ``out``.  ``also``: a second tensor that receives the rows."""
+    writes into ``out``.  ``also``: a second tensor that receives the rows.  ``conv`` (index of a norm, weight [width, taps], history, dtype), in
+    a step ``ctx`` of one token a sequence: that norm's rows go through ``conv_add`` on the way and are not stored themselves;
+    ``prepared_conv`` finds the result."""
     _dev(history, weights, out, also, *(w for w, _, _ in norms))
     rows, d = out.shape
     _need(history.dtype == torch.float32 and history.dim() == 3 and 1 <= n <= history.shape[0], "average_norms: float32 [runs, T, width]")
@@ -1816,11 +1846,26 @@ def average_norms(history: torch.Tensor, n: int, weights, out: torch.Tensor, nor
         _need(t.dtype == torch.float32 and tuple(t.shape) == tuple(history.shape[1:]), "average_norms out: float32 [T, width]")
         _drop_row_stats(t)
     _need(1 <= len(norms) <= 2 and all(w.dtype == torch.float32 and w.shape == (d,) for w, _, _ in norms), "average_norms: one or two float32 weights [width]")
-    made = [torch.empty(out.shape, dtype=dt, device=out.device) for _, _, dt in norms]
-    recs = [_RowNorm(w.data_ptr(), m.data_ptr(), eps, DT[m.dtype]) for (w, eps, _), m in zip(norms, made)] + [_RowNorm()]
+    of, cv = -1, None
+    if conv is not None:
+        of, cw, state, dtype = conv
+        _dev(cw, state)
+        _need(0 <= of < len(norms) and cw.dtype == torch.float32 and cw.dim() == 2 and cw.shape[0] == d and cw.is_contiguous()
+              and state.dtype == torch.float32 and tuple(state.shape[1:]) == (cw.shape[1] - 1, d) and state.is_contiguous(),
+              "average_norms: a convolution [width, taps] of one of the norms, with its history")
+        _need(ctx.n_tokens == ctx.n_seqs == rows, "average_norms: a convolution rides along where every sequence brings one token")
+        _i32(ctx.pos, rows, "positions")
+        _i32(ctx.tok_slot, rows, "slots")
+        u = torch.empty(out.shape, dtype=dtype, device=out.device)
+        cv = _NormConv(cw.data_ptr(), state.data_ptr(), ctx.pos.data_ptr(), ctx.tok_slot.data_ptr(), u.data_ptr(), DT[dtype], cw.shape[1], of)
+    made = [torch.empty(out.shape, dtype=dt, device=out.device) if k != of else None for k, (_, _, dt) in enumerate(norms)]
+    recs = [_RowNorm(w.data_ptr(), m.data_ptr() if m is not None else None, eps, DT[dt]) for (w, eps, dt), m in zip(norms, made)] + [_RowNorm()]
     _check(hybrid().li_average_norms(_ptr(history), c_int64(history.stride(0)), _ptr(weights), n, _ptr(out), _ptr(also), rows, d,
-                                     ctypes.byref(recs[0]), ctypes.byref(recs[1]), _stream()), "average_norms")
-    out._li_normed = [(m, w, float(eps), out._version) for m, (w, eps, _) in zip(made, norms)]
+                                     ctypes.byref(recs[0]), ctypes.byref(recs[1]), ctypes.byref(cv) if cv is not None else None, _stream()),
+           "average_norms")
+    out._li_normed = [(m, w, float(eps), out._version) for m, (w, eps, _) in zip(made, norms) if m is not None]
+    if cv is not None:
+        out._li_convolved = (u, norms[of][0], float(norms[of][1]), cw, state.data_ptr(), out._version)
     return out
 
 
@@ -1830,6 +1875,11 @@ def average_norms_fit(history, weights, out, norms) -> bool:
     tensors = [history, out] + [w for w, _, _ in norms]
     return (1 <= len(norms) <= 2 and d % 4 == 0 and d <= 8192 and all(t.data_ptr() % 16 == 0 for t in tensors)
             and all(w.dtype == torch.float32 and w.shape == (d,) for w, _, _ in norms))
+
+
+def norm_conv_fits(weight, history) -> bool:
+    """Whether ``average_norms`` takes a convolution of this weight [width, taps] and history along."""
+    return 2 <= weight.shape[1] <= 4 and weight.data_ptr() % 16 == 0 and history.data_ptr() % 16 == 0 and weight.is_contiguous() and history.is_contiguous()
 
 
 def softcap(x: torch.Tensor, cap: float) -> torch.Tensor:

@@ -106,13 +106,29 @@ class ParallelBlock(Block):
         """What reads the residual stream first: (norm, type of its result) of every branch."""
         return [(s.norm, torch.float32 if getattr(s.part, "reads_float32", False) else s.norm.dtype) for s in self.sublayers]
 
+    def input_convs(self, cache_views):
+        """For every branch the short convolution that its part begins with, (weight, history, type), or None."""
+        views = iter(cache_views)
+        out = []
+        for s in self.sublayers:
+            view = next(views) if s.role == "mixer" else None
+            out.append(s.part.input_conv(view) if hasattr(s.part, "input_conv") else None)
+        return out
+
+    def _normed(self, s, x, view):
+        if hasattr(s.part, "input_conv"):
+            ready = ops.prepared_conv(x, s.norm.weight, s.norm.eps, *s.part.input_conv(view)[:2])
+            if ready is not None:
+                return ready
+        return s.norm.forward(x, out_dtype=torch.float32) if getattr(s.part, "reads_float32", False) else s.norm.forward(x)
+
     def forward(self, x, ctx, cache_views, owns_cache=True):
         views = iter(cache_views)
         ops.expect_norm(x, None)                 # the rows are complete only after the last part: no norm rides along
-        normed = [s.norm.forward(x, out_dtype=torch.float32) if getattr(s.part, "reads_float32", False) else s.norm.forward(x)
-                  for s in self.sublayers]
-        for s, h in zip(self.sublayers, normed):
-            _run_part(s, h, ctx, next(views) if s.role == "mixer" else None, x, owns_cache)
+        each = [next(views) if s.role == "mixer" else None for s in self.sublayers]
+        normed = [self._normed(s, x, view) for s, view in zip(self.sublayers, each)]
+        for s, h, view in zip(self.sublayers, normed, each):
+            _run_part(s, h, ctx, view, x, owns_cache)
 
 
 def _run_part(s, h, ctx, view, out, owns_cache):

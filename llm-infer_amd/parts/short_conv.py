@@ -43,12 +43,19 @@ class ConvMixer(Part):
     def cache_specs(self):
         return [StateSpec((max(self.taps - 1, 1), self.hidden_size), "float32")] + cache_specs_of(self.inner)
 
+    def input_conv(self, views):
+        """What the convolution needs beside the normed rows: (weight, history, type of its result)."""
+        return self.weight, views[0].state, self.dtype
+
     def forward(self, h, ctx, views, residual, owns_cache=True):
-        """``h``: the normed rows in float32; the inner mixer's result is added into ``residual``."""
+        """``h``: the normed rows in float32, or ``ops.ConvolvedRows``; the inner mixer's result is added into ``residual``."""
         if not owns_cache:
             raise ValueError("a mixer behind a short convolution keeps a state of its own in every run")
-        if h.dtype != torch.float32:
-            raise ValueError("the short convolution reads float32 rows")
-        u = ops.conv_add(h, self.weight, views[0].state, ctx, self.dtype)
+        if isinstance(h, ops.ConvolvedRows):                   # (the pass that took the norm has convolved its rows)
+            u = h.rows
+        else:
+            if h.dtype != torch.float32:
+                raise ValueError("the short convolution reads float32 rows")
+            u = ops.conv_add(h, self.weight, views[0].state, ctx, self.dtype)
         inner_views, _ = views_for(self.inner, views, 1)
         self.inner.forward(u, ctx, inner_views, residual, owns_cache)

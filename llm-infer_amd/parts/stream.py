@@ -81,13 +81,14 @@ class DepthAverage(Part):
     def bind(self, tensors):
         self.weight = tensors[self.name]
 
-    takes_norms = True          # forward_after accepts ``norms``
+    takes_norms = True          # forward_after accepts ``norms`` and ``conv``
 
-    def forward_after(self, history, n, out, ctx, norms=()):
+    def forward_after(self, history, n, out, ctx, norms=(), conv=None):
         """``history`` float32 [runs, T, width] of which the first ``n`` hold X_0 .. X_{n-1}; writes ``out``.  ``norms``: up to two
-        RMS norms (weight, eps, type) that read it next, taken in the same pass where its kernel takes them."""
+        RMS norms (weight, eps, type) that read it next, taken in the same pass where its kernel takes them; ``conv``: a short
+        convolution over one of them (``ops.average_norms``)."""
         if n != self.n_terms:
             raise ValueError(f"depth average over {self.n_terms} terms after {n} values of the stream")
         if norms and ops.average_norms_fit(history, self.weight, out, norms):
-            return ops.average_norms(history, n, self.weight, out, norms)
+            return ops.average_norms(history, n, self.weight, out, norms, conv=conv, ctx=ctx)
         return ops.depth_average(history, n, self.weight, out)

@@ -681,3 +681,41 @@ def test_matrix_memory_of_one_token_is_the_walk(lib, H, d, dv):
         assert torch.equal(a, b)
     for s in (1, 2):
         assert torch.equal(got[0][1][s], S0[s]) and torch.equal(got[0][2][s], n0[s])
+
+
+@pytest.mark.parametrize("rows,width,taps", [(1, 4, 2), (9, 64, 3), (3, 260, 4), (8, 2048, 3), (2, 4100, 4), (3, 8192, 2)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_norm_with_the_convolution_that_reads_it(lib, rows, width, taps, dtype):
+    """A norm and the short convolution behind it in the pass over the rows: result and histories are, bit for bit, those of the
+    norm kernel and ``conv_add``, from a sequence's first token on; what was taken is found once, and only as what it is."""
+    from types import SimpleNamespace
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows * width + taps)
+    cw, nw = torch.randn(width, taps, generator=g).to(DEV), [torch.randn(width, generator=g).to(DEV) for _ in range(2)]
+    slots = torch.randperm(rows + 2, generator=g)[:rows].to(torch.int32).to(DEV)
+    states = [torch.zeros(rows + 2, taps - 1, width, device=DEV) for _ in range(2)]
+    assert ops.norm_conv_fits(cw, states[0]) and not ops.norm_conv_fits(torch.zeros(width, 5, device=DEV), states[0])
+    for step in range(taps + 1):
+        pos = torch.tensor([step + (i if step else 0) for i in range(rows)], dtype=torch.int32, device=DEV)
+        ctx = SimpleNamespace(pos=pos, tok_slot=slots, seq_slot=slots, n_tokens=rows, n_seqs=rows)
+        x = torch.randn(1, rows, width, generator=g).to(DEV)
+        for of in (0, 1):
+            norms = [(nw[0], 1e-5, torch.float32), (nw[1], 1e-6, dtype)]
+            if of:
+                norms.reverse()
+            mine, theirs = states[0].clone(), states[1].clone()
+            out = torch.empty_like(x[0])
+            ops.average_norms(x, 1, None, out, norms, conv=(of, cw, mine, dtype), ctx=ctx)
+            w, eps, _ = norms[of]
+            got = ops.prepared_conv(out, w, eps, cw, mine).rows
+            want = ops.conv_add(ops.rmsnorm(x[0], w, eps, torch.float32), cw, theirs, ctx, dtype)
+            assert torch.equal(got, want) and torch.equal(mine, theirs) and torch.equal(out, x[0])
+            other = norms[1 - of]
+            assert torch.equal(ops.prepared_rmsnorm(out, *other), ops.rmsnorm(x[0], *other))
+            assert ops.prepared_conv(out, w, eps, cw, mine) is None and ops.prepared_rmsnorm(out, w, eps, torch.float32) is None or w is other[0]
+        states = [mine, theirs]
+    ops.average_norms(x, 1, None, out, norms, conv=(1, cw, mine, dtype), ctx=ctx)
+    with pytest.raises(ops.KernelError):
+        ops.prepared_conv(out, nw[1], 1e-3, cw, mine)
+    with pytest.raises(ops.KernelError):
+        ops.average_norms(x, 1, None, out, norms)
