@@ -194,6 +194,14 @@ __device__ __forceinline__ float gate_activation(float g, bool gelu) {
     return g / (1.f + expf(-g));
 }
 
+// The activations of feed-forwards without a gate.  act: 0 gelu (erf), 1 gelu (tanh), 2 silu, 3 the square of relu.
+__device__ __forceinline__ float plain_activation(float z, int act) {
+    if (act == 3) { const float r = fmaxf(z, 0.f); return r * r; }
+    if (act == 2) return z / (1.f + expf(-z));
+    if (act == 1) return gate_activation(z, true);
+    return 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
+}
+
 // A score's soft cap, c tanh(x / c), with a = 2 log2(e) / c beside c: tanh z = 1 - 2 / (e^(2z) + 1) by the hardware's
 // 2^x and reciprocal (an error of some 1e-7 c; for large |x| the exponential becomes infinite or 0 and the result +-c).
 __device__ __forceinline__ float soft_cap(float x, float c, float a) {

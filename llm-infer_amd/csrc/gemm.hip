@@ -307,7 +307,7 @@ struct XGroups {
 // quarter of them, four tokens two thirds (4,096 wide, experts of 3,584, a step of four tokens 0.91 -> 0.79 ms).
 enum { EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
 struct ExpertBlocks {
-    static constexpr bool chosen_only = true;
+    static constexpr bool chosen_only = true, activated = false;
     const float* w;
     int cols, n, ff, over;
 };
@@ -340,10 +340,32 @@ __device__ __forceinline__ void store_weighted(const Epilogue& e, const ExpertBl
     *(v2*)((T*)e.C + (int64_t)m * (e.N >> 1) + col) = v2{h[0], h[1]};
 }
 
-// EB: ExpertBlocks, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
+// The up product of experts without a gate (or, with n 0 and no weights, of a feed-forward without one): the hidden values themselves, act(weight *
+// sum) or weight * act(sum), 0 for a weight of 0, what expert_act_kernel makes of stored sums.  `over` EXPERTS_IN_N, or 0: every expert is
+// read.  Up to 16 rows, where the kernel behind the product is a launch and little else (8 experts of 1,024 and one of 2,048, width 2,048, 8
+// rows: a launch of 4.9 us in a recorded step).
+struct ExpertActs : ExpertBlocks {
+    static constexpr bool activated = true;
+    int act, on_input;
+};
+
+// Row m, rows n .. n + 3 of W.
+template <class T>
+__device__ __forceinline__ void store_activated(const Epilogue& e, const ExpertActs& x, int m, int n, const float* v) {
+    if (m >= e.M || n >= e.N) return;
+    typename Vec<T>::v4 h;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const float w = x.w ? x.w[m * x.cols + min((n + j) / x.ff, x.n)] : 1.f;
+        h[j] = from_f32<T>(w == 0.f ? 0.f : x.on_input ? plain_activation(w * v[j], x.act) : w * plain_activation(v[j], x.act));
+    }
+    *(typename Vec<T>::v4*)((T*)e.C + (int64_t)m * e.N + n) = h;
+}
+
+// EB: ExpertBlocks, ExpertActs, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
 // cost a whole matrix's product some 0.3 us, 1% of a decode step.)
 struct NoExperts {
-    static constexpr bool chosen_only = false;
+    static constexpr bool chosen_only = false, activated = false;
 };
 
 template <class T, int NT, int MT, int KW, class EB, bool HALF = false>
@@ -367,7 +389,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     const int per = ((steps + KW - 1) / KW + SL - 1) / SL * SL;
     int s_begin = wave * per, s_end = min(steps, s_begin + per), s_next = U * SL;
     unsigned long long chosen = ~0ull;
-    if constexpr (EXPERTS) {
+    if constexpr (EXPERTS) if (!EB::activated || ex.over) {
         chosen = chosen_experts(ex, e.M);
         if (ex.over == EXPERTS_IN_K) {               // the waves take turns, so that what is left out is left out for all of them
             s_begin = wave * U * SL;
@@ -530,7 +552,10 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
 #pragma unroll
         for (int j = 0; j < MT; ++j) {
             float v[4] = {acc[t][j][0], acc[t][j][1], acc[t][j][2], acc[t][j][3]};
-            if constexpr (EXPERTS) if (ex.over == EXPERTS_GATED) {
+            if constexpr (EB::activated) {
+                if (mine) store_activated<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 8 * half + 4 * g, v);
+                continue;
+            } else if constexpr (EXPERTS) if (ex.over == EXPERTS_GATED) {
                 if (mine) store_weighted<T>(e, ex, 16 * j + r, (tile0 + t) * 16 + 8 * half + 4 * g, v);
                 continue;
             }
@@ -906,7 +931,9 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     if (rc) return rc;
     const int mt = (M + 15) / 16;
     int blocks = 0;
-    gemv_tiled_shape(M, N, K, nt, kw, blocks, !EB::chosen_only && !ro && !rsc);
+    bool plain = !EB::chosen_only && !ro && !rsc;
+    if constexpr (EB::activated) plain = !ex.over && !rsc;
+    gemv_tiled_shape(M, N, K, nt, kw, blocks, plain);
     if (kw < 2 || (nt < 0 && M > 8)) return LI_BAD_ARG;
     const RowsOut no_out{};
     const RowScale no_scale{};
@@ -922,7 +949,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
 #define PICK(T)                                           \
     do {                                                  \
         if (nt < 0 && kw == 8) LAUNCH(T, 1, 1, 8, true);  \
-        else if (nt < 0 && kw == 4 && !EB::chosen_only) LAUNCH(T, 1, 1, 4, true); \
+        else if (nt < 0 && kw == 4 && (!EB::chosen_only || EB::activated)) LAUNCH(T, 1, 1, 4, true); \
         else if (nt < 0) return LI_BAD_ARG;               \
         else if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
         else if (mt == 1 && nt == 2) PICK_KW(T, 2, 1);    \
@@ -965,6 +992,19 @@ extern "C" int li_gemv_tiled_experts(const void* X, const void* Wt, int dt, void
     if (mode == EPI_CLAMPGLU && (!rs || ((const GluParams*)rs)->bias)) return LI_BAD_ARG;
     return gemv_tiled(X, Wt, dt, C, out_dt, mode, M, N, K, 0, 0, rs, ro, nullptr, XGroups{0, 1, 0},
                       ExpertBlocks{weights, cols, n, ff, over}, stream);
+}
+
+// The hidden values of experts without a gate (see ExpertActs), for at most 16 rows and a multiple of 4 rows of W, in the type of X; `weights` null: one
+// feed-forward, n 0.  skip: an expert that no token chose is not read.  rsc as for li_gemv_tiled.
+extern "C" int li_gemv_tiled_act(const void* X, const void* Wt, int dt, void* C, int M, int N, int K, const RowScale* rsc, const float* weights,
+                                 int cols, int n, int ff, int skip, int act, int on_input, hipStream_t stream) {
+    if (M > 16 || (N & 3) || ((uintptr_t)C & 7) || n < 0 || ff < 1 || act < 0 || act > 3) return LI_BAD_ARG;
+    if (weights ? (cols < n || cols > 64 || (int64_t)n * ff > N || (cols == n && (int64_t)n * ff != N)) : (n || skip)) return LI_BAD_ARG;
+    ExpertActs ex;
+    static_cast<ExpertBlocks&>(ex) = ExpertBlocks{weights, cols, n, ff, skip ? EXPERTS_IN_N : 0};
+    ex.act = act;
+    ex.on_input = on_input;
+    return gemv_tiled(X, Wt, dt, C, dt, EPI_STORE, M, N, K, 0, 0, nullptr, nullptr, rsc, XGroups{0, 1, 0}, ex, stream);
 }
 
 // X [groups, M, K]: the rows of W from g * group_rows on (a multiple of 32; the last group: all that are left) against X[g].

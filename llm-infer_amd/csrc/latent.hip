@@ -1198,13 +1198,6 @@ extern "C" int li_gated_head_norm(const float* y, const float* w, const float* g
 // product is linear); else out = weight * act(z).  A weight of zero gives zero.  act: 0 gelu (erf), 1 gelu (tanh),
 // 2 silu, 3 the square of relu.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float lt_act(float z, int act) {
-    if (act == 3) { const float r = fmaxf(z, 0.f); return r * r; }
-    if (act == 2) return z / (1.f + expf(-z));
-    if (act == 1) return gate_activation(z, true);
-    return 0.5f * z * (1.f + erff(z * 0.70710678118654752f));
-}
-
 template <class T>
 __global__ void expert_act_kernel(const float* __restrict__ z, const float* __restrict__ wgt, int wcols,
                                   const int* __restrict__ idx, int col, T* __restrict__ out, int n_blocks, int ff, int tail,
@@ -1216,7 +1209,7 @@ __global__ void expert_act_kernel(const float* __restrict__ z, const float* __re
         const int e = col >= 0 ? col : (i < n_blocks * ff ? i / ff : n_blocks);
         const float w = wgt ? wgt[r * wcols + e] : 1.f;
         const float v = z[row * cols + i];
-        out[row * cols + i] = from_f32<T>(w == 0.f ? 0.f : (on_input ? lt_act(w * v, act) : w * lt_act(v, act)));
+        out[row * cols + i] = from_f32<T>(w == 0.f ? 0.f : (on_input ? plain_activation(w * v, act) : w * plain_activation(v, act)));
     }
 }
 

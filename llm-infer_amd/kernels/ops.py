@@ -515,6 +515,34 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
     return out
 
 
+def activated_fits(x, w, n_experts: int, n_out: int) -> bool:
+    """True if ``linear_activated`` takes the product: at most 16 rows of a 16-bit model against a tiled weight."""
+    return (is_tiled(w) and x.dtype == w.dtype and x.shape[0] <= 16 and n_out % 4 == 0 and n_experts + 1 <= 64
+            and (isinstance(x, LazyNorm) or x.data_ptr() % 16 == 0) and w.data_ptr() % 16 == 0)
+
+
+def linear_activated(x, w, kind: str, weights=None, n_blocks: int = 0, ff: int = 1, on_input: bool = False, skip: bool = False) -> torch.Tensor:
+    """act(X W^T) in the type of ``x``, or with ``weights`` float32 [m, blocks (+ 1)] the hidden rows of experts without a gate side by side,
+    as ``expert_act`` makes them of the product's float32 sums.  ``skip``: experts that no token chose are not read."""
+    lazy = x if isinstance(x, LazyNorm) else None
+    if lazy is not None:
+        x = lazy.xw
+    _dev(x, w, weights)
+    m, k = x.shape
+    n = matrix_shape(w)[0]
+    _need(activated_fits(x, w, n_blocks, n) and kind in ACTIVATIONS and matrix_shape(w)[1] == k, "linear_activated: few rows against a tiled weight")
+    _need(weights is None or (weights.dtype == torch.float32 and weights.dim() == 2 and weights.shape[0] == m and weights.is_contiguous()),
+          "linear_activated: float32 weights, a row for every token")
+    out = torch.empty((m, n), dtype=x.dtype, device=x.device)
+    if m == 0:
+        return out
+    rsc = _finish_norm(lazy, x) if lazy is not None else None
+    _check(core().li_gemv_tiled_act(_ptr(x), _ptr(w), DT[x.dtype], _ptr(out), m, n, k, ctypes.byref(rsc) if rsc is not None else None,
+                                    _ptr(weights), weights.shape[1] if weights is not None else 0, n_blocks, ff, int(bool(skip)),
+                                    ACTIVATIONS[kind], int(bool(on_input)), _stream()), "gemv_tiled_act")
+    return out
+
+
 def linear_groups(x: torch.Tensor, w, group_rows: int) -> torch.Tensor:
     """Several products of few rows as one launch: ``x`` [groups, m <= 32, K] against a tiled weight whose rows from g *
     ``group_rows`` on (a multiple of 32; the last group: all that are left) read x[g].  Returns float32 [m, N]."""

@@ -145,6 +145,8 @@ class DenseMLP(Part):
     def _hidden(self, h):
         if self.activation in ops.EPI_ACTS:          # on the product's float32 sums, in its epilogue
             return ops.linear(h, self.w_up, ops.EPI_BIAS, out_dtype=self.dtype, params=ops.glu_params(act=self.activation))
+        if ops.activated_fits(h, self.w_up, 0, self.intermediate_size):
+            return ops.linear_activated(h, self.w_up, self.activation)
         return ops.activation(ops.linear(h, self.w_up, out_dtype=torch.float32), self.activation, self.dtype)
 
     def forward(self, h, residual):
@@ -348,6 +350,8 @@ class RoutedExperts(Part):
 
     def _hidden(self, rows, w_up, weights, idx, col, blocks, ff, tail, experts=None):
         """The hidden rows of experts without a gate: the activation of the up product's sums, with the routing weight."""
+        if idx is None and col is None and ops.activated_fits(rows, w_up, blocks, blocks * ff + tail):
+            return ops.linear_activated(rows, w_up, self.activation, weights, blocks, ff, self.on_input, experts is not None)
         z = ops.linear(rows, w_up, out_dtype=torch.float32, experts=experts)
         return ops.expert_act(z, weights, blocks, ff, tail, self.activation, self.on_input, self.dtype, idx, col)
 

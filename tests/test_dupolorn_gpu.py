@@ -719,3 +719,38 @@ def test_norm_with_the_convolution_that_reads_it(lib, rows, width, taps, dtype):
         ops.prepared_conv(out, nw[1], 1e-3, cw, mine)
     with pytest.raises(ops.KernelError):
         ops.average_norms(x, 1, None, out, norms)
+
+
+@pytest.mark.parametrize("rows", [1, 2, 8, 9, 16])
+@pytest.mark.parametrize("kind", ["relu2", "gelu", "gelu_tanh", "silu"])
+def test_hidden_rows_in_the_up_product(lib, rows, kind):
+    """Activation and routing weight in the product's epilogue: bit for bit the product, stored, and the kernel behind it; blocks of
+    every width, weights of zero, infinite sums; tiles that the last block ends in."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows)
+    for dtype, width, blocks, ff, tail in ((torch.float16, 128, 4, 20, 44), (torch.bfloat16, 2048, 8, 256, 512), (torch.float16, 96, 3, 7, 3),
+                                           (torch.bfloat16, 64, 0, 1, 4096 + 20)):
+        n = blocks * ff + tail
+        x = torch.randn(rows, width, generator=g).to(DEV, dtype)
+        w = torch.randn(n, width, generator=g).to(DEV, dtype)
+        if dtype == torch.bfloat16:
+            w[n // 2] *= 1e37                                     # (some of its sums are infinite)
+        tw = ops.prepare_weight(w)
+        assert ops.is_tiled(tw) and ops.activated_fits(x, tw, blocks, n)
+        if not blocks:
+            got = ops.linear_activated(x, tw, kind)
+            want = ops.activation(ops.linear(x, tw, out_dtype=torch.float32), kind, dtype)
+            assert torch.equal(got, want) or torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num())
+            continue
+        weights = torch.rand(rows, blocks + 1, generator=g)
+        weights[:, :blocks][torch.rand(rows, blocks, generator=g) < 0.5] = 0.0
+        weights = weights.to(DEV)
+        z = ops.linear(x, tw, out_dtype=torch.float32)
+        for on_input in (False, True):
+            want = ops.expert_act(z, weights, blocks, ff, tail, kind, on_input, dtype)
+            for skip in (False, True):
+                got = ops.linear_activated(x, tw, kind, weights, blocks, ff, on_input, skip)
+                if skip:                                          # (whole tiles of W: other orders of a sum)
+                    zs = ops.linear(x, tw, out_dtype=torch.float32, experts=(weights, blocks, ff, ops.EXPERTS_IN_N))
+                    want = ops.expert_act(zs, weights, blocks, ff, tail, kind, on_input, dtype)
+                assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(), want.nan_to_num()), (dtype, on_input, skip)
