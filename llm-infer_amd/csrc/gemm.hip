@@ -307,7 +307,7 @@ struct XGroups {
 // quarter of them, four tokens two thirds (4,096 wide, experts of 3,584, a step of four tokens 0.91 -> 0.79 ms).
 enum { EXPERTS_IN_K = 1, EXPERTS_IN_N = 2, EXPERTS_GATED = 3 };
 struct ExpertBlocks {
-    static constexpr bool chosen_only = true, activated = false;
+    static constexpr bool chosen_only = true, activated = false, second = false;
     const float* w;
     int cols, n, ff, over;
 };
@@ -362,10 +362,20 @@ __device__ __forceinline__ void store_activated(const Epilogue& e, const ExpertA
     *(typename Vec<T>::v4*)((T*)e.C + (int64_t)m * e.N + n) = h;
 }
 
-// EB: ExpertBlocks, ExpertActs, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
+// A second product of as many rows behind the first's workgroups: mixers that run side by side end with one each, and a launch of its own
+// is what a short one costs most (us in a recorded chain, two launches and one: 1 row x 4,096 x 4,096 and 4,096 x 2,048 12.2 and 9.6, x 2,048 x
+// 2,048 twice 7.6 and 5.2, 8 rows 14.4 and 11.1, 8.5 and 6.5, 16 rows 17.4 and 12.7, 11.6 and 6.3).
+struct TwoProducts {
+    static constexpr bool chosen_only = false, activated = false, second = true;
+    const void *X, *W;
+    float* C;
+    int K, N, blocks;            // `blocks`: workgroups of the first
+};
+
+// EB: ExpertBlocks, ExpertActs, TwoProducts, or NoExperts for every other product.  (A kernel of its own: asked at run time, that there are no experts
 // cost a whole matrix's product some 0.3 us, 1% of a decode step.)
 struct NoExperts {
-    static constexpr bool chosen_only = false, activated = false;
+    static constexpr bool chosen_only = false, activated = false, second = false;
 };
 
 template <class T, int NT, int MT, int KW, class EB, bool HALF = false>
@@ -373,7 +383,18 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                                                              int K, Epilogue e, RowsOut ro, RowScale rsc, XGroups xg,
                                                              EB ex) {
     constexpr bool EXPERTS = EB::chosen_only;
-    const int tile0 = HALF ? blockIdx.x >> 1 : blockIdx.x * NT;
+    int block = blockIdx.x;
+    if constexpr (EB::second) {
+        if (block >= ex.blocks) {
+            block -= ex.blocks;
+            X = (const T*)ex.X;
+            Wt = (const T*)ex.W;
+            K = ex.K;
+            e.C = ex.C;
+            e.N = ex.N;
+        }
+    }
+    const int tile0 = HALF ? block >> 1 : block * NT;
     if (xg.rows) X += min(tile0 * 16 / xg.rows, xg.n - 1) * xg.stride;
     // NT tiles of 16 rows of W and MT tiles of 16 rows of X per wave; W comes from HBM once, the
     // rows of X from the caches (they are few)
@@ -406,7 +427,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     const T* wt[NT];
     // HALF: rows 8 h .. 8 h + 7 of a tile (h: the workgroup's half).  Lanes of r < 8 hold those at step s, the others the same
     // rows at step s + 1, and likewise the columns of X: of the 16 x 16 sums the two diagonal quarters are wanted, and added
-    const int half = HALF ? blockIdx.x & 1 : 0, later = HALF ? r >> 3 : 0;
+    const int half = HALF ? block & 1 : 0, later = HALF ? r >> 3 : 0;
     const int w_lane = HALF ? later * 64 + 16 * g + 8 * half + (r & 7) : lane;
 #pragma unroll
     for (int t = 0; t < NT; ++t) wt[t] = Wt + ((int64_t)min(tile0 + t, n_tiles - 1) * steps * 64 + w_lane) * 8;
@@ -934,6 +955,13 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
     bool plain = !EB::chosen_only && !ro && !rsc;
     if constexpr (EB::activated) plain = !ex.over && !rsc;
     gemv_tiled_shape(M, N, K, nt, kw, blocks, plain);
+    if constexpr (EB::second) {
+        int nt2 = 0, kw2 = 0, blocks2 = 0;
+        gemv_tiled_shape(M, ex.N, ex.K, nt2, kw2, blocks2, plain);
+        if (nt2 != nt || kw2 != kw) return LI_UNSUPPORTED;
+        ex.blocks = blocks;
+        blocks += blocks2;
+    }
     if (kw < 2 || (nt < 0 && M > 8)) return LI_BAD_ARG;
     const RowsOut no_out{};
     const RowScale no_scale{};
@@ -953,7 +981,7 @@ static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt
         else if (nt < 0) return LI_BAD_ARG;               \
         else if (mt == 1 && nt == 1) PICK_KW(T, 1, 1);         \
         else if (mt == 1 && nt == 2) PICK_KW(T, 2, 1);    \
-        else if constexpr (!EB::chosen_only) { \
+        else if constexpr (!EB::chosen_only && !EB::second) { \
             if (mt == 2 && nt == 1) PICK_KW(T, 1, 2);     \
             else if (mt == 2 && nt == 2) PICK_KW(T, 2, 2); \
             else if (mt <= 4 && nt == 2) PICK_KW(T, 2, 4); \
@@ -1005,6 +1033,26 @@ extern "C" int li_gemv_tiled_act(const void* X, const void* Wt, int dt, void* C,
     ex.act = act;
     ex.on_input = on_input;
     return gemv_tiled(X, Wt, dt, C, dt, EPI_STORE, M, N, K, 0, 0, nullptr, nullptr, rsc, XGroups{0, 1, 0}, ex, stream);
+}
+
+// Two products of M rows (at most 16) in one launch: C = X . W^T and C2 = X2 . W2^T, float32.  Only where both would be launched in one shape of
+// workgroup (li_gemv_tiled_two_fits).
+extern "C" int li_gemv_tiled_two_fits(int M, int N, int K, int N2, int K2) {
+    int nt = 0, kw = 0, blocks = 0, nt2 = 0, kw2 = 0;
+    if (M < 1 || M > 16) return 0;
+    gemv_tiled_shape(M, N, K, nt, kw, blocks, true);
+    gemv_tiled_shape(M, N2, K2, nt2, kw2, blocks, true);
+    return nt == nt2 && kw == kw2;
+}
+extern "C" int li_gemv_tiled_two(const void* X, const void* Wt, void* C, int N, int K, const void* X2, const void* Wt2, void* C2, int N2, int K2,
+                                 int dt, int M, hipStream_t stream) {
+    if (M > 16) return LI_BAD_ARG;
+    int rc = check_common(X2, Wt2, C2, M, N2, K2, EPI_STORE, DT_F32);
+    if (rc) return rc;
+    if (K2 % 32 != 0 || ((uintptr_t)X2 & 15) || ((uintptr_t)Wt2 & 15)) return LI_UNSUPPORTED;
+    if (!li_gemv_tiled_two_fits(M, N, K, N2, K2)) return M == 0 ? LI_OK : LI_UNSUPPORTED;
+    return gemv_tiled(X, Wt, dt, C, DT_F32, EPI_STORE, M, N, K, 0, 0, nullptr, nullptr, nullptr, XGroups{0, 1, 0},
+                      TwoProducts{X2, Wt2, (float*)C2, K2, N2, 0}, stream);
 }
 
 // X [groups, M, K]: the rows of W from g * group_rows on (a multiple of 32; the last group: all that are left) against X[g].

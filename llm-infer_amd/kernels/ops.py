@@ -543,6 +543,31 @@ def linear_activated(x, w, kind: str, weights=None, n_blocks: int = 0, ff: int =
     return out
 
 
+class PendingProduct:
+    """A mixer's output product that is still to be run: ``x`` [T, k] against ``w``, float32 rows.  (What stands beside it may end with one
+    too: ``finish_products``.)"""
+
+    def __init__(self, x, w):
+        self.x, self.w = x, w
+
+
+def finish_products(pending) -> list:
+    """The float32 rows of every ``PendingProduct``: two of at most 16 rows against tiled weights in one launch, where their kernel
+    would take both in one shape of workgroup."""
+    if len(pending) == 2:
+        a, b = pending
+        m, shapes = a.x.shape[0], (*matrix_shape(a.w), *matrix_shape(b.w))
+        if (1 <= m <= 16 and b.x.shape[0] == m and all(is_tiled(p.w) and p.x.dtype == p.w.dtype == a.w.dtype and p.x.is_contiguous()
+                                                      and p.x.shape[1] == matrix_shape(p.w)[1] and (p.x.data_ptr() | p.w.data_ptr()) % 16 == 0 for p in pending)
+                and core().li_gemv_tiled_two_fits(m, *shapes)):
+            _dev(a.x, a.w, b.x, b.w)
+            out = [torch.empty((m, n), dtype=torch.float32, device=a.x.device) for n in shapes[::2]]
+            _check(core().li_gemv_tiled_two(_ptr(a.x), _ptr(a.w), _ptr(out[0]), *shapes[:2], _ptr(b.x), _ptr(b.w), _ptr(out[1]), *shapes[2:],
+                                            DT[a.x.dtype], m, _stream()), "gemv_tiled_two")
+            return out
+    return [linear(p.x, p.w, out_dtype=torch.float32) for p in pending]
+
+
 def linear_groups(x: torch.Tensor, w, group_rows: int) -> torch.Tensor:
     """Several products of few rows as one launch: ``x`` [groups, m <= 32, K] against a tiled weight whose rows from g *
     ``group_rows`` on (a multiple of 32; the last group: all that are left) read x[g].  Returns float32 [m, N]."""

@@ -197,7 +197,7 @@ class GatedAttention(Part):
                 splits = min(splits, max(1, (span + self.keep_first) // 64))
         return 1 << (splits.bit_length() - 1)
 
-    def attend(self, h, ctx, views, owns_cache, proj=None, col0=0):
+    def before_output(self, h, ctx, views, owns_cache=True, proj=None, col0=0):
         """The heads' gated outputs side by side, [T, H * dv] in the model's type.  ``proj`` (float32 [T, n]) with this
         mixer's columns from ``col0`` on: the product is not run here."""
         if owns_cache == self.reads_kv:
@@ -240,16 +240,16 @@ class GatedAttention(Part):
                                   gate_elem=self.gate_elem, keep_first=self.keep_first)
 
     def forward(self, h, ctx, views, residual, owns_cache=True):
-        ops.linear(self.attend(h, ctx, views, owns_cache), self.wo, ops.EPI_ADD, out=residual)
+        ops.linear(self.before_output(h, ctx, views, owns_cache), self.wo, ops.EPI_ADD, out=residual)
 
     def forward_into(self, h, out, ctx, views, owns_cache=True):
         """The mixer's result written over the float32 rows ``out`` (nothing is added to what they held)."""
-        ops.linear(self.attend(h, ctx, views, owns_cache), self.wo, out=out)
+        ops.linear(self.before_output(h, ctx, views, owns_cache), self.wo, out=out)
         return None
 
     def rows(self, h, ctx, views, owns_cache=True, proj=None, col0=0):
         """The mixer's result as float32 rows."""
-        return ops.linear(self.attend(h, ctx, views, owns_cache, proj, col0), self.wo, out_dtype=torch.float32)
+        return ops.linear(self.before_output(h, ctx, views, owns_cache, proj, col0), self.wo, out_dtype=torch.float32)
 
     def addends(self, h, ctx, views, owns_cache=True, proj=None, col0=0):
         return [(self.rows(h, ctx, views, owns_cache, proj, col0), 1.0)]

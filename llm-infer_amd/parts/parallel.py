@@ -16,7 +16,8 @@ class ParallelMixers(Part):
 
     Branches that keep a stacked input matrix (``w_in`` [``in_rows()``, hidden], and ``addends(..., proj=, col0=)``)
     share one product: once all tensors are bound their matrices are stacked once more, the rows of the input
-    are multiplied once, and each branch is handed its columns.  No row's sum changes by that.
+    are multiplied once, and each branch is handed its columns.  No row's sum changes by that.  Branches that have ``before_output`` (what
+    their output product ``wo`` reads, [T, k] in the model's type) leave that product to this part, which runs those of few rows in one launch.
 
     ``norms``: local names of two weights [hidden]; the two branches' results are then each divided by their root mean
     square over the row (``norm_eps``) and multiplied by their weight before they are added (their scales are equal)."""
@@ -65,15 +66,18 @@ class ParallelMixers(Part):
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32) if getattr(self, "w_in", None) is not None else None
         for i, (branch, scale) in enumerate(zip(self.branches, self.scales)):
             view, at = views_for(branch, views, at)
-            if proj is not None and self._col0[i] is not None:
-                out += [(y, s * scale) for y, s in branch.addends(h, ctx, view, owns_cache, proj=proj, col0=self._col0[i])]
+            shared = {"proj": proj, "col0": self._col0[i]} if proj is not None and self._col0[i] is not None else {}
+            if hasattr(branch, "before_output"):
+                # all but its output product, which runs with the others'
+                out.append((ops.PendingProduct(branch.before_output(h, ctx, view, owns_cache, **shared), branch.wo), scale))
             elif hasattr(branch, "addends"):
-                out += [(y, s * scale) for y, s in branch.addends(h, ctx, view, owns_cache)]
+                out += [(y, s * scale) for y, s in branch.addends(h, ctx, view, owns_cache, **shared)]
             else:
                 y = torch.zeros((h.shape[0], branch.hidden_size), dtype=torch.float32, device=h.device)
                 branch.forward(h, ctx, view, y, owns_cache)
                 out.append((y, scale))
-        return out
+        ready = iter(ops.finish_products([y for y, _ in out if isinstance(y, ops.PendingProduct)]))
+        return [(next(ready) if isinstance(y, ops.PendingProduct) else y, s) for y, s in out]
 
     def forward_rows(self, h, ctx, views, owns_cache=True):
         """With ``norms``: the two results with their norms, still to be added up."""

@@ -94,7 +94,8 @@ class GatedDelta(Part):
         return [StateSpec((self.n_heads, self.head_dim, self.v_head_dim), "float32"),
                 StateSpec((max(self.conv_taps - 1, 1), self.channels), "float32")]
 
-    def _heads(self, h, ctx, views, owns_cache, proj, col0):
+    def before_output(self, h, ctx, views, owns_cache=True, proj=None, col0=0):
+        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's columns from ``col0`` on: the input product is not run here."""
         _own_state(owns_cache, "the delta rule")
         H, G, d, dv = self.n_heads, self.n_kv_heads, self.head_dim, self.v_head_dim
         if proj is None:
@@ -108,15 +109,14 @@ class GatedDelta(Part):
         return ops.gated_head_norm(o, self.norm, proj, col0 + self.g_col, H, self.norm_eps, self.dtype, gate_silu=True)
 
     def addends(self, h, ctx, views, owns_cache=True, proj=None, col0=0):
-        """``proj`` (float32 [T, n]) with this mixer's columns from ``col0`` on: the input product is not run here."""
-        return [(ops.linear(self._heads(h, ctx, views, owns_cache, proj, col0), self.wo, out_dtype=torch.float32), 1.0)]
+        return [(ops.linear(self.before_output(h, ctx, views, owns_cache, proj, col0), self.wo, out_dtype=torch.float32), 1.0)]
 
     def forward_into(self, h, out, ctx, views, owns_cache=True):
-        ops.linear(self._heads(h, ctx, views, owns_cache, None, 0), self.wo, out=out)
+        ops.linear(self.before_output(h, ctx, views, owns_cache, None, 0), self.wo, out=out)
         return None
 
     def forward(self, h, ctx, views, residual, owns_cache=True):
-        ops.linear(self._heads(h, ctx, views, owns_cache, None, 0), self.wo, ops.EPI_ADD, out=residual)
+        ops.linear(self.before_output(h, ctx, views, owns_cache, None, 0), self.wo, ops.EPI_ADD, out=residual)
 
 
 @register_mixer("selective_scan")

@@ -71,8 +71,8 @@ class SigmoidAttention(Part):
     def in_rows(self) -> int:
         return (self.n_heads + self.n_kv_heads) * self.head_dim + self.n_kv_heads * self.v_head_dim
 
-    def addends(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
-        """``proj`` (float32 [T, n]) with this mixer's q, k, v from column ``col0`` on: the product is not run here."""
+    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
+        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v from column ``col0`` on: the input product is not run here."""
         if not owns_cache:
             raise ValueError("sigmoid attention writes its own keys and values in every run")
         H, G, d, dv = self.n_heads, self.n_kv_heads, self.head_dim, self.v_head_dim
@@ -94,7 +94,10 @@ class SigmoidAttention(Part):
         else:
             a = ops.sigmoid_attention_prefill(q, kv, ops.prefill_meta(ctx), self.bias, H, G, self.k_dim, dv,
                                               self.v_dim, self.scale, self.window)
-        return [(ops.linear(a.view(a.shape[0], H * dv), self.wo, out_dtype=torch.float32), 1.0)]
+        return a.view(a.shape[0], H * dv)
+
+    def addends(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
+        return [(ops.linear(self.before_output(h, ctx, view, owns_cache, proj, col0), self.wo, out_dtype=torch.float32), 1.0)]
 
     def forward(self, h, ctx, view, residual, owns_cache=True):
         ops.add_scaled(residual, self.addends(h, ctx, view, owns_cache))
