@@ -52,13 +52,18 @@ __device__ __forceinline__ void to_operand16(f32x4& v) {
 // 2 KW on.  The lanes of r < 8 hold the first chain of a pair, the others the second of the same rows, and likewise the columns
 // of X: of the 16 x 16 sums the two diagonal quarters are the two chains, each in its order.  Twice the workgroups and no
 // instruction more: 2,048 x 2,048 9.8 -> 7.6 us at 3 rows, 2,048 x 8,192 29.0 -> 19.6 (8 rows 32.5 -> 24.0); 4,096 x 4,096 17.5
-// and 18.3, where every CU has its workgroup without it.  U is 8 here, four or five waves a SIMD: a CU has one workgroup anyway
-// (3 rows, U of 4 and 8: 2,048 x 512 7.8 and 5.9 us, 2,048 x 2,048 9.4 and 7.4, 2,048 x 8,192 19.6 and 19.3).
+// and 18.3, where every CU has its workgroup without it.
+// WHOLE (K a multiple of a wave's chain, or pair of them): a chain's sixteen steps under no condition, U of them on their way and the
+// next one asked for as soon as a step's registers are free, in the order that is written (left to itself the compiler asked for two steps
+// and waited for them, and a step's condition was a branch).  A wave's loads are then what a step waits for, so it pays where a wave has one chain
+// or a CU one workgroup; else four steps at a time in more waves are as fast.  us at 1, 3 and 8 rows, before and now: 2,048 x 2,048 7.3 -> 6.1, 7.5 ->
+// 6.2, 7.7 -> 6.9; 2,048 x 8,192 18.5 -> 15.9, 19.5 -> 16.8, 23.8 -> 20.4; 3,072 x 2,048 9.9 -> 8.0, 10.0 -> 8.3, 10.2 -> 9.0; 16,384 x 2,048
+// 28.1 -> 24.8, 27.6 -> 25.7, 30.8 -> 29.4; 4,096 x 14,336 53.6 -> 45.2, 55.5 -> 46.4, 61.7 -> 51.9; but 28,672 x 4,096 at 4 rows 88.3 and 89.6.
 // ===========================================================================
-template <int NT, int MT, int KW, int U, bool HALF = false>
+template <int NT, int MT, int KW, int U, bool HALF = false, bool WHOLE = false>
 __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, Epilogue e) {
     __shared__ f32x4 part[KW][NT * MT][64];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
     constexpr int ROWS = HALF ? 8 : 16, CL = HALF ? 2 : 1;               // rows of W, and of X, of a tile; chains of one accumulator
     const int n0 = blockIdx.x * ROWS * NT, m0 = blockIdx.y * ROWS * MT;
     const int row = HALF ? r & 7 : r, later = HALF ? r >> 3 : 0;         // (HALF: lanes of r >= 8 hold the same rows in the next chain)
@@ -85,6 +90,41 @@ __global__ __launch_bounds__(64 * KW) void gemv_f32_kernel(const float* __restri
             const int k0 = c * CHAIN, steps = min(CHAIN, K - k0) >> 4;
             const int mine = HALF && later ? max(0, min(CHAIN, K - k0 - CHAIN)) >> 4 : steps;
             const int from = HALF && later ? min(k0 + CHAIN, K - 16) : k0;
+            if constexpr (WHOLE) {
+                constexpr int STEPS = CHAIN / 16;
+                f32x4 a[U][NT], b[U][MT];
+                const float *wc[NT], *xc[MT];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) wc[t] = wp[t] + from;
+#pragma unroll
+                for (int j = 0; j < MT; ++j) xc[j] = xp[j] + from;
+                auto fetch = [&](int s) {
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) a[s % U][t] = *(const f32x4*)(wc[t] + 16 * s);
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) b[s % U][j] = *(const f32x4*)(xc[j] + 16 * s);
+                };
+#pragma unroll
+                for (int s = 0; s < U; ++s) fetch(s);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int s = 0; s < STEPS; ++s) {
+                    const int u = s % U;
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) to_operand16(a[u][t]);
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) to_operand16(b[u][j]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int t = 0; t < NT; ++t)
+#pragma unroll
+                            for (int j = 0; j < MT; ++j) acc[t][j] = mfma16_f32(a[u][t][i], b[u][j][i], acc[t][j]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (s + U < STEPS) fetch(s + U);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            } else
             for (int s0 = 0; s0 < steps; s0 += U) {
                 f32x4 a[U][NT], b[U][MT];
 #pragma unroll
@@ -278,13 +318,31 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
         // sixteen waves where half the CUs have no workgroup (2,048 x 8,192 at 3 rows, whole blocks: 28 against 32 us), else eight; two
         // blocks of W a wave where there are workgroups enough (28,672 x 4,096 at 32 rows: 164 against 169 us)
         const int kw = chains <= 4 ? 4 : (mt == 1 && chains >= 16 && blocks <= 256 ? 16 : 8);
-        // up to 128 blocks and 8 rows: half blocks, so that every CU has a workgroup, a wave for each pair of chains
-        if (M <= 8 && blocks <= 128) {
-            const int pairs = (chains + 1) / 2;
+        // up to 128 blocks and 8 rows: half blocks, so that every CU has a workgroup, a wave for each pair of chains.  Beyond 256 blocks with two
+        // chains and more a wave, half blocks where the rows are few (us of whole and half ones at 1, 2, 4 and 8 rows: 5,120 x 4,096 24.6 and 19.3,
+        // 23.4 and 20.1, 25.2 and 22.4, 28.0 and 26.8; 8,192 x 4,096 29.2 and 26.7, 27.7 and 26.2, 28.0 and 28.9, 30.2 and 36.7; 28,672 x 4,096 88.9
+        // and 78.7, 84.2 and 81.5, 88.6 and 92.4)
+        const bool pairs_whole = K % (2 * CHAIN) == 0;
+        const bool few = pairs_whole && chains >= 16 && blocks > 256 && (M <= 2 || (M <= 4 && blocks <= 384));
+        if (few || (M <= 8 && blocks <= 128)) {
+            const int pairs = (chains + 1) / 2, waves = pairs <= 4 ? 4 : pairs <= 8 || few ? 8 : 16;
             const unsigned grid = (N + 7) / 8;
-            if (pairs <= 4) gemv_f32_kernel<1, 1, 4, 8, true><<<grid, 256, 0, stream>>>(X, W, K, e);
-            else if (pairs <= 8) gemv_f32_kernel<1, 1, 8, 8, true><<<grid, 512, 0, stream>>>(X, W, K, e);
-            else gemv_f32_kernel<1, 1, 16, 8, true><<<grid, 1024, 0, stream>>>(X, W, K, e);
+#define HALVES(KW)                                                                                                   \
+    do {                                                                                                            \
+        if (pairs_whole) gemv_f32_kernel<1, 1, KW, 8, true, true><<<grid, 64 * KW, 0, stream>>>(X, W, K, e);        \
+        else gemv_f32_kernel<1, 1, KW, 8, true><<<grid, 64 * KW, 0, stream>>>(X, W, K, e);                          \
+    } while (0)
+            if (waves == 4) HALVES(4); else if (waves == 8) HALVES(8); else HALVES(16);
+#undef HALVES
+            LI_CHECK_LAUNCH();
+            return LI_OK;
+        }
+        // one block of W and of X: whole chains where a wave has one of them, or a CU one workgroup
+        if (nt == 1 && mt == 1 && K % CHAIN == 0 && (chains <= kw || blocks <= 256)) {
+            const unsigned grid = blocks;
+            if (kw == 4) gemv_f32_kernel<1, 1, 4, 8, false, true><<<grid, 256, 0, stream>>>(X, W, K, e);
+            else if (kw == 8) gemv_f32_kernel<1, 1, 8, 8, false, true><<<grid, 512, 0, stream>>>(X, W, K, e);
+            else gemv_f32_kernel<1, 1, 16, 8, false, true><<<grid, 1024, 0, stream>>>(X, W, K, e);
             LI_CHECK_LAUNCH();
             return LI_OK;
         }

@@ -112,6 +112,10 @@ F32_CASES = [(1, 1, 16), (3, 33, 48), (8, 16400, 256), (9, 16400, 272), (16, 130
              (64, 100, 4096), (65, 64, 32), (100, 200, 2064), (128, 4112, 512), (129, 130, 304), (300, 514, 8208)]
 # half blocks: chains that are single, short, missing beside the last; one to sixteen pairs and more than one round of them
 F32_CASES += [(1, 8, 256), (2, 7, 272), (8, 2048, 768), (7, 2050, 2320), (5, 100, 4112), (8, 40, 8448), (4, 64, 16400)]
+# whole chains and pairs of them in the order that is written: one round of waves and several, a last round that some waves sit out, half blocks of
+# few rows beyond 256 blocks and the sizes on either side of their rule
+F32_CASES += [(3, 2050, 512), (8, 24, 9216), (2, 4112, 4096), (3, 6130, 4608), (4, 6144, 4352), (5, 4112, 4096), (3, 6160, 4096), (9, 36, 256), (16, 4096, 4352),
+              (12, 2100, 2048), (8, 2064, 1024)]
 
 
 @pytest.mark.parametrize("M,N,K", F32_CASES)
