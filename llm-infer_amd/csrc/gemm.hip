@@ -403,7 +403,7 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     constexpr int SL = HALF ? 2 : 1;                                   // so many 32-element steps of K
     __shared__ float part[KW][NT * MT][64][4];
     __shared__ float ss_wave[KW][16];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, g = lane >> 4;
     const int n_tiles = (e.N + 15) >> 4;
     const int steps = K >> 5;
@@ -431,70 +431,150 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
     const int w_lane = HALF ? later * 64 + 16 * g + 8 * half + (r & 7) : lane;
 #pragma unroll
     for (int t = 0; t < NT; ++t) wt[t] = Wt + ((int64_t)min(tile0 + t, n_tiles - 1) * steps * 64 + w_lane) * 8;
-    bool have_x[MT];
-    const T* xrow[MT];
+    const T* xrow[MT];                                    // (rows beyond M are the last again: their columns of the sums are nobody's)
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-        const int row = HALF ? r & 7 : 16 * j + r;
-        have_x[j] = row < e.M;
-        xrow[j] = X + (int64_t)(have_x[j] ? row : 0) * K + 32 * later + 8 * g;
-    }
+    for (int j = 0; j < MT; ++j) xrow[j] = X + (int64_t)min(HALF ? r & 7 : 16 * j + r, e.M - 1) * K + 32 * later + 8 * g;
     f32x4 acc[NT][MT];
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < MT; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     // RowScale (rows 0..15 only): the partial sums of squares of row r are dealt to the waves, and within a
-    // wave to the four lanes of the row; the loads are issued here and used after the main loop
-    float ss_mine = 0.f;
+    // wave to the four lanes of the row; they are asked for ahead of W and X, and added up while those are on their way
+    constexpr int SS = 16;
+    float ss_mine = 0.f, ss_v[SS];
+    int ss_lo = 0, ss_hi = 0;
     if (MT == 1 && rsc.ss) {
         // partial sum p of row r lies at ss[p * 16 + r]: the 16 lanes of a group read 64 contiguous bytes
         const float* p = rsc.ss + r;
         const int share = (rsc.P + 4 * KW - 1) / (4 * KW);
-        const int lo = (wave * 4 + g) * share, hi = min(rsc.P, lo + share);
-        for (int i = lo; i < hi; i += 8) {
-            float v[8];
+        ss_lo = (wave * 4 + g) * share;
+        ss_hi = min(rsc.P, ss_lo + share);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) v[c] = p[min(i + c, hi - 1) * 16];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) ss_mine += (i + c < hi) ? v[c] : 0.f;
-        }
+        for (int c = 0; c < SS; ++c) ss_v[c] = p[max(0, min(ss_lo + c, ss_hi - 1)) * 16];
     }
-    for (int s0 = s_begin; s0 < s_end; s0 += s_next) {
-        if constexpr (EXPERTS) if (ex.over == EXPERTS_IN_K) {
-            const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U * SL, steps) * 32 - 1) / ex.ff, ex.n);
-            bool any = false;
-            for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
-            if (!any) continue;
-        }
-        v8 a[U][NT], b[U][MT];
-        auto fetch = [&](auto once) {
+    auto add_squares = [&]() {
+        if (MT == 1 && rsc.ss) {
+            const float* p = rsc.ss + r;
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int s = s0 + u * SL;
-                const bool in = s + later < s_end;
-                const v8 z = {};
+            for (int c = 0; c < SS; ++c) ss_mine += (ss_lo + c < ss_hi) ? ss_v[c] : 0.f;
+            for (int i = ss_lo + SS; i < ss_hi; i += 8) {
+                float v[8];
 #pragma unroll
-                for (int t = 0; t < NT; ++t) {
-                    const T* from = wt[t] + (int64_t)s * 512;
-                    a[u][t] = !in ? z : decltype(once)::value ? load_once<v8>(from) : *(const v8*)from;
-                }
+                for (int c = 0; c < 8; ++c) v[c] = p[min(i + c, ss_hi - 1) * 16];
 #pragma unroll
-                for (int j = 0; j < MT; ++j) b[u][j] = (in && have_x[j]) ? *(const v8*)(xrow[j] + s * 32) : z;
+                for (int c = 0; c < 8; ++c) ss_mine += (i + c < ss_hi) ? v[c] : 0.f;
             }
-        };
-        // (17 to 32 rows: a matrix of less than 32 MiB through the caches; figures at li_gemm_rows.  Up to 16 rows past them, us through the
-        // caches and past them, 2 GB of such matrices in turn: 1 row x 1,024 x 1,024 3.5 and 2.9, x 2,048 x 2,048 4.4 and 3.8, 16 rows 4.6 and 4.0, 6.2
-        // and 5.6, x 4,096 x 4,096 10.4 and 9.5; 180 MB, a model that the caches hold: 3.1 and 3.0, 4.0 and 3.9, 3.8 and 4.0, 5.1 and 5.7, 8.4 and 9.3)
-        if (MT == 1 || (int64_t)e.N * K >= 1 << 24) fetch(std::true_type{});
-        else fetch(std::false_type{});
+        }
+    };
+    // (17 to 32 rows: a matrix of less than 32 MiB through the caches; figures at li_gemm_rows.  Up to 16 rows past them, us through the
+    // caches and past them, 2 GB of such matrices in turn: 1 row x 1,024 x 1,024 3.5 and 2.9, x 2,048 x 2,048 4.4 and 3.8, 16 rows 4.6 and 4.0, 6.2
+    // and 5.6, x 4,096 x 4,096 10.4 and 9.5; 180 MB, a model that the caches hold: 3.1 and 3.0, 4.0 and 3.9, 3.8 and 4.0, 5.1 and 5.7, 8.4 and 9.3)
+    const bool past = MT == 1 || (int64_t)e.N * K >= 1 << 24;
+    // A wave's steps as a ring, D of them on their way: as soon as a step's registers are free the next is asked for, under no condition and in the
+    // order that is written.  (Batches of U steps with a condition for every one waited for a whole batch before they multiplied, and a condition was
+    // a branch around each load.  us, batches and ring, at 8 rows: 4,096 x 4,096 8.2 and 7.7, 28,672 x 4,096 38.0 and 36.5, 4,096 x 14,336 21.3 and
+    // 20.3, 3,072 x 2,048 5.0 and 4.6, 16,384 x 2,048 13.4 and 12.7; at 16 rows 9.5 and 8.6, 46.8 and 44.9, 26.3 and 25.4, 5.9 and 5.3, 14.6 and 13.9; one
+    // row, which memory bounds, 0 to 2% less, but 128,256 x 4,096 146 and 148.  With the partial sums of squares ahead of them instead of waited for first, requests of
+    // the 8B shape: chat 75.7 -> 73.0 ms, 8 sequences on 8,192 tokens 79.2 -> 76.5.  Sixteen steps deep: 36.0 us at one row of the second, 9.2 at
+    // 8 of the first.)  A short share is one batch of its own length.
+    auto ring = [&](auto depth, auto once) {
+        constexpr int D = decltype(depth)::value;
+        const int n = (s_end - s_begin) / (SL * D) * D;
+        v8 a[D][NT], b[D][MT];
+        const T *wr[NT], *xr[MT];
 #pragma unroll
-        for (int u = 0; u < U; ++u)
+        for (int t = 0; t < NT; ++t) wr[t] = wt[t] + (int64_t)s_begin * 512;
+#pragma unroll
+        for (int j = 0; j < MT; ++j) xr[j] = xrow[j] + s_begin * 32;
+        auto fetch = [&](int u, int ahead) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                const T* from = wr[t] + ahead * SL * 512;
+                a[u][t] = decltype(once)::value ? load_once<v8>(from) : *(const v8*)from;
+            }
+#pragma unroll
+            for (int j = 0; j < MT; ++j) b[u][j] = *(const v8*)(xr[j] + ahead * SL * 32);
+        };
+        auto multiply = [&](int u) {
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[u][t], b[u][j], acc[t][j]);
-    }
+        };
+#pragma unroll
+        for (int u = 0; u < D; ++u) fetch(u, u);
+        __builtin_amdgcn_sched_barrier(0);
+        add_squares();
+        for (int i = D; i < n; i += D) {
+#pragma unroll
+            for (int u = 0; u < D; ++u) {
+                multiply(u);
+                __builtin_amdgcn_sched_barrier(0);
+                fetch(u, D + u);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int t = 0; t < NT; ++t) wr[t] += D * SL * 512;
+#pragma unroll
+            for (int j = 0; j < MT; ++j) xr[j] += D * SL * 32;
+        }
+#pragma unroll
+        for (int u = 0; u < D; ++u) multiply(u);
+        s_begin += n * SL;
+    };
+    // What the ring leaves: the last steps of a share that is no multiple of its depth, and experts in K, whose part may be left out.
+    auto batches = [&](auto once) {
+        for (int s0 = s_begin; s0 < s_end; s0 += s_next) {
+            if constexpr (EXPERTS) if (ex.over == EXPERTS_IN_K) {
+                const int first = min(s0 * 32 / ex.ff, ex.n), last = min((min(s0 + U * SL, steps) * 32 - 1) / ex.ff, ex.n);
+                bool any = false;
+                for (int i = first; i <= last; ++i) any |= (chosen >> i) & 1;
+                if (!any) continue;
+            }
+            v8 a[U][NT], b[U][MT];
+            const bool whole = s0 + U * SL <= s_end;
+            auto fetch = [&](auto all) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const int s = s0 + u * SL;
+                    const bool in = decltype(all)::value || s + later < s_end;
+                    const v8 z = {};
+#pragma unroll
+                    for (int t = 0; t < NT; ++t) {
+                        const T* from = wt[t] + (int64_t)s * 512;
+                        a[u][t] = !in ? z : decltype(once)::value ? load_once<v8>(from) : *(const v8*)from;
+                    }
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) b[u][j] = in ? *(const v8*)(xrow[j] + s * 32) : z;
+                }
+            };
+            if (whole) fetch(std::true_type{}); else fetch(std::false_type{});
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[u][t], b[u][j], acc[t][j]);
+        }
+    };
+    auto products = [&](auto once) {
+        const int n = (s_end - s_begin) / SL;
+        bool in_order = MT <= 2;
+        if constexpr (EXPERTS) in_order = ex.over != EXPERTS_IN_K;
+        if constexpr (MT <= 2) {
+            if (in_order && U == 8 && n >= 8) ring(std::integral_constant<int, 8>{}, once);
+            else if (in_order && U == 8 && n == 6) ring(std::integral_constant<int, 6>{}, once);
+            else if (in_order && n >= 4) ring(std::integral_constant<int, U < 4 ? U : 4>{}, once);
+            else if (in_order && n == 2) ring(std::integral_constant<int, 2>{}, once);
+            else if (in_order && n == 3) ring(std::integral_constant<int, 3>{}, once);
+            else add_squares();
+        }
+        if (s_begin < s_end) batches(once);
+    };
+    if constexpr (MT == 1) products(std::true_type{});
+    else if (past) products(std::true_type{});
+    else products(std::false_type{});
     if (MT == 1 && rsc.ss) {
         ss_mine = sum_halves(sum_quarters(ss_mine));
         if (g == 0) ss_wave[wave][r] = ss_mine;

@@ -336,6 +336,38 @@ def test_half_tiles(ops, M, N, K, dt):
 
 
 @pytest.mark.parametrize("dt", F16S)
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 11, 12, 15, 16, 17, 24, 31])
+def test_few_rows_with_shares_of_every_length(ops, steps, dt):
+    """gemv_tiled's waves with so many steps of K each, and with a last wave that has fewer: every depth of its ring, what the ring
+    leaves, whole tiles, two of them and halves (sums of up to 8,000 products of numbers of about 1 / sqrt(K): 2e-4 as above)."""
+    g = torch.Generator().manual_seed(steps)
+    for kw in (4, 8):
+        for K in (32 * kw * steps, 32 * (kw * steps - 1)):
+            for N in (48, 30):
+                w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV)
+                wt = ops.tile_weight(w)
+                for M, nt in ((1, -1), (8, -1), (1, 1), (16, 1), (5, 2), (17, 1), (32, 2)):
+                    x = torch.randn(M, K, generator=g).to(dt).to(DEV)
+                    ref = _linear_ref(x, w, 0)
+                    out = ops.gemv_tiled(x, wt, out_dtype=torch.float32, nt=nt, kw=kw)
+                    assert (out.double() - ref).abs().max().item() < 2e-4 * (1 + ref.abs().max().item()), (kw, K, N, M, nt)
+
+
+@pytest.mark.parametrize("parts", [1, 15, 16, 64, 255, 256, 257, 512, 700])
+@pytest.mark.parametrize("M,N,K", [(1, 48, 64), (8, 4096, 256), (9, 100, 2048), (16, 6144, 4096)])
+def test_a_norm_of_many_partial_sums_finished_by_the_product(ops, parts, M, N, K):
+    """The rows' sums of squares come in any number of parts: those that the product asks for ahead of W and those behind them."""
+    g = torch.Generator().manual_seed(parts + K)
+    dt = torch.bfloat16
+    xw, w = torch.randn(M, K, generator=g).to(dt).to(DEV), (torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV)
+    ss = torch.rand(parts, 16, generator=g).to(DEV) + 0.1
+    lazy = ops.LazyNorm(torch.zeros(M, K, device=DEV), None, 1e-5, dt, xw, ss, 1.0)
+    out = ops.linear(lazy, ops.tile_weight(w), out_dtype=torch.float32)
+    ref = _linear_ref(xw, w, 0) / (ss.double().sum(0)[:M, None] / K + 1e-5).sqrt()
+    assert ((out.double() - ref) / (1 + ref.abs().max())).abs().max().item() < 2e-4
+
+
+@pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M,N,K", [(129, 72, 32), (130, 256, 64), (257, 200, 160), (300, 1000, 96), (511, 528, 96), (384, 1024, 256)])
 def test_tiled_products_write_whole_rows(ops, M, N, K, dt):
     """The epilogues that store whole rows of a tile, 16 bytes a lane, beside the ones that go through it quad by quad (taken
