@@ -1159,7 +1159,7 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
     Epilogue e;
     rc = make_epilogue(e, C, mode, out_dt, M, N, rs);
     if (rc) return rc;
-    const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 64 ? 4 : (M <= 96 ? 6 : 8)));
+    const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : (M <= 48 ? 3 : (M <= 64 ? 4 : (M <= 96 ? 6 : 8))));
     const int tiles = (N + 15) / 16;
     if (nt <= 0) nt = tiles >= 1024 ? 2 : 1;          // enough workgroups for 256 CUs either way
     if (kw <= 0) kw = 4;
@@ -1170,11 +1170,13 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
     const RowsOut no_out{};
     const int blocks = (tiles + nt - 1) / nt;
     // Matrices of less than 32 MiB stay in the caches beyond 16 rows: all of a small model's matrices together fit them, and in a large
-    // model these are bound by latency.  us past the caches and through them, of 100 MB of such matrices in turn and of 1.6 GB: 64 rows x
-    // 2,048 x 2,048 8.9 and 7.4, 8.3 and 8.5, x 512 x 4,096 12.2 and 9.1, 11.9 and 12.1, x 3,072 x 2,048 9.7 and 8.4, 8.7 and 8.8; 24 rows x 2,048 x
-    // 2,048 9.9 and 8.6, 9.2 and 9.5; larger ones, 48 rows x 4,096 x 4,096 17.1 and 15.4, 13.0 and 13.5, x 6,144 x 4,096 (600 MB) 17.6 and 18.4
+    // model these are bound by latency.  us past the caches and through them, of 200 MB of such matrices in turn and of 1.6 GB: 64 rows x
+    // 2,048 x 2,048 7.9 and 6.0, 7.8 and 8.0, x 512 x 4,096 11.2 and 8.2, 11.3 and 11.6, x 3,072 x 2,048 8.1 and 6.4, 8.0 and 8.3; 24 rows x 2,048 x
+    // 2,048 5.9 and 4.8, 5.8 and 6.1; larger ones of 1.6 GB, 48 rows x 4,096 x 4,096 11.6 and 12.1, x 6,144 x 4,096 19.8 and 19.8
     const bool once = (int64_t)N * K * 2 >= 32 << 20;
-    // stages of 64 of K a wave: what 128 KiB of LDS hold for the workgroup's waves
+    // D, stages of 64 of K a wave: two.  With more, LDS holds one workgroup a CU, whose waves wait for their own W with nobody beside them
+    // (us with 4 stages and with 2: 24 rows x 4,096 x 4,096, eight waves, 10.5 and 9.6, 32 rows x 6,144 x 4,096, two tiles, eight waves,
+    // 16.0 and 14.3, 64 rows x 4,096 x 4,096, four waves, 13.9 and 13.3).  Up to 16 rows four: the LDS has room, X is small beside W
 #define LAUNCH(T, NT, MT, KW, D, ONCE)                                                                    \
     do {                                                                                                  \
         auto kfn = gemm_rows_kernel<T, NT, MT, KW, D, ONCE>;                                              \
@@ -1194,11 +1196,13 @@ extern "C" int li_gemm_rows(const void* X, const void* Wt, int dt, void* C, int 
     } while (0)
 #define BY_MT(T, NT)                                            \
     do {                                                        \
-        if (mt == 1 && kw == 4) GO(T, NT, 1, 4, 8);             \
-        else if (mt == 1) GO(T, NT, 1, 8, 8);                   \
-        else if (mt == 2 && kw == 4) GO(T, NT, 2, 4, 6);        \
-        else if (mt == 2) GO(T, NT, 2, 8, 4);                   \
-        else if (mt == 4 && kw == 4) GO(T, NT, 4, 4, 4);        \
+        if (mt == 1 && kw == 4) GO(T, NT, 1, 4, 4);             \
+        else if (mt == 1) GO(T, NT, 1, 8, 4);                   \
+        else if (mt == 2 && kw == 4) GO(T, NT, 2, 4, 2);        \
+        else if (mt == 2) GO(T, NT, 2, 8, 2);                   \
+        else if (mt == 3 && kw == 4) GO(T, NT, 3, 4, 2);        \
+        else if (mt == 3) GO(T, NT, 3, 8, 2);                   \
+        else if (mt == 4 && kw == 4) GO(T, NT, 4, 4, 2);        \
         else if (mt == 4) GO(T, NT, 4, 8, 2);                   \
         else if (mt == 6) GO(T, NT, 6, 4, 2);                   \
         else GO(T, NT, 8, 4, 2);                                \

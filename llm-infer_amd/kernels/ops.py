@@ -378,21 +378,24 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
     kind = force or ("f32" if f32_ok else "fma" if not fast_ok else ("gemv_mfma" if m <= 16 else ("big" if m > 32 else "mfma")))
     if tiled:
         _need(fast_ok and kind != "fma", "a tiled weight needs 16-bit activations of its dtype")
-        # up to 16 rows (32 for a small matrix) every wave fetches the rows of X itself; beyond that
-        # the tiled GEMM is faster
+        # up to 16 rows (32 for a wide and shallow matrix) every wave fetches the rows of X itself; beyond that gemm_rows and
+        # the tiled GEMM are faster (us at 24 rows, gemv_tiled and gemm_rows: 2,048 x 2,048 9.4 and 6.0, 2,048 x 8,192 23.6 and
+        # 14.2, 3,072 x 2,048 9.1 and 6.3, 4,096 x 4,096 14.4 and 9.2; but 16,384 x 512 6.9 and 7.5, x 1,024 9.8 and 10.1: a
+        # workgroup's few steps of K do not pay for its stages)
         # 9 to 16 rows against a wide matrix with an activation (gate and up): the tiled GEMM's tile of 64 rows of X
         # fetches the rows of X once per 112 rows of W, gemv_tiled once per 16 or 32 (measured at 16 rows and
         # 28,672 x 4,096: 44.6 against 51.7 us, at 12 rows 44.2 against 48.7, at 8 rows 44.0 against 43.5)
         wide = (force is None and 8 < m <= 16 and mode in GATED and n * k >= (1 << 26) and m * k * 2 < (1 << 32)
                 and _wreg_plan(m, n, k) == (2, 1))
-        if not wide and (kind == "gemv_mfma" or (force is None and (m <= 16 or (m <= 32 and n * k <= (1 << 25))))):
+        if not wide and (kind == "gemv_mfma" or (force is None and (m <= 16 or (m <= 32 and k <= 1024 and 12288 <= n and n * k <= (1 << 25))))):
             ro = rsc = None
-            # 9 to 16 rows with the residual sum against a matrix with a long K (down): gemm_rows, one tile of W a
-            # workgroup (measured at 16 rows and 4,096 x 14,336: 25.5 against 30.3 us, at 12 rows 24.4 against 27.1, at 8
-            # rows the same; 4,096 x 11,008 at 16 rows 20.9 against 25.9, 2,048 x 8,192 10.2 against 11.9; against
-            # 4,096 x 4,096 gemv_tiled is as fast)
-            tall = (force is None and 8 < m <= 16 and mode == EPI_ADD and lazy is None and k >= 8192 and n >= 2048 and n % 16 == 0
-                    and x.stride(0) % 8 == 0 and x.stride(1) == 1)
+            # 9 to 16 rows, nothing of a norm to finish, against a matrix with a long K (output products, down): gemm_rows, one
+            # tile of W a workgroup, whose rows of X come in whole lines (us, gemv_tiled and gemm_rows, at 9, 12 and 16 rows: 4,096 x
+            # 14,336 20.5 and 21.4, 22.2 and 20.8, 25.4 and 22.0; 2,048 x 8,192 10.6 and 10.3, 11.8 and 11.0, 13.1 and 11.6; 2,048 x
+            # 4,096 6.6 and 6.5, 7.0 and 6.7, 7.7 and 7.1; but 2,048 x 2,048 4.6 and 4.8, 4.8 and 4.8, 5.2 and 5.2, 4,096 x 4,096 7.6 and
+            # 8.4, 7.9 and 8.1, 8.4 and 8.8)
+            tall = (force is None and 8 < m <= 16 and mode in (EPI_ADD, EPI_STORE) and lazy is None and experts is None and n % 16 == 0
+                    and ((k >= 8192 and m >= 12) or (k >= 4096 and n <= 2048)) and x.stride(0) % 8 == 0 and x.stride(1) == 1)
             nxt = getattr(out, "_li_next_norm", None) if mode == EPI_ADD else None
             if (nxt is not None and m <= 16 and n % 32 == 0 and out.data_ptr() % 16 == 0 and nxt.dtype == torch.float32
                     and nxt.shape == (n,) and nxt.is_cuda and nxt.data_ptr() % 16 == 0):
@@ -653,15 +656,16 @@ def _wreg_plan(m: int, n: int, k: int) -> tuple[int, int]:
 
 
 def _rows_cost(nt: int, m: int, n: int, k: int) -> float:
-    """Estimated microseconds of one gemm_rows launch, fitted to measurements on MI355X (24 to 128 rows against
-    the matrices of the 8B shape): W streamed once (at the rate of 256 workgroups, slower with fewer), plus the
-    rows of X, which every workgroup fetches from L2 in blocks of 16, plus a launch."""
-    blocks16 = 2 if m <= 32 else (4 if m <= 64 else (6 if m <= 96 else 8))
+    """Estimated microseconds of one gemm_rows launch, fitted to measurements on MI355X (17 to 128 rows against 61 matrices of
+    320 to 28,672 rows and 512 to 14,336 of K; the kernel it names is 1.1% slower in the mean than the fastest): W streamed once (at the
+    rate of 256 workgroups, slower with fewer), plus the rows of X, which every workgroup fetches from L2 in blocks of 16, plus a
+    workgroup's start and end, plus a launch."""
+    blocks16 = 2 if m <= 32 else (3 if m <= 48 else (4 if m <= 64 else (6 if m <= 96 else 8)))
     groups = -(-(-(-n // 16)) // nt)
     w_mb, x_mb = n * k * 2 / 1e6, groups * blocks16 * 16 * k * 2 / 1e6
-    # one workgroup a CU at a time (its stages fill the LDS): a last round that is not full runs as long as a full one
+    # a last round of 256 workgroups that is not full runs as long as a full one
     uneven = -(-groups // 256) * 256 / groups
-    return 2.5 + (w_mb / 6.2 + x_mb / 22.0) * uneven
+    return 2.5 + (w_mb / 7.0 + x_mb / 22.0 + 1.2 * groups / 256) * uneven
 
 
 @functools.lru_cache(maxsize=4096)

@@ -314,6 +314,28 @@ def test_linear_tiled_weights(ops, M, N, K, dt):
 
 
 @pytest.mark.parametrize("dt", F16S)
+@pytest.mark.parametrize("M,N,K", [(17, 16, 32), (32, 40, 96), (33, 100, 544), (48, 520, 1056), (49, 72, 64), (64, 48, 4128),       # blocks of rows of X
+                                   (12, 2064, 8192), (16, 2048, 4096), (9, 32, 4128), (11, 2064, 8192), (12, 16, 4064),             # either side of "a long K"
+                                   (17, 12288, 1024), (32, 12304, 96), (32, 12272, 1024), (24, 12288, 1056)])                        # of "wide and shallow"
+def test_more_rows_than_one_block_and_the_rules_beside_them(ops, M, N, K, dt):
+    """gemm_rows with one to four blocks of 16 rows of X, shares of K with and without whole stages, and the planner's choice on
+    either side of its rules, as tall products with the residual sum and without (K sums in float32: 2e-4 as above)."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(dt).to(DEV)
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV)
+    res = torch.randn(M, N, generator=g).to(DEV)
+    wt = ops.tile_weight(w)
+    for kind in (None, "rows:1:4", "rows:1:8", "rows:2:4", "rows:2:8"):
+        ref = _linear_ref(x, w, 0)
+        out = ops.linear(x, wt, out_dtype=torch.float32, force=kind)
+        assert (out.double() - ref).abs().max().item() < 2e-4 * (1 + ref.abs().max().item()), kind
+        out = res.clone()
+        ops.linear(x, wt, 1, out=out, force=kind)
+        ref = _linear_ref(x, w, 1, res)
+        assert (out.double() - ref).abs().max().item() < 2e-4 * (1 + ref.abs().max().item()), kind
+
+
+@pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(8, 32), (16, 64), (24, 96), (100, 544), (2048, 1056), (2050, 160), (4096, 8192)])
 def test_half_tiles(ops, M, N, K, dt):
