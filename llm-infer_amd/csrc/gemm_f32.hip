@@ -2,17 +2,19 @@
 //
 // v_mfma_f32_16x16x4_f32 adds its products one after the other in ascending k, each as a fused multiply-add rounded to
 // nearest, subnormal numbers kept: an accumulator that takes k in ascending order is bit for bit the chain of fmaf that
-// gemm_fma runs (compared on an MI355X, operands, products and sums below 2^-126 among them).  Both kernels here sum as gemm_fma does, chains
+// gemm_fma runs (compared on an MI355X, operands, products and sums below 2^-126 among them).  The kernels here sum as gemm_fma does, chains
 // over 256 consecutive k that are added up in ascending order, so a result depends neither on the kernel nor on the batch,
 // and a call that these do not take (K no multiple of 16, an address that is not 16-byte aligned) gives the same numbers
 // through gemm_fma.
 //
 //   gemv_f32   few rows of X: W from memory straight into operand A, the waves of a workgroup take chains in turn
-//   gemm_f32   more rows: tiles of W and X through LDS
+//   gemm_f32   many rows: tiles of W and X through LDS
+//   gemm_f32_chains   rows between: smaller tiles, whose chains the waves of a workgroup take in turn
 //
 // The operands lie row-major, so a lane fetches four consecutive k of its row with one 16-byte load; what instruction j
 // wants instead is k = 4 j + lane / 16.  gemv_f32 turns one into the other in registers, by four swaps of half waves and
-// of quarters (v_permlane32_swap, v_permlane16_swap) for four instructions; gemm_f32 on the way into LDS.
+// of quarters (v_permlane32_swap, v_permlane16_swap) for four instructions; gemm_f32 on the way into LDS;
+// gemm_f32_chains reads LDS word by word.
 #include "gemm_common.h"
 
 #define CHAIN 256                       // consecutive k of one chain of multiply-adds (as in gemm_fma)
@@ -296,23 +298,159 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_kernel(const float* __restric
 }
 
 // ===========================================================================
+// gemm_f32_chains: 32 rows of W x 32 rows of X, KW waves that take the chains of K in turn (wave w: w, w + KW, ...), each for the whole
+// tile (four sums of 16 x 16), and add the finished ones up in ascending order through LDS, as gemv_f32 does: a quarter of gemm_f32's
+// tile and a quarter of its serial chain.
+// A wave brings 32 of K of its 64 rows, a stage, into LDS of its own by global_load_lds, in units of 8 rows x 128 bytes (whole lines);
+// nobody else reads it, so there is no barrier but at the chains' ends.  Two stages in LDS and one in registers: a stage is read while the one
+// before it is multiplied, and the one two on is fetched into its place.
+// Operands are read word by word (lane (r, g) wants k = 4 j + g of row r; two blocks of 16 rows an instruction); chunk c of 16 bytes of row r lies
+// at place c ^ (r / 2 % 8), so that the sixteen rows are on different banks.
+// Bound by the rows it fetches (32 bytes a cycle and CU at the matrix cores' rate; it gets 12 to 13 TB/s in all) where there are many tiles, by a
+// tile's own 7 us of instructions at K = 2,048 where there are few.  us, before (gemv_f32 up to 64 or 128 rows, gemm_f32) and now: 32 rows x 2,048 x
+// 2,048 15.2 and 13.3, x 2,048 x 8,192 57.1 and 46.2, x 6,144 x 4,096 55.9 and 29.1; 64 rows 23.9 and 13.2, 91.4 and 43.5, 85.5 and 45.4; 200 rows
+// 45.2 and 23.0, 174 and 77.6, 149 and 118; 375 rows 45.9 and 34.2, 174 and 118, 226 and 183.  Stages read in the first third of the
+// one before, so that the next is fetched earlier: 14% slower; one stage in LDS and three workgroups a CU: a third slower; two waves a workgroup: 10 to 60%.
+// ===========================================================================
+template <int KW>
+__global__ __launch_bounds__(64 * KW, 2) void gemm_f32_chains_kernel(const float* __restrict__ X, const float* __restrict__ W, int K, int tiles_m, int tiles,
+                                                                    Epilogue e) {
+    constexpr int STAGE = 8 * 1024, STAGES = CHAIN / 32, OWN = 4 / KW;
+    static_assert(KW == 2 || KW == 4, "the four blocks are dealt to the waves");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char f32_smem[];       // KW x (two stages), then KW x (four blocks of sums)
+    const int id = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);           // (as gemm_f32)
+    if (id >= tiles) return;
+    const int n0 = id / tiles_m * 32, m0 = id % tiles_m * 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15, g = lane >> 4;
+    const int chains = K / CHAIN;                                                     // (K is a multiple of a chain)
+    const int mine = (chains - wave + KW - 1) / KW, all = mine * STAGES;             // this wave's chains and stages
+    unsigned char* region = f32_smem + wave * 2 * STAGE;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)region;
+    const uint32_t sums = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char*)f32_smem + KW * 2 * STAGE + lane * 16;
+    // unit q < 4: rows 8 q .. of W, then of X; lane 8 p + c brings chunk c ^ (row / 2 % 8) of row 8 q + p (rows beyond the last: the last)
+    const float* from[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const int p = lane >> 3, row = 8 * (q & 3) + p, chunk = (lane & 7) ^ ((row >> 1) & 7);
+        from[q] = (q < 4 ? W + (int64_t)min(n0 + row, e.N - 1) * K : X + (int64_t)min(m0 + row, e.M - 1) * K) + 4 * chunk;
+    }
+    auto fetch = [&](int t) {                        // stage t of this wave into place t % 2 (t beyond the last: the last again, unused)
+        const int s = min(t, all - 1), k = (wave + KW * (s / STAGES)) * CHAIN + s % STAGES * 32;
+#pragma unroll
+        for (int q = 0; q < 8; ++q)
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(from[q] + k),
+                                             (__attribute__((address_space(3))) void*)(region + (t & 1) * STAGE + q * 1024), 16, 0, 0);
+    };
+    uint32_t at[8];                                  // chunk c of row r of a block; the next block lies 2 KiB on
+#pragma unroll
+    for (int c = 0; c < 8; ++c) at[c] = lds0 + (r >> 3) * 1024 + (r & 7) * 128 + ((c ^ (r >> 1)) * 16) + 4 * g;
+    f32x2 a[2][8], b[2][8];                          // [stage's parity][chunk]: both blocks of W, both of X
+#define READ(SET, C)                                                                                                             \
+    do {                                                                                                                        \
+        asm volatile("ds_read2st64_b32 %0, %1 offset0:0 offset1:8" : "=v"(a[SET][C]) : "v"(at[C] + (SET) * STAGE) : "memory");   \
+        asm volatile("ds_read2st64_b32 %0, %1 offset0:16 offset1:24" : "=v"(b[SET][C]) : "v"(at[C] + (SET) * STAGE) : "memory"); \
+    } while (0)
+    f32x4 acc[2][2], total[OWN];
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) total[o] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (all > 0) {
+        fetch(0);
+        fetch(1);
+        __builtin_amdgcn_s_waitcnt(0x0F78);                                           // vmcnt(8): stage 0 has landed
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) READ(0, c);
+        __builtin_amdgcn_s_waitcnt(0xC07F);                                           // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(2);
+    }
+    for (int c0 = 0; c0 < chains; c0 += KW) {
+        const int t0 = c0 / KW * STAGES;
+        if (c0 + wave < chains) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = t0; t < t0 + STAGES; t += 2) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_s_waitcnt(0x0F78);                               // vmcnt(8): stage t + u + 1 has landed
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) {
+                        READ(u ^ 1, c);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[i >> 1][i & 1] = mfma16_f32(a[u][c][i >> 1], b[u][c][i & 1], acc[i >> 1][i & 1]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    __builtin_amdgcn_s_waitcnt(0xC07F);                               // lgkmcnt(0)
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch(t + u + 3);                // the next stage is in registers: its place is free
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            // (the compiler does not know that the stores below read what a matrix instruction writes: 19 cycles after the last one)
+            asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(sums + wave * 4096), "v"(acc[i >> 1][i & 1]), "n"(i * 1024) : "memory");
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        const int have = min(KW, chains - c0);
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+            f32x4 part[KW];
+#pragma unroll
+            for (int w = 0; w < KW; ++w)
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(part[w]) : "v"(sums + (wave + o * KW) * 1024), "n"(w * 4096) : "memory");
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int w = 0; w < KW; ++w)
+                if (w < have) total[o] += part[w];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+    }
+    __builtin_amdgcn_s_waitcnt(0x0F70);              // nothing is in flight into LDS when the workgroup ends
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+        const int q = wave + o * KW;
+        const float v[4] = {total[o][0], total[o][1], total[o][2], total[o][3]};
+        epilogue4(e, m0 + 16 * (q & 1) + r, n0 + 16 * (q >> 1) + 4 * g, v);
+    }
+#undef READ
+}
+
+// ===========================================================================
 // C interface
 // ===========================================================================
-// kind: 0 = by the sizes, 1 = gemv_f32 (at most 128 rows), 2 = gemm_f32.
+// kind: 0 = by the sizes, 1 = gemv_f32 (at most 128 rows), 2 = gemm_f32, 3 = gemm_f32_chains (whole chains only).
 extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, int mode, int M, int N, int K, int kind,
                            const RopeStore* rs, hipStream_t stream) {
     int rc = check_common(X, W, C, M, N, K, mode, out_dt);
     if (rc) return rc;
-    if (K % 16 != 0 || (((uintptr_t)X | (uintptr_t)W) & 15) || kind < 0 || kind > 2 || (kind == 1 && M > 128)) return LI_UNSUPPORTED;
+    if (K % 16 != 0 || (((uintptr_t)X | (uintptr_t)W) & 15) || kind < 0 || kind > 3 || (kind == 1 && M > 128) || (kind == 3 && K % CHAIN)) return LI_UNSUPPORTED;
     if (M == 0) return LI_OK;
     Epilogue e;
     rc = make_epilogue(e, C, mode, out_dt, M, N, rs);
     if (rc) return rc;
     const int chains = (K + CHAIN - 1) / CHAIN, blocks = (N + 15) / 16;
-    // gemv_f32 has its workgroups by the rows of W alone, gemm_f32 fills the chip only where both sides have enough
+    // Whole chains: gemv_f32 up to 16 rows (20: 3,072 x 2,048 at 17 rows 14.0 us, gemm_f32_chains 14.7, at 24 rows 15.2 and 14.7), fewer against many
+    // rows of W (6,144 x 4,096 at 9 and 16 rows 29.0 and 28.0, 33.7 and 28.3, at 8 rows 28.9 and 28.1; but 8,192 x 512 6.9 and 7.9).  Beyond, the rounds
+    // of 256 tiles: gemm_f32's take 36.7 us at K = 2,048 (one alone 43.5), gemm_f32_chains' 10.3 (375 rows x 16,384 x 2,048, 6 rounds and 24, 225 and 245
+    // us; x 3,072 x 2,048, 2 and 5, 76 and 53).
+    // Else gemv_f32 has its workgroups by the rows of W alone, gemm_f32 fills the chip only where both sides have enough
     // rows.  us at 64 rows of X: 2,048 x 2,048 25 against 41, 2,048 x 8,192 89 against 160, but 16,384 x 2,048 71 against 49; at
     // 32 rows 16,384 x 2,048 46 against 49
-    if (kind == 0) kind = M <= 32 || (M <= 64 && blocks < 1024) || (M <= 128 && blocks <= 256) ? 1 : 2;
+    auto rounds = [&](int side) { return ((int64_t)((M + side - 1) / side) * ((N + side - 1) / side) + 255) / 256; };
+    if (kind == 0 && K % CHAIN == 0) {
+        const int64_t n64 = rounds(64);
+        if (M <= 8 || (M <= 20 && (blocks < 384 || chains < 8))) kind = 1;
+        else kind = 10.3 * rounds(32) < 36.7 * n64 + (n64 == 1 ? 7 : 3) && (int64_t)((M + 31) / 32) * ((N + 31) / 32) <= F32_TILES ? 3 : 2;
+    } else if (kind == 0) kind = M <= 32 || (M <= 64 && blocks < 1024) || (M <= 128 && blocks <= 256) ? 1 : 2;
     if (kind == 1) {
         const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4), nt = M > 8 && blocks >= 1024 ? 2 : 1;
         // sixteen waves where half the CUs have no workgroup (2,048 x 8,192 at 3 rows, whole blocks: 28 against 32 us), else eight; two
@@ -356,6 +494,20 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
         GO(2, 1, 4, 4) GO(2, 1, 8, 4) GO(2, 2, 4, 4) GO(2, 2, 8, 4) GO(2, 4, 4, 4) GO(2, 4, 8, 4)
 #undef GO
         return LI_UNSUPPORTED;
+    }
+    if (kind == 3) {
+        constexpr int KW = 4, LDS = KW * (2 * 8192 + 4096);
+        const int tiles_m = (M + 31) / 32;
+        const int64_t tiles = (int64_t)tiles_m * ((N + 31) / 32);
+        if (tiles > F32_TILES) return LI_UNSUPPORTED;
+        static bool allowed = false;               // more than 64 KiB of LDS is asked for once
+        if (!allowed) {
+            if (hipFuncSetAttribute((const void*)gemm_f32_chains_kernel<KW>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess) return LI_HIP_ERROR;
+            allowed = true;
+        }
+        gemm_f32_chains_kernel<KW><<<(int)((tiles + 7) / 8 * 8), 64 * KW, LDS, stream>>>(X, W, K, tiles_m, (int)tiles, e);
+        LI_CHECK_LAUNCH();
+        return LI_OK;
     }
     const int tiles_m = (M + 63) / 64;
     const int64_t tiles = (int64_t)tiles_m * ((N + 63) / 64);

@@ -142,6 +142,30 @@ def test_float32_products_on_the_matrix_cores_are_bit_equal(ops, M, N, K):
         assert torch.equal(ops.linear(x, off), ops.linear(x, w))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 1, 256), (33, 30, 512), (32, 33, 768), (64, 130, 1024), (65, 64, 1280), (31, 2050, 2304), (200, 520, 8192),
+                                   (21, 4096, 2048), (20, 6144, 2048), (9, 6160, 2048), (256, 3072, 2048), (300, 4112, 512)])
+def test_float32_products_that_share_their_chains_among_waves_are_bit_equal(ops, M, N, K):
+    """gemm_f32_chains against gemm_fma: one chain (three waves without), rounds of four that are full and not, ragged tiles, rows of
+    every magnitude and subnormal products; and the kernel that the sizes choose, on either side of its rules."""
+    g = torch.Generator().manual_seed(M + N + K)
+    scale = torch.exp2(torch.randint(-40, 40, (N, 1), generator=g).float())
+    x, w = torch.randn(M, K, generator=g).to(DEV), (torch.randn(N, K, generator=g) * scale).to(DEV)
+    res = torch.randn(M, N, generator=g).to(DEV)
+    for kind in (None, "f32:3"):
+        for mode in (0, 1, 2):
+            if mode == 2 and N % 2:
+                continue
+            outs = [ops.linear(x, w, mode, out=res.clone() if mode == 1 else None, force=k) for k in ("fma", kind)]
+            assert torch.equal(*outs), (kind, mode)
+    tiny = (x * 2.0 ** -100).contiguous()
+    assert torch.equal(ops.linear(tiny, w, force="f32:3"), ops.linear(tiny, w, force="fma"))
+    if M * K > 4096:
+        x[0, 5], x[-1, 7] = float("inf"), float("nan")
+        assert torch.equal(ops.linear(x, w, force="f32:3").isnan(), ops.linear(x, w, force="fma").isnan())
+    with pytest.raises(ops.KernelError):
+        ops.linear(x[:, :240].contiguous(), w[:, :240].contiguous(), force="f32:3")
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 33, 48), (17, 257, 528), (100, 200, 2064), (129, 130, 304)])
 def test_float32_products_of_subnormal_numbers_are_bit_equal(ops, M, N, K):
     """Operands, products and sums below 2^-126: no kernel takes them for zeros."""
