@@ -389,12 +389,12 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
                 and _wreg_plan(m, n, k) == (2, 1))
         if not wide and (kind == "gemv_mfma" or (force is None and (m <= 16 or (m <= 32 and k <= 1024 and 12288 <= n and n * k <= (1 << 25))))):
             ro = rsc = None
-            # 9 to 16 rows, nothing of a norm to finish, against a matrix with a long K (output products, down): gemm_rows, one
-            # tile of W a workgroup, whose rows of X come in whole lines (us, gemv_tiled and gemm_rows, at 9, 12 and 16 rows: 4,096 x
+            # 9 to 16 rows with the residual sum against a matrix with a long K (output products, down): gemm_rows, one tile of W
+            # a workgroup, whose rows of X come in whole lines (us, gemv_tiled and gemm_rows, at 9, 12 and 16 rows: 4,096 x
             # 14,336 20.5 and 21.4, 22.2 and 20.8, 25.4 and 22.0; 2,048 x 8,192 10.6 and 10.3, 11.8 and 11.0, 13.1 and 11.6; 2,048 x
             # 4,096 6.6 and 6.5, 7.0 and 6.7, 7.7 and 7.1; but 2,048 x 2,048 4.6 and 4.8, 4.8 and 4.8, 5.2 and 5.2, 4,096 x 4,096 7.6 and
             # 8.4, 7.9 and 8.1, 8.4 and 8.8)
-            tall = (force is None and 8 < m <= 16 and mode in (EPI_ADD, EPI_STORE) and lazy is None and experts is None and n % 16 == 0
+            tall = (force is None and 8 < m <= 16 and mode == EPI_ADD and lazy is None and experts is None and n % 16 == 0
                     and ((k >= 8192 and m >= 12) or (k >= 4096 and n <= 2048)) and x.stride(0) % 8 == 0 and x.stride(1) == 1)
             nxt = getattr(out, "_li_next_norm", None) if mode == EPI_ADD else None
             if (nxt is not None and m <= 16 and n % 32 == 0 and out.data_ptr() % 16 == 0 and nxt.dtype == torch.float32
