@@ -3,6 +3,8 @@
 // every size taken at run time.
 #include "common.h"
 
+#include <chrono>
+
 // ---------------------------------------------------------------------------
 // x[t, :] = float(table[token[t], :])          (src/model/model.cpp:101-118)
 // ---------------------------------------------------------------------------
@@ -242,12 +244,33 @@ extern "C" int li_rope_table(const float* inv_freq, const int* pos, float* out, 
 // sin of pos * inv_freq as rope_table_kernel does, so that a step needs no
 // second small kernel before its first layer.
 // ---------------------------------------------------------------------------
+// What the step before chose, for the host (ring null: not wanted): row i's token and the number of this step in one word of page-locked memory,
+// written past the caches, so that neither order nor a flag is needed; the host polls for the number.  `steps`: one counter a row, all of them `rows`
+// advanced by every step.
+struct TokensOut {
+    const int* tokens;
+    unsigned* steps;
+    unsigned long long* ring;                        // [TOKEN_RING][rows]
+    int rows;
+};
+enum { TOKEN_RING = 4 };
+
 __global__ void decode_prepare_kernel(const int* __restrict__ seq_slot, int* __restrict__ lens,
                                       int* __restrict__ pos, int* __restrict__ ctx, int n, int scratch_slot,
-                                      const float* __restrict__ inv_freq, float* __restrict__ cos_sin, int n_freq) {
+                                      const float* __restrict__ inv_freq, float* __restrict__ cos_sin, int n_freq, TokensOut out) {
     // one workgroup a row: thread 0 does the bookkeeping, all threads the row's angles
     const int i = blockIdx.x;
     const int s = seq_slot[i];
+    if (out.ring) {
+        if (threadIdx.x == 0) {
+            const unsigned step = out.steps[i] + 1;
+            out.steps[i] = step;
+            __hip_atomic_store(out.ring + (int64_t)(step % TOKEN_RING) * out.rows + i, (unsigned long long)step << 32 | (unsigned)out.tokens[i],
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (i == 0)
+            for (int j = n + threadIdx.x; j < out.rows; j += blockDim.x) out.steps[j] += 1;
+    }
     const int l = s == scratch_slot ? 0 : lens[s];
     __syncthreads();                                  // every thread has read the length before it changes
     if (threadIdx.x == 0) {
@@ -265,11 +288,34 @@ __global__ void decode_prepare_kernel(const int* __restrict__ seq_slot, int* __r
 }
 
 extern "C" int li_decode_prepare(const int* seq_slot, int* lens, int* pos, int* ctx, int n, int scratch_slot,
-                                 const float* inv_freq, float* cos_sin, int n_freq, hipStream_t stream) {
+                                 const float* inv_freq, float* cos_sin, int n_freq, const int* tokens, unsigned* steps,
+                                 unsigned long long* ring, int rows, hipStream_t stream) {
     if (n <= 0) return LI_OK;
     if (cos_sin && (!inv_freq || n_freq <= 0)) return LI_BAD_ARG;
-    decode_prepare_kernel<<<n, 64, 0, stream>>>(seq_slot, lens, pos, ctx, n, scratch_slot, inv_freq, cos_sin, n_freq);
+    if (ring && (!tokens || !steps || rows < n || ((uintptr_t)ring & 7))) return LI_BAD_ARG;
+    // the device's address of the ring, which has to be page-locked memory
+    if (ring && hipHostGetDevicePointer((void**)&ring, ring, 0) != hipSuccess) return LI_BAD_ARG;
+    decode_prepare_kernel<<<n, 64, 0, stream>>>(seq_slot, lens, pos, ctx, n, scratch_slot, inv_freq, cos_sin, n_freq,
+                                                TokensOut{tokens, steps, ring, rows});
     LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
+// Waits on the host until the first n rows of `ring` bear step number `step`, at most `micros`; their tokens go to `out`.  1: not yet.
+extern "C" int li_wait_tokens(const unsigned long long* ring, int rows, int n, unsigned step, int* out, int64_t micros) {
+    const unsigned long long* p = ring + (int64_t)(step % TOKEN_RING) * rows;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(micros);
+    for (int i = 0, spins = 0; i < n;) {
+        const unsigned long long v = __atomic_load_n(p + i, __ATOMIC_ACQUIRE);
+        if ((unsigned)(v >> 32) == step) {
+            out[i++] = (int)(unsigned)v;
+            continue;
+        }
+        if (++spins % 64 == 0 && std::chrono::steady_clock::now() >= until) return 1;
+#if !defined(__HIP_DEVICE_COMPILE__)
+        __builtin_ia32_pause();
+#endif
+    }
     return LI_OK;
 }
 

@@ -112,15 +112,15 @@ class GraphDecodeRunner:
             self.bufs = {k: torch.zeros((n,), dtype=torch.int32, device=dev) for k in ("tokens", "slots", "pos", "ctx")}
             self.bufs["rows"] = torch.arange(n, dtype=torch.int32, device=dev)
             self.bufs["temperature"] = torch.ones((1,), dtype=torch.float32, device=dev)
-            # where the tokens of the steps in flight arrive on the host
-            self.bufs["host"] = [Tensor.pinned((n,), torch.int32) for _ in range(3)]
-            self.bufs["done"] = [torch.cuda.Event() for _ in range(3)]
+            # where the tokens arrive on the host: those of a step that another follows by that step's bookkeeping kernel (counters on the
+            # device, the ring), the last step's by a copy
+            self.bufs["steps"] = torch.zeros((n,), dtype=torch.int32, device=dev)
+            self.bufs["host"] = [Tensor.pinned((ops.TOKEN_RING, n), torch.int64), Tensor.pinned((n,), torch.int32)]
+            self.bufs["launched"] = 0              # steps enqueued so far: what the counters will stand at
             engine._graph_bufs = self.bufs
         self.current = None            # the rows' slots now in the buffers
         self._ahead = None             # a step enqueued before its predecessor's tokens were read
         self._fed = None               # slot -> the token that step was fed on the device
-        self._host, self._done = self.bufs["host"], self.bufs["done"]
-        self._turn = 0
         # one table of rotation angles for the whole model: the bookkeeping kernel fills it
         wanted = [p.step_table() for p in engine.model.positions.values() if hasattr(p, "step_table")]
         wanted = [w for w in wanted if w is not None]
@@ -130,17 +130,28 @@ class GraphDecodeRunner:
         eng, b = self.engine, self.bufs
         ctx = _GraphContext(b, n, bucket, pages)
         table = ops.decode_prepare(b["slots"], eng.cache.lens_dev, b["pos"], b["ctx"], n, eng.cache.scratch_slot,
-                                   self._table[1] if self._table else None)
+                                   self._table[1] if self._table else None, (b["tokens"], b["steps"], b["host"][0]))
         if table is not None:
             ctx.shared(self._table[0], lambda: table)
         logits = eng.model.forward(ctx, eng.cache)
-        # the sampled tokens go where the next step reads its tokens (the copy to the host is enqueued
-        # between the two steps)
+        # the sampled tokens go where the next step reads its tokens, and sends them to the host
         self.sampler.sample(logits, b["slots"][:n], eng.cache, out=b["tokens"], temperature_dev=b["temperature"])
 
     def _launch(self, slots, tokens):
-        """Enqueues one step for ``slots`` and the copy of its tokens to pinned host memory.
+        """Enqueues one step for ``slots``; returns them and the step's number.
         ``tokens`` None: the tokens the step before left on the device are fed."""
+        b = self.bufs
+        try:
+            self._enqueue(slots, tokens)
+        except BaseException:
+            # whether the step's first kernel ran is not known: go on from a number that none has had
+            b["launched"] += 2
+            b["steps"].fill_((b["launched"] + (1 << 31)) % (1 << 32) - (1 << 31))
+            raise
+        b["launched"] += 1
+        return list(slots), b["launched"]
+
+    def _enqueue(self, slots, tokens):
         eng, cache, b = self.engine, self.engine.cache, self.bufs
         n = len(slots)
         rows = batch_bucket(n, cache.n_slots)
@@ -181,16 +192,18 @@ class GraphDecodeRunner:
             if graphs[old] != "seen":
                 torch.cuda.synchronize()         # a recorded step may still be running: let it finish first
             del graphs[old]
-        self._turn = (self._turn + 1) % len(self._host)
-        host, done = self._host[self._turn], self._done[self._turn]
-        host[:n].copy_(b["tokens"][:n], non_blocking=True)
-        done.record()
-        return list(slots), host, done
 
-    @staticmethod
-    def _collect(step):
-        slots, host, done = step
-        done.synchronize()
+    def _collect(self, step):
+        """The tokens of ``step``, the newest one or the one before it.  Where a step has been enqueued behind it, that step's first kernel
+        sends them and the host polls for them: no copy and no event between two recorded steps (a step
+        of four layers 2,048 wide, batch 1, 263.9 -> 256.2 us, batch 8 373.7 -> 368.5; 4,096 wide 480.1 -> 474.8)."""
+        slots, number = step
+        b = self.bufs
+        if self._ahead is not None and self._ahead[1] == number + 1:
+            return ops.wait_tokens(b["host"][0], len(slots), number + 1)
+        host = b["host"][1]
+        host[:len(slots)].copy_(b["tokens"][:len(slots)], non_blocking=True)
+        torch.cuda.current_stream().synchronize()
         return host[:len(slots)].tolist()
 
     def run(self, slots, tokens, may_follow: bool = False):
@@ -222,5 +235,6 @@ class GraphDecodeRunner:
         """Waits for a step enqueued ahead and drops its tokens.  Its sequences have moved on by
         that step all the same: they can be freed, not continued with other tokens."""
         if self._ahead is not None:
-            self._collect(self._ahead)
-            self._ahead = self._fed = None
+            step, self._ahead = self._ahead, None
+            self._collect(step)
+            self._fed = None

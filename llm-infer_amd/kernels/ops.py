@@ -770,11 +770,16 @@ def linear_rope_store(x, w, inv_freq, rotary_dim, pos, tok_slot, page_table, pag
     return q
 
 
-def decode_prepare(seq_slot, lens, pos, ctx, n, scratch_slot: int = -1, inv_freq=None):
+TOKEN_RING = 4           # steps whose tokens decode_prepare's ring holds
+
+
+def decode_prepare(seq_slot, lens, pos, ctx, n, scratch_slot: int = -1, inv_freq=None, tokens_out=None):
     """The bookkeeping of a decode step on the device: row i's token gets position lens[seq_slot[i]], its
     context is one more, the length grows by one; a row on ``scratch_slot`` (an idle row) gets position 0 and
     changes no length.  With ``inv_freq`` the kernel also fills and returns the step's table of angles
-    (what ``rope_table`` computes from these positions)."""
+    (what ``rope_table`` computes from these positions).  ``tokens_out`` (tokens, steps, ring): the rows' tokens, as they are
+    before this step, go to the host (``wait_tokens``): int32 tokens and zeroed int32 counters on the device, a row each, and
+    page-locked int64 [TOKEN_RING, rows]."""
     _dev(seq_slot, lens, pos, ctx, inv_freq)
     for a in (seq_slot, lens, pos, ctx):
         _need(a.dtype == torch.int32, "decode_prepare: int32 arrays")
@@ -783,10 +788,29 @@ def decode_prepare(seq_slot, lens, pos, ctx, n, scratch_slot: int = -1, inv_freq
     if inv_freq is not None:
         _need(inv_freq.dtype == torch.float32 and inv_freq.numel() > 0, "decode_prepare: float32 frequencies")
         table = torch.empty((n, inv_freq.numel(), 2), dtype=torch.float32, device=inv_freq.device)
+    tokens, steps, ring = tokens_out or (None, None, None)
+    if tokens_out is not None:
+        _dev(tokens, steps)
+        _need(tokens.dtype == torch.int32 and steps.dtype == torch.int32 and ring.dtype == torch.int64 and ring.is_pinned()
+              and ring.is_contiguous() and ring.dim() == 2 and ring.shape[0] == TOKEN_RING
+              and min(tokens.numel(), steps.numel()) >= ring.shape[1] >= n, "decode_prepare: tokens, counters and a ring of as many rows")
     _check(core().li_decode_prepare(_ptr(seq_slot), _ptr(lens), _ptr(pos), _ptr(ctx), n, int(scratch_slot),
                                     _ptr(inv_freq), _ptr(table), inv_freq.numel() if inv_freq is not None else 0,
-                                    _stream()), "decode_prepare")
+                                    _ptr(tokens), _ptr(steps), c_void_p(ring.data_ptr()) if ring is not None else None,
+                                    ring.shape[1] if ring is not None else 0, _stream()), "decode_prepare")
     return table
+
+
+def wait_tokens(ring, n: int, step: int) -> list[int]:
+    """The first ``n`` rows' tokens that the decode_prepare of step number ``step`` sent to ``ring`` (the newest step or
+    one of the TOKEN_RING - 1 before it).  Polls (as a wait for an event does); if the stream ends without them, that is an error."""
+    _need(0 < n <= ring.shape[1], "wait_tokens: the rows of the ring")
+    out = (ctypes.c_int * n)()
+    wait = lambda micros: core().li_wait_tokens(c_void_p(ring.data_ptr()), ring.shape[1], n, ctypes.c_uint(step & 0xFFFFFFFF), out, c_int64(micros))
+    while wait(1_000_000):
+        if torch.cuda.current_stream().query() and wait(0):          # (a failed launch raises here)
+            raise KernelError(f"wait_tokens: the device is done and step {step}'s tokens have not come")
+    return list(out)
 
 
 EDIT_WORDS = 896         # what li_cache_edit takes in one launch

@@ -1110,3 +1110,38 @@ def test_sampling_kernels(ops):
     freq = torch.bincount(drawn.cpu().long(), minlength=V).double() / n
     sigma = torch.sqrt(p * (1 - p) / n)
     assert ((freq - p).abs() < 5 * sigma + 1e-9).all(), (freq.tolist(), p.tolist())
+
+
+@pytest.mark.parametrize("rows,n", [(1, 1), (5, 3), (130, 130), (130, 66)])
+def test_a_steps_first_kernel_sends_the_tokens_before_it_to_the_host(ops, rows, n):
+    """decode_prepare's ring of tokens, recorded and replayed: every step's own tokens, rows that a smaller step leaves out keep
+    count, a number that no step had is an error and not a wait for ever."""
+    from llm_infer_amd.tensor import Tensor
+    i32 = lambda v: torch.full((rows,), v, dtype=torch.int32, device=DEV)
+    slots = torch.arange(rows, dtype=torch.int32, device=DEV)
+    lens, pos, ctx, tokens, steps = i32(7), i32(0), i32(0), i32(0), i32(0)
+    ring = Tensor.pinned((ops.TOKEN_RING, rows), torch.int64)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())                  # (the kernel indexes by what the lines above fill in)
+    torch.cuda.synchronize()
+    assert slots.tolist() == list(range(rows)) and lens.tolist() == [7] * rows
+    graphs = {}
+    with torch.cuda.stream(side):
+        ops.decode_prepare(slots, lens, pos, ctx, rows, -1, None, (tokens, steps, ring))
+        assert ops.wait_tokens(ring, rows, 1) == [0] * rows
+        for k in (rows, n):
+            graphs[k] = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graphs[k], stream=side):
+                ops.decode_prepare(slots, lens, pos, ctx, k, -1, None, (tokens, steps, ring))
+        for step in range(2, 12):
+            k = rows if step % 3 else n
+            tokens.copy_(torch.arange(rows, dtype=torch.int32) * 1000 + step - (1 << 20))
+            graphs[k].replay()
+            assert ops.wait_tokens(ring, k, step) == [r * 1000 + step - (1 << 20) for r in range(k)]
+        with pytest.raises(ops.KernelError):
+            ops.wait_tokens(ring, n, 12)
+    assert steps.tolist() == [11] * rows
+    with pytest.raises(ops.KernelError):
+        ops.decode_prepare(slots, lens, pos, ctx, rows, -1, None, (tokens, steps, ring[:2]))
+    with pytest.raises(ops.KernelError):
+        ops.wait_tokens(ring, rows + 1, 1)
