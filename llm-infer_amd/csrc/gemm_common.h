@@ -6,7 +6,7 @@
 enum { EPI_STORE = 0, EPI_ADD = 1, EPI_SWIGLU = 2, EPI_ROPE = 3, EPI_GEGLU = 4, EPI_BIAS = 5, EPI_CLAMPGLU = 6 };
 
 // What EPI_BIAS and EPI_CLAMPGLU need (handed over where EPI_ROPE's RopeStore is).  EPI_BIAS: C = act(sums + bias[n]),
-// act 0: none, 1: the square of relu, 2: tanh (with an activation the bias may be null).
+// act 0: none, 1: the square of relu, 2: tanh, 3: limit * tanh(. / limit) (with an activation the bias may be null).
 // EPI_CLAMPGLU: columns 2j (gate) and 2j + 1 (up), each plus its bias (null: none), give
 //   h[m, j] = g sigmoid(alpha g) (u + shift),  g = min(gate, limit),  u = clamp(up, -limit, limit);
 // the outputs from tail_col on (an expert of another kind behind the others) take tail_limit.
@@ -136,6 +136,7 @@ __device__ __forceinline__ void epilogue_extra4(const Epilogue& e, int m, int n,
         o[j] = v[j] + (e.gp.bias && n + j < e.N ? e.gp.bias[n + j] : 0.f);
         if (e.gp.act == 1) { const float r = fmaxf(o[j], 0.f); o[j] = r * r; }
         else if (e.gp.act == 2) o[j] = tanhf(o[j]);
+        else if (e.gp.act == 3) o[j] = e.gp.limit * tanhf(o[j] / e.gp.limit);
     }
     if ((e.N & 3) == 0) store_four(e.C, e.out_dt, (int64_t)m * e.N + n, o);
     else {
@@ -394,7 +395,7 @@ static int make_epilogue(Epilogue& e, void* C, int mode, int out_dt, int M, int 
     e.gp = GluParams{};
     if (mode == EPI_BIAS || mode == EPI_CLAMPGLU) {
         const GluParams* gp = (const GluParams*)rs;            // these modes' own parameters come in the same place
-        if (!gp || (mode == EPI_BIAS && ((!gp->bias && !gp->act) || gp->act < 0 || gp->act > 2)) || (mode == EPI_CLAMPGLU && !(gp->limit > 0.f && gp->tail_limit > 0.f)))
+        if (!gp || (mode == EPI_BIAS && ((!gp->bias && !gp->act) || gp->act < 0 || gp->act > 3 || (gp->act == 3 && !(gp->limit > 0.f)))) || (mode == EPI_CLAMPGLU && !(gp->limit > 0.f && gp->tail_limit > 0.f)))
             return LI_BAD_ARG;
         e.gp = *gp;
         return LI_OK;

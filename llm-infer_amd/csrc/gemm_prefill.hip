@@ -299,6 +299,7 @@ __device__ __forceinline__ void rows_out(const Epilogue& e, const f32x4 (&acc)[N
                         for (int q = 0; q < 4; ++q) {
                             if (e.gp.act == 1) { const float t = fmaxf(v[q], 0.f); v[q] = t * t; }
                             else if (e.gp.act == 2) v[q] = tanhf(v[q]);
+                            else if (e.gp.act == 3) v[q] = e.gp.limit * tanhf(v[q] / e.gp.limit);
                         }
                     }
                     struct alignas(4 * sizeof(OT)) Four { OT v[4]; };

@@ -17,7 +17,7 @@ from ..tensor import Tensor
 PAGE = 64
 DT = {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}
 EPI_STORE, EPI_ADD, EPI_SWIGLU, EPI_ROPE, EPI_GEGLU, EPI_BIAS, EPI_CLAMPGLU = 0, 1, 2, 3, 4, 5, 6
-EPI_ACTS = {None: 0, "relu2": 1, "tanh": 2}       # activations that EPI_BIAS can apply
+EPI_ACTS = {None: 0, "relu2": 1, "tanh": 2, "softcap": 3}       # activations that EPI_BIAS can apply
 GATED = (EPI_SWIGLU, EPI_GEGLU, EPI_CLAMPGLU)   # gate and up rows interleaved in W, act(gate) * up written
 _STATUS = {1: "bad argument", 2: "unsupported size or alignment", 3: "HIP launch error"}
 
@@ -239,8 +239,8 @@ class _GluParams(ctypes.Structure):
 
 def glu_params(bias=None, limit: float = 1.0, tail_limit: float | None = None, alpha: float = 1.702, shift: float = 1.0,
                tail_col: int | None = None, act: str | None = None):
-    """What ``linear`` needs for EPI_BIAS (``bias`` float32 [N]; ``act`` "relu2", the square of relu, or "tanh" of the sums and
-    the bias, which may then be None) and EPI_CLAMPGLU (gate and up columns interleaved; a bias
+    """What ``linear`` needs for EPI_BIAS (``bias`` float32 [N]; ``act`` "relu2", the square of relu, "tanh" or "softcap",
+    limit * tanh(. / limit), of the sums and the bias, which may then be None) and EPI_CLAMPGLU (gate and up columns interleaved; a bias
     for every column or None; g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(alpha g) (u + shift); the
     outputs from ``tail_col`` on take ``tail_limit``).  Keeps the bias alive as long as it lives itself."""
     _need(bias is None or (bias.dtype == torch.float32 and bias.dim() == 1 and bias.is_contiguous() and bias.is_cuda),

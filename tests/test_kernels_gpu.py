@@ -1112,6 +1112,19 @@ def test_sampling_kernels(ops):
     assert ((freq - p).abs() < 5 * sigma + 1e-9).all(), (freq.tolist(), p.tolist())
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 2050, 256), (8, 3000, 512), (17, 130, 96), (40, 72, 160), (130, 520, 2048), (3, 33, 40)])
+def test_a_soft_cap_in_the_products_epilogue(ops, M, N, K):
+    """Bit for bit the product and the pass over its values behind it, for every kernel that the sizes and types choose."""
+    g = torch.Generator().manual_seed(M + N + K)
+    for dt in (torch.float32, torch.float16, torch.bfloat16):
+        x, w = torch.randn(M, K, generator=g).to(DEV, dt), torch.randn(N, K, generator=g).to(DEV, dt)
+        for weight in (w, ops.prepare_weight(w)):
+            got = ops.linear(x, weight, ops.EPI_BIAS, out_dtype=torch.float32, params=ops.glu_params(act="softcap", limit=3.5))
+            assert torch.equal(got, ops.softcap(ops.linear(x, weight, out_dtype=torch.float32), 3.5))
+    with pytest.raises(ops.KernelError):
+        ops.linear(x, w, ops.EPI_BIAS, out_dtype=torch.float32, params=ops.glu_params(act="softcap", limit=0.0))
+
+
 @pytest.mark.parametrize("rows,n", [(1, 1), (5, 3), (130, 130), (130, 66)])
 def test_a_steps_first_kernel_sends_the_tokens_before_it_to_the_host(ops, rows, n):
     """decode_prepare's ring of tokens, recorded and replayed: every step's own tokens, rows that a smaller step leaves out keep
