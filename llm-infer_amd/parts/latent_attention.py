@@ -37,6 +37,7 @@ class LatentAttention(Part):
     product follows.  ``names``: local tensor names."""
 
     takes_lazy_norm = True
+    writes_rows = True          # forward_into overwrites the rows it is handed
 
     def __init__(self, *, hidden_size, n_heads, head_dim, rot_dim, v_head_dim, kv_rank, scale, norm_eps, sink=False,
                  gate=False, window=None, q_rank=None, names=None, position=None, prefix, dtype, device):
@@ -98,6 +99,15 @@ class LatentAttention(Part):
         return KVSpec(1, ops.padded_map_dim(self.key_dim), self.window, self.kv_rank, None, "maps")
 
     def forward(self, h, ctx, view, residual, owns_cache=True):
+        ops.linear(self._outputs(h, ctx, view, owns_cache), self.wo, ops.EPI_ADD, out=residual)
+
+    def forward_into(self, h, out, ctx, view, owns_cache=True):
+        """The mixer's result written over the float32 rows ``out`` (nothing is added to what they held)."""
+        ops.linear(self._outputs(h, ctx, view, owns_cache), self.wo, out=out)
+        return None
+
+    def _outputs(self, h, ctx, view, owns_cache):
+        """The heads' outputs side by side, [T, H * dv] in the model's type."""
         if not owns_cache:
             raise ValueError("latent attention writes its own latents in every run")
         H, d, rd, dv, r = self.n_heads, self.head_dim, self.rot_dim, self.v_head_dim, self.kv_rank
@@ -122,4 +132,4 @@ class LatentAttention(Part):
                                key_shares=ctx.page_shares(1, H) if sixteen and ctx.is_decode else 1)
         o = torch.empty((a.shape[0], H * dv), dtype=self.dtype, device=a.device)
         ops.head_linear(a, 0, r, self.w_uv, o, 0, dv, gate=proj if self.gate else None, gate_col=kv_col + r + rd)
-        ops.linear(o, self.wo, ops.EPI_ADD, out=residual)
+        return o
