@@ -147,15 +147,26 @@ __device__ __forceinline__ float block_total(float v, float (&mine)[16], int wav
     return waves_in_order<W>(mine, waves);
 }
 
+// A token shift that reads the normed rows, in a step of one token a sequence (mu null: none): see token_shift_kernel.  A thread reads the
+// elements of the state that it then writes.
+struct RowShift {
+    const float* mu;
+    float* state;                // [slots, d]
+    const int* pos;
+    const int* tok_slot;
+};
+
 // The same with 16-byte loads: N4 pieces of four elements a thread (d a multiple of 4, 16-byte aligned rows), of up to 512 threads
 // up to two pieces.  With its launch, alpha x + y1 + y2 and its norm behind a product: 1 row of 2,048 2.5 -> 2.3 us, of 4,096 3.1 -> 2.6 (a
 // piece after the other and four barriers; now everything at once and two).
-template <class TC, int N4, bool TOGETHER>
+// SHIFT: `copy` takes the shifted rows.  The state and its weights come with the rest, so that the shift costs no launch (a decode step of
+// four layers 4,096 wide, three of which another follows: 470 -> 451 us).
+template <class TC, int N4, bool TOGETHER, bool SHIFT = false>
 __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restrict__ x, float alpha,
                                                                  const float* __restrict__ y1, float s1,
                                                                  const float* __restrict__ y2, float s2,
                                                                  const float* __restrict__ w, float eps,
-                                                                 TC* __restrict__ copy, int d) {
+                                                                 TC* __restrict__ copy, int d, RowShift sh) {
     struct alignas(4 * sizeof(TC)) Out4 { TC v[4]; };
     constexpr int W = N4 <= 2 ? 8 : 16;
     __shared__ float st[2][16];
@@ -164,8 +175,14 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     f32x4* x4 = (f32x4*)(x + base);
     const f32x4 *a4 = (const f32x4*)(y1 + base), *b4 = y2 ? (const f32x4*)(y2 + base) : nullptr, *w4 = (const f32x4*)w;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 v[N4], av[N4], bv[N4], wv[N4];
+    f32x4 v[N4], av[N4], bv[N4], wv[N4], pv[SHIFT ? N4 : 1], mv[SHIFT ? N4 : 1];
     int at[N4];
+    float* old = nullptr;                                // the row that this sequence's step before left
+    bool first = true;
+    if constexpr (SHIFT) {
+        old = sh.state + (int64_t)sh.tok_slot[blockIdx.x] * d;
+        first = sh.pos[blockIdx.x] == 0;
+    }
     float s = 0.f, ss = 0.f;
     auto fetch = [&](int u) {
         v[u] = x4[at[u]];
@@ -189,7 +206,11 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
     for (int u = 0; u < N4; ++u) at[u] = min((int)(threadIdx.x + u * blockDim.x), n4 - 1);
     if constexpr (TOGETHER) {
 #pragma unroll
-        for (int u = 0; u < N4; ++u) { fetch(u); wv[u] = w4[at[u]]; }
+        for (int u = 0; u < N4; ++u) {
+            fetch(u);
+            wv[u] = w4[at[u]];
+            if constexpr (SHIFT) { pv[u] = ((const f32x4*)old)[at[u]]; mv[u] = ((const f32x4*)sh.mu)[at[u]]; }
+        }
 #pragma unroll
         for (int u = 0; u < N4; ++u) add(u);
     } else {
@@ -213,8 +234,13 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
             Out4 c4;
             if (!TOGETHER) wv[u] = w4[at[u]];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) { r[q] = v[u][q] / sd * wv[u][q]; c4.v[q] = from_f32<TC>(r[q]); }
+            for (int q = 0; q < 4; ++q) {
+                r[q] = v[u][q] / sd * wv[u][q];
+                if constexpr (SHIFT) c4.v[q] = from_f32<TC>(r[q] + ((first ? 0.f : pv[u][q]) - r[q]) * mv[u][q]);
+                else c4.v[q] = from_f32<TC>(r[q]);
+            }
             x4[at[u]] = r;
+            if constexpr (SHIFT) ((f32x4*)old)[at[u]] = r;
             if (copy) ((Out4*)(copy + base))[at[u]] = c4;
         }
     }
@@ -222,15 +248,32 @@ __global__ __launch_bounds__(1024) void add_layernorm_vec_kernel(float* __restri
 
 extern "C" int li_add_layernorm(float* x, float alpha, const float* y1, float s1, const float* y2, float s2,
                                 const float* w, float eps, void* copy, int copy_dt, int n_rows, int d,
-                                hipStream_t stream) {
+                                const float* mu, float* state, const int* pos, const int* tok_slot, hipStream_t stream) {
     if (n_rows <= 0) return LI_OK;
     if (d <= 0 || !y1) return LI_BAD_ARG;
+    const RowShift sh{mu, state, pos, tok_slot};
+    if (mu) {                                    // rows of up to 8,192, which stay in a workgroup's registers
+        if (!state || !pos || !tok_slot || !copy) return LI_BAD_ARG;
+        if (d % 4 || d > 8192 || (((uintptr_t)x | (uintptr_t)y1 | (uintptr_t)y2 | (uintptr_t)w | (uintptr_t)copy | (uintptr_t)mu | (uintptr_t)state) & 15)) return LI_UNSUPPORTED;
+        const int per = d <= 2048 ? 1 : (d <= 4096 ? 2 : 4);
+        const dim3 vb(((d / 4 + per - 1) / per + 63) / 64 * 64);
+#define GO1(TC, N) add_layernorm_vec_kernel<TC, N, true, true><<<n_rows, vb, 0, stream>>>(x, alpha, y1, s1, y2, s2, w, eps, (TC*)copy, d, sh)
+#define GO(TC) do { if (per == 1) GO1(TC, 1); else if (per == 2) GO1(TC, 2); else GO1(TC, 4); } while (0)
+        if (copy_dt == DT_F32) GO(float);
+        else if (copy_dt == DT_F16) GO(f16);
+        else if (copy_dt == DT_BF16) GO(bf16);
+        else return LI_BAD_ARG;
+#undef GO
+#undef GO1
+        LI_CHECK_LAUNCH();
+        return LI_OK;
+    }
     dim3 grid(n_rows), block(d >= 2048 ? 512 : (d >= 256 ? 256 : 64));
     const bool aligned = d % 4 == 0 && !(((uintptr_t)x | (uintptr_t)y1 | (uintptr_t)y2 | (uintptr_t)w | (uintptr_t)copy) & 15);
     if (aligned && d <= 32 * 1024) {
         const int n4 = d / 4, per = n4 <= 512 ? 1 : (n4 <= 1024 ? 2 : (n4 <= 4096 ? 4 : 8));
         dim3 vb(((n4 + per - 1) / per + 63) / 64 * 64);
-#define GO1(TC, N, TOGETHER) add_layernorm_vec_kernel<TC, N, TOGETHER><<<grid, vb, 0, stream>>>(x, alpha, y1, s1, y2, s2, w, eps, (TC*)copy, d)
+#define GO1(TC, N, TOGETHER) add_layernorm_vec_kernel<TC, N, TOGETHER><<<grid, vb, 0, stream>>>(x, alpha, y1, s1, y2, s2, w, eps, (TC*)copy, d, sh)
 #define GO(TC) do { if (per == 1) GO1(TC, 1, true); else if (per == 2) GO1(TC, 2, true); else if (vb.x <= 512) GO1(TC, 4, true); \
                     else if (per == 4) GO1(TC, 4, false); else GO1(TC, 8, false); } while (0)
         if (!copy || copy_dt == DT_F32) GO(float);

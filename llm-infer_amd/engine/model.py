@@ -183,6 +183,18 @@ class DecoderModel(Part):
                 norms.append((n.weight, n.eps, dt))
         return norms, conv
 
+    def _shift_of_entry(self, i, x, ctx, cache):
+        """The token shift of the rows ``x`` with which the layer of schedule entry ``i`` begins, as the pass that finishes them takes it
+        (``ops.add_layernorm``), or None: in a step of one token a sequence, where nothing rewrites the stream ahead of the layer."""
+        if i >= len(self.schedule) or self._before[i] is not None or ctx.n_tokens != ctx.n_seqs or x.data_ptr() % 16:
+            return None
+        entry = self.schedule[i]
+        layer = self.layers[entry.layer]
+        if entry.cache_from is not None or not hasattr(layer, "input_shift"):
+            return None
+        shift = layer.input_shift(self._views_of(i, cache))
+        return (*shift[:2], ctx, shift[2]) if shift is not None and ops.shift_fits(*shift[:2]) else None
+
     # -- the forward pass of one step ---------------------------------------
     def forward(self, ctx, cache) -> torch.Tensor:
         """Runs the step's tokens through the schedule; returns float32 logits [n_want, vocab]."""
@@ -223,6 +235,8 @@ class DecoderModel(Part):
                     if hasattr(part, "addends"):
                         extra["also"], entered = part.addends(x0, self.schedule[i + 1].pass_no), True
                 layer.forward(x, ctx, views, e.cache_from is None, next_norm=first() if first else None, **extra)
+            elif getattr(layer, "takes_next_shift", False):
+                layer.forward(x, ctx, views, e.cache_from is None, next_shift=self._shift_of_entry(i + 1, x, ctx, cache) if self._after[i] is None else None)
             else:
                 layer.forward(x, ctx, views, e.cache_from is None)
             if self._after[i] is not None:

@@ -180,6 +180,8 @@ def _drop_row_stats(x) -> None:
             x._li_normed = None
         if getattr(x, "_li_convolved", None) is not None:      # (its history has moved on: it cannot be taken again)
             raise KernelError("rows are written over before the convolution that was taken of their norm has been read")
+        if getattr(x, "_li_shifted", None) is not None:        # (the state has moved on, likewise)
+            raise KernelError("rows are written over before the token shift that was taken of them has been read")
         x = getattr(x, "_base", None)
 
 
@@ -1120,10 +1122,28 @@ def layernorm(x: torch.Tensor, w: torch.Tensor, eps: float, out_dtype, rows: tor
     return out
 
 
-def add_layernorm(x, alpha: float, addends, w, eps: float, copy_dtype=None):
+def shift_fits(mu, state) -> bool:
+    """True if ``add_layernorm`` can take along a token shift with these weights and this state."""
+    return (mu.dim() == 1 and mu.numel() % 4 == 0 and mu.numel() <= 8192 and mu.dtype == state.dtype == torch.float32
+            and mu.is_contiguous() and state.is_contiguous() and (mu.data_ptr() | state.data_ptr()) % 16 == 0)
+
+
+def shifted_rows(x, mu, state):
+    """The token shift of the rows ``x`` that ``add_layernorm`` has taken along, once; None where it has taken none."""
+    rec = getattr(x, "_li_shifted", None)
+    if rec is None:
+        return None
+    out, weight, of, version = rec
+    _need(weight is mu and of == state.data_ptr() and version == x._version, "the token shift taken of these rows is not the one that is asked for")
+    x._li_shifted = None
+    return out
+
+
+def add_layernorm(x, alpha: float, addends, w, eps: float, copy_dtype=None, shift=None):
     """x <- LN(alpha * x + sum of scale_i * y_i) * w in place on the float32 rows of ``x``; ``addends``: one or
     two (y, scale) with y float32 of x's shape.  ``copy_dtype`` (a 16-bit type): the new rows are returned in
-    that type as well (else None)."""
+    that type as well (else None).  ``shift`` (mu, state, ctx, dtype; no copy with it; ``shift_fits``): the token shift of the new rows in a
+    step of one token a sequence is taken along where all rows are aligned to 16 bytes; ``shifted_rows`` finds it."""
     _need(1 <= len(addends) <= 2, "add_layernorm: one or two addends")
     (y1, s1), (y2, s2) = addends[0], (addends[1] if len(addends) > 1 else (None, 0.0))
     _dev(x, y1, y2, w)
@@ -1135,9 +1155,24 @@ def add_layernorm(x, alpha: float, addends, w, eps: float, copy_dtype=None):
     copy = None
     if copy_dtype is not None and copy_dtype != torch.float32:
         copy = torch.empty(x.shape, dtype=copy_dtype, device=x.device)
+    mu = state = pos = slot = None
+    if shift is not None and any(t is not None and t.data_ptr() % 16 for t in (x, y1, y2, w)):
+        shift = None                                   # (rows that the pass does not take four at a time: the shift runs by itself)
+    if shift is not None:
+        mu, state, ctx, dtype = shift
+        pos, slot, t = ctx.pos, ctx.tok_slot, x.shape[0]
+        _dev(mu, state, pos, slot)
+        _need(copy is None and shift_fits(mu, state) and mu.numel() == x.shape[1] and state.dim() == 2 and state.shape[1] == x.shape[1]
+              and ctx.n_tokens == ctx.n_seqs == t, "add_layernorm: a token shift of these rows, one token a sequence, and no copy")
+        _i32(pos, t, "positions")
+        _i32(slot, t, "slots")
+        copy = torch.empty(x.shape, dtype=dtype, device=x.device)
     _check(mixers().li_add_layernorm(_ptr(x), c_float(alpha), _ptr(y1), c_float(s1), _ptr(y2), c_float(s2), _ptr(w),
                                      c_float(eps), _ptr(copy), DT[copy.dtype] if copy is not None else 0, x.shape[0],
-                                     x.shape[1], _stream()), "add_layernorm")
+                                     x.shape[1], _ptr(mu), _ptr(state), _ptr(pos), _ptr(slot), _stream()), "add_layernorm")
+    if shift is not None:
+        x._li_shifted = (copy, mu, state.data_ptr(), x._version)
+        return None
     return copy
 
 

@@ -200,6 +200,8 @@ class PostNormBlock(Block):
     the float32 rows as they are; the others get them in the compute dtype, a copy that the norm kernel of
     the sub-layer before writes along."""
 
+    takes_next_shift = True         # forward accepts ``next_shift``
+
     def __init__(self, sublayers, alpha: float = 1.0):
         super().__init__(sublayers)
         self.alpha = float(alpha)
@@ -218,7 +220,13 @@ class PostNormBlock(Block):
             s.part.forward(h, y)
         return [(y, 1.0)]
 
-    def forward(self, x, ctx, cache_views, owns_cache=True):
+    def input_shift(self, cache_views):
+        """The token shift with which this layer begins, as the layer before's last pass takes it, or None."""
+        s = self.sublayers[0]
+        return s.part.input_shift(cache_views[0]) if s.role == "mixer" and hasattr(s.part, "input_shift") else None
+
+    def forward(self, x, ctx, cache_views, owns_cache=True, next_shift=None):
+        """``next_shift`` (mu, state, ctx, type): the token shift that reads ``x`` after this layer."""
         views = iter(cache_views)
         copy = None                                  # the rows of x in the compute dtype, if the last norm left them
         for i, s in enumerate(self.sublayers):
@@ -236,4 +244,4 @@ class PostNormBlock(Block):
             nxt = self.sublayers[i + 1] if i + 1 < len(self.sublayers) else None
             wants_copy = nxt is not None and not getattr(nxt.part, "reads_residual", False)
             copy = ops.add_layernorm(x, self.alpha, adds, s.post_norm.weight, s.post_norm.eps,
-                                     nxt.post_norm.dtype if wants_copy else None)
+                                     nxt.post_norm.dtype if wants_copy else None, next_shift if nxt is None else None)

@@ -39,7 +39,14 @@ class ShiftedMixer(Part):
     def cache_specs(self):
         return [StateSpec((self.hidden_size,), "float32")] + cache_specs_of(self.inner)
 
+    def input_shift(self, views):
+        """What the pass that finishes the rows needs to take this part's mixing along (``ops.add_layernorm``)."""
+        return self.mu, views[0].state, self.dtype
+
     def _shift(self, x, ctx, views):
+        ready = ops.shifted_rows(x, self.mu, views[0].state)
+        if ready is not None:
+            return ready
         return ops.token_shift(x, self.mu, views[0].state, ctx.pos, ctx.tok_slot, self.dtype,
                                single=ctx.n_tokens == ctx.n_seqs)
 

@@ -480,3 +480,31 @@ def test_command_line_and_model_info(lib, models):
     info = subprocess.run([sys.executable, os.path.join(root, "bin", "model_info"), folder], capture_output=True, text=True,
                           timeout=300)
     assert info.returncode == 0 and "Architecture: Manirax" in info.stdout and "The tensors fit the model." in info.stdout
+
+
+@pytest.mark.parametrize("rows,d", [(1, 4), (3, 68), (8, 2048), (2, 2052), (5, 4096), (1, 4100), (17, 8192)])
+def test_a_token_shift_in_the_pass_that_finishes_its_rows(rows, d):
+    """Bit for bit the norm and the shift behind it, and the state that either leaves: first tokens and later ones, slots in any order, with one
+    addend and two, in every type; rows that are not aligned to 16 bytes run in two launches as before."""
+    import types
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(rows + d)
+    rand = lambda *shape: torch.randn(*shape, generator=g).to(DEV)
+    x, w, mu, state = rand(rows, d), rand(d), rand(d), rand(rows + 3, d)
+    ctx = types.SimpleNamespace(n_tokens=rows, n_seqs=rows, pos=torch.tensor([0 if i % 3 == 1 else 5 + i for i in range(rows)], dtype=torch.int32, device=DEV),
+                                tok_slot=(torch.randperm(rows + 3, generator=g)[:rows]).to(torch.int32).to(DEV))
+    assert ops.shift_fits(mu, state) and not ops.shift_fits(mu[1:], state)
+    for dtype in (torch.float32, torch.float16, torch.bfloat16):
+        for adds in ([(rand(rows, d), 0.5)], [(rand(rows, d), 1.0), (rand(rows, d), -0.25)]):
+            a, b, sa, sb = x.clone(), x.clone(), state.clone(), state.clone()
+            ops.add_layernorm(a, 1.5, adds, w, 1e-5)
+            want = ops.token_shift(a, mu, sa, ctx.pos, ctx.tok_slot, dtype, single=True)
+            assert ops.add_layernorm(b, 1.5, adds, w, 1e-5, shift=(mu, sb, ctx, dtype)) is None
+            got = ops.shifted_rows(b, mu, sb)
+            assert torch.equal(a, b) and torch.equal(got, want) and torch.equal(sa, sb) and ops.shifted_rows(b, mu, sb) is None
+    odd = torch.empty(rows * d + 1, device=DEV)[1:].view(rows, d).copy_(x)
+    ops.add_layernorm(odd, 1.5, adds, w, 1e-5, shift=(mu, sb, ctx, dtype))
+    assert ops.shifted_rows(odd, mu, sb) is None
+    ops.add_layernorm(b, 1.5, adds, w, 1e-5, shift=(mu, sb, ctx, dtype))
+    with pytest.raises(ops.KernelError):
+        ops.add_layernorm(b, 1.5, adds, w, 1e-5)
