@@ -5,7 +5,7 @@
 // per sequence, the gated RMS norm behind it, and the PolyNorm activation.  Every size is a run-time value.
 // Whatever a norm, a score, an attention weight or a recurrent state is made of is float32 here, whatever
 // the type of the matrices.
-#include "common.h"
+#include "shares.h"
 
 struct Pages {
     const void* k;
@@ -1208,11 +1208,25 @@ __global__ __launch_bounds__(1024) void gated_rmsnorm_kernel(const float* __rest
 // row of 2,048 4.0, 4.0, 3.9 us, of 4,096 4.7, 4.1, 4.7, of 16,384 10.4, 8.3, 9.0; 256 rows of 4,096 8.4, 5.4, 6.2, of 8,192 14.0, 8.2, 9.5; 2,000 rows of
 // 4,096 22.2, 16.3, 18.9, of 5,120 27.4, 20.3, 24.6, of 8,192 40.2, 30.7, 36.9 (32 elements with the spills 45.7).  (16 bytes a load: behind a
 // product 2.2 and 2.8 us for one row of 2,048 and 4,096 where this takes 2.4 and 3.0; but other elements to a thread, so other bits.)
+// Beside the norm, in workgroups of its own: the partial sums of an attention that ran before (part null: none), which would be a launch of their own
+// (a decode step of four layers 4,096 wide: 451 -> 445 us).
+template <class TO>
+struct SharesOf {
+    const float* part;           // [rows, splits, dv]
+    TO* out;
+    int rows, splits, dv;
+};
+
 template <class TO, int N, int THREADS>
 __global__ __launch_bounds__(THREADS) void gated_rmsnorm_reg_kernel(const float* __restrict__ o, const float* __restrict__ w,
                                                                     const float* __restrict__ gate, int gate_stride, TO* __restrict__ out,
-                                                                    int n, float eps) {
+                                                                    int n, float eps, int n_rows, SharesOf<TO> mg) {
     __shared__ float scratch[16];
+    if ((int)blockIdx.x >= n_rows) {
+        const int64_t i = (int64_t)(blockIdx.x - n_rows) * blockDim.x + threadIdx.x;
+        if (i < (int64_t)mg.rows * mg.dv) mg.out[i] = from_f32<TO>(merged_shares(mg.part, i / mg.dv, (int)(i % mg.dv), mg.splits, mg.dv));
+        return;
+    }
     const int64_t t = blockIdx.x;
     const float *orow = o + t * n, *grow = gate + t * gate_stride;
     float v[N], g[N], wv[N];
@@ -1235,12 +1249,15 @@ __global__ __launch_bounds__(THREADS) void gated_rmsnorm_reg_kernel(const float*
 }
 
 extern "C" int li_gated_rmsnorm(const float* o, const float* w, const float* gate, int gate_stride, void* out,
-                                int out_dt, int n_rows, int n, float eps, hipStream_t stream) {
-    if (n_rows <= 0) return LI_OK;
-    if (n <= 0 || gate_stride < n) return LI_BAD_ARG;
+                                int out_dt, int n_rows, int n, float eps, const float* part, void* merged, int rows, int splits, int dv,
+                                hipStream_t stream) {
+    if (n_rows <= 0) return part ? LI_BAD_ARG : LI_OK;
+    if (n <= 0 || gate_stride < n || (part && (!merged || rows < 1 || splits < 1 || dv < 1))) return LI_BAD_ARG;
+    if (part && (n_rows >= 256 || n > 16 * 1024)) return LI_UNSUPPORTED;          // (few rows: the kernel that has them in registers)
     const int wide = min(1024, (n / 4 + 63) / 64 * 64);
     const int threads = n_rows < 256 && wide > 64 ? wide : (n >= 1024 ? 256 : 64);
-#define GO1(TO, N, THREADS) gated_rmsnorm_reg_kernel<TO, N, THREADS><<<n_rows, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps)
+    const int more = part ? (int)(((int64_t)rows * dv + threads - 1) / threads) : 0;
+#define GO1(TO, N, THREADS) gated_rmsnorm_reg_kernel<TO, N, THREADS><<<n_rows + more, threads, 0, stream>>>(o, w, gate, gate_stride, (TO*)out, n, eps, n_rows, SharesOf<TO>{part, (TO*)merged, rows, splits, dv})
 #define GO(TO) do { \
         if (n <= 4 * threads) GO1(TO, 4, 1024); else if (n <= 8 * threads) GO1(TO, 8, 1024); else if (n <= 16 * threads) GO1(TO, 16, 1024); \
         else if (threads <= 256 && n <= 24 * threads) GO1(TO, 24, 256); else if (threads <= 256 && n <= 32 * threads) GO1(TO, 32, 256); \

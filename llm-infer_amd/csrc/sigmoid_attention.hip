@@ -13,7 +13,7 @@
 //            fetched once for the four, through two stages of LDS
 //   decode : one wave per (sequence, key/value head, split of the context); with more than one split the
 //            partial sums are added in ascending order by a second kernel
-#include "common.h"
+#include "shares.h"
 
 #if !defined(KEY_DIM) || !defined(VALUE_DIM)
 #error "compile with -DKEY_DIM=<n> -DVALUE_DIM=<n>"
@@ -287,21 +287,7 @@ __global__ __launch_bounds__(64) void sigmoid_decode_kernel(
 
 template <class T>
 __global__ void sigmoid_merge_kernel(const float* __restrict__ part, T* __restrict__ out, int S, int dv) {
-    const int64_t bh = blockIdx.x;
-    for (int d = threadIdx.x; d < dv; d += blockDim.x) {
-        const float* p = part + bh * S * dv + d;
-        float acc = 0.f;
-        int s = 0;
-        for (; s + 8 <= S; s += 8) {               // eight loads in flight, added in ascending order
-            float v[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = p[(int64_t)(s + i) * dv];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) acc += v[i];
-        }
-        for (; s < S; ++s) acc += p[(int64_t)s * dv];
-        out[bh * dv + d] = from_f32<T>(acc);
-    }
+    for (int d = threadIdx.x; d < dv; d += blockDim.x) out[(int64_t)blockIdx.x * dv + d] = from_f32<T>(merged_shares(part, blockIdx.x, d, S, dv));
 }
 
 // ---------------------------------------------------------------------------
@@ -337,10 +323,23 @@ extern "C" int li_sigattn_prefill(const void* q, void* out, int dt, const void* 
     return LI_OK;
 }
 
+// part [rows, splits, dv] added up: out [rows, dv].
+extern "C" int li_sigattn_merge(const float* part, void* out, int dt, int rows, int splits, int dv, hipStream_t stream) {
+    if (rows <= 0) return LI_OK;
+    if (!part || !out || splits < 1 || dv < 1) return LI_BAD_ARG;
+    const int threads = dv <= 64 ? 64 : (dv <= 128 ? 128 : 256);
+    if (dt == DT_F16) sigmoid_merge_kernel<f16><<<rows, threads, 0, stream>>>(part, (f16*)out, splits, dv);
+    else if (dt == DT_BF16) sigmoid_merge_kernel<bf16><<<rows, threads, 0, stream>>>(part, (bf16*)out, splits, dv);
+    else return LI_BAD_ARG;
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
+// later: the partial sums are left to whoever adds them up (li_sigattn_merge, li_gated_rmsnorm).
 extern "C" int li_sigattn_decode(const void* q, void* out, int dt, const void* k, const void* v, int64_t page_stride,
                                  const int* page_table, int max_pages, const int* seq_slot, const int* seq_ctx,
                                  const float* bias, int n_seqs, int H, int G, int dv, float scale, int window, int splits,
-                                 float* part, hipStream_t stream) {
+                                 float* part, int later, hipStream_t stream) {
     if (check_heads(H, G, dv) || splits < 1 || splits > 64 || (splits > 1 && !part)) return LI_BAD_ARG;
     if (n_seqs <= 0) return LI_OK;
     CachePtrs c{k, v, page_stride, page_table, max_pages};
@@ -352,7 +351,7 @@ extern "C" int li_sigattn_decode(const void* q, void* out, int dt, const void* k
     do {                                                                                                             \
         auto kfn = group > 32 ? sigmoid_decode_kernel<T, false> : sigmoid_decode_kernel<T, true>;                   \
         kfn<<<grid, block, 0, stream>>>((const T*)q, (T*)out, part, c, seq_slot, seq_ctx, bias, H, G, dv, scale, window); \
-        if (splits > 1) sigmoid_merge_kernel<T><<<n_seqs * H, dv <= 64 ? 64 : (dv <= 128 ? 128 : 256), 0, stream>>>(part, (T*)out, splits, dv); \
+        if (splits > 1 && !later) sigmoid_merge_kernel<T><<<n_seqs * H, dv <= 64 ? 64 : (dv <= 128 ? 128 : 256), 0, stream>>>(part, (T*)out, splits, dv); \
     } while (0)
     if (dt == DT_F16) GO(f16); else if (dt == DT_BF16) GO(bf16); else return LI_BAD_ARG;
 #undef GO

@@ -29,8 +29,9 @@ MIXER_SOURCES = ("mixers.hip",)
 # the headers a library's sources include (its stamp covers them)
 HEADERS = {"libli_core.so": ("common.h", "gemm_common.h", "no_alloc.h"), "libli_hybrid.so": ("common.h", "conv.h"),
            "libli_recurrent.so": ("common.h", "conv.h"), "libli_experts.so": ("common.h", "gemm_common.h"),
-           "libli_f32.so": ("common.h", "gemm_common.h")}
+           "libli_f32.so": ("common.h", "gemm_common.h"), "libli_mixers.so": ("common.h", "shares.h")}
 DEFAULT_HEADERS = ("common.h",)
+SIGMOID_ATTN_HEADERS = ("common.h", "shares.h")
 FLAGS = ["--offload-arch=" + ARCH, "-O3", "-std=c++17", "-fPIC",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", "-Wno-unused-command-line-argument"]
 
@@ -75,7 +76,7 @@ def _hipcc() -> str:
 
 def _stamp(sources, defines, lib_name="") -> str:
     h = hashlib.sha256()
-    for name in tuple(sources) + HEADERS.get(lib_name, DEFAULT_HEADERS):
+    for name in tuple(sources) + HEADERS.get(lib_name, SIGMOID_ATTN_HEADERS if lib_name.startswith("libli_sigattn") else DEFAULT_HEADERS):
         with open(os.path.join(CSRC, name), "rb") as f:
             h.update(name.encode() + b"\0" + f.read())
     h.update(" ".join(FLAGS + list(defines)).encode())

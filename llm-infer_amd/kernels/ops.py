@@ -1369,9 +1369,10 @@ def sigmoid_attention_prefill(q, kv, meta, bias, n_heads, n_kv_heads, k_dim, v_h
 
 
 def sigmoid_attention_decode(q, kv, seq_slot, seq_ctx, n_seqs, bias, n_heads, n_kv_heads, k_dim, v_head_dim, v_dim,
-                             scale, window=None, splits: int = 1):
+                             scale, window=None, splits: int = 1, later: bool = False):
     """16-bit sigmoid attention for one new token per sequence; q [B, H, k_dim].  The context is cut into
-    ``splits`` parts whose sums are added in ascending order."""
+    ``splits`` parts whose sums are added in ascending order; ``later``: by whoever takes the ``PendingMerge`` that comes back
+    with the rows, (rows, None or that)."""
     k_pages, v_pages, page_stride, page_table = _sigattn_check(q, kv, bias, n_heads, n_kv_heads, k_dim, v_head_dim, v_dim)
     _dev(seq_slot, seq_ctx)
     _need(q.shape[0] == n_seqs and seq_slot.numel() >= n_seqs and seq_ctx.numel() >= n_seqs, "per-sequence arrays too short")
@@ -1383,8 +1384,24 @@ def sigmoid_attention_decode(q, kv, seq_slot, seq_ctx, n_seqs, bias, n_heads, n_
     _check(_sigattn_lib(k_dim, v_dim).li_sigattn_decode(
         _ptr(q), _ptr(out), DT[q.dtype], _ptr(k_pages), _ptr(v_pages), c_int64(page_stride), _ptr(page_table),
         page_table.shape[1], _ptr(seq_slot), _ptr(seq_ctx), _ptr(bias), n_seqs, n_heads, n_kv_heads, v_head_dim,
-        c_float(scale), int(window or 0), splits, _ptr(part), _stream()), "sigattn_decode")
+        c_float(scale), int(window or 0), splits, _ptr(part), int(bool(later)), _stream()), "sigattn_decode")
+    if later:
+        return out, PendingMerge(part, out, _sigattn_lib(k_dim, v_dim)) if splits > 1 else None
     return out
+
+
+class PendingMerge:
+    """Partial sums [B, H, splits, dv] that are still to be added up into the rows ``out`` [B, H, dv]: by a kernel that takes them along
+    (``gated_rmsnorm``), else by ``finish``."""
+
+    def __init__(self, part, out, lib):
+        self.part, self.out, self.lib = part, out, lib
+        self.rows, self.splits, self.dv = part.shape[0] * part.shape[1], part.shape[2], part.shape[3]
+
+    def finish(self):
+        if self.part is not None:
+            _check(self.lib.li_sigattn_merge(_ptr(self.part), _ptr(self.out), DT[self.out.dtype], self.rows, self.splits, self.dv, _stream()), "sigattn_merge")
+            self.part = None
 
 
 DECAY_CHUNK = 32        # tokens of one chunk of the chunked decay attention
@@ -1460,9 +1477,9 @@ def decay_attention(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstar
     return out
 
 
-def gated_rmsnorm(o, w, gate_rows, gate_off, eps, out_dtype) -> torch.Tensor:
+def gated_rmsnorm(o, w, gate_rows, gate_off, eps, out_dtype, merge: PendingMerge | None = None) -> torch.Tensor:
     """o / sqrt(mean(o^2) + eps) * w * sigmoid(gate): o float32 [T, n]; the gate is columns gate_off .. gate_off + n
-    of the float32 rows ``gate_rows``."""
+    of the float32 rows ``gate_rows``.  ``merge``: taken along where the rows are few and of one type with it, else finished first."""
     _dev(o, w, gate_rows)
     _f32_rows(o, "gated_rmsnorm o")
     _f32_rows(gate_rows, "gated_rmsnorm gate")
@@ -1471,8 +1488,14 @@ def gated_rmsnorm(o, w, gate_rows, gate_off, eps, out_dtype) -> torch.Tensor:
     _need(gate_rows.shape[0] == t and gate_off + n <= gate_rows.shape[1], "gate columns outside their rows")
     out = torch.empty((t, n), dtype=out_dtype, device=o.device)
     gate = gate_rows.view(-1)[gate_off:]
+    if merge is not None and (merge.part is None or merge.out.dtype != out_dtype or not 1 <= t < 256 or n > 16 * 1024):
+        merge.finish()
+        merge = None
+    along = (_ptr(merge.part), _ptr(merge.out), merge.rows, merge.splits, merge.dv) if merge is not None else (_ptr(None), _ptr(None), 0, 0, 0)
     _check(mixers().li_gated_rmsnorm(_ptr(o), _ptr(w), _ptr(gate), gate_rows.shape[1], _ptr(out), DT[out_dtype], t, n,
-                                     c_float(eps), _stream()), "gated_rmsnorm")
+                                     c_float(eps), *along, _stream()), "gated_rmsnorm")
+    if merge is not None:
+        merge.part = None
     return out
 
 

@@ -54,8 +54,11 @@ class DecayLinearAttention(Part):
     def in_rows(self) -> int:
         return 2 * self.n_heads * (self.head_dim + self.v_head_dim)
 
-    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
-        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v, g from column ``col0`` on: the input product is not run here."""
+    takes_merge = True              # before_output accepts ``merge``
+
+    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, merge=None):
+        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v, g from column ``col0`` on: the input product is not run here.
+        ``merge``: an ``ops.PendingMerge`` of the mixer before, taken along."""
         if not owns_cache:
             raise ValueError("decay attention keeps a state of its own in every run")
         H, d, dv = self.n_heads, self.head_dim, self.v_head_dim
@@ -69,7 +72,7 @@ class DecayLinearAttention(Part):
                                 getattr(ctx, "seq_qstart", None), getattr(ctx, "seq_qlen", None), ctx.n_seqs, H, d, dv,
                                 round_to=self.dtype if sixteen else None, chunked=chunked,
                                 chunks=ops.decay_chunks(ctx) if chunked else None)
-        return ops.gated_rmsnorm(o, self.norm, proj, col0 + 2 * H * d + H * dv, self.norm_eps, self.dtype)
+        return ops.gated_rmsnorm(o, self.norm, proj, col0 + 2 * H * d + H * dv, self.norm_eps, self.dtype, merge)
 
     def addends(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
         return [(ops.linear(self.before_output(h, ctx, view, owns_cache, proj, col0), self.wo, out_dtype=torch.float32), 1.0)]

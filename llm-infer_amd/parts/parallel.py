@@ -62,14 +62,21 @@ class ParallelMixers(Part):
         return [s for b in self.branches for s in cache_specs_of(b)]
 
     def addends(self, h, ctx, views, owns_cache=True):
-        out, at = [], 0
+        out, at, merge = [], 0, None
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32) if getattr(self, "w_in", None) is not None else None
         for i, (branch, scale) in enumerate(zip(self.branches, self.scales)):
             view, at = views_for(branch, views, at)
             shared = {"proj": proj, "col0": self._col0[i]} if proj is not None and self._col0[i] is not None else {}
             if hasattr(branch, "before_output"):
-                # all but its output product, which runs with the others'
-                out.append((ops.PendingProduct(branch.before_output(h, ctx, view, owns_cache, **shared), branch.wo), scale))
+                # all but its output product, which runs with the others'; what completes its rows rides in the next branch's last kernel
+                follows = self.branches[i + 1] if i + 1 < len(self.branches) else None
+                if getattr(branch, "merges_later", False) and merge is None and getattr(follows, "takes_merge", False):
+                    rows, merge = branch.before_output(h, ctx, view, owns_cache, later=True, **shared)
+                elif merge is not None and getattr(branch, "takes_merge", False):
+                    rows, merge = branch.before_output(h, ctx, view, owns_cache, merge=merge, **shared), None
+                else:
+                    rows = branch.before_output(h, ctx, view, owns_cache, **shared)
+                out.append((ops.PendingProduct(rows, branch.wo), scale))
             elif hasattr(branch, "addends"):
                 out += [(y, s * scale) for y, s in branch.addends(h, ctx, view, owns_cache, **shared)]
             else:

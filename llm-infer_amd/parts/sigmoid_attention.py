@@ -71,8 +71,11 @@ class SigmoidAttention(Part):
     def in_rows(self) -> int:
         return (self.n_heads + self.n_kv_heads) * self.head_dim + self.n_kv_heads * self.v_head_dim
 
-    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
-        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v from column ``col0`` on: the input product is not run here."""
+    merges_later = True             # before_output accepts ``later``
+
+    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, later=False):
+        """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v from column ``col0`` on: the input product is not run here.
+        ``later``: (the rows, None or the ``ops.PendingMerge`` that completes them)."""
         if not owns_cache:
             raise ValueError("sigmoid attention writes its own keys and values in every run")
         H, G, d, dv = self.n_heads, self.n_kv_heads, self.head_dim, self.v_head_dim
@@ -90,11 +93,14 @@ class SigmoidAttention(Part):
                                       self.scale, self.window)
         elif ctx.is_decode:
             a = ops.sigmoid_attention_decode(q, kv, ctx.seq_slot, ctx.seq_ctx, ctx.n_seqs, self.bias, H, G, self.k_dim,
-                                             dv, self.v_dim, self.scale, self.window, ctx.decode_splits(G, H))
+                                             dv, self.v_dim, self.scale, self.window, ctx.decode_splits(G, H), later)
+            if later:
+                return a[0].view(a[0].shape[0], H * dv), a[1]
         else:
             a = ops.sigmoid_attention_prefill(q, kv, ops.prefill_meta(ctx), self.bias, H, G, self.k_dim, dv,
                                               self.v_dim, self.scale, self.window)
-        return a.view(a.shape[0], H * dv)
+        a = a.view(a.shape[0], H * dv)
+        return (a, None) if later else a
 
     def addends(self, h, ctx, view, owns_cache=True, proj=None, col0=0):
         return [(ops.linear(self.before_output(h, ctx, view, owns_cache, proj, col0), self.wo, out_dtype=torch.float32), 1.0)]
