@@ -665,18 +665,18 @@ extern "C" int li_token_shift(const float* x, const float* mu, float* state, con
 // One wave a head; a lane keeps up to 4 dimensions (heads of up to 256).
 // ---------------------------------------------------------------------------
 template <class T>
-__global__ __launch_bounds__(256) void rope_norm_store_kernel(
+__device__ __forceinline__ void rope_norm_store_row(
     const float* __restrict__ qkv, int row_stride, const float* __restrict__ inv_freq,
     const float* __restrict__ cos_sin, int rot, int half_pairing, float unit_eps, const int* __restrict__ pos,
-    const int* __restrict__ tok_slot, Pages c, T* __restrict__ q_out, int H, int G, int d, int dv, int dq, int dk,
-    int dvp) {
-    const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
+    const int* __restrict__ tok_slot, const Pages& c, T* __restrict__ q_out, int H, int G, int d, int dv, int dq, int dk,
+    int dvp, int t, int part, int parts) {
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n_waves = blockDim.x >> 6;
     const int p = pos[t];
     const float* row = qkv + (int64_t)t * row_stride;
     int64_t page = 0;
     if (G > 0) page = c.page_table[(int64_t)tok_slot[t] * c.max_pages + p / PAGE];
     const int tp = p % PAGE, half = rot >> 1;
-    for (int head = blockIdx.y * n_waves + wave; head < H + 2 * G; head += n_waves * gridDim.y) {
+    for (int head = part * n_waves + wave; head < H + 2 * G; head += n_waves * parts) {
         if (head < H + G) {
             const float* src = row + (int64_t)head * d;
             float val[4];
@@ -730,24 +730,14 @@ __global__ __launch_bounds__(256) void rope_norm_store_kernel(
     }
 }
 
-extern "C" int li_rope_norm_store(const float* qkv, int row_stride, const float* inv_freq, const float* cos_sin, int rot,
-                                  int half_pairing, float unit_eps, const int* pos, const int* tok_slot, const void* k_pages,
-                                  const void* v_pages, int64_t page_stride, const int* page_table, int max_pages,
-                                  void* q_out, int dt, int n_tokens, int H, int G, int d, int dv, int dq, int dk,
-                                  int dvp, hipStream_t stream) {
-    if (n_tokens <= 0) return LI_OK;
-    if (H <= 0 || G < 0 || d <= 0 || d > 256 || dq < d || dq > 256 || rot < 0 || rot > d || (rot & 1)) return LI_BAD_ARG;
-    if (G > 0 && (dv <= 0 || dk < d || dk > 256 || dk % 16 || dvp < dv || dvp % 16 || !page_table)) return LI_BAD_ARG;
-    if (row_stride < (H + G) * d + G * dv || (rot > 0 && !inv_freq)) return LI_BAD_ARG;
-    Pages c{k_pages, v_pages, page_stride, page_table, max_pages};
-    // few tokens: the heads spread over the grid as well
-    dim3 grid(n_tokens, n_tokens >= 512 ? 1 : (H + 2 * G + 3) / 4), block(256);
-#define GO(T) rope_norm_store_kernel<T><<<grid, block, 0, stream>>>(qkv, row_stride, inv_freq, cos_sin, rot, half_pairing, \
-        unit_eps, pos, tok_slot, c, (T*)q_out, H, G, d, dv, dq, dk, dvp)
-    if (dt == DT_F32) GO(float); else if (dt == DT_F16) GO(f16); else if (dt == DT_BF16) GO(bf16); else return LI_BAD_ARG;
-#undef GO
-    LI_CHECK_LAUNCH();
-    return LI_OK;
+template <class T>
+__global__ __launch_bounds__(256) void rope_norm_store_kernel(
+    const float* __restrict__ qkv, int row_stride, const float* __restrict__ inv_freq,
+    const float* __restrict__ cos_sin, int rot, int half_pairing, float unit_eps, const int* __restrict__ pos,
+    const int* __restrict__ tok_slot, Pages c, T* __restrict__ q_out, int H, int G, int d, int dv, int dq, int dk,
+    int dvp) {
+    rope_norm_store_row<T>(qkv, row_stride, inv_freq, cos_sin, rot, half_pairing, unit_eps, pos, tok_slot, c, q_out, H, G, d, dv, dq, dk, dvp,
+                           blockIdx.x, blockIdx.y, gridDim.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -836,18 +826,18 @@ extern "C" int li_sigmoid_attn(const void* q, void* out, int dt, const void* k_p
 template <class T> __device__ __forceinline__ float rounded_to(float v) { return to_f32(from_f32<T>(v)); }
 template <> __device__ __forceinline__ float rounded_to<float>(float v) { return v; }
 
-template <int ROWS, class TR, bool WHOLE, int THREADS>
-__global__ __launch_bounds__(THREADS) void decay_attn_kernel(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
+template <int ROWS, class TR, bool WHOLE>
+__device__ __forceinline__ void decay_attn_part(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
                                   float* __restrict__ state, const float* __restrict__ decay,
                                   const int* __restrict__ seq_slot, const int* __restrict__ seq_qstart,
-                                  const int* __restrict__ seq_qlen, float* __restrict__ out, int H, int d, int dv) {
-    extern __shared__ float lds[];
-    const int cols = dv / gridDim.z, RG = blockDim.x / cols;
+                                  const int* __restrict__ seq_qlen, float* __restrict__ out, int H, int d, int dv, float* lds,
+                                  int seq, int h, int piece, int pieces) {
+    const int cols = dv / pieces, RG = blockDim.x / cols;
     float* sq = lds;                    // [d]
     float* sk = sq + d;                 // [d]
     float* sv = sk + d;                 // [cols]
     float* red = sv + cols;             // [RG, cols]
-    const int seq = blockIdx.x, h = blockIdx.y, j0 = blockIdx.z * cols, tid = threadIdx.x;
+    const int j0 = piece * cols, tid = threadIdx.x;
     const int jc = tid % cols, j = j0 + jc, rg = tid / cols, r0 = rg * ROWS;
     const int q0 = seq_qstart ? seq_qstart[seq] : seq, n = seq_qlen ? seq_qlen[seq] : 1;
     float* S = state + (((int64_t)seq_slot[seq] * H + h) * d) * dv;
@@ -885,20 +875,37 @@ __global__ __launch_bounds__(THREADS) void decay_attn_kernel(const float* __rest
     for (int r = 0; r < ROWS; ++r) if (WHOLE || r0 + r < d) S[(int64_t)(r0 + r) * dv + j] = s[r];
 }
 
+template <int ROWS, class TR, bool WHOLE, int THREADS>
+__global__ __launch_bounds__(THREADS) void decay_attn_kernel(const float* __restrict__ proj, int stride, int q_off, int k_off, int v_off,
+                                  float* __restrict__ state, const float* __restrict__ decay,
+                                  const int* __restrict__ seq_slot, const int* __restrict__ seq_qstart,
+                                  const int* __restrict__ seq_qlen, float* __restrict__ out, int H, int d, int dv) {
+    extern __shared__ float lds[];
+    decay_attn_part<ROWS, TR, WHOLE>(proj, stride, q_off, k_off, v_off, state, decay, seq_slot, seq_qstart, seq_qlen, out, H, d, dv, lds,
+                                     blockIdx.x, blockIdx.y, blockIdx.z, gridDim.z);
+}
+
+// The rows of S of a thread, and the pieces of a head's columns, for n_seqs sequences (figures: li_decay_attn).
+static void decay_shape(int n_seqs, int H, int d, int dv, int& rows, int& split) {
+    rows = 4;
+    while (rows < 64 && ((d + rows - 1) / rows) * dv > 512) rows *= 2;
+    const int RG = (d + rows - 1) / rows;
+    // few sequences: a head's columns over several workgroups, a line of 128 bytes of a row of S each at the least, until every CU
+    // has one (16 heads of 128 x 128, 1 sequence 6.4 -> 4.1 us, 8 7.6 -> 6.6)
+    split = 1;
+    while ((int64_t)n_seqs * H * split < 256 && dv % (2 * split) == 0 && dv / (2 * split) >= 32) split *= 2;
+    if (rows == 64 && RG * (dv / split) > 512 && dv % (2 * split) == 0) split *= 2;       // (so that 64 rows have the registers, below)
+}
+
 extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off, int v_off, float* state,
                              const float* decay, const int* seq_slot, const int* seq_qstart, const int* seq_qlen,
                              float* out, int n_seqs, int H, int d, int dv, int round_dt, hipStream_t stream) {
     if (n_seqs <= 0) return LI_OK;
     if (H <= 0 || d <= 0 || dv <= 0 || dv > 256 || d > 256 || round_dt < DT_F32 || round_dt > DT_BF16) return LI_BAD_ARG;
-    int rows = 4;
-    while (rows < 64 && ((d + rows - 1) / rows) * dv > 512) rows *= 2;
+    int rows, split;
+    decay_shape(n_seqs, H, d, dv, rows, split);
     const int RG = (d + rows - 1) / rows;
     if (RG * dv > 1024) return LI_UNSUPPORTED;
-    // few sequences: a head's columns over several workgroups, a line of 128 bytes of a row of S each at the least, until every CU
-    // has one (16 heads of 128 x 128, 1 sequence 6.4 -> 4.1 us, 8 7.6 -> 6.6)
-    int split = 1;
-    while ((int64_t)n_seqs * H * split < 256 && dv % (2 * split) == 0 && dv / (2 * split) >= 32) split *= 2;
-    if (rows == 64 && RG * (dv / split) > 512 && dv % (2 * split) == 0) split *= 2;       // (so that 64 rows have the registers, below)
     const int cols = dv / split;
     // 32 and 64 rows a thread with all their loads on their way want up to 227 registers: in workgroups of up to 512 threads they have
     // them (1,024 threads have 128 each, and 18 to 95 of them were spilled).  One token a sequence, 16 heads, us with 1,024 and with 512: 128 x
@@ -921,6 +928,77 @@ extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off
 #undef GO
 #undef GO1
 #undef GO2
+    LI_CHECK_LAUNCH();
+    return LI_OK;
+}
+
+// ---------------------------------------------------------------------------
+// A decode step of the recurrence (one token a sequence) in workgroups beside those that store the other mixer's keys and values: both read the
+// input product and neither the other's result (a decode step of four layers 4,096 wide: 445 -> 432 us).
+// ---------------------------------------------------------------------------
+struct DecayStep {
+    const float* proj;
+    int stride, q_off, k_off, v_off;
+    float* state;
+    const float* decay;
+    const int* seq_slot;
+    float* out;
+    int n_seqs, H, d, dv, round_dt;
+};
+
+template <class T>
+__global__ __launch_bounds__(512) void store_beside_decay_kernel(
+    const float* __restrict__ qkv, int row_stride, const float* __restrict__ inv_freq, const float* __restrict__ cos_sin, int rot, int half_pairing,
+    float unit_eps, const int* __restrict__ pos, const int* __restrict__ tok_slot, Pages c, T* __restrict__ q_out, int H, int G, int d, int dv, int dq,
+    int dk, int dvp, int store_blocks, int parts, int split, DecayStep b) {
+    extern __shared__ float lds[];
+    const int i = blockIdx.x;
+    if (i < store_blocks) {
+        rope_norm_store_row<T>(qkv, row_stride, inv_freq, cos_sin, rot, half_pairing, unit_eps, pos, tok_slot, c, q_out, H, G, d, dv, dq, dk, dvp,
+                               i / parts, i % parts, parts);
+        return;
+    }
+    const int j = i - store_blocks, of = b.H * split;
+    decay_attn_part<32, T, true>(b.proj, b.stride, b.q_off, b.k_off, b.v_off, b.state, b.decay, b.seq_slot, nullptr, nullptr, b.out, b.H, b.d, b.dv, lds,
+                                 j / of, j % of / split, j % split, split);
+}
+
+// beside (or null): a step of the recurrence that is run along, in the same launch where its sizes allow.
+extern "C" int li_rope_norm_store(const float* qkv, int row_stride, const float* inv_freq, const float* cos_sin, int rot,
+                                  int half_pairing, float unit_eps, const int* pos, const int* tok_slot, const void* k_pages,
+                                  const void* v_pages, int64_t page_stride, const int* page_table, int max_pages,
+                                  void* q_out, int dt, int n_tokens, int H, int G, int d, int dv, int dq, int dk,
+                                  int dvp, const DecayStep* beside, hipStream_t stream) {
+    if (n_tokens <= 0) return LI_OK;
+    if (H <= 0 || G < 0 || d <= 0 || d > 256 || dq < d || dq > 256 || rot < 0 || rot > d || (rot & 1)) return LI_BAD_ARG;
+    if (G > 0 && (dv <= 0 || dk < d || dk > 256 || dk % 16 || dvp < dv || dvp % 16 || !page_table)) return LI_BAD_ARG;
+    if (row_stride < (H + G) * d + G * dv || (rot > 0 && !inv_freq)) return LI_BAD_ARG;
+    Pages c{k_pages, v_pages, page_stride, page_table, max_pages};
+    if (beside) {
+        const DecayStep& b = *beside;
+        int rows = 0, split = 1;
+        if (b.n_seqs > 0 && b.H > 0 && b.d > 0 && b.dv > 0 && b.d <= 256 && b.dv <= 256) decay_shape(b.n_seqs, b.H, b.d, b.dv, rows, split);
+        const int threads = rows ? b.d / rows * (b.dv / split) : 0;
+        if (rows == 32 && b.d % 32 == 0 && threads <= 512 && threads % 64 == 0 && n_tokens < 512 && dt != DT_F32 && b.round_dt == dt) {
+            const int parts = (H + 2 * G + threads / 64 - 1) / (threads / 64), cols = b.dv / split;
+            const size_t lds = (size_t)(2 * b.d + cols + threads) * sizeof(float);
+#define GO(T) store_beside_decay_kernel<T><<<n_tokens * parts + b.n_seqs * b.H * split, threads, lds, stream>>>(qkv, row_stride, inv_freq, cos_sin, rot, \
+        half_pairing, unit_eps, pos, tok_slot, c, (T*)q_out, H, G, d, dv, dq, dk, dvp, n_tokens * parts, parts, split, b)
+            if (dt == DT_F16) GO(f16); else GO(bf16);
+#undef GO
+            LI_CHECK_LAUNCH();
+            return LI_OK;
+        }
+        const int rc = li_decay_attn(b.proj, b.stride, b.q_off, b.k_off, b.v_off, b.state, b.decay, b.seq_slot, nullptr, nullptr, b.out, b.n_seqs, b.H, b.d,
+                                     b.dv, b.round_dt, stream);
+        if (rc) return rc;
+    }
+    // few tokens: the heads spread over the grid as well
+    dim3 grid(n_tokens, n_tokens >= 512 ? 1 : (H + 2 * G + 3) / 4), block(256);
+#define GO(T) rope_norm_store_kernel<T><<<grid, block, 0, stream>>>(qkv, row_stride, inv_freq, cos_sin, rot, half_pairing, \
+        unit_eps, pos, tok_slot, c, (T*)q_out, H, G, d, dv, dq, dk, dvp)
+    if (dt == DT_F32) GO(float); else if (dt == DT_F16) GO(f16); else if (dt == DT_BF16) GO(bf16); else return LI_BAD_ARG;
+#undef GO
     LI_CHECK_LAUNCH();
     return LI_OK;
 }

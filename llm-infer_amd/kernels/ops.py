@@ -1277,13 +1277,13 @@ def token_shift(x, mu, state, pos, tok_slot, out_dtype, single: bool = False) ->
 
 
 def rope_norm_store(qkv, inv_freq, rotary_dim, half_pairing, unit_eps, pos, tok_slot, kv, n_heads, n_kv_heads,
-                    head_dim, v_head_dim, q_dim, k_dim, v_dim, out_dtype, col0: int = 0, cos_sin=None) -> torch.Tensor:
+                    head_dim, v_head_dim, q_dim, k_dim, v_dim, out_dtype, col0: int = 0, cos_sin=None, beside=None) -> torch.Tensor:
     """q and k of a step rotated by position (half or adjacent pairing), then, with ``unit_eps`` not None,
     divided by their root mean square per head; k and v written into the pages (``kv`` = (k_pages, v_pages,
     page_stride, page_table); head sizes ``k_dim`` and ``v_dim`` in the pages, zeros beyond the true ones).
     ``col0``: the column of ``qkv`` at which q begins (a product shared with other mixers).  ``cos_sin``: the
     step's table of angles (``rope_table`` of the same frequencies and positions), read instead of computed.
-    Returns q [T, H, q_dim]."""
+    ``beside``: a ``PendingDecay`` that is run along.  Returns q [T, H, q_dim]."""
     k_pages, v_pages, page_stride, page_table = kv
     _dev(qkv, inv_freq, pos, tok_slot, k_pages, v_pages, page_table)
     _f32_rows(qkv, "rope_norm_store qkv")
@@ -1309,8 +1309,31 @@ def rope_norm_store(qkv, inv_freq, rotary_dim, half_pairing, unit_eps, pos, tok_
         c_void_p(qkv.data_ptr() + 4 * col0), qkv.shape[1], _ptr(inv_freq), _ptr(cos_sin), rotary_dim, int(half_pairing),
         c_float(-1.0 if unit_eps is None else unit_eps), _ptr(pos), _ptr(tok_slot), _ptr(k_pages), _ptr(v_pages),
         c_int64(page_stride), _ptr(page_table), page_table.shape[1], _ptr(q), DT[out_dtype], t, n_heads, n_kv_heads,
-        head_dim, v_head_dim, q_dim, k_dim, v_dim, _stream()), "rope_norm_store")
+        head_dim, v_head_dim, q_dim, k_dim, v_dim, ctypes.byref(beside.step) if beside is not None else None, _stream()), "rope_norm_store")
+    if beside is not None:
+        beside.done = True
     return q
+
+
+class _DecayStep(ctypes.Structure):
+    _fields_ = [("proj", c_void_p), ("stride", c_int), ("q_off", c_int), ("k_off", c_int), ("v_off", c_int), ("state", c_void_p), ("decay", c_void_p),
+                ("seq_slot", c_void_p), ("out", c_void_p), ("n_seqs", c_int), ("H", c_int), ("d", c_int), ("dv", c_int), ("round_dt", c_int)]
+
+
+class PendingDecay:
+    """``decay_attention`` of one token a sequence that is still to be run, by ``rope_norm_store`` beside its own work or by ``rows``."""
+
+    def __init__(self, proj, q_off, k_off, v_off, state, decay, seq_slot, n_seqs, n_heads, head_dim, v_head_dim, round_to=None):
+        self.done, self.args = False, (proj, q_off, k_off, v_off, state, decay, seq_slot, None, None, n_seqs, n_heads, head_dim, v_head_dim, round_to)
+        self.out = _decay_rows(*self.args)
+        self.step = _DecayStep(proj.data_ptr(), proj.shape[1], q_off, k_off, v_off, state.data_ptr(), decay.data_ptr(), seq_slot.data_ptr(), self.out.data_ptr(),
+                               n_seqs, n_heads, head_dim, v_head_dim, DT[round_to or torch.float32])
+
+    def rows(self) -> torch.Tensor:
+        if not self.done:
+            self.out = decay_attention(*self.args)
+            self.done = True
+        return self.out
 
 
 def sigmoid_attention(q, kv, pos, tok_slot, bias, n_heads, n_kv_heads, k_dim, v_head_dim, v_dim, scale, window=None):
@@ -1435,14 +1458,8 @@ def decay_chunks(ctx) -> dict:
     return ctx.shared(("decay_attention_chunks", DECAY_CHUNK), make)
 
 
-def decay_attention(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstart, seq_qlen, n_seqs, n_heads,
-                    head_dim, v_head_dim, round_to=None, chunked: bool = False, chunks=None) -> torch.Tensor:
-    """Linear attention with a constant decay per head over the tokens of a step, from and into the float32
-    ``state`` [slots, H, d, dv]: S <- decay S + k v^T, o = S^T q, with q, k, v = silu of the columns of ``proj``
-    (float32 [T, n]) at the given offsets.  ``seq_qstart`` / ``seq_qlen`` None: one token per sequence.
-    ``round_to`` (a 16-bit type): q, k and v take that type's values after the silu.  ``chunked`` (needs
-    ``round_to``, the per-sequence arrays and ``chunks`` = ``decay_chunks(ctx)``): 32 tokens at a time on the
-    matrix cores, for prompts; else token by token.  Returns float32 [T, H * dv]."""
+def _decay_rows(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstart, seq_qlen, n_seqs, n_heads, head_dim, v_head_dim, round_to):
+    """The rows that ``decay_attention`` fills, once what it is given has been checked."""
     _dev(proj, state, decay, seq_slot, seq_qstart, seq_qlen)
     _f32_rows(proj, "decay_attention proj")
     H, d, dv = n_heads, head_dim, v_head_dim
@@ -1456,7 +1473,19 @@ def decay_attention(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstar
         _need(seq_qlen is not None and seq_qstart.dtype == torch.int32 and seq_qlen.dtype == torch.int32 and
               seq_qstart.numel() >= n_seqs and seq_qlen.numel() >= n_seqs, "seq_qstart, seq_qlen: int32 [sequences]")
     _need(round_to in (None, torch.float32, torch.float16, torch.bfloat16), "round_to: a 16-bit type or None")
-    out = torch.empty((proj.shape[0], H * dv), dtype=torch.float32, device=proj.device)
+    return torch.empty((proj.shape[0], H * dv), dtype=torch.float32, device=proj.device)
+
+
+def decay_attention(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstart, seq_qlen, n_seqs, n_heads,
+                    head_dim, v_head_dim, round_to=None, chunked: bool = False, chunks=None) -> torch.Tensor:
+    """Linear attention with a constant decay per head over the tokens of a step, from and into the float32
+    ``state`` [slots, H, d, dv]: S <- decay S + k v^T, o = S^T q, with q, k, v = silu of the columns of ``proj``
+    (float32 [T, n]) at the given offsets.  ``seq_qstart`` / ``seq_qlen`` None: one token per sequence.
+    ``round_to`` (a 16-bit type): q, k and v take that type's values after the silu.  ``chunked`` (needs
+    ``round_to``, the per-sequence arrays and ``chunks`` = ``decay_chunks(ctx)``): 32 tokens at a time on the
+    matrix cores, for prompts; else token by token.  Returns float32 [T, H * dv]."""
+    out = _decay_rows(proj, q_off, k_off, v_off, state, decay, seq_slot, seq_qstart, seq_qlen, n_seqs, n_heads, head_dim, v_head_dim, round_to)
+    H, d, dv = n_heads, head_dim, v_head_dim
     if chunked:
         _need(round_to in (torch.float16, torch.bfloat16) and seq_qstart is not None and chunks is not None,
               "the chunked kernels multiply 16-bit numbers and need the sequences' rows and the list of chunks")

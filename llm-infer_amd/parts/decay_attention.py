@@ -54,11 +54,18 @@ class DecayLinearAttention(Part):
     def in_rows(self) -> int:
         return 2 * self.n_heads * (self.head_dim + self.v_head_dim)
 
-    takes_merge = True              # before_output accepts ``merge``
+    takes_merge = True              # before_output accepts ``merge`` and ``step``
 
-    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, merge=None):
+    def pending_step(self, ctx, view, proj, col0):
+        """A recorded decode step's recurrence, for the kernel that can run it along (``ops.PendingDecay``), else None."""
+        if not ctx.is_decode or self.dtype == torch.float32 or getattr(ctx, "seq_qstart", None) is not None:
+            return None
+        H, d = self.n_heads, self.head_dim
+        return ops.PendingDecay(proj, col0, col0 + H * d, col0 + 2 * H * d, view.state, self.decay, ctx.seq_slot, ctx.n_seqs, H, d, self.v_head_dim, self.dtype)
+
+    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, merge=None, step=None):
         """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v, g from column ``col0`` on: the input product is not run here.
-        ``merge``: an ``ops.PendingMerge`` of the mixer before, taken along."""
+        ``merge``: an ``ops.PendingMerge`` of the mixer before, taken along; ``step``: the ``pending_step`` that it has run."""
         if not owns_cache:
             raise ValueError("decay attention keeps a state of its own in every run")
         H, d, dv = self.n_heads, self.head_dim, self.v_head_dim
@@ -68,7 +75,7 @@ class DecayLinearAttention(Part):
         # 16-bit values of q, k and v; a float32 model runs token by token throughout
         sixteen = self.dtype != torch.float32
         chunked = sixteen and not ctx.is_decode
-        o = ops.decay_attention(proj, col0, col0 + H * d, col0 + 2 * H * d, view.state, self.decay, ctx.seq_slot,
+        o = step.rows() if step is not None else ops.decay_attention(proj, col0, col0 + H * d, col0 + 2 * H * d, view.state, self.decay, ctx.seq_slot,
                                 getattr(ctx, "seq_qstart", None), getattr(ctx, "seq_qlen", None), ctx.n_seqs, H, d, dv,
                                 round_to=self.dtype if sixteen else None, chunked=chunked,
                                 chunks=ops.decay_chunks(ctx) if chunked else None)

@@ -62,7 +62,7 @@ class ParallelMixers(Part):
         return [s for b in self.branches for s in cache_specs_of(b)]
 
     def addends(self, h, ctx, views, owns_cache=True):
-        out, at, merge = [], 0, None
+        out, at, merge, step = [], 0, None, None
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32) if getattr(self, "w_in", None) is not None else None
         for i, (branch, scale) in enumerate(zip(self.branches, self.scales)):
             view, at = views_for(branch, views, at)
@@ -70,10 +70,13 @@ class ParallelMixers(Part):
             if hasattr(branch, "before_output"):
                 # all but its output product, which runs with the others'; what completes its rows rides in the next branch's last kernel
                 follows = self.branches[i + 1] if i + 1 < len(self.branches) else None
-                if getattr(branch, "merges_later", False) and merge is None and getattr(follows, "takes_merge", False):
-                    rows, merge = branch.before_output(h, ctx, view, owns_cache, later=True, **shared)
-                elif merge is not None and getattr(branch, "takes_merge", False):
-                    rows, merge = branch.before_output(h, ctx, view, owns_cache, merge=merge, **shared), None
+                if getattr(branch, "merges_later", False) and step is None and getattr(follows, "takes_merge", False):
+                    # and the next branch's recurrence beside its keys and values
+                    if shared and self._col0[i + 1] is not None and owns_cache:
+                        step = follows.pending_step(ctx, views_for(follows, views, at)[0], proj, self._col0[i + 1])
+                    rows, merge = branch.before_output(h, ctx, view, owns_cache, later=True, beside=step, **shared)
+                elif (merge is not None or step is not None) and getattr(branch, "takes_merge", False):
+                    rows, merge, step = branch.before_output(h, ctx, view, owns_cache, merge=merge, step=step, **shared), None, None
                 else:
                     rows = branch.before_output(h, ctx, view, owns_cache, **shared)
                 out.append((ops.PendingProduct(rows, branch.wo), scale))

@@ -71,11 +71,12 @@ class SigmoidAttention(Part):
     def in_rows(self) -> int:
         return (self.n_heads + self.n_kv_heads) * self.head_dim + self.n_kv_heads * self.v_head_dim
 
-    merges_later = True             # before_output accepts ``later``
+    merges_later = True             # before_output accepts ``later`` and ``beside``
 
-    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, later=False):
+    def before_output(self, h, ctx, view, owns_cache=True, proj=None, col0=0, later=False, beside=None):
         """What the output product reads.  ``proj`` (float32 [T, n]) with this mixer's q, k, v from column ``col0`` on: the input product is not run here.
-        ``later``: (the rows, None or the ``ops.PendingMerge`` that completes them)."""
+        ``later``: (the rows, None or the ``ops.PendingMerge`` that completes them).  ``beside``: an ``ops.PendingDecay`` that the kernel of the
+        keys and values runs along."""
         if not owns_cache:
             raise ValueError("sigmoid attention writes its own keys and values in every run")
         H, G, d, dv = self.n_heads, self.n_kv_heads, self.head_dim, self.v_head_dim
@@ -87,7 +88,7 @@ class SigmoidAttention(Part):
         # position part shares it through the step; a float32 model computes them where they are used)
         table = self.position._table(ctx) if rot and hasattr(self.position, "_table") else None
         q = ops.rope_norm_store(proj, inv_freq, rot, half, self.unit_norm_eps, ctx.pos, ctx.tok_slot, kv, H, G, d, dv,
-                                self.k_dim, self.k_dim, self.v_dim, self.dtype, col0=col0, cos_sin=table)
+                                self.k_dim, self.k_dim, self.v_dim, self.dtype, col0=col0, cos_sin=table, beside=beside)
         if self.dtype == torch.float32:
             a = ops.sigmoid_attention(q, kv, ctx.pos, ctx.tok_slot, self.bias, H, G, self.k_dim, dv, self.v_dim,
                                       self.scale, self.window)

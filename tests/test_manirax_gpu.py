@@ -531,3 +531,34 @@ def test_partial_sums_added_beside_a_gated_norm(rows, n, splits, dv, shares):
         assert all(torch.equal(a, b) for a, b in zip(*outs))
         want = part.double().sum(2)
         assert (outs[0][1].double() - want).abs().max().item() < 2.0 ** -8 * (1 + want.abs().max().item())
+
+
+@pytest.mark.parametrize("B,H,G,d,dv,Hd,dd,ddv", [(1, 16, 4, 128, 128, 8, 128, 128), (8, 4, 2, 64, 64, 16, 128, 128), (3, 8, 8, 48, 32, 3, 96, 128),
+                                                  (17, 2, 1, 64, 64, 2, 64, 256), (2, 4, 2, 64, 64, 4, 64, 64), (1, 4, 4, 64, 64, 2, 80, 96), (1, 2, 2, 64, 64, 2, 256, 256)])
+def test_a_recurrence_step_beside_the_kernel_of_the_keys(B, H, G, d, dv, Hd, dd, ddv):
+    """Bit for bit the two launches, where the sizes allow one and where they do not."""
+    from llm_infer_amd.kernels import ops
+    g = torch.Generator().manual_seed(B + H + dd)
+    up = lambda n: (n + 15) // 16 * 16
+    n1, n2 = (H + G) * d + G * dv, 2 * Hd * dd + Hd * ddv
+    proj = torch.randn(B, n1 + n2 + 5, generator=g).to(DEV)
+    pos = torch.randint(0, 60, (B,), generator=g, dtype=torch.int32).to(DEV)
+    slot = torch.randperm(B + 2, generator=g)[:B].to(torch.int32).to(DEV)
+    table = torch.arange(B + 2, dtype=torch.int32, device=DEV).view(B + 2, 1)
+    state, decay = torch.randn(B + 2, Hd, dd, ddv, generator=g).to(DEV), torch.rand(Hd, generator=g).to(DEV)
+    freq = (0.5 ** torch.arange(d // 4, dtype=torch.float32)).to(DEV)
+    for dt in (torch.float16, torch.bfloat16, torch.float32):
+        results = []
+        for together in (False, True):
+            full = (up(dv) + 31) // 32 * 32
+            per = G * 64 * up(d), G * 64 * full
+            k, v = (torch.zeros((B + 2) * (per[0] + per[1]), dtype=dt, device=DEV) for _ in range(2))
+            s = state.clone()
+            run = ops.PendingDecay(proj, n1, n1 + Hd * dd, n1 + 2 * Hd * dd, s, decay, slot, B, Hd, dd, ddv, None if dt == torch.float32 else dt)
+            if not together:
+                run.rows()
+            q = ops.rope_norm_store(proj, freq, d // 2, True, 1e-6, pos, slot, (k, v, per[0] + per[1], table), H, G, d, dv, up(d), up(d), up(dv), dt,
+                                    beside=run if together else None)
+            results.append((q, k, v, run.rows(), s))
+        assert all(torch.equal(a, b) for a, b in zip(*results))
+        assert not torch.equal(results[0][4], state)
