@@ -1014,6 +1014,13 @@ extern "C" int li_gemv_tiled_blocks(int M, int N, int K, int nt, int kw) {
     return blocks;
 }
 
+// waves among which li_gemv_tiled shares K for this product
+extern "C" int li_gemv_tiled_waves(int M, int N, int K) {
+    int nt = 0, kw = 0, blocks = 0;
+    gemv_tiled_shape(M, N, K, nt, kw, blocks);
+    return kw;
+}
+
 template <class EB>
 static int gemv_tiled(const void* X, const void* Wt, int dt, void* C, int out_dt, int mode, int M, int N, int K, int nt, int kw,
                       const RopeStore* rs, const RowsOut* ro, const RowScale* rsc, XGroups xg, EB ex, hipStream_t stream) {

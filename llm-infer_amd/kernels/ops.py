@@ -380,30 +380,31 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
     kind = force or ("f32" if f32_ok else "fma" if not fast_ok else ("gemv_mfma" if m <= 16 else ("big" if m > 32 else "mfma")))
     if tiled:
         _need(fast_ok and kind != "fma", "a tiled weight needs 16-bit activations of its dtype")
-        # up to 16 rows (32 for a wide and shallow matrix) every wave fetches the rows of X itself; beyond that gemm_rows and
-        # the tiled GEMM are faster (us at 24 rows, gemv_tiled and gemm_rows: 2,048 x 2,048 9.4 and 6.0, 2,048 x 8,192 23.6 and
-        # 14.2, 3,072 x 2,048 9.1 and 6.3, 4,096 x 4,096 14.4 and 9.2; but 16,384 x 512 6.9 and 7.5, x 1,024 9.8 and 10.1: a
-        # workgroup's few steps of K do not pay for its stages)
+        # up to 16 rows (32 for a small matrix) every wave fetches the rows of X itself, or gemm_rows brings them in whole lines where
+        # that is faster and gives the same bits (_rows_like_tiled); beyond that gemm_rows and the tiled GEMM are faster
         # 9 to 16 rows against a wide matrix with an activation (gate and up): the tiled GEMM's tile of 64 rows of X
         # fetches the rows of X once per 112 rows of W, gemv_tiled once per 16 or 32 (measured at 16 rows and
         # 28,672 x 4,096: 44.6 against 51.7 us, at 12 rows 44.2 against 48.7, at 8 rows 44.0 against 43.5)
         wide = (force is None and 8 < m <= 16 and mode in GATED and n * k >= (1 << 26) and m * k * 2 < (1 << 32)
                 and _wreg_plan(m, n, k) == (2, 1))
-        if not wide and (kind == "gemv_mfma" or (force is None and (m <= 16 or (m <= 32 and k <= 1024 and 12288 <= n and n * k <= (1 << 25))))):
+        if not wide and (kind == "gemv_mfma" or (force is None and (m <= 16 or (m <= 32 and n * k <= (1 << 25))))):
             ro = rsc = None
             # 9 to 16 rows with the residual sum against a matrix with a long K (output products, down): gemm_rows, one tile of W
-            # a workgroup, whose rows of X come in whole lines (us, gemv_tiled and gemm_rows, at 9, 12 and 16 rows: 4,096 x
-            # 14,336 20.5 and 21.4, 22.2 and 20.8, 25.4 and 22.0; 2,048 x 8,192 10.6 and 10.3, 11.8 and 11.0, 13.1 and 11.6; 2,048 x
-            # 4,096 6.6 and 6.5, 7.0 and 6.7, 7.7 and 7.1; but 2,048 x 2,048 4.6 and 4.8, 4.8 and 4.8, 5.2 and 5.2, 4,096 x 4,096 7.6 and
-            # 8.4, 7.9 and 8.1, 8.4 and 8.8)
-            tall = (force is None and 8 < m <= 16 and mode == EPI_ADD and lazy is None and experts is None and n % 16 == 0
-                    and ((k >= 8192 and m >= 12) or (k >= 4096 and n <= 2048)) and x.stride(0) % 8 == 0 and x.stride(1) == 1)
+            # a workgroup, whose rows of X come in whole lines: with four waves from 2,048 rows of W on, with as many as gemv_tiled has
+            # below, where four (K in half as many parts) would add 1.3 to 1.4 times its error against 64 bits.  (us, gemv_tiled, four waves
+            # and eight, at 9, 12 and 16 rows: 4,096 x 14,336 22.8, 21.7, 22.5; 24.6, 22.2, 23.4; 28.5, 22.3, 23.2; 2,048 x 8,192 12.0, 11.1,
+            # 11.8; 12.7, 11.0, 11.7; 13.7, 11.9, 12.6; 1,024 x 8,192 10.5, 9.4, 10.3; 11.7, 10.0, 11.0; 13.2, 10.9, 11.8; but at 12 and 16
+            # rows 2,048 x 4,096 8.1, 6.9, 8.1; 8.1, 7.1, 8.2, 512 x 4,096 7.0, 6.1, 7.1; 7.7, 6.5, 7.6)
+            like = None
+            if force is None and m > 8 and lazy is None and experts is None and (m > 16 or (mode == EPI_ADD and k >= 8192 and n % 16 == 0)):
+                four = m <= 16 and (n == 2048 or (n > 2048 and m >= 12))
+                like = (1, 4) if four else _rows_like_tiled(m, n, k) if m > 16 or n < 2048 else None
             nxt = getattr(out, "_li_next_norm", None) if mode == EPI_ADD else None
             if (nxt is not None and m <= 16 and n % 32 == 0 and out.data_ptr() % 16 == 0 and nxt.dtype == torch.float32
                     and nxt.shape == (n,) and nxt.is_cuda and nxt.data_ptr() % 16 == 0):
                 # the rows of `out` are about to be complete rows of a residual stream that this norm reads
                 # next: leave x * weight in 16 bits and the sums of squares for the product behind the norm
-                blocks = n // 16 if tall else lib.li_gemv_tiled_blocks(m, n, k, 0, 0)
+                blocks = n // 16 if like else lib.li_gemv_tiled_blocks(m, n, k, 0, 0)
                 ss = torch.empty((blocks, 16), dtype=torch.float32, device=x.device)
                 xw = torch.empty((m, n), dtype=x.dtype, device=x.device)
                 scale = 0.125 if x.dtype == torch.float16 else 1.0        # x * w stays inside float16's range
@@ -420,8 +421,8 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
                 _check(lib.li_gemv_tiled_experts(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, rs,
                                                  ctypes.byref(ro) if ro is not None else None, _ptr(weights), weights.shape[1],
                                                  number, ff, over, _stream()), "gemv_tiled_experts")
-            elif tall:
-                _check(lib.li_gemm_rows(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, x.stride(0), 1, 4,
+            elif like:
+                _check(lib.li_gemm_rows(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, x.stride(0), *like,
                                         rs, ctypes.byref(ro) if ro is not None else None, _stream()), "gemm_rows")
             else:
                 _check(lib.li_gemv_tiled(_ptr(x), _ptr(wd), DT[x.dtype], _ptr(out), out_dt, mode, m, n, k, 0, 0, rs,
@@ -655,6 +656,26 @@ def _wreg_plan(m: int, n: int, k: int) -> tuple[int, int]:
     read; the narrower tiles are for products whose tiles would leave much of the last round empty."""
     options = [(t, s) for t in (0, 1, 2) for s in (1, 2, 3, 4, 6, 8, 12, 16) if s == 1 or k // s >= 1024]
     return min(options, key=lambda o: (_wreg_cost(o[0], o[1], m, n, k), o[1], o[0]))
+
+
+@functools.lru_cache(maxsize=4096)
+def _rows_like_tiled(m: int, n: int, k: int) -> tuple[int, int] | None:
+    """Tiles of W a workgroup and waves with which gemm_rows takes a product of 9 to 32 rows in gemv_tiled's place: the waves that
+    gemv_tiled would have, each with the same share of K, so that the result is the same bit for bit; None where the shares are
+    not whole steps of 64 of K, or gemv_tiled is as fast.  (us at 17, 24 and 32 rows, gemv_tiled and this.  Eight waves: 512 x 512 4.4 and
+    3.8, 4.6 and 3.8, 4.7 and 3.9; 2,048 x 2,048 8.2 and 6.2, 9.0 and 6.6, 9.9 and 7.0; 4,096 x 4,096 12.7 and 9.2, 14.4 and 10.0, 16.2 and
+    10.9; 2,048 x 8,192 19.9 and 13.3, 23.0 and 14.6, 26.6 and 16.0; two tiles, 6,144 x 2,048 9.8 and 8.9, 10.4 and 9.0, 10.7 and 9.5;
+    8,192 x 1,024 7.2 and 6.9, 7.4 and 7.1, 7.5 and 7.4; but x 512 5.6 and 6.4, 5.8 and 6.8, 5.9 and 7.1.  Four waves: 10,240 x 512 6.5
+    and 6.1, 6.6 and 6.4, 7.0 and 6.9; 14,336 x 1,024 9.6 and 9.3, 10.2 and 9.7, 10.6 and 10.1; 16,384 x 2,048 15.5 and 15.3, 16.8 and 16.0,
+    18.4 and 16.2; but x 512 7.0 and 6.8, 6.9 and 7.2, 7.2 and 7.9, x 1,024 9.5 and 10.0, 10.4 and 10.5, 10.6 and 10.8)"""
+    waves = core().li_gemv_tiled_waves(m, n, k)
+    if k % 64 or -(-k // (32 * waves)) % 2:
+        return None
+    if n <= 4096:
+        return 1, waves
+    if k < (1024 if waves == 8 else 512) or (n > 14336 and k <= 1024):
+        return None
+    return 2, waves
 
 
 def _rows_cost(nt: int, m: int, n: int, k: int) -> float:

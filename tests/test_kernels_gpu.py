@@ -360,6 +360,37 @@ def test_more_rows_than_one_block_and_the_rules_beside_them(ops, M, N, K, dt):
 
 
 @pytest.mark.parametrize("dt", F16S)
+@pytest.mark.parametrize("M,N,K,rows", [(17, 512, 512, (1, 8)), (24, 4096, 4096, (1, 8)), (32, 2048, 8192, (1, 8)), (19, 320, 1408, (1, 8)),
+                                        (24, 3072, 2048, (1, 8)), (32, 48, 320, (1, 8)), (17, 6144, 2048, (2, 8)), (24, 4112, 1024, (2, 8)),
+                                        (32, 8192, 4096, (2, 8)), (17, 10240, 512, (2, 4)), (24, 14336, 1024, (2, 4)), (18, 14352, 1280, (2, 4)),
+                                        (32, 16384, 2048, (2, 4)), (9, 1024, 8192, (1, 8)), (16, 2032, 8192, (1, 8)), (12, 256, 14336, (1, 8)),
+                                        (31, 100, 864, None), (24, 1024, 1056, None), (20, 8192, 512, None), (32, 14352, 1024, None),
+                                        (20, 10240, 288, None), (12, 1024, 8224, None), (16, 2048, 4096, "short"), (12, 512, 8128, "short")])
+def test_a_products_sums_do_not_depend_on_the_kernel_of_few_rows(ops, M, N, K, rows, dt):
+    """Products of 9 to 32 rows that gemm_rows takes in gemv_tiled's place (tiles, waves; None: it does not): K in the same parts, added up
+    in the same order, so the same bits with every epilogue that either side of the rules meets (fewer parts would be a larger error
+    against 64 bits)."""
+    assert rows == "short" or ops._rows_like_tiled(M, N, K) == rows
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(dt).to(DEV)
+    wt = ops.tile_weight((torch.randn(N, K, generator=g) / math.sqrt(K)).to(dt).to(DEV))
+    res, nw = torch.randn(M, N, generator=g).to(DEV), torch.randn(N, generator=g).to(DEV)
+    assert torch.equal(ops.linear(x, wt, out_dtype=torch.float32), ops.linear(x, wt, out_dtype=torch.float32, force="gemv_mfma"))
+    assert torch.equal(ops.linear(x, wt, 2), ops.linear(x, wt, 2, force="gemv_mfma"))
+    bias = ops.glu_params(nw, act="tanh")
+    assert torch.equal(ops.linear(x, wt, ops.EPI_BIAS, params=bias), ops.linear(x, wt, ops.EPI_BIAS, params=bias, force="gemv_mfma"))
+    outs = [res.clone(), res.clone()]
+    for out, kind in zip(outs, (None, "gemv_mfma")):
+        ops.expect_norm(out, nw, 1e-5)
+        ops.linear(x, wt, 1, out=out, force=kind)
+    assert torch.equal(*outs)
+    recs = [getattr(out, "_li_rows", None) for out in outs]
+    assert (recs[0] is None) == (recs[1] is None)
+    if recs[0] is not None:                              # (what the product left for the norm behind it)
+        assert torch.equal(recs[0][0], recs[1][0]) and torch.equal(recs[0][1], recs[1][1])
+
+
+@pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(8, 32), (16, 64), (24, 96), (100, 544), (2048, 1056), (2050, 160), (4096, 8192)])
 def test_half_tiles(ops, M, N, K, dt):
