@@ -679,16 +679,19 @@ def _rows_like_tiled(m: int, n: int, k: int) -> tuple[int, int] | None:
 
 
 def _rows_cost(nt: int, m: int, n: int, k: int) -> float:
-    """Estimated microseconds of one gemm_rows launch, fitted to measurements on MI355X (17 to 128 rows against 61 matrices of
-    320 to 28,672 rows and 512 to 14,336 of K; the kernel it names is 1.1% slower in the mean than the fastest): W streamed once (at the
-    rate of 256 workgroups, slower with fewer), plus the rows of X, which every workgroup fetches from L2 in blocks of 16, plus a
-    workgroup's start and end, plus a launch."""
-    blocks16 = 2 if m <= 32 else (3 if m <= 48 else (4 if m <= 64 else (6 if m <= 96 else 8)))
+    """Estimated microseconds of one gemm_rows launch, fitted to measurements on MI355X (24 to 128 rows against
+    the matrices of the 8B shape) with one workgroup a CU at a time: W streamed once (at the rate of 256 workgroups, slower
+    with fewer), plus the rows of X, which every workgroup fetches from L2 in blocks of 16, plus a launch.
+    It says in how many parts K is summed, too (four here, the splits of gemm_wreg there).  Fitted to gemm_rows with two stages a
+    wave, which runs two workgroups a CU, it would give wide and shallow products to gemm_wreg in one part (us and error
+    against 64 bits, gemm_rows and gemm_wreg: 48 rows x 10,240 x 1,536 14.7, 1.33e-7 and 15.7, 2.5e-7; x 28,672 x 512 14.0, 0.9e-7 and
+    10.9, 1.5e-7) and 48 rows x 4,096 x 8,192 (gemm_wreg, eight parts 21.5, 2.1e-7; gemm_rows 22.0, 2.9e-7) the other way."""
+    blocks16 = 2 if m <= 32 else (4 if m <= 64 else (6 if m <= 96 else 8))
     groups = -(-(-(-n // 16)) // nt)
     w_mb, x_mb = n * k * 2 / 1e6, groups * blocks16 * 16 * k * 2 / 1e6
     # a last round of 256 workgroups that is not full runs as long as a full one
     uneven = -(-groups // 256) * 256 / groups
-    return 2.5 + (w_mb / 7.0 + x_mb / 22.0 + 1.2 * groups / 256) * uneven
+    return 2.5 + (w_mb / 6.2 + x_mb / 22.0) * uneven
 
 
 @functools.lru_cache(maxsize=4096)

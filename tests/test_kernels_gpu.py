@@ -390,6 +390,17 @@ def test_a_products_sums_do_not_depend_on_the_kernel_of_few_rows(ops, M, N, K, r
         assert torch.equal(recs[0][0], recs[1][0]) and torch.equal(recs[0][1], recs[1][1])
 
 
+@pytest.mark.parametrize("M,N,K,kind", [(33, 10240, 1536, "rows:2"), (64, 12288, 1536, "rows:2"), (48, 28672, 512, "rows:2"), (128, 32000, 512, "rows:2"),
+                                        (48, 4096, 8192, "wreg"), (32, 4096, 11008, "wreg"), (24, 16384, 5120, "wreg"), (40, 4096, 4096, "rows:1")])
+def test_the_parts_in_which_some_dozen_rows_sum_their_products(ops, M, N, K, kind):
+    """On either side of the estimate between gemm_rows (K in four parts) and gemm_wreg (in its splits): the kernel that the sums
+    belong to, bit for bit."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g).to(torch.bfloat16).to(DEV)
+    wt = ops.tile_weight((torch.randn(N, K, generator=g) / math.sqrt(K)).to(torch.bfloat16).to(DEV))
+    assert torch.equal(ops.linear(x, wt, out_dtype=torch.float32), ops.linear(x, wt, out_dtype=torch.float32, force=kind))
+
+
 @pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M", [1, 2, 7, 8])
 @pytest.mark.parametrize("N,K", [(8, 32), (16, 64), (24, 96), (100, 544), (2048, 1056), (2050, 160), (4096, 8192)])
