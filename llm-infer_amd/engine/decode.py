@@ -91,6 +91,14 @@ def batch_bucket(n: int, limit: int) -> int:
     return max(n, min(b, limit))
 
 
+class _Step:
+    """A step that has been enqueued: its sequences, its number, and the stream it runs on."""
+    __slots__ = ("slots", "number", "stream")
+
+    def __init__(self, slots, number, stream):
+        self.slots, self.number, self.stream = list(slots), number, stream
+
+
 class GraphDecodeRunner:
     """Replays a recorded step while the set of live sequences stays the same; when it
     changes, the slots and tokens are uploaded anew and the graph of the new size is used.
@@ -98,7 +106,9 @@ class GraphDecodeRunner:
     sequences rounded up to a ``batch_bucket`` (idle rows run on the cache's scratch slot and their tokens
     are dropped); the temperature is read from the device, so it is no part of the key.  The first step of an
     engine is run eagerly (whatever is built or loaded at first use must not happen while a graph is being
-    recorded) and recorded when its key comes again; every later key is recorded when it is first seen.  An
+    recorded) and recorded when its key comes again; every later key is recorded when it is first seen.  A step
+    runs on the stream that is current when it is enqueued, behind the step before it, and its tokens are waited for there, whatever
+    stream is current by then.  An
     engine keeps at most MAX_RECORDED_STEPS recorded steps and counts what it did in ``engine.decode_counts``
     (steps run eagerly, steps recorded, steps replayed)."""
 
@@ -117,6 +127,7 @@ class GraphDecodeRunner:
             self.bufs["steps"] = torch.zeros((n,), dtype=torch.int32, device=dev)
             self.bufs["host"] = [Tensor.pinned((ops.TOKEN_RING, n), torch.int64), Tensor.pinned((n,), torch.int32)]
             self.bufs["launched"] = 0              # steps enqueued so far: what the counters will stand at
+            self.bufs["stream"] = None             # where the newest of them was
             engine._graph_bufs = self.bufs
         self.current = None            # the rows' slots now in the buffers
         self._ahead = None             # a step enqueued before its predecessor's tokens were read
@@ -138,9 +149,12 @@ class GraphDecodeRunner:
         self.sampler.sample(logits, b["slots"][:n], eng.cache, out=b["tokens"], temperature_dev=b["temperature"])
 
     def _launch(self, slots, tokens):
-        """Enqueues one step for ``slots``; returns them and the step's number.
-        ``tokens`` None: the tokens the step before left on the device are fed."""
+        """Enqueues one step for ``slots``.  ``tokens`` None: the tokens the step before left on the device are fed."""
         b = self.bufs
+        stream = torch.cuda.current_stream(self.engine.device)
+        if b["stream"] is not None and b["stream"] != stream:
+            stream.wait_stream(b["stream"])      # the step before works in the same buffers, and on the same sequences
+        b["stream"] = stream
         try:
             self._enqueue(slots, tokens)
         except BaseException:
@@ -149,7 +163,7 @@ class GraphDecodeRunner:
             b["steps"].fill_((b["launched"] + (1 << 31)) % (1 << 32) - (1 << 31))
             raise
         b["launched"] += 1
-        return list(slots), b["launched"]
+        return _Step(slots, b["launched"], stream)
 
     def _enqueue(self, slots, tokens):
         eng, cache, b = self.engine, self.engine.cache, self.bufs
@@ -197,14 +211,14 @@ class GraphDecodeRunner:
         """The tokens of ``step``, the newest one or the one before it.  Where a step has been enqueued behind it, that step's first kernel
         sends them and the host polls for them: no copy and no event between two recorded steps (a step
         of four layers 2,048 wide, batch 1, 263.9 -> 256.2 us, batch 8 373.7 -> 368.5; 4,096 wide 480.1 -> 474.8)."""
-        slots, number = step
-        b = self.bufs
-        if self._ahead is not None and self._ahead[1] == number + 1:
-            return ops.wait_tokens(b["host"][0], len(slots), number + 1)
+        b, n = self.bufs, len(step.slots)
+        if self._ahead is not None and self._ahead.number == step.number + 1:
+            return ops.wait_tokens(b["host"][0], n, self._ahead.number, self._ahead.stream)
         host = b["host"][1]
-        host[:len(slots)].copy_(b["tokens"][:len(slots)], non_blocking=True)
-        torch.cuda.current_stream().synchronize()
-        return host[:len(slots)].tolist()
+        with torch.cuda.stream(step.stream):
+            host[:n].copy_(b["tokens"][:n], non_blocking=True)
+        step.stream.synchronize()
+        return host[:n].tolist()
 
     def run(self, slots, tokens, may_follow: bool = False):
         """One token for each of ``slots``.  ``may_follow``: the caller will ask for the same
@@ -216,12 +230,12 @@ class GraphDecodeRunner:
         slots = list(slots)
         if self._ahead is not None:
             step, self._ahead = self._ahead, None
-            if list(tokens) != [self._fed[s] for s in slots] or any(s not in step[0] for s in slots):
+            if list(tokens) != [self._fed[s] for s in slots] or any(s not in step.slots for s in slots):
                 raise RuntimeError("a step was enqueued ahead for other sequences or tokens than those asked for now")
-            if slots == step[0] and may_follow:
+            if slots == step.slots and may_follow:
                 self._ahead = self._launch(slots, None)
             every = self._collect(step)
-            out = [every[step[0].index(s)] for s in slots]
+            out = [every[step.slots.index(s)] for s in slots]
         else:
             step = self._launch(slots, tokens)
             if may_follow:

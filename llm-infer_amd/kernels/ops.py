@@ -827,14 +827,15 @@ def decode_prepare(seq_slot, lens, pos, ctx, n, scratch_slot: int = -1, inv_freq
     return table
 
 
-def wait_tokens(ring, n: int, step: int) -> list[int]:
+def wait_tokens(ring, n: int, step: int, stream=None) -> list[int]:
     """The first ``n`` rows' tokens that the decode_prepare of step number ``step`` sent to ``ring`` (the newest step or
-    one of the TOKEN_RING - 1 before it).  Polls (as a wait for an event does); if the stream ends without them, that is an error."""
+    one of the TOKEN_RING - 1 before it).  Polls (as a wait for an event does); if ``stream``, which that step was enqueued on (None: the
+    current one), ends without them, that is an error."""
     _need(0 < n <= ring.shape[1], "wait_tokens: the rows of the ring")
     out = (ctypes.c_int * n)()
     wait = lambda micros: core().li_wait_tokens(c_void_p(ring.data_ptr()), ring.shape[1], n, ctypes.c_uint(step & 0xFFFFFFFF), out, c_int64(micros))
     while wait(1_000_000):
-        if torch.cuda.current_stream().query() and wait(0):          # (a failed launch raises here)
+        if (stream or torch.cuda.current_stream()).query() and wait(0):          # (a failed launch raises here)
             raise KernelError(f"wait_tokens: the device is done and step {step}'s tokens have not come")
     return list(out)
 

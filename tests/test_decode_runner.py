@@ -1,0 +1,156 @@
+"""The recorded decode runner's waits, on the CPU: streams are queues of what was enqueued on them and run only when
+something waits for them, so a wait that is missing shows as the numbers of before."""
+import threading
+import time
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from llm_infer_amd.engine import decode
+from llm_infer_amd.kernels import ops
+
+
+class Stream:
+    def __init__(self):
+        self.queue = []
+
+    def run(self):
+        while self.queue:
+            self.queue.pop(0)()
+
+    synchronize = run
+
+    def wait_stream(self, other):
+        self.queue.append(other.run)
+
+    def query(self):
+        return not self.queue
+
+
+class Buffer:
+    """Numbers on the device: what is copied into them or out of them is enqueued on the current stream."""
+
+    def __init__(self, device, values, n=None):
+        self.device, self.values, self.n = device, values, n
+
+    def __getitem__(self, part):
+        return Buffer(self.device, self.values, part.stop)
+
+    def copy_(self, src, non_blocking=False):
+        if isinstance(src, Buffer):
+            self.device.current.queue.append(lambda: self.values.__setitem__(slice(0, self.n), src.values[:src.n]))
+        else:
+            numbers = src.tolist()
+            self.device.current.queue.append(lambda: self.values.__setitem__(slice(0, self.n), numbers))
+
+    def fill_(self, v):
+        self.device.current.queue.append(lambda: self.values.__setitem__(slice(0, len(self.values)), [v] * len(self.values)))
+
+    def tolist(self):
+        return list(self.values[:self.n])
+
+
+class Graphs(dict):
+    """An engine's recorded steps: none is ever kept, so every step runs eagerly."""
+
+    def __setitem__(self, key, entry):
+        pass
+
+
+class Device:
+    """Two streams and an engine whose step adds the slot's number to each row's token."""
+
+    def __init__(self, monkeypatch, n_slots=4):
+        self.a, self.b = Stream(), Stream()
+        self.current, self.ring, self.fails = self.a, {}, 0
+        monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: self.current)
+        monkeypatch.setattr(torch.cuda, "stream", self.on)
+        monkeypatch.setattr(decode.Tensor, "pinned", staticmethod(lambda shape, dtype: torch.zeros(shape, dtype=dtype)))
+        monkeypatch.setattr(ops, "wait_tokens", self.wait_tokens)
+        cache = SimpleNamespace(n_slots=n_slots, scratch_slot=n_slots, lens=[5] * n_slots, lens_dev=None, grow=self.grow,
+                                trim_windows=lambda slots: None)
+        self.engine = SimpleNamespace(cache=cache, device="cpu", model=SimpleNamespace(positions={}), _graphs=Graphs(), _graph_bufs=None,
+                                      decode_counts={"eager": 0, "recorded": 0, "replayed": 0})
+
+    def grow(self, slots, lens, sync_lens):
+        for s, n in zip(slots, lens):
+            self.engine.cache.lens[s] = n
+
+    def on(self, stream):
+        from contextlib import contextmanager
+
+        @contextmanager
+        def inside():
+            before, self.current = self.current, stream
+            yield
+            self.current = before
+        return inside()
+
+    def runner(self):
+        runner = decode.GraphDecodeRunner(self.engine, SimpleNamespace(temperature=0.0))
+        b = runner.bufs
+        if not isinstance(b["tokens"], Buffer):
+            for name in ("tokens", "slots", "steps"):
+                b[name] = Buffer(self, [0] * self.engine.cache.n_slots)
+            b["host"][1] = Buffer(self, [0] * self.engine.cache.n_slots)
+
+        def body(n, bucket, pages):
+            def prepare():
+                number = b["steps"].values[0] + 1
+                b["steps"].values[:] = [number] * len(b["steps"].values)
+                self.ring[number] = list(b["tokens"].values)
+
+            def rest():
+                b["tokens"].values[:n] = [t + s + 1 for t, s in zip(b["tokens"].values[:n], b["slots"].values[:n])]
+
+            if self.fails:
+                self.fails -= 1
+                raise RuntimeError("this step fails")
+            self.current.queue += [prepare, rest]
+        runner._body = body
+        return runner
+
+    def wait_tokens(self, ring, n, step, stream=None):
+        """The device goes on by itself while the host polls; a stream that is done without the step's tokens is an error."""
+        queue = (stream or self.current).queue
+        while step not in self.ring:
+            if not queue:
+                raise ops.KernelError("the device is done")
+            queue.pop(0)()
+        return self.ring[step][:n]
+
+
+def test_a_step_is_waited_for_on_its_own_stream(monkeypatch):
+    """Steps launched ahead under one stream, collected or dropped under another."""
+    dev = Device(monkeypatch)
+    runner = dev.runner()
+    assert runner.run([0, 2], [10, 20], may_follow=True) == [11, 23]
+    dev.current = dev.b
+    assert runner.run([0, 2], [11, 23]) == [12, 26]                      # the one ahead, from its own stream
+    assert runner.run([0, 2], [12, 26], may_follow=True) == [13, 29]
+    dev.current = dev.a
+    assert runner.run([0, 2], [13, 29], may_follow=True) == [14, 32]     # the next one behind it, on this stream
+    dev.current = dev.b
+    assert not dev.a.query()
+    runner.drain()
+    assert dev.a.query()                                                 # nothing is left that works on the slots
+
+
+def test_tokens_that_are_waited_for_come_from_the_steps_own_stream(monkeypatch):
+    """Another stream that is idle says nothing about the step's: no error while that one still runs."""
+    idle, busy = SimpleNamespace(query=lambda: True), SimpleNamespace(query=lambda: False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: idle)
+    ring = torch.zeros((ops.TOKEN_RING, 2), dtype=torch.int64)
+
+    def later():
+        time.sleep(1.3)
+        ring[3, 0], ring[3, 1] = 7 << 32 | 40, 7 << 32 | 41
+    writer = threading.Thread(target=later)
+    writer.start()
+    try:
+        assert ops.wait_tokens(ring, 2, 7, busy) == [40, 41]
+    finally:
+        writer.join()
+    with pytest.raises(ops.KernelError):
+        ops.wait_tokens(ring, 2, 8)

@@ -211,3 +211,38 @@ def test_random_weights_without_a_folder_are_the_folders(dtype, tmp_path):
         logits.append(eng.step(slots, tokens, want).float().cpu())
     assert torch.equal(logits[0], logits[1])
     assert not torch.equal(logits[0], logits[2])
+
+
+@pytest.mark.parametrize("pattern", ["AAAAAB", "ABABAB", "AABBAA", "ABBBBA"])
+def test_decoding_goes_on_where_the_stream_changes(pattern):
+    """A decode runner that is called under other streams from step to step, each of them behind work of its own: the tokens of one stream
+    alone; a step that is dropped is done when ``drain`` returns."""
+    import llm_infer_amd
+    from llm_infer_amd.sampling import Sampler
+    eng = llm_infer_amd.random_model(llm_infer_amd.config_from_dict(ALL["A"]), seed=3, dtype="bfloat16", max_tokens=1024)
+    g = torch.Generator().manual_seed(2)
+    prompts = [torch.randint(0, eng.vocab_size, (n,), generator=g).tolist() for n in (20, 7, 33)]
+    streams = {"A": torch.cuda.Stream(), "B": torch.cuda.Stream()}
+    big, out = torch.randn(4096, 4096, device="cuda", dtype=torch.bfloat16), {k: torch.empty(4096, 4096, device="cuda", dtype=torch.bfloat16) for k in streams}
+
+    def tokens(names, busy, drop=False):
+        slots = [eng.alloc_slot() for _ in prompts]
+        toks = [eng.step(slots, prompts).argmax(-1).tolist()]
+        runner = eng.decode_runner(Sampler(0.0))
+        torch.cuda.synchronize()
+        for i, name in enumerate(names):
+            with torch.cuda.stream(streams[name]):
+                for _ in range(4 if busy else 0):
+                    torch.mm(big, big, out=out[name])
+                toks.append(runner.run(slots, toks[-1], may_follow=drop or i + 1 < len(names)))
+        if drop:
+            runner.drain()                               # (under a stream that is idle)
+            assert streams[names[-1]].query()
+        torch.cuda.synchronize()
+        for s in slots:
+            eng.free_slot(s)
+        return toks
+    want = tokens("AAAAAA", False)
+    assert tokens("AAAAAA", False) == want
+    for drop in (False, True):
+        assert tokens(pattern, True, drop) == want
