@@ -92,11 +92,11 @@ def batch_bucket(n: int, limit: int) -> int:
 
 
 class _Step:
-    """A step that has been enqueued: its sequences, its number, and the stream it runs on."""
-    __slots__ = ("slots", "number", "stream")
+    """A step that has been enqueued: its sequences, its number, the stream it runs on, and its tokens once the host has them."""
+    __slots__ = ("slots", "number", "stream", "tokens")
 
     def __init__(self, slots, number, stream):
-        self.slots, self.number, self.stream = list(slots), number, stream
+        self.slots, self.number, self.stream, self.tokens = list(slots), number, stream, None
 
 
 class GraphDecodeRunner:
@@ -128,8 +128,9 @@ class GraphDecodeRunner:
             self.bufs["host"] = [Tensor.pinned((ops.TOKEN_RING, n), torch.int64), Tensor.pinned((n,), torch.int32)]
             self.bufs["launched"] = 0              # steps enqueued so far: what the counters will stand at
             self.bufs["stream"] = None             # where the newest of them was
+            # what the buffers hold, which all runners of the engine share: the rows' slots, and the newest step, whose tokens they are
+            self.bufs["held"] = self.bufs["last"] = None
             engine._graph_bufs = self.bufs
-        self.current = None            # the rows' slots now in the buffers
         self._ahead = None             # a step enqueued before its predecessor's tokens were read
         self._fed = None               # slot -> the token that step was fed on the device
         # one table of rotation angles for the whole model: the bookkeeping kernel fills it
@@ -163,7 +164,8 @@ class GraphDecodeRunner:
             b["steps"].fill_((b["launched"] + (1 << 31)) % (1 << 32) - (1 << 31))
             raise
         b["launched"] += 1
-        return _Step(slots, b["launched"], stream)
+        b["last"] = _Step(slots, b["launched"], stream)
+        return b["last"]
 
     def _enqueue(self, slots, tokens):
         eng, cache, b = self.engine, self.engine.cache, self.bufs
@@ -172,12 +174,16 @@ class GraphDecodeRunner:
         new_lens = [cache.lens[s] + 1 for s in slots]
         cache.grow(slots, new_lens, sync_lens=False)
         padded = list(slots) + [cache.scratch_slot] * (rows - n)
-        if self.current != padded:
-            if tokens is None:
+        last, held = b["last"], b["held"]
+        b["last"] = b["held"] = None
+        if tokens is None:
+            if held != padded:
                 raise RuntimeError("a new set of sequences needs its tokens")
+        elif held != padded or last is None or last.tokens != list(tokens):
+            if last is not None:
+                self._tokens_of(last)            # (a step that another runner has enqueued ahead: its tokens lie where these go)
             b["slots"][:rows].copy_(torch.tensor(padded, dtype=torch.int32))
             b["tokens"][:rows].copy_(torch.tensor(list(tokens) + [0] * (rows - n), dtype=torch.int32))
-            self.current = padded
         bucket, pages = split_bucket(max(new_lens)), steady_pages(new_lens)
         hot = self.sampler.temperature > 0.0
         if hot and b.get("temperature_value") != self.sampler.temperature:
@@ -201,6 +207,7 @@ class GraphDecodeRunner:
                 counts["replayed"] += 1
             entry.replay()
         graphs[key] = entry
+        b["held"] = padded
         while len(graphs) > MAX_RECORDED_STEPS:
             old = next(iter(graphs))
             if graphs[old] != "seen":
@@ -211,14 +218,19 @@ class GraphDecodeRunner:
         """The tokens of ``step``, the newest one or the one before it.  Where a step has been enqueued behind it, that step's first kernel
         sends them and the host polls for them: no copy and no event between two recorded steps (a step
         of four layers 2,048 wide, batch 1, 263.9 -> 256.2 us, batch 8 373.7 -> 368.5; 4,096 wide 480.1 -> 474.8)."""
-        b, n = self.bufs, len(step.slots)
-        if self._ahead is not None and self._ahead.number == step.number + 1:
-            return ops.wait_tokens(b["host"][0], n, self._ahead.number, self._ahead.stream)
-        host = b["host"][1]
-        with torch.cuda.stream(step.stream):
-            host[:n].copy_(b["tokens"][:n], non_blocking=True)
-        step.stream.synchronize()
-        return host[:n].tolist()
+        if step.tokens is None and self._ahead is not None and self._ahead.number == step.number + 1:
+            step.tokens = ops.wait_tokens(self.bufs["host"][0], len(step.slots), self._ahead.number, self._ahead.stream)
+        return self._tokens_of(step)
+
+    def _tokens_of(self, step):
+        """The tokens of the newest step, which lie where it left them, or of one whose tokens the host has."""
+        if step.tokens is None:
+            host, n = self.bufs["host"][1], len(step.slots)
+            with torch.cuda.stream(step.stream):
+                host[:n].copy_(self.bufs["tokens"][:n], non_blocking=True)
+            step.stream.synchronize()
+            step.tokens = host[:n].tolist()
+        return step.tokens
 
     def run(self, slots, tokens, may_follow: bool = False):
         """One token for each of ``slots``.  ``may_follow``: the caller will ask for the same
@@ -232,7 +244,7 @@ class GraphDecodeRunner:
             step, self._ahead = self._ahead, None
             if list(tokens) != [self._fed[s] for s in slots] or any(s not in step.slots for s in slots):
                 raise RuntimeError("a step was enqueued ahead for other sequences or tokens than those asked for now")
-            if slots == step.slots and may_follow:
+            if slots == step.slots and may_follow and self.bufs["last"] is step:      # (no other runner's step since)
                 self._ahead = self._launch(slots, None)
             every = self._collect(step)
             out = [every[step.slots.index(s)] for s in slots]
@@ -240,7 +252,7 @@ class GraphDecodeRunner:
             step = self._launch(slots, tokens)
             if may_follow:
                 self._ahead = self._launch(slots, None)
-            out = self._collect(step)
+            out = list(self._collect(step))
         self._fed = dict(zip(slots, out)) if self._ahead is not None else None
         self.engine.cache.trim_windows(slots)
         return out

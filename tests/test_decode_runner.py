@@ -137,6 +137,27 @@ def test_a_step_is_waited_for_on_its_own_stream(monkeypatch):
     assert dev.a.query()                                                 # nothing is left that works on the slots
 
 
+def test_runners_of_one_engine_keep_their_own_tokens(monkeypatch):
+    """Another runner's step, for other sequences, more of them or the same, between a step that was enqueued ahead and the call that
+    asks for its tokens; and tokens that are not those of the step before."""
+    dev = Device(monkeypatch)
+    one, two = dev.runner(), dev.runner()
+    assert one.run([0, 2], [10, 20], may_follow=True) == [11, 23]
+    assert two.run([1], [50], may_follow=True) == [52]
+    assert one.run([0, 2], [11, 23]) == [12, 26]                         # the one that was ahead of the other runner's
+    assert one.run([0, 2], [12, 26], may_follow=True) == [13, 29]
+    assert two.run([1], [52], may_follow=True) == [54]                   # likewise: and none is enqueued behind it
+    assert two.run([1], [54], may_follow=True) == [56]
+    assert one.run([0, 2], [13, 29], may_follow=True) == [14, 32]
+    assert two.run([1], [56]) == [58]
+    one.drain()
+    assert two.run([0, 2], [70, 80]) == [71, 83]
+    assert one.run([0, 2], [90, 40]) == [91, 43]                         # the same sequences, not the tokens that lie there
+    got = one.run([0, 2], [91, 43])
+    got[0] = 7
+    assert one.run([0, 2], got) == [8, 49]
+
+
 def test_tokens_that_are_waited_for_come_from_the_steps_own_stream(monkeypatch):
     """Another stream that is idle says nothing about the step's: no error while that one still runs."""
     idle, busy = SimpleNamespace(query=lambda: True), SimpleNamespace(query=lambda: False)

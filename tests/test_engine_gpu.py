@@ -246,3 +246,26 @@ def test_decoding_goes_on_where_the_stream_changes(pattern):
     assert tokens("AAAAAA", False) == want
     for drop in (False, True):
         assert tokens(pattern, True, drop) == want
+
+
+def test_two_decode_runners_of_one_engine():
+    """Two runners whose steps, enqueued ahead, take turns on the engine's buffers: each gets the tokens that it gets alone."""
+    import llm_infer_amd
+    from llm_infer_amd.sampling import Sampler
+    eng = llm_infer_amd.random_model(llm_infer_amd.config_from_dict(ALL["A"]), seed=3, dtype="bfloat16", max_tokens=1024)
+    g = torch.Generator().manual_seed(2)
+    prompts = [[torch.randint(0, eng.vocab_size, (n,), generator=g).tolist() for n in lens] for lens in ((20, 7, 33), (11, 64))]
+    turns = [(0, True), (1, True), (0, False), (0, True), (1, True), (1, True), (0, True), (0, True), (1, False), (0, False)]
+
+    def tokens(order):
+        slots = [[eng.alloc_slot() for _ in p] for p in prompts]
+        toks = [[eng.step(s, p).argmax(-1).tolist()] for s, p in zip(slots, prompts)]
+        runners = [eng.decode_runner(Sampler(0.0)) for _ in prompts]
+        for who, follow in order:
+            toks[who].append(runners[who].run(slots[who], toks[who][-1], may_follow=follow))
+        for s in slots[0] + slots[1]:
+            eng.free_slot(s)
+        return toks
+    want = tokens(sorted((who, False) for who, _ in turns))
+    for _ in range(3):
+        assert tokens(turns) == want
