@@ -126,7 +126,8 @@ class GraphDecodeRunner:
             # device, the ring), the last step's by a copy
             self.bufs["steps"] = torch.zeros((n,), dtype=torch.int32, device=dev)
             self.bufs["host"] = [Tensor.pinned((ops.TOKEN_RING, n), torch.int64), Tensor.pinned((n,), torch.int32)]
-            self.bufs["launched"] = 0              # steps enqueued so far: what the counters will stand at
+            self.bufs["launched"] = 0              # steps enqueued so far: what the counters will stand at,
+            self.bufs["counted"] = True            # unless a step failed while it was being enqueued
             self.bufs["stream"] = None             # where the newest of them was
             # what the buffers hold, which all runners of the engine share: the rows' slots, and the newest step, whose tokens they are
             self.bufs["held"] = self.bufs["last"] = None
@@ -156,14 +157,14 @@ class GraphDecodeRunner:
         if b["stream"] is not None and b["stream"] != stream:
             stream.wait_stream(b["stream"])      # the step before works in the same buffers, and on the same sequences
         b["stream"] = stream
-        try:
-            self._enqueue(slots, tokens)
-        except BaseException:
-            # whether the step's first kernel ran is not known: go on from a number that none has had
-            b["launched"] += 2
+        counted, b["counted"] = b["counted"], False
+        if not counted:
+            # whether the first kernel of the step that failed ran is not known: go on from a number that none has had
+            b["launched"] += 1
             b["steps"].fill_((b["launched"] + (1 << 31)) % (1 << 32) - (1 << 31))
-            raise
+        self._enqueue(slots, tokens)
         b["launched"] += 1
+        b["counted"] = True
         b["last"] = _Step(slots, b["launched"], stream)
         return b["last"]
 

@@ -104,10 +104,11 @@ class Device:
             def rest():
                 b["tokens"].values[:n] = [t + s + 1 for t, s in zip(b["tokens"].values[:n], b["slots"].values[:n])]
 
+            self.current.queue.append(prepare)
             if self.fails:
                 self.fails -= 1
                 raise RuntimeError("this step fails")
-            self.current.queue += [prepare, rest]
+            self.current.queue.append(rest)
         runner._body = body
         return runner
 
@@ -156,6 +157,30 @@ def test_runners_of_one_engine_keep_their_own_tokens(monkeypatch):
     got = one.run([0, 2], [91, 43])
     got[0] = 7
     assert one.run([0, 2], got) == [8, 49]
+
+
+@pytest.mark.parametrize("fails", [1, 2])
+def test_a_step_that_fails_says_why_and_the_next_ones_are_right(monkeypatch, fails):
+    """An error while a step is being enqueued reaches the caller as it is, whatever state the device is in, and no later step is taken
+    for the one that failed, whose first kernel may have run."""
+    dev = Device(monkeypatch)
+    runner = dev.runner()
+    assert runner.run([0, 2], [10, 20], may_follow=True) == [11, 23]
+    fill, lost = Buffer.fill_, lambda self, v: (_ for _ in ()).throw(ValueError("the device is lost"))
+    dev.fails = 1
+    monkeypatch.setattr(Buffer, "fill_", lost)
+    with pytest.raises(RuntimeError, match="this step fails"):
+        runner.run([0, 2], [11, 23], may_follow=True)                    # (fails as the one behind it is enqueued)
+    monkeypatch.setattr(Buffer, "fill_", fill)
+    dev.fails = fails - 1
+    for _ in range(fails - 1):
+        with pytest.raises(RuntimeError, match="this step fails"):
+            runner.run([0, 2], [30, 40])
+    assert runner.run([0, 2], [30, 40], may_follow=True) == [31, 43]
+    assert runner.run([0, 2], [31, 43], may_follow=True) == [32, 46]
+    assert runner.run([0, 2], [32, 46]) == [33, 49]
+    assert runner.run([1], [5], may_follow=True) == [7]
+    runner.drain()
 
 
 def test_tokens_that_are_waited_for_come_from_the_steps_own_stream(monkeypatch):

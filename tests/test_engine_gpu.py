@@ -269,3 +269,44 @@ def test_two_decode_runners_of_one_engine():
     want = tokens(sorted((who, False) for who, _ in turns))
     for _ in range(3):
         assert tokens(turns) == want
+
+
+@pytest.mark.parametrize("step", [0, 1, 2, 5])
+def test_a_decode_step_that_fails_leaves_the_runner_usable(step, monkeypatch):
+    """A part that raises while a step is enqueued (run eagerly, recorded, or recorded behind one whose tokens are still out): the
+    caller sees that error, and the next sequences get the tokens that they get on an engine that never failed."""
+    import llm_infer_amd
+    from llm_infer_amd.sampling import Sampler
+    cfg = llm_infer_amd.config_from_dict(ALL["A"])
+    prompts = [list(range(5, 25)), [3] * 60]                 # (the second grows into another bucket of contexts: another recording)
+
+    def tokens(eng, n, fail_at=None):
+        slots = [eng.alloc_slot() for _ in prompts]
+        toks = [eng.step(slots, prompts).argmax(-1).tolist()]
+        runner, forward, calls = eng.decode_runner(Sampler(0.0)), eng.model.head.forward, []
+
+        def failing(h):
+            calls.append(0)
+            if len(calls) == 1:
+                raise ValueError("this part fails")
+            return forward(h)
+        try:
+            for i in range(n):
+                if i == fail_at:
+                    torch.cuda.synchronize()                 # (a recorded step may still be running)
+                    eng._graphs.clear()                      # (this one is run eagerly, the next one recorded, anew)
+                    monkeypatch.setattr(eng.model.head, "forward", failing)
+                toks.append(runner.run(slots, toks[-1], may_follow=i + 1 < n))
+        finally:
+            monkeypatch.undo()
+            runner.drain()
+            torch.cuda.synchronize()
+            for s in slots:
+                eng.free_slot(s)
+        return toks
+    want = tokens(llm_infer_amd.random_model(cfg, seed=3, dtype="bfloat16", max_tokens=1024), 8)
+    eng = llm_infer_amd.random_model(cfg, seed=3, dtype="bfloat16", max_tokens=1024)
+    with pytest.raises(ValueError, match="this part fails"):
+        tokens(eng, 8, step)
+    for _ in range(3):
+        assert tokens(eng, 8) == want
