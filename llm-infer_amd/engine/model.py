@@ -156,16 +156,17 @@ class DecoderModel(Part):
                 for e in self.schedule for m in self.layer_mixers[e.layer]
                 for j, spec in enumerate(cache_specs_of(m))] + self._embedding_specs()
 
-    def _views_of(self, i, cache) -> list:
-        """One cache view for each mixer of schedule entry ``i``, or the list of its views for one that asks several things of the cache."""
-        return [[cache.view(u) for u in self._seen[i, k]] if multi else cache.view(self._seen[i, k][0])
-                for k, multi in enumerate(self._multi[self.schedule[i].layer])]
+    def _views_of(self, cache) -> list:
+        """For every schedule entry one cache view for each of its mixers, or the list of its views for one that asks several things of
+        the cache."""
+        return [[[cache.view(u) for u in self._seen[i, k]] if multi else cache.view(self._seen[i, k][0])
+                 for k, multi in enumerate(self._multi[e.layer])] for i, e in enumerate(self.schedule)]
 
-    def _norms_of_entry(self, i, ctx, cache) -> tuple:
+    def _norms_of_entry(self, i, ctx, views) -> tuple:
         """The RMS norms (weight, eps, type) that read the residual stream as the layer of schedule entry ``i`` begins, where
         the layer says so (``input_norms``) and nothing rewrites the stream ahead of it: at most two, the others run by themselves.  With them
         the short convolution that reads one of them (``input_convs``) in a step of one token a sequence, as ``ops.average_norms`` takes
-        it, or None."""
+        it, or None.  ``views``: every entry's."""
         if i >= len(self.schedule) or self._before[i] is not None:
             return [], None
         entry = self.schedule[i]
@@ -174,7 +175,7 @@ class DecoderModel(Part):
             return [], None
         convs = [None] * len(layer.sublayers)
         if ctx.n_tokens == ctx.n_seqs and entry.cache_from is None and hasattr(layer, "input_convs"):
-            convs = layer.input_convs(self._views_of(i, cache))
+            convs = layer.input_convs(views[i])
         norms, conv = [], None
         for (n, dt), c in zip(layer.input_norms(), convs):
             if isinstance(n, RMSNorm) and n.weight is not None and len(norms) < 2:
@@ -183,7 +184,7 @@ class DecoderModel(Part):
                 norms.append((n.weight, n.eps, dt))
         return norms, conv
 
-    def _shift_of_entry(self, i, x, ctx, cache):
+    def _shift_of_entry(self, i, x, ctx, views):
         """The token shift of the rows ``x`` with which the layer of schedule entry ``i`` begins, as the pass that finishes them takes it
         (``ops.add_layernorm``), or None: in a step of one token a sequence, where nothing rewrites the stream ahead of the layer."""
         if i >= len(self.schedule) or self._before[i] is not None or ctx.n_tokens != ctx.n_seqs or x.data_ptr() % 16:
@@ -192,7 +193,7 @@ class DecoderModel(Part):
         layer = self.layers[entry.layer]
         if entry.cache_from is not None or not hasattr(layer, "input_shift"):
             return None
-        shift = layer.input_shift(self._views_of(i, cache))
+        shift = layer.input_shift(views[i])
         return (*shift[:2], ctx, shift[2]) if shift is not None and ops.shift_fits(*shift[:2]) else None
 
     # -- the forward pass of one step ---------------------------------------
@@ -202,12 +203,13 @@ class DecoderModel(Part):
             x = x0 = self.embedding.forward(ctx, [cache.view(u) for u in self._embedding_units])
         else:
             x = x0 = self.embedding.forward(ctx)
-        history, n_hist = None, 0
+        # (made once a step: an eager step of few tokens is the host's)
+        views, history, n_hist = self._views_of(cache), None, 0
         if self._n_after:
             # the stream's values side by side: the embedding's output, then the result of every run that an
             # ``after`` part follows (the run works in place on the row that the part before it has written)
             history = torch.empty((self._n_after + 2,) + tuple(x0.shape), dtype=torch.float32, device=x0.device)
-            x, n_hist, (norms, conv) = history[1], 1, self._norms_of_entry(0, ctx, cache)
+            x, n_hist, (norms, conv) = history[1], 1, self._norms_of_entry(0, ctx, views)
             if norms and ops.average_norms_fit(x0, None, x, norms):
                 ops.average_norms(x0.unsqueeze(0), 1, None, x, norms, also=history[0], conv=conv, ctx=ctx)
             else:
@@ -222,7 +224,6 @@ class DecoderModel(Part):
                 x = part.forward(x, x0, ctx, e.pass_no) if getattr(part, "takes_pass", False) else part.forward(x, x0, ctx)
             elif x is x0 and self.stream_parts and history is None:
                 x = ops.copy_rows(x0)            # the layers add in place, and a later part reads the embedding's output
-            views = self._views_of(i, cache)
             layer = self.layers[e.layer]
             if getattr(layer, "takes_next_norm", False):
                 # the norm that reads the residual stream after this layer: the next layer's first
@@ -234,15 +235,15 @@ class DecoderModel(Part):
                     part = self.stream_parts[self._before[i + 1]]
                     if hasattr(part, "addends"):
                         extra["also"], entered = part.addends(x0, self.schedule[i + 1].pass_no), True
-                layer.forward(x, ctx, views, e.cache_from is None, next_norm=first() if first else None, **extra)
+                layer.forward(x, ctx, views[i], e.cache_from is None, next_norm=first() if first else None, **extra)
             elif getattr(layer, "takes_next_shift", False):
-                layer.forward(x, ctx, views, e.cache_from is None, next_shift=self._shift_of_entry(i + 1, x, ctx, cache) if self._after[i] is None else None)
+                layer.forward(x, ctx, views[i], e.cache_from is None, next_shift=self._shift_of_entry(i + 1, x, ctx, views) if self._after[i] is None else None)
             else:
-                layer.forward(x, ctx, views, e.cache_from is None)
+                layer.forward(x, ctx, views[i], e.cache_from is None)
             if self._after[i] is not None:
                 n_hist += 1                      # x is history[n_hist - 1], now a finished value of the stream
                 part = self.stream_parts[self._after[i]]
-                norms, conv = self._norms_of_entry(i + 1, ctx, cache) if getattr(part, "takes_norms", False) else ([], None)
+                norms, conv = self._norms_of_entry(i + 1, ctx, views) if getattr(part, "takes_norms", False) else ([], None)
                 x = part.forward_after(history, n_hist, history[n_hist], ctx, **({"norms": norms, "conv": conv} if norms else {}))
         if ctx.n_want == 0:
             return torch.empty((0, self.spec.vocab_size), dtype=torch.float32, device=x.device)

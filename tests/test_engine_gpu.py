@@ -310,3 +310,24 @@ def test_a_decode_step_that_fails_leaves_the_runner_usable(step, monkeypatch):
         tokens(eng, 8, step)
     for _ in range(3):
         assert tokens(eng, 8) == want
+
+
+@pytest.mark.parametrize("design", ["manirax", "dupolorn", "dopivik", "favizen", "pusisun", "risonex"])
+def test_a_step_asks_for_every_view_of_the_cache_once(design, monkeypatch):
+    """An eager step of few tokens is bound by the host: also where a pass takes along what the next layer begins with, the views
+    of the cache are made once a step."""
+    import importlib
+    from collections import Counter
+    import llm_infer_amd
+    models = importlib.import_module(design + "_models")
+    for cfg in models.ALL.values():
+        eng = llm_infer_amd.random_model(llm_infer_amd.config_from_dict(cfg), seed=1, dtype="bfloat16", max_tokens=256)
+        eng.record_prefill = False
+        slots, view, asked = [eng.alloc_slot(), eng.alloc_slot()], eng.cache.view, Counter()
+        monkeypatch.setattr(eng.cache, "view", lambda unit: (asked.update([unit]), view(unit))[1])
+        # (a run that reads another's cache asks for that one's views)
+        times = Counter(u for units in eng.model._seen.values() for u in units) + Counter(eng.model._embedding_units)
+        for toks in ([[1, 2, 3], [4, 5]], [[6], [7]]):
+            asked.clear()
+            eng.step(slots, toks)
+            assert asked == times
