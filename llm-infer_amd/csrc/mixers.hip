@@ -934,7 +934,11 @@ extern "C" int li_decay_attn(const float* proj, int stride, int q_off, int k_off
 
 // ---------------------------------------------------------------------------
 // A decode step of the recurrence (one token a sequence) in workgroups beside those that store the other mixer's keys and values: both read the
-// input product and neither the other's result (a decode step of four layers 4,096 wide: 445 -> 432 us).
+// input product and neither the other's result (a decode step of four layers 4,096 wide: 445 -> 432 us).  For every number of rows of S a
+// thread has, where those divide a head's and a workgroup is whole waves.  us at 1, 4, 16 and 64 sequences, two launches and one, 16 heads of
+// 128 x 128 beside as many queries (32 rows) 6.0 and 3.5, 6.5 and 4.1, 9.7 and 7.2, 31.7 and 23.8; of 64 x 64 (8) 5.3 and 2.9, 5.4 and 2.9, 6.2 and 4.3,
+// 10.1 and 8.8; of 64 x 128 (16) 5.6 and 3.1, 5.8 and 3.5, 7.4 and 5.3, 16.2 and 12.4; 8 of 256 x 256 (64) 7.1 and 4.6, 8.2 and 5.5, 14.4 and 12.9,
+// 54.6 and 45.3; 8 of 32 x 32 (4) 5.1 and 2.8, 5.3 and 2.8, 5.3 and 2.9, 5.8 and 3.6.
 // ---------------------------------------------------------------------------
 struct DecayStep {
     const float* proj;
@@ -946,7 +950,7 @@ struct DecayStep {
     int n_seqs, H, d, dv, round_dt;
 };
 
-template <class T>
+template <class T, int ROWS>
 __global__ __launch_bounds__(512) void store_beside_decay_kernel(
     const float* __restrict__ qkv, int row_stride, const float* __restrict__ inv_freq, const float* __restrict__ cos_sin, int rot, int half_pairing,
     float unit_eps, const int* __restrict__ pos, const int* __restrict__ tok_slot, Pages c, T* __restrict__ q_out, int H, int G, int d, int dv, int dq,
@@ -959,11 +963,24 @@ __global__ __launch_bounds__(512) void store_beside_decay_kernel(
         return;
     }
     const int j = i - store_blocks, of = b.H * split;
-    decay_attn_part<32, T, true>(b.proj, b.stride, b.q_off, b.k_off, b.v_off, b.state, b.decay, b.seq_slot, nullptr, nullptr, b.out, b.H, b.d, b.dv, lds,
+    decay_attn_part<ROWS, T, true>(b.proj, b.stride, b.q_off, b.k_off, b.v_off, b.state, b.decay, b.seq_slot, nullptr, nullptr, b.out, b.H, b.d, b.dv, lds,
                                  j / of, j % of / split, j % split, split);
 }
 
-// beside (or null): a step of the recurrence that is run along, in the same launch where its sizes allow.
+// Threads of a workgroup in which the step runs beside the keys and values of so many tokens of type dt (0: in a launch of its own), the rows of S of
+// a thread, and the pieces of a head's columns.
+static int beside_shape(const DecayStep& b, int n_tokens, int dt, int& rows, int& split) {
+    if (b.n_seqs <= 0 || b.H <= 0 || b.d <= 0 || b.dv <= 0 || b.d > 256 || b.dv > 256 || n_tokens >= 512 || dt == DT_F32 || b.round_dt != dt) return 0;
+    decay_shape(b.n_seqs, b.H, b.d, b.dv, rows, split);
+    const int threads = b.d / rows * (b.dv / split);
+    return b.d % rows == 0 && threads <= 512 && threads % 64 == 0 ? threads : 0;
+}
+extern "C" int li_decay_rides(const DecayStep* b, int n_tokens, int dt) {
+    int rows, split;
+    return beside_shape(*b, n_tokens, dt, rows, split) > 0;
+}
+
+// beside (or null): a step of the recurrence that is run along, in the same launch where its sizes allow (li_decay_rides).
 extern "C" int li_rope_norm_store(const float* qkv, int row_stride, const float* inv_freq, const float* cos_sin, int rot,
                                   int half_pairing, float unit_eps, const int* pos, const int* tok_slot, const void* k_pages,
                                   const void* v_pages, int64_t page_stride, const int* page_table, int max_pages,
@@ -977,14 +994,16 @@ extern "C" int li_rope_norm_store(const float* qkv, int row_stride, const float*
     if (beside) {
         const DecayStep& b = *beside;
         int rows = 0, split = 1;
-        if (b.n_seqs > 0 && b.H > 0 && b.d > 0 && b.dv > 0 && b.d <= 256 && b.dv <= 256) decay_shape(b.n_seqs, b.H, b.d, b.dv, rows, split);
-        const int threads = rows ? b.d / rows * (b.dv / split) : 0;
-        if (rows == 32 && b.d % 32 == 0 && threads <= 512 && threads % 64 == 0 && n_tokens < 512 && dt != DT_F32 && b.round_dt == dt) {
+        const int threads = beside_shape(b, n_tokens, dt, rows, split);
+        if (threads) {
             const int parts = (H + 2 * G + threads / 64 - 1) / (threads / 64), cols = b.dv / split;
             const size_t lds = (size_t)(2 * b.d + cols + threads) * sizeof(float);
-#define GO(T) store_beside_decay_kernel<T><<<n_tokens * parts + b.n_seqs * b.H * split, threads, lds, stream>>>(qkv, row_stride, inv_freq, cos_sin, rot, \
+#define GO(T, ROWS) store_beside_decay_kernel<T, ROWS><<<n_tokens * parts + b.n_seqs * b.H * split, threads, lds, stream>>>(qkv, row_stride, inv_freq, cos_sin, rot, \
         half_pairing, unit_eps, pos, tok_slot, c, (T*)q_out, H, G, d, dv, dq, dk, dvp, n_tokens * parts, parts, split, b)
-            if (dt == DT_F16) GO(f16); else GO(bf16);
+#define BY_ROWS(T) do { switch (rows) { case 4: GO(T, 4); break; case 8: GO(T, 8); break; case 16: GO(T, 16); break; case 32: GO(T, 32); break; \
+                                default: GO(T, 64); } } while (0)
+            if (dt == DT_F16) BY_ROWS(f16); else if (dt == DT_BF16) BY_ROWS(bf16); else return LI_BAD_ARG;
+#undef BY_ROWS
 #undef GO
             LI_CHECK_LAUNCH();
             return LI_OK;

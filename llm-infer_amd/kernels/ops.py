@@ -1354,6 +1354,10 @@ class PendingDecay:
         self.step = _DecayStep(proj.data_ptr(), proj.shape[1], q_off, k_off, v_off, state.data_ptr(), decay.data_ptr(), seq_slot.data_ptr(), self.out.data_ptr(),
                                n_seqs, n_heads, head_dim, v_head_dim, DT[round_to or torch.float32])
 
+    def rides(self, n_tokens: int, dtype) -> bool:
+        """True if ``rope_norm_store`` of so many tokens in this type runs it in its own launch."""
+        return bool(mixers().li_decay_rides(ctypes.byref(self.step), n_tokens, DT[dtype]))
+
     def rows(self) -> torch.Tensor:
         if not self.done:
             self.out = decay_attention(*self.args)

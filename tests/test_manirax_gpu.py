@@ -533,10 +533,14 @@ def test_partial_sums_added_beside_a_gated_norm(rows, n, splits, dv, shares):
         assert (outs[0][1].double() - want).abs().max().item() < 2.0 ** -8 * (1 + want.abs().max().item())
 
 
-@pytest.mark.parametrize("B,H,G,d,dv,Hd,dd,ddv", [(1, 16, 4, 128, 128, 8, 128, 128), (8, 4, 2, 64, 64, 16, 128, 128), (3, 8, 8, 48, 32, 3, 96, 128),
-                                                  (17, 2, 1, 64, 64, 2, 64, 256), (2, 4, 2, 64, 64, 4, 64, 64), (1, 4, 4, 64, 64, 2, 80, 96), (1, 2, 2, 64, 64, 2, 256, 256)])
-def test_a_recurrence_step_beside_the_kernel_of_the_keys(B, H, G, d, dv, Hd, dd, ddv):
-    """Bit for bit the two launches, where the sizes allow one and where they do not."""
+@pytest.mark.parametrize("B,H,G,d,dv,Hd,dd,ddv,rides", [
+    (1, 16, 4, 128, 128, 8, 128, 128, True), (8, 4, 2, 64, 64, 16, 128, 128, True), (3, 8, 8, 48, 32, 3, 96, 128, False), (17, 2, 1, 64, 64, 2, 64, 256, True),
+    (2, 4, 2, 64, 64, 4, 64, 64, True), (1, 2, 2, 64, 64, 2, 256, 256, True), (5, 3, 1, 64, 80, 3, 32, 32, True), (33, 4, 4, 128, 128, 9, 64, 128, True),
+    (1, 4, 4, 64, 64, 2, 80, 96, False), (2, 4, 2, 64, 64, 2, 72, 64, False), (2, 4, 2, 64, 64, 2, 70, 64, False), (512, 2, 1, 16, 16, 1, 16, 64, False),
+    (511, 2, 1, 16, 16, 1, 16, 64, True)])
+def test_a_recurrence_step_beside_the_kernel_of_the_keys(B, H, G, d, dv, Hd, dd, ddv, rides):
+    """Bit for bit the two launches, where the sizes allow one and where they do not: 4 to 64 rows a thread, rows that do not divide a
+    head's, workgroups that are no whole waves, many tokens."""
     from llm_infer_amd.kernels import ops
     g = torch.Generator().manual_seed(B + H + dd)
     up = lambda n: (n + 15) // 16 * 16
@@ -555,6 +559,7 @@ def test_a_recurrence_step_beside_the_kernel_of_the_keys(B, H, G, d, dv, Hd, dd,
             k, v = (torch.zeros((B + 2) * (per[0] + per[1]), dtype=dt, device=DEV) for _ in range(2))
             s = state.clone()
             run = ops.PendingDecay(proj, n1, n1 + Hd * dd, n1 + 2 * Hd * dd, s, decay, slot, B, Hd, dd, ddv, None if dt == torch.float32 else dt)
+            assert run.rides(B, dt) == (rides and dt != torch.float32)
             if not together:
                 run.rows()
             q = ops.rope_norm_store(proj, freq, d // 2, True, 1e-6, pos, slot, (k, v, per[0] + per[1], table), H, G, d, dv, up(d), up(d), up(dv), dt,
