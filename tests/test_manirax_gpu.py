@@ -512,20 +512,24 @@ def test_a_token_shift_in_the_pass_that_finishes_its_rows(rows, d):
 
 @pytest.mark.parametrize("rows,n", [(1, 64), (3, 260), (8, 2048), (2, 4100), (255, 300), (256, 300), (1, 16384), (1, 16388)])
 @pytest.mark.parametrize("splits,dv,shares", [(2, 32, 5), (16, 128, 32), (11, 48, 3)])
-def test_partial_sums_added_beside_a_gated_norm(rows, n, splits, dv, shares):
+def test_partial_sums_added_beside_a_gated_norm(rows, n, splits, dv, shares, monkeypatch):
     """Bit for bit the two launches, where the norm takes the sums along and where it does not (many rows, wide rows, another type)."""
     from llm_infer_amd.kernels import build, ops
     g = torch.Generator().manual_seed(rows + n + splits)
     rand = lambda *shape: torch.randn(*shape, generator=g).to(DEV)
     o, w, gate, part = rand(rows, n), rand(n), rand(rows, n + 7), rand(1, shares, splits, dv)
     lib = build.sigmoid_attention_library(48, 32)
+    finish, alone = ops.PendingMerge.finish, []
+    monkeypatch.setattr(ops.PendingMerge, "finish", lambda self: (alone.append(self.part is not None), finish(self))[1])
     for dtype, of in ((torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float16)):
         outs = []
         for along in (False, True):
             pending = ops.PendingMerge(part, torch.full((1, shares, dv), 9.0, dtype=of, device=DEV), lib)
             if not along:
                 pending.finish()
+            alone.clear()
             normed = ops.gated_rmsnorm(o, w, gate, 7, 1e-5, dtype, pending if along else None)
+            assert not along or any(alone) == (rows >= 256 or n > 16 * 1024 or dtype != of)
             pending.finish()                             # (nothing is left of it)
             outs.append((normed, pending.out))
         assert all(torch.equal(a, b) for a, b in zip(*outs))
