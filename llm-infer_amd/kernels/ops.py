@@ -391,7 +391,7 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
             ro = rsc = None
             # 9 to 16 rows with the residual sum against a matrix with a long K (output products, down): gemm_rows, one tile of W
             # a workgroup, whose rows of X come in whole lines: with four waves from 2,048 rows of W on, with as many as gemv_tiled has
-            # below, where four (K in half as many parts) would add 1.3 to 1.4 times its error against 64 bits.  (us, gemv_tiled, four waves
+            # below (four sum K in half as many parts: 1.3 to 1.4 times gemv_tiled's error against 64 bits).  (us, gemv_tiled, four waves
             # and eight, at 9, 12 and 16 rows: 4,096 x 14,336 22.8, 21.7, 22.5; 24.6, 22.2, 23.4; 28.5, 22.3, 23.2; 2,048 x 8,192 12.0, 11.1,
             # 11.8; 12.7, 11.0, 11.7; 13.7, 11.9, 12.6; 1,024 x 8,192 10.5, 9.4, 10.3; 11.7, 10.0, 11.0; 13.2, 10.9, 11.8; but at 12 and 16
             # rows 2,048 x 4,096 8.1, 6.9, 8.1; 8.1, 7.1, 8.2, 512 x 4,096 7.0, 6.1, 7.1; 7.7, 6.5, 7.6)

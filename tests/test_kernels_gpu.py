@@ -339,8 +339,8 @@ def test_linear_tiled_weights(ops, M, N, K, dt):
 
 @pytest.mark.parametrize("dt", F16S)
 @pytest.mark.parametrize("M,N,K", [(17, 16, 32), (32, 40, 96), (33, 100, 544), (48, 520, 1056), (49, 72, 64), (64, 48, 4128),       # blocks of rows of X
-                                   (12, 2064, 8192), (16, 2048, 4096), (9, 32, 4128), (11, 2064, 8192), (12, 16, 4064),             # either side of "a long K"
-                                   (17, 12288, 1024), (32, 12304, 96), (32, 12272, 1024), (24, 12288, 1056)])                        # of "wide and shallow"
+                                   (12, 2064, 8192), (16, 2048, 4096), (9, 32, 4128), (11, 2064, 8192), (12, 16, 4064),             # few rows and a long K
+                                   (17, 12288, 1024), (32, 12304, 96), (32, 12272, 1024), (24, 12288, 1056)])                        # wide and shallow
 def test_more_rows_than_one_block_and_the_rules_beside_them(ops, M, N, K, dt):
     """gemm_rows with one to four blocks of 16 rows of X, shares of K with and without whole stages, and the planner's choice on
     either side of its rules, as tall products with the residual sum and without (K sums in float32: 2e-4 as above)."""
