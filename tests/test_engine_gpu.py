@@ -223,7 +223,7 @@ def test_decoding_goes_on_where_the_stream_changes(pattern):
     g = torch.Generator().manual_seed(2)
     prompts = [torch.randint(0, eng.vocab_size, (n,), generator=g).tolist() for n in (20, 7, 33)]
     streams = {"A": torch.cuda.Stream(), "B": torch.cuda.Stream()}
-    big, out = torch.randn(4096, 4096, device="cuda", dtype=torch.bfloat16), {k: torch.empty(4096, 4096, device="cuda", dtype=torch.bfloat16) for k in streams}
+    big, out = torch.ones(4096, 4096, device="cuda", dtype=torch.bfloat16), {k: torch.empty(4096, 4096, device="cuda", dtype=torch.bfloat16) for k in streams}
 
     def tokens(names, busy, drop=False):
         slots = [eng.alloc_slot() for _ in prompts]
