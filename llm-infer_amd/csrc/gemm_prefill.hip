@@ -258,7 +258,10 @@ __device__ __forceinline__ void wreg_epilogue(const Epilogue& e, int m, int n, c
 // goes through them, with 4 bytes a lane a store, they were 5 to 20% of a product (us before and after, bfloat16, gate and up:
 // 12,700 x 28,672 x 4,096 2,396 and 2,201, 33,186 x 16,384 x 2,048 1,831 and 1,639, 777 x 16,384 x 2,048 64 and 50; plain
 // store 12,700 x 4,096 x 4,096 341 and 318).
-template <class OT, int NI, int MJ, int MODE>
+// TANH: the activations of EPI_BIAS that take a tanhf, in code of their own and with one tanhf a value.  With tanh and the soft cap as two in the
+// code that all of EPI_BIAS shares, every quad of the others ran past 95 KiB more (us, float16, with tanh alone there, with both, and now: relu2 1,680 x
+// 14,336 x 4,096 190, 201, 186, 512 x 32,000 x 2,048 60.6, 67.5, 57.9; tanh 211, 221, 206, and 73.3, 77.7, 69.6; the soft cap 226 and 204, 79.4 and 67.5).
+template <class OT, int NI, int MJ, int MODE, bool TANH = false>
 __device__ __forceinline__ void rows_out(const Epilogue& e, const f32x4 (&acc)[NI][MJ], unsigned char* stage, int lane, int m0, int nb) {
     constexpr bool GATED_MODE = MODE == EPI_SWIGLU || MODE == EPI_GEGLU || MODE == EPI_CLAMPGLU;
     constexpr int STRIPS = 2;                                  // of 16 rows a turn
@@ -295,11 +298,13 @@ __device__ __forceinline__ void rows_out(const Epilogue& e, const f32x4 (&acc)[N
                     *(Two*)(at + (8 * i + 2 * g) * sizeof(OT)) = two;
                 } else {
                     if constexpr (MODE == EPI_BIAS) {
+                        if constexpr (TANH) {
+                            float z[4] = {v[0], v[1], v[2], v[3]};
+                            tanh_activation(e.gp, z);
+                            v = f32x4{z[0], z[1], z[2], z[3]};
+                        } else if (e.gp.act == 1) {
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            if (e.gp.act == 1) { const float t = fmaxf(v[q], 0.f); v[q] = t * t; }
-                            else if (e.gp.act == 2) v[q] = tanhf(v[q]);
-                            else if (e.gp.act == 3) v[q] = e.gp.limit * tanhf(v[q] / e.gp.limit);
+                            for (int q = 0; q < 4; ++q) { const float t = fmaxf(v[q], 0.f); v[q] = t * t; }
                         }
                     }
                     struct alignas(4 * sizeof(OT)) Four { OT v[4]; };
@@ -643,8 +648,15 @@ __global__ __launch_bounds__(256, A == 4 ? 1 : 2) void gemm_wreg_kernel(const T*
                 if (e.mode == EPI_SWIGLU) rows_out<T, NI, MJ, EPI_SWIGLU>(e, acc, rows, lane, m0, nb);
                 else if (e.out_dt == DT_F32) rows_out<float, NI, MJ, EPI_STORE>(e, acc, rows, lane, m0, nb);
                 else rows_out<T, NI, MJ, EPI_STORE>(e, acc, rows, lane, m0, nb);
-            } else if (e.out_dt == DT_F32) rows_out<float, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
-            else rows_out<T, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
+            } else {
+                if constexpr (MODE == EPI_BIAS) if (e.gp.act >= 2) {
+                    if (e.out_dt == DT_F32) rows_out<float, NI, MJ, MODE, true>(e, acc, rows, lane, m0, nb);
+                    else rows_out<T, NI, MJ, MODE, true>(e, acc, rows, lane, m0, nb);
+                    return;
+                }
+                if (e.out_dt == DT_F32) rows_out<float, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
+                else rows_out<T, NI, MJ, MODE>(e, acc, rows, lane, m0, nb);
+            }
             return;
         }
     }

@@ -1167,6 +1167,25 @@ def test_a_soft_cap_in_the_products_epilogue(ops, M, N, K):
         ops.linear(x, w, ops.EPI_BIAS, out_dtype=torch.float32, params=ops.glu_params(act="softcap", limit=0.0))
 
 
+@pytest.mark.parametrize("N", [592, 583])
+@pytest.mark.parametrize("M,force", [(300, "wreg:0"), (300, "wreg:1"), (300, "wreg:2"), (50, "wreg:2:1:1"), (100, "wreg:2:1:3"), (129, "wreg:2:2")])
+def test_activations_in_the_epilogue_of_prompts_products(ops, M, force, N):
+    """Bit for bit the activation of the stored float32 sums, with a bias and without: whole rows and the last columns, every tile, K whole and
+    split.  tanh is the soft cap of 1."""
+    g = torch.Generator().manual_seed(M + N)
+    for dt in (torch.float16, torch.bfloat16):
+        x, w = torch.randn(M, 256, generator=g).to(DEV, dt), ops.prepare_weight((torch.randn(N, 256, generator=g) / 8).to(DEV, dt))
+        bias = torch.randn(N, generator=g).to(DEV)
+        run = lambda out=torch.float32, **p: ops.linear(x, w, ops.EPI_BIAS, out_dtype=out, force=force, params=ops.glu_params(**p))
+        plain = ops.linear(x, w, out_dtype=torch.float32, force=force)
+        for b, sums in ((None, plain), (bias, plain + bias)):
+            for out in (torch.float32, dt):
+                assert torch.equal(run(out, bias=b, act="relu2"), sums.clamp(min=0).square().to(out))
+                assert torch.equal(run(out, bias=b, act="tanh"), ops.softcap(sums.clone(), 1.0).to(out))
+                assert torch.equal(run(out, bias=b, act="softcap", limit=3.5), ops.softcap(sums.clone(), 3.5).to(out))
+        assert torch.equal(run(bias=bias), plain + bias)
+
+
 @pytest.mark.parametrize("rows,n", [(1, 1), (5, 3), (130, 130), (130, 66)])
 def test_a_steps_first_kernel_sends_the_tokens_before_it_to_the_host(ops, rows, n):
     """decode_prepare's ring of tokens, recorded and replayed: every step's own tokens, rows that a smaller step leaves out keep
