@@ -177,9 +177,10 @@ class DecoderModel(Part):
         if ctx.n_tokens == ctx.n_seqs and entry.cache_from is None and hasattr(layer, "input_convs"):
             convs = layer.input_convs(views[i])
         norms, conv = [], None
+        first = next((c for c in convs if c is not None), None)        # (the layer asks for its branches' in this order)
         for (n, dt), c in zip(layer.input_norms(), convs):
             if isinstance(n, RMSNorm) and n.weight is not None and len(norms) < 2:
-                if c is not None and conv is None and ops.norm_conv_fits(*c[:2]):
+                if c is not None and c is first and ops.norm_conv_fits(*c[:2]):
                     conv = (len(norms),) + tuple(c)
                 norms.append((n.weight, n.eps, dt))
         return norms, conv

@@ -174,3 +174,25 @@ def test_random_weights_mode_writes_a_folder_of_the_design(tmp_path):
     assert set(f.names()) == set(M.random_weights(M.TINY_B, 0))
     assert tuple(f.info("l0.norm1")[1]) == () and tuple(f.info("l2.dwa")[1]) == (4,)
     assert abs(float(f.tensor("l2.dwa").float().sum()) - 1.0) < 0.5
+
+
+@pytest.mark.parametrize("taps,rides", [((3, 5), 0), ((5, 3), None), ((5, 5), None), ((2, 4), 0), ((None, 3), 1), ((3, None), 0)])
+def test_which_convolution_rides_with_the_norms(taps, rides):
+    """The first of a layer's branches that begin with a convolution, which is the first that asks for its result, where the pass takes so many
+    taps; never a later one's in its place."""
+    from types import SimpleNamespace
+    from llm_infer_amd.engine.model import DecoderModel
+    from llm_infer_amd.parts import ParallelBlock, RMSNorm
+    subs = []
+    for n in taps:
+        norm = RMSNorm(size=8, eps=1e-5, prefix="", dtype=torch.float32, device="cpu")
+        norm.weight = torch.ones(8)
+        part = SimpleNamespace() if n is None else SimpleNamespace(input_conv=lambda view: (view, view.new_zeros(2, view.shape[1] - 1, 8), torch.float32))
+        subs.append(SimpleNamespace(role="mixer", norm=norm, post_norm=None, part=part))
+    layer = ParallelBlock(subs)
+    model = SimpleNamespace(schedule=[SimpleNamespace(layer=0, cache_from=None)], _before=[None], layers=[layer])
+    views = [[torch.zeros(8, n or 1) for n in taps]]
+    norms, conv = DecoderModel._norms_of_entry(model, 0, SimpleNamespace(n_tokens=2, n_seqs=2), views)
+    assert [w is s.norm.weight for (w, _, _), s in zip(norms, subs)] == [True, True]
+    assert (conv[0], conv[1] is views[0][rides]) == (rides, True) if rides is not None else conv is None
+    assert DecoderModel._norms_of_entry(model, 0, SimpleNamespace(n_tokens=3, n_seqs=2), views)[1] is None
