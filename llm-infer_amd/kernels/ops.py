@@ -1549,7 +1549,7 @@ def gated_rmsnorm(o, w, gate_rows, gate_off, eps, out_dtype, merge: PendingMerge
     if merge is not None and (merge.part is None or merge.out.dtype != out_dtype or not 1 <= t < 256 or n > 16 * 1024):
         merge.finish()
         merge = None
-    along = (_ptr(merge.part), _ptr(merge.out), merge.rows, merge.splits, merge.dv) if merge is not None else (_ptr(None), _ptr(None), 0, 0, 0)
+    along = (_ptr(merge.part), _ptr(merge.out), merge.rows, merge.splits, merge.dv) if merge is not None else (None, None, 0, 0, 0)
     _check(mixers().li_gated_rmsnorm(_ptr(o), _ptr(w), _ptr(gate), gate_rows.shape[1], _ptr(out), DT[out_dtype], t, n,
                                      c_float(eps), *along, _stream()), "gated_rmsnorm")
     if merge is not None:

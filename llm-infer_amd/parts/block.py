@@ -116,7 +116,7 @@ class ParallelBlock(Block):
         return out
 
     def _normed(self, s, x, view):
-        if hasattr(s.part, "input_conv"):
+        if getattr(x, "_li_convolved", None) is not None and hasattr(s.part, "input_conv"):
             ready = ops.prepared_conv(x, s.norm.weight, s.norm.eps, *s.part.input_conv(view)[:2])
             if ready is not None:
                 return ready

@@ -63,11 +63,13 @@ class ParallelMixers(Part):
 
     def addends(self, h, ctx, views, owns_cache=True):
         out, at, merge, step = [], 0, None, None
+        # (in longer prompts nothing is taken together, and the host has its launches to make)
+        together = ctx.is_decode or h.shape[0] <= 16
         proj = ops.linear(h, self.w_in, out_dtype=torch.float32) if getattr(self, "w_in", None) is not None else None
         for i, (branch, scale) in enumerate(zip(self.branches, self.scales)):
             view, at = views_for(branch, views, at)
             shared = {"proj": proj, "col0": self._col0[i]} if proj is not None and self._col0[i] is not None else {}
-            if hasattr(branch, "before_output"):
+            if together and hasattr(branch, "before_output"):
                 # all but its output product, which runs with the others'; what completes its rows rides in the next branch's last kernel
                 follows = self.branches[i + 1] if i + 1 < len(self.branches) else None
                 if getattr(branch, "merges_later", False) and step is None and getattr(follows, "takes_merge", False):
@@ -86,6 +88,8 @@ class ParallelMixers(Part):
                 y = torch.zeros((h.shape[0], branch.hidden_size), dtype=torch.float32, device=h.device)
                 branch.forward(h, ctx, view, y, owns_cache)
                 out.append((y, scale))
+        if not together:
+            return out
         ready = iter(ops.finish_products([y for y, _ in out if isinstance(y, ops.PendingProduct)]))
         return [(next(ready) if isinstance(y, ops.PendingProduct) else y, s) for y, s in out]
 
