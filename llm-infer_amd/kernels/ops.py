@@ -394,11 +394,14 @@ def linear(x: torch.Tensor, w, mode: int = EPI_STORE, out: torch.Tensor | None =
             # below (four sum K in half as many parts: 1.3 to 1.4 times gemv_tiled's error against 64 bits).  (us, gemv_tiled, four waves
             # and eight, at 9, 12 and 16 rows: 4,096 x 14,336 22.8, 21.7, 22.5; 24.6, 22.2, 23.4; 28.5, 22.3, 23.2; 2,048 x 8,192 12.0, 11.1,
             # 11.8; 12.7, 11.0, 11.7; 13.7, 11.9, 12.6; 1,024 x 8,192 10.5, 9.4, 10.3; 11.7, 10.0, 11.0; 13.2, 10.9, 11.8; but at 12 and 16
-            # rows 2,048 x 4,096 8.1, 6.9, 8.1; 8.1, 7.1, 8.2, 512 x 4,096 7.0, 6.1, 7.1; 7.7, 6.5, 7.6)
+            # rows 2,048 x 4,096 8.1, 6.9, 8.1; 8.1, 7.1, 8.2, 512 x 4,096 7.0, 6.1, 7.1; 7.7, 6.5, 7.6.)  9 to 11 rows against more than 2,048
+            # rows of W: gemv_tiled, but for the longest K gemm_rows with eight (us at 9, 10 and 11 rows: 5,120 x 13,824 36.5 and 35.7, 37.7
+            # and 36.5, 37.3 and 35.8; 4,096 x 14,336 22.9 and 22.9, 21.9 and 21.5, 22.3 and 21.7; but 4,096 x 8,192 14.4 and 15.0, 13.9 and 14.6,
+            # 13.9 and 14.6, 5,120 x 8,192 21.8 and 22.8, 21.8 and 22.6, 22.2 and 23.1, 6,144 x 16,384 45.0, 45.9 and 46.2 either way)
             like = None
             if force is None and m > 8 and lazy is None and experts is None and (m > 16 or (mode == EPI_ADD and k >= 8192 and n % 16 == 0)):
                 four = m <= 16 and (n == 2048 or (n > 2048 and m >= 12))
-                like = (1, 4) if four else _rows_like_tiled(m, n, k) if m > 16 or n < 2048 else None
+                like = (1, 4) if four else _rows_like_tiled(m, n, k) if m > 16 or n < 2048 or (k >= 12288 and n <= 5120) else None
             nxt = getattr(out, "_li_next_norm", None) if mode == EPI_ADD else None
             if (nxt is not None and m <= 16 and n % 32 == 0 and out.data_ptr() % 16 == 0 and nxt.dtype == torch.float32
                     and nxt.shape == (n,) and nxt.is_cuda and nxt.data_ptr() % 16 == 0):
@@ -671,7 +674,7 @@ def _rows_like_tiled(m: int, n: int, k: int) -> tuple[int, int] | None:
     waves = core().li_gemv_tiled_waves(m, n, k)
     if k % 64 or -(-k // (32 * waves)) % 2:
         return None
-    if n <= 4096:
+    if n <= 4096 or m <= 16:
         return 1, waves
     if k < (1024 if waves == 8 else 512) or (n > 14336 and k <= 1024):
         return None

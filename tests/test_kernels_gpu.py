@@ -364,6 +364,7 @@ def test_more_rows_than_one_block_and_the_rules_beside_them(ops, M, N, K, dt):
                                         (24, 3072, 2048, (1, 8)), (32, 48, 320, (1, 8)), (17, 6144, 2048, (2, 8)), (24, 4112, 1024, (2, 8)),
                                         (32, 8192, 4096, (2, 8)), (17, 10240, 512, (2, 4)), (24, 14336, 1024, (2, 4)), (18, 14352, 1280, (2, 4)),
                                         (32, 16384, 2048, (2, 4)), (9, 1024, 8192, (1, 8)), (16, 2032, 8192, (1, 8)), (12, 256, 14336, (1, 8)),
+                                        (9, 5120, 13824, (1, 8)), (11, 2064, 12288, (1, 8)),
                                         (31, 100, 864, None), (24, 1024, 1056, None), (20, 8192, 512, None), (32, 14352, 1024, None),
                                         (20, 10240, 288, None), (12, 1024, 8224, None), (16, 2048, 4096, "short"), (12, 512, 8128, "short")])
 def test_a_products_sums_do_not_depend_on_the_kernel_of_few_rows(ops, M, N, K, rows, dt):
