@@ -439,17 +439,23 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
     if (rc) return rc;
     const int chains = (K + CHAIN - 1) / CHAIN, blocks = (N + 15) / 16;
     // Whole chains: gemv_f32 up to 16 rows (20: 3,072 x 2,048 at 17 rows 14.0 us, gemm_f32_chains 14.7, at 24 rows 15.2 and 14.7), fewer against many
-    // rows of W (6,144 x 4,096 at 9 and 16 rows 29.0 and 28.0, 33.7 and 28.3, at 8 rows 28.9 and 28.1; but 8,192 x 512 6.9 and 7.9).  Beyond, the rounds
-    // of 256 tiles: gemm_f32's take 36.7 us at K = 2,048 (one alone 43.5), gemm_f32_chains' 10.3 (375 rows x 16,384 x 2,048, 6 rounds and 24, 225 and 245
-    // us; x 3,072 x 2,048, 2 and 5, 76 and 53).
+    // rows of W (6,144 x 4,096 at 9 and 16 rows 29.0 and 28.0, 33.7 and 28.3, at 8 rows 28.9 and 28.1; but 8,192 x 512 6.9 and 7.9).  Beyond, an
+    // estimate of both in us, fitted to 2,348 products of 21 to 1,000 rows, 320 to 28,672 rows of W and K of 256 to 8,192: rounds of 256 tiles (one that is
+    // not full counts for nearly a whole one), each as long as its K for gemm_f32, and for gemm_f32_chains as the chains of its busiest wave and all
+    // of them.  What it names takes 0.2% more than the faster one in the mean, 15% at most; by the rounds alone, with K = 2,048 in mind, it was 3%, where four
+    // waves do not share K evenly most (677 rows x 1,024 x 512 13.9 and 16.7, 195 x 28,672 x 1,536 204 and 231, 200 x 8,192 x 256 15.7 and 26.2).
     // Else gemv_f32 has its workgroups by the rows of W alone, gemm_f32 fills the chip only where both sides have enough
     // rows.  us at 64 rows of X: 2,048 x 2,048 25 against 41, 2,048 x 8,192 89 against 160, but 16,384 x 2,048 71 against 49; at
     // 32 rows 16,384 x 2,048 46 against 49
-    auto rounds = [&](int side) { return ((int64_t)((M + side - 1) / side) * ((N + side - 1) / side) + 255) / 256; };
+    auto rounds = [&](int side, double last) {
+        const int64_t tiles = (int64_t)((M + side - 1) / side) * ((N + side - 1) / side);
+        return last * ((tiles + 255) / 256) + (1 - last) * tiles / 256;
+    };
     if (kind == 0 && K % CHAIN == 0) {
-        const int64_t n64 = rounds(64);
+        const double whole = rounds(64, 0.9) * (1.4 + 0.0156 * K) + 2.7 + 0.004 * K;
+        const double shared = (rounds(32, 0.85) + 0.2) * (0.55 + 2.0 * ((chains + 3) / 4) + 0.62 * chains) + 4.4;
         if (M <= 8 || (M <= 20 && (blocks < 384 || chains < 8))) kind = 1;
-        else kind = 10.3 * rounds(32) < 36.7 * n64 + (n64 == 1 ? 7 : 3) && (int64_t)((M + 31) / 32) * ((N + 31) / 32) <= F32_TILES ? 3 : 2;
+        else kind = shared < whole && (int64_t)((M + 31) / 32) * ((N + 31) / 32) <= F32_TILES ? 3 : 2;
     } else if (kind == 0) kind = M <= 32 || (M <= 64 && blocks < 1024) || (M <= 128 && blocks <= 256) ? 1 : 2;
     if (kind == 1) {
         const int mt = M <= 16 ? 1 : (M <= 32 ? 2 : 4), nt = M > 8 && blocks >= 1024 ? 2 : 1;
