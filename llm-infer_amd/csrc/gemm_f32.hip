@@ -465,9 +465,10 @@ extern "C" int li_gemm_f32(const float* X, const float* W, void* C, int out_dt, 
         // up to 128 blocks and 8 rows: half blocks, so that every CU has a workgroup, a wave for each pair of chains.  Beyond 256 blocks with two
         // chains and more a wave, half blocks where the rows are few (us of whole and half ones at 1, 2, 4 and 8 rows: 5,120 x 4,096 24.6 and 19.3,
         // 23.4 and 20.1, 25.2 and 22.4, 28.0 and 26.8; 8,192 x 4,096 29.2 and 26.7, 27.7 and 26.2, 28.0 and 28.9, 30.2 and 36.7; 28,672 x 4,096 88.9
-        // and 78.7, 84.2 and 81.5, 88.6 and 92.4)
+        // and 78.7, 84.2 and 81.5, 88.6 and 92.4; but with pairs that eight waves do not share evenly 2 rows x 8,192 x 14,336 89 and 96, x 11,008 x 5,120 50
+        // and 52)
         const bool pairs_whole = K % (2 * CHAIN) == 0;
-        const bool few = pairs_whole && chains >= 16 && blocks > 256 && (M <= 2 || (M <= 4 && blocks <= 384));
+        const bool few = K % (16 * CHAIN) == 0 && blocks > 256 && (M <= 2 || (M <= 4 && blocks <= 384));
         if (few || (M <= 8 && blocks <= 128)) {
             const int pairs = (chains + 1) / 2, waves = pairs <= 4 ? 4 : pairs <= 8 || few ? 8 : 16;
             const unsigned grid = (N + 7) / 8;
