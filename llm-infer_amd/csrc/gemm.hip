@@ -558,6 +558,23 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
                     for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[u][t], b[u][j], acc[t][j]);
         }
     };
+    // One step that is left, or all that a short K gives a wave: under no condition either (us, a whole batch under its condition, and now: 1 row x 14,336 x
+    // 64 4.8 and 4.35, x 2,048 x 64 2.91 and 2.75, x 4,096 x 256 3.31 and 3.09, 3 rows x 14,336 x 64 3.3 and 3.08).  Asked for behind the ring alone: as one of
+    // the ring's own depths it cost every other product 0.04 us.
+    auto last_step = [&](auto once) {
+        v8 a[NT], b[MT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const T* from = wt[t] + (int64_t)s_begin * 512;
+            a[t] = decltype(once)::value ? load_once<v8>(from) : *(const v8*)from;
+        }
+#pragma unroll
+        for (int j = 0; j < MT; ++j) b[j] = *(const v8*)(xrow[j] + s_begin * 32);
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int j = 0; j < MT; ++j) acc[t][j] = mfma16(a[t], b[j], acc[t][j]);
+    };
     auto products = [&](auto once) {
         const int n = (s_end - s_begin) / SL;
         bool in_order = MT <= 2;
@@ -570,7 +587,10 @@ __global__ __launch_bounds__(64 * KW) void gemv_tiled_kernel(const T* __restrict
             else if (in_order && n == 3) ring(std::integral_constant<int, 3>{}, once);
             else add_squares();
         }
-        if (s_begin < s_end) batches(once);
+        if (s_begin < s_end) {
+            if (in_order && s_begin + SL == s_end) last_step(once);
+            else batches(once);
+        }
     };
     if constexpr (MT == 1) products(std::true_type{});
     else if (past) products(std::true_type{});
