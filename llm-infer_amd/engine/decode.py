@@ -219,7 +219,7 @@ class GraphDecodeRunner:
         """The tokens of ``step``, the newest one or the one before it.  Where a step has been enqueued behind it, that step's first kernel
         sends them and the host polls for them: no copy and no event between two recorded steps (a step
         of four layers 2,048 wide, batch 1, 263.9 -> 256.2 us, batch 8 373.7 -> 368.5; 4,096 wide 480.1 -> 474.8)."""
-        if step.tokens is None and self._ahead is not None and self._ahead.number == step.number + 1:
+        if step.tokens is None and self._ahead is not None:          # (enqueued right behind it: by its own number, which a failure may have moved)
             step.tokens = ops.wait_tokens(self.bufs["host"][0], len(step.slots), self._ahead.number, self._ahead.stream)
         return self._tokens_of(step)
 

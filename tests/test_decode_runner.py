@@ -183,6 +183,22 @@ def test_a_step_that_fails_says_why_and_the_next_ones_are_right(monkeypatch, fai
     runner.drain()
 
 
+def test_a_step_ahead_outlives_another_runners_failure(monkeypatch):
+    """Another runner's step that fails on the host, as one that the cache has no room for does, takes nothing from a step enqueued ahead:
+    its tokens are its own, and not those of the step that is then enqueued behind it under a number that is not the next."""
+    dev = Device(monkeypatch)
+    one, two = dev.runner(), dev.runner()
+    assert one.run([0, 2], [10, 20], may_follow=True) == [11, 23]
+    grow = dev.engine.cache.grow
+    dev.engine.cache.grow = lambda *args, **kw: (_ for _ in ()).throw(RuntimeError("no room"))
+    with pytest.raises(RuntimeError, match="no room"):
+        two.run([1], [50])
+    dev.engine.cache.grow = grow
+    assert one.run([0, 2], [11, 23], may_follow=True) == [12, 26]
+    assert one.run([0, 2], [12, 26]) == [13, 29]
+    assert two.run([1], [50]) == [52]
+
+
 def test_tokens_that_are_waited_for_come_from_the_steps_own_stream(monkeypatch):
     """Another stream that is idle says nothing about the step's: no error while that one still runs."""
     idle, busy = SimpleNamespace(query=lambda: True), SimpleNamespace(query=lambda: False)
